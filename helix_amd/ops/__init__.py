@@ -188,7 +188,7 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                             window, cu_seqlens_k)
 
 
-# Flash-decoding split-K quantum (must match PART_QUANT in
+# Tokens that decode attention cuts sequences in (must match UNIT in
 # paged_attn_decode.hip).
 DECODE_PARTITION = 128
 

@@ -1,23 +1,36 @@
 // Paged-attention decode (single query token per sequence) for CDNA4.
 //
-// Replaces the decode attention the reference delegates to vLLM
-// (SURVEY.md §2.8 "Decode attention (paged KV)").
+// Replaces the decode attention the reference delegates to vLLM. Bound by the
+// cache: every key and value is read once for the G = Hq / Hkv query heads
+// that share it.
 //
-// Design (MI355X-first, v3 — templated + load-batched):
-//  - KV-bandwidth-bound: each KV byte is read once per kv-head and
-//    amortized across the G = Hq/Hkv GQA query heads.
-//  - grid = (num_seqs, Hkv, num_partitions): flash-decoding split-K, host
-//    sizes partitions to fill the 256 CUs (>= ~1024 workgroups).
-//  - DHEAD and G are template parameters so every inner loop fully
-//    unrolls; K rows and V tiles are loaded into registers in batches
-//    BEFORE any math so the wave keeps many VMEM ops in flight (v2's
-//    runtime-D loops serialized load->use and reached only 0.5 TB/s —
-//    profiles/r01_decode_profile_v1.md).
-//  - 128-thread blocks (2 waves) walk the partition in 128-token chunks:
-//      A: thread t loads K row of token t (DHEAD/8 x 16B batched), dots
-//         against the G query vectors in LDS (broadcast reads).
-//      B: per-head online softmax (running m, l), one wave per head.
-//      C: V accumulation, thread owns a dim pair, 8-token load batches.
+//  - A wave works alone on tiles of 32 keys and passes nothing through LDS
+//    until the waves of a workgroup put their results together, so no barrier
+//    stands between loads. Keys go straight from their pages into MFMA
+//    operands (scores key x query); they are permuted so that lane group hi
+//    ends up with the scores of the 8 keys whose values it loads itself. The
+//    query columns repeat every four lanes, so a weight of another head is a
+//    quad broadcast away and the value product runs in fp32 on whole 16-byte
+//    rows, without a transpose and without rounding the weights.
+//  - The next tile's keys are under way during softmax and value product, its
+//    values during the next scores; page numbers are read a tile earlier.
+//  - Work is cut by the lengths themselves, on the device, because a captured
+//    graph only knows its bucket: all (sequence, head) pairs share TARGET
+//    workgroups in proportion to their tokens, in units of 128. Sequences in
+//    one piece are written at once, others are merged by a second launch.
+//
+// Before, a partition was a share of the bucket, its two waves met at three
+// barriers per 128 tokens and the value product waited for the softmax of all
+// heads. Measured with 32 heads on 8, 16-token pages in random order, merge
+// included (us before -> now, TB/s now):
+//   1 row of 777            22.5 -> 10.3      (launches and latency)
+//   8 of 300..6000, window  89 -> 32          3.2
+//   61 of 1000..4096        345 -> 134        4.7
+//   512 of 513..640         279 -> 226        5.35
+//   24 of 4000..16000, fp8  487 -> 117        4.4
+// A large read-only sum reaches 6.1 TB/s. TARGET of 512 to 2048 is within 5%
+// of each other; the results' distance from 64 bits is what it was (their
+// rounding to bf16).
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -26,548 +39,460 @@ using namespace helix;
 
 namespace {
 
-constexpr int NTHREADS = 128;
-constexpr int CHUNK = 128;
-constexpr int MAX_G = 8;
-constexpr int PART_QUANT = 128;
+constexpr int NT = 256, NW = NT / WAVE;
+constexpr int KT = 32;                        // keys of a tile
+constexpr int UNIT = KT * NW;                 // tokens that work is cut in
+constexpr int TARGET = 1024;                  // workgroups: 4 on each CU
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float NEG = -1e30f;
 
-// MFMA_A: phase A computes scores with f32_16x16x32_bf16 matrix ops
-// (16 tokens x G queries per instruction) instead of per-thread VALU
-// dots — motivated by the B=512 PMC: 37 VALU per vector load and
-// wait:busy 14:1 (profiles/r01_pmc_decode_b512.txt).
-// KV8: the paged cache holds OCP e4m3 bytes (opt-in
-// kv_cache_dtype="fp8"): halves the KV traffic this kernel is
-// latency/BW-bound on; dequant is one v_cvt per element in the math
-// loops. MFMA_A and KV8 are mutually exclusive instantiations.
-// VPS: phase-C V rows staged RAW (u16x8) per batch — the round-2
-// deep-pipelining lever (PMC wait:busy 14:1, latency-bound): more V
-// bytes in flight per wave before any conversion VALU touches them.
-// OCC: launch_bounds waves/SIMD floor override (0 = round-1 default).
-// KPRE: inter-chunk K prefetch. The r2 ISA audit (profiles/
-// r02_decode_kpre.md) showed the compiler sinking phase A's 16-deep raw
-// K staging into the consume loop — steady state s_waitcnt vmcnt(1),
-// i.e. only ~2 VMEM loads in flight per wave, matching the 14:1
-// wait:busy PMC. KPRE hoists the next chunk's 16 b128 K loads to just
-// after the current chunk's scores are consumed, so they land during
-// phases B+C (softmax + V) instead of head-of-line blocking phase A.
-template <int DHEAD, int G, bool MFMA_A, bool KV8, int VPS = 4, int OCC = 0,
-          bool KPRE = false>
-__global__ __launch_bounds__(NTHREADS, (OCC > 0 ? OCC : (G <= 2 ? 4 : 3))) void paged_attn_decode_kernel(
-    uint16_t* __restrict__ out,          // [B, Hq, D] (used when nparts==1)
-    float* __restrict__ tmp_out,         // [B, Hq, maxP, D]
-    float* __restrict__ tmp_ml,          // [B, Hq, maxP, 2]
-    const uint16_t* __restrict__ q,      // [B, Hq, D]
-    const uint16_t* __restrict__ k_cache,// [nblocks, Hkv, bs, D]
-    const uint16_t* __restrict__ v_cache,
-    const int* __restrict__ block_tables,// [B, max_blocks]
-    const int* __restrict__ seq_lens,    // [B]
-    float scale, int Hkv, int block_size, int max_blocks,
-    int partition_size, int max_parts, int window) {
-  const int seq = blockIdx.x;
-  const int hkv = blockIdx.y;
-  const int part = blockIdx.z;
-  const int nparts = gridDim.z;
-  const int Hq = Hkv * G;
-  const int len = seq_lens[seq];
-  const int kv_lo = (window > 0) ? max(0, len - window) : 0;
-  int p_start = part * partition_size;
-  const int p_hi = min(len, p_start + partition_size);
-  if (p_start < kv_lo) p_start = kv_lo;
-  if (p_start >= len || p_hi <= kv_lo) {
-    if (nparts > 1 && threadIdx.x == 0) {
+struct Rows {
+  const int* bt;               // [B, max_blocks]
+  const int* lens;             // [B]
+  uint16_t* out;               // [B, Hq, D]
+  float* part;                 // [B, Hq, max_parts, D]
+  float* ml;                   // [B, Hq, max_parts, 2]
+  int B, Hkv, bs, shift, max_blocks, max_parts, window, limit;
+  bool split;
+  float mul;                   // scale * log2(e)
+};
+
+__device__ __forceinline__ float max_over_groups(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const unsigned w = __float_as_uint(x);
+  const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float sum_over_groups(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const unsigned w = __float_as_uint(x);
+  const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// Lane j of every four, in all four.
+template <int J>
+__device__ __forceinline__ float quad(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(
+      __float_as_int(v), J * 0x55, 0xf, 0xf, true));
+}
+template <int J>
+__device__ __forceinline__ float of_head(const float* v) {
+  return quad<(J & 3)>(v[J >> 2]);
+}
+
+// Tokens that sequence b's query sees are [first, len); units are whole.
+// No more than the caller's bound, which the grid is sized by.
+__device__ __forceinline__ int len_of(const Rows& m, int b) {
+  return min(m.lens[b], m.limit);
+}
+__device__ __forceinline__ int first_key(const Rows& m, int len) {
+  return m.window > 0 ? max(0, len - m.window) : 0;
+}
+__device__ __forceinline__ int units_of(const Rows& m, int b) {
+  if (b >= m.B) return 0;
+  const int len = len_of(m, b);
+  return len > 0 ? cdiv(len - first_key(m, len) / KT * KT, UNIT) : 0;
+}
+
+// Units of a workgroup such that all pieces come to about TARGET.
+__device__ __forceinline__ int piece_for(const Rows& m, int units) {
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int hq = hkv * G + g;
-        float* ml = tmp_ml + (((int64_t)seq * Hq + hq) * max_parts + part) * 2;
-        ml[0] = -INFINITY;
-        ml[1] = 0.f;
-      }
+  for (int off = 32; off > 0; off >>= 1) units += __shfl_xor(units, off, WAVE);
+  return max(1, cdiv(units * m.Hkv, TARGET));
+}
+// Pieces of a sequence (one, if it is empty: its zeros have to be written).
+__device__ __forceinline__ int pieces_of(const Rows& m, int units, int c) {
+  return min(max(1, cdiv(units, c)), m.max_parts);
+}
+
+// Number `left` of the pieces of 64 sequences, `mine` of them this lane's.
+__device__ __forceinline__ bool find_in(int mine, int& left, int& at, int& p,
+                                        int& n) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  int upto = mine;
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const int v = __shfl_up(upto, off, WAVE);
+    if (lane >= off) upto += v;
+  }
+  const int total = __shfl(upto, WAVE - 1, WAVE);
+  if (left >= total) {
+    left -= total;
+    return false;
+  }
+  at = __ffsll((unsigned long long)__ballot(left < upto)) - 1;
+  n = __shfl(mine, at, WAVE);
+  p = left - (__shfl(upto, at, WAVE) - n);
+  return true;
+}
+
+// Sequence and piece number of this workgroup; false where none is left.
+__device__ __forceinline__ bool find(const Rows& m, int& seq, int& p,
+                                     int& n) {
+  seq = blockIdx.x;
+  p = 0;
+  n = 1;
+  if (!m.split) return true;
+  const int lane = threadIdx.x & (WAVE - 1);
+  int left = blockIdx.x;
+  if (m.B <= WAVE) {                          // each length is read once
+    const int u = units_of(m, lane), c = piece_for(m, u);
+    return find_in(lane < m.B ? pieces_of(m, u, c) : 0, left, seq, p, n);
+  }
+  int u = 0;
+  for (int b = lane; b < m.B; b += WAVE) u += units_of(m, b);
+  const int c = piece_for(m, u);
+  for (int b0 = 0; b0 < m.B; b0 += WAVE) {
+    const int b = b0 + lane;
+    if (find_in(b < m.B ? pieces_of(m, units_of(m, b), c) : 0, left, seq, p,
+                n)) {
+      seq += b0;
+      return true;
     }
-    return;
   }
-  const int p_end = p_hi;
+  return false;
+}
 
-  __shared__ float q_lds[G][DHEAD];
-  __shared__ float s_lds[G][CHUNK];
-  __shared__ float head_m[MAX_G], head_l[MAX_G], head_corr[MAX_G];
+// A key row's or value row's elements of this lane as they lie in memory.
+template <int BYTES> struct Raw;
+template <> struct Raw<4> { typedef uint32_t T; };
+template <> struct Raw<8> { typedef u32x2 T; };
+template <> struct Raw<16> { typedef u32x4 T; };
 
-  for (int idx = threadIdx.x; idx < G * DHEAD; idx += NTHREADS) {
-    const int g = idx / DHEAD, d = idx % DHEAD;
-    q_lds[g][d] =
-        bf16_to_f32(q[((int64_t)seq * Hq + hkv * G + g) * DHEAD + d]) * scale;
-  }
-  if (threadIdx.x < MAX_G) {
-    head_m[threadIdx.x] = -INFINITY;
-    head_l[threadIdx.x] = 0.f;
-  }
-  __syncthreads();
-
-  // Q fragments for the MFMA path: A[row=query g][k=dim], rows >= G
-  // zero.  Lane holds A[lane&15][(lane>>4)*8+i] per 32-dim step.
-  constexpr int NKK = DHEAD / 32;
-  bf16x8 qfrag[MFMA_A ? NKK : 1];
-  if constexpr (MFMA_A) {
-    const int l_lo = threadIdx.x & 15;
-    const int l_hi = (threadIdx.x & (WAVE - 1)) >> 4;
+template <bool F8, int DPL>
+__device__ __forceinline__ void widen(const void* raw, float* v) {
+  const uint32_t* w = (const uint32_t*)raw;
+  if constexpr (F8) {
 #pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) {
+    for (int i = 0; i < DPL / 4; ++i) {
+      const auto a = __builtin_amdgcn_cvt_pk_f32_fp8(w[i], false);
+      const auto b = __builtin_amdgcn_cvt_pk_f32_fp8(w[i], true);
+      v[4 * i] = a[0];
+      v[4 * i + 1] = a[1];
+      v[4 * i + 2] = b[0];
+      v[4 * i + 3] = b[1];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < DPL / 2; ++i) {
+      v[2 * i] = __uint_as_float(w[i] << 16);
+      v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+  }
+}
+
+// 8 e4m3 values as bf16 (exact).
+__device__ __forceinline__ bf16x8 widen8(uint32_t a, uint32_t b) {
+  const auto p = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 1.f, false);
+  const auto q = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 1.f, true);
+  const auto r = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 1.f, false);
+  const auto s = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 1.f, true);
+  return bf16x8{p[0], p[1], q[0], q[1], r[0], r[1], s[0], s[1]};
+}
+
+// The part of the wave's work that every head adds for itself.
+template <int G, int J, int DPL>
+__device__ __forceinline__ void add_values(float (*acc)[DPL], const float* pg,
+                                           const float* v) {
+  if constexpr (J < G) {
+    const float w = G == 1 ? pg[0] : of_head<J>(pg);
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) acc[J][d] += w * v[d];
+    add_values<G, J + 1, DPL>(acc, pg, v);
+  }
+}
+template <int G, int J, int DPL>
+__device__ __forceinline__ void rescale(float (*acc)[DPL], const float* c) {
+  if constexpr (J < G) {
+    const float w = G == 1 ? c[0] : of_head<J>(c);
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) acc[J][d] *= w;
+    rescale<G, J + 1, DPL>(acc, c);
+  }
+}
+
+// What fits the registers without spilling.
+constexpr int waves_per_simd(int D, int G) {
+  return D == 128 ? (G > 4 ? 2 : 3) : (G > 4 ? 3 : 4);
+}
+
+// PAGE8: pages are a power of two of at least 8 tokens, so the 8 keys of a
+// lane group lie in one page.
+template <int D, int G, bool F8, bool PAGE8>
+__global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
+    const uint16_t* __restrict__ q, const void* __restrict__ kc,
+    const void* __restrict__ vc, Rows m) {
+  constexpr int NC = D / 32;                  // inner steps of the scores
+  constexpr int DPL = D / 16;                 // value dimensions of a lane
+  constexpr int QS = G > 4 ? G / 4 : 1;       // sets of query columns
+  constexpr int EB = F8 ? 1 : 2;              // bytes of a cached element
+  // keys: a lane's 16 bytes of a row hold one step in bf16, two in e4m3
+  constexpr int KL = F8 ? NC / 2 : NC;
+  typedef typename Raw<DPL * EB>::T VRaw;
+  __shared__ float sh[NW][G][D];
+  __shared__ float st[2][NW][G];
+
+  const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+  const int lo = lane & 15, hi = lane >> 4;
+  int seq, part, parts;
+  if (!find(m, seq, part, parts)) return;
+  const int g = blockIdx.y, Hq = m.Hkv * G;
+  const int len = len_of(m, seq), first = first_key(m, len);
+  const int tile0 = first / KT, tiles = max(0, cdiv(len, KT) - tile0);
+  const int per = cdiv(tiles, parts);
+  const int t_end = tile0 + min(tiles, (part + 1) * per);
+  int t = tile0 + part * per + wid;
+
+  // Queries: the inner dimension is numbered as keys are loaded
+  bf16x8 qf[QS][NC];
+#pragma unroll
+  for (int s = 0; s < QS; ++s)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int h = g * G + s * 4 + (lo & (G < 4 ? G - 1 : 3));
+      const int d = F8 ? (j >> 1) * 64 + hi * 16 + (j & 1) * 8
+                       : j * 32 + hi * 8;
+      qf[s][j] = *reinterpret_cast<const bf16x8*>(
+          q + ((int64_t)seq * Hq + h) * D + d);
+    }
+
+  const int* bt = m.bt + (int64_t)seq * m.max_blocks;
+  const int last = len - 1;
+  auto page = [&](int key) {
+    key = min(key, last);
+    return bt[PAGE8 ? key >> m.shift : key / m.bs];
+  };
+  // Byte offset of a key's row. With PAGE8 the rows of a lane group follow
+  // each other; those past the end are there as well, and masked.
+  auto row_at = [&](int pg, int key) {
+    if constexpr (!PAGE8) key = min(key, last);
+    const int off = PAGE8 ? key & (m.bs - 1) : key % m.bs;
+    return (((int64_t)pg * m.Hkv + g) * m.bs + off) * (D * EB);
+  };
+  // operand row lo of half s is key 8 (lo / 4) + 4 s + lo % 4
+  const int key_k = (lo >> 2) * 8 + (lo & 3), key_v = hi * 8;
+  constexpr int KG = PAGE8 ? 1 : 2, VG = PAGE8 ? 1 : 8;
+  int kp[KG], vp[VG];
+  auto pages = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < KG; ++i) kp[i] = page(tile * KT + key_k + 4 * i);
+#pragma unroll
+    for (int i = 0; i < VG; ++i) vp[i] = page(tile * KT + key_v + i);
+  };
+  u32x4 kr[2][KL];
+  VRaw vr[8];
+  auto load_k = [&](int tile) {
+    const char* row[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      row[s] = s < KG ? (const char*)kc + hi * 16 +
+                            row_at(kp[s % KG], tile * KT + key_k + 4 * s)
+                      : row[0] + 4 * D * EB;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < KL; ++j)
+        kr[s][j] = *reinterpret_cast<const u32x4*>(row[s] + j * 64);
+  };
+  auto load_v = [&](int tile) {
+    const char* row[VG];
+#pragma unroll
+    for (int i = 0; i < VG; ++i)
+      row[i] = (const char*)vc + row_at(vp[i], tile * KT + key_v + i) +
+               lo * DPL * EB;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      vr[i] = *reinterpret_cast<const VRaw*>(row[i % VG] +
+                                             (i / VG) * D * EB);
+  };
+
+  float acc[G][DPL], m_run[QS], l[QS];
+#pragma unroll
+  for (int j = 0; j < G; ++j)
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) acc[j][d] = 0.f;
+#pragma unroll
+  for (int s = 0; s < QS; ++s) {
+    m_run[s] = NEG;
+    l[s] = 0.f;
+  }
+  if (t < t_end) {
+    pages(t);
+    load_k(t);
+    load_v(t);
+    pages(min(t + NW, t_end - 1));
+  }
+  for (; t < t_end; t += NW) {
+    const bool more = t + NW < t_end;
+    floatx4 x[QS][2];
+#pragma unroll
+    for (int s = 0; s < QS; ++s)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        x[s][u] = floatx4{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+          bf16x8 k;
+          if constexpr (F8) {
+            const u32x4 r = kr[u][j >> 1];
+            k = (j & 1) ? widen8(r[2], r[3]) : widen8(r[0], r[1]);
+          } else {
+            k = __builtin_bit_cast(bf16x8, kr[u][j]);
+          }
+          x[s][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[s][j],
+                                                            x[s][u], 0, 0, 0);
+        }
+      }
+    load_k(more ? t + NW : t);
+    __builtin_amdgcn_sched_barrier(0);
+    const int key0 = t * KT + key_v;
+    const bool edge = t * KT < first || (t + 1) * KT > len;
+    float p[8][QS], corr[QS];
+    bool keep = true;
+#pragma unroll
+    for (int s = 0; s < QS; ++s) {
+      float mx = m_run[s];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float qv = (l_lo < G)
-            ? q_lds[l_lo][kk * 32 + l_hi * 8 + i] : 0.f;
-        reinterpret_cast<uint16_t*>(&qfrag[kk])[i] = f32_to_bf16(qv);
+        float v = x[s][i >> 2][i & 3] * m.mul;
+        if (edge && (key0 + i < first || key0 + i >= len)) v = NEG;
+        p[i][s] = v;
+        mx = fmaxf(mx, v);
+      }
+      mx = max_over_groups(mx);
+      corr[s] = __builtin_amdgcn_exp2f(m_run[s] - mx);
+      keep = keep && mx == m_run[s];
+      m_run[s] = mx;
+      l[s] *= corr[s];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        p[i][s] = __builtin_amdgcn_exp2f(p[i][s] - mx);
+        l[s] += p[i][s];
       }
     }
+    // nothing that lies past the end may meet even a weight of zero
+    if (edge) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        vr[i] = key0 + i < first || key0 + i >= len ? VRaw(0) : vr[i];
+    }
+    if (!__all(keep)) rescale<G, 0, DPL>(acc, corr);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float v[DPL];
+      widen<F8, DPL>(&vr[i], v);
+      add_values<G, 0, DPL>(acc, p[i], v);
+      // else all values are widened at once and registers run out
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    load_v(more ? t + NW : t);
+    pages(min(t + 2 * NW, t_end - 1));
   }
 
-  // Phase-C ownership: a thread owns 8 consecutive dims (one 16B load
-  // per token) — the ablation probe showed b32 V loads were 64% of the
-  // kernel (8x more VMEM instructions per byte than phase A's b128s).
-  constexpr int NGRP = DHEAD / 8;            // dim-groups (16 for D=128)
-  constexpr int C_PAR = NTHREADS / NGRP;     // token parities (8 / 16)
-  const int d8 = (threadIdx.x % NGRP) * 8;   // my dims [d8, d8+8)
-  const int cpar = threadIdx.x / NGRP;
-  float acc[G][8];
+  // the lane groups, then the waves together
 #pragma unroll
-  for (int g = 0; g < G; ++g)
+  for (int s = 0; s < QS; ++s) {
+    l[s] = sum_over_groups(l[s]);
+    if (lane < min(4, G)) {
+      st[0][wid][s * 4 + lane] = m_run[s];
+      st[1][wid][s * 4 + lane] = l[s];
+    }
+  }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
-
-  const int* btable = block_tables + (int64_t)seq * max_blocks;
-  const int nwaves = NTHREADS / WAVE;
-  const int wid = threadIdx.x / WAVE;
-  const int lane = threadIdx.x & (WAVE - 1);
-
-  // KPRE: raw K rows for the chunk about to be scored, loaded one full
-  // chunk ahead (16 b128 loads live across phases B+C of the previous
-  // chunk — the latency they need to hide).
-  constexpr bool USE_KPRE = KPRE && !MFMA_A && !KV8;
-  constexpr bool USE_KPRE8 = KPRE && !MFMA_A && KV8;
-  u16x8 kpre[USE_KPRE ? DHEAD / 8 : 1];
-  u8x16 kpre8[USE_KPRE8 ? DHEAD / 16 : 1];
-  auto issue_kpre = [&](int cbase) {
-    const int tok = min(cbase + (int)threadIdx.x, p_end - 1);
-    const int64_t roff =
-        (((int64_t)btable[tok / block_size] * Hkv + hkv) *
-             (int64_t)block_size + tok % block_size) * DHEAD;
-    if constexpr (USE_KPRE8) {
-      const uint8_t* krow = (const uint8_t*)k_cache + roff;
+  for (int j = 0; j < G; ++j)
 #pragma unroll
-      for (int j = 0; j < DHEAD / 16; ++j)
-        kpre8[j] = *reinterpret_cast<const u8x16*>(krow + j * 16);
+    for (int d = 0; d < DPL; ++d) {
+      const float v = sum_over_groups(acc[j][d]);
+      if (hi == (j & 3)) sh[wid][j][lo * DPL + d] = v;
+    }
+  __syncthreads();
+  for (int i = threadIdx.x; i < G * D; i += NT) {
+    const int j = i / D, d = i % D;
+    float top = NEG, sum = 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) top = fmaxf(top, st[0][w][j]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = __builtin_amdgcn_exp2f(st[0][w][j] - top);
+      sum += f * st[1][w][j];
+      o += f * sh[w][j][d];
+    }
+    const int64_t row = (int64_t)seq * Hq + g * G + j;
+    if (parts == 1) {
+      m.out[row * D + d] = f32_to_bf16(o / fmaxf(sum, 1e-20f));
     } else {
-      const uint16_t* krow = k_cache + roff;
-#pragma unroll
-      for (int j = 0; j < (USE_KPRE ? DHEAD / 8 : 1); ++j)
-        kpre[j] = *reinterpret_cast<const u16x8*>(krow + j * 8);
-    }
-  };
-  if constexpr (USE_KPRE || USE_KPRE8) issue_kpre(p_start);
-
-  for (int base = p_start; base < p_end; base += CHUNK) {
-    const int chunk_n = min(CHUNK, p_end - base);
-
-    // --- Phase A: scores -------------------------------------------------
-    if constexpr (MFMA_A) {
-      // 16-token MFMA tiles; each wave owns alternating groups of 4.
-      const int ntiles = (chunk_n + 15) / 16;
-      const int l = threadIdx.x & (WAVE - 1);
-      const int l_lo = l & 15, l_hi = l >> 4;
-      for (int t0 = wid * 4; t0 < ntiles; t0 += nwaves * 4) {
-        const int nt = min(4, ntiles - t0);
-        u16x8 bfr[4][NKK];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if (u >= nt) continue;
-          const int tok = min(base + (t0 + u) * 16 + l_lo, p_end - 1);
-          const int64_t blk = btable[tok / block_size];
-          const uint16_t* krow =
-              k_cache + (((blk * Hkv + hkv) * (int64_t)block_size +
-                          tok % block_size)) * DHEAD;
-#pragma unroll
-          for (int kk = 0; kk < NKK; ++kk)
-            bfr[u][kk] = *reinterpret_cast<const u16x8*>(
-                krow + kk * 32 + l_hi * 8);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if (u >= nt) continue;
-          floatx4 sacc = floatx4{0, 0, 0, 0};
-#pragma unroll
-          for (int kk = 0; kk < NKK; ++kk)
-            sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                qfrag[kk], *reinterpret_cast<bf16x8*>(&bfr[u][kk]), sacc,
-                0, 0, 0);
-          // C[row=l_hi*4+r][col=l_lo]: row = query g, col = token
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int g = l_hi * 4 + r;
-            const int ci = (t0 + u) * 16 + l_lo;
-            if (g < G && ci < chunk_n) s_lds[g][ci] = sacc[r];
-          }
-        }
+      const int64_t at = row * m.max_parts + part;
+      m.part[at * D + d] = o;
+      if (d == 0) {
+        m.ml[at * 2] = top;
+        m.ml[at * 2 + 1] = sum;
       }
-    } else if constexpr (USE_KPRE) {
-      if ((int)threadIdx.x < chunk_n) {
-        float s[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) s[g] = 0.f;
-#pragma unroll
-        for (int j = 0; j < DHEAD / 8; ++j) {
-          float kv[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) kv[i] = bf16_to_f32(kpre[j][i]);
-#pragma unroll
-          for (int g = 0; g < G; ++g) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              s[g] += q_lds[g][j * 8 + i] * kv[i];
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) s_lds[g][threadIdx.x] = s[g];
-      }
-      // scores consumed: issue the NEXT chunk's K rows now so they
-      // fly during softmax + V accumulation
-      if (base + CHUNK < p_end) issue_kpre(base + CHUNK);
-    } else if constexpr (USE_KPRE8) {
-      if ((int)threadIdx.x < chunk_n) {
-        float s[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) s[g] = 0.f;
-#pragma unroll
-        for (int j = 0; j < DHEAD / 16; ++j) {
-          float kv[16];
-#pragma unroll
-          for (int i = 0; i < 16; ++i) kv[i] = fp8_to_f32(kpre8[j][i]);
-#pragma unroll
-          for (int g = 0; g < G; ++g) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-              s[g] += q_lds[g][j * 16 + i] * kv[i];
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) s_lds[g][threadIdx.x] = s[g];
-      }
-      if (base + CHUNK < p_end) issue_kpre(base + CHUNK);
-    } else if ((int)threadIdx.x < chunk_n) {
-      const int tok = base + threadIdx.x;
-      const int64_t blk = btable[tok / block_size];
-      const int64_t roff =
-          (((blk * Hkv + hkv) * (int64_t)block_size + tok % block_size)) *
-          DHEAD;
-      float s[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) s[g] = 0.f;
-      if constexpr (KV8) {
-        const uint8_t* krow = (const uint8_t*)k_cache + roff;
-        u8x16 kraw[DHEAD / 16];
-#pragma unroll
-        for (int j = 0; j < DHEAD / 16; ++j)
-          kraw[j] = *reinterpret_cast<const u8x16*>(krow + j * 16);
-#pragma unroll
-        for (int j = 0; j < DHEAD / 16; ++j) {
-          float kv[16];
-#pragma unroll
-          for (int i = 0; i < 16; ++i) kv[i] = fp8_to_f32(kraw[j][i]);
-#pragma unroll
-          for (int g = 0; g < G; ++g) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-              s[g] += q_lds[g][j * 16 + i] * kv[i];
-          }
-        }
-      } else {
-        const uint16_t* krow = k_cache + roff;
-        u16x8 kraw[DHEAD / 8];
-#pragma unroll
-        for (int j = 0; j < DHEAD / 8; ++j)
-          kraw[j] = *reinterpret_cast<const u16x8*>(krow + j * 8);
-#pragma unroll
-        for (int j = 0; j < DHEAD / 8; ++j) {
-          float kv[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) kv[i] = bf16_to_f32(kraw[j][i]);
-#pragma unroll
-          for (int g = 0; g < G; ++g) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              s[g] += q_lds[g][j * 8 + i] * kv[i];
-          }
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) s_lds[g][threadIdx.x] = s[g];
-    }
-    __syncthreads();
-
-    // --- Phase B: online softmax per head --------------------------------
-    for (int g = wid; g < G; g += nwaves) {
-      float m_chunk = -INFINITY;
-      for (int i = lane; i < chunk_n; i += WAVE)
-        m_chunk = fmaxf(m_chunk, s_lds[g][i]);
-      m_chunk = wave_reduce_max(m_chunk);
-      const float m_old = head_m[g];
-      const float m_new = fmaxf(m_old, m_chunk);
-      const float corr = (m_old == -INFINITY) ? 0.f : __expf(m_old - m_new);
-      float l_add = 0.f;
-      for (int i = lane; i < chunk_n; i += WAVE) {
-        const float p = __expf(s_lds[g][i] - m_new);
-        s_lds[g][i] = p;
-        l_add += p;
-      }
-      l_add = wave_reduce_sum(l_add);
-      if (lane == 0) {
-        head_l[g] = head_l[g] * corr + l_add;
-        head_m[g] = m_new;
-        head_corr[g] = corr;
-      }
-    }
-    __syncthreads();
-
-    // --- Phase C: V accumulation (16B lane loads, 4-pass batches) --------
-    {
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[g][i] *= head_corr[g];
-      const int npass = (chunk_n - cpar + C_PAR - 1) / C_PAR;  // my tokens
-      auto vrow_off = [&](int tok) {
-        const int64_t blk = btable[tok / block_size];
-        return (((blk * Hkv + hkv) * (int64_t)block_size +
-                 tok % block_size)) * DHEAD + d8;
-      };
-      auto load_v = [&](int64_t off, float v[8]) {
-        if constexpr (KV8) {
-          const u8x8 raw = *reinterpret_cast<const u8x8*>(
-              (const uint8_t*)v_cache + off);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] = fp8_to_f32(raw[i]);
-        } else {
-          const u16x8 raw = *reinterpret_cast<const u16x8*>(v_cache + off);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] = bf16_to_f32(raw[i]);
-        }
-      };
-      int ps = 0;
-      if constexpr (!KV8) {
-        // raw-staged batches: VPS x 16B loads issue back-to-back (pure,
-        // no dependent converts between them); conversion + FMA consume
-        // them in order while later loads are still in flight
-        for (; ps + VPS <= npass; ps += VPS) {
-          u16x8 vraw[VPS];
-#pragma unroll
-          for (int u = 0; u < VPS; ++u)
-            vraw[u] = *reinterpret_cast<const u16x8*>(
-                v_cache + vrow_off(base + (ps + u) * C_PAR + cpar));
-#pragma unroll
-          for (int u = 0; u < VPS; ++u) {
-            const int tok_i = (ps + u) * C_PAR + cpar;
-            float v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = bf16_to_f32(vraw[u][i]);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const float pv = s_lds[g][tok_i];
-#pragma unroll
-              for (int i = 0; i < 8; ++i) acc[g][i] += pv * v[i];
-            }
-          }
-        }
-      } else {
-        for (; ps + 4 <= npass; ps += 4) {
-          int64_t voff[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            voff[u] = vrow_off(base + (ps + u) * C_PAR + cpar);
-          float v4[4][8];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) load_v(voff[u], v4[u]);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int tok_i = (ps + u) * C_PAR + cpar;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const float pv = s_lds[g][tok_i];
-#pragma unroll
-              for (int i = 0; i < 8; ++i) acc[g][i] += pv * v4[u][i];
-            }
-          }
-        }
-      }
-      for (; ps < npass; ++ps) {
-        const int tok_i = ps * C_PAR + cpar;
-        float v[8];
-        load_v(vrow_off(base + tok_i), v);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float pv = s_lds[g][tok_i];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[g][i] += pv * v[i];
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  // Combine the C_PAR token parities via LDS, then write out.
-  __shared__ float comb[G * DHEAD];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (cpar == 0) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) comb[g * DHEAD + d8 + i] = acc[g][i];
     }
   }
+}
+
+// Pieces of a sequence into one: a workgroup has a query head, each of its
+// D / 4 lanes four dimensions of every eighth (D = 64: sixteenth) piece.
+template <int D>
+__global__ __launch_bounds__(NT) void paged_merge_kernel(Rows m, int Hq) {
+  constexpr int LANES = D / 4, ROWS = NT / LANES;
+  __shared__ f32x4 os[ROWS][LANES];
+  __shared__ float ls[ROWS];
+  const int seq = blockIdx.x, tid = threadIdx.x;
+  int u = 0;
+  for (int b = tid & (WAVE - 1); b < m.B; b += WAVE) u += units_of(m, b);
+  const int parts = pieces_of(m, units_of(m, seq), piece_for(m, u));
+  if (parts == 1) return;
+  const int64_t row = (int64_t)seq * Hq + blockIdx.y;
+  const float2* ml = (const float2*)m.ml + row * m.max_parts;
+  const float* part = m.part + row * m.max_parts * D + tid % LANES * 4;
+  float top = NEG;
+  for (int p = tid & (WAVE - 1); p < parts; p += WAVE)
+    top = fmaxf(top, ml[p].x);
+  top = wave_reduce_max(top);
+  f32x4 o = {0, 0, 0, 0};
+  float sum = 0.f;
+#pragma unroll 4
+  for (int p = tid / LANES; p < parts; p += ROWS) {
+    const float2 v = ml[p];
+    const f32x4 x = *reinterpret_cast<const f32x4*>(part + (int64_t)p * D);
+    const float f = __builtin_amdgcn_exp2f(v.x - top);
+    sum += f * v.y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] += f * x[i];
+  }
+  os[tid / LANES][tid % LANES] = o;
+  if (tid % LANES == 0) ls[tid / LANES] = sum;
   __syncthreads();
-  for (int p = 1; p < C_PAR; ++p) {
-    if (cpar == p) {
+  if (tid >= D) return;
+  float s = 0.f, r = 0.f;
 #pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          comb[g * DHEAD + d8 + i] += acc[g][i];
-    }
-    __syncthreads();
+  for (int i = 0; i < ROWS; ++i) {
+    s += ls[i];
+    r += os[i][tid / 4][tid % 4];
   }
-  if (cpar == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int hq = hkv * G + g;
-      if (nparts == 1) {
-        const float inv_l = 1.f / fmaxf(head_l[g], 1e-20f);
-        float o[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          o[i] = comb[g * DHEAD + d8 + i] * inv_l;
-        store_bf16x8(out + ((int64_t)seq * Hq + hq) * DHEAD + d8, o);
-      } else {
-        float* tp =
-            tmp_out + (((int64_t)seq * Hq + hq) * max_parts + part) * DHEAD;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) tp[d8 + i] = comb[g * DHEAD + d8 + i];
-        if (d8 == 0) {
-          float* ml =
-              tmp_ml + (((int64_t)seq * Hq + hq) * max_parts + part) * 2;
-          ml[0] = head_m[g];
-          ml[1] = head_l[g];
-        }
-      }
-    }
-  }
+  m.out[row * D + tid] = f32_to_bf16(r / fmaxf(s, 1e-20f));
 }
 
-// Reduce partials: out[seq, hq, :] = sum_p w_p * tmp_out[p] / L
-__global__ __launch_bounds__(128) void paged_attn_reduce_kernel(
-    uint16_t* __restrict__ out, const float* __restrict__ tmp_out,
-    const float* __restrict__ tmp_ml, const int* __restrict__ seq_lens,
-    int Hq, int D, int partition_size, int max_parts) {
-  const int seq = blockIdx.x;
-  const int hq = blockIdx.y;
-  const int nparts =
-      min(max_parts, (seq_lens[seq] + partition_size - 1) / partition_size);
-  const float* ml = tmp_ml + ((int64_t)seq * Hq + hq) * max_parts * 2;
-
-  __shared__ float w[512];
-  __shared__ float l_sh;
-  if (threadIdx.x == 0) {
-    float M = -INFINITY;
-    for (int p = 0; p < nparts; ++p) M = fmaxf(M, ml[p * 2]);
-    float L = 0.f;
-    for (int p = 0; p < nparts; ++p) {
-      const float e = (ml[p * 2] == -INFINITY) ? 0.f : __expf(ml[p * 2] - M);
-      w[p] = e;
-      L += e * ml[p * 2 + 1];
-    }
-    l_sh = fmaxf(L, 1e-20f);
-  }
-  __syncthreads();
-  const float* tp = tmp_out + ((int64_t)seq * Hq + hq) * max_parts * D;
-  for (int d = threadIdx.x; d < D; d += blockDim.x) {
-    float o = 0.f;
-    for (int p = 0; p < nparts; ++p) {
-      // skip dead partitions explicitly: their tmp_out is uninitialized
-      // and 0 * NaN would poison the sum (windowed-out partitions)
-      if (w[p] != 0.f) o += w[p] * tp[p * D + d];
-    }
-    out[((int64_t)seq * Hq + hq) * D + d] = f32_to_bf16(o / l_sh);
-  }
-}
-
-static bool use_mfma_a() {
-  static int v = -1;
-  if (v < 0) {
-    const char* e = getenv("HELIX_DECODE_MFMA");
-    v = (e != nullptr && e[0] == '1') ? 1 : 0;
-  }
-  return v == 1;
-}
-
-static int env_int(const char* name, int dflt) {
-  const char* e = getenv(name);
-  return e ? atoi(e) : dflt;
-}
-// A/B knobs for the round-2 decode pipeline (defaults = measured best)
-static int decode_vps() {
-  static int v = -1;
-  if (v < 0) v = env_int("HELIX_DECODE_VPS", 4);
-  return v;
-}
-static int decode_occ() {
-  static int v = -1;
-  if (v < 0) v = env_int("HELIX_DECODE_OCC", 0);
-  return v;
-}
-static int decode_kpre() {
-  static int v = -1;
-  if (v < 0) v = env_int("HELIX_DECODE_KPRE", 1);
-  return v;
-}
-
-template <int DHEAD, int G>
-void launch_decode(uint16_t* out, float* tmp_out, float* tmp_ml,
-                   const uint16_t* q, const uint16_t* kc, const uint16_t* vc,
-                   const int* bt, const int* lens, float scale, int B,
-                   int Hkv, int block_size, int max_blocks, int eff_part,
-                   int nparts, int max_parts, int window, bool kv8,
-                   hipStream_t stream) {
-#define LAUNCH_PD(MF, K8, VPS, OCC, KP)                                      \
-  hipLaunchKernelGGL(                                                        \
-      (paged_attn_decode_kernel<DHEAD, G, MF, K8, VPS, OCC, KP>),            \
-      dim3(B, Hkv, nparts), dim3(NTHREADS), 0, stream, out,                  \
-      tmp_out, tmp_ml, q, kc, vc, bt, lens, scale, Hkv,                      \
-      block_size, max_blocks, eff_part, max_parts, window)
-  if (kv8) {
-    if (decode_kpre()) LAUNCH_PD(false, true, 4, 2, true);
-    else               LAUNCH_PD(false, true, 4, 0, false);
-  } else if (use_mfma_a()) {
-    LAUNCH_PD(true, false, 4, 0, false);
+template <int D, int G>
+void launch(const uint16_t* q, const void* kc, const void* vc, const Rows& m,
+            bool f8, dim3 grid, hipStream_t stream) {
+#define HELIX_PD(F8, P8)                                                     \
+  hipLaunchKernelGGL((paged_rows_kernel<D, G, F8, P8>), grid, dim3(NT), 0,   \
+                     stream, q, kc, vc, m)
+  if (m.shift >= 3) {
+    if (f8) HELIX_PD(true, true);
+    else HELIX_PD(false, true);
   } else {
-    const int vps = decode_vps(), occ = decode_occ();
-    if (decode_kpre()) {
-      // measured defaults (profiles/r02_decode_kpre.md): K-prefetch +
-      // waves/EU floor 2 everywhere (+5.4% e2e at B=512). When the
-      // grid underfills the chip (< 2048 workgroups on 256 CUs x 4
-      // SIMDs), per-wave pipelining has to replace occupancy-based
-      // latency hiding: the 8-deep V staging wins those shapes
-      // (4.25-4.29 vs 3.6-3.7 TB/s at B<=64 / L>=2048) but loses the
-      // full-grid B=512 headline (27.5k vs 28.1k tok/s), so it is
-      // grid-gated, not global. HELIX_DECODE_VPS / _OCC override.
-      const bool vps_forced = getenv("HELIX_DECODE_VPS") != nullptr;
-      const bool small_grid = B * Hkv * nparts < 2048;
-      const bool deep = vps_forced ? (vps >= 8) : small_grid;
-      if (deep)                      LAUNCH_PD(false, false, 8, 2, true);
-      else if (occ == 0 || occ == 2) LAUNCH_PD(false, false, 4, 2, true);
-      else                           LAUNCH_PD(false, false, 4, 0, true);
-    }
-    else if (occ == 2)        LAUNCH_PD(false, false, 4, 2, false);
-    else if (vps >= 8 && occ >= 4) LAUNCH_PD(false, false, 8, 4, false);
-    else if (vps >= 8)        LAUNCH_PD(false, false, 8, 0, false);
-    else if (occ >= 4)        LAUNCH_PD(false, false, 4, 4, false);
-    else                      LAUNCH_PD(false, false, 4, 0, false);
+    if (f8) HELIX_PD(true, false);
+    else HELIX_PD(false, false);
   }
-#undef LAUNCH_PD
+#undef HELIX_PD
 }
 
 }  // namespace
@@ -582,45 +507,45 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   const int Hq = q.size(1);
   const int D = q.size(2);
   const int Hkv = k_cache.size(1);
-  const int block_size = k_cache.size(2);
-  const int max_blocks = block_tables.size(1);
-  const int max_parts = tmp_out.size(2);
   const int G = Hq / Hkv;
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
-  TORCH_CHECK(G <= MAX_G && Hq % Hkv == 0);
+  TORCH_CHECK(G <= 8 && Hq % Hkv == 0);
   TORCH_CHECK(G == 1 || G == 2 || G == 4 || G == 8, "G must be 1/2/4/8");
   TORCH_CHECK(block_tables.scalar_type() == torch::kInt32);
   TORCH_CHECK(seq_lens.scalar_type() == torch::kInt32);
+  if (B == 0) return;
 
-  const int max_len = (int)max_len_hint;
-  const int max_useful = cdiv(max_len, PART_QUANT);
-  // split-K sizing target: enough workgroups to fill 256 CUs. 1024 was
-  // round-1's tuning; HELIX_DECODE_TARGET_WGS re-tunes it for the
-  // round-2 pipeline on underfilled (small-B, long-L) shapes.
-  static int target_wgs = [] {
-    const char* e = getenv("HELIX_DECODE_TARGET_WGS");
-    return e ? atoi(e) : 1024;
-  }();
-  int nparts = std::max(1, target_wgs / std::max(1, B * Hkv));
-  nparts = std::min({nparts, max_useful, max_parts});
-  int eff_part = cdiv(cdiv(max_len, nparts), PART_QUANT) * PART_QUANT;
-  nparts = cdiv(max_len, eff_part);
+  Rows m{};
+  m.bt = block_tables.data_ptr<int>();
+  m.lens = seq_lens.data_ptr<int>();
+  m.out = (uint16_t*)out.data_ptr();
+  m.part = tmp_out.data_ptr<float>();
+  m.ml = tmp_ml.data_ptr<float>();
+  m.B = B;
+  m.Hkv = Hkv;
+  m.bs = k_cache.size(2);
+  m.shift = (m.bs & (m.bs - 1)) == 0 ? __builtin_ctz(m.bs) : -1;
+  m.max_blocks = block_tables.size(1);
+  m.max_parts = tmp_out.size(2);
+  m.window = (int)window;
+  m.limit = cdiv((int)max_len_hint, UNIT) * UNIT;
+  m.mul = (float)scale * LOG2E;
+  // Nothing to cut where a row is at most a unit long, nor where the rows
+  // alone fill the chip twice and none can be long: 512 rows of 513..640 take
+  // 226 us without and 231 with cuts, most of it the merge launch.
+  const int most = cdiv((int)(window > 0 ? std::min(max_len_hint, window + KT)
+                                         : max_len_hint), UNIT);
+  m.split = m.max_parts > 1 && most > 1 &&
+            !(B * Hkv >= 2 * TARGET && most <= 8);
+  // a workgroup without a piece costs its search, so no more than can be
+  const dim3 grid(m.split ? std::min(B * most, B + TARGET / Hkv + 1) : B,
+                  Hkv);
 
   auto stream = at::hip::getCurrentHIPStream();
-  auto* o = (uint16_t*)out.data_ptr();
-  auto* to = tmp_out.data_ptr<float>();
-  auto* tm = tmp_ml.data_ptr<float>();
-  auto* qp = (const uint16_t*)q.data_ptr();
-  auto* kp = (const uint16_t*)k_cache.data_ptr();
-  auto* vp = (const uint16_t*)v_cache.data_ptr();
-  auto* bp = block_tables.data_ptr<int>();
-  auto* lp = seq_lens.data_ptr<int>();
-
-  const bool kv8 = k_cache.scalar_type() == torch::kUInt8;
+  const bool f8 = k_cache.scalar_type() == torch::kUInt8;
 #define DISPATCH(DH, GG)                                                     \
-  launch_decode<DH, GG>(o, to, tm, qp, kp, vp, bp, lp, (float)scale, B,     \
-                        Hkv, block_size, max_blocks, eff_part, nparts,      \
-                        max_parts, (int)window, kv8, stream)
+  launch<DH, GG>((const uint16_t*)q.data_ptr(), k_cache.data_ptr(),          \
+                 v_cache.data_ptr(), m, f8, grid, stream)
   if (D == 128) {
     if (G == 1) DISPATCH(128, 1);
     else if (G == 2) DISPATCH(128, 2);
@@ -633,11 +558,11 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
     else DISPATCH(64, 8);
   }
 #undef DISPATCH
-
-  if (nparts > 1) {
-    hipLaunchKernelGGL(paged_attn_reduce_kernel, dim3(B, Hq), dim3(128), 0,
-                       stream, o, to, tm, lp, Hq, D, eff_part, max_parts);
-    // note: dead (windowed-out) partitions wrote ml = -inf and are
-    // skipped by the reduce weighting
-  }
+  if (!m.split) return;
+  if (D == 128)
+    hipLaunchKernelGGL(paged_merge_kernel<128>, dim3(B, Hq), dim3(NT), 0,
+                       stream, m, Hq);
+  else
+    hipLaunchKernelGGL(paged_merge_kernel<64>, dim3(B, Hq), dim3(NT), 0,
+                       stream, m, Hq);
 }

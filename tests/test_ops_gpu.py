@@ -254,6 +254,47 @@ def test_paged_attn_decode_sliding_window(window, lens):
     assert_close_bf16(got, want, atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("hq,hkv,d,bs,fp8,window,lens", [
+    (32, 8, 128, 16, False, 0, [1, 31, 32, 33, 127, 128, 129, 1500]),
+    (8, 4, 128, 16, True, 0, [1, 40, 1029]),
+    (16, 2, 64, 32, False, 100, [99, 100, 101, 612]),
+    (4, 4, 64, 24, True, 0, [7, 8, 500]),
+    (8, 2, 128, 4, False, 77, [3, 300]),
+    (4, 1, 64, 8, False, 0, [1 + 37 * i % 90 for i in range(70)]),
+    (32, 8, 128, 16, False, 0, [130] * 256),          # no cuts, no merge
+])
+def test_paged_attn_decode_edges(hq, hkv, d, bs, fp8, window, lens):
+    """Ends of tiles, units and pages, pages of any size, many and few
+    sequences; what lies behind a sequence's end is not a number."""
+    torch.manual_seed(21)
+    B = len(lens)
+    need = [-(-n // bs) for n in lens]
+    q = torch.randn(B, hq, d, dtype=torch.bfloat16)
+    kc = torch.randn(sum(need), hkv, bs, d, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    order = torch.randperm(sum(need), dtype=torch.int32)
+    bt = torch.zeros(B, max(need), dtype=torch.int32)
+    for b, pages in enumerate(order.split(need)):
+        bt[b, :need[b]] = pages
+    seq_lens = torch.tensor(lens, dtype=torch.int32)
+    if fp8:
+        kc, vc = ops.kv_fp8_quant(kc), ops.kv_fp8_quant(vc)
+    want = ref.paged_attn_decode(
+        q.float(), *((ops.kv_fp8_dequant(t) if fp8 else t).float()
+                     for t in (kc, vc)), bt, seq_lens, d ** -0.5, window)
+    nan = 0x7f if fp8 else float("nan")
+    for b, n in enumerate(lens):
+        if n % bs:
+            for t in (kc, vc):
+                t[bt[b, need[b] - 1].long(), :, n % bs:] = nan
+    got = ops.paged_attn_decode(q.to(DEV), kc.to(DEV), vc.to(DEV),
+                                bt.to(DEV), seq_lens.to(DEV), d ** -0.5,
+                                window=window)
+    # rounded to bf16 (2^-9, doubled); sums of 32 bits over <= 1500 values
+    torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
+                               atol=5e-5)
+
+
 @pytest.mark.parametrize("qlens,klens", [([32], [160]), ([7, 64], [7, 200]),
                                          ([128], [128])])
 def test_attn_prefill_cached_prefix(qlens, klens):
