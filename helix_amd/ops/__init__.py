@@ -180,7 +180,7 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if cu_seqlens_k is None:
         cu_seqlens_k = cu_seqlens
     if q.is_cuda:
-        out = torch.empty_like(q)
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _native().attn_prefill(out, q, k, v, cu_seqlens, cu_seqlens_k,
                                max_seqlen, scale, causal, window)
         return out

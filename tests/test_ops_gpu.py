@@ -227,6 +227,48 @@ def test_attn_prefill_sliding_window(window, lens):
     assert_close_bf16(got, want, atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("hq,hkv,d,causal,window,qlens,before", [
+    (4, 2, 128, True, 0, [1, 31, 32, 33, 63, 64, 65, 127, 128, 129], 0),
+    (4, 1, 64, True, 0, [1, 128, 200], 0),
+    (4, 2, 128, True, 0, [5, 130], 191),
+    (4, 2, 128, True, 60, [1, 129, 300], 0),
+    (2, 2, 64, True, 1, [70], 60),
+    (2, 1, 128, True, 128, [130], 63),
+    (3, 3, 64, False, 0, [1, 63, 64, 65, 300], 0),
+    (2, 1, 128, False, 0, [40, 129], 0),
+])
+@pytest.mark.parametrize("rows", ["dense", "slices"])
+def test_attn_prefill_edges(hq, hkv, d, causal, window, qlens, before, rows):
+    """Ends of query and key tiles, windows that start anywhere, slices of a
+    fused projection, a negative scale."""
+    torch.manual_seed(22)
+    scale = d ** -0.5 if rows == "dense" else -(d ** -0.5)
+    klens = [n + before for n in qlens]
+    Tk = sum(klens)
+    z = torch.randn(Tk, (hq + 2 * hkv) * d, dtype=torch.bfloat16)
+    q, k, v = (t.view(Tk, -1, d) for t in
+               z.split([hq * d, hkv * d, hkv * d], -1))
+    q = q[:sum(qlens)]
+    if rows == "dense":
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    cu = [torch.tensor([0] + n, dtype=torch.int32).cumsum(0).int()
+          for n in (qlens, klens)]
+    want = ref.attn_prefill(q.float(), k.float(), v.float(), cu[0],
+                            max(qlens), scale, causal, window, cu[1])
+    z = z.to(DEV)
+    dq, dk, dv = (t.view(Tk, -1, d) for t in
+                  z.split([hq * d, hkv * d, hkv * d], -1))
+    dq = dq[:sum(qlens)]
+    if rows == "dense":
+        dq, dk, dv = dq.contiguous(), dk.contiguous(), dv.contiguous()
+    got = ops.attn_prefill(dq, dk, dv, cu[0].to(DEV), max(qlens), scale,
+                           causal, window, cu[1].to(DEV))
+    # weights rounded to bf16 (2^-9) times values of at most 4.6, and the
+    # result's own rounding
+    torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
+                               atol=4.6 * 2 ** -9)
+
+
 @pytest.mark.parametrize("window,lens", [(64, [200]), (256, [100, 700]),
                                          (512, [2048])])
 def test_paged_attn_decode_sliding_window(window, lens):
