@@ -133,12 +133,27 @@ PRESETS = {
 
 
 class HLinear(nn.Linear):
-    """nn.Linear routed through ops.linear: decode-shaped (skinny-M)
-    GEMMs run the owned split-K MFMA kernel, prefill-shaped ones stay on
-    hipBLASLt (SURVEY §2.8 'Q/K/V + O projections, MLP GEMMs')."""
+    """nn.Linear routed through ops.linear: a few rows run the owned MFMA
+    kernel, prefill-shaped ones stay on hipBLASLt.
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.linear(x, self.weight, self.bias)
+    form: "rows" -> [T, N]; "sums" -> what ops.linear_sums gives, for a
+    reader that adds it up; "glu" -> silu(first half) * second half."""
+
+    def forward(self, x: torch.Tensor, form: str = "rows") -> torch.Tensor:
+        if self.bias is None and form == "sums":
+            return ops.linear_sums(x, self.weight)
+        if self.bias is None and form == "glu":
+            return ops.linear_silu_mul(x, self.weight)
+        out = ops.linear(x, self.weight, self.bias)
+        return ops.silu_and_mul(out) if form == "glu" else out
+
+
+def _project(proj: nn.Module, x: torch.Tensor, form: str) -> torch.Tensor:
+    """proj(x) in that form; other kinds of projections know only rows."""
+    if isinstance(proj, HLinear):
+        return proj(x, form)
+    out = proj(x)
+    return ops.silu_and_mul(out) if form == "glu" else out
 
 
 class Attention(nn.Module):
@@ -157,9 +172,9 @@ class Attention(nn.Module):
         self.o_proj = HLinear(q, h, bias=False)
 
     def forward(self, x: torch.Tensor, cos_sin: torch.Tensor, kv_cache,
-                meta) -> torch.Tensor:
+                meta, form: str = "rows") -> torch.Tensor:
         T = x.shape[0]
-        qkv = self.qkv_proj(x)
+        qkv = _project(self.qkv_proj, x, "sums")
         # fused strided split + rope + paged-cache write (one kernel, no
         # .contiguous() copies); compact K/V emitted only when the
         # fresh-prefill attention path consumes them directly
@@ -182,11 +197,11 @@ class Attention(nn.Module):
             o = self._attend_prefill(q, k, v, kv_cache, meta)
         else:
             o = self._attend_decode(q, kv_cache, meta)
-        out = self.o_proj(o.view(T, -1))
+        o = o.view(T, -1)
         if self.tp_size > 1:
             from helix_amd import parallel
-            out = parallel.tp_all_reduce(out)
-        return out
+            return parallel.tp_all_reduce(self.o_proj(o))
+        return _project(self.o_proj, o, form)
 
     def _attend_prefill(self, q, k, v, kv_cache, meta):
         if meta.cu_seqlens_k is None:
@@ -223,12 +238,12 @@ class MLP(nn.Module):
         self.gate_up_proj = HLinear(cfg.hidden_size, 2 * i, bias=False)
         self.down_proj = HLinear(i, cfg.hidden_size, bias=False)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        out = self.down_proj(ops.silu_and_mul(self.gate_up_proj(x)))
+    def forward(self, x: torch.Tensor, form: str = "rows") -> torch.Tensor:
+        h = _project(self.gate_up_proj, x, "glu")
         if self.tp_size > 1:
             from helix_amd import parallel
-            out = parallel.tp_all_reduce(out)
-        return out
+            return parallel.tp_all_reduce(self.down_proj(h))
+        return _project(self.down_proj, h, form)
 
 
 class DecoderLayer(nn.Module):
@@ -240,17 +255,19 @@ class DecoderLayer(nn.Module):
         self.mlp = MLP(cfg, tp_size)
         self.eps = cfg.rms_norm_eps
 
-    def forward(self, x, residual, cos_sin, kv_cache, meta):
+    def forward(self, x, residual, cos_sin, kv_cache, meta,
+                form: str = "rows"):
+        """form "sums": the result's stretches, for the next norm."""
         if residual is None:
             residual = x.clone()
             h = ops.rms_norm(x, self.input_norm_w, self.eps)
         else:
             h, residual = ops.fused_add_rms_norm(x, residual,
                                                  self.input_norm_w, self.eps)
-        h = self.attn(h, cos_sin, kv_cache, meta)
+        h = self.attn(h, cos_sin, kv_cache, meta, "sums")
         h, residual = ops.fused_add_rms_norm(h, residual, self.post_norm_w,
                                              self.eps)
-        h = self.mlp(h)
+        h = self.mlp(h, form)
         return h, residual
 
 
@@ -290,9 +307,9 @@ class LlamaForCausalLM(nn.Module):
         residual = None
         for i, layer in enumerate(self.layers):
             cache = kv_caches[i] if kv_caches is not None else None
-            x, residual = layer(x, residual, self.cos_sin, cache, meta)
-        x = (x.float() + residual.float()).to(x.dtype)
-        return ops.rms_norm(x, self.final_norm_w, self.cfg.rms_norm_eps)
+            x, residual = layer(x, residual, self.cos_sin, cache, meta, "sums")
+        return ops.fused_add_rms_norm(x, residual, self.final_norm_w,
+                                      self.cfg.rms_norm_eps)[0]
 
     @torch.inference_mode()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:

@@ -58,7 +58,13 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 
 def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor,
                        w: torch.Tensor, eps: float):
-    """In-place on GPU: x <- norm(x+res), residual <- x+res. Returns both."""
+    """In-place on GPU: x <- norm(x+res), residual <- x+res. Returns both.
+    x may be the stretches of a product (linear_sums), which stay as they
+    are."""
+    if x.dim() == 3:
+        h = torch.empty_like(residual)
+        _native().add_sums_rms_norm(h, x, residual, w, eps)
+        return h, residual
     if x.is_cuda:
         _native().fused_add_rms_norm(x, residual, w, eps)
         return x, residual
@@ -103,18 +109,20 @@ def rope_qkv_cache(positions: torch.Tensor, qkv: torch.Tensor,
                    cos_sin: torch.Tensor, num_q: int, num_kv: int,
                    head_dim: int, kv_cache=None, slot_mapping=None,
                    want_kv: bool = False):
-    """Fused QKV epilogue: strided split + rope + paged-cache write.
+    """Fused QKV epilogue: strided split + rope + paged-cache write. qkv is
+    [T, C], or the stretches of that product (linear_sums).
 
     Returns (q [T, num_q, head_dim], k, v) — k/v are None unless
     want_kv (fresh-prefill path needs compact K/V for attn_prefill).
     """
-    T = qkv.shape[0]
+    T = qkv.shape[-2]
     if qkv.is_cuda:
-        q_out = torch.empty(T, num_q * head_dim, dtype=qkv.dtype,
+        dtype = torch.bfloat16
+        q_out = torch.empty(T, num_q * head_dim, dtype=dtype,
                             device=qkv.device)
         k_out = v_out = None
         if want_kv:
-            k_out = torch.empty(T, num_kv * head_dim, dtype=qkv.dtype,
+            k_out = torch.empty(T, num_kv * head_dim, dtype=dtype,
                                 device=qkv.device)
             v_out = torch.empty_like(k_out)
         kc = vc = None
@@ -335,16 +343,66 @@ def gemm_skinny_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
     return out
 
 
+ROWS_MAX_M = 64                   # of gemm_rows.hip
+ROWS_CHUNK = 256
+
+
+def _rows_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the kernel for a few rows takes x @ w^T. It knows nothing of
+    gradients, so it only runs where there are none to be had."""
+    return (x.is_cuda and torch.is_inference_mode_enabled()
+            and x.dim() == 2 and 0 < x.shape[0] <= ROWS_MAX_M
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and x.shape[1] > 0 and x.shape[1] % ROWS_CHUNK == 0
+            and w.shape[0] > 0 and w.shape[0] % 8 == 0
+            and x.is_contiguous() and w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
-    """Projection dispatch: skinny-M decode GEMMs on the owned kernel,
-    everything else (prefill-sized M, CPU, odd dims) via torch/hipBLASLt."""
+    """Projection dispatch: a few rows on the owned kernel, everything else
+    (prefill-sized M, CPU, odd dims) via torch/hipBLASLt.
+
+    The line is where both were measured equal: up to 16 rows the owned kernel
+    is faster (28672 x 4096: 45 against 65 us) but for vocabularies (128256 x
+    4096: 191 against 189); from 17 to 64 rows it stays so where the inner
+    dimension is the longer one (4096 x 14336: 30 against 34 and 35 against
+    42), elsewhere adding up the stretches costs what it gains."""
     if (_SKINNY_ENABLED and x.is_cuda and x.dtype == torch.bfloat16
             and x.dim() == 2
             and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= _SKINNY_MAX_M
             and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0
             and x.is_contiguous() and w.is_contiguous()):
         return gemm_skinny_bf16(x, w, bias)
+    if _rows_fit(x, w) and w.shape[0] <= 65536 and \
+            (x.shape[0] <= 16 or x.shape[1] >= 2 * w.shape[0]):
+        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
+                          device=x.device)
+        _native().gemm_rows(out, x, w, bias)
+        return out
     return torch.nn.functional.linear(x, w, bias)
+
+
+def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w^T for a reader that adds up stretches of the inner dimension
+    (fused_add_rms_norm, rope_qkv_cache): [stretches, M, N] fp32 for a few
+    rows, else [M, N] in x's type. Wide matrices fill the chip without
+    stretches, and 64 rows of 16384 sums are more bytes than they save."""
+    if _rows_fit(x, w) and w.shape[0] <= 8192:
+        return _native().gemm_rows_sums(x, w)
+    return linear(x, w)
+
+
+def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x @ gate^T) * (x @ up^T), w = [gate; up]. A few rows: one launch,
+    whose halves stay in registers (55 us at 64 rows of 2 x 14336 x 4096,
+    product and activation apart 57; 45 against 68 at one)."""
+    if _rows_fit(x, w):
+        out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                          device=x.device)
+        _native().gemm_rows_glu(out, x, w)
+        return out
+    return silu_and_mul(linear(x, w))
 
 
 def mfma_probe(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:

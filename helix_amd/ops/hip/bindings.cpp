@@ -4,6 +4,8 @@
 void rms_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w, double eps);
 void fused_add_rms_norm(torch::Tensor x, torch::Tensor residual,
                         torch::Tensor w, double eps);
+void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
+                       torch::Tensor residual, torch::Tensor w, double eps);
 void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                 torch::Tensor b, double eps);
 void rotary_embedding(torch::Tensor positions, torch::Tensor q,
@@ -49,6 +51,10 @@ void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                       c10::optional<torch::Tensor> bias,
                       c10::optional<torch::Tensor> scratch, int64_t split_k,
                       int64_t act, int64_t swizzle);
+void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias);
+torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w);
+void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w);
 void gemm_fp8(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               torch::Tensor x_scale, torch::Tensor w_scale,
               c10::optional<torch::Tensor> bias, int64_t act);
@@ -65,6 +71,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16, CDNA4)");
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "Fused residual-add + RMSNorm (in-place)");
+  m.def("add_sums_rms_norm", &add_sums_rms_norm,
+        "Sum of a product's stretches + residual-add + RMSNorm");
   m.def("layer_norm", &layer_norm, "LayerNorm (bf16)");
   m.def("rotary_embedding", &rotary_embedding,
         "Apply rotary embedding to q,k in-place");
@@ -84,6 +92,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_bf16", &gemm_bf16, "MFMA bf16 GEMM: x @ w^T (+bias, act)");
   m.def("gemm_skinny_bf16", &gemm_skinny_bf16,
         "Skinny-M decode GEMM: split-K + XCD-chunked tile swizzle");
+  m.def("gemm_rows", &gemm_rows, "x @ w^T (+bias) of at most 64 rows");
+  m.def("gemm_rows_sums", &gemm_rows_sums,
+        "x @ w^T of at most 64 rows, stretches of the inner dimension apart");
+  m.def("gemm_rows_glu", &gemm_rows_glu,
+        "silu(x @ gate^T) * (x @ up^T) of at most 64 rows");
   m.def("gemm_fp8", &gemm_fp8,
         "MX-fp8 e4m3 MFMA GEMM with epilogue per-row/col dequant");
   m.def("mfma_probe", &mfma_probe, "16x16x32 MFMA layout probe");

@@ -83,6 +83,57 @@ __global__ void fused_add_rms_norm_kernel(uint16_t* __restrict__ x,
   }
 }
 
+// residual' = sum of x's stretches + residual ; h = rmsnorm(residual') * w
+// x is a product whose inner dimension was cut (fp32 [stretches, T, H]); its
+// sum is taken here, in order, instead of in a launch of its own (2.5 to 3 us)
+// and is not rounded before it meets the residual.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void add_sums_rms_norm_kernel(
+    uint16_t* __restrict__ h, const float* __restrict__ x,
+    uint16_t* __restrict__ residual, const uint16_t* __restrict__ w,
+    float eps, int H, int stretches) {
+  __shared__ float red[BLOCK / WAVE];
+  const int t = blockIdx.x;
+  const int64_t all = (int64_t)gridDim.x * H;
+  const float* xrow = x + (int64_t)t * H;
+  uint16_t* rrow = residual + (int64_t)t * H;
+  uint16_t* hrow = h + (int64_t)t * H;
+
+  float ss = 0.f;
+  const int nvec = H / 8;
+  for (int v = threadIdx.x; v < nvec; v += BLOCK) {
+    float a[8] = {0, 0, 0, 0, 0, 0, 0, 0}, b[8];
+    load_bf16x8(rrow + v * 8, b);
+#pragma unroll 8
+    for (int s = 0; s < stretches; ++s) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(xrow + s * all + v * 8);
+      const f32x4 u = p[0], z = p[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a[i] += u[i];
+        a[4 + i] += z[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      a[i] += b[i];
+      ss += a[i] * a[i];
+    }
+    store_bf16x8(rrow + v * 8, a);  // new residual
+  }
+  ss = block_reduce_sum(ss, red);
+  const float inv = rsqrtf(ss / H + eps);
+
+  for (int v = threadIdx.x; v < nvec; v += BLOCK) {
+    float e[8], ww[8];
+    load_bf16x8(rrow + v * 8, e);
+    load_bf16x8(w + v * 8, ww);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) e[i] = e[i] * inv * ww[i];
+    store_bf16x8(hrow + v * 8, e);
+  }
+}
+
 // LayerNorm (for encoder / bge-class models): out = (x - mu)/sigma * w + b
 template <int BLOCK>
 __global__ void layer_norm_kernel(uint16_t* __restrict__ out,
@@ -151,6 +202,24 @@ void fused_add_rms_norm(torch::Tensor x, torch::Tensor residual,
                      stream, (uint16_t*)x.data_ptr(),
                      (uint16_t*)residual.data_ptr(),
                      (const uint16_t*)w.data_ptr(), (float)eps, H);
+}
+
+void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
+                       torch::Tensor residual, torch::Tensor w, double eps) {
+  TORCH_CHECK(x.dim() == 3 && x.is_contiguous() &&
+              x.scalar_type() == torch::kFloat32 && h.is_contiguous() &&
+              residual.is_contiguous() && residual.dim() == 2 &&
+              residual.size(0) == x.size(1) && residual.size(1) == x.size(2) &&
+              h.sizes() == residual.sizes());
+  const int T = x.size(1);
+  const int H = x.size(2);
+  TORCH_CHECK(H % 8 == 0, "H must be a multiple of 8");
+  auto stream = at::hip::getCurrentHIPStream();
+  hipLaunchKernelGGL((add_sums_rms_norm_kernel<512>), dim3(T), dim3(512), 0,
+                     stream, (uint16_t*)h.data_ptr(), x.data_ptr<float>(),
+                     (uint16_t*)residual.data_ptr(),
+                     (const uint16_t*)w.data_ptr(), (float)eps, H,
+                     (int)x.size(0));
 }
 
 void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,

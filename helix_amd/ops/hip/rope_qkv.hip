@@ -1,14 +1,15 @@
 // Fused QKV epilogue: one pass over the fused qkv projection output.
 //
 // Reads qkv [T, (Hq+2*Hkv)*D] (row stride = the projection's output
-// width, so no .contiguous() splits), applies rotate-half rope to Q and
-// K, writes compact roped Q for the attention kernels, scatters roped K
-// and V straight into the paged cache, and optionally emits compact K/V
-// for the fresh-prefill attention path.
+// width, so no .contiguous() splits) or its stretches (fp32, summed here in
+// order), applies rotate-half rope to Q and K, writes compact roped Q for the
+// attention kernels, scatters roped K and V straight into the paged cache, and
+// optionally emits compact K/V for the fresh-prefill attention path.
 //
-// Replaces 5 kernels (3 split copies + rope + reshape_and_cache) with 1:
-// the split copies alone were ~0.5 ms/step at B=512 (see
-// profiles/r01_decode_profile_v1.md batch-512 window breakdown).
+// Replaces 5 kernels (3 split copies + rope + reshape_and_cache) with 1. A
+// thread has 8 pairs of a head or 8 values, and a token's threads are spread
+// over workgroups of 128: with one workgroup of 256 a token, a pair a thread
+// at a time, a row took 7.8 us and 16k rows 115.
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -17,95 +18,120 @@ using namespace helix;
 
 namespace {
 
-__global__ void rope_qkv_cache_kernel(
-    const int64_t* __restrict__ positions,
-    const uint16_t* __restrict__ qkv, int64_t qkv_stride,
-    uint16_t* __restrict__ q_out,
-    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
-    const int64_t* __restrict__ slot_mapping,
-    uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out,
-    const float* __restrict__ cos_sin,
-    int Hq, int Hkv, int D, int block_size, int kv8) {
-  const int t = blockIdx.x;
-  const int64_t pos = positions[t];
-  const float* cs = cos_sin + pos * D;
-  const int half = D / 2;
-  const uint16_t* src = qkv + (int64_t)t * qkv_stride;
-  const int64_t slot = slot_mapping ? slot_mapping[t] : -1;
-  int64_t cblock = 0;
-  int coff = 0;
-  if (slot >= 0) {
-    cblock = slot / block_size;
-    coff = (int)(slot % block_size);
-  }
+constexpr int NT = 128;
 
-  // --- Q and K rotation pairs (q heads first, then k heads) ---
-  const int qk_pairs = (Hq + Hkv) * half;
-  for (int idx = threadIdx.x; idx < qk_pairs; idx += blockDim.x) {
-    const int h = idx / half;
-    const int d = idx % half;
-    const float c = cs[d];
-    const float sn = cs[half + d];
-    const uint16_t* b = src + h * D;
-    const float x1 = bf16_to_f32(b[d]);
-    const float x2 = bf16_to_f32(b[d + half]);
-    const uint16_t y1 = f32_to_bf16(x1 * c - x2 * sn);
-    const uint16_t y2 = f32_to_bf16(x2 * c + x1 * sn);
-    if (h < Hq) {
-      uint16_t* o = q_out + ((int64_t)t * Hq + h) * D;
-      o[d] = y1;
-      o[d + half] = y2;
-    } else {
-      const int hk = h - Hq;
-      if (k_out != nullptr) {
-        uint16_t* o = k_out + ((int64_t)t * Hkv + hk) * D;
-        o[d] = y1;
-        o[d + half] = y2;
-      }
-      if (slot >= 0) {
-        const int64_t ko =
-            ((cblock * Hkv + hk) * (int64_t)block_size + coff) * D;
-        if (kv8) {           // OCP e4m3 cache (kv_cache_dtype="fp8")
-          uint8_t* o = (uint8_t*)k_cache + ko;
-          o[d] = f32_to_fp8(x1 * c - x2 * sn);
-          o[d + half] = f32_to_fp8(x2 * c + x1 * sn);
-        } else {
-          uint16_t* o = k_cache + ko;
-          o[d] = y1;
-          o[d + half] = y2;
-        }
-      }
-    }
-  }
+struct Epilogue {
+  const int64_t* positions;
+  const int64_t* slots;
+  const void* qkv;
+  int64_t stride, all;         // of a row; of a stretch
+  uint16_t *q, *k, *v;         // compact; k and v may be null
+  void *kc, *vc;
+  const float* cs;
+  int Hq, Hkv, D, bs, stretches;
+};
 
-  // --- V pass-through (vectorized) ---
-  const uint16_t* vsrc = src + (Hq + Hkv) * D;
-  const int nvec = Hkv * D / 8;
-  for (int idx = threadIdx.x; idx < nvec; idx += blockDim.x) {
-    const int h = (idx * 8) / D;
-    const int d = (idx * 8) % D;
-    const u16x8 val = *reinterpret_cast<const u16x8*>(vsrc + idx * 8);
-    if (v_out != nullptr)
-      *reinterpret_cast<u16x8*>(v_out + (int64_t)t * Hkv * D + idx * 8) =
-          val;
-    if (slot >= 0) {
-      const int64_t vo =
-          ((cblock * Hkv + h) * (int64_t)block_size + coff) * D + d;
-      if (kv8) {
-        u8x8 q8;
+// N values of a row at column c.
+template <int N, bool SUMS>
+__device__ __forceinline__ void read(const Epilogue& m, int64_t t, int c,
+                                     float* o) {
+  if constexpr (SUMS) {
+    const float* p = (const float*)m.qkv + t * m.stride + c;
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          q8[e] = f32_to_fp8(bf16_to_f32(val[e]));
-        *reinterpret_cast<u8x8*>((uint8_t*)v_cache + vo) = q8;
+    for (int i = 0; i < N; ++i) o[i] = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < m.stretches; ++s, p += m.all) {
+      if constexpr (N == 8) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(p);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o[i] += a[i];
+          o[4 + i] += b[i];
+        }
       } else {
-        *reinterpret_cast<u16x8*>(v_cache + vo) = val;
+        o[0] += p[0];
       }
     }
+  } else {
+    const uint16_t* p = (const uint16_t*)m.qkv + t * m.stride + c;
+    if constexpr (N == 8) load_bf16x8(p, o);
+    else o[0] = bf16_to_f32(*p);
+  }
+}
+template <int N>
+__device__ __forceinline__ void write(uint16_t* p, const float* v) {
+  if constexpr (N == 8) store_bf16x8(p, v);
+  else *p = f32_to_bf16(*v);
+}
+template <int N, bool F8>
+__device__ __forceinline__ void write_cache(void* c, int64_t at,
+                                            const float* v) {
+  if constexpr (!F8) {
+    write<N>((uint16_t*)c + at, v);
+  } else if constexpr (N == 8) {       // OCP e4m3 cache
+    u8x8 q;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = f32_to_fp8(v[i]);
+    *reinterpret_cast<u8x8*>((uint8_t*)c + at) = q;
+  } else {
+    ((uint8_t*)c)[at] = f32_to_fp8(*v);
+  }
+}
+
+template <int N, bool SUMS, bool F8>
+__global__ __launch_bounds__(NT) void rope_qkv_cache_kernel(Epilogue m) {
+  const int64_t t = blockIdx.x;
+  const int half = m.D / 2, per = half / N;
+  const int turned = (m.Hq + m.Hkv) * per;    // then the values
+  int i = blockIdx.y * NT + threadIdx.x;
+  if (i >= turned + m.Hkv * m.D / N) return;
+  const int64_t slot = m.slots != nullptr ? m.slots[t] : -1;
+  const int64_t page = slot >= 0 ? slot / m.bs : 0;
+  const int off = slot >= 0 ? (int)(slot % m.bs) : 0;
+  auto place = [&](int h) {
+    return ((page * m.Hkv + h) * m.bs + off) * m.D;
+  };
+  if (i >= turned) {
+    i = (i - turned) * N;
+    float v[N];
+    read<N, SUMS>(m, t, (m.Hq + m.Hkv) * m.D + i, v);
+    if (m.v != nullptr) write<N>(m.v + t * m.Hkv * m.D + i, v);
+    if (slot >= 0) write_cache<N, F8>(m.vc, place(i / m.D) + i % m.D, v);
+    return;
+  }
+  const int h = i / per, d = i % per * N;
+  const float* cs = m.cs + m.positions[t] * m.D + d;
+  float x[N], y[N];
+  read<N, SUMS>(m, t, h * m.D + d, x);
+  read<N, SUMS>(m, t, h * m.D + half + d, y);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float a = x[j], b = y[j], c = cs[j], s = cs[half + j];
+    x[j] = a * c - b * s;
+    y[j] = b * c + a * s;
+  }
+  if (h < m.Hq) {
+    uint16_t* o = m.q + (t * m.Hq + h) * m.D + d;
+    write<N>(o, x);
+    write<N>(o + half, y);
+    return;
+  }
+  const int g = h - m.Hq;
+  if (m.k != nullptr) {
+    uint16_t* o = m.k + (t * m.Hkv + g) * m.D + d;
+    write<N>(o, x);
+    write<N>(o + half, y);
+  }
+  if (slot >= 0) {
+    write_cache<N, F8>(m.kc, place(g) + d, x);
+    write_cache<N, F8>(m.kc, place(g) + half + d, y);
   }
 }
 
 }  // namespace
 
+// qkv: [T, C] bf16, or [stretches, T, C] fp32
 void rope_qkv_cache(torch::Tensor positions, torch::Tensor qkv,
                     torch::Tensor q_out,
                     c10::optional<torch::Tensor> k_cache,
@@ -117,32 +143,55 @@ void rope_qkv_cache(torch::Tensor positions, torch::Tensor qkv,
                     int64_t num_kv_heads, int64_t head_dim) {
   const int T = positions.size(0);
   if (T == 0) return;
+  const bool sums = qkv.dim() == 3;
   TORCH_CHECK(positions.scalar_type() == torch::kInt64);
   TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32);
   TORCH_CHECK(qkv.stride(-1) == 1, "qkv innermost must be contiguous");
+  TORCH_CHECK(qkv.scalar_type() ==
+              (sums ? torch::kFloat32 : torch::kBFloat16));
   TORCH_CHECK(head_dim % 8 == 0);
-  int block_size = 1;
-  int kv8 = 0;
-  uint16_t* kc = nullptr;
-  uint16_t* vc = nullptr;
-  const int64_t* slots = nullptr;
+  Epilogue m{};
+  m.positions = positions.data_ptr<int64_t>();
+  m.qkv = qkv.data_ptr();
+  m.stride = qkv.stride(-2);
+  m.all = sums ? qkv.stride(0) : 0;
+  m.stretches = sums ? qkv.size(0) : 1;
+  m.q = (uint16_t*)q_out.data_ptr();
+  m.k = k_out.has_value() ? (uint16_t*)k_out->data_ptr() : nullptr;
+  m.v = v_out.has_value() ? (uint16_t*)v_out->data_ptr() : nullptr;
+  m.cs = cos_sin.data_ptr<float>();
+  m.Hq = num_q_heads;
+  m.Hkv = num_kv_heads;
+  m.D = head_dim;
+  m.bs = 1;
+  bool f8 = false;
   if (k_cache.has_value()) {
-    kv8 = (k_cache->scalar_type() == torch::kUInt8) ? 1 : 0;
+    f8 = k_cache->scalar_type() == torch::kUInt8;
     TORCH_CHECK(v_cache.has_value() && slot_mapping.has_value());
     TORCH_CHECK(slot_mapping->scalar_type() == torch::kInt64);
-    block_size = k_cache->size(2);
-    kc = (uint16_t*)k_cache->data_ptr();
-    vc = (uint16_t*)v_cache->data_ptr();
-    slots = slot_mapping->data_ptr<int64_t>();
+    m.bs = k_cache->size(2);
+    m.kc = k_cache->data_ptr();
+    m.vc = v_cache->data_ptr();
+    m.slots = slot_mapping->data_ptr<int64_t>();
   }
+  // 8 values at a time where halves of a head and rows begin on 16 bytes
+  const bool vec = head_dim % 16 == 0 && m.stride % 8 == 0 &&
+                   (uintptr_t)m.qkv % 16 == 0;
+  const int items = ((m.Hq + m.Hkv) * m.D / 2 + m.Hkv * m.D) / (vec ? 8 : 1);
+  const dim3 grid(T, cdiv(items, NT));
   auto stream = at::hip::getCurrentHIPStream();
-  const int threads = 256;
-  hipLaunchKernelGGL(
-      rope_qkv_cache_kernel, dim3(T), dim3(threads), 0, stream,
-      positions.data_ptr<int64_t>(), (const uint16_t*)qkv.data_ptr(),
-      qkv.stride(0), (uint16_t*)q_out.data_ptr(), kc, vc, slots,
-      k_out.has_value() ? (uint16_t*)k_out->data_ptr() : nullptr,
-      v_out.has_value() ? (uint16_t*)v_out->data_ptr() : nullptr,
-      cos_sin.data_ptr<float>(), (int)num_q_heads, (int)num_kv_heads,
-      (int)head_dim, block_size, kv8);
+#define LAUNCH(N, S, F)                                                      \
+  hipLaunchKernelGGL((rope_qkv_cache_kernel<N, S, F>), grid, dim3(NT), 0,    \
+                     stream, m)
+#define KIND(N)                                                              \
+  do {                                                                       \
+    if (sums) {                                                              \
+      if (f8) LAUNCH(N, true, true); else LAUNCH(N, true, false);            \
+    } else {                                                                 \
+      if (f8) LAUNCH(N, false, true); else LAUNCH(N, false, false);          \
+    }                                                                        \
+  } while (0)
+  if (vec) KIND(8); else KIND(1);
+#undef KIND
+#undef LAUNCH
 }

@@ -558,6 +558,68 @@ def test_gemm_skinny_bf16(m, n, k):
     assert_close_bf16(got2, want2, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(8, 256), (72, 512), (4104, 2304),
+                                 (256, 4096)])
+def test_gemm_rows(m, n, k):
+    """Few rows: plain, with bias, as stretches, gated; columns that do not
+    fill a workgroup, chunks that do not fill a stretch."""
+    torch.manual_seed(23)
+    x = torch.randn(m, k, dtype=torch.bfloat16)
+    w = torch.randn(n, k, dtype=torch.bfloat16) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16)
+    dx, dw, db = x.to(DEV), w.to(DEV), b.to(DEV)
+    want = x.float() @ w.float().t()
+    # fp32 sums of k products, then the rounding to bf16
+    tol = dict(rtol=2 ** -8, atol=2e-5)
+    with torch.inference_mode():
+        got = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+        ops._native().gemm_rows(got, dx, dw, db)
+        torch.testing.assert_close(got.float().cpu(), want + b.float(), **tol)
+        sums = ops.linear_sums(dx, dw)
+        assert sums.dim() == 3
+        torch.testing.assert_close(sums.sum(0).cpu(), want, rtol=1e-5,
+                                   atol=2e-5)
+        res = torch.randn(m, n, dtype=torch.bfloat16)
+        nw = torch.randn(n, dtype=torch.bfloat16)
+        dres = res.to(DEV)
+        h, new = ops.fused_add_rms_norm(sums, dres, nw.to(DEV), 1e-5)
+        assert new is dres
+        total = want + res.float()
+        torch.testing.assert_close(new.float().cpu(), total, **tol)
+        # the norm reads the rounded sum: two roundings
+        torch.testing.assert_close(
+            h.float().cpu(), ref.rms_norm(total, nw.float(), 1e-5),
+            rtol=2 ** -7, atol=2e-4)
+        got = ops.linear_silu_mul(dx, dw)
+        g, u = want.chunk(2, -1)
+        torch.testing.assert_close(
+            got.float().cpu(), torch.nn.functional.silu(g) * u, rtol=2 ** -8,
+            atol=5e-5)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_rope_qkv_cache_from_stretches(fp8):
+    """The epilogue over a product's stretches is that over their sum."""
+    torch.manual_seed(24)
+    T, hq, hkv, d, bs = 3, 4, 2, 128, 16
+    sums = torch.randn(5, T, (hq + 2 * hkv) * d, device=DEV)
+    # exact in bf16, so that both read the same values
+    sums = (sums * 4).round() / 4
+    pos = torch.tensor([0, 7, 130], device=DEV)
+    slots = torch.tensor([3, -1, 40], device=DEV)
+    cs = ref.make_cos_sin_cache(d, 256).to(DEV)
+    out = []
+    for z in (sums, sums.sum(0).bfloat16()):
+        kv = [torch.zeros(4, hkv, bs, d, device=DEV,
+                          dtype=torch.uint8 if fp8 else torch.bfloat16)
+              for _ in range(2)]
+        out.append([*ops.rope_qkv_cache(pos, z, cs, hq, hkv, d, kv, slots,
+                                        True), *kv])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 def test_linear_dispatch_matches_torch():
     """ops.linear (the HLinear route) must agree with F.linear on the
     decode shapes it owns."""
