@@ -201,6 +201,28 @@ def test_gemm_bf16(m, n, k):
     assert_close_bf16(got, want, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 64), (33, 70, 128), (64, 62, 64),          # tiles of 32 x 64
+    (65, 64, 192), (130, 1030, 64),                   # of 64
+    (2049, 2050, 64),                                 # of 128
+    (3585, 3500, 64),                                 # of 256
+])
+def test_gemm_bf16_tiles(m, n, k, act):
+    """Remainders of rows and columns for every tile, one step and several,
+    columns that are not stored four at a time."""
+    torch.manual_seed(25)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    bias = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    got = ops.gemm_bf16(x, w, bias, act)
+    want = x.double() @ w.double().t() + bias.double()
+    if act:
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    # fp32 sums of k products, then the rounding to bf16 (2^-9, doubled)
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2e-5)
+
+
 def test_gemm_bf16_gelu():
     torch.manual_seed(12)
     x = torch.randn(100, 768, dtype=torch.bfloat16, device=DEV) / 5
