@@ -64,21 +64,17 @@ class BertLayer(nn.Module):
         T = x.shape[0]
         h = self.cfg.hidden_size
         qkv = ops.gemm_bf16(x, self.qkv_w, self.qkv_b)
-        q, k, v = qkv.split([h, h, h], dim=-1)
         nh = self.cfg.num_heads
-        o = ops.attn_prefill(q.contiguous().view(T, nh, self.hd),
-                             k.contiguous().view(T, nh, self.hd),
-                             v.contiguous().view(T, nh, self.hd),
-                             cu, max_len, self.scale, causal=False)
+        q, k, v = (t.view(T, nh, self.hd)
+                   for t in qkv.split([h, h, h], dim=-1))
+        o = ops.attn_prefill(q, k, v, cu, max_len, self.scale, causal=False)
         a = ops.gemm_bf16(o.view(T, h), self.attn_out_w, self.attn_out_b)
-        x = ops.layer_norm((x.float() + a.float()).to(x.dtype),
-                           self.attn_ln_w, self.attn_ln_b,
-                           self.cfg.layer_norm_eps)
+        x = ops.add_layer_norm(x, a, self.attn_ln_w, self.attn_ln_b,
+                               self.cfg.layer_norm_eps)
         m = ops.gemm_bf16(x, self.up_w, self.up_b, act=1)   # fused GELU
         m = ops.gemm_bf16(m, self.down_w, self.down_b)
-        return ops.layer_norm((x.float() + m.float()).to(x.dtype),
-                              self.out_ln_w, self.out_ln_b,
-                              self.cfg.layer_norm_eps)
+        return ops.add_layer_norm(x, m, self.out_ln_w, self.out_ln_b,
+                                  self.cfg.layer_norm_eps)
 
 
 class BertEmbeddingModel(nn.Module):
@@ -96,23 +92,27 @@ class BertEmbeddingModel(nn.Module):
     def forward(self, input_ids: torch.Tensor, cu_seqlens: torch.Tensor,
                 max_len: int) -> torch.Tensor:
         """input_ids: [T] varlen concat; returns [B, H] L2-normalized."""
-        positions = torch.cat([
-            torch.arange(int(cu_seqlens[i + 1] - cu_seqlens[i]),
-                         device=input_ids.device)
-            for i in range(cu_seqlens.shape[0] - 1)])
+        T = input_ids.shape[0]
+        # one read by the host, for the checks and the mean's bounds
+        cu = cu_seqlens.tolist()
+        if cu[0] != 0 or cu[-1] != T or any(
+                b < a for a, b in zip(cu, cu[1:])):
+            raise ValueError(f"boundaries {cu} do not cut {T} tokens")
+        if self.cfg.pooling != "mean" and cu[-2] == T:
+            raise IndexError("a last text without tokens")
+        start = cu_seqlens[:-1].long()
+        positions = torch.arange(T, device=input_ids.device) - \
+            torch.repeat_interleave(start, cu_seqlens.diff(), output_size=T)
         x = self.word_emb(input_ids) + self.pos_emb(positions)
         x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
                            self.cfg.layer_norm_eps)
         for layer in self.layers:
             x = layer(x, cu_seqlens, max_len)
-        outs = []
-        for i in range(cu_seqlens.shape[0] - 1):
-            s, e = int(cu_seqlens[i]), int(cu_seqlens[i + 1])
-            if self.cfg.pooling == "mean":
-                outs.append(x[s:e].float().mean(0))
-            else:
-                outs.append(x[s].float())
-        emb = torch.stack(outs)
+        if self.cfg.pooling == "mean":
+            emb = torch.stack([x[s:e].float().mean(0)
+                               for s, e in zip(cu, cu[1:])])
+        else:
+            emb = x[start].float()
         return torch.nn.functional.normalize(emb, dim=-1)
 
     @torch.inference_mode()

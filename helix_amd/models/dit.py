@@ -13,7 +13,8 @@ MI355X-first rectified-flow DiT ("flux-lite" architecture class):
   — the same `ops.attn_prefill` the bge/ViT encoders run;
 - DiT blocks with adaLN modulation from (timestep, pooled prompt);
   every projection runs on the hand-written MFMA bf16 GEMM
-  (`ops.gemm_bf16`), norms on `ops.layer_norm`;
+  (`ops.gemm_bf16`), norms with their modulation and the gated sum
+  before them on `ops.modulated_norm`;
 - Euler integration of the rectified-flow ODE (velocity prediction,
   sigma-shifted schedule), deterministic per seed: noise is drawn on a
   CPU generator so CPU and GPU runs of the same seed share a prior.
@@ -139,9 +140,6 @@ class DiTBlock(nn.Module):
         self.down_b = nn.Parameter(torch.zeros(h))
         self.mod_w = nn.Parameter(torch.empty(6 * h, h))
         self.mod_b = nn.Parameter(torch.zeros(6 * h))
-        # affine-free LayerNorm operands for ops.layer_norm
-        self.register_buffer("ln_w", torch.ones(h), persistent=False)
-        self.register_buffer("ln_b", torch.zeros(h), persistent=False)
         self.hd = h // cfg.heads
         self.scale = self.hd ** -0.5
 
@@ -149,25 +147,19 @@ class DiTBlock(nn.Module):
                 cu: torch.Tensor, L: int) -> torch.Tensor:
         h = self.cfg.hidden
         T = x.shape[0]
-        mod = ops.gemm_bf16(cond, self.mod_w, self.mod_b)
-        sa, ca, ga, sm, cm, gm = (m.repeat_interleave(L, dim=0)
-                                  for m in mod.chunk(6, dim=-1))
-        n = ops.layer_norm(x, self.ln_w, self.ln_b, self.cfg.eps)
-        n = (n * (1 + ca) + sa).to(x.dtype)
+        sa, ca, ga, sm, cm, gm = ops.gemm_bf16(
+            cond, self.mod_w, self.mod_b).chunk(6, dim=-1)
+        _, n = ops.modulated_norm(x, ca, sa, L, self.cfg.eps)
         qkv = ops.gemm_bf16(n, self.qkv_w, self.qkv_b)
-        q, k, v = qkv.split([h, h, h], dim=-1)
         nh = self.cfg.heads
-        o = ops.attn_prefill(q.contiguous().view(T, nh, self.hd),
-                             k.contiguous().view(T, nh, self.hd),
-                             v.contiguous().view(T, nh, self.hd),
-                             cu, L, self.scale, causal=False)
+        q, k, v = (t.view(T, nh, self.hd)
+                   for t in qkv.split([h, h, h], dim=-1))
+        o = ops.attn_prefill(q, k, v, cu, L, self.scale, causal=False)
         a = ops.gemm_bf16(o.view(T, h), self.out_w, self.out_b)
-        x = (x.float() + ga.float() * a.float()).to(x.dtype)
-        n = ops.layer_norm(x, self.ln_w, self.ln_b, self.cfg.eps)
-        n = (n * (1 + cm) + sm).to(x.dtype)
+        x, n = ops.modulated_norm(x, cm, sm, L, self.cfg.eps, a, ga)
         m = ops.gemm_bf16(n, self.up_w, self.up_b, act=1)     # fused GELU
         m = ops.gemm_bf16(m, self.down_w, self.down_b)
-        return (x.float() + gm.float() * m.float()).to(x.dtype)
+        return ops.gated_add(x, m, gm, L)
 
 
 class DiTModel(nn.Module):
@@ -195,8 +187,6 @@ class DiTModel(nn.Module):
         self.fin_mod_b = nn.Parameter(torch.zeros(2 * h))
         self.fin_w = nn.Parameter(torch.empty(cfg.patch_dim, h))
         self.fin_b = nn.Parameter(torch.zeros(cfg.patch_dim))
-        self.register_buffer("ln_w", torch.ones(h), persistent=False)
-        self.register_buffer("ln_b", torch.zeros(h), persistent=False)
 
     def _patchify(self, lat: torch.Tensor) -> torch.Tensor:
         p = self.cfg.patch
@@ -237,11 +227,9 @@ class DiTModel(nn.Module):
                           device=lat.device)
         for blk in self.blocks:
             x = blk(x, cond, cu, L)
-        n = ops.layer_norm(x, self.ln_w, self.ln_b, cfg.eps)
         fm = ops.gemm_bf16(cond, self.fin_mod_w, self.fin_mod_b)
-        shift, scale = (m.repeat_interleave(L, dim=0)
-                        for m in fm.chunk(2, dim=-1))
-        n = (n * (1 + scale) + shift).to(dtype)
+        shift, scale = fm.chunk(2, dim=-1)
+        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps)
         out = ops.gemm_bf16(n, self.fin_w, self.fin_b)
         patch_rows = out.view(B, L, -1)[:, Tt:, :].reshape(
             B * P, cfg.patch_dim)
@@ -318,7 +306,7 @@ class DiffusionImageModel(nn.Module):
             torch.cuda.manual_seed(seed)
         g = None if on_gpu else torch.Generator().manual_seed(seed)
         for name, p in self.named_parameters():
-            if name.endswith(("_b", "ln_w", "ln_b", ".bias")):
+            if name.endswith(("_b", ".bias")):
                 continue
             # conv weights get variance-preserving init so the VAE
             # stack neither saturates nor flattens random-init images

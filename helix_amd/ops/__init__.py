@@ -83,6 +83,55 @@ def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor,
     return ref.layer_norm(x, w, b, eps)
 
 
+def _rows_of_8(x: torch.Tensor) -> bool:
+    """Whether encoder.hip takes these rows (a lane has up to 8 vectors)."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2
+            and x.shape[1] % 8 == 0 and x.shape[1] <= 4096
+            and x.is_contiguous())
+
+
+def add_layer_norm(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor,
+                   b: torch.Tensor, eps: float) -> torch.Tensor:
+    """Layer norm of x + y."""
+    if _rows_of_8(x) and y.is_contiguous():
+        out = torch.empty_like(x)
+        _native().add_norm(None, out, x, y, None, w, b, 0, eps)
+        return out
+    return layer_norm((x.float() + y.float()).to(x.dtype), w, b, eps)
+
+
+def modulated_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor,
+                   L: int, eps: float, y: torch.Tensor | None = None,
+                   gate: torch.Tensor | None = None):
+    """(s, norm(s) (1 + scale) + shift), s = x + gate y (x without y). norm
+    is a layer norm without weights; gate, scale and shift have a row for
+    every L rows of x."""
+    if _rows_of_8(x) and (y is None or y.is_contiguous()):
+        out = torch.empty_like(x)
+        s = x if y is None else torch.empty_like(x)
+        _native().add_norm(None if y is None else s, out, x, y, gate, scale,
+                           shift, L, eps)
+        return s, out
+    if y is not None:
+        x = gated_add(x, y, gate, L)
+    h = x.shape[-1]
+    n = layer_norm(x, torch.ones(h, dtype=x.dtype, device=x.device),
+                   torch.zeros(h, dtype=x.dtype, device=x.device), eps)
+    c, s = (t.repeat_interleave(L, dim=0) for t in (scale, shift))
+    return x, (n * (1 + c) + s).to(x.dtype)
+
+
+def gated_add(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor,
+              L: int) -> torch.Tensor:
+    """x + gate y; gate has a row for every L rows of x."""
+    if _rows_of_8(x) and y.is_contiguous():
+        out = torch.empty_like(x)
+        _native().gated_add(out, x, y, gate, L)
+        return out
+    g = gate.repeat_interleave(L, dim=0)
+    return (x.float() + g.float() * y.float()).to(x.dtype)
+
+
 def rotary_embedding(positions: torch.Tensor, q: torch.Tensor,
                      k: torch.Tensor, cos_sin: torch.Tensor, head_dim: int):
     """In-place on GPU. Returns (q, k)."""

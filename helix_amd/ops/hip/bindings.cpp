@@ -4,6 +4,12 @@
 void rms_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w, double eps);
 void fused_add_rms_norm(torch::Tensor x, torch::Tensor residual,
                         torch::Tensor w, double eps);
+void add_norm(c10::optional<torch::Tensor> sum, torch::Tensor out,
+              torch::Tensor x, c10::optional<torch::Tensor> y,
+              c10::optional<torch::Tensor> gate, torch::Tensor a,
+              torch::Tensor b, int64_t L, double eps);
+void gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
+               torch::Tensor gate, int64_t L);
 void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
                        torch::Tensor residual, torch::Tensor w, double eps);
 void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -71,6 +77,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16, CDNA4)");
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "Fused residual-add + RMSNorm (in-place)");
+  m.def("add_norm", &add_norm,
+        "(Gated) add + LayerNorm with weights or an image's modulation");
+  m.def("gated_add", &gated_add, "x + gate * y, a gate per image");
   m.def("add_sums_rms_norm", &add_sums_rms_norm,
         "Sum of a product's stretches + residual-add + RMSNorm");
   m.def("layer_norm", &layer_norm, "LayerNorm (bf16)");

@@ -65,6 +65,39 @@ def test_layer_norm():
     assert_close_bf16(got, want)
 
 
+@pytest.mark.parametrize("T,H", [(1, 8), (5, 512), (7, 520), (66, 768),
+                                 (9, 1032), (4, 2056), (3, 4096)])
+def test_add_norm(T, H):
+    """Sum and layer norm, with weights and with an image's modulation; rows
+    that end within a lane's vectors."""
+    torch.manual_seed(26)
+    L = 3
+    x, y = (torch.randn(T, H, dtype=torch.bfloat16, device=DEV) * 3 + 1
+            for _ in range(2))
+    w, b = (torch.randn(H, dtype=torch.bfloat16, device=DEV)
+            for _ in range(2))
+    mod = torch.randn(-(-T // L), 3 * H, dtype=torch.bfloat16, device=DEV)
+    gate, scale, shift = mod.chunk(3, -1)
+    g, c, s = (t.repeat_interleave(L, 0)[:T].double()
+               for t in (gate, scale, shift))
+    norm = lambda t: torch.nn.functional.layer_norm(t, (H,), eps=1e-6)  # noqa: E731
+    # 32-bit sums of H values, then the rounding to bf16 (2^-9, doubled)
+    tol = dict(rtol=2 ** -8, atol=2e-5)
+    got = ops.add_layer_norm(x, y, w, b, 1e-6)
+    want = norm(x.double() + y.double()) * w.double() + b.double()
+    torch.testing.assert_close(got.double(), want, **tol)
+    total = x.double() + g * y.double()
+    new, got = ops.modulated_norm(x, scale, shift, L, 1e-6, y, gate)
+    torch.testing.assert_close(new.double(), total, **tol)
+    torch.testing.assert_close(got.double(), norm(total) * (1 + c) + s, **tol)
+    same, got = ops.modulated_norm(x, scale, shift, L, 1e-6)
+    assert same is x
+    torch.testing.assert_close(got.double(), norm(x.double()) * (1 + c) + s,
+                               **tol)
+    torch.testing.assert_close(ops.gated_add(x, y, gate, L).double(), total,
+                               **tol)
+
+
 @pytest.mark.parametrize("hq,hk,d", [(32, 8, 128), (12, 12, 64)])
 def test_rope(hq, hk, d):
     torch.manual_seed(3)
