@@ -21,6 +21,7 @@ import torch.nn.functional as F
 from helix_amd import ops
 from helix_amd.models.meta import (DecodeMeta, KVLayer,  # noqa: F401
                                    MixedMeta, PrefillMeta)
+from helix_amd.models.quant import FP8Linear
 from helix_amd.ops import make_cos_sin_cache
 
 
@@ -150,7 +151,7 @@ class HLinear(nn.Linear):
 
 def _project(proj: nn.Module, x: torch.Tensor, form: str) -> torch.Tensor:
     """proj(x) in that form; other kinds of projections know only rows."""
-    if isinstance(proj, HLinear):
+    if isinstance(proj, (HLinear, FP8Linear)):
         return proj(x, form)
     out = proj(x)
     return ops.silu_and_mul(out) if form == "glu" else out

@@ -315,6 +315,13 @@ def sample_tokens_ext(logits: torch.Tensor, temperatures: torch.Tensor,
 def quantize_fp8(t: torch.Tensor, dim: int = -1):
     """Per-row (dim=-1 reduces over the last axis) e4m3 quantization.
     Returns (bytes uint8 view, float32 scales)."""
+    if t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 2 and \
+            dim in (-1, 1) and t.shape[1] > 0 and t.shape[1] % 8 == 0 and \
+            t.is_contiguous() and t.data_ptr() % 16 == 0:
+        q = torch.empty(t.shape, dtype=torch.uint8, device=t.device)
+        scale = torch.empty(t.shape[0], dtype=torch.float32, device=t.device)
+        _native().quantize_rows(q, scale, t)
+        return q, scale
     amax = t.float().abs().amax(dim=dim, keepdim=True).clamp(min=1e-8)
     scale = amax / 448.0                      # e4m3fn max normal
     q = (t.float() / scale).to(torch.float8_e4m3fn)
@@ -330,6 +337,10 @@ def gemm_fp8(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,
     M, N = x8.shape[0], w8.shape[0]
     if x8.is_cuda:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=x8.device)
+        if act == 0 and _rows_fit(x8, w8):
+            _native().gemm_rows(out, x8, w8, bias, x_scale.contiguous(),
+                                w_scale.contiguous())
+            return out
         _native().gemm_fp8(out, x8, w8, x_scale.contiguous(),
                            w_scale.contiguous(), bias, act)
         return out
@@ -393,16 +404,18 @@ def gemm_skinny_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
 
 
 ROWS_MAX_M = 64                   # of gemm_rows.hip
-ROWS_CHUNK = 256
+ROWS_CHUNK = 512                  # bytes
 
 
 def _rows_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether the kernel for a few rows takes x @ w^T. It knows nothing of
-    gradients, so it only runs where there are none to be had."""
-    return (x.is_cuda and torch.is_inference_mode_enabled()
-            and x.dim() == 2 and 0 < x.shape[0] <= ROWS_MAX_M
-            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and x.shape[1] > 0 and x.shape[1] % ROWS_CHUNK == 0
+    """Whether the kernel for a few rows takes x @ w^T, bf16 or e4m3 bytes.
+    It knows nothing of gradients, so bf16 only runs where there are none to
+    be had."""
+    return (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= ROWS_MAX_M
+            and (x.dtype == torch.uint8 or x.dtype == torch.bfloat16
+                 and torch.is_inference_mode_enabled())
+            and x.dtype == w.dtype and x.shape[1] > 0
+            and x.shape[1] * x.element_size() % ROWS_CHUNK == 0
             and w.shape[0] > 0 and w.shape[0] % 8 == 0
             and x.is_contiguous() and w.is_contiguous()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
@@ -427,7 +440,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
             (x.shape[0] <= 16 or x.shape[1] >= 2 * w.shape[0]):
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
-        _native().gemm_rows(out, x, w, bias)
+        _native().gemm_rows(out, x, w, bias, None, None)
         return out
     return torch.nn.functional.linear(x, w, bias)
 
@@ -438,7 +451,7 @@ def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     rows, else [M, N] in x's type. Wide matrices fill the chip without
     stretches, and 64 rows of 16384 sums are more bytes than they save."""
     if _rows_fit(x, w) and w.shape[0] <= 8192:
-        return _native().gemm_rows_sums(x, w)
+        return _native().gemm_rows_sums(x, w, None, None)
     return linear(x, w)
 
 
@@ -449,9 +462,29 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if _rows_fit(x, w):
         out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                           device=x.device)
-        _native().gemm_rows_glu(out, x, w)
+        _native().gemm_rows_glu(out, x, w, None, None)
         return out
     return silu_and_mul(linear(x, w))
+
+
+def gemm_fp8_sums(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,
+                  w_scale: torch.Tensor) -> torch.Tensor:
+    """gemm_fp8 for a reader that adds up stretches (linear_sums)."""
+    if _rows_fit(x8, w8) and w8.shape[0] <= 8192:
+        return _native().gemm_rows_sums(x8, w8, x_scale, w_scale)
+    return gemm_fp8(x8, w8, x_scale, w_scale)
+
+
+def gemm_fp8_silu_mul(x8: torch.Tensor, w8: torch.Tensor,
+                      x_scale: torch.Tensor,
+                      w_scale: torch.Tensor) -> torch.Tensor:
+    """silu(first half) * second half of gemm_fp8's columns."""
+    if _rows_fit(x8, w8):
+        out = torch.empty(x8.shape[0], w8.shape[0] // 2,
+                          dtype=torch.bfloat16, device=x8.device)
+        _native().gemm_rows_glu(out, x8, w8, x_scale, w_scale)
+        return out
+    return silu_and_mul(gemm_fp8(x8, w8, x_scale, w_scale))
 
 
 def mfma_probe(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:

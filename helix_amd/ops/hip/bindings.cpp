@@ -57,10 +57,14 @@ void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                       c10::optional<torch::Tensor> bias,
                       c10::optional<torch::Tensor> scratch, int64_t split_k,
                       int64_t act, int64_t swizzle);
-void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias);
-torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w);
-void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w);
+using OptT = c10::optional<torch::Tensor>;
+void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
+               OptT x_scale, OptT w_scale);
+torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
+                             OptT w_scale);
+void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                   OptT x_scale, OptT w_scale);
+void quantize_rows(torch::Tensor out, torch::Tensor scales, torch::Tensor x);
 void gemm_fp8(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               torch::Tensor x_scale, torch::Tensor w_scale,
               c10::optional<torch::Tensor> bias, int64_t act);
@@ -106,6 +110,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "x @ w^T of at most 64 rows, stretches of the inner dimension apart");
   m.def("gemm_rows_glu", &gemm_rows_glu,
         "silu(x @ gate^T) * (x @ up^T) of at most 64 rows");
+  m.def("quantize_rows", &quantize_rows,
+        "bf16 rows to e4m3 bytes with a scale each");
   m.def("gemm_fp8", &gemm_fp8,
         "MX-fp8 e4m3 MFMA GEMM with epilogue per-row/col dequant");
   m.def("mfma_probe", &mfma_probe, "16x16x32 MFMA layout probe");

@@ -1,9 +1,9 @@
-// Product of a few rows with a large matrix: x[M,K] @ w[N,K]^T, bf16 with fp32
-// sums, M <= 64.
+// Product of a few rows with a large matrix: x[M,K] @ w[N,K]^T, bf16 or e4m3
+// with fp32 sums, M <= 64.
 //
 // Bound by reading w once. A wave streams its columns of w straight into MFMA
-// operands, a chunk of 256 of the inner dimension ahead; x goes to LDS by
-// direct loads, once for the columns of all waves. 16-byte piece p of row r
+// operands, a chunk of 512 bytes of the inner dimension ahead; x goes to LDS
+// by direct loads, once for the columns of all waves. 16-byte piece p of row r
 // lies at p ^ r % 16, so operands leave LDS without bank conflicts.
 //
 // Narrow matrices leave CUs idle, so the inner dimension is cut into stretches
@@ -22,8 +22,13 @@
 //   M 64   17.6 (18.0)  12.2 (15.2)   55.4 (52.3)   31.9 (41.9)
 // Adding them up in a launch takes 2.5 to 3 us more. The gated product
 // replaces a launch of 4.5 us as well. Reading 28672 x 4096 at 44.5 us is 5.3
-// TB/s. Eight waves a workgroup, chunks of 128 or 512, 32 columns a wave and
-// 256 or 768 workgroups were each slower on most of these.
+// TB/s. Eight waves a workgroup, chunks half or twice as long, 32 columns a
+// wave and 256 or 768 workgroups were each slower on most of these.
+//
+// e4m3 (weights with a scale per column, x with one per row) runs the scaled
+// 16x16x128 instruction with unity scales; the scales meet the fp32 sums of
+// every stretch. us at 32 rows of the four matrices, the tiles of gemm_fp8.hip
+// in brackets: 9.4 (49.5), 7.4 (51.6), 27.4 (53.9), 16.0 (158).
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -32,62 +37,81 @@ using namespace helix;
 
 namespace {
 
-constexpr int KC = 256;                       // inner dimension of a chunk
+constexpr int CB = 512;                       // bytes of a chunk's row
 constexpr int WANT = 512;                     // workgroups, 2 on each CU
+constexpr int UNITY = 0x7F7F7F7F;             // e8m0 2^0 in all four bytes
+
+typedef int v8i __attribute__((ext_vector_type(8)));
 
 struct Product {
   const uint16_t* bias;
-  int M, N, K, n_tiles, per;   // per: chunks of a stretch
+  const float *xs, *ws;        // e4m3: scales of rows and columns
+  int64_t row;                 // bytes of a row of x and w
+  int M, N, n_tiles, chunks, per;             // per: chunks of a stretch
 };
 
+__device__ __forceinline__ v8i join(u32x4 a, u32x4 b) {
+  return v8i{(int)a[0], (int)a[1], (int)a[2], (int)a[3],
+             (int)b[0], (int)b[1], (int)b[2], (int)b[3]};
+}
+
 // 16 MI rows, NW waves. GLU: columns n and N + n are a pair of a wave.
-template <int MI, int NW, bool GLU>
+template <int MI, int NW, bool GLU, bool F8>
 __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
     uint16_t* __restrict__ out, float* __restrict__ sums,
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-    Product m) {
+    const char* __restrict__ x, const char* __restrict__ w, Product m) {
   constexpr int NI = GLU ? 2 : 1;
   constexpr int TH = NW * WAVE, BM = MI * 16;
-  constexpr int PR = KC / 8, XL = BM * PR / TH, U = KC / 32;
+  constexpr int PR = CB / 16, XL = BM * PR / TH, U = CB / 64;
   static_assert(BM * PR % TH == 0, "x tile");
-  __shared__ __attribute__((aligned(16))) uint16_t xl[2][BM * KC];
+  __shared__ __attribute__((aligned(16))) char xl[2][BM * CB];
   const int stretch = blockIdx.x / m.n_tiles;
   const int tid = threadIdx.x, wid = tid / WAVE, lane = tid & (WAVE - 1);
   const int lo = lane & 15, hi = lane >> 4;
   const int n0 = (blockIdx.x % m.n_tiles * NW + wid) * 16;
-  const int c0 = stretch * m.per, c1 = min(m.K / KC, c0 + m.per);
-  const uint16_t* wp[NI];
+  const int c0 = stretch * m.per, c1 = min(m.chunks, c0 + m.per);
+  // a lane's 16 bytes u of a chunk's row: bf16 has four lane groups to 64
+  // bytes, e4m3 two pieces side by side to 128
+  auto piece = [&](int u) {
+    return F8 ? (u >> 1) * 8 + hi * 2 + (u & 1) : u * 4 + hi;
+  };
+  const char* wp[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j)
-    wp[j] = w + ((int64_t)j * m.N + min(n0 + lo, m.N - 1)) * m.K + hi * 8;
-  const uint16_t* xp[XL];
+    wp[j] = w + ((int64_t)j * m.N + min(n0 + lo, m.N - 1)) * m.row;
+  const char* xp[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int e = i * TH + tid, r = e / PR, p = e % PR ^ (r & 15);
-    xp[i] = x + (int64_t)min(r, m.M - 1) * m.K + p * 8;
+    xp[i] = x + min(r, m.M - 1) * m.row + p * 16;
   }
   auto load_x = [&](int c, int b) {
 #pragma unroll
     for (int i = 0; i < XL; ++i)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) uint32_t*)(xp[i] + c * KC),
+          (const __attribute__((address_space(1))) uint32_t*)(xp[i] + c * CB),
           (__attribute__((address_space(3))) uint32_t*)(
-              xl[b] + (i * TH + wid * WAVE) * 8),
+              xl[b] + (i * TH + wid * WAVE) * 16),
           16, 0, 0);
   };
-  u16x8 wr[2][U][NI];
+  u32x4 wr[2][U][NI];
   auto load_w = [&](int c, int b) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int j = 0; j < NI; ++j)
-        wr[b][u][j] = ld_u16x8(wp[j] + c * KC + u * 32);
+        wr[b][u][j] = *reinterpret_cast<const u32x4*>(wp[j] + c * CB +
+                                                      piece(u) * 16);
   };
   floatx4 acc[NI][MI];
 #pragma unroll
   for (int j = 0; j < NI; ++j)
 #pragma unroll
     for (int i = 0; i < MI; ++i) acc[j][i] = floatx4{0, 0, 0, 0};
+  auto x_at = [&](int b, int i, int u) {
+    return *reinterpret_cast<const u32x4*>(xl[b] + (i * 16 + lo) * CB +
+                                           (piece(u) ^ lo) * 16);
+  };
   auto step = [&](int c, int b) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -97,14 +121,23 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; u += F8 ? 2 : 1)
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        const u16x8 xf =
-            ld_u16x8(xl[b] + (i * 16 + lo) * KC + ((u * 4 + hi) ^ lo) * 8);
+        if constexpr (F8) {
+          const v8i xf = join(x_at(b, i, u), x_at(b, i, u + 1));
 #pragma unroll
-        for (int j = 0; j < NI; ++j)
-          acc[j][i] = mfma16(wr[b][u][j], xf, acc[j][i]);
+          for (int j = 0; j < NI; ++j)
+            acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                join(wr[b][u][j], wr[b][u + 1][j]), xf, acc[j][i], 0, 0, 0,
+                UNITY, 0, UNITY);
+        } else {
+          const u16x8 xf = __builtin_bit_cast(u16x8, x_at(b, i, u));
+#pragma unroll
+          for (int j = 0; j < NI; ++j)
+            acc[j][i] = mfma16(__builtin_bit_cast(u16x8, wr[b][u][j]), xf,
+                               acc[j][i]);
+        }
       }
   };
   if (c0 < c1) {
@@ -122,6 +155,14 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
   for (int i = 0; i < MI; ++i) {
     const int r = i * 16 + lo;
     if (r >= m.M) continue;
+    if constexpr (F8) {
+      const float xs = m.xs[r];
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          acc[j][i][q] = acc[j][i][q] * xs * m.ws[j * m.N + n + q];
+    }
     float v[4];
     if constexpr (GLU) {
 #pragma unroll
@@ -161,39 +202,50 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(
   st_bf16x4(out + i, v);
 }
 
+using OptT = c10::optional<torch::Tensor>;
+
+// x_scale, w_scale: both (e4m3 bytes) or neither (bf16).
 Product product_of(const torch::Tensor& x, const torch::Tensor& w, int64_t N,
-                   int columns) {
+                   int columns, const OptT& x_scale, const OptT& w_scale) {
+  const bool f8 = x_scale.has_value();
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.is_cuda() &&
-                t.scalar_type() == torch::kBFloat16 &&
+                t.scalar_type() == (f8 ? torch::kUInt8 : torch::kBFloat16) &&
                 (uintptr_t)t.data_ptr() % 16 == 0);
   Product m{};
   m.M = x.size(0);
-  m.K = x.size(1);
   m.N = N;
-  TORCH_CHECK(w.size(1) == m.K && m.M >= 1 && m.M <= 64);
-  TORCH_CHECK(m.N >= 4 && m.N % 4 == 0 && m.K >= KC && m.K % KC == 0);
+  m.row = x.size(1) * (f8 ? 1 : 2);
+  TORCH_CHECK(w.size(1) == x.size(1) && m.M >= 1 && m.M <= 64);
+  TORCH_CHECK(m.N >= 4 && m.N % 4 == 0 && m.row >= CB && m.row % CB == 0);
+  TORCH_CHECK(w_scale.has_value() == f8);
+  if (f8) {
+    for (const auto& t : {*x_scale, *w_scale})
+      TORCH_CHECK(t.is_contiguous() && t.scalar_type() == torch::kFloat32);
+    TORCH_CHECK(x_scale->numel() == m.M && w_scale->numel() == w.size(0));
+    m.xs = x_scale->data_ptr<float>();
+    m.ws = w_scale->data_ptr<float>();
+  }
   m.n_tiles = cdiv(m.N, columns);
-  m.per = m.K / KC;
+  m.chunks = m.per = m.row / CB;
   return m;
 }
 
 // Stretches of the inner dimension: about WANT workgroups in all.
 int cut(Product& m) {
-  const int chunks = m.K / KC;
-  m.per = cdiv(chunks, std::max(1, std::min(WANT / m.n_tiles, chunks)));
-  return cdiv(chunks, m.per);
+  m.per = cdiv(m.chunks,
+               std::max(1, std::min(WANT / m.n_tiles, m.chunks)));
+  return cdiv(m.chunks, m.per);
 }
 
-template <int NW, bool GLU>
-void run(uint16_t* out, float* sums, const torch::Tensor& x,
-         const torch::Tensor& w, const Product& m, int stretches) {
+template <int NW, bool GLU, bool F8>
+void run_as(uint16_t* out, float* sums, const torch::Tensor& x,
+            const torch::Tensor& w, const Product& m, int stretches) {
 #define HELIX_GR(MI)                                                         \
-  hipLaunchKernelGGL((gemm_rows_kernel<MI, NW, GLU>),                        \
+  hipLaunchKernelGGL((gemm_rows_kernel<MI, NW, GLU, F8>),                    \
                      dim3(m.n_tiles * stretches), dim3(NW * WAVE), 0,        \
                      at::hip::getCurrentHIPStream(), out, sums,              \
-                     (const uint16_t*)x.data_ptr(),                          \
-                     (const uint16_t*)w.data_ptr(), m)
+                     (const char*)x.data_ptr(), (const char*)w.data_ptr(), m)
   if (m.M <= 16) HELIX_GR(1);
   else if (m.M <= 32) HELIX_GR(2);
   else if (m.M <= 48) HELIX_GR(3);
@@ -201,24 +253,41 @@ void run(uint16_t* out, float* sums, const torch::Tensor& x,
 #undef HELIX_GR
 }
 
+template <int NW, bool GLU>
+void run(uint16_t* out, float* sums, const torch::Tensor& x,
+         const torch::Tensor& w, const Product& m, int stretches) {
+  if (m.xs != nullptr) run_as<NW, GLU, true>(out, sums, x, w, m, stretches);
+  else run_as<NW, GLU, false>(out, sums, x, w, m, stretches);
+}
+
+torch::Tensor sums_for(const torch::Tensor& x, const Product& m,
+                       int stretches) {
+  return torch::empty({stretches, m.M, m.N},
+                      x.options().dtype(torch::kFloat32));
+}
+
+void check_out(const torch::Tensor& out, const Product& m) {
+  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 &&
+              out.scalar_type() == torch::kBFloat16 && out.size(0) == m.M &&
+              out.size(1) == m.N && (uintptr_t)out.data_ptr() % 8 == 0);
+}
+
 }  // namespace
 
 // Sums [stretches, M, N] for a reader that adds them up.
-torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w) {
-  Product m = product_of(x, w, w.size(0), 64);
+torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
+                             OptT w_scale) {
+  Product m = product_of(x, w, w.size(0), 64, x_scale, w_scale);
   const int stretches = cut(m);
-  torch::Tensor sums = torch::empty({stretches, m.M, m.N},
-                                    x.options().dtype(torch::kFloat32));
+  torch::Tensor sums = sums_for(x, m, stretches);
   run<4, false>(nullptr, sums.data_ptr<float>(), x, w, m, stretches);
   return sums;
 }
 
-void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias) {
-  Product m = product_of(x, w, w.size(0), 64);
-  TORCH_CHECK(out.is_contiguous() && out.scalar_type() == x.scalar_type() &&
-              out.size(0) == m.M && out.size(1) == m.N &&
-              (uintptr_t)out.data_ptr() % 8 == 0);
+void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
+               OptT x_scale, OptT w_scale) {
+  Product m = product_of(x, w, w.size(0), 64, x_scale, w_scale);
+  check_out(out, m);
   if (bias.has_value()) {
     TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 &&
                 bias->is_contiguous() && bias->numel() == m.N);
@@ -230,8 +299,7 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     run<4, false>(o, nullptr, x, w, m, 1);
     return;
   }
-  torch::Tensor sums = torch::empty({stretches, m.M, m.N},
-                                    x.options().dtype(torch::kFloat32));
+  torch::Tensor sums = sums_for(x, m, stretches);
   run<4, false>(nullptr, sums.data_ptr<float>(), x, w, m, stretches);
   const int64_t MN = (int64_t)m.M * m.N;
   hipLaunchKernelGGL(gemm_join_kernel, dim3((MN + 1023) / 1024), dim3(256), 0,
@@ -240,11 +308,10 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 }
 
 // out[M,N] = silu(x w[:N]^T) * (x w[N:]^T)
-void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
+void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                   OptT x_scale, OptT w_scale) {
   TORCH_CHECK(w.size(0) % 2 == 0);
-  Product m = product_of(x, w, w.size(0) / 2, 32);
-  TORCH_CHECK(out.is_contiguous() && out.scalar_type() == x.scalar_type() &&
-              out.size(0) == m.M && out.size(1) == m.N &&
-              (uintptr_t)out.data_ptr() % 8 == 0);
+  Product m = product_of(x, w, w.size(0) / 2, 32, x_scale, w_scale);
+  check_out(out, m);
   run<2, true>((uint16_t*)out.data_ptr(), nullptr, x, w, m, 1);
 }

@@ -629,7 +629,7 @@ def test_gemm_rows(m, n, k):
     tol = dict(rtol=2 ** -8, atol=2e-5)
     with torch.inference_mode():
         got = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
-        ops._native().gemm_rows(got, dx, dw, db)
+        ops._native().gemm_rows(got, dx, dw, db, None, None)
         torch.testing.assert_close(got.float().cpu(), want + b.float(), **tol)
         sums = ops.linear_sums(dx, dw)
         assert sums.dim() == 3
@@ -651,6 +651,55 @@ def test_gemm_rows(m, n, k):
         torch.testing.assert_close(
             got.float().cpu(), torch.nn.functional.silu(g) * u, rtol=2 ** -8,
             atol=5e-5)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 8, 512), (17, 72, 1024),
+                                   (48, 256, 4096), (64, 4104, 1536)])
+def test_gemm_rows_e4m3(m, n, k):
+    torch.manual_seed(27)
+    x8, xs = ops.quantize_fp8(torch.randn(m, k, dtype=torch.bfloat16,
+                                          device=DEV))
+    w8, ws = ops.quantize_fp8(torch.randn(n, k, dtype=torch.bfloat16,
+                                          device=DEV) / k ** 0.5)
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    wide = lambda t, s: t.view(torch.float8_e4m3fn).double() * s[:, None].double()  # noqa: E731
+    want = wide(x8, xs) @ wide(w8, ws).t()
+    # The matrix instruction aligns its 128 products before it adds them, so
+    # what is lost is a share of their magnitudes, not of the sum: below 2^-18
+    # where sums are kept to 24 bits and a step's carry takes up to 6.
+    lost = float((wide(x8, xs).abs() @ wide(w8, ws).abs().t()).max()) * 2 ** -18
+    tol = dict(rtol=2 ** -8, atol=2 * lost)
+    torch.testing.assert_close(
+        ops.gemm_fp8(x8, w8, xs, ws, b).double(), want + b.double(), **tol)
+    sums = ops.gemm_fp8_sums(x8, w8, xs, ws)
+    assert sums.dim() == 3
+    torch.testing.assert_close(sums.double().sum(0), want, rtol=1e-5,
+                               atol=lost)
+    g, u = want.chunk(2, -1)
+    torch.testing.assert_close(
+        ops.gemm_fp8_silu_mul(x8, w8, xs, ws).double(),
+        torch.nn.functional.silu(g) * u, rtol=2 ** -8,
+        atol=2 * lost * float(want.abs().max() + 1))
+
+
+@pytest.mark.parametrize("T,K", [(1, 8), (3, 264), (33, 4096), (5, 14336)])
+def test_quantize_rows_bytes(T, K):
+    """Bytes and scales are those of the same steps as library calls."""
+    torch.manual_seed(28)
+    x = torch.randn(T, K, dtype=torch.bfloat16, device=DEV) * 7
+    x[-1] = 0
+    x[0, -1] = 300.0
+    if T > 3:
+        x[1, 2], x[2, 5] = float("nan"), float("inf")
+    got, scale = ops.quantize_fp8(x)
+    f = x.float()
+    s = f.abs().amax(-1, keepdim=True).clamp(min=1e-8) / 448.0
+    want = (f / s).to(torch.float8_e4m3fn)
+    assert torch.equal(scale.isnan(), s[:, 0].isnan())
+    assert torch.equal(scale.nan_to_num(), s[:, 0].nan_to_num())
+    got = got.view(torch.float8_e4m3fn).float()
+    assert torch.equal(got.isnan(), want.float().isnan())
+    assert torch.equal(got.nan_to_num(), want.float().nan_to_num())
 
 
 @pytest.mark.parametrize("fp8", [False, True])
