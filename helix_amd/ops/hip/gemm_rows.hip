@@ -1,5 +1,5 @@
 // Product of a few rows with a large matrix: x[M,K] @ w[N,K]^T, bf16 or e4m3
-// with fp32 sums, M <= 64.
+// with fp32 sums, M <= 128.
 //
 // Bound by reading w once. A wave streams its columns of w straight into MFMA
 // operands, a chunk of 512 bytes of the inner dimension ahead; x goes to LDS
@@ -20,10 +20,15 @@
 //   M 16   12.4 (15.7)   8.9 (15.6)   45.4 (65.1)   25.2 (27.3)
 //   M 32   15.2 (16.3)  10.4 (13.9)   51.8 (54.2)   27.8 (33.8)
 //   M 64   17.6 (18.0)  12.2 (15.2)   55.4 (52.3)   31.9 (41.9)
+// From 65 rows on a wave has 32 columns, so that x is read from LDS half as
+// often, chunks are half as long and 256 workgroups are enough; matrices as
+// wide as 28672 are the library's there (52, here 66 us):
+//   M 128  20.0 (24.6)  15.5 (24.7)                   34.6 (73.9)
 // Adding them up in a launch takes 2.5 to 3 us more. The gated product
 // replaces a launch of 4.5 us as well. Reading 28672 x 4096 at 44.5 us is 5.3
-// TB/s. Eight waves a workgroup, chunks half or twice as long, 32 columns a
-// wave and 256 or 768 workgroups were each slower on most of these.
+// TB/s. Eight waves a workgroup, chunks half or twice as long, and for up to
+// 64 rows 32 columns a wave and 256 or 768 workgroups were each slower on most
+// of these.
 //
 // e4m3 (weights with a scale per column, x with one per row) runs the scaled
 // 16x16x128 instruction with unity scales; the scales meet the fp32 sums of
@@ -37,8 +42,12 @@ using namespace helix;
 
 namespace {
 
-constexpr int CB = 512;                       // bytes of a chunk's row
-constexpr int WANT = 512;                     // workgroups, 2 on each CU
+// Up to 64 rows, and up to 128: bytes of a chunk's row, columns of a workgroup
+// and the workgroups that stretches are cut for.
+struct Shape {
+  int chunk, columns, want;
+};
+constexpr Shape FEW{512, 64, 512}, MORE{256, 128, 256};
 constexpr int UNITY = 0x7F7F7F7F;             // e8m0 2^0 in all four bytes
 
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -47,7 +56,7 @@ struct Product {
   const uint16_t* bias;
   const float *xs, *ws;        // e4m3: scales of rows and columns
   int64_t row;                 // bytes of a row of x and w
-  int M, N, n_tiles, chunks, per;             // per: chunks of a stretch
+  int M, N, n_tiles, chunks, per, want;       // per: chunks of a stretch
 };
 
 __device__ __forceinline__ v8i join(u32x4 a, u32x4 b) {
@@ -55,12 +64,13 @@ __device__ __forceinline__ v8i join(u32x4 a, u32x4 b) {
              (int)b[0], (int)b[1], (int)b[2], (int)b[3]};
 }
 
-// 16 MI rows, NW waves. GLU: columns n and N + n are a pair of a wave.
-template <int MI, int NW, bool GLU, bool F8>
+// 16 MI rows, NW waves of 16 NI columns each, chunks of CB bytes. GLU (NI 2):
+// columns n and N + n are a pair of a wave.
+template <int MI, int NI, int NW, int CB, bool GLU, bool F8>
 __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
     uint16_t* __restrict__ out, float* __restrict__ sums,
     const char* __restrict__ x, const char* __restrict__ w, Product m) {
-  constexpr int NI = GLU ? 2 : 1;
+  constexpr int CN = GLU ? 1 : NI;            // 16-column tiles of the output
   constexpr int TH = NW * WAVE, BM = MI * 16;
   constexpr int PR = CB / 16, XL = BM * PR / TH, U = CB / 64;
   static_assert(BM * PR % TH == 0, "x tile");
@@ -68,7 +78,7 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
   const int stretch = blockIdx.x / m.n_tiles;
   const int tid = threadIdx.x, wid = tid / WAVE, lane = tid & (WAVE - 1);
   const int lo = lane & 15, hi = lane >> 4;
-  const int n0 = (blockIdx.x % m.n_tiles * NW + wid) * 16;
+  const int n0 = (blockIdx.x % m.n_tiles * NW + wid) * 16 * CN;
   const int c0 = stretch * m.per, c1 = min(m.chunks, c0 + m.per);
   // a lane's 16 bytes u of a chunk's row: bf16 has four lane groups to 64
   // bytes, e4m3 two pieces side by side to 128
@@ -78,7 +88,8 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
   const char* wp[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j)
-    wp[j] = w + ((int64_t)j * m.N + min(n0 + lo, m.N - 1)) * m.row;
+    wp[j] = w + (GLU ? (int64_t)j * m.N + min(n0 + lo, m.N - 1)
+                     : (int64_t)min(n0 + j * 16 + lo, m.N - 1)) * m.row;
   const char* xp[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
@@ -149,37 +160,41 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
     if (c + 1 < c1) step(c + 1, 1);
   }
   // lane: columns 4 hi + q of row lo
-  const int n = n0 + hi * 4;
-  if (n >= m.N) return;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int r = i * 16 + lo;
     if (r >= m.M) continue;
-    if constexpr (F8) {
-      const float xs = m.xs[r];
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
+    for (int j = 0; j < CN; ++j) {
+      const int n = n0 + j * 16 + hi * 4;
+      if (n >= m.N) continue;
+      if constexpr (F8) {
+        const float xs = m.xs[r];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[j][i][q] = acc[j][i][q] * xs * m.ws[n + q];
+          if constexpr (GLU)
+            acc[1][i][q] = acc[1][i][q] * xs * m.ws[m.N + n + q];
+        }
+      }
+      float v[4];
+      if constexpr (GLU) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          acc[j][i][q] = acc[j][i][q] * xs * m.ws[j * m.N + n + q];
-    }
-    float v[4];
-    if constexpr (GLU) {
+          v[q] = acc[0][i][q] / (1.f + __expf(-acc[0][i][q])) * acc[1][i][q];
+      } else {
+        if (sums != nullptr) {
+          *reinterpret_cast<floatx4*>(
+              sums + ((int64_t)stretch * m.M + r) * m.N + n) = acc[j][i];
+          continue;
+        }
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        v[q] = acc[0][i][q] / (1.f + __expf(-acc[0][i][q])) * acc[1][i][q];
-    } else {
-      if (sums != nullptr) {
-        *reinterpret_cast<floatx4*>(
-            sums + ((int64_t)stretch * m.M + r) * m.N + n) = acc[0][i];
-        continue;
+        for (int q = 0; q < 4; ++q)
+          v[q] = acc[j][i][q] +
+                 (m.bias != nullptr ? bf16_to_f32(m.bias[n + q]) : 0.f);
       }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        v[q] = acc[0][i][q] +
-               (m.bias != nullptr ? bf16_to_f32(m.bias[n + q]) : 0.f);
+      st_bf16x4(out + (int64_t)r * m.N + n, v);
     }
-    st_bf16x4(out + (int64_t)r * m.N + n, v);
   }
 }
 
@@ -205,8 +220,8 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(
 using OptT = c10::optional<torch::Tensor>;
 
 // x_scale, w_scale: both (e4m3 bytes) or neither (bf16).
-Product product_of(const torch::Tensor& x, const torch::Tensor& w, int64_t N,
-                   int columns, const OptT& x_scale, const OptT& w_scale) {
+Product product_of(const torch::Tensor& x, const torch::Tensor& w,
+                   const OptT& x_scale, const OptT& w_scale) {
   const bool f8 = x_scale.has_value();
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.is_cuda() &&
@@ -214,10 +229,11 @@ Product product_of(const torch::Tensor& x, const torch::Tensor& w, int64_t N,
                 (uintptr_t)t.data_ptr() % 16 == 0);
   Product m{};
   m.M = x.size(0);
-  m.N = N;
+  m.N = w.size(0);
   m.row = x.size(1) * (f8 ? 1 : 2);
-  TORCH_CHECK(w.size(1) == x.size(1) && m.M >= 1 && m.M <= 64);
-  TORCH_CHECK(m.N >= 4 && m.N % 4 == 0 && m.row >= CB && m.row % CB == 0);
+  TORCH_CHECK(w.size(1) == x.size(1) && m.M >= 1 && m.M <= 128);
+  const Shape s = m.M <= 64 ? FEW : MORE;
+  TORCH_CHECK(m.N >= 4 && m.N % 4 == 0 && m.row > 0 && m.row % s.chunk == 0);
   TORCH_CHECK(w_scale.has_value() == f8);
   if (f8) {
     for (const auto& t : {*x_scale, *w_scale})
@@ -226,38 +242,44 @@ Product product_of(const torch::Tensor& x, const torch::Tensor& w, int64_t N,
     m.xs = x_scale->data_ptr<float>();
     m.ws = w_scale->data_ptr<float>();
   }
-  m.n_tiles = cdiv(m.N, columns);
-  m.chunks = m.per = m.row / CB;
+  m.n_tiles = cdiv(m.N, s.columns);
+  m.chunks = m.per = m.row / s.chunk;
+  m.want = s.want;
   return m;
 }
 
-// Stretches of the inner dimension: about WANT workgroups in all.
+// Stretches of the inner dimension: about m.want workgroups in all.
 int cut(Product& m) {
   m.per = cdiv(m.chunks,
-               std::max(1, std::min(WANT / m.n_tiles, m.chunks)));
+               std::max(1, std::min(m.want / m.n_tiles, m.chunks)));
   return cdiv(m.chunks, m.per);
 }
 
-template <int NW, bool GLU, bool F8>
+template <bool GLU, bool F8>
 void run_as(uint16_t* out, float* sums, const torch::Tensor& x,
             const torch::Tensor& w, const Product& m, int stretches) {
-#define HELIX_GR(MI)                                                         \
-  hipLaunchKernelGGL((gemm_rows_kernel<MI, NW, GLU, F8>),                    \
+#define HELIX_GR(MI, NI, NW, CB)                                             \
+  hipLaunchKernelGGL((gemm_rows_kernel<MI, NI, NW, CB, GLU, F8>),            \
                      dim3(m.n_tiles * stretches), dim3(NW * WAVE), 0,        \
                      at::hip::getCurrentHIPStream(), out, sums,              \
                      (const char*)x.data_ptr(), (const char*)w.data_ptr(), m)
-  if (m.M <= 16) HELIX_GR(1);
-  else if (m.M <= 32) HELIX_GR(2);
-  else if (m.M <= 48) HELIX_GR(3);
-  else HELIX_GR(4);
+  constexpr int NI = GLU ? 2 : 1, NW = GLU ? 2 : 4;
+  if (m.M <= 16) HELIX_GR(1, NI, NW, 512);
+  else if (m.M <= 32) HELIX_GR(2, NI, NW, 512);
+  else if (m.M <= 48) HELIX_GR(3, NI, NW, 512);
+  else if (m.M <= 64) HELIX_GR(4, NI, NW, 512);
+  else if constexpr (!GLU) {
+    if (m.M <= 96) HELIX_GR(6, 2, 4, 256);
+    else HELIX_GR(8, 2, 4, 256);
+  }
 #undef HELIX_GR
 }
 
-template <int NW, bool GLU>
+template <bool GLU>
 void run(uint16_t* out, float* sums, const torch::Tensor& x,
          const torch::Tensor& w, const Product& m, int stretches) {
-  if (m.xs != nullptr) run_as<NW, GLU, true>(out, sums, x, w, m, stretches);
-  else run_as<NW, GLU, false>(out, sums, x, w, m, stretches);
+  if (m.xs != nullptr) run_as<GLU, true>(out, sums, x, w, m, stretches);
+  else run_as<GLU, false>(out, sums, x, w, m, stretches);
 }
 
 torch::Tensor sums_for(const torch::Tensor& x, const Product& m,
@@ -277,16 +299,16 @@ void check_out(const torch::Tensor& out, const Product& m) {
 // Sums [stretches, M, N] for a reader that adds them up.
 torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
                              OptT w_scale) {
-  Product m = product_of(x, w, w.size(0), 64, x_scale, w_scale);
+  Product m = product_of(x, w, x_scale, w_scale);
   const int stretches = cut(m);
   torch::Tensor sums = sums_for(x, m, stretches);
-  run<4, false>(nullptr, sums.data_ptr<float>(), x, w, m, stretches);
+  run<false>(nullptr, sums.data_ptr<float>(), x, w, m, stretches);
   return sums;
 }
 
 void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
                OptT x_scale, OptT w_scale) {
-  Product m = product_of(x, w, w.size(0), 64, x_scale, w_scale);
+  Product m = product_of(x, w, x_scale, w_scale);
   check_out(out, m);
   if (bias.has_value()) {
     TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 &&
@@ -296,11 +318,11 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
   const int stretches = cut(m);
   uint16_t* o = (uint16_t*)out.data_ptr();
   if (stretches == 1) {
-    run<4, false>(o, nullptr, x, w, m, 1);
+    run<false>(o, nullptr, x, w, m, 1);
     return;
   }
   torch::Tensor sums = sums_for(x, m, stretches);
-  run<4, false>(nullptr, sums.data_ptr<float>(), x, w, m, stretches);
+  run<false>(nullptr, sums.data_ptr<float>(), x, w, m, stretches);
   const int64_t MN = (int64_t)m.M * m.N;
   hipLaunchKernelGGL(gemm_join_kernel, dim3((MN + 1023) / 1024), dim3(256), 0,
                      at::hip::getCurrentHIPStream(), o,
@@ -310,8 +332,10 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
 // out[M,N] = silu(x w[:N]^T) * (x w[N:]^T)
 void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    OptT x_scale, OptT w_scale) {
-  TORCH_CHECK(w.size(0) % 2 == 0);
-  Product m = product_of(x, w, w.size(0) / 2, 32, x_scale, w_scale);
+  Product m = product_of(x, w, x_scale, w_scale);
+  TORCH_CHECK(m.M <= 64 && m.N % 8 == 0);
+  m.N /= 2;                                   // 32 columns of a workgroup
+  m.n_tiles = cdiv(m.N, 32);
   check_out(out, m);
-  run<2, true>((uint16_t*)out.data_ptr(), nullptr, x, w, m, 1);
+  run<true>((uint16_t*)out.data_ptr(), nullptr, x, w, m, 1);
 }
