@@ -454,10 +454,33 @@ def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     rows, else [M, N] in x's type. Wide matrices fill the chip without
     stretches, and 64 rows of 16384 sums are more bytes than they save. At 64
     rows of 6144 x 4096 it is 17.6 us against the library's 18.0, at 128 rows
-    20 against 25."""
+    20 against 25. From 129 rows on see _sums_tile."""
     if _rows_fit(x, w) and w.shape[0] <= 8192:
         return _native().gemm_rows_sums(x, w, None, None)
+    tile = _sums_tile(*x.shape, w.shape[0]) if x.dim() == 2 else 0
+    if tile and _rows_fit(x, w, SUMS_MAX_M):
+        return _native().gemm_bf16_sums(x, w, tile)
     return linear(x, w)
+
+
+SUMS_MAX_M = 2048
+
+
+def _sums_tile(M: int, K: int, N: int) -> int:
+    """Tile of gemm_bf16_sums for M > 128 rows, 0 where the library is as
+    fast. A product that is three times as deep as wide has too few tiles to
+    fill the chip without stretches. With the norm that reads the result, us
+    of 4096 x 14336 and the library's: 200 rows 50 and 61 (128), 512 rows 80
+    and 97, 1024 rows 128 and 145, 1540 rows 197 and 337 (256). Between, too
+    few workgroups are left over: 768 rows 113 and 117, 1400 rows 185 and
+    181; products as deep as wide gain nothing (512 rows of 4096 x 4096: 36
+    and 35)."""
+    if not 128 < M <= SUMS_MAX_M or K < 3 * N or N > 8192:
+        return 0
+    tiles = -(-M // 256) * -(-N // 256)
+    if M > 256 and tiles <= 256 and tiles * min(256 // tiles, 8) >= 208:
+        return 256
+    return 128 if M <= 640 else 0
 
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -53,6 +53,7 @@ void sample_tokens_ext(torch::Tensor out, torch::Tensor logits,
                        c10::optional<torch::Tensor> row_map);
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, int64_t act);
+torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile);
 void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                       c10::optional<torch::Tensor> bias,
                       c10::optional<torch::Tensor> scratch, int64_t split_k,
@@ -103,6 +104,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tokens_ext", &sample_tokens_ext,
         "Fused top-k/top-p/penalty Gumbel sampling (histogram threshold)");
   m.def("gemm_bf16", &gemm_bf16, "MFMA bf16 GEMM: x @ w^T (+bias, act)");
+  m.def("gemm_bf16_sums", &gemm_bf16_sums,
+        "x @ w^T, stretches of the inner dimension apart");
   m.def("gemm_skinny_bf16", &gemm_skinny_bf16,
         "Skinny-M decode GEMM: split-K + XCD-chunked tile swizzle");
   m.def("gemm_rows", &gemm_rows, "x @ w^T (+bias) of at most 64 rows");

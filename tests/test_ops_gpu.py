@@ -655,6 +655,31 @@ def test_gemm_rows(m, n, k):
             atol=5e-5)
 
 
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (257, 260, 192),
+                                   (130, 516, 4160), (700, 1024, 1088)])
+def test_gemm_bf16_sums(m, n, k, tile):
+    """One step, fewer steps than buffers, stretches of unequal length,
+    remainders of rows and columns."""
+    torch.manual_seed(29)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    sums = ops._native().gemm_bf16_sums(x, w, tile)
+    want = x.double() @ w.double().t()
+    torch.testing.assert_close(sums.double().sum(0), want, rtol=1e-5,
+                               atol=2e-5)       # fp32 sums of k products
+
+
+def test_gemm_bf16_pair():
+    """256 x 256 tiles by two halves: 192 of them and a long inner dimension."""
+    torch.manual_seed(30)
+    x = torch.randn(4000, 2112, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(3002, 2112, dtype=torch.bfloat16, device=DEV) / 46
+    got = ops.gemm_bf16(x, w, None)
+    torch.testing.assert_close(got.double(), x.double() @ w.double().t(),
+                               rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 8, 512), (17, 72, 1024),
                                    (48, 256, 4096), (64, 4104, 1536),
                                    (96, 136, 512), (127, 264, 1024)])
