@@ -23,11 +23,13 @@
 // barriers per 128 tokens and the value product waited for the softmax of all
 // heads. Measured with 32 heads on 8, 16-token pages in random order, merge
 // included (us before -> now, TB/s now):
-//   1 row of 777            22.5 -> 10.3      (launches and latency)
-//   8 of 300..6000, window  89 -> 32          3.2
-//   61 of 1000..4096        345 -> 134        4.7
-//   512 of 513..640         279 -> 226        5.35
-//   24 of 4000..16000, fp8  487 -> 117        4.4
+//   1 row of 777            22.5 -> 10.0      (launches and latency)
+//   8 of 300..6000, window  89 -> 31          3.3
+//   61 of 1000..4096        345 -> 127        5.0
+//   512 of 513..640         279 -> 209        5.8
+//   24 of 4000..16000, fp8  487 -> 113        4.5
+// Values by ordinary loads: 133 us for the 61, 226 for the 512; keys by
+// streaming loads as well: 128 and 218.
 // A large read-only sum reaches 6.1 TB/s. TARGET of 512 to 2048 is within 5%
 // of each other; the results' distance from 64 bits is what it was (their
 // rounding to bf16).
@@ -305,10 +307,12 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
     for (int i = 0; i < VG; ++i)
       row[i] = (const char*)vc + row_at(vp[i], tile * KT + key_v + i) +
                lo * DPL * EB;
+    // read once, by whole lines: they need not stay in the caches (keys come
+    // by half lines and do)
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      vr[i] = *reinterpret_cast<const VRaw*>(row[i % VG] +
-                                             (i / VG) * D * EB);
+      vr[i] = __builtin_nontemporal_load(reinterpret_cast<const VRaw*>(
+          row[i % VG] + (i / VG) * D * EB));
   };
 
   float acc[G][DPL], m_run[QS], l[QS];
@@ -531,8 +535,8 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   m.limit = cdiv((int)max_len_hint, UNIT) * UNIT;
   m.mul = (float)scale * LOG2E;
   // Nothing to cut where a row is at most a unit long, nor where the rows
-  // alone fill the chip twice and none can be long: 512 rows of 513..640 take
-  // 226 us without and 231 with cuts, most of it the merge launch.
+  // alone fill the chip twice and none can be long: cuts cost 512 rows of
+  // 513..640 5 us, most of it the merge launch.
   const int most = cdiv((int)(window > 0 ? std::min(max_len_hint, window + KT)
                                          : max_len_hint), UNIT);
   m.split = m.max_parts > 1 && most > 1 &&
