@@ -1,33 +1,40 @@
 // Flash-attention prefill (varlen, causal/bidirectional, GQA) for CDNA4.
 //
 // Replaces the prefill attention the reference delegates to vLLM. Bound by
-// instruction issue: of a wave's 2500 cycles per tile the matrix cores have
-// 1020 and the vector ALU 1250 (half of it exponentials), and counters show
-// that the two hardly overlap, neither within a wave (the next scores computed
-// beside the exponentials changed nothing) nor between the two waves of a SIMD
-// (nor did their priorities).
+// instruction issue and power: of a wave's 2200 cycles per tile the matrix
+// cores have 1020, and a SIMD issues one vector instruction in about 5 (170 a
+// tile, half of them for exponentials, and 64 more where a maximum grew); the
+// clock is at 1.85 GHz (on zeros 1 x 8192 takes 451 us instead of 606). LDS is
+// busy for a third. A third wave on a SIMD (tiles of 32 keys), the next scores
+// computed beside the exponentials and two halves of waves a phase apart
+// change nothing or cost.
 //
-//  - A workgroup has 128 queries of one head, each of its 4 waves 32 of them.
-//    Scores are computed transposed (key x query): a lane has one query, its
-//    statistics cost two lane swaps, and 8 neighbouring keys of its weights
-//    are an operand of the value product as they lie.
+//  - A workgroup has 128 queries of one head, each of its 4 waves 32 of them,
+//    in products of 32x32. Scores are computed transposed (key x query): a lane
+//    has one query, its statistics cost one lane swap, and 8 neighbouring keys
+//    of its weights are an operand of the value product as they lie.
 //  - Tiles of 64 keys and values go straight to LDS, the next one while the
 //    last is worked on, with one barrier a tile. Rows lie as in memory; their
 //    16-byte pieces are stored crosswise, so that keys leave LDS as operands
 //    and values through the transposing load without bank conflicts.
+//  - The loop has a body for each of the two buffers, and places in memory are
+//    unsigned 32-bit offsets from a scalar base: no addresses are computed in
+//    it.
 //  - All tiles of a (sequence, head) run on one XCD, the latest, which see
 //    the most keys, first.
 //
-// The kernel before had 64 queries, stored values transposed element by
-// element and passed weights through LDS. 32 heads on 8 of 128, us before ->
-// now (TFLOP/s now): 1 x 8192 2551 -> 645 (850), 8 x 2048 1918 -> 413 (665),
-// 31 of 400..620 440 -> 188 (384), 1500 behind 5001 with a window of 4096
-// 466 -> 173 (582). 12 heads of 64, 64 texts of 20..500: 178 -> 68. Workgroups
-// of 64 queries (2 waves) take 1.1 to 1.8 times as long from 100 queries on,
-// and no less time below. The distance from 64 bits is what it was.
+// 32 heads on 8 of 128, us of the first kernel (64 queries, values transposed
+// element by element) -> products of 16x16 with addresses computed per tile
+// (340 vector instructions) -> now (TFLOP/s now): 1 x 8192 2551 -> 645 -> 606
+// (907), 8 x 2048 1918 -> 413 -> 395 (695), 31 of 400..620 440 -> 188 -> 183
+// (393), 1500 behind 5001 with a window of 4096 466 -> 173 -> 159 (632). 12
+// heads of 64, 64 texts of 20..500: 178 -> 68 -> 62. Workgroups of 64 queries
+// (2 waves) took 1.1 to 1.8 times as long from 100 queries on, and no less time
+// below. The distance from 64 bits is what it was.
 //
-// MFMA fragment layouts (gfx950, f32_16x16x32_bf16), hi = lane / 16,
-// lo = lane % 16: A[lo][8 hi + i], B[8 hi + i][lo], D[4 hi + r][lo].
+// MFMA fragment layouts (gfx950, f32_32x32x16_bf16), hi = lane / 32,
+// lo = lane % 32: A[lo][8 hi + i], B[8 hi + i][lo],
+// D[8 (r / 4) + 4 hi + r % 4][lo].
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -53,13 +60,18 @@ struct Prefill {
   float mul;                   // |scale| * log2(e)
 };
 
-__device__ __forceinline__ float max_over_groups(float v) {
+typedef __attribute__((ext_vector_type(16))) float floatx16;
+
+__device__ __forceinline__ floatx16 mfma32(u16x8 a, u16x8 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+      __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+      0);
+}
+
+__device__ __forceinline__ float max_over_halves(float v) {
   const unsigned u = __float_as_uint(v);
   const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const float x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const unsigned w = __float_as_uint(x);
-  const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
 
 // Four rows of one column from LDS: the 16 lanes of a quarter wave name 4
@@ -71,11 +83,12 @@ __device__ __forceinline__ u16x4 ld_tr4(const uint16_t* p) {
       (__attribute__((address_space(3))) i16x4*)p));
 }
 
-// Piece p of row r lies at p ^ cross(r): the 16 rows 8 a + 4 s + b (a, b < 4)
-// of a score operand, and the 16 of a value operand, meet every bank equally.
+// Piece p of row r lies at p ^ cross(r): 16 rows of a score operand, and 4
+// rows of 4 pieces of a value operand, meet every bank equally.
 template <int D>
 __device__ __forceinline__ int cross(int r) {
-  return D == 128 ? (r & 3) | (r >> 1 & 12) : (r >> 1 & 1) | (r >> 2 & 6);
+  return D == 128 ? (r & 3) << 2 | (r >> 2 & 3)
+                  : (r >> 1 & 1) << 2 | (r >> 2 & 3);
 }
 
 template <int D, bool CAUSAL>
@@ -83,7 +96,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     Prefill m) {
-  constexpr int NK = D / 32, NV = D / 16, PR = D / 8;
+  constexpr int NK = D / 16, NV = D / 32, PR = D / 8;
   constexpr int LOADS = KT * PR / NT;
   __shared__ __attribute__((aligned(16))) uint16_t kl[2][KT * D];
   __shared__ __attribute__((aligned(16))) uint16_t vl[2][KT * D];
@@ -98,17 +111,18 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
   const int key0 = m.cu_k[b], klen = m.cu_k[b + 1] - key0;
   const int ctx = klen - qlen;                // cached tokens before
 
-  const int tid = threadIdx.x, wid = tid / WAVE, lane = tid & (WAVE - 1);
-  const int lo = lane & 15, hi = lane >> 4;
-  u16x8 qf[2][NK];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int qi = min(q0 + wid * 32 + u * 16 + lo, qlen - 1);
-    const uint16_t* qr = q + (row0 + qi) * m.q_stride + h * D + hi * 8;
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int lo = lane & 31, hi = lane >> 5;
+  u16x8 qf[NK];
+  const int qi = q0 + wid * 32 + lo;          // of this lane
+  {
+    const uint16_t* qr =
+        q + (row0 + min(qi, qlen - 1)) * m.q_stride + h * D + hi * 8;
 #pragma unroll
     for (int c = 0; c < NK; ++c) {
-      qf[u][c] = ld_u16x8(qr + c * 32);
-      if (m.flip) qf[u][c] ^= (uint16_t)0x8000;
+      qf[c] = ld_u16x8(qr + c * 16);
+      if (m.flip) qf[c] ^= (uint16_t)0x8000;
     }
   }
 
@@ -116,15 +130,16 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
   const uint16_t* vb = v + key0 * m.v_stride + g * D;
   // This lane's pieces of a tile: where they lie is the same in every tile but
   // a partial one, whose rows past the end repeat the last and are masked.
-  int ko[LOADS], vo[LOADS];
-  auto places = [&](int rows, int64_t stride, int* o) {
+  unsigned ko[LOADS], vo[LOADS];
+  auto places = [&](int rows, int64_t stride, unsigned* o) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int e = (i * NW + wid) * WAVE + lane, r = e / PR;
       o[i] = (min(r, rows - 1) * (int)stride + (e % PR ^ cross<D>(r)) * 8) * 2;
+      asm volatile("" : "+v"(o[i]));         // kept, not computed again
     }
   };
-  auto fetch = [&](const uint16_t* base, int64_t stride, int* o, int t,
+  auto fetch = [&](const uint16_t* base, int64_t stride, unsigned* o, int t,
                    uint16_t* lds) {
     if (t + KT > klen) places(klen - t, stride, o);
     const char* from = (const char*)(base + t * stride);
@@ -138,161 +153,144 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
   };
   places(KT, m.k_stride, ko);
   places(KT, m.v_stride, vo);
-  // where this lane reads, within 16 rows of keys and 4 of values
-  int ka[NK], va[NV];
-  const int kr = (lo >> 2) * 8 + (lo & 3), vr = hi * 8 + (lo >> 2);
+  // Where this lane reads. Keys: row 8 a + 4 h + b of a score operand is key
+  // 16 (a / 2) + 8 h + 4 (a % 2) + b of its 32, so that a lane's scores 8 i..
+  // are the neighbouring keys 16 i + 8 hi.., an operand of the value product.
+  // Values: columns 32 d.. of keys 8 hi.. and of the 4 behind them.
+  int ka[NK], va[NV][2];
+  const int kr = (lo >> 4) * 16 + (lo >> 2 & 1) * 8 + (lo >> 3 & 1) * 4 +
+                 (lo & 3);
 #pragma unroll
   for (int c = 0; c < NK; ++c)
-    ka[c] = kr * D + ((c * 4 + hi) ^ cross<D>(kr)) * 8;
+    ka[c] = kr * D + ((c * 2 + hi) ^ cross<D>(kr)) * 8;
 #pragma unroll
   for (int d = 0; d < NV; ++d)
-    va[d] = vr * D + ((d * 2 + (lo >> 1 & 1)) ^ cross<D>(vr)) * 8 +
-            (lo & 1) * 4;
-
-  floatx4 acc[NV][2];
-  float m_run[2] = {NEG, NEG}, l[2] = {0.f, 0.f};
 #pragma unroll
-  for (int d = 0; d < NV; ++d) acc[d][0] = acc[d][1] = floatx4{0, 0, 0, 0};
+    for (int j = 0; j < 2; ++j) {
+      const int r = hi * 8 + j * 4 + (lo >> 2 & 3);
+      va[d][j] = r * D +
+                 ((d * 4 + (lo >> 4) * 2 + (lo >> 1 & 1)) ^ cross<D>(r)) * 8 +
+                 (lo & 1) * 4;
+    }
+
+  floatx16 acc[NV];
+  float m_run = NEG, l = 0.f;
+#pragma unroll
+  for (int d = 0; d < NV; ++d) acc[d] = floatx16{};
   const int last = CAUSAL ? min(klen, ctx + q0 + QT) : klen;
   const int qa = ctx + q0 + wid * 32, qz = qa + 31;       // of this wave
   const bool windowed = CAUSAL && m.window > 0;
   int t = windowed ? max(0, ctx + q0 - m.window + 1) / KT * KT : 0;
 
-  // scores of 64 keys: [32 keys][half][query tile]
-  auto product = [&](const uint16_t* keys, floatx4 (*s)[2][2]) {
-#pragma unroll
-    for (int w = 0; w < 2; ++w)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        s[w][j][0] = s[w][j][1] = floatx4{0, 0, 0, 0};
-#pragma unroll
-        for (int c = 0; c < NK; ++c) {
-          const u16x8 a = ld_u16x8(keys + (w * 32 + j * 4) * D + ka[c]);
-          s[w][j][0] = mfma16(a, qf[0][c], s[w][j][0]);
-          s[w][j][1] = mfma16(a, qf[1][c], s[w][j][1]);
-        }
-      }
-  };
   if (t < last) {
     fetch(kb, m.k_stride, ko, t, kl[0]);
     fetch(vb, m.v_stride, vo, t, vl[0]);
   }
-  for (int buf = 0; t < last; t += KT, buf ^= 1) {
+  auto step = [&](auto half) {
+    constexpr int buf = decltype(half)::value;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (t + KT < last) {
       fetch(kb, m.k_stride, ko, t + KT, kl[buf ^ 1]);
       fetch(vb, m.v_stride, vo, t + KT, vl[buf ^ 1]);
     }
-    if (CAUSAL && t > qz) continue;
-    floatx4 s[2][2][2];
-    product(kl[buf], s);
-    // operands leave LDS a group ahead of their products
-    __builtin_amdgcn_sched_group_barrier(DS_READ, 2 * NK, 0);
+    if (CAUSAL && t > qz) return;
+    floatx16 s[KT / 32];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      __builtin_amdgcn_sched_group_barrier(MFMA, 2 * NK, 0);
-      __builtin_amdgcn_sched_group_barrier(DS_READ, NK, 0);
+    for (int w = 0; w < KT / 32; ++w) s[w] = floatx16{};
+#pragma unroll
+    for (int c = 0; c < NK; ++c)
+#pragma unroll
+      for (int w = 0; w < KT / 32; ++w)
+        s[w] = mfma32(ld_u16x8(kl[buf] + w * 32 * D + ka[c]), qf[c], s[w]);
+    // operands leave LDS a group ahead of their products
+    __builtin_amdgcn_sched_group_barrier(DS_READ, 4, 0);
+#pragma unroll
+    for (int i = 0; i < NK - 2; ++i) {
+      __builtin_amdgcn_sched_group_barrier(MFMA, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(DS_READ, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(MFMA, 4 * NK, 0);
+    __builtin_amdgcn_sched_group_barrier(MFMA, 4, 0);
 
     const bool edge = (CAUSAL && t + KT - 1 > qa) || t + KT > klen ||
                       (windowed && t <= qz - m.window);
     if (edge) {
+      const int at = ctx + qi;
+      const int low = windowed ? at - m.window : -1;
+      const int top = CAUSAL ? min(at, klen - 1) : klen - 1;
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int qi = qa + u * 16 + lo;
-        const int low = windowed ? qi - m.window : -1;
-        const int top = CAUSAL ? min(qi, klen - 1) : klen - 1;
+      for (int w = 0; w < KT / 32; ++w)
 #pragma unroll
-        for (int w = 0; w < 2; ++w)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int key = t + w * 32 + hi * 8 + i;
-            if (key > top || key <= low) s[w][i >> 2][u][i & 3] = NEG;
-          }
-      }
+        for (int i = 0; i < 16; ++i) {
+          const int key = t + w * 32 + (i >> 3) * 16 + hi * 8 + (i & 7);
+          if (key > top || key <= low) s[w][i] = NEG;
+        }
     }
-    float mx[2], base[2];
-    bool stay = true;
+    float mx = m_run;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      mx[u] = m_run[u];
+    for (int w = 0; w < KT / 32; ++w)
 #pragma unroll
-      for (int w = 0; w < 2; ++w)
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[w][i]);
+    mx = max_over_halves(mx);
+    if (!__all(mx == m_run)) {
+      const float corr = __builtin_amdgcn_exp2f((m_run - mx) * m.mul);
+      l *= corr;
+      m_run = mx;
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          mx[u] = fmaxf(mx[u], s[w][i >> 2][u][i & 3]);
-      mx[u] = max_over_groups(mx[u]);
-      stay = stay && mx[u] == m_run[u];
-    }
-    if (!__all(stay)) {
+      for (int d = 0; d < NV; ++d)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const float corr = __builtin_amdgcn_exp2f((m_run[u] - mx[u]) * m.mul);
-        l[u] *= corr;
-        m_run[u] = mx[u];
-#pragma unroll
-        for (int d = 0; d < NV; ++d)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[d][u][i] *= corr;
-      }
+        for (int i = 0; i < 16; ++i) acc[d][i] *= corr;
     }
     // a query that has seen no key yet keeps weights of exactly zero
+    const float base = m_run <= NEG ? 0.f : m_run * m.mul;
+    u16x8 pf[KT / 16];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-      base[u] = m_run[u] <= NEG ? 0.f : m_run[u] * m.mul;
-    u16x8 pf[2][2];
-    auto weights = [&]() {
+    for (int k = 0; k < KT / 16; ++k) {
+      float p[8];
 #pragma unroll
-      for (int w = 0; w < 2; ++w)
+      for (int i = 0; i < 8; ++i) {
+        p[i] = __builtin_amdgcn_exp2f(
+            fmaf(s[k >> 1][(k & 1) * 8 + i], m.mul, -base));
+        l += p[i];
+      }
+      pf[k] = pack8(p);
+    }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          float p[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            p[i] = __builtin_amdgcn_exp2f(
-                fmaf(s[w][i >> 2][u][i & 3], m.mul, -base[u]));
-            l[u] += p[i];
-          }
-          pf[w][u] = pack8(p);
-        }
-    };
-    weights();
-#pragma unroll
-    for (int w = 0; w < 2; ++w)
+    for (int k = 0; k < KT / 16; ++k)
 #pragma unroll
       for (int d = 0; d < NV; ++d) {
-        const uint16_t* at = vl[buf] + w * 32 * D + va[d];
-        const u16x4 x = ld_tr4(at), y = ld_tr4(at + 4 * D);
+        const u16x4 x = ld_tr4(vl[buf] + k * 16 * D + va[d][0]);
+        const u16x4 y = ld_tr4(vl[buf] + k * 16 * D + va[d][1]);
         const u16x8 a = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-        acc[d][0] = mfma16(a, pf[w][0], acc[d][0]);
-        acc[d][1] = mfma16(a, pf[w][1], acc[d][1]);
+        acc[d] = mfma32(a, pf[k], acc[d]);
       }
-    __builtin_amdgcn_sched_group_barrier(DS_READ, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(DS_READ, 4, 0);
 #pragma unroll
-    for (int i = 0; i < 2 * NV - 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(MFMA, 2, 0);
+    for (int i = 0; i < KT / 16 * NV - 2; ++i) {
+      __builtin_amdgcn_sched_group_barrier(MFMA, 1, 0);
       __builtin_amdgcn_sched_group_barrier(DS_READ, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(MFMA, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(MFMA, 2, 0);
+  };
+  while (t < last) {
+    step(std::integral_constant<int, 0>());
+    if ((t += KT) >= last) break;
+    step(std::integral_constant<int, 1>());
+    t += KT;
   }
 
+  l += __shfl_xor(l, 32, WAVE);
+  if (qi >= qlen) return;
+  const float f = 1.f / fmaxf(l, 1e-20f);
+  uint16_t* dst = out + ((int64_t)(row0 + qi) * m.Hq + h) * D + hi * 4;
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    l[u] += __shfl_xor(l[u], 16, WAVE);
-    l[u] += __shfl_xor(l[u], 32, WAVE);
-    const float f = 1.f / fmaxf(l[u], 1e-20f);
-    const int qi = q0 + wid * 32 + u * 16 + lo;
-    if (qi >= qlen) continue;
-    uint16_t* dst = out + ((int64_t)(row0 + qi) * m.Hq + h) * D + hi * 4;
+  for (int d = 0; d < NV; ++d)
 #pragma unroll
-    for (int d = 0; d < NV; ++d) {
-      const float x[4] = {acc[d][u][0] * f, acc[d][u][1] * f,
-                          acc[d][u][2] * f, acc[d][u][3] * f};
-      st_bf16x4(dst + d * 16, x);
+    for (int i = 0; i < 4; ++i) {
+      const float x[4] = {acc[d][i * 4] * f, acc[d][i * 4 + 1] * f,
+                          acc[d][i * 4 + 2] * f, acc[d][i * 4 + 3] * f};
+      st_bf16x4(dst + d * 32 + i * 8, x);
     }
-  }
 }
 
 // Rows of [T, H, D] with their heads side by side, 16-byte aligned, anywhere;
