@@ -154,6 +154,27 @@ def kv_fp8_dequant(t: torch.Tensor, dtype=torch.bfloat16) -> torch.Tensor:
     return t.view(torch.float8_e4m3fn).to(dtype)
 
 
+def gather_kv(k_cache: torch.Tensor, v_cache: torch.Tensor,
+              blk: torch.Tensor, off: torch.Tensor, dtype=torch.bfloat16):
+    """Rows [T, Hkv, D] of a paged cache at offsets off of pages blk; e4m3
+    bytes become dtype."""
+    if (k_cache.is_cuda and dtype == torch.bfloat16 and
+            k_cache.dtype in (torch.bfloat16, torch.uint8) and
+            k_cache.shape[3] % 8 == 0 and
+            all(c.is_contiguous() and c.data_ptr() % 16 == 0
+                for c in (k_cache, v_cache)) and
+            blk.is_contiguous() and off.is_contiguous()):
+        k = torch.empty(blk.numel(), k_cache.shape[1], k_cache.shape[3],
+                        dtype=dtype, device=k_cache.device)
+        v = torch.empty_like(k)
+        _native().gather_kv(k, v, k_cache, v_cache, blk, off)
+        return k, v
+    k, v = k_cache[blk, :, off], v_cache[blk, :, off]
+    if k.dtype == torch.uint8:
+        k, v = kv_fp8_dequant(k, dtype), kv_fp8_dequant(v, dtype)
+    return k, v
+
+
 def rope_qkv_cache(positions: torch.Tensor, qkv: torch.Tensor,
                    cos_sin: torch.Tensor, num_q: int, num_kv: int,
                    head_dim: int, kv_cache=None, slot_mapping=None,

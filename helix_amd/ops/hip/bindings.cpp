@@ -31,6 +31,8 @@ void gelu_tanh(torch::Tensor out, torch::Tensor x);
 void reshape_and_cache(torch::Tensor k, torch::Tensor v,
                        torch::Tensor k_cache, torch::Tensor v_cache,
                        torch::Tensor slot_mapping);
+void gather_kv(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
+               torch::Tensor v_cache, torch::Tensor blk, torch::Tensor off);
 void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                        torch::Tensor k_cache, torch::Tensor v_cache,
                        torch::Tensor block_tables, torch::Tensor seq_lens,
@@ -96,6 +98,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu_tanh", &gelu_tanh, "GELU (tanh approx)");
   m.def("reshape_and_cache", &reshape_and_cache,
         "Scatter K/V rows into paged cache");
+  m.def("gather_kv", &gather_kv, "Gather K/V rows from paged cache");
   m.def("paged_attn_decode", &paged_attn_decode,
         "Paged decode attention (GQA, flash-decoding partitions)");
   m.def("attn_prefill", &attn_prefill,

@@ -145,6 +145,27 @@ def test_reshape_and_cache():
     assert_close_bf16(vc, vc_ref, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("T,H,D,page", [
+    (1, 1, 8, 1), (5, 8, 128, 16), (300, 2, 64, 16), (33, 3, 40, 8),
+    (9, 40, 256, 4)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_gather_kv(T, H, D, page, fp8):
+    """Rows of pages, heads and lengths that do not fill a workgroup: the
+    same bits as indexing, and every finite e4m3 value exactly."""
+    torch.manual_seed(T)
+    kc, vc = (torch.randn(7, H, page, D, device="cuda").bfloat16()
+              for _ in range(2))
+    if fp8:
+        byte = torch.arange(kc.numel(), device="cuda").view(kc.shape) % 256
+        kc = torch.where(byte % 128 == 127, 0, byte).to(torch.uint8)
+        vc = kc.flip(0).contiguous()
+    blk = torch.randint(0, 7, (T,), device="cuda")
+    off = torch.randint(0, page, (T,), device="cuda")
+    for got, cache in zip(ops.gather_kv(kc, vc, blk, off), (kc, vc)):
+        want = cache[blk, :, off]
+        assert torch.equal(got, ops.kv_fp8_dequant(want) if fp8 else want)
+
+
 @pytest.mark.parametrize("hq,hkv,d,lens", [
     (32, 8, 128, [1, 17, 128, 63]),
     (8, 8, 128, [200]),
