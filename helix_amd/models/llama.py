@@ -189,11 +189,11 @@ class Attention(nn.Module):
             want_kv=want_kv)
         if mixed:
             n = meta.num_decode
-            o = torch.cat([
-                self._attend_decode(q[:n], kv_cache, meta.decode),
-                self._attend_prefill(q[n:], k[n:] if want_kv else None,
-                                     v[n:] if want_kv else None, kv_cache,
-                                     prefill)])
+            o = torch.empty_like(q)
+            self._attend_decode(q[:n], kv_cache, meta.decode, o[:n])
+            self._attend_prefill(q[n:], k[n:] if want_kv else None,
+                                 v[n:] if want_kv else None, kv_cache,
+                                 prefill, o[n:])
         elif meta.is_prefill:
             o = self._attend_prefill(q, k, v, kv_cache, meta)
         else:
@@ -204,11 +204,11 @@ class Attention(nn.Module):
             return parallel.tp_all_reduce(self.o_proj(o))
         return _project(self.o_proj, o, form)
 
-    def _attend_prefill(self, q, k, v, kv_cache, meta):
+    def _attend_prefill(self, q, k, v, kv_cache, meta, out=None):
         if meta.cu_seqlens_k is None:
             return ops.attn_prefill(q, k, v, meta.cu_seqlens,
                                     meta.max_seqlen, self.scale,
-                                    window=self.window)
+                                    window=self.window, out=out)
         # cached-prefix prefill: full-context K/V gathered from the paged
         # cache (new tokens were just written)
         k_all, v_all = ops.gather_kv(*kv_cache, meta.gather_blk,
@@ -216,14 +216,14 @@ class Attention(nn.Module):
         return ops.attn_prefill(q, k_all, v_all, meta.cu_seqlens,
                                 meta.max_seqlen, self.scale,
                                 window=self.window,
-                                cu_seqlens_k=meta.cu_seqlens_k)
+                                cu_seqlens_k=meta.cu_seqlens_k, out=out)
 
-    def _attend_decode(self, q, kv_cache, meta):
+    def _attend_decode(self, q, kv_cache, meta, out=None):
         k_cache, v_cache = kv_cache
         return ops.paged_attn_decode(q, k_cache, v_cache, meta.block_tables,
                                      meta.seq_lens, self.scale,
                                      meta.workspace, meta.max_len or None,
-                                     window=self.window)
+                                     window=self.window, out=out)
 
 
 class MLP(nn.Module):

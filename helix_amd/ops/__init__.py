@@ -251,19 +251,23 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                  cu_seqlens: torch.Tensor, max_seqlen: int,
                  scale: float, causal: bool = True,
                  window: int = 0,
-                 cu_seqlens_k: torch.Tensor | None = None) -> torch.Tensor:
+                 cu_seqlens_k: torch.Tensor | None = None,
+                 out: torch.Tensor | None = None) -> torch.Tensor:
     """Varlen attention. When cu_seqlens_k is given, q rows are the
     SUFFIX of each sequence (cached-prefix prefill): kv rows cover the
-    full context and causal positions are offset by klen - qlen."""
+    full context and causal positions are offset by klen - qlen. out: a
+    contiguous place for the result."""
     if cu_seqlens_k is None:
         cu_seqlens_k = cu_seqlens
     if q.is_cuda:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        if out is None:
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _native().attn_prefill(out, q, k, v, cu_seqlens, cu_seqlens_k,
                                max_seqlen, scale, causal, window)
         return out
-    return ref.attn_prefill(q, k, v, cu_seqlens, max_seqlen, scale, causal,
-                            window, cu_seqlens_k)
+    o = ref.attn_prefill(q, k, v, cu_seqlens, max_seqlen, scale, causal,
+                         window, cu_seqlens_k)
+    return o if out is None else out.copy_(o)
 
 
 # Tokens that decode attention cuts sequences in (must match UNIT in
@@ -286,9 +290,12 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor,
                       v_cache: torch.Tensor, block_tables: torch.Tensor,
                       seq_lens: torch.Tensor, scale: float,
                       workspace=None, max_len: int | None = None,
-                      window: int = 0) -> torch.Tensor:
+                      window: int = 0,
+                      out: torch.Tensor | None = None) -> torch.Tensor:
+    """out: a contiguous place for the result."""
     if q.is_cuda:
-        out = torch.empty_like(q)
+        if out is None:
+            out = torch.empty_like(q)
         if max_len is None:
             max_len = int(seq_lens.max())   # host sync — pass max_len to avoid
         if workspace is None:
@@ -303,8 +310,9 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor,
     if k_cache.dtype == torch.uint8:            # fp8 KV cache
         k_cache = kv_fp8_dequant(k_cache)
         v_cache = kv_fp8_dequant(v_cache)
-    return ref.paged_attn_decode(q, k_cache, v_cache, block_tables, seq_lens,
-                                 scale, window)
+    o = ref.paged_attn_decode(q, k_cache, v_cache, block_tables, seq_lens,
+                              scale, window)
+    return o if out is None else out.copy_(o)
 
 
 def sample_tokens(logits: torch.Tensor, temperatures: torch.Tensor,
