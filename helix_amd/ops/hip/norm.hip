@@ -3,8 +3,8 @@
 // Memory-bound: fully vectorized bf16x8 loads/stores (guide G13), fp32
 // accumulation, one workgroup per token row.
 //
-// Reference behavior: replaces the RMSNorm the reference delegates to vLLM
-// containers (see SURVEY.md §2.8 "RMSNorm, residual add").
+// Replaces the RMSNorm and the residual addition that the reference delegates
+// to vLLM's containers.
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
