@@ -62,7 +62,7 @@ void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                       int64_t act, int64_t swizzle);
 using OptT = c10::optional<torch::Tensor>;
 void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
-               OptT x_scale, OptT w_scale);
+               OptT x_scale, OptT w_scale, bool gelu);
 torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
                              OptT w_scale);
 void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -111,9 +111,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "x @ w^T, stretches of the inner dimension apart");
   m.def("gemm_skinny_bf16", &gemm_skinny_bf16,
         "Skinny-M decode GEMM: split-K + XCD-chunked tile swizzle");
-  m.def("gemm_rows", &gemm_rows, "x @ w^T (+bias) of at most 64 rows");
+  m.def("gemm_rows", &gemm_rows, "x @ w^T (+bias, GELU) of at most 128 rows",
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("bias"),
+        py::arg("x_scale"), py::arg("w_scale"), py::arg("gelu") = false);
   m.def("gemm_rows_sums", &gemm_rows_sums,
-        "x @ w^T of at most 64 rows, stretches of the inner dimension apart");
+        "x @ w^T of at most 128 rows, stretches of the inner dimension apart");
   m.def("gemm_rows_glu", &gemm_rows_glu,
         "silu(x @ gate^T) * (x @ up^T) of at most 64 rows");
   m.def("quantize_rows", &quantize_rows,

@@ -1,7 +1,7 @@
 // bf16 MFMA GEMM for gfx950: out[M,N] = act(x[M,K] @ w[N,K]^T + bias).
 //
-// The encoder's and the image model's projections (act: none or GELU, tanh),
-// and Llama's narrow ones at a few hundred rows, whose inner dimension is cut
+// The encoder's and the image model's projections (act: none or GELU, tanh) of
+// more than a few rows, and Llama's narrow ones at a few hundred rows, whose inner dimension is cut
 // into stretches that a later reader adds up (fp32 [stretch][M][N]).
 //
 // Bound by the matrix cores and by LDS reads, which take about as long. Tiles
@@ -27,6 +27,7 @@
 // scheduling hints for the reads from LDS gave nothing. Tile counts: 108 of
 // 256 against 432 of 128 (2304 x 3072 x 1024) 34 and 23; 144 of 128 against
 // 576 of 64 (2304 x 1024 x 1024) 14.8 and 12.9.
+#include "gelu.h"
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -52,12 +53,7 @@ __device__ __forceinline__ int xcd_chunk(int orig, int nwg) {
 
 __device__ __forceinline__ float finish(float v, float b, int gelu) {
   v += b;
-  if (!gelu) return v;
-  // v (1 + tanh u) / 2 = v / (1 + 2^-(2 u log2 e)), u = sqrt(2 / pi)
-  // (v + 0.044715 v^3)
-  constexpr float C = -2.f * 0.7978845608028654f * 1.4426950408889634f;
-  const float e = v * fmaf(v * v, C * 0.044715f, C);
-  return v * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(e));
+  return gelu ? gelu_tanh_f32(v) : v;
 }
 
 // What a workgroup does: its tile and its part of the inner dimension.

@@ -24,7 +24,9 @@
 // often, chunks are half as long and 256 workgroups are enough; matrices as
 // wide as 28672 are the library's there (52, here 66 us):
 //   M 128  20.0 (24.6)  15.5 (24.7)                   34.6 (73.9)
-// Adding them up in a launch takes 2.5 to 3 us more. The gated product
+// Adding them up in a launch, with bias and GELU, takes 2.5 to 3 us more; so do
+// the encoder's and the image model's products, with which by tiles in brackets
+// 8 rows of 6144 x 1024 take 7.6 (14.1) and 33 of 768 x 3072 7.3 (25.1). The gated product
 // replaces a launch of 4.5 us as well. Reading 28672 x 4096 at 44.5 us is 5.3
 // TB/s. Eight waves a workgroup, chunks half or twice as long, and for up to
 // 64 rows 32 columns a wave and 256 or 768 workgroups were each slower on most
@@ -34,6 +36,7 @@
 // 16x16x128 instruction with unity scales; the scales meet the fp32 sums of
 // every stretch. us at 32 rows of the four matrices, the tiles of gemm_fp8.hip
 // in brackets: 9.4 (49.5), 7.4 (51.6), 27.4 (53.9), 16.0 (158).
+#include "gelu.h"
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -198,10 +201,11 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
   }
 }
 
-// The sums of all stretches, in order.
+// The sums of all stretches, in order; then bias and GELU.
 __global__ __launch_bounds__(256) void gemm_join_kernel(
     uint16_t* __restrict__ out, const float* __restrict__ sums,
-    const uint16_t* __restrict__ bias, int64_t MN, int N, int stretches) {
+    const uint16_t* __restrict__ bias, int64_t MN, int N, int stretches,
+    bool gelu) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= MN) return;
   float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -214,6 +218,9 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(
   if (bias != nullptr)
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] += bf16_to_f32(bias[i % N + j]);
+  if (gelu)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_f32(v[j]);
   st_bf16x4(out + i, v);
 }
 
@@ -307,7 +314,7 @@ torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
 }
 
 void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
-               OptT x_scale, OptT w_scale) {
+               OptT x_scale, OptT w_scale, bool gelu) {
   Product m = product_of(x, w, x_scale, w_scale);
   check_out(out, m);
   if (bias.has_value()) {
@@ -317,7 +324,7 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
   }
   const int stretches = cut(m);
   uint16_t* o = (uint16_t*)out.data_ptr();
-  if (stretches == 1) {
+  if (stretches == 1 && !gelu) {
     run<false>(o, nullptr, x, w, m, 1);
     return;
   }
@@ -326,7 +333,8 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
   const int64_t MN = (int64_t)m.M * m.N;
   hipLaunchKernelGGL(gemm_join_kernel, dim3((MN + 1023) / 1024), dim3(256), 0,
                      at::hip::getCurrentHIPStream(), o,
-                     sums.data_ptr<float>(), m.bias, MN, m.N, stretches);
+                     sums.data_ptr<float>(), m.bias, MN, m.N, stretches,
+                     gelu);
 }
 
 // out[M,N] = silu(x w[:N]^T) * (x w[N:]^T)

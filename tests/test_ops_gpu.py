@@ -634,6 +634,27 @@ def test_gemm_skinny_bf16(m, n, k):
     assert_close_bf16(got2, want2, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 256), (8, 6144, 1024), (64, 72, 768), (65, 72, 768),
+    (128, 256, 512), (129, 256, 512), (3, 32776, 256)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_gemm_bf16_few_rows(m, n, k, act):
+    """Streamed and by tiles, at the lines between them; so wide that there is
+    one stretch."""
+    torch.manual_seed(m)
+    x = torch.randn(m, k, dtype=torch.bfloat16)
+    w = torch.randn(n, k, dtype=torch.bfloat16) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16)
+    want = x.float() @ w.float().t() + b.float()
+    if act:
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    with torch.inference_mode():
+        got = ops.gemm_bf16(x.to(DEV), w.to(DEV), b.to(DEV), act)
+    # fp32 sums of k products and GELU's exponential, the rounding to bf16
+    torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
+                               atol=2e-5)
+
+
 @pytest.mark.parametrize("m", [1, 15, 16, 17, 33, 48, 64, 65, 96, 97, 128])
 @pytest.mark.parametrize("n,k", [(8, 256), (72, 512), (4104, 2304),
                                  (256, 4096)])
