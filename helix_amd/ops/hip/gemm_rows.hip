@@ -36,7 +36,7 @@
 // 16x16x128 instruction with unity scales; the scales meet the fp32 sums of
 // every stretch. us at 32 rows of the four matrices, the tiles of gemm_fp8.hip
 // in brackets: 9.4 (49.5), 7.4 (51.6), 27.4 (53.9), 16.0 (158).
-#include "gelu.h"
+#include "gemm_join.h"
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -199,29 +199,6 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
       st_bf16x4(out + (int64_t)r * m.N + n, v);
     }
   }
-}
-
-// The sums of all stretches, in order; then bias and GELU.
-__global__ __launch_bounds__(256) void gemm_join_kernel(
-    uint16_t* __restrict__ out, const float* __restrict__ sums,
-    const uint16_t* __restrict__ bias, int64_t MN, int N, int stretches,
-    bool gelu) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= MN) return;
-  float v[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = 0; s < stretches; ++s) {
-    const f32x4 p = *reinterpret_cast<const f32x4*>(sums + s * MN + i);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] += p[j];
-  }
-  if (bias != nullptr)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] += bf16_to_f32(bias[i % N + j]);
-  if (gelu)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_f32(v[j]);
-  st_bf16x4(out + i, v);
 }
 
 using OptT = c10::optional<torch::Tensor>;

@@ -636,11 +636,12 @@ def test_gemm_skinny_bf16(m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [
     (1, 8, 256), (8, 6144, 1024), (64, 72, 768), (65, 72, 768),
-    (128, 256, 512), (129, 256, 512), (3, 32776, 256)])
+    (128, 256, 512), (129, 256, 512), (3, 32776, 256),
+    (130, 260, 3136), (640, 768, 3072), (641, 768, 3072), (2561, 1020, 4096)])
 @pytest.mark.parametrize("act", [0, 1])
 def test_gemm_bf16_few_rows(m, n, k, act):
-    """Streamed and by tiles, at the lines between them; so wide that there is
-    one stretch."""
+    """Streamed, by tiles and in stretches of tiles, at the lines between them;
+    so wide that there is one stretch."""
     torch.manual_seed(m)
     x = torch.randn(m, k, dtype=torch.bfloat16)
     w = torch.randn(n, k, dtype=torch.bfloat16) / k ** 0.5
