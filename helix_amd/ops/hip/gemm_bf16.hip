@@ -327,8 +327,14 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(w.size(1) == m.K);
   TORCH_CHECK(m.K % 64 == 0, "K must be a multiple of 64");
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous());
-  if (m.M == 0 || m.N == 0) return;
   if (bias.has_value()) m.bias = (const uint16_t*)bias->data_ptr();
+  if (m.M == 0 || m.N == 0) return;
+  if (m.K == 0) {              // no operands to load: act(bias)
+    const torch::Tensor b = bias.has_value() ? bias->reshape({1, m.N})
+                                             : at::zeros_like(out);
+    out.copy_(m.gelu ? at::gelu(b.to(torch::kFloat32), "tanh") : b);
+    return;
+  }
   uint16_t* o = (uint16_t*)out.data_ptr();
   const uint16_t* xp = (const uint16_t*)x.data_ptr();
   const uint16_t* wp = (const uint16_t*)w.data_ptr();

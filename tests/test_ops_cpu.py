@@ -4,6 +4,7 @@ These pin the semantics the HIP kernels are tested against.
 """
 import math
 
+import pytest
 import torch
 
 import helix_amd.ops as ops
@@ -131,3 +132,18 @@ def test_sliding_window_reference_consistency():
     # and differs from full attention (the window actually applies)
     full = ops.attn_prefill(q, k, v, cu, L, scale)
     assert not torch.allclose(full[-1].float(), pre[-1].float(), atol=1e-3)
+
+
+def _out(x, w):
+    return torch.empty(x.shape[0], w.shape[0], dtype=x.dtype)
+
+
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_bf16_without_inner_dimension(bias, act):
+    """act(bias), decided on the host: there is nothing to load."""
+    x, w = (torch.empty(n, 0, dtype=torch.bfloat16) for n in (3, 10))
+    b = torch.randn(20, dtype=torch.bfloat16)[::2] if bias else None
+    out = _out(x, w)
+    ops._native().gemm_bf16(out, x, w, b, act)
+    assert torch.equal(out, ref.gemm_bf16(x, w, b, act))
