@@ -319,6 +319,7 @@ int cut(Gemm& m) {
 
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, int64_t act) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2, "x and w are matrices");
   Gemm m{};
   m.M = x.size(0);
   m.K = x.size(1);
@@ -327,7 +328,18 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(w.size(1) == m.K);
   TORCH_CHECK(m.K % 64 == 0, "K must be a multiple of 64");
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous());
-  if (bias.has_value()) m.bias = (const uint16_t*)bias->data_ptr();
+  for (const auto& t : {x, w, out})
+    TORCH_CHECK(t.scalar_type() == torch::kBFloat16 &&
+                t.device() == x.device(), "bf16 on one device");
+  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == m.M &&
+              out.size(1) == m.N, "out is [M, N]");
+  if (bias.has_value()) {
+    TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 &&
+                bias->numel() == m.N && bias->device() == x.device(),
+                "a bias of N values in bf16");
+    bias = bias->contiguous();
+    m.bias = (const uint16_t*)bias->data_ptr();
+  }
   if (m.M == 0 || m.N == 0) return;
   if (m.K == 0) {              // no operands to load: act(bias)
     const torch::Tensor b = bias.has_value() ? bias->reshape({1, m.N})
@@ -335,6 +347,10 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     out.copy_(m.gelu ? at::gelu(b.to(torch::kFloat32), "tanh") : b);
     return;
   }
+  TORCH_CHECK(x.is_cuda(), "operands on the GPU");
+  // tiles are loaded 16 bytes at a time
+  if ((uintptr_t)x.data_ptr() % 16 != 0) x = x.clone();
+  if ((uintptr_t)w.data_ptr() % 16 != 0) w = w.clone();
   uint16_t* o = (uint16_t*)out.data_ptr();
   const uint16_t* xp = (const uint16_t*)x.data_ptr();
   const uint16_t* wp = (const uint16_t*)w.data_ptr();

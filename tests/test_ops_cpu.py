@@ -147,3 +147,23 @@ def test_gemm_bf16_without_inner_dimension(bias, act):
     out = _out(x, w)
     ops._native().gemm_bf16(out, x, w, b, act)
     assert torch.equal(out, ref.gemm_bf16(x, w, b, act))
+
+
+@pytest.mark.parametrize("case,says", [
+    ("bias", "a bias of N"), ("bias type", "a bias of N"),
+    ("type", "bf16 on one"), ("out", "out is"), ("host", "on the GPU")])
+def test_gemm_bf16_refuses(case, says):
+    """What the kernels would misread is refused before any launch."""
+    x = torch.zeros(3, 64, dtype=torch.bfloat16)
+    w = torch.zeros(10, 64, dtype=torch.bfloat16)
+    out, b = _out(x, w), torch.zeros(10, dtype=torch.bfloat16)
+    if case == "bias":
+        b = b[:1]
+    elif case == "bias type":
+        b = b.float()
+    elif case == "type":
+        x = x.half()
+    elif case == "out":
+        out = out[:, :8]
+    with pytest.raises(RuntimeError, match=says):
+        ops._native().gemm_bf16(out, x, w, b, 0)
