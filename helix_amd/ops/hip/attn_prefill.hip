@@ -38,6 +38,7 @@
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <cfloat>
 
 using namespace helix;
 
@@ -47,7 +48,8 @@ constexpr int NT = 256, NW = NT / WAVE;
 constexpr int QT = NW * 32;                   // queries of a workgroup
 constexpr int KT = 64;                        // keys of a tile
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr float NEG = -1e30f;
+// Before the first key: below every score but those of no weight.
+constexpr float LOWEST = -FLT_MAX;
 // instruction classes of the scheduling hints
 constexpr int MFMA = 0x008, DS_READ = 0x100;
 
@@ -174,7 +176,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
     }
 
   floatx16 acc[NV];
-  float m_run = NEG, l = 0.f;
+  float m_run = LOWEST, l = 0.f;
 #pragma unroll
   for (int d = 0; d < NV; ++d) acc[d] = floatx16{};
   const int last = CAUSAL ? min(klen, ctx + q0 + QT) : klen;
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int key = t + w * 32 + (i >> 3) * 16 + hi * 8 + (i & 7);
-          if (key > top || key <= low) s[w][i] = NEG;
+          if (key > top || key <= low) s[w][i] = -INFINITY;
         }
     }
     float mx = m_run;
@@ -242,7 +244,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
         for (int i = 0; i < 16; ++i) acc[d][i] *= corr;
     }
     // a query that has seen no key yet keeps weights of exactly zero
-    const float base = m_run <= NEG ? 0.f : m_run * m.mul;
+    float base = m_run <= LOWEST ? 0.f : m_run * m.mul;
     u16x8 pf[KT / 16];
 #pragma unroll
     for (int k = 0; k < KT / 16; ++k) {
@@ -281,7 +283,10 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
 
   l += __shfl_xor(l, 32, WAVE);
   if (qi >= qlen) return;
-  const float f = 1.f / fmaxf(l, 1e-20f);
+  // zeros where a query sees no key; scores of -inf alone are no number
+  const int top = CAUSAL ? min(ctx + qi, klen - 1) : klen - 1;
+  const bool sees = top >= (windowed ? max(0, ctx + qi - m.window + 1) : 0);
+  const float f = sees ? 1.f / l : 0.f;
   uint16_t* dst = out + ((int64_t)(row0 + qi) * m.Hq + h) * D + hi * 4;
 #pragma unroll
   for (int d = 0; d < NV; ++d)
@@ -320,10 +325,15 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
               k.size(2) == D && v.size(2) == D && v.size(0) == k.size(0));
   TORCH_CHECK(out.is_contiguous() && out.sizes() == q.sizes());
   if (B <= 0 || max_seqlen <= 0 || q.numel() == 0) return;
+  Prefill m{};
+  m.mul = (float)std::abs(scale) * LOG2E;
+  if (m.mul == 0.f) {          // masks are set on scores before they are scaled
+    q = at::zeros_like(q);
+    m.mul = LOG2E;
+  }
   q = rows(q);
   k = rows(k);
   v = rows(v);
-  Prefill m{};
   m.cu_q = cu_seqlens.data_ptr<int>();
   m.cu_k = cu_seqlens_k.data_ptr<int>();
   m.q_stride = q.stride(0);
@@ -335,7 +345,6 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
   m.seqs = B;
   m.window = (int)window;
   m.flip = scale < 0;
-  m.mul = (float)std::abs(scale) * LOG2E;
   const dim3 grid(8 * cdiv(B * Hq, 8) * m.q_tiles);
   auto stream = at::hip::getCurrentHIPStream();
 #define LAUNCH(DH, C)                                                        \

@@ -345,6 +345,26 @@ def test_attn_prefill_edges(hq, hkv, d, causal, window, qlens, before, rows):
                                atol=4.6 * 2 ** -9)
 
 
+@pytest.mark.parametrize("scale", [0.0, 1e-36, -1e-30, 0.125])
+@pytest.mark.parametrize("d,causal,window", [(128, True, 0), (64, True, 70),
+                                             (64, False, 0)])
+def test_attn_prefill_masks(scale, d, causal, window):
+    """Masked keys weigh nothing at any scale."""
+    torch.manual_seed(31)
+    lens = [1, 63, 130, 200]
+    q, k, v = (torch.randn(sum(lens), 2, d, dtype=torch.bfloat16)
+               for _ in range(3))
+    cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).int()
+    want = ref.attn_prefill(q.float(), k.float(), v.float(), cu, max(lens),
+                            scale, causal, window)
+    got = ops.attn_prefill(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV),
+                           max(lens), scale, causal, window)
+    # weights rounded to bf16 (2^-9) times values of at most 4.6, and the
+    # result's own rounding
+    torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
+                               atol=4.6 * 2 ** -9)
+
+
 @pytest.mark.parametrize("window,lens", [(64, [200]), (256, [100, 700]),
                                          (512, [2048])])
 def test_paged_attn_decode_sliding_window(window, lens):
