@@ -50,6 +50,12 @@ constexpr int KT = 64;                        // keys of a tile
 constexpr float LOG2E = 1.4426950408889634f;
 // Before the first key: below every score but those of no weight.
 constexpr float LOWEST = -FLT_MAX;
+// A weight is 2^(score mul - maximum mul), in one operation: what is rounded
+// off maximum mul is in all weights alike and falls out, until it exceeds the
+// exponents (from 2^31 on, 2^6 before). Scores that differ at all are then 2^7
+// apart and only the largest counts, for any factor as large; a power of two
+// rounds nothing off.
+constexpr float FAR = 0x1p31f;
 // instruction classes of the scheduling hints
 constexpr int MFMA = 0x008, DS_READ = 0x100;
 
@@ -59,7 +65,7 @@ struct Prefill {
   int64_t q_stride, k_stride, v_stride;       // of a row, in elements
   int Hq, G, q_tiles, seqs, window;
   bool flip;                   // negative scale: of negated queries
-  float mul;                   // |scale| * log2(e)
+  float mul, far_mul;          // |scale| * log2(e); a power of two above it
 };
 
 typedef __attribute__((ext_vector_type(16))) float floatx16;
@@ -176,7 +182,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
     }
 
   floatx16 acc[NV];
-  float m_run = LOWEST, l = 0.f;
+  float m_run = LOWEST, l = 0.f, mul = m.mul;
 #pragma unroll
   for (int d = 0; d < NV; ++d) acc[d] = floatx16{};
   const int last = CAUSAL ? min(klen, ctx + q0 + QT) : klen;
@@ -238,13 +244,14 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
       const float corr = __builtin_amdgcn_exp2f((m_run - mx) * m.mul);
       l *= corr;
       m_run = mx;
+      mul = fabsf(mx * m.mul) < FAR ? m.mul : m.far_mul;
 #pragma unroll
       for (int d = 0; d < NV; ++d)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[d][i] *= corr;
     }
     // a query that has seen no key yet keeps weights of exactly zero
-    float base = m_run <= LOWEST ? 0.f : m_run * m.mul;
+    const float base = m_run <= LOWEST ? 0.f : m_run * mul;
     u16x8 pf[KT / 16];
 #pragma unroll
     for (int k = 0; k < KT / 16; ++k) {
@@ -252,7 +259,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         p[i] = __builtin_amdgcn_exp2f(
-            fmaf(s[k >> 1][(k & 1) * 8 + i], m.mul, -base));
+            fmaf(s[k >> 1][(k & 1) * 8 + i], mul, -base));
         l += p[i];
       }
       pf[k] = pack8(p);
@@ -331,6 +338,7 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
     q = at::zeros_like(q);
     m.mul = LOG2E;
   }
+  m.far_mul = (float)std::ldexp(1.0, std::ilogb(m.mul) + 1);
   q = rows(q);
   k = rows(k);
   v = rows(v);

@@ -348,15 +348,22 @@ def test_attn_prefill_edges(hq, hkv, d, causal, window, qlens, before, rows):
 @pytest.mark.parametrize("scale", [0.0, 1e-36, -1e-30, 0.125])
 @pytest.mark.parametrize("d,causal,window", [(128, True, 0), (64, True, 70),
                                              (64, False, 0)])
-def test_attn_prefill_masks(scale, d, causal, window):
-    """Masked keys weigh nothing at any scale."""
+@pytest.mark.parametrize("large", ["no", "apart", "alike"])
+def test_attn_prefill_masks(scale, d, causal, window, large):
+    """Masked keys weigh nothing at any scale, nor beside scores of some 2^40
+    that are far apart or near the end of the type."""
     torch.manual_seed(31)
     lens = [1, 63, 130, 200]
     q, k, v = (torch.randn(sum(lens), 2, d, dtype=torch.bfloat16)
                for _ in range(3))
+    if large == "apart":
+        q, k = q * 2.0 ** 18, k * 2.0 ** 18
+    if large == "alike":       # one score for all, of some -2^126
+        q, k = (torch.full_like(t, 2.0 ** 63 / d ** 0.5) * s
+                for t, s in ((q, 1), (k, -1)))
     cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).int()
-    want = ref.attn_prefill(q.float(), k.float(), v.float(), cu, max(lens),
-                            scale, causal, window)
+    want = ref.attn_prefill(q.float() * (large != "alike"), k.float(), v.float(),
+                            cu, max(lens), scale, causal, window)
     got = ops.attn_prefill(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV),
                            max(lens), scale, causal, window)
     # weights rounded to bf16 (2^-9) times values of at most 4.6, and the
