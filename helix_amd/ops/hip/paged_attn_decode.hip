@@ -265,8 +265,10 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
 
   const int* bt = m.bt + (int64_t)seq * m.max_blocks;
   const int last = len - 1;
+  // the table is read from the window's first key on: a tile begins up to 31
+  // before it, where pages may have been given back
   auto page = [&](int key) {
-    key = min(key, last);
+    key = max(min(key, last), first);
     return bt[PAGE8 ? key >> m.shift : key / m.bs];
   };
   // Byte offset of a key's row. With PAGE8 the rows of a lane group follow

@@ -440,6 +440,31 @@ def test_paged_attn_decode_edges(hq, hkv, d, bs, fp8, window, lens):
                                atol=5e-5)
 
 
+@pytest.mark.parametrize("bs", [4, 8, 16])
+@pytest.mark.parametrize("window,n", [(5, 70), (100, 613), (129, 4000)])
+def test_paged_attn_decode_pages_given_back(window, n, bs):
+    """Pages before the window have left the table, and the table is read from
+    the window's first key on."""
+    torch.manual_seed(32)
+    need = -(-n // bs)
+    q = torch.randn(1, 4, 128, dtype=torch.bfloat16)
+    kc, vc = (torch.randn(need, 2, bs, 128, dtype=torch.bfloat16)
+              for _ in range(2))
+    bt = torch.randperm(need, dtype=torch.int32)[None]
+    lens = torch.tensor([n], dtype=torch.int32)
+    want = ref.paged_attn_decode(q.float(), kc.float(), vc.float(), bt, lens,
+                                 128 ** -0.5, window)
+    gone = (n - window) // bs
+    for t in (kc, vc):
+        t[bt[0, :gone].long()] = float("nan")
+    bt[0, :gone] = -1
+    got = ops.paged_attn_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                                lens.to(DEV), 128 ** -0.5, window=window)
+    # rounded to bf16 (2^-9, doubled); sums of 32 bits over <= 129 values
+    torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
+                               atol=5e-5)
+
+
 @pytest.mark.parametrize("qlens,klens", [([32], [160]), ([7, 64], [7, 200]),
                                          ([128], [128])])
 def test_attn_prefill_cached_prefix(qlens, klens):
