@@ -36,6 +36,7 @@
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <cfloat>
 
 using namespace helix;
 
@@ -46,7 +47,8 @@ constexpr int KT = 32;                        // keys of a tile
 constexpr int UNIT = KT * NW;                 // tokens that work is cut in
 constexpr int TARGET = 1024;                  // workgroups: 4 on each CU
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr float NEG = -1e30f;
+// Before the first key: below every score but those of no weight.
+constexpr float LOWEST = -FLT_MAX;
 
 struct Rows {
   const int* bt;               // [B, max_blocks]
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
     for (int d = 0; d < DPL; ++d) acc[j][d] = 0.f;
 #pragma unroll
   for (int s = 0; s < QS; ++s) {
-    m_run[s] = NEG;
+    m_run[s] = LOWEST;
     l[s] = 0.f;
   }
   if (t < t_end) {
@@ -366,7 +368,7 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         float v = x[s][i >> 2][i & 3] * m.mul;
-        if (edge && (key0 + i < first || key0 + i >= len)) v = NEG;
+        if (edge && (key0 + i < first || key0 + i >= len)) v = -INFINITY;
         p[i][s] = v;
         mx = fmaxf(mx, v);
       }
@@ -419,7 +421,7 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
   __syncthreads();
   for (int i = threadIdx.x; i < G * D; i += NT) {
     const int j = i / D, d = i % D;
-    float top = NEG, sum = 0.f, o = 0.f;
+    float top = LOWEST, sum = 0.f, o = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) top = fmaxf(top, st[0][w][j]);
 #pragma unroll
@@ -430,7 +432,8 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
     }
     const int64_t row = (int64_t)seq * Hq + g * G + j;
     if (parts == 1) {
-      m.out[row * D + d] = f32_to_bf16(o / fmaxf(sum, 1e-20f));
+      // zeros where there are no keys; scores of -inf alone are no number
+      m.out[row * D + d] = f32_to_bf16(len > 0 ? o / sum : 0.f);
     } else {
       const int64_t at = row * m.max_parts + part;
       m.part[at * D + d] = o;
@@ -457,7 +460,7 @@ __global__ __launch_bounds__(NT) void paged_merge_kernel(Rows m, int Hq) {
   const int64_t row = (int64_t)seq * Hq + blockIdx.y;
   const float2* ml = (const float2*)m.ml + row * m.max_parts;
   const float* part = m.part + row * m.max_parts * D + tid % LANES * 4;
-  float top = NEG;
+  float top = LOWEST;
   for (int p = tid & (WAVE - 1); p < parts; p += WAVE)
     top = fmaxf(top, ml[p].x);
   top = wave_reduce_max(top);
@@ -482,7 +485,7 @@ __global__ __launch_bounds__(NT) void paged_merge_kernel(Rows m, int Hq) {
     s += ls[i];
     r += os[i][tid / 4][tid % 4];
   }
-  m.out[row * D + tid] = f32_to_bf16(r / fmaxf(s, 1e-20f));
+  m.out[row * D + tid] = f32_to_bf16(r / s);
 }
 
 template <int D, int G>

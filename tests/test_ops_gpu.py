@@ -465,6 +465,31 @@ def test_paged_attn_decode_pages_given_back(window, n, bs):
                                atol=5e-5)
 
 
+@pytest.mark.parametrize("max_len", [300, 4096])
+def test_paged_attn_decode_large_scores(max_len):
+    """Scores of some -2^126, of -inf for some keys or for all, and no keys."""
+    torch.manual_seed(33)
+    lens = [1, 33, 300, 300, 0]
+    q = torch.full((5, 2, 64), 2.0 ** 60, dtype=torch.bfloat16)
+    kc = torch.full((5, 1, 320, 64), -2.0 ** 60, dtype=torch.bfloat16)
+    vc = torch.randn(5, 1, 320, 64, dtype=torch.bfloat16)
+    q[2:4] = 1
+    kc[2, 0, 5:290] = float("-inf")
+    kc[3] = float("-inf")
+    want = torch.stack([vc[0, 0, 0].float(), vc[1, 0, :33].float().mean(0),
+                        vc[2, 0, list(range(5)) + list(range(290, 300))]
+                        .float().mean(0), torch.full((64,), float("nan")),
+                        torch.zeros(64)])
+    bt = torch.arange(5, dtype=torch.int32)[:, None]
+    got = ops.paged_attn_decode(
+        q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+        torch.tensor(lens, dtype=torch.int32, device=DEV), 0.125,
+        ops.decode_workspace(5, 2, 64, max_len, DEV), max_len)
+    for h in range(2):             # rounded to bf16 (2^-9, doubled)
+        torch.testing.assert_close(got[:, h].float().cpu(), want,
+                                   rtol=2 ** -8, atol=5e-5, equal_nan=True)
+
+
 @pytest.mark.parametrize("qlens,klens", [([32], [160]), ([7, 64], [7, 200]),
                                          ([128], [128])])
 def test_attn_prefill_cached_prefix(qlens, klens):
