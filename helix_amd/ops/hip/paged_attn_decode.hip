@@ -523,6 +523,21 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(block_tables.scalar_type() == torch::kInt32);
   TORCH_CHECK(seq_lens.scalar_type() == torch::kInt32);
   if (B == 0) return;
+  // everything below goes by raw addresses
+  TORCH_CHECK(q.is_contiguous() && q.scalar_type() == torch::kBFloat16,
+              "q is packed bf16");
+  TORCH_CHECK(out.is_contiguous() && out.scalar_type() == q.scalar_type() &&
+              out.sizes() == q.sizes(), "out is packed bf16 of q's shape");
+  TORCH_CHECK((k_cache.scalar_type() == torch::kBFloat16 ||
+               k_cache.scalar_type() == torch::kUInt8) &&
+              v_cache.scalar_type() == k_cache.scalar_type() &&
+              k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              v_cache.sizes() == k_cache.sizes() && k_cache.size(3) == D,
+              "caches are packed pages of q's head_dim, bf16 or e4m3");
+  TORCH_CHECK(block_tables.is_contiguous() && block_tables.size(0) >= B &&
+              seq_lens.is_contiguous() && seq_lens.numel() >= B,
+              "a length and a row of the table for every sequence");
+  if ((uintptr_t)q.data_ptr() % 16 != 0) q = q.clone();
 
   Rows m{};
   m.bt = block_tables.data_ptr<int>();
@@ -537,7 +552,9 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   m.max_blocks = block_tables.size(1);
   m.max_parts = tmp_out.size(2);
   m.window = (int)window;
-  m.limit = cdiv((int)max_len_hint, UNIT) * UNIT;
+  // nor more than the table has pages for
+  m.limit = (int)std::min<int64_t>(
+      cdiv((int)max_len_hint, UNIT) * UNIT, (int64_t)m.max_blocks * m.bs);
   m.mul = (float)scale * LOG2E;
   // Nothing to cut where a row is at most a unit long, nor where the rows
   // alone fill the chip twice and none can be long: cuts cost 512 rows of
@@ -546,6 +563,15 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                                          : max_len_hint), UNIT);
   m.split = m.max_parts > 1 && most > 1 &&
             !(B * Hkv >= 2 * TARGET && most <= 8);
+  const int64_t pieces = (int64_t)B * Hq * m.max_parts;
+  TORCH_CHECK(!m.split || (tmp_out.is_contiguous() && tmp_ml.is_contiguous() &&
+                           tmp_out.numel() >= pieces * D &&
+                           tmp_ml.numel() >= pieces * 2),
+              "a workspace of [B, Hq, parts, D] and [B, Hq, parts, 2]");
+  for (const auto& t : {q, out, k_cache, v_cache, block_tables, seq_lens,
+                        tmp_out, tmp_ml})
+    TORCH_CHECK(t.is_cuda() && t.device() == q.device(),
+                "everything on one GPU");
   // a workgroup without a piece costs its search, so no more than can be
   const dim3 grid(m.split ? std::min(B * most, B + TARGET / Hkv + 1) : B,
                   Hkv);

@@ -167,3 +167,37 @@ def test_gemm_bf16_refuses(case, says):
         out = out[:, :8]
     with pytest.raises(RuntimeError, match=says):
         ops._native().gemm_bf16(out, x, w, b, 0)
+
+
+@pytest.mark.parametrize("case,says", [
+    ("out shape", "out is packed"), ("out rows", "out is packed"),
+    ("q", "q is packed"), ("cache", "caches are"), ("pages", "caches are"),
+    ("lens", "a length and"), ("table", "a length and"),
+    ("workspace", "a workspace of"), ("host", "on one GPU")])
+def test_paged_attn_decode_refuses(case, says):
+    """What would be read or written out of range is refused before any
+    launch."""
+    q = torch.zeros(3, 4, 64, dtype=torch.bfloat16)
+    kc = torch.zeros(9, 2, 128, 64, dtype=torch.bfloat16)
+    vc, out = kc.clone(), torch.empty_like(q)
+    bt = torch.zeros(3, 3, dtype=torch.int32)
+    lens = torch.full((3,), 300, dtype=torch.int32)
+    ws = ops.decode_workspace(2 if case == "workspace" else 3, 4, 64, 384,
+                              "cpu")
+    if case == "out shape":
+        out = out[:2]
+    elif case == "out rows":
+        out = torch.empty(3, 4, 128, dtype=torch.bfloat16)[..., :64]
+    elif case == "q":
+        q = torch.zeros(3, 64, 4, dtype=torch.bfloat16).transpose(1, 2)
+    elif case == "cache":
+        vc = vc.half()
+    elif case == "pages":
+        kc = kc[:, :, ::2]
+    elif case == "lens":
+        lens = lens[:2]
+    elif case == "table":
+        bt = bt[:2]
+    with pytest.raises(RuntimeError, match=says):
+        ops._native().paged_attn_decode(out, q, kc, vc, bt, lens, 0.125,
+                                        *ws, 384, 0)
