@@ -59,9 +59,9 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor,
                        w: torch.Tensor, eps: float):
     """In-place on GPU: x <- norm(x+res), residual <- x+res. Returns both.
-    x may be the stretches of a product (linear_sums), which stay as they
-    are."""
-    if x.dim() == 3:
+    On GPU x may be the stretches of a product (linear_sums, fp32
+    [n, T, H]), which stay as they are."""
+    if x.is_cuda and x.dim() == 3 and x.dtype == torch.float32:
         h = torch.empty_like(residual)
         _native().add_sums_rms_norm(h, x, residual, w, eps)
         return h, residual
@@ -180,12 +180,14 @@ def rope_qkv_cache(positions: torch.Tensor, qkv: torch.Tensor,
                    head_dim: int, kv_cache=None, slot_mapping=None,
                    want_kv: bool = False):
     """Fused QKV epilogue: strided split + rope + paged-cache write. qkv is
-    [T, C], or the stretches of that product (linear_sums).
+    [T, C] or [T, heads, head_dim], or in fp32 the stretches [n, T, C] of that
+    product (linear_sums).
 
     Returns (q [T, num_q, head_dim], k, v) — k/v are None unless
     want_kv (fresh-prefill path needs compact K/V for attn_prefill).
     """
-    T = qkv.shape[-2]
+    sums = qkv.dim() == 3 and qkv.dtype == torch.float32
+    T = qkv.shape[1 if sums else 0]
     if qkv.is_cuda:
         dtype = torch.bfloat16
         q_out = torch.empty(T, num_q * head_dim, dtype=dtype,

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(NT) void rope_qkv_cache_kernel(Epilogue m) {
 
 }  // namespace
 
-// qkv: [T, C] bf16, or [stretches, T, C] fp32
+// qkv: [T, C] or [T, heads, head_dim] bf16, or [stretches, T, C] fp32
 void rope_qkv_cache(torch::Tensor positions, torch::Tensor qkv,
                     torch::Tensor q_out,
                     c10::optional<torch::Tensor> k_cache,
@@ -143,17 +143,16 @@ void rope_qkv_cache(torch::Tensor positions, torch::Tensor qkv,
                     int64_t num_kv_heads, int64_t head_dim) {
   const int T = positions.size(0);
   if (T == 0) return;
-  const bool sums = qkv.dim() == 3;
+  const bool sums = qkv.dim() == 3 && qkv.scalar_type() == torch::kFloat32;
   TORCH_CHECK(positions.scalar_type() == torch::kInt64);
   TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32);
   TORCH_CHECK(qkv.stride(-1) == 1, "qkv innermost must be contiguous");
-  TORCH_CHECK(qkv.scalar_type() ==
-              (sums ? torch::kFloat32 : torch::kBFloat16));
+  TORCH_CHECK(sums || qkv.scalar_type() == torch::kBFloat16);
   TORCH_CHECK(head_dim % 8 == 0);
   Epilogue m{};
   m.positions = positions.data_ptr<int64_t>();
   m.qkv = qkv.data_ptr();
-  m.stride = qkv.stride(-2);
+  m.stride = qkv.stride(sums ? 1 : 0);
   m.all = sums ? qkv.stride(0) : 0;
   m.stretches = sums ? qkv.size(0) : 1;
   m.q = (uint16_t*)q_out.data_ptr();

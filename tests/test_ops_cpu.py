@@ -201,3 +201,14 @@ def test_paged_attn_decode_refuses(case, says):
     with pytest.raises(RuntimeError, match=says):
         ops._native().paged_attn_decode(out, q, kc, vc, bt, lens, 0.125,
                                         *ws, 384, 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_fused_add_rms_norm_of_batches(dtype):
+    """[B, T, H] is a batch of rows, not a product's stretches."""
+    x, r = torch.randn(2, 3, 5, 16, dtype=dtype)
+    w = torch.randn(16, dtype=dtype)
+    want = ref.fused_add_rms_norm(x, r, w, 1e-5)
+    got = ops.fused_add_rms_norm(x.clone(), r.clone(), w, 1e-5)
+    for a, b in zip(got, want):
+        assert a.shape == (3, 5, 16) and torch.equal(a, b)

@@ -852,6 +852,23 @@ def test_quantize_rows_bytes(T, K):
     assert torch.equal(got.nan_to_num(), want.float().nan_to_num())
 
 
+def test_three_dimensions_of_bf16():
+    """Batches of rows and rows of heads are not a product's stretches."""
+    torch.manual_seed(34)
+    x, r = torch.randn(2, 3, 5, 256, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(256, dtype=torch.bfloat16, device=DEV)
+    flat = ops.fused_add_rms_norm(x.view(15, 256).clone(),
+                                  r.view(15, 256).clone(), w, 1e-5)
+    for a, b in zip(ops.fused_add_rms_norm(x, r, w, 1e-5), flat):
+        assert torch.equal(a.view(15, 256), b)
+    qkv = torch.randn(7, 8, 64, dtype=torch.bfloat16, device=DEV)
+    cs = ref.make_cos_sin_cache(64, 16).to(DEV)
+    pos = torch.arange(7, device=DEV)
+    for a, b in zip(*(ops.rope_qkv_cache(pos, z, cs, 4, 2, 64, want_kv=True)
+                      for z in (qkv, qkv.view(7, 512)))):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_rope_qkv_cache_from_stretches(fp8):
     """The epilogue over a product's stretches is that over their sum."""
