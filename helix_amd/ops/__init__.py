@@ -368,7 +368,7 @@ def gemm_fp8(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,
     M, N = x8.shape[0], w8.shape[0]
     if x8.is_cuda:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=x8.device)
-        if act == 0 and _rows_fit(x8, w8):
+        if act == 0 and _rows_fit(x8, w8) and _bias_fits(bias, w8):
             _native().gemm_rows(out, x8, w8, bias, x_scale.contiguous(),
                                 w_scale.contiguous())
             return out
@@ -396,11 +396,8 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
     if x.is_cuda:
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
-        if (_rows_fit(x, w, 128 if w.shape[1] >= 2 * w.shape[0] else 64)
-                and x.dtype == torch.bfloat16 and w.shape[1] == x.shape[1]
-                and (bias is None or bias.dtype == x.dtype
-                     and bias.is_contiguous()
-                     and bias.numel() == w.shape[0])):
+        if (x.dtype == torch.bfloat16 and _bias_fits(bias, w) and
+                _rows_fit(x, w, 128 if w.shape[1] >= 2 * w.shape[0] else 64)):
             _native().gemm_rows(out, x, w, bias, None, None, act == 1)
         else:
             _native().gemm_bf16(out, x, w, bias, act)
@@ -457,14 +454,24 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor,
     """Whether the kernel for a few rows takes x @ w^T, bf16 or e4m3 bytes.
     It knows nothing of gradients, so bf16 only runs where there are none to
     be had."""
-    return (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= most
+    return (x.is_cuda and x.dim() == 2 and w.dim() == 2
+            and 0 < x.shape[0] <= most
             and (x.dtype == torch.uint8 or x.dtype == torch.bfloat16
                  and torch.is_inference_mode_enabled())
-            and x.dtype == w.dtype and x.shape[1] > 0
+            and x.dtype == w.dtype and x.device == w.device
+            and x.get_device() == torch.cuda.current_device()
+            and x.shape[1] == w.shape[1] > 0
             and x.shape[1] * x.element_size() % ROWS_CHUNK == 0
             and w.shape[0] > 0 and w.shape[0] % 8 == 0
             and x.is_contiguous() and w.is_contiguous()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def _bias_fits(bias, w: torch.Tensor) -> bool:
+    """Whether the kernel for a few rows reads this bias as it lies."""
+    return bias is None or (
+        bias.shape == w.shape[:1] and bias.dtype == torch.bfloat16
+        and bias.device == w.device and bias.is_contiguous())
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
@@ -482,13 +489,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
             and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0
             and x.is_contiguous() and w.is_contiguous()):
         return gemm_skinny_bf16(x, w, bias)
-    M, N, K = x.shape[0], w.shape[0], w.shape[1]
-    if _rows_fit(x, w) and (M <= 16 and N <= 65536 or K >= 2 * N or
-                            M > 64 and N <= 8192):
-        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
-                          device=x.device)
-        _native().gemm_rows(out, x, w, bias, None, None)
-        return out
+    if _rows_fit(x, w) and _bias_fits(bias, w):
+        (M, K), N = x.shape, w.shape[0]
+        if (M <= 16 and N <= 65536 or K >= 2 * N or M > 64 and N <= 8192):
+            out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+            _native().gemm_rows(out, x, w, bias, None, None)
+            return out
     return torch.nn.functional.linear(x, w, bias)
 
 

@@ -209,6 +209,7 @@ Product product_of(const torch::Tensor& x, const torch::Tensor& w,
   const bool f8 = x_scale.has_value();
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.is_cuda() &&
+                t.device() == x.device() &&
                 t.scalar_type() == (f8 ? torch::kUInt8 : torch::kBFloat16) &&
                 (uintptr_t)t.data_ptr() % 16 == 0);
   Product m{};
@@ -221,7 +222,8 @@ Product product_of(const torch::Tensor& x, const torch::Tensor& w,
   TORCH_CHECK(w_scale.has_value() == f8);
   if (f8) {
     for (const auto& t : {*x_scale, *w_scale})
-      TORCH_CHECK(t.is_contiguous() && t.scalar_type() == torch::kFloat32);
+      TORCH_CHECK(t.is_contiguous() && t.scalar_type() == torch::kFloat32 &&
+                  t.device() == x.device());
     TORCH_CHECK(x_scale->numel() == m.M && w_scale->numel() == w.size(0));
     m.xs = x_scale->data_ptr<float>();
     m.ws = w_scale->data_ptr<float>();
@@ -272,8 +274,10 @@ torch::Tensor sums_for(const torch::Tensor& x, const Product& m,
                       x.options().dtype(torch::kFloat32));
 }
 
-void check_out(const torch::Tensor& out, const Product& m) {
+void check_out(const torch::Tensor& out, const torch::Tensor& x,
+               const Product& m) {
   TORCH_CHECK(out.is_contiguous() && out.dim() == 2 &&
+              out.device() == x.device() &&
               out.scalar_type() == torch::kBFloat16 && out.size(0) == m.M &&
               out.size(1) == m.N && (uintptr_t)out.data_ptr() % 8 == 0);
 }
@@ -293,10 +297,11 @@ torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
 void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
                OptT x_scale, OptT w_scale, bool gelu) {
   Product m = product_of(x, w, x_scale, w_scale);
-  check_out(out, m);
+  check_out(out, x, m);
   if (bias.has_value()) {
     TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 &&
-                bias->is_contiguous() && bias->numel() == m.N);
+                bias->is_contiguous() && bias->numel() == m.N &&
+                bias->device() == x.device());
     m.bias = (const uint16_t*)bias->data_ptr();
   }
   const int stretches = cut(m);
@@ -321,6 +326,6 @@ void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(m.M <= 64 && m.N % 8 == 0);
   m.N /= 2;                                   // 32 columns of a workgroup
   m.n_tiles = cdiv(m.N, 32);
-  check_out(out, m);
+  check_out(out, x, m);
   run<true>((uint16_t*)out.data_ptr(), nullptr, x, w, m, 1);
 }

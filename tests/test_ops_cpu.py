@@ -212,3 +212,11 @@ def test_fused_add_rms_norm_of_batches(dtype):
     got = ops.fused_add_rms_norm(x.clone(), r.clone(), w, 1e-5)
     for a, b in zip(got, want):
         assert a.shape == (3, 5, 16) and torch.equal(a, b)
+
+
+def test_linear_with_a_vector():
+    """A weight of one dimension, as torch's linear takes it."""
+    x, w = torch.randn(5, 16), torch.randn(16)
+    for z in (x, x[0]):
+        assert torch.equal(ops.linear(z, w),
+                           torch.nn.functional.linear(z, w))

@@ -891,6 +891,32 @@ def test_rope_qkv_cache_from_stretches(fp8):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("form", ["strided", "one", "row", "rows", "vector"])
+def test_linear_takes_what_torch_takes(form):
+    """Biases and weights that only the library's product reads."""
+    torch.manual_seed(35)
+    x = torch.randn(4, 512, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(64, 512, dtype=torch.bfloat16, device=DEV) / 22
+    b = torch.randn(4, 128, dtype=torch.bfloat16, device=DEV)
+    b = {"strided": b[0, ::2], "one": b[0, :1], "row": b[:1, :64],
+         "rows": b[:, :64].contiguous(), "vector": None}[form]
+    if form == "vector":
+        w = w[0]
+    with torch.inference_mode():
+        got = ops.linear(x, w, b)
+        want = torch.nn.functional.linear(x, w, b)
+    assert torch.equal(got, want)
+
+
+def test_linear_refuses_a_bias_of_the_host():
+    x = torch.zeros(4, 512, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(64, 512, dtype=torch.bfloat16, device=DEV)
+    b = torch.zeros(64, dtype=torch.bfloat16)
+    for f in (ops.linear, ops.gemm_bf16):
+        with torch.inference_mode(), pytest.raises(RuntimeError):
+            f(x, w, b)
+
+
 def test_linear_dispatch_matches_torch():
     """ops.linear (the HLinear route) must agree with F.linear on the
     decode shapes it owns."""
