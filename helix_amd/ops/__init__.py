@@ -454,7 +454,7 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor,
     """Whether the kernel for a few rows takes x @ w^T, bf16 or e4m3 bytes.
     It knows nothing of gradients, so bf16 only runs where there are none to
     be had."""
-    return (x.is_cuda and x.dim() == 2 and w.dim() == 2
+    return (x.is_cuda and _eager() and x.dim() == 2 and w.dim() == 2
             and 0 < x.shape[0] <= most
             and (x.dtype == torch.uint8 or x.dtype == torch.bfloat16
                  and torch.is_inference_mode_enabled())
@@ -463,8 +463,21 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor,
             and x.shape[1] == w.shape[1] > 0
             and x.shape[1] * x.element_size() % ROWS_CHUNK == 0
             and w.shape[0] > 0 and w.shape[0] % 8 == 0
-            and x.is_contiguous() and w.is_contiguous()
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and x.is_contiguous() and w.is_contiguous() and _aligned(x, w))
+
+
+def _eager() -> bool:
+    """Neither under autocast nor a tracer, which have to see torch's own."""
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch.is_autocast_enabled("cuda"))
+
+
+def _aligned(*ts: torch.Tensor) -> bool:
+    """Whether these are memory, on 16-byte boundaries."""
+    try:
+        return all(t.data_ptr() % 16 == 0 for t in ts)
+    except RuntimeError:           # within vmap and the like they have none
+        return False
 
 
 def _bias_fits(bias, w: torch.Tensor) -> bool:

@@ -908,6 +908,23 @@ def test_linear_takes_what_torch_takes(form):
     assert torch.equal(got, want)
 
 
+def test_linear_under_transforms():
+    """vmap, autocast and tracing see torch's linear, as without the kernel
+    for a few rows."""
+    torch.manual_seed(36)
+    x = torch.randn(3, 4, 512, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(64, 512, dtype=torch.bfloat16, device=DEV) / 22
+    with torch.inference_mode():
+        got = torch.vmap(lambda t: ops.linear(t, w))(x)
+        torch.testing.assert_close(got, torch.nn.functional.linear(x, w))
+        with torch.autocast("cuda", torch.float16):
+            assert ops.linear(x[0], w).dtype == torch.float16
+    with torch.inference_mode():
+        f = torch.jit.trace(lambda t: ops.linear(t, w), (x[0],))
+        torch.testing.assert_close(f(x[1]),
+                                   torch.nn.functional.linear(x[1], w))
+
+
 def test_linear_refuses_a_bias_of_the_host():
     x = torch.zeros(4, 512, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(64, 512, dtype=torch.bfloat16, device=DEV)
