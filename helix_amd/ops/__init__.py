@@ -397,7 +397,8 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
         if (x.dtype == torch.bfloat16 and _bias_fits(bias, w) and
-                _rows_fit(x, w, 128 if w.shape[1] >= 2 * w.shape[0] else 64)):
+                _rows_fit(x, w, 128 if w.shape[1] >= 2 * w.shape[0] else 64,
+                          grads=False)):
             _native().gemm_rows(out, x, w, bias, None, None, act == 1)
         else:
             _native().gemm_bf16(out, x, w, bias, act)
@@ -449,15 +450,15 @@ ROWS_MAX_M_GLU = 64               # of its gated form
 ROWS_CHUNK = 512                  # bytes
 
 
-def _rows_fit(x: torch.Tensor, w: torch.Tensor,
-              most: int = ROWS_MAX_M) -> bool:
+def _rows_fit(x: torch.Tensor, w: torch.Tensor, most: int = ROWS_MAX_M,
+              grads: bool = True) -> bool:
     """Whether the kernel for a few rows takes x @ w^T, bf16 or e4m3 bytes.
-    It knows nothing of gradients, so bf16 only runs where there are none to
-    be had."""
+    It knows nothing of gradients, so where it stands for torch's product
+    (grads) bf16 only runs where there are none to be had."""
     return (x.is_cuda and _eager() and x.dim() == 2 and w.dim() == 2
             and 0 < x.shape[0] <= most
             and (x.dtype == torch.uint8 or x.dtype == torch.bfloat16
-                 and torch.is_inference_mode_enabled())
+                 and (not grads or torch.is_inference_mode_enabled()))
             and x.dtype == w.dtype and x.device == w.device
             and x.get_device() == torch.cuda.current_device()
             and x.shape[1] == w.shape[1] > 0

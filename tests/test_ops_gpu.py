@@ -934,6 +934,21 @@ def test_linear_refuses_a_bias_of_the_host():
             f(x, w, b)
 
 
+def test_gemm_bf16_in_any_mode():
+    """It never had gradients: a few rows are streamed with and without them,
+    to the same bits."""
+    torch.manual_seed(37)
+    x = torch.randn(33, 3072, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(768, 3072, dtype=torch.bfloat16, device=DEV) / 55
+    w.requires_grad_()
+    out = []
+    for mode in (torch.enable_grad, torch.no_grad, torch.inference_mode):
+        with mode():
+            out.append(ops.gemm_bf16(x, w))
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[2])
+    assert not out[0].requires_grad
+
+
 def test_linear_dispatch_matches_torch():
     """ops.linear (the HLinear route) must agree with F.linear on the
     decode shapes it owns."""
