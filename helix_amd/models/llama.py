@@ -17,6 +17,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from helix_amd import ops
 from helix_amd.models.meta import (DecodeMeta, KVLayer,  # noqa: F401
@@ -137,7 +138,8 @@ class HLinear(nn.Linear):
     """nn.Linear routed through ops.linear: a few rows run the owned MFMA
     kernel, prefill-shaped ones stay on hipBLASLt.
 
-    form: "rows" -> [T, N]; "sums" -> what ops.linear_sums gives, for a
+    A plain call returns rows [T, N]. The modules here ask each other for
+    other forms (_own says when): "sums" -> what ops.linear_sums gives, for a
     reader that adds it up; "glu" -> silu(first half) * second half."""
 
     def forward(self, x: torch.Tensor, form: str = "rows") -> torch.Tensor:
@@ -149,9 +151,18 @@ class HLinear(nn.Linear):
         return ops.silu_and_mul(out) if form == "glu" else out
 
 
+def _own(m: nn.Module, *kinds: type) -> bool:
+    """Whether m is one of these modules as written here: a subclass, a module
+    put in its place or a hook gets and returns what torch's linear would,
+    [T, N], and never a form."""
+    return type(m) in kinds and not (
+        m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+        or _has_any_global_hook())
+
+
 def _project(proj: nn.Module, x: torch.Tensor, form: str) -> torch.Tensor:
     """proj(x) in that form; other kinds of projections know only rows."""
-    if isinstance(proj, (HLinear, FP8Linear)):
+    if _own(proj, HLinear, FP8Linear):
         return proj(x, form)
     out = proj(x)
     return ops.silu_and_mul(out) if form == "glu" else out
@@ -261,10 +272,11 @@ class DecoderLayer(nn.Module):
         else:
             h, residual = ops.fused_add_rms_norm(x, residual,
                                                  self.input_norm_w, self.eps)
-        h = self.attn(h, cos_sin, kv_cache, meta, "sums")
+        h = self.attn(h, cos_sin, kv_cache, meta,
+                      *(["sums"] if _own(self.attn, Attention) else []))
         h, residual = ops.fused_add_rms_norm(h, residual, self.post_norm_w,
                                              self.eps)
-        h = self.mlp(h, form)
+        h = self.mlp(h, *([form] if _own(self.mlp, MLP) else []))
         return h, residual
 
 
@@ -301,10 +313,14 @@ class LlamaForCausalLM(nn.Module):
     @torch.inference_mode()
     def forward(self, input_ids: torch.Tensor, kv_caches, meta) -> torch.Tensor:
         x = self.embed_tokens(input_ids)
-        residual = None
+        residual, own = None, True
         for i, layer in enumerate(self.layers):
             cache = kv_caches[i] if kv_caches is not None else None
-            x, residual = layer(x, residual, self.cos_sin, cache, meta, "sums")
+            own = _own(layer, DecoderLayer)
+            x, residual = layer(x, residual, self.cos_sin, cache, meta,
+                                *(["sums"] if own else []))
+        if not own:                # what a hook has kept stays as it was
+            x, residual = x.clone(), residual.clone()
         return ops.fused_add_rms_norm(x, residual, self.final_norm_w,
                                       self.cfg.rms_norm_eps)[0]
 

@@ -533,3 +533,75 @@ def test_llama31_rope_scaling_cache():
                                                    max_tokens=3,
                                                    ignore_eos=True))
     assert len(out[0]) == 3
+
+
+def _llama_prefill(device="cpu", change=lambda m: None):
+    """Hidden states of a prompt in a tiny model."""
+    import torch
+    from helix_amd.models.llama import (PRESETS, LlamaForCausalLM,
+                                        PrefillMeta)
+    m = LlamaForCausalLM(PRESETS["tiny"])
+    m.init_random(3)
+    m = m.to(torch.bfloat16).to(device)
+    change(m)
+    n = 9
+    meta = PrefillMeta(positions=torch.arange(n, device=device),
+                       cu_seqlens=torch.tensor([0, n], dtype=torch.int32,
+                                               device=device),
+                       max_seqlen=n, slot_mapping=None)
+    return m(torch.arange(n, device=device) * 7, None, meta)
+
+
+def test_llama_hooks_see_plain_results():
+    """Hooks get a projection's [T, N] and a call without a form."""
+    import torch
+    seen, kept = {}, []
+
+    def watch(m):
+        for name, mod in m.named_modules():
+            if name.endswith(("_proj", "attn", "mlp")):
+                mod.register_forward_pre_hook(
+                    lambda mod, args: seen.setdefault("args", set()).update(
+                        [any(isinstance(a, str) for a in args)]))
+            if name.endswith("_proj"):
+                mod.register_forward_hook(
+                    lambda mod, args, out, name=name: seen.__setitem__(
+                        name, (mod.out_features, out.shape, out.dtype)))
+        m.layers[-1].register_forward_hook(
+            lambda mod, args, out: kept.extend((*out, out[0].clone(),
+                                                out[1].clone())))
+
+    want = _llama_prefill()
+    assert torch.equal(_llama_prefill(change=watch), want)
+    assert seen.pop("args") == {False} and len(seen) == 8
+    for n, shape, dtype in seen.values():
+        assert shape == (9, n) and dtype == torch.bfloat16
+    assert torch.equal(kept[0], kept[2]) and torch.equal(kept[1], kept[3])
+
+
+def test_llama_modules_put_in_place():
+    """Modules of one's own are called with what torch's linear and the
+    feed-forward block take."""
+    import torch
+    from helix_amd.models.llama import HLinear
+
+    class Mine(HLinear):
+        def forward(self, x):
+            return torch.nn.functional.linear(x, self.weight)
+
+    class Block(torch.nn.Module):
+        def __init__(self, mlp):
+            super().__init__()
+            self.mlp = mlp
+
+        def forward(self, x):
+            return self.mlp(x)
+
+    def change(m):
+        for layer in m.layers:
+            for mod in (layer.attn.qkv_proj, layer.attn.o_proj,
+                        layer.mlp.gate_up_proj):
+                mod.__class__ = Mine
+            layer.mlp = Block(layer.mlp)
+
+    assert torch.equal(_llama_prefill(change=change), _llama_prefill())

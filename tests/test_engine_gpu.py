@@ -166,3 +166,42 @@ def test_vision_embeddings_gpu_matches_cpu():
     vc = [np.array(v) for v in cpu.embed(imgs)]
     for g, c in zip(vg, vc):
         assert g @ c > 0.98, f"gpu/cpu cosine {g @ c}"
+
+
+@pytest.mark.parametrize("rows", [5, 200])
+@pytest.mark.parametrize("weights", ["bf16", "fp8"])
+def test_hooks_see_plain_results(rows, weights):
+    """Where products are handed on as stretches or gated halves, hooks still
+    see [T, N] in bf16, and the last layer's results stay as they were."""
+    from helix_amd.models.llama import (PRESETS, LlamaForCausalLM,
+                                        PrefillMeta)
+    from helix_amd.models.quant import quantize_model_fp8
+    m = LlamaForCausalLM(PRESETS["tiny-gqa"])
+    m.init_random(3)
+    m = m.to(torch.bfloat16).to("cuda")
+    if weights == "fp8":
+        quantize_model_fp8(m)
+    pos = torch.arange(rows, device="cuda")
+    meta = PrefillMeta(cu_seqlens=torch.tensor([0, rows], dtype=torch.int32,
+                                               device="cuda"),
+                       max_seqlen=rows, slot_mapping=None, positions=pos)
+    want = m(pos % 100, None, meta)
+    shapes, kept = [], []
+    for name, mod in m.named_modules():
+        if name.endswith("_proj"):
+            mod.register_forward_hook(lambda mod, args, out: shapes.append(
+                (out.shape, out.dtype, mod.out_features)))
+    m.layers[-1].register_forward_hook(
+        lambda mod, args, out: kept.extend((*out, *(t.clone() for t in out))))
+    got = m(pos % 100, None, meta)
+    assert len(shapes) == 4 * len(m.layers)
+    for shape, dtype, n in shapes:
+        assert shape == (rows, n) and dtype == torch.bfloat16
+    assert torch.equal(kept[0], kept[2]) and torch.equal(kept[1], kept[3])
+    # Products are now rounded to bf16 before norms and activation: 2^-9 of a
+    # value a time, four times a layer, 2^-6 for 2 to 4 layers with room. Of
+    # activations in e4m3 (steps of 2^-3) such a difference lets 2^-9 / 2^-3
+    # fall the other way, by a step: 2^-3 (2^-6)^(1/2) = 2^-6 a product, 2^-3
+    # for the 4 of each layer if all added up.
+    off = float((got.float() - want.float()).norm() / want.float().norm())
+    assert off < (2 ** -6 if weights == "bf16" else 2 ** -3), off
