@@ -157,13 +157,18 @@ def kv_fp8_dequant(t: torch.Tensor, dtype=torch.bfloat16) -> torch.Tensor:
 def gather_kv(k_cache: torch.Tensor, v_cache: torch.Tensor,
               blk: torch.Tensor, off: torch.Tensor, dtype=torch.bfloat16):
     """Rows [T, Hkv, D] of a paged cache at offsets off of pages blk; e4m3
-    bytes become dtype."""
+    bytes become dtype. Other places than int64 of the same GPU are for torch's
+    indexing, as are caches of other types or packing."""
     if (k_cache.is_cuda and dtype == torch.bfloat16 and
             k_cache.dtype in (torch.bfloat16, torch.uint8) and
             k_cache.shape[3] % 8 == 0 and
-            all(c.is_contiguous() and c.data_ptr() % 16 == 0
-                for c in (k_cache, v_cache)) and
-            blk.is_contiguous() and off.is_contiguous()):
+            v_cache.dtype == k_cache.dtype and
+            v_cache.shape == k_cache.shape and
+            k_cache.is_contiguous() and v_cache.is_contiguous() and
+            blk.shape == off.shape and blk.dim() == 1 and
+            all(t.dtype == torch.int64 and t.is_contiguous() and
+                t.device == k_cache.device for t in (blk, off)) and
+            v_cache.device == k_cache.device and _aligned(k_cache, v_cache)):
         k = torch.empty(blk.numel(), k_cache.shape[1], k_cache.shape[3],
                         dtype=dtype, device=k_cache.device)
         v = torch.empty_like(k)

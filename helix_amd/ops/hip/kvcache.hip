@@ -146,6 +146,9 @@ void gather_kv(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
   TORCH_CHECK(blk.scalar_type() == torch::kInt64 && blk.is_contiguous() &&
               off.scalar_type() == torch::kInt64 && off.is_contiguous() &&
               off.numel() == T);
+  for (const auto& t : {k, v, k_cache, v_cache, blk, off})
+    TORCH_CHECK(t.is_cuda() && t.device() == k.device(),
+                "everything on one GPU");
   TORCH_CHECK(k.is_contiguous() && v.is_contiguous() &&
               k.scalar_type() == torch::kBFloat16 &&
               v.scalar_type() == torch::kBFloat16 &&

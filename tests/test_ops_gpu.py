@@ -166,6 +166,26 @@ def test_gather_kv(T, H, D, page, fp8):
         assert torch.equal(got, ops.kv_fp8_dequant(want) if fp8 else want)
 
 
+@pytest.mark.parametrize("places", ["int32", "host", "broadcast", "mixed"])
+def test_gather_kv_places(places):
+    """What torch's indexing takes for places, and caches of two types."""
+    torch.manual_seed(38)
+    kc, vc = (torch.randn(7, 2, 16, 64, device=DEV).bfloat16()
+              for _ in range(2))
+    blk = torch.randint(0, 7, (5,), device=DEV)
+    off = torch.randint(0, 16, (5,), device=DEV)
+    if places == "int32":
+        blk, off = blk.int(), off.int()
+    elif places == "host":
+        blk, off = blk.cpu(), off.cpu()
+    elif places == "broadcast":
+        off = off[:1]
+    else:
+        vc = vc.half()
+    for got, cache in zip(ops.gather_kv(kc, vc, blk, off), (kc, vc)):
+        assert torch.equal(got, cache[blk, :, off])
+
+
 @pytest.mark.parametrize("hq,hkv,d,lens", [
     (32, 8, 128, [1, 17, 128, 63]),
     (8, 8, 128, [200]),
