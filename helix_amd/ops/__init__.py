@@ -83,17 +83,32 @@ def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor,
     return ref.layer_norm(x, w, b, eps)
 
 
-def _rows_of_8(x: torch.Tensor) -> bool:
+def _rows_of_8(*rows: torch.Tensor | None) -> bool:
     """Whether encoder.hip takes these rows (a lane has up to 8 vectors)."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2
+    x, *more = (t for t in rows if t is not None)
+    return (x.is_cuda and x.dim() == 2
             and x.shape[1] % 8 == 0 and x.shape[1] <= 4096
-            and x.is_contiguous())
+            and all(t.dtype == torch.bfloat16 and t.device == x.device
+                    and t.shape == x.shape and t.is_contiguous()
+                    for t in (x, *more)) and _aligned(x, *more))
+
+
+def _modulates(x: torch.Tensor, L: int, *rows: torch.Tensor | None) -> bool:
+    """Whether encoder.hip takes these rows for every L of x: slices of one
+    product, or packed."""
+    first, *more = (t for t in rows if t is not None)
+    return (first.dim() == 2 and first.stride(0) % 8 == 0
+            and first.shape[0] * L >= x.shape[0]
+            and all(t.dtype == torch.bfloat16 and t.device == x.device
+                    and t.shape == (first.shape[0], x.shape[1])
+                    and t.stride() == (first.stride(0), 1)
+                    for t in (first, *more)) and _aligned(first, *more))
 
 
 def add_layer_norm(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor,
                    b: torch.Tensor, eps: float) -> torch.Tensor:
     """Layer norm of x + y."""
-    if _rows_of_8(x) and y.is_contiguous():
+    if _rows_of_8(x, y) and _aligned(w, b):
         out = torch.empty_like(x)
         _native().add_norm(None, out, x, y, None, w, b, 0, eps)
         return out
@@ -106,7 +121,7 @@ def modulated_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor,
     """(s, norm(s) (1 + scale) + shift), s = x + gate y (x without y). norm
     is a layer norm without weights; gate, scale and shift have a row for
     every L rows of x."""
-    if _rows_of_8(x) and (y is None or y.is_contiguous()):
+    if _rows_of_8(x, y) and _modulates(x, L, scale, shift, gate):
         out = torch.empty_like(x)
         s = x if y is None else torch.empty_like(x)
         _native().add_norm(None if y is None else s, out, x, y, gate, scale,
@@ -124,7 +139,7 @@ def modulated_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor,
 def gated_add(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor,
               L: int) -> torch.Tensor:
     """x + gate y; gate has a row for every L rows of x."""
-    if _rows_of_8(x) and y.is_contiguous():
+    if _rows_of_8(x, y) and _modulates(x, L, gate):
         out = torch.empty_like(x)
         _native().gated_add(out, x, y, gate, L)
         return out

@@ -98,6 +98,43 @@ def test_add_norm(T, H):
                                **tol)
 
 
+@pytest.mark.parametrize("form", ["fp32 y", "off", "strides", "columns",
+                                  "fp32 mod"])
+def test_add_norm_forms(form):
+    """Other types, boundaries and strides go as separate steps."""
+    torch.manual_seed(39)
+    T, H, L = 6, 64, 3
+    x, y = torch.randn(2, T, H, dtype=torch.bfloat16, device=DEV)
+    w, b = torch.randn(2, H, dtype=torch.bfloat16, device=DEV)
+    mod = torch.randn(2, 3 * H, dtype=torch.bfloat16, device=DEV)
+    gate, scale, shift = mod.chunk(3, -1)
+    if form == "fp32 y":
+        y = y.float()
+    elif form == "off":
+        x = torch.randn(T * H + 1, dtype=torch.bfloat16,
+                        device=DEV)[1:].view(T, H)
+    elif form == "strides":
+        shift = shift.contiguous()
+    elif form == "columns":
+        scale = scale.t().contiguous().t()
+    else:
+        gate, scale, shift = (t.float() for t in (gate, scale, shift))
+    g, c, s = (t.repeat_interleave(L, 0).double() for t in (gate, scale, shift))
+    norm = lambda t: torch.nn.functional.layer_norm(t, (H,), eps=1e-6)  # noqa: E731
+    # three roundings to bf16 (2^-9 of values of up to 16, norms of up to 4
+    # times modulations of up to 5)
+    tol = dict(rtol=2 ** -7, atol=20 * 2 ** -8)
+    want = norm(x.double() + y.double()) * w.double() + b.double()
+    torch.testing.assert_close(
+        ops.add_layer_norm(x, y, w, b, 1e-6).double(), want, **tol)
+    total = x.double() + g * y.double()
+    new, got = ops.modulated_norm(x, scale, shift, L, 1e-6, y, gate)
+    torch.testing.assert_close(new.double(), total, **tol)
+    torch.testing.assert_close(got.double(), norm(total) * (1 + c) + s, **tol)
+    torch.testing.assert_close(ops.gated_add(x, y, gate, L).double(), total,
+                               **tol)
+
+
 @pytest.mark.parametrize("hq,hk,d", [(32, 8, 128), (12, 12, 64)])
 def test_rope(hq, hk, d):
     torch.manual_seed(3)
