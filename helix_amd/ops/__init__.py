@@ -7,6 +7,7 @@ logic is testable without a GPU.
 """
 from __future__ import annotations
 
+import functools
 import os
 from dataclasses import dataclass
 
@@ -550,21 +551,40 @@ def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 SUMS_MAX_M = 2048
 
 
+@functools.lru_cache(maxsize=4096)
 def _sums_tile(M: int, K: int, N: int) -> int:
-    """Tile of gemm_bf16_sums for M > 128 rows, 0 where the library is as
-    fast. A product that is three times as deep as wide has too few tiles to
-    fill the chip without stretches. With the norm that reads the result, us
-    of 4096 x 14336 and the library's: 200 rows 50 and 61 (128), 512 rows 80
-    and 97, 1024 rows 128 and 145, 1540 rows 197 and 337 (256). Between, too
-    few workgroups are left over: 768 rows 113 and 117, 1400 rows 185 and
-    181; products as deep as wide gain nothing (512 rows of 4096 x 4096: 36
-    and 35)."""
-    if not 128 < M <= SUMS_MAX_M or K < 3 * N or N > 8192:
+    """Tile of gemm_bf16_sums for M > 128 rows, 0 where the library takes no
+    longer. Stretches pay where a product has too few tiles to fill the chip:
+    at least two to a tile, and work for four fifths of it (256 workgroups of
+    256 x 256, 512 of 128 x 128).
+
+    Both sides are estimated in us, with the norm that reads the result, from
+    176 sizes measured with weights from memory (130 to 2048 rows of 1024 to
+    8192 columns, 4096 to 28672 deep). Ours, off by 3%: launches, steps of 64,
+    sums written and read. The library's, off by 5%: a launch, steps, 1.3
+    PFLOP/s, weights at 6 TB/s; a size in fifteen takes 1.4 to 2 times that
+    (1540 rows of 4096 x 14336 336 us, 194 in stretches; 1800 203 and 213), so
+    it has to be a tenth faster. Over the sizes 0.90 of the library's times, at
+    worst 1.08; some, the library's and ours: 200 rows of 4096 x 14336 63 and
+    49 (128), 512 98 and 79 (256), 1024 138 and 123; 640 rows of 8192 x 28672
+    273 and 347, left to the library."""
+    if not 128 < M <= SUMS_MAX_M or N > 8192:
         return 0
-    tiles = -(-M // 256) * -(-N // 256)
-    if M > 256 and tiles <= 256 and tiles * min(256 // tiles, 8) >= 208:
-        return 256
-    return 128 if M <= 640 else 0
+    steps = K // 64
+    library = 4 + 0.116 * steps + M * N * K / 650e6 + N * K / 3e6
+    best, tile = 1.1 * library, 0
+    for side, room, fixed, written in ((128, 512, 15.5, 59e6),
+                                       (256, 256, 12.4, 6.5e6)):
+        tiles = -(-M // side) * -(-N // side)
+        per = -(-steps // max(1, min(room // tiles, steps, 8)))
+        n = -(-steps // per)
+        if n < 2 or tiles * n < 0.8 * room:
+            continue
+        step = 1.55 if side == 256 else max(0.28, 0.6 * tiles * n / 256)
+        ours = fixed + per * step + n * M * N * 8 / written
+        if ours < best:
+            best, tile = ours, side
+    return tile
 
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

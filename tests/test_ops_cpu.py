@@ -220,3 +220,14 @@ def test_linear_with_a_vector():
     for z in (x, x[0]):
         assert torch.equal(ops.linear(z, w),
                            torch.nn.functional.linear(z, w))
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (128, 4096, 14336, 0), (130, 4096, 14336, 128), (512, 4096, 14336, 256),
+    (1540, 4096, 14336, 256), (2049, 4096, 14336, 0), (640, 8192, 28672, 0),
+    (2048, 8192, 28672, 0), (200, 1024, 4096, 0), (2048, 1024, 4096, 0),
+    (1024, 4096, 4096, 0), (200, 8200, 32768, 0), (130, 8, 64, 0)])
+def test_sums_tile(M, N, K, tile):
+    """Where the library's product is the faster one it stays: at the ends of
+    the range, where tiles alone fill the chip, where there is little to do."""
+    assert ops._sums_tile(M, K, N) == tile
