@@ -790,6 +790,26 @@ def test_gemm_bf16_few_rows(m, n, k, act):
                                atol=2e-5)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (65, 68, 768), (65, 68, 832), (66, 4, 1984), (129, 132, 2112),
+    (200, 260, 3136), (288, 1024, 4096), (300, 2052, 1600), (65, 8, 16448)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_bf16_stretches(m, n, k, bias):
+    """The deepest of its width that is whole and the shallowest in stretches,
+    the most stretches, last ones that are shorter, hardly a tile."""
+    torch.manual_seed(m)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV) if bias else None
+    got = ops.gemm_bf16(x, w, b, 1)
+    want = x.double() @ w.double().t()
+    if bias:
+        want += b.double()
+    want = torch.nn.functional.gelu(want, approximate="tanh")
+    # fp32 sums of k products and GELU's exponential, the rounding to bf16
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("m", [1, 15, 16, 17, 33, 48, 64, 65, 96, 97, 128])
 @pytest.mark.parametrize("n,k", [(8, 256), (72, 512), (4104, 2304),
                                  (256, 4096)])
