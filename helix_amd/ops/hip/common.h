@@ -122,6 +122,14 @@ __device__ __forceinline__ float block_reduce_max(float v, float* scratch) {
 
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
 
+// Workgroup number orig of nwg to the number of its work, such that works with
+// neighbouring numbers are done on one XCD: workgroups go round the 8 of them.
+__device__ __forceinline__ int xcd_chunk(int orig, int nwg) {
+  const int q = nwg / 8, r = nwg % 8;
+  const int xcd = orig % 8, pos = orig / 8;
+  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + pos;
+}
+
 // splitmix64 — cheap per-element RNG for sampling kernels.
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
   x += 0x9e3779b97f4a7c15ull;

@@ -44,13 +44,6 @@ struct Gemm {
   int M, N, K, m_tiles, n_tiles, stretch, gelu;
 };
 
-// Neighbouring numbers on one XCD.
-__device__ __forceinline__ int xcd_chunk(int orig, int nwg) {
-  const int q = nwg / 8, r = nwg % 8;
-  const int xcd = orig % 8, pos = orig / 8;
-  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + pos;
-}
-
 __device__ __forceinline__ float finish(float v, float b, int gelu) {
   v += b;
   return gelu ? gelu_tanh_f32(v) : v;

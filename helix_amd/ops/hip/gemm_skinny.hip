@@ -23,14 +23,6 @@ namespace {
 
 constexpr int BN = 128, BK = 64;
 
-// blockIdx.x -> linear tile id such that consecutive linear ids land on
-// the SAME XCD (hardware round-robins workgroups across the 8 XCDs).
-__device__ __forceinline__ int xcd_chunked(int orig, int nwg) {
-  const int q = nwg / 8, r = nwg % 8;
-  const int xcd = orig % 8, pos = orig / 8;
-  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + pos;
-}
-
 template <int BM>
 __global__ __launch_bounds__(256) void gemm_skinny_kernel(
     uint16_t* __restrict__ out,       // [M,N] bf16 (gridDim.z == 1)
@@ -43,7 +35,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(
   __shared__ uint16_t b_lds[BN * BK];
 
   int lin = blockIdx.x;
-  if (swz) lin = xcd_chunked(lin, gridDim.x);
+  if (swz) lin = xcd_chunk(lin, gridDim.x);
   const int tile_m = lin % mtiles;
   const int tile_n = lin / mtiles;
   const int m0 = tile_m * BM, n0 = tile_n * BN;

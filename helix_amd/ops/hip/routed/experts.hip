@@ -39,13 +39,6 @@ __device__ __forceinline__ float finish(const Mix& m, float v) {
   return u * u;
 }
 
-// Workgroups of neighbouring tiles on one XCD.
-__device__ __forceinline__ int xcd_chunk(int orig, int nwg) {
-  const int q = nwg / 8, r = nwg % 8;
-  const int xcd = orig % 8, pos = orig / 8;
-  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + pos;
-}
-
 // --- streams: 16 MI rows x 16 NI columns of a workgroup; a wave has every
 // fourth stretch of 32 U of the inner dimension.
 template <int MI, int NI, int U>
