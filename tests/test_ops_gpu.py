@@ -317,7 +317,7 @@ def test_gemm_bf16(m, n, k):
     (1, 8, 64), (33, 70, 128), (64, 62, 64),          # tiles of 32 x 64
     (65, 64, 192), (130, 1030, 64),                   # of 64
     (2049, 2050, 64),                                 # of 128
-    (3585, 3500, 64),                                 # of 256
+    (3585, 3500, 64),                                 # of 128 as well
 ])
 def test_gemm_bf16_tiles(m, n, k, act):
     """Remainders of rows and columns for every tile, one step and several,
@@ -493,6 +493,46 @@ def test_paged_attn_decode_edges(hq, hkv, d, bs, fp8, window, lens):
                                 bt.to(DEV), seq_lens.to(DEV), d ** -0.5,
                                 window=window)
     # rounded to bf16 (2^-9, doubled); sums of 32 bits over <= 1500 values
+    torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
+                               atol=5e-5)
+
+
+@pytest.mark.parametrize("hq,hkv,window,lens", [
+    # the search goes on past 64 sequences; pieces of several units
+    (16, 8, 0, [0, 1, 1500] + [1 + 397 * i % 1500 for i in range(67)]),
+    (16, 8, 0, [1 + 211 * i % 1500 for i in range(129)]),
+    (4, 4, 300, [20 + 397 * i % 1500 for i in range(100)]),
+    # as many pieces as there can be, the last ones shorter or empty
+    (16, 8, 0, [20000, 129, 13001, 7937]),
+    (8, 8, 0, [0, 0, 5000]),
+    (2, 1, 0, [128 * 9]),
+])
+@pytest.mark.parametrize("bucket,parts", [(1, None), (4, None), (1, 3)])
+def test_paged_attn_decode_cuts(hq, hkv, window, lens, bucket, parts):
+    """Work cut on the device: bounds far above the lengths, as a captured
+    graph has them, and workspaces of fewer pieces than there could be."""
+    torch.manual_seed(40)
+    B, bs, d = len(lens), 16, 64
+    need = [-(-n // bs) for n in lens]
+    q = torch.randn(B, hq, d, dtype=torch.bfloat16)
+    kc = torch.randn(sum(need), hkv, bs, d, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    bt = torch.zeros(B, max(need), dtype=torch.int32)
+    for b, pages in enumerate(torch.randperm(sum(need)).int().split(need)):
+        bt[b, :need[b]] = pages
+    seq_lens = torch.tensor(lens, dtype=torch.int32)
+    full = [b for b in range(B) if lens[b]]
+    want = torch.zeros(B, hq, d)
+    want[full] = ref.paged_attn_decode(
+        q[full].float(), kc.float(), vc.float(), bt[full], seq_lens[full],
+        d ** -0.5, window)
+    max_len = bucket * max(lens)
+    ws = ops.decode_workspace(B, hq, d, 128 * parts if parts else max_len, DEV)
+    got = ops.paged_attn_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                                seq_lens.to(DEV), d ** -0.5, ws, max_len,
+                                window)
+    # rounded to bf16 (2^-9, doubled); sums of 32 bits over <= 20000 values of
+    # weights that add up to 1
     torch.testing.assert_close(got.float().cpu(), want, rtol=2 ** -8,
                                atol=5e-5)
 
@@ -875,6 +915,22 @@ def test_gemm_bf16_pair():
     got = ops.gemm_bf16(x, w, None)
     torch.testing.assert_close(got.double(), x.double() @ w.double().t(),
                                rtol=2 ** -8, atol=2e-5)
+
+
+@pytest.mark.parametrize("n,act", [(3002, 0), (3002, 1), (3004, 1)])
+def test_gemm_bf16_pair_epilogue(n, act):
+    """Bias and GELU of 256 x 256 tiles, columns stored one and four at a
+    time."""
+    torch.manual_seed(41)
+    x = torch.randn(4000, 2112, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, 2112, dtype=torch.bfloat16, device=DEV) / 46
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    got = ops.gemm_bf16(x, w, b, act)
+    want = x.double() @ w.double().t() + b.double()
+    if act:
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    # fp32 sums of k products and GELU's exponential, the rounding to bf16
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2e-5)
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 8, 512), (17, 72, 1024),
