@@ -139,14 +139,14 @@ class HLinear(nn.Linear):
     kernel, prefill-shaped ones stay on hipBLASLt.
 
     A plain call returns rows [T, N]. The modules here ask each other for
-    other forms (_own says when): "sums" -> what ops.linear_sums gives, for a
-    reader that adds it up; "glu" -> silu(first half) * second half."""
+    other forms (_own says when): "sums" -> what ops.linear_sums_or_rows
+    gives, for a reader that adds it up; "glu" -> silu(first half) * second half."""
 
     def forward(self, x: torch.Tensor, form: str = "rows") -> torch.Tensor:
         if self.bias is None and form == "sums":
-            return ops.linear_sums(x, self.weight)
+            return ops.linear_sums_or_rows(x, self.weight)
         if self.bias is None and form == "glu":
-            return ops.linear_silu_mul(x, self.weight)
+            return ops.gated_linear(x, self.weight)
         out = ops.linear(x, self.weight, self.bias)
         return ops.silu_and_mul(out) if form == "glu" else out
 

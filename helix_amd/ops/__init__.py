@@ -517,7 +517,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     is faster (28672 x 4096: 45 against 65 us) but for vocabularies (128256 x
     4096: 191 against 189); from 17 to 64 rows it stays so where the inner
     dimension is the longer one (4096 x 14336: 30 against 34 and 35 against
-    42), elsewhere adding up the stretches costs what it gains."""
+    42), elsewhere adding up the stretches costs what it gains. From 65 rows on
+    see _rows_many."""
     if (_SKINNY_ENABLED and x.is_cuda and x.dtype == torch.bfloat16
             and x.dim() == 2
             and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= _SKINNY_MAX_M
@@ -526,11 +527,23 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
         return gemm_skinny_bf16(x, w, bias)
     if _rows_fit(x, w) and _bias_fits(bias, w):
         (M, K), N = x.shape, w.shape[0]
-        if (M <= 16 and N <= 65536 or K >= 2 * N or M > 64 and N <= 8192):
+        if (M <= 16 and N <= 65536 or K >= 2 * N if M <= 64 else
+                _rows_many(N, K) and (N <= 6144 or K > N)):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             _native().gemm_rows(out, x, w, bias, None, None)
             return out
     return torch.nn.functional.linear(x, w, bias)
+
+
+def _rows_many(N: int, K: int) -> bool:
+    """Whether 65 to 128 rows stream their weights: matrices of some 2^24
+    values, neither wide, for which x is read too often, nor small, which the
+    library's tiles fill the chip with at a launch's cost. us at 128 rows,
+    streamed and joined, and the library's: 4096 x 8192 28 and 44, 2048 x 8192
+    20.5 and 21.8, 1024 x 14336 21 and 26, 4096 x 4096 20 and 25; 6144 x 2048 22
+    and 18, 1024 x 8192 17.5 and 15.4, 2048 x 2048 17 and 9, 14336 x 4096 65
+    and 51."""
+    return N <= 8192 and N * K >= 13 << 20
 
 
 def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -539,13 +552,23 @@ def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     rows, else [M, N] in x's type. Wide matrices fill the chip without
     stretches, and 64 rows of 16384 sums are more bytes than they save. At 64
     rows of 6144 x 4096 it is 17.6 us against the library's 18.0, at 128 rows
-    20 against 25. From 129 rows on see _sums_tile."""
+    20 against 25. From 65 rows on see _rows_many, from 129 on _sums_tile."""
     if _rows_fit(x, w) and w.shape[0] <= 8192:
         return _native().gemm_rows_sums(x, w, None, None)
     tile = _sums_tile(*x.shape, w.shape[0]) if x.dim() == 2 else 0
     if tile and _rows_fit(x, w, SUMS_MAX_M):
         return _native().gemm_bf16_sums(x, w, tile)
     return linear(x, w)
+
+
+def linear_sums_or_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear_sums where stretches are the faster form for its reader, rows
+    [M, N] elsewhere: 65 to 128 rows of a small or wide matrix (with the norm,
+    us at 128 rows of 2048 x 2048: 20.9 and 11.8)."""
+    if x.dim() == 2 and 64 < x.shape[0] <= ROWS_MAX_M \
+            and not _rows_many(*w.shape):
+        return linear(x, w)
+    return linear_sums(x, w)
 
 
 SUMS_MAX_M = 2048
@@ -587,6 +610,23 @@ def _sums_tile(M: int, K: int, N: int) -> int:
     return tile
 
 
+def _glu_fits(M: int, N: int, K: int) -> bool:
+    """Whether the gated product of a few rows takes no longer than product and
+    activation apart. It is not cut along the inner dimension, so it needs
+    columns enough to fill the chip, or few chunks. us apart and at once, with
+    weights from memory: one row of 28672 x 4096 66 and 50, 10240 x 4096 28 and
+    29, 4096 x 4096 18 and 27, 16384 x 1024 12.3 and 10.2. From 17 rows on x is read by
+    every workgroup, and the library's product is the faster one but for inner
+    dimensions of a power of two: 64 rows of 28672 x 4096 60 and 60, 17 of them
+    62 and 51, 64 of 28672 x 5120 64 and 75, of 57344 x 8192 192 and 218. Widths
+    that the activation alone does not take go here."""
+    if K <= 1024 or N % 16 != 0:
+        return True
+    if M <= 16:
+        return N >= 3 * K
+    return N >= 13 << 11 and K in (2048, 4096)
+
+
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T), w = [gate; up]. A few rows: one launch,
     whose halves stay in registers (55 us at 64 rows of 2 x 14336 x 4096,
@@ -597,6 +637,14 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         _native().gemm_rows_glu(out, x, w, None, None)
         return out
     return silu_and_mul(linear(x, w))
+
+
+def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear_silu_mul where one launch is the faster form, product and
+    activation apart elsewhere."""
+    if x.dim() == 2 and w.dim() == 2 and not _glu_fits(x.shape[0], *w.shape):
+        return silu_and_mul(linear(x, w))
+    return linear_silu_mul(x, w)
 
 
 def gemm_fp8_sums(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,

@@ -231,3 +231,15 @@ def test_sums_tile(M, N, K, tile):
     """Where the library's product is the faster one it stays: at the ends of
     the range, where tiles alone fill the chip, where there is little to do."""
     assert ops._sums_tile(M, K, N) == tile
+
+
+def test_few_rows_where_they_pay():
+    """The lines between the products of few rows and the library's."""
+    many = ops._rows_many
+    assert many(4096, 4096) and many(1024, 14336) and many(8192, 2048)
+    assert not (many(6144, 2048) or many(1024, 8192) or many(14336, 4096))
+    glu = ops._glu_fits
+    assert glu(1, 28672, 4096) and glu(16, 12288, 4096) and glu(64, 64, 1024)
+    assert glu(17, 28672, 4096) and glu(64, 26624, 2048)
+    assert not (glu(1, 8192, 4096) or glu(17, 26560, 4096) or
+                glu(32, 28672, 5120) or glu(64, 57344, 8192))

@@ -892,6 +892,45 @@ def test_gemm_rows(m, n, k):
             atol=5e-5)
 
 
+@pytest.mark.parametrize("m", [1, 17, 64])
+@pytest.mark.parametrize("n,k", [(4104, 2304), (256, 4096), (26624, 2048),
+                                 (512, 512)])
+def test_gemm_rows_forms(m, n, k):
+    """The gated form and the joined one of at most two chunks, on either side
+    of the rules that take them."""
+    torch.manual_seed(42)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    want = x.double() @ w.double().t()
+    g, u = want.chunk(2, -1)
+    glu = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_rows_glu(glu, x, w, None, None)
+    with torch.inference_mode():
+        rows, whole = ops.linear(x, w), ops.gated_linear(x, w)
+    # fp32 sums of k products, then the rounding to bf16
+    torch.testing.assert_close(rows.double(), want, rtol=2 ** -8, atol=2e-5)
+    gated = torch.nn.functional.silu(g) * u
+    torch.testing.assert_close(glu.double(), gated, rtol=2 ** -8, atol=5e-5)
+    # apart, both halves are rounded as well: 2^-9 each of up to 5 x 5
+    torch.testing.assert_close(whole.double(), gated, rtol=2 ** -7,
+                               atol=25 * 2 ** -8)
+
+
+@pytest.mark.parametrize("m", [64, 65, 128, 129])
+def test_linear_sums_or_rows(m):
+    torch.manual_seed(43)
+    for n, k, many in ((2048, 2048, False), (4096, 4096, True)):
+        x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+        w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+        with torch.inference_mode():
+            got = ops.linear_sums_or_rows(x, w)
+        assert m > 128 or (got.dim() == 3) == (many or m <= 64)
+        if got.dim() == 3:
+            got = got.sum(0)
+        torch.testing.assert_close(got.double(), x.double() @ w.double().t(),
+                                   rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("m,n,k", [(1, 8, 64), (257, 260, 192),
                                    (130, 516, 4160), (700, 1024, 1088)])
