@@ -184,7 +184,8 @@ def gather_kv(k_cache: torch.Tensor, v_cache: torch.Tensor,
             blk.shape == off.shape and blk.dim() == 1 and
             all(t.dtype == torch.int64 and t.is_contiguous() and
                 t.device == k_cache.device for t in (blk, off)) and
-            v_cache.device == k_cache.device and _aligned(k_cache, v_cache)):
+            v_cache.device == k_cache.device and _aligned(k_cache, v_cache) and
+            k_cache.get_device() == torch.cuda.current_device()):
         k = torch.empty(blk.numel(), k_cache.shape[1], k_cache.shape[3],
                         dtype=dtype, device=k_cache.device)
         v = torch.empty_like(k)
@@ -369,7 +370,8 @@ def quantize_fp8(t: torch.Tensor, dim: int = -1):
     Returns (bytes uint8 view, float32 scales)."""
     if t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 2 and \
             dim in (-1, 1) and t.shape[1] > 0 and t.shape[1] % 8 == 0 and \
-            t.is_contiguous() and t.data_ptr() % 16 == 0:
+            t.is_contiguous() and _aligned(t) and \
+            t.get_device() == torch.cuda.current_device():
         q = torch.empty(t.shape, dtype=torch.uint8, device=t.device)
         scale = torch.empty(t.shape[0], dtype=torch.float32, device=t.device)
         _native().quantize_rows(q, scale, t)
@@ -476,30 +478,35 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, most: int = ROWS_MAX_M,
     """Whether the kernel for a few rows takes x @ w^T, bf16 or e4m3 bytes.
     It knows nothing of gradients, so where it stands for torch's product
     (grads) bf16 only runs where there are none to be had."""
-    return (x.is_cuda and _eager() and x.dim() == 2 and w.dim() == 2
-            and 0 < x.shape[0] <= most
-            and (x.dtype == torch.uint8 or x.dtype == torch.bfloat16
-                 and (not grads or torch.is_inference_mode_enabled()))
-            and x.dtype == w.dtype and x.device == w.device
-            and x.get_device() == torch.cuda.current_device()
-            and x.shape[1] == w.shape[1] > 0
-            and x.shape[1] * x.element_size() % ROWS_CHUNK == 0
-            and w.shape[0] > 0 and w.shape[0] % 8 == 0
-            and x.is_contiguous() and w.is_contiguous() and _aligned(x, w))
-
-
-def _eager() -> bool:
-    """Neither under autocast nor a tracer, which have to see torch's own."""
-    return not (torch.jit.is_tracing() or torch.compiler.is_compiling()
-                or torch.is_autocast_enabled("cuda"))
+    if not x.is_cuda or torch.jit.is_tracing() or x.dim() != 2 \
+            or w.dim() != 2:
+        return False
+    (M, K), (N, Kw) = x.shape, w.shape
+    if not 0 < M <= most or N == 0 or N % 8 != 0 or not 0 < K == Kw:
+        return False
+    dtype = x.dtype
+    if dtype == torch.bfloat16:
+        if K * 2 % ROWS_CHUNK or grads and not torch.is_inference_mode_enabled():
+            return False
+    elif dtype != torch.uint8 or K % ROWS_CHUNK:
+        return False
+    return (dtype == w.dtype and x.is_contiguous() and w.is_contiguous()
+            and x.get_device() == w.get_device() == torch.cuda.current_device()
+            and _aligned(x, w)
+            # those have to see torch's own
+            and not torch.is_autocast_enabled("cuda")
+            and not torch.compiler.is_compiling())
 
 
 def _aligned(*ts: torch.Tensor) -> bool:
     """Whether these are memory, on 16-byte boundaries."""
     try:
-        return all(t.data_ptr() % 16 == 0 for t in ts)
+        for t in ts:
+            if t.data_ptr() & 15:
+                return False
     except RuntimeError:           # within vmap and the like they have none
         return False
+    return True
 
 
 def _bias_fits(bias, w: torch.Tensor) -> bool:
