@@ -414,14 +414,15 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
     weights instead of going by tiles (us with weights from memory, tiles and
     streamed: 8 rows of 6144 x 1024 14.1 and 7.6, 33 of 768 x 3072 25.1 and
     7.3, 64 of 3072 x 768 9.0 and 8.2); up to 128 where the inner dimension is
-    the longer one (768 x 3072 26.9 and 14.1), else tiles are as fast (2304 x
-    768 9.6 and 12.3)."""
+    long (2048 x 8192 23.8 and 20.5, 1024 x 8192 23.0 and 17.5), else tiles or
+    their stretches are as fast (1024 x 2048 11.9 and 12.9, 2304 x 768 9.6 and
+    12.3)."""
     if x.is_cuda:
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
         if (x.dtype == torch.bfloat16 and _bias_fits(bias, w) and
-                _rows_fit(x, w, 128 if w.shape[1] >= 2 * w.shape[0] else 64,
-                          grads=False)):
+                _rows_fit(x, w, 128 if w.shape[1] >= max(
+                    2 * w.shape[0], 4096) else 64, grads=False)):
             _native().gemm_rows(out, x, w, bias, None, None, act == 1)
         else:
             _native().gemm_bf16(out, x, w, bias, act)
