@@ -430,6 +430,9 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
     return ref.gemm_bf16(x, w, bias, act)
 
 
+# The earlier kernel for few rows: called directly, or by linear with
+# HELIX_SKINNY_GEMM=1. Llama's projections ask linear_sums and linear_silu_mul
+# first, so that switch compares little of a decode step.
 _SKINNY_MAX_M = 1024
 _SKINNY_SCRATCH: dict = {}        # device -> fp32 workspace tensor
 _SKINNY_SWIZZLE = os.environ.get("HELIX_SKINNY_SWIZZLE", "1") == "1"

@@ -1,8 +1,9 @@
 // bf16 MFMA GEMM for gfx950: out[M,N] = act(x[M,K] @ w[N,K]^T + bias).
 //
 // The encoder's and the image model's projections (act: none or GELU, tanh) of
-// more than a few rows, and Llama's narrow ones at a few hundred rows, whose inner dimension is cut
-// into stretches that a later reader adds up (fp32 [stretch][M][N]).
+// more than a few rows, and Llama's deep ones at a few hundred rows, whose inner
+// dimension is cut into stretches that a later reader adds up (fp32
+// [stretch][M][N]).
 //
 // Bound by the matrix cores and by LDS reads, which take about as long. Tiles
 // of both operands go straight to LDS; their 16-byte pieces lie crosswise, so
@@ -14,15 +15,19 @@
 //    on the same SIMDs. Four tiles of 32 of the inner dimension are in LDS.
 //  - smaller tiles with two buffers of 64 and one barrier a step; several
 //    workgroups on a CU fill each other's gaps.
+//  - 128 x 128 tiles in stretches where tiles leave CUs idle (cut).
 //
 // Before, 128 x 128 tiles of all sizes, one buffer, rows as in memory (8 lanes
-// on a bank). us before -> now (tile; TFLOP/s), M x N x K:
-//   16600 x 2304 x 768   131 -> 104  (128; 568)   2304 x 3072 x 1024  33 -> 23
-//   16600 x 768 x 768     54 -> 35   (128; 565)   2304 x 1024 x 1024  28 -> 13
-//   16600 x 3072 x 768   203 -> 126  (128; 623)   2304 x 4096 x 1024  68 -> 37
-//   16600 x 768 x 3072   149 -> 82   (256; 956)   2304 x 1024 x 4096  86 -> 41
-//   300 x 768 x 3072      66 -> 17   (64)         8 x 6144 x 1024     21 -> 6
-// 8192^3 runs at 1240 TFLOP/s. 256 x 256 as 128 is, with two buffers, takes 10%
+// on a bank). us before -> now with weights in the caches (tile, or stretches of
+// 128; TFLOP/s), M x N x K:
+//   16600 x 2304 x 768   131 -> 105  (128; 562)   2304 x 3072 x 1024  33 -> 24
+//   16600 x 768 x 768     54 -> 35   (128; 557)   2304 x 1024 x 1024  28 -> 13
+//   16600 x 3072 x 768   203 -> 123  (128; 639)   2304 x 4096 x 1024  68 -> 36
+//   16600 x 768 x 3072   149 -> 83   (256; 950)   2304 x 1024 x 4096  86 -> 36
+//   300 x 768 x 3072      66 -> 14   (6 stretches; the one above: 3)
+// Products of few rows stream their weights instead (gemm_rows.hip): 8 x 6144 x
+// 1024 takes 6.4 from the caches, 7.6 from memory, by tiles 14.1.
+// 8192^3 runs at 1248 TFLOP/s. 256 x 256 as 128 is, with two buffers, takes 10%
 // longer; three buffers, steps of 32 for the smaller tiles, 256 x 128 and
 // scheduling hints for the reads from LDS gave nothing. Tile counts: 108 of
 // 256 against 432 of 128 (2304 x 3072 x 1024) 34 and 23; 144 of 128 against

@@ -7,7 +7,7 @@
 // lies at p ^ r % 16, so operands leave LDS without bank conflicts.
 //
 // Narrow matrices leave CUs idle, so the inner dimension is cut into stretches
-// until there are about WANT workgroups. Their sums (fp32, [stretch][M][N])
+// until there are about as many workgroups as Shape wants (cut). Their sums (fp32, [stretch][M][N])
 // are added by whatever reads the result (norm, rotation), in order, or by a
 // launch of their own; nothing is added with atomics.
 //
