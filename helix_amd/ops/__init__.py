@@ -84,35 +84,13 @@ def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor,
     return ref.layer_norm(x, w, b, eps)
 
 
-def _rows_of_8(*rows: torch.Tensor | None) -> bool:
-    """Whether encoder.hip takes these rows (a lane has up to 8 vectors)."""
-    x, *more = (t for t in rows if t is not None)
-    return (x.is_cuda and x.dim() == 2
-            and x.shape[1] % 8 == 0 and x.shape[1] <= 4096
-            and all(t.dtype == torch.bfloat16 and t.device == x.device
-                    and t.shape == x.shape and t.is_contiguous()
-                    for t in (x, *more)) and _aligned(x, *more))
-
-
-def _modulates(x: torch.Tensor, L: int, *rows: torch.Tensor | None) -> bool:
-    """Whether encoder.hip takes these rows for every L of x: slices of one
-    product, or packed."""
-    first, *more = (t for t in rows if t is not None)
-    return (first.dim() == 2 and first.stride(0) % 8 == 0
-            and first.shape[0] * L >= x.shape[0]
-            and all(t.dtype == torch.bfloat16 and t.device == x.device
-                    and t.shape == (first.shape[0], x.shape[1])
-                    and t.stride() == (first.stride(0), 1)
-                    for t in (first, *more)) and _aligned(first, *more))
-
-
 def add_layer_norm(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor,
                    b: torch.Tensor, eps: float) -> torch.Tensor:
     """Layer norm of x + y."""
-    if _rows_of_8(x, y) and _aligned(w, b):
+    if x.is_cuda:
         out = torch.empty_like(x)
-        _native().add_norm(None, out, x, y, None, w, b, 0, eps)
-        return out
+        if _native().add_norm(None, out, x, y, None, w, b, 0, eps):
+            return out
     return layer_norm((x.float() + y.float()).to(x.dtype), w, b, eps)
 
 
@@ -122,12 +100,12 @@ def modulated_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor,
     """(s, norm(s) (1 + scale) + shift), s = x + gate y (x without y). norm
     is a layer norm without weights; gate, scale and shift have a row for
     every L rows of x."""
-    if _rows_of_8(x, y) and _modulates(x, L, scale, shift, gate):
+    if x.is_cuda:
         out = torch.empty_like(x)
         s = x if y is None else torch.empty_like(x)
-        _native().add_norm(None if y is None else s, out, x, y, gate, scale,
-                           shift, L, eps)
-        return s, out
+        if _native().add_norm(None if y is None else s, out, x, y, gate,
+                              scale, shift, L, eps):
+            return s, out
     if y is not None:
         x = gated_add(x, y, gate, L)
     h = x.shape[-1]
@@ -140,10 +118,10 @@ def modulated_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor,
 def gated_add(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor,
               L: int) -> torch.Tensor:
     """x + gate y; gate has a row for every L rows of x."""
-    if _rows_of_8(x, y) and _modulates(x, L, gate):
+    if x.is_cuda:
         out = torch.empty_like(x)
-        _native().gated_add(out, x, y, gate, L)
-        return out
+        if _native().gated_add(out, x, y, gate, L):
+            return out
     g = gate.repeat_interleave(L, dim=0)
     return (x.float() + g.float() * y.float()).to(x.dtype)
 
@@ -420,9 +398,9 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
     if x.is_cuda:
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
-        if (x.dtype == torch.bfloat16 and _bias_fits(bias, w) and
-                _rows_fit(x, w, 128 if w.shape[1] >= max(
-                    2 * w.shape[0], 4096) else 64, grads=False)):
+        if (_rows_fit(x, w, 128 if w.shape[1] >= max(2 * w.shape[0], 4096)
+                      else 64, grads=False)
+                and x.dtype == torch.bfloat16 and _bias_fits(bias, w)):
             _native().gemm_rows(out, x, w, bias, None, None, act == 1)
         else:
             _native().gemm_bf16(out, x, w, bias, act)
@@ -482,11 +460,11 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, most: int = ROWS_MAX_M,
     """Whether the kernel for a few rows takes x @ w^T, bf16 or e4m3 bytes.
     It knows nothing of gradients, so where it stands for torch's product
     (grads) bf16 only runs where there are none to be had."""
-    if not x.is_cuda or torch.jit.is_tracing() or x.dim() != 2 \
-            or w.dim() != 2:
+    if not x.is_cuda or x.dim() != 2 or x.shape[0] > most or w.dim() != 2 \
+            or torch.jit.is_tracing():
         return False
     (M, K), (N, Kw) = x.shape, w.shape
-    if not 0 < M <= most or N == 0 or N % 8 != 0 or not 0 < K == Kw:
+    if M == 0 or N == 0 or N % 8 != 0 or not 0 < K == Kw:
         return False
     dtype = x.dtype
     if dtype == torch.bfloat16:

@@ -4,11 +4,11 @@
 void rms_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w, double eps);
 void fused_add_rms_norm(torch::Tensor x, torch::Tensor residual,
                         torch::Tensor w, double eps);
-void add_norm(c10::optional<torch::Tensor> sum, torch::Tensor out,
+bool add_norm(c10::optional<torch::Tensor> sum, torch::Tensor out,
               torch::Tensor x, c10::optional<torch::Tensor> y,
               c10::optional<torch::Tensor> gate, torch::Tensor a,
               torch::Tensor b, int64_t L, double eps);
-void gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
+bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L);
 void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
                        torch::Tensor residual, torch::Tensor w, double eps);

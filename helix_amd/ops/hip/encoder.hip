@@ -101,85 +101,94 @@ __global__ __launch_bounds__(NT) void gated_add_kernel(Rows m, int64_t total) {
   store_bf16x8(m.out + i, x);
 }
 
-void check(const torch::Tensor& t, const Rows& m, bool rows) {
-  TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
-              t.size(-1) == m.H && t.stride(-1) == 1 &&
-              (uintptr_t)t.data_ptr() % 16 == 0);
-  if (rows)
-    TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.size(0) == m.T);
+// Whether these are values as the kernels read them: bf16 on x's device, on
+// 16-byte boundaries.
+bool reads(const torch::Tensor& t, const torch::Tensor& x) {
+  return t.scalar_type() == torch::kBFloat16 && t.device() == x.device() &&
+         (uintptr_t)t.data_ptr() % 16 == 0;
 }
-
-// A row per image, all of one stride.
-const uint16_t* of_image(const torch::Tensor& t, Rows& m) {
-  check(t, m, false);
-  TORCH_CHECK(t.dim() == 2 && t.stride(0) % 8 == 0 && m.L > 0 &&
-              t.size(0) * m.L >= m.T &&
-              (m.mod_stride == 0 || m.mod_stride == t.stride(0)));
+// Packed rows like x.
+bool like(const torch::Tensor& t, const torch::Tensor& x) {
+  return reads(t, x) && t.is_contiguous() && t.sizes() == x.sizes();
+}
+// A row for every L of x, each as far from the next as m's others.
+bool of_image(const torch::Tensor& t, const torch::Tensor& x, Rows& m,
+              const uint16_t** at) {
+  if (!reads(t, x) || t.dim() != 2 || t.size(1) != m.H || t.stride(1) != 1 ||
+      t.stride(0) % 8 != 0 || m.L <= 0 || t.size(0) * m.L < m.T ||
+      (m.mod_stride != 0 && m.mod_stride != t.stride(0)))
+    return false;
   m.mod_stride = t.stride(0);
-  return (const uint16_t*)t.data_ptr();
+  *at = (const uint16_t*)t.data_ptr();
+  return true;
 }
 
-Rows rows_of(const torch::Tensor& x, const torch::Tensor& out, int64_t L) {
-  Rows m{};
+bool rows_of(const torch::Tensor& x, const torch::Tensor& out, int64_t L,
+             Rows& m) {
+  if (!x.is_cuda() || x.dim() != 2 || x.size(1) % 8 != 0 || x.size(1) > 4096 ||
+      !like(x, x) || !like(out, x))
+    return false;
   m.T = x.size(0);
-  m.H = x.size(-1);
+  m.H = x.size(1);
   m.L = L;
-  TORCH_CHECK(m.H % 8 == 0);
-  check(x, m, true);
-  check(out, m, true);
   m.x = (const uint16_t*)x.data_ptr();
   m.out = (uint16_t*)out.data_ptr();
-  return m;
+  return true;
 }
 
 }  // namespace
 
 // L = 0: out = norm(x + y) a + b with weights a, b; else rows of images of L
-// tokens each: sum = x + gate y, out = norm(sum) (1 + a) + b.
-void add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
+// tokens each: sum = x + gate y, out = norm(sum) (1 + a) + b. False, and nothing
+// done, for other forms of operands than the kernel reads.
+bool add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
               torch::Tensor a, torch::Tensor b, int64_t L, double eps) {
-  Rows m = rows_of(x, out, L);
+  Rows m{};
+  if (!rows_of(x, out, L, m)) return false;
   m.eps = (float)eps;
   if (y.has_value()) {
-    check(*y, m, true);
+    if (!like(*y, x)) return false;
     m.y = (const uint16_t*)y->data_ptr();
   }
   if (sum.has_value()) {
-    check(*sum, m, true);
+    if (!like(*sum, x)) return false;
     m.sum = (uint16_t*)sum->data_ptr();
   }
   if (L > 0) {
-    m.a = of_image(a, m);
-    m.b = of_image(b, m);
-    if (gate.has_value()) m.gate = of_image(*gate, m);
+    if (!of_image(a, x, m, &m.a) || !of_image(b, x, m, &m.b) ||
+        (gate.has_value() && !of_image(*gate, x, m, &m.gate)))
+      return false;
   } else {
-    check(a, m, false);
-    check(b, m, false);
-    TORCH_CHECK(a.dim() == 1 && b.dim() == 1 && !gate.has_value());
+    for (const auto& t : {a, b})
+      TORCH_CHECK(t.scalar_type() == torch::kBFloat16 && t.is_contiguous() &&
+                  t.dim() == 1 && t.numel() == m.H, "weights of H values");
+    if (!reads(a, x) || !reads(b, x) || gate.has_value()) return false;
     m.a = (const uint16_t*)a.data_ptr();
     m.b = (const uint16_t*)b.data_ptr();
   }
-  if (m.T == 0) return;
+  if (m.T == 0) return true;
   const dim3 grid(cdiv(m.T, NT / WAVE));
   auto stream = at::hip::getCurrentHIPStream();
 #define HELIX_AN(NV)                                                         \
   hipLaunchKernelGGL(add_norm_kernel<NV>, grid, dim3(NT), 0, stream, m)
-  TORCH_CHECK(m.H <= 8 * 512, "rows of at most 4096");
   if (m.H <= 512) HELIX_AN(1);
   else if (m.H <= 1024) HELIX_AN(2);
   else if (m.H <= 2048) HELIX_AN(4);
   else HELIX_AN(8);
 #undef HELIX_AN
+  return true;
 }
 
-void gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
+// out = x + gate y; false as above.
+bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L) {
-  Rows m = rows_of(x, out, L);
-  check(y, m, true);
+  Rows m{};
+  if (!rows_of(x, out, L, m) || !like(y, x) || !of_image(gate, x, m, &m.gate))
+    return false;
   m.y = (const uint16_t*)y.data_ptr();
-  m.gate = of_image(gate, m);
   const int64_t total = (int64_t)m.T * m.H;
-  if (total == 0) return;
+  if (total == 0) return true;
   hipLaunchKernelGGL(gated_add_kernel, dim3((total / 8 + NT - 1) / NT),
                      dim3(NT), 0, at::hip::getCurrentHIPStream(), m, total);
+  return true;
 }

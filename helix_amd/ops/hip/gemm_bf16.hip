@@ -302,21 +302,22 @@ void run_pair(Gemm m, uint16_t* out, const uint16_t* x, const uint16_t* w,
 // by a launch; 1 where whole tiles take no longer. Both are estimated in us:
 //   whole:      0.6 a step of 64, times rounds of 256 tiles
 //   stretches:  6, 0.6 a step or 0.37 for each 256 workgroups, and their sums
-//               written and read at 4.5 TB/s
+//               written and read at 4.5 TB/s; 4 more, as the launch that joins
+//               them costs a host that is behind
 // from 693 sizes (66 to 4500 rows of 256 to 4096 columns, 512 to 14336 deep,
 // weights from memory) timed whole and in 2, 3, 4, 6 and 8 stretches. What is
-// taken is within 1.3% of the best of these, at worst 24%; whole tiles alone
+// taken is within 2.2% of the best of these, at worst 48%; whole tiles alone
 // take 1.54 times as long. Some, whole and as taken: 2304 x 1024 x 4096 48.1
 // and 36.3, 300 of its rows 44.0 and 18.5, 700 x 768 x 3072 25.5 and 19.0, 200
-// x 2048 x 2048 21.1 and 16.0, 66 x 768 x 1024 10.9 and 8.4; as taken and in
-// two: 1000 x 768 x 1024 11.3 and 15.1, 1500 x 4096 x 4096 64.9 and 75.3.
+// x 2048 x 2048 21.1 and 16.0; as taken and in two: 1000 x 768 x 1024 11.3 and
+// 15.1, 1500 x 4096 x 4096 64.9 and 75.3.
 int cut(Gemm& m) {
   const int tiles = cdiv(m.M, 128) * cdiv(m.N, 128), steps = m.K / 64;
   if (m.M <= 64 || m.N % 4 != 0) return 1;
   float best = 0.6f * steps * std::max(1.f, tiles / 256.f);
   int n = 1;
   for (int i = 2; i <= std::min(steps, 8); ++i) {
-    const float us = 6 + cdiv(steps, i) * std::max(0.6f, 0.37f * tiles * i / 256)
+    const float us = 10 + cdiv(steps, i) * std::max(0.6f, 0.37f * tiles * i / 256)
                      + 8.f * i * m.M * m.N / 4.5e6f;
     if (us < best) best = us, n = i;
   }

@@ -831,7 +831,7 @@ def test_gemm_bf16_few_rows(m, n, k, act):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (65, 68, 768), (65, 68, 832), (66, 4, 1984), (129, 132, 2112),
+    (65, 68, 1216), (65, 68, 1280), (66, 4, 1984), (129, 132, 2112),
     (200, 260, 3136), (288, 1024, 4096), (300, 2052, 1600), (65, 8, 16448)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_gemm_bf16_stretches(m, n, k, bias):
