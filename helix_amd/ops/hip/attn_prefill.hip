@@ -331,6 +331,13 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
   TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0 && v.size(1) == Hkv &&
               k.size(2) == D && v.size(2) == D && v.size(0) == k.size(0));
   TORCH_CHECK(out.is_contiguous() && out.sizes() == q.sizes());
+  for (const auto& t : {out, q, k, v})
+    TORCH_CHECK(t.scalar_type() == torch::kBFloat16, "rows are bf16");
+  TORCH_CHECK(cu_seqlens.is_contiguous() && cu_seqlens_k.is_contiguous() &&
+              cu_seqlens_k.numel() >= B + 1, "a boundary more than sequences");
+  for (const auto& t : {out, q, k, v, cu_seqlens, cu_seqlens_k})
+    TORCH_CHECK(t.is_cuda() && t.device() == q.device(),
+                "everything on one GPU");
   if (B <= 0 || max_seqlen <= 0 || q.numel() == 0) return;
   Prefill m{};
   m.mul = (float)std::abs(scale) * LOG2E;

@@ -211,6 +211,11 @@ void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
               residual.is_contiguous() && residual.dim() == 2 &&
               residual.size(0) == x.size(1) && residual.size(1) == x.size(2) &&
               h.sizes() == residual.sizes());
+  for (const auto& t : {h, residual, w})
+    TORCH_CHECK(t.scalar_type() == torch::kBFloat16 &&
+                t.device() == x.device() && t.is_contiguous(),
+                "packed bf16 beside the stretches");
+  TORCH_CHECK(w.numel() == x.size(2) && x.is_cuda(), "weights of a row");
   const int T = x.size(1);
   const int H = x.size(2);
   TORCH_CHECK(H % 8 == 0, "H must be a multiple of 8");

@@ -243,3 +243,23 @@ def test_few_rows_where_they_pay():
     assert glu(17, 28672, 4096) and glu(64, 26624, 2048)
     assert not (glu(1, 8192, 4096) or glu(17, 26560, 4096) or
                 glu(32, 28672, 5120) or glu(64, 57344, 8192))
+
+
+@pytest.mark.parametrize("case,says", [
+    ("type", "rows are bf16"), ("out", "rows are bf16"),
+    ("keys", "a boundary more"), ("host", "on one GPU")])
+def test_attn_prefill_refuses(case, says):
+    """What would be misread, or read by the host's addresses, is refused
+    before any launch."""
+    q, k, v, out = (torch.zeros(9, 2, 64, dtype=torch.bfloat16)
+                    for _ in range(4))
+    cu = torch.tensor([0, 4, 9], dtype=torch.int32)
+    cu_k = cu
+    if case == "type":
+        k = k.half()
+    elif case == "out":
+        out = out.float()
+    elif case == "keys":
+        cu_k = cu[:2]
+    with pytest.raises(RuntimeError, match=says):
+        ops._native().attn_prefill(out, q, k, v, cu, cu_k, 5, 0.125, True, 0)
