@@ -155,9 +155,11 @@ def _own(m: nn.Module, *kinds: type) -> bool:
     """Whether m is one of these modules as written here: a subclass, a module
     put in its place or a hook gets and returns what torch's linear would,
     [T, N], and never a form."""
-    return type(m) in kinds and not (
-        m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
-        or _has_any_global_hook())
+    if type(m) not in kinds:
+        return False
+    d = m.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"]
+                or "forward" in d or _has_any_global_hook())
 
 
 def _project(proj: nn.Module, x: torch.Tensor, form: str) -> torch.Tensor:

@@ -473,8 +473,7 @@ def _rows_fit(x: torch.Tensor, w: torch.Tensor, most: int = ROWS_MAX_M,
     elif dtype != torch.uint8 or K % ROWS_CHUNK:
         return False
     return (dtype == w.dtype and x.is_contiguous() and w.is_contiguous()
-            and x.get_device() == w.get_device() == torch.cuda.current_device()
-            and _aligned(x, w)
+            and x.get_device() == w.get_device() and _aligned(x, w)
             # those have to see torch's own
             and not torch.is_autocast_enabled("cuda")
             and not torch.compiler.is_compiling())

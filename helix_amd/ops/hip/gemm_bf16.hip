@@ -36,6 +36,7 @@
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <c10/core/DeviceGuard.h>
 
 using namespace helix;
 
@@ -393,12 +394,14 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 // Sums [stretches, M, N] of as many stretches as there are workgroups for: up
 // to 256 of 256 x 256 or 512 of 128 x 128, at most 8.
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile) {
+  const c10::DeviceGuard on(x.device());
   Gemm m{};
   m.M = x.size(0);
   m.K = x.size(1);
   m.N = w.size(0);
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.is_cuda() &&
+                t.device() == x.device() &&
                 t.scalar_type() == torch::kBFloat16 &&
                 (uintptr_t)t.data_ptr() % 16 == 0);
   TORCH_CHECK(w.size(1) == m.K && m.K > 0 && m.K % 64 == 0 && m.M >= 1 &&

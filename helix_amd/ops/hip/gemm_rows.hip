@@ -40,6 +40,7 @@
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <c10/core/DeviceGuard.h>
 
 using namespace helix;
 
@@ -292,6 +293,7 @@ void check_out(const torch::Tensor& out, const torch::Tensor& x,
 // Sums [stretches, M, N] for a reader that adds them up.
 torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
                              OptT w_scale) {
+  const c10::DeviceGuard on(x.device());
   Product m = product_of(x, w, x_scale, w_scale);
   const int stretches = cut(m, false);
   torch::Tensor sums = sums_for(x, m, stretches);
@@ -301,6 +303,7 @@ torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
 
 void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
                OptT x_scale, OptT w_scale, bool gelu) {
+  const c10::DeviceGuard on(x.device());
   Product m = product_of(x, w, x_scale, w_scale);
   check_out(out, x, m);
   if (bias.has_value()) {
@@ -327,6 +330,7 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
 // out[M,N] = silu(x w[:N]^T) * (x w[N:]^T)
 void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    OptT x_scale, OptT w_scale) {
+  const c10::DeviceGuard on(x.device());
   Product m = product_of(x, w, x_scale, w_scale);
   TORCH_CHECK(m.M <= 64 && m.N % 8 == 0);
   m.N /= 2;                                   // 32 columns of a workgroup
