@@ -54,7 +54,7 @@ void sample_tokens_ext(torch::Tensor out, torch::Tensor logits,
                        c10::optional<torch::Tensor> seen,
                        c10::optional<torch::Tensor> row_map);
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, int64_t act);
+               c10::optional<torch::Tensor> bias, int64_t act, int64_t tile);
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile);
 void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                       c10::optional<torch::Tensor> bias,
@@ -106,7 +106,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tokens", &sample_tokens, "Greedy/Gumbel token sampling");
   m.def("sample_tokens_ext", &sample_tokens_ext,
         "Fused top-k/top-p/penalty Gumbel sampling (histogram threshold)");
-  m.def("gemm_bf16", &gemm_bf16, "MFMA bf16 GEMM: x @ w^T (+bias, act)");
+  m.def("gemm_bf16", &gemm_bf16, "MFMA bf16 GEMM: x @ w^T (+bias, act)",
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("bias"),
+        py::arg("act"), py::arg("tile") = 0);
   m.def("gemm_bf16_sums", &gemm_bf16_sums,
         "x @ w^T, stretches of the inner dimension apart");
   m.def("gemm_skinny_bf16", &gemm_skinny_bf16,

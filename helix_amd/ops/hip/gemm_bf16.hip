@@ -1,41 +1,15 @@
 // bf16 MFMA GEMM for gfx950: out[M,N] = act(x[M,K] @ w[N,K]^T + bias).
 //
-// The encoder's and the image model's projections (act: none or GELU, tanh) of
-// more than a few rows, and Llama's deep ones at a few hundred rows, whose inner
-// dimension is cut into stretches that a later reader adds up (fp32
+// The encoder's and the image model's projections (act: none or GELU, tanh),
+// and Llama's of more than a few rows; deep ones of few tiles are cut into
+// stretches of the inner dimension that a later reader adds up (fp32
 // [stretch][M][N]).
 //
-// Bound by the matrix cores and by LDS reads, which take about as long. Tiles
-// of both operands go straight to LDS; their 16-byte pieces lie crosswise, so
-// that the 16 rows of an operand meet every bank once. Workgroups that follow
-// each other on an XCD share rows of x and, GROUP at a time, columns of w.
-//
-//  - 256 x 256 by two halves of 4 waves, a phase apart: while one reads its
-//    operands (and orders the tiles of three steps later) the other multiplies,
-//    on the same SIMDs. Four tiles of 32 of the inner dimension are in LDS.
-//  - smaller tiles with two buffers of 64 and one barrier a step; several
-//    workgroups on a CU fill each other's gaps.
-//  - 128 x 128 tiles in stretches where tiles leave CUs idle (cut).
-//
-// Before, 128 x 128 tiles of all sizes, one buffer, rows as in memory (8 lanes
-// on a bank). us before -> now with weights in the caches (tile, or stretches of
-// 128; TFLOP/s), M x N x K:
-//   16600 x 2304 x 768   131 -> 105  (128; 562)   2304 x 3072 x 1024  33 -> 24
-//   16600 x 768 x 768     54 -> 35   (128; 557)   2304 x 1024 x 1024  28 -> 13
-//   16600 x 3072 x 768   203 -> 123  (128; 639)   2304 x 4096 x 1024  68 -> 36
-//   16600 x 768 x 3072   149 -> 83   (256; 950)   2304 x 1024 x 4096  86 -> 36
-//   300 x 768 x 3072      66 -> 14   (6 stretches; the one above: 3)
-// Products of few rows stream their weights instead (gemm_rows.hip): 8 x 6144 x
-// 1024 takes 6.4 from the caches, 7.6 from memory, by tiles 14.1.
-// 8192^3 runs at 1248 TFLOP/s. 256 x 256 as 128 is, with two buffers, takes 10%
-// longer; three buffers, steps of 32 for the smaller tiles, 256 x 128 and
-// scheduling hints for the reads from LDS gave nothing. Tile counts: 108 of
-// 256 against 432 of 128 (2304 x 3072 x 1024) 34 and 23; 144 of 128 against
-// 576 of 64 (2304 x 1024 x 1024) 14.8 and 12.9.
+// gemm_ring.h has the kernel, its times and what bounds it. Here are its tiles
+// and the rule that chooses one, and the kernel for what it does not take:
+// columns that are no multiple of 8, results off 16-byte boundaries.
 #include "gemm_join.h"
-#include "hybrid/tile.h"
-#include <torch/extension.h>
-#include <ATen/hip/HIPContext.h>
+#include "gemm_ring.h"
 #include <c10/core/DeviceGuard.h>
 
 using namespace helix;
@@ -46,8 +20,7 @@ constexpr int GROUP = 4;                      // tiles of rows
 
 struct Gemm {
   const uint16_t* bias;
-  float* sums;                 // null: out
-  int M, N, K, m_tiles, n_tiles, stretch, gelu;
+  int M, N, K, m_tiles, n_tiles, gelu;
 };
 
 __device__ __forceinline__ float finish(float v, float b, int gelu) {
@@ -55,30 +28,22 @@ __device__ __forceinline__ float finish(float v, float b, int gelu) {
   return gelu ? gelu_tanh_f32(v) : v;
 }
 
-// What a workgroup does: its tile and its part of the inner dimension.
 struct Place {
-  int m0, n0, split, k0, k1;
+  int m0, n0;
 };
 __device__ __forceinline__ Place place(const Gemm& m, int BM, int BN) {
-  const int all = xcd_chunk(blockIdx.x, gridDim.x);
-  const int tiles = m.m_tiles * m.n_tiles, at = all % tiles;
+  const int at = xcd_chunk(blockIdx.x, gridDim.x);
   const int first = at / (GROUP * m.n_tiles) * GROUP;
   const int rows = min(GROUP, m.m_tiles - first);
   const int in = at % (GROUP * m.n_tiles);
   Place p;
-  p.split = all / tiles;
   p.m0 = (first + in % rows) * BM;
   p.n0 = in / rows * BN;
-  p.k0 = p.split * m.stretch;
-  p.k1 = min(m.K, p.k0 + m.stretch);
   return p;
 }
 
-// Piece p of a row of BK elements lies at p ^ cross(row).
-template <int BK>
-__device__ __forceinline__ int cross(int r) {
-  return BK == 64 ? r >> 1 & 7 : r >> 2 & 3;
-}
+// Piece p of a row of 64 elements lies at p ^ cross(row).
+__device__ __forceinline__ int cross(int r) { return r >> 1 & 7; }
 
 // This thread's 16-byte pieces of a tile; rows past the end repeat the last
 // one and are not stored.
@@ -92,7 +57,7 @@ struct Pieces {
     for (int i = 0; i < N; ++i) {
       const int e = i * TH + threadIdx.x, r = e / PR;
       from[i] = a + (int64_t)min(row0 + r, rows - 1) * K +
-                (e % PR ^ cross<BK>(r)) * 8;
+                (e % PR ^ cross(r)) * 8;
     }
   }
   __device__ __forceinline__ void load(int k, uint16_t* lds) const {
@@ -109,8 +74,8 @@ struct Pieces {
 
 // lane: columns c + 4 hi + q (tiles of 16 apart) of rows r + lo
 template <int MI, int NI>
-__device__ __forceinline__ void store(const Gemm& m, uint16_t* out, int split,
-                                      int row0, int col0,
+__device__ __forceinline__ void store(const Gemm& m, uint16_t* out, int row0,
+                                      int col0,
                                       const floatx4 (*acc)[MI]) {
   const int lane = threadIdx.x & (WAVE - 1), lo = lane & 15, hi = lane >> 4;
 #pragma unroll
@@ -125,12 +90,6 @@ __device__ __forceinline__ void store(const Gemm& m, uint16_t* out, int split,
     for (int i = 0; i < MI; ++i) {
       const int r = row0 + i * 16 + lo;
       if (r >= m.M) continue;
-      if (m.sums != nullptr) {                // N % 4 == 0
-        if (c < m.N)
-          *reinterpret_cast<floatx4*>(
-              m.sums + ((int64_t)split * m.M + r) * m.N + c) = acc[j][i];
-        continue;
-      }
       uint16_t* o = out + (int64_t)r * m.N + c;
       float v[4];
 #pragma unroll
@@ -166,12 +125,12 @@ __global__ __launch_bounds__(WM* WN* WAVE) void gemm_tiles_kernel(
 #pragma unroll
     for (int i = 0; i < MI; ++i) acc[j][i] = floatx4{0, 0, 0, 0};
 
-  xs.load(p.k0, lds);
-  ws.load(p.k0, lds + BM * BK);
-  for (int k = p.k0, cur = 0; k < p.k1; k += BK, cur ^= 1) {
+  xs.load(0, lds);
+  ws.load(0, lds + BM * BK);
+  for (int k = 0, cur = 0; k < m.K; k += BK, cur ^= 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (k + BK < p.k1) {
+    if (k + BK < m.K) {
       xs.load(k + BK, lds + (cur ^ 1) * HALF);
       ws.load(k + BK, lds + (cur ^ 1) * HALF + BM * BK);
     }
@@ -179,7 +138,7 @@ __global__ __launch_bounds__(WM* WN* WAVE) void gemm_tiles_kernel(
     const uint16_t* wl = lds + cur * HALF + (BM + wc * NI * 16 + lo) * BK;
 #pragma unroll
     for (int kk = 0; kk < BK / 32; ++kk) {
-      const int piece = ((kk * 4 + hi) ^ cross<BK>(lo)) * 8;
+      const int piece = ((kk * 4 + hi) ^ cross(lo)) * 8;
       u16x8 xf[MI], wf[NI];
 #pragma unroll
       for (int i = 0; i < MI; ++i) xf[i] = ld_u16x8(xl + i * 16 * BK + piece);
@@ -192,144 +151,108 @@ __global__ __launch_bounds__(WM* WN* WAVE) void gemm_tiles_kernel(
           acc[j][i] = mfma16(wf[j], xf[i], acc[j][i]);
     }
   }
-  store<MI, NI>(m, out, p.split, p.m0 + wr * MI * 16, p.n0 + wc * NI * 16,
-                acc);
-}
-
-// 256 x 256, 2 x 4 waves, the second row of waves a phase behind the first. A
-// step of 32 has two phases, with a barrier after each: operands from LDS,
-// products. What a half orders in step t lands in the buffer that both have
-// read in step t - 1; before the barrier that ends its reading of step t a
-// half waits for its own part of step t + 1, so that the other half, which is
-// a phase ahead or behind, finds all of it there.
-constexpr int PAIR = 256;
-
-__global__ __launch_bounds__(512, 2) void gemm_pair_kernel(
-    uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
-    const uint16_t* __restrict__ w, Gemm m) {
-  constexpr int BK = 32, TH = 512, MI = 8, NI = 4, BUF = 2 * PAIR * BK;
-  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  const Place p = place(m, PAIR, PAIR);
-  const int wid = threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
-  const int lo = lane & 15, hi = lane >> 4;
-  const int wr = wid / 4, wc = wid % 4;
-  const Pieces<PAIR, TH, BK> xs(x, p.m0, m.M, m.K);
-  const Pieces<PAIR, TH, BK> ws(w, p.n0, m.N, m.K);
-  floatx4 acc[NI][MI];
-#pragma unroll
-  for (int j = 0; j < NI; ++j)
-#pragma unroll
-    for (int i = 0; i < MI; ++i) acc[j][i] = floatx4{0, 0, 0, 0};
-  auto load = [&](int step) {
-    uint16_t* to = lds + (step & 3) * BUF;
-    xs.load(p.k0 + step * BK, to);
-    ws.load(p.k0 + step * BK, to + PAIR * BK);
-  };
-  const int steps = (p.k1 - p.k0) / BK;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-    if (i < steps) load(i);
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  if (wr == 1) asm volatile("s_barrier" ::: "memory");
-  const int piece = (hi ^ cross<BK>(lo)) * 8;
-  for (int t = 0; t < steps; ++t) {
-    const uint16_t* at = lds + (t & 3) * BUF + lo * BK + piece;
-    u16x8 xf[MI], wf[NI];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-      xf[i] = ld_u16x8(at + (wr * MI + i) * 16 * BK);
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-      wf[j] = ld_u16x8(at + (PAIR + (wc * NI + j) * 16) * BK);
-    if (t + 3 < steps) {
-      load(t + 3);                            // 4 pieces of this thread
-      asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-        acc[j][i] = mfma16(wf[j], xf[i], acc[j][i]);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_barrier" ::: "memory");
-  }
-  if (wr == 0) asm volatile("s_barrier" ::: "memory");
-  store<MI, NI>(m, out, p.split, p.m0 + wr * MI * 16, p.n0 + wc * NI * 16,
-                acc);
-}
-
-void start(const void* kernel, int threads, int bytes, Gemm& m, int bm, int bn,
-           int stretches, uint16_t* out, const uint16_t* x,
-           const uint16_t* w) {
-  m.m_tiles = cdiv(m.M, bm);
-  m.n_tiles = cdiv(m.N, bn);
-  void* args[] = {&out, &x, &w, &m};
-  const hipError_t err = hipLaunchKernel(
-      kernel, dim3(m.m_tiles * m.n_tiles * stretches), dim3(threads), args,
-      bytes, at::hip::getCurrentHIPStream());
-  TORCH_CHECK(err == hipSuccess, hipGetErrorString(err));
-}
-
-void allow(const void* kernel) {
-  TORCH_CHECK(hipFuncSetAttribute(
-                  kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                  160 * 1024) == hipSuccess, "LDS size refused");
+  store<MI, NI>(m, out, p.m0 + wr * MI * 16, p.n0 + wc * NI * 16, acc);
 }
 
 template <int BM, int BN, int WM, int WN>
-void run_tiles(Gemm m, uint16_t* out, const uint16_t* x, const uint16_t* w,
-               int stretches = 1) {
-  const void* k = (const void*)gemm_tiles_kernel<BM, BN, WM, WN>;
-  static const bool once = (allow(k), true);
-  (void)once;
-  start(k, WM * WN * WAVE, 2 * (BM + BN) * 64 * 2, m, BM, BN, stretches, out,
-        x, w);
+void run_tiles(Gemm m, uint16_t* out, const uint16_t* x, const uint16_t* w) {
+  m.m_tiles = cdiv(m.M, BM);
+  m.n_tiles = cdiv(m.N, BN);
+  hipLaunchKernelGGL((gemm_tiles_kernel<BM, BN, WM, WN>),
+                     dim3(m.m_tiles * m.n_tiles), dim3(WM * WN * WAVE),
+                     2 * (BM + BN) * 64 * 2, at::hip::getCurrentHIPStream(),
+                     out, x, w, m);
 }
 
-void run_pair(Gemm m, uint16_t* out, const uint16_t* x, const uint16_t* w,
-              int stretches = 1) {
-  const void* k = (const void*)gemm_pair_kernel;
-  static const bool once = (allow(k), true);
-  (void)once;
-  start(k, 512, 4 * 2 * PAIR * 32 * 2, m, PAIR, PAIR, stretches, out, x, w);
+// Of 23 tiles of 64 to 256 rows and columns these are needed for times within
+// 1% of the best of all (150 sizes, see ring_us).
+#define HELIX_RING_ROWS(TILE)                                                \
+  TILE(2, 2) TILE(3, 4) TILE(4, 2) TILE(4, 8) TILE(5, 2) TILE(5, 4)          \
+  TILE(5, 6) TILE(5, 8) TILE(6, 4) TILE(6, 6) TILE(7, 8) TILE(8, 8)
+#define HELIX_RING_SUMS(TILE)                                                \
+  TILE(2, 2) TILE(4, 2) TILE(4, 4) TILE(4, 8) TILE(5, 4) TILE(5, 8)          \
+  TILE(8, 8)
+#define HELIX_TILE(MI, NI) {MI, NI},
+constexpr RingTile ROWS_TILES[] = {HELIX_RING_ROWS(HELIX_TILE)};
+constexpr RingTile SUMS_TILES[] = {HELIX_RING_SUMS(HELIX_TILE)};
+#undef HELIX_TILE
+
+void run_ring(const Ring& m, RingTile t) {
+#define HELIX_RUN(MI, NI)                                                    \
+  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, ROWS>(m, 1);
+  HELIX_RING_ROWS(HELIX_RUN)
+#undef HELIX_RUN
+  TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni);
 }
 
-// Stretches of 128 x 128 tiles for a product whose tiles leave CUs idle, joined
-// by a launch; 1 where whole tiles take no longer. Both are estimated in us:
-//   whole:      0.6 a step of 64, times rounds of 256 tiles
-//   stretches:  6, 0.6 a step or 0.37 for each 256 workgroups, and their sums
-//               written and read at 4.5 TB/s; 4 more, as the launch that joins
-//               them costs a host that is behind
-// from 693 sizes (66 to 4500 rows of 256 to 4096 columns, 512 to 14336 deep,
-// weights from memory) timed whole and in 2, 3, 4, 6 and 8 stretches. What is
-// taken is within 2.2% of the best of these, at worst 48%; whole tiles alone
-// take 1.54 times as long. Some, whole and as taken: 2304 x 1024 x 4096 48.1
-// and 36.3, 300 of its rows 44.0 and 18.5, 700 x 768 x 3072 25.5 and 19.0, 200
-// x 2048 x 2048 21.1 and 16.0; as taken and in two: 1000 x 768 x 1024 11.3 and
-// 15.1, 1500 x 4096 x 4096 64.9 and 75.3.
-int cut(Gemm& m) {
-  const int tiles = cdiv(m.M, 128) * cdiv(m.N, 128), steps = m.K / 64;
-  if (m.M <= 64 || m.N % 4 != 0) return 1;
-  float best = 0.6f * steps * std::max(1.f, tiles / 256.f);
-  int n = 1;
-  for (int i = 2; i <= std::min(steps, 8); ++i) {
-    const float us = 10 + cdiv(steps, i) * std::max(0.6f, 0.37f * tiles * i / 256)
-                     + 8.f * i * m.M * m.N / 4.5e6f;
-    if (us < best) best = us, n = i;
+void run_ring_sums(const Ring& m, RingTile t, int stretches) {
+#define HELIX_RUN(MI, NI)                                                    \
+  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, SUMS>(m, stretches);
+  HELIX_RING_SUMS(HELIX_RUN)
+#undef HELIX_RUN
+  TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni, " for sums");
+}
+
+// Tile and stretches, and their time in us with what it takes to read the
+// stretches: their bytes at 4.5 TB/s.
+struct Plan {
+  RingTile tile{0, 0};
+  int stretches = 1;
+  double us = 1e30;
+};
+Plan plan_rows(const Ring& m) {
+  Plan best;
+  const int cus = ring_cus();
+  for (const RingTile t : ROWS_TILES) {
+    const double us = ring_us(m, ROWS, t, 1, cus);
+    if (us < best.us) best = Plan{t, 1, us};
   }
-  m.stretch = cdiv(steps, n) * 64;
+  return best;
+}
+Plan plan_sums(const Ring& m, int from) {
+  Plan best;
+  const int steps = m.K / 64, cus = ring_cus();
+  for (const RingTile t : SUMS_TILES)
+    for (int n = from; n <= std::min(8, steps); ++n) {
+      const double us = ring_us(m, SUMS, t, n, cus) +
+                        4. * n * m.M * m.N / 4.5e6;
+      if (us < best.us) best = Plan{t, n, us};
+    }
+  return best;
+}
+
+// The last stretch may be shorter; there are as many as have something to do.
+int cut(Ring& m, int stretches) {
+  m.stretch = cdiv(m.K / 64, stretches) * 64;
   return cdiv(m.K, m.stretch);
+}
+
+torch::Tensor sums_of(const torch::Tensor& x, Ring& m, RingTile t,
+                      int stretches) {
+  stretches = cut(m, stretches);
+  torch::Tensor sums = torch::empty({stretches, m.M, m.N},
+                                    x.options().dtype(torch::kFloat32));
+  m.sums = sums.data_ptr<float>();
+  run_ring_sums(m, t, stretches);
+  return sums;
+}
+
+Ring ring_of(const torch::Tensor& x, const torch::Tensor& w) {
+  Ring m{};
+  m.M = x.size(0);
+  m.K = m.stretch = x.size(1);
+  m.N = w.size(0);
+  m.x = (const uint16_t*)x.data_ptr();
+  m.w = (const uint16_t*)w.data_ptr();
+  return m;
 }
 
 }  // namespace
 
+// tile: that one of 32 * (tile / 10) rows and 32 * (tile % 10) columns, 0 the
+// one that takes least time.
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, int64_t act) {
+               c10::optional<torch::Tensor> bias, int64_t act, int64_t tile) {
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2, "x and w are matrices");
   Gemm m{};
   m.M = x.size(0);
@@ -363,60 +286,61 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   if ((uintptr_t)x.data_ptr() % 16 != 0) x = x.clone();
   if ((uintptr_t)w.data_ptr() % 16 != 0) w = w.clone();
   uint16_t* o = (uint16_t*)out.data_ptr();
-  const uint16_t* xp = (const uint16_t*)x.data_ptr();
-  const uint16_t* wp = (const uint16_t*)w.data_ptr();
-  m.stretch = m.K;
-  // The largest tile of which there are enough for the 256 CUs: operands are
-  // read least often, and a CU without work costs more than that. The two
-  // halves of 256 x 256 need a long inner dimension, as nothing runs beside
-  // their first loads and their stores (768: 16600 x 2304 105 us, 104 with
-  // 128; 3072: 16600 x 768 82, 100 with 128).
-  auto tiles = [&](int bm, int bn) {
-    return (int64_t)cdiv(m.M, bm) * cdiv(m.N, bn);
-  };
-  if (m.K >= 2048 && tiles(PAIR, PAIR) >= 192) run_pair(m, o, xp, wp);
-  else if (const int n = cut(m); n > 1) {
-    torch::Tensor sums =
-        torch::empty({n, m.M, m.N}, x.options().dtype(torch::kFloat32));
-    const uint16_t* b = m.bias;
+  Ring r = ring_of(x, w);
+  if (ring_fits(r, ROWS) && (uintptr_t)o % 16 == 0) {
+    if (m.bias != nullptr && (uintptr_t)m.bias % 16 != 0) {
+      bias = bias->clone();
+      m.bias = (const uint16_t*)bias->data_ptr();
+    }
+    r.out = o;
+    r.gelu = m.gelu;
+    if (tile != 0) {
+      r.bias = m.bias;
+      return run_ring(r, RingTile{(int)tile / 10, (int)tile % 10});
+    }
+    // A launch that joins stretches takes 3 us more than what it reads (with
+    // it, and whole: 300 x 1024 x 4096 13 and 18, 288 x 768 x 3072 9.6 and 12.1;
+    // 2304 x 768 x 3072 20 and 18).
+    const Plan rows = plan_rows(r), sums = plan_sums(r, 2);
+    if (rows.us <= sums.us + 4) {
+      r.bias = m.bias;
+      return run_ring(r, rows.tile);
+    }
+    const torch::Tensor t = sums_of(x, r, sums.tile, sums.stretches);
     const int64_t MN = (int64_t)m.M * m.N;
-    m.sums = sums.data_ptr<float>();
-    run_tiles<128, 128, 2, 4>(m, nullptr, xp, wp, n);
     hipLaunchKernelGGL(gemm_join_kernel, dim3((MN + 1023) / 1024), dim3(256),
                        0, at::hip::getCurrentHIPStream(), o,
-                       sums.data_ptr<float>(), b, MN, m.N, n, m.gelu != 0);
+                       t.data_ptr<float>(), m.bias, MN, m.N, (int)t.size(0),
+                       m.gelu != 0);
+    return;
   }
-  else if (tiles(128, 128) >= 256) run_tiles<128, 128, 2, 4>(m, o, xp, wp);
-  else if (m.M > 64) run_tiles<64, 64, 2, 2>(m, o, xp, wp);
+  TORCH_CHECK(tile == 0, "not a product of tiles");
+  const uint16_t* xp = (const uint16_t*)x.data_ptr();
+  const uint16_t* wp = (const uint16_t*)w.data_ptr();
+  if (m.M > 64) run_tiles<64, 64, 2, 2>(m, o, xp, wp);
   else run_tiles<32, 64, 2, 2>(m, o, xp, wp);
 }
 
-// Sums [stretches, M, N] of as many stretches as there are workgroups for: up
-// to 256 of 256 x 256 or 512 of 128 x 128, at most 8.
+// Sums [stretches, M, N] for a reader that adds them up: as many stretches of
+// 128 x 128 (256 x 256) tiles as there are workgroups for, up to 512 (256) and
+// 8. tile 0: those that take least time with their reader.
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile) {
   const c10::DeviceGuard on(x.device());
-  Gemm m{};
-  m.M = x.size(0);
-  m.K = x.size(1);
-  m.N = w.size(0);
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.is_cuda() &&
                 t.device() == x.device() &&
                 t.scalar_type() == torch::kBFloat16 &&
                 (uintptr_t)t.data_ptr() % 16 == 0);
+  Ring m = ring_of(x, w);
   TORCH_CHECK(w.size(1) == m.K && m.K > 0 && m.K % 64 == 0 && m.M >= 1 &&
-              m.N >= 4 && m.N % 4 == 0 && (tile == PAIR || tile == 128));
-  const int tiles = cdiv(m.M, (int)tile) * cdiv(m.N, (int)tile);
-  const int most = (tile == PAIR ? 256 : 512) / tiles;
-  const int steps = m.K / 64;
-  m.stretch = cdiv(steps, std::max(1, std::min({most, steps, 8}))) * 64;
-  const int n = cdiv(m.K, m.stretch);
-  torch::Tensor sums =
-      torch::empty({n, m.M, m.N}, x.options().dtype(torch::kFloat32));
-  m.sums = sums.data_ptr<float>();
-  const uint16_t* xp = (const uint16_t*)x.data_ptr();
-  const uint16_t* wp = (const uint16_t*)w.data_ptr();
-  if (tile == PAIR) run_pair(m, nullptr, xp, wp, n);
-  else run_tiles<128, 128, 2, 4>(m, nullptr, xp, wp, n);
-  return sums;
+              m.N >= 4 && m.N % 4 == 0 &&
+              (tile == 0 || tile == 256 || tile == 128));
+  TORCH_CHECK(ring_fits(m, SUMS), "a product of more than the offsets reach");
+  if (tile == 0) {
+    const Plan p = plan_sums(m, 1);
+    return sums_of(x, m, p.tile, p.stretches);
+  }
+  const int side = (int)tile, tiles = cdiv(m.M, side) * cdiv(m.N, side);
+  const int most = std::min({(side == 256 ? 256 : 512) / tiles, m.K / 64, 8});
+  return sums_of(x, m, RingTile{side / 32, side / 32}, std::max(1, most));
 }

@@ -1,0 +1,413 @@
+// Products of bf16 matrices, x[M,K] @ w[N,K]^T with fp32 sums, by persistent
+// workgroups whose loads never pause. gemm_bf16.hip and gemm_gated.hip choose
+// the tile and launch.
+//
+// Bound by the matrix cores, and for large products by the power they draw (the
+// clock falls to 1.7 to 1.9 GHz). A workgroup has one wave a SIMD, 2 x 2 of
+// them, each with 16 MI x 16 NI sums in accumulation registers:
+//
+//  - Tiles of 64 of the inner dimension go straight to LDS, as many steps ahead
+//    as 160 KB hold. Rows are 128 bytes, so a load takes whole cache lines
+//    (with 32 of the inner dimension at a time 8192 x 4096 x 4096 took 204 us,
+//    with 64 185). 16-byte piece p of row r lies at p ^ r / 2 % 8: operands
+//    leave LDS without bank conflicts.
+//  - A step has two halves of 32. While one is multiplied, the operands of the
+//    next one come from LDS and a later step's loads are ordered, one of them at
+//    a time between two products: what stands together holds the matrix cores
+//    up (2423 cycles a step of 256 x 256 with a read, a load and then four
+//    products, 2286 one by one; the products alone take 2048). One barrier a
+//    step.
+//  - Loads go on from tile to tile: the next tile's first steps arrive during
+//    the last ones of this tile and while its results are stored, and nobody
+//    waits for the stores (before, 5.5 us of 1 x 768 steps of 256 x 256 were
+//    first loads, 7.5 the stores). Rows of w are put into LDS in such an order
+//    that a lane has 8 neighbouring columns: 16-byte stores.
+//
+// us by the kernels that were here before -> now, weights in the caches; the
+// former had 256 x 256 by two halves of waves a phase apart, and 128 x 128 with
+// one barrier and all loads drained each step (tile now; TFLOP/s):
+//   16600 x 2304 x 768    84 -> 59  (160 x 192;  998)
+//   16600 x 768 x 768     32 -> 21  (224 x 256;  919)
+//   16600 x 768 x 3072    74 -> 58  (224 x 256; 1350)
+//   2304 x 3072 x 1024    22 -> 17  (256 x 128;  853)
+//   2304 x 1024 x 1024  12.1 -> 8.9 (160 x 64;   544)
+//   2304 x 1024 x 4096    33 -> 24  (160 x 64;   793)
+//   8192 x 4096 x 4096   221 -> 182 (256 x 256; 1511)
+// Steps of 32 and 3 to 5 buffers of them, reads of LDS early in a half, loads
+// closer together gave nothing or cost.
+#pragma once
+#include "gelu.h"
+#include "hybrid/tile.h"
+#include <ATen/hip/HIPContext.h>
+#include <torch/extension.h>
+
+namespace helix {
+namespace {
+
+enum RingForm { ROWS, GATED, SUMS };          // of the result
+
+constexpr int RING_GROUP = 4;                 // tiles of rows that share columns
+constexpr int RING_LDS = 160 * 1024;
+
+// Quotients of a fixed number below 2^31: d <= 2^shift, mul the rounded up rest
+// of 2^(32 + shift) / d above 2^32.
+struct Divide {
+  uint32_t mul, shift;
+  Divide() = default;
+  explicit Divide(uint32_t d) : shift(0) {
+    while ((1ull << shift) < d) ++shift;
+    mul = (uint32_t)((((1ull << shift) - d) << 32) / d + 1);
+  }
+  __device__ __forceinline__ int operator()(uint32_t n) const {
+    return (__umulhi(n, mul) + n) >> shift;
+  }
+};
+
+// x, w, bias on 16-byte boundaries; out as well and N % 8 == 0, sums N % 4 == 0.
+// GATED: w has N rows of the gate and N of the other factor.
+struct Ring {
+  const uint16_t *x, *w, *bias;               // bias may be null
+  uint16_t* out;
+  float* sums;                                // [stretch][M][N]
+  int M, N, K, m_tiles, n_tiles, tiles, total, stretch, gelu;
+  Divide by_tiles, by_group;
+};
+
+struct RingItem {
+  int m0, n0, split, k0, k1;
+};
+
+// A thread's 16-byte pieces of ROWS_ rows of 64, as offsets in bytes.
+template <int N_ROWS>
+struct RingUnit {
+  int off[N_ROWS / 32];
+  template <typename F>
+  __device__ __forceinline__ RingUnit(int K, F row) {
+#pragma unroll
+    for (int i = 0; i < N_ROWS / 32; ++i) {
+      const int e = i * 256 + threadIdx.x, r = e / 8;
+      off[i] = (int)((row(r) * K + ((e % 8) ^ (r >> 1 & 7)) * 8) * 2);
+    }
+  }
+};
+
+#ifdef __HIP_DEVICE_COMPILE__
+// 64 lanes' pieces to 1024 bytes of LDS. What lies past the end of the
+// descriptor is zero and not read.
+__device__ __forceinline__ void ring_load(const uint16_t* base, int bytes,
+                                          int off, int k, uint16_t* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000),
+      (__attribute__((address_space(3))) void*)lds, 16, off, k * 2, 0, 0);
+}
+
+// Dropped past the end of the descriptor, but issued all the same.
+__device__ __forceinline__ void ring_store(void* base, int bytes, int off,
+                                           u32x4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(
+      v, __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000), off, 0,
+      0);
+}
+
+// c (+)= a b in place. As a builtin the sums wander from register to register,
+// at two moves a product. A product reads its sums four or more products after
+// it wrote them.
+template <bool FIRST>
+__device__ __forceinline__ void ring_mma(floatx4& c, u16x8 a, u16x8 b) {
+  if constexpr (FIRST)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
+                 : "=a"(c) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                 : "+a"(c) : "v"(a), "v"(b));
+}
+
+// All but the last VM memory operations and all reads of LDS are through, here
+// and in the other waves.
+template <int VM>
+__device__ __forceinline__ void ring_wait() {
+  constexpr int V = VM > 63 ? 63 : VM;        // the counter's range
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((V & 15) | 7 << 4 | (V >> 4) << 14);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+#endif
+
+template <int MI, int NI, RingForm FORM>
+__global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int BM = 32 * MI, BN = 32 * NI, BK = 64, AU = BM * BK, BU = BN * BK;
+  // steps of w in LDS, and one more of x: x is ordered in the first half of a
+  // step, into what the step before has read, w in the second half, into what
+  // this step has read by then; both for NB steps later
+  constexpr int NB = (RING_LDS / 2 - AU) / (AU + BU), NA = NB + 1;
+  constexpr int OUT_N = FORM == GATED ? BN / 2 : BN;
+  // loads ordered since those of the next step, when half of a step is done
+  constexpr int ALLOW = (NB - 1) * MI + (NB - 2) * NI;
+  constexpr int STORES = MI * NI / (FORM == SUMS ? 1 : FORM == GATED ? 4 : 2);
+  static_assert(NB >= 2 && NI % (FORM == GATED ? 4 : 2) == 0, "tile");
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int lo = lane & 15, hi = lane >> 4, wr = wid / 2, wc = wid % 2;
+
+  // Workgroups of an XCD have neighbouring items of a round, also of the last
+  // one, which may not have one for each.
+  auto item_of = [&](int round, RingItem& p)
+      __attribute__((always_inline)) -> bool {
+    const int all = gridDim.x, n = min(all, m.total - round * all);
+    if ((int)blockIdx.x >= n) return false;
+    const int at = round * all + xcd_chunk(blockIdx.x, n);
+    p.split = m.by_tiles(at);
+    const int tile = at - p.split * m.tiles, group = m.by_group(tile);
+    const int in = tile - group * RING_GROUP * m.n_tiles;
+    const int first = group * RING_GROUP;
+    const int rows = min(RING_GROUP, m.m_tiles - first);
+    const int col = rows == 4 ? in >> 2 : rows == 2 ? in >> 1
+                    : rows == 3 ? (int)__umulhi(in, 0x55555556u) : in;
+    p.m0 = (first + in - col * rows) * BM;
+    p.n0 = col * OUT_N;
+    p.k0 = p.split * m.stretch;
+    p.k1 = min(m.K, p.k0 + m.stretch);
+    return true;
+  };
+
+  const RingUnit<BM> xu(m.K, [](int r) -> int64_t { return r; });
+  // row 16 s + 4 a + b of 32 in LDS is column 8 a + 4 s + b, so that two
+  // neighbouring products leave 8 columns to a lane
+  const RingUnit<BN> wu(m.K, [&](int r) -> int64_t {
+    const int n = (r & ~31) | (r & 12) << 1 | (r & 16) >> 2 | (r & 3);
+    if constexpr (FORM == GATED) {            // half of a wave's from either
+      const int wave = n / (16 * NI), c = n % (16 * NI);
+      return wave * 8 * NI + (c < 8 * NI ? c : (int64_t)m.N + c - 8 * NI);
+    }
+    return n;
+  });
+
+  // where loads are, NB steps ahead; empty descriptors after the last item
+  const uint16_t *x_at = m.x, *w_at = m.w;
+  int x_bytes = 0, w_bytes = 0, k = 0, k_end = 0x7fffffff, load_round = 0;
+  auto order_from = [&](const RingItem& p, bool on)
+      __attribute__((always_inline)) {
+    x_bytes = w_bytes = k = 0;
+    k_end = 0x7fffffff;
+    if (!on) return;
+    x_at = m.x + (int64_t)p.m0 * m.K;
+    w_at = m.w + (int64_t)p.n0 * m.K;
+    x_bytes = min(BM, m.M - p.m0) * m.K * 2;
+    w_bytes = FORM == GATED ? (2 * m.N - p.n0) * m.K * 2
+                            : min(BN, m.N - p.n0) * m.K * 2;
+    k = p.k0;
+    k_end = p.k1;
+  };
+  RingItem cur, next;
+  if (!item_of(0, cur)) return;
+  order_from(cur, true);
+  auto advance = [&]() __attribute__((always_inline)) {
+    k += BK;
+    if (k < k_end) return;
+    const bool more = item_of(++load_round, next);
+    order_from(next, more);
+  };
+
+  uint16_t* const xs = lds;
+  uint16_t* const ws = lds + NA * AU;
+  const int mine = wid * WAVE * 8;
+  const int p0 = (hi ^ (lo >> 1 & 7)) * 8, p1 = ((4 + hi) ^ (lo >> 1 & 7)) * 8;
+  const uint16_t* const xl = xs + (wr * MI * 16 + lo) * BK;
+  const uint16_t* const wl = ws + (wc * NI * 16 + lo) * BK;
+  floatx4 acc[NI][MI];
+  // products of xa and wa; meanwhile xb and wb are read and a unit is ordered
+  auto half = [&](auto first, auto of_w, u16x8 (&xa)[MI], u16x8 (&wa)[NI],
+                  u16x8 (&xb)[MI], u16x8 (&wb)[NI], const uint16_t* xr,
+                  const uint16_t* wr_, uint16_t* to)
+      __attribute__((always_inline)) {
+    constexpr bool W = decltype(of_w)::value;
+    constexpr int Q = MI * NI, R = MI + NI, L = W ? NI : MI;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      ring_mma<decltype(first)::value>(acc[q / MI][q % MI], wa[q / MI],
+                                       xa[q % MI]);
+#pragma unroll
+      for (int r = 0; r < R; ++r)             // in three quarters of the half
+        if (r * 3 * Q / (4 * R) == q) {
+          if (r < MI) xb[r < MI ? r : 0] = ld_u16x8(xr + r * 16 * BK);
+          else wb[r < MI ? 0 : r - MI] = ld_u16x8(wr_ + (r - MI) * 16 * BK);
+        }
+#pragma unroll
+      for (int l = 0; l < L; ++l)
+        if (l * Q / L + Q / L / 4 == q) {
+          if (W) ring_load(w_at, w_bytes, wu.off[W ? l : 0], k, to + l * 2048);
+          else ring_load(x_at, x_bytes, xu.off[W ? 0 : l], k, to + l * 2048);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < NB; ++s) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+      ring_load(x_at, x_bytes, xu.off[i], k, xs + s * AU + mine + i * 2048);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      ring_load(w_at, w_bytes, wu.off[i], k, ws + s * BU + mine + i * 2048);
+    advance();
+  }
+  ring_wait<(NB - 1) * (MI + NI)>();
+  u16x8 xa[MI], wa[NI], xb[MI], wb[NI], bias[NI / 2];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) xa[i] = ld_u16x8(xl + i * 16 * BK + p0);
+#pragma unroll
+  for (int j = 0; j < NI; ++j) wa[j] = ld_u16x8(wl + j * 16 * BK + p0);
+  // places in LDS: of this step's x and w, and of the x that is ordered
+  int sx = 0, sw = 0, so = NB;
+  // steps whose operands were ordered before the last tile's stores, for which
+  // nobody has to wait then
+  int stores_open = 0;
+  auto step = [&](auto first) __attribute__((always_inline)) {
+    half(first, std::false_type{}, xa, wa, xb, wb, xl + sx * AU + p1,
+         wl + sw * BU + p1, xs + so * AU + mine);
+    if (stores_open > 0) {
+      --stores_open;
+      ring_wait<ALLOW + STORES>();
+    } else {
+      ring_wait<ALLOW>();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int free_w = sw;
+    so = sx;
+    sx = sx + 1 == NA ? 0 : sx + 1;
+    sw = sw + 1 == NB ? 0 : sw + 1;
+    if constexpr (decltype(first)::value && FORM == ROWS) {
+      // more operations in flight than the waits count: they wait for more
+#pragma unroll
+      for (int j = 0; j < NI / 2; ++j)
+        bias[j] = m.bias == nullptr ? u16x8{0, 0, 0, 0, 0, 0, 0, 0}
+                                    : ld_u16x8(m.bias + min(
+                      cur.n0 + wc * 16 * NI + j * 32 + hi * 8, m.N - 8));
+    }
+    half(std::false_type{}, std::true_type{}, xb, wb, xa, wa,
+         xl + sx * AU + p0, wl + sw * BU + p0, ws + free_w * BU + mine);
+    advance();
+  };
+  for (int round = 1;; ++round) {
+    step(std::true_type{});
+    for (int n = (cur.k1 - cur.k0) / BK; --n > 0;) step(std::false_type{});
+    // the last products reach their registers before these are read
+    asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) asm volatile("" : "+a"(acc[j][i]));
+    // lane: 8 columns from 8 hi of 32, rows lo of 16. All stores are issued,
+    // also those that are dropped: stores_open counts on them.
+    constexpr int NONE = 0x7fffff00;          // past the end of any tile
+    constexpr int SIZE = FORM == SUMS ? 4 : 2;
+    const int row = wr * 16 * MI + lo, down = 16 * m.N * SIZE;
+    const int bytes = min(BM, m.M - cur.m0) * m.N * SIZE;
+    const int64_t at = ((int64_t)cur.split * m.M + cur.m0) * m.N;
+#pragma unroll
+    for (int j = 0; j < NI / (FORM == GATED ? 4 : 2); ++j) {
+      const int c = cur.n0 + wc * (OUT_N / 2) + j * 32 + hi * 8;
+      const int o = (row * m.N + c) * SIZE;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if constexpr (FORM == SUMS) {
+          ring_store(m.sums + at, bytes, c < m.N ? o + i * down : NONE,
+                     __builtin_bit_cast(u32x4, acc[2 * j][i]));
+          ring_store(m.sums + at, bytes, c + 4 < m.N ? o + i * down + 16 : NONE,
+                     __builtin_bit_cast(u32x4, acc[2 * j + 1][i]));
+        } else {
+          float v[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            v[q] = acc[2 * j + q / 4][i][q % 4];
+            if constexpr (FORM == GATED)
+              v[q] = v[q] / (1.f + __expf(-v[q])) *
+                     acc[NI / 2 + 2 * j + q / 4][i][q % 4];
+            else
+              v[q] += bf16_to_f32(bias[j][q]);
+          }
+          if (FORM == ROWS && m.gelu)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = gelu_tanh_f32(v[q]);
+          ring_store(m.out + at, bytes, c < m.N ? o + i * down : NONE,
+                     __builtin_bit_cast(u32x4, pack8(v)));
+        }
+      }
+    }
+    if (!item_of(round, cur)) break;
+    stores_open = NB - 1;
+  }
+  // LDS goes to another workgroup when no load is on its way to it
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+}
+
+// What the kernel's offsets of 32 bits reach.
+bool ring_fits(const Ring& m, RingForm form) {
+  return m.K % 64 == 0 && m.K <= 1 << 21 && m.N <= 1 << 20 &&
+         m.N % (form == SUMS ? 4 : 8) == 0 &&
+         (form != GATED || (int64_t)4 * m.N * m.K < INT32_MAX);
+}
+
+// Tiles of 32 mi x 32 ni by workgroups as there are CUs, in us, from 150 sizes
+// (130 to 16600 rows, 768 to 28672 columns, 768 to 14336 deep, weights from
+// memory) with 23 tiles each: what it picks takes 1.6% longer than the best of
+// them, at worst 40% (130 rows of 28672 x 4096, bound by its weights).
+// Workgroups that are alone run faster.
+struct RingTile {
+  int mi, ni;
+};
+double ring_us(const Ring& m, RingForm form, RingTile t, int stretches,
+               int cus) {
+  const int64_t items = (int64_t)cdiv(m.M, 32 * t.mi) *
+                        cdiv(m.N, (form == GATED ? 16 : 32) * t.ni) * stretches;
+  const int steps = cdiv(m.K / 64, stretches), q = t.mi * t.ni;
+  const double item = steps * (0.077 + 0.0147 * q + 0.0209 * (t.mi + t.ni)) +
+                      q * (form == ROWS ? m.gelu ? 0.13 : 0.057
+                           : form == GATED ? 0.08 : 0.1);
+  const double rest = (double)(items % cus) / cus;
+  const double us = (double)(items / cus) + (rest > 0 ? 0.685 + 0.315 * rest : 0);
+  return std::max(3.5 + us * item,
+                  (form == GATED ? 2 : 1) * (double)m.N * m.K / 2e6);
+}
+
+int ring_cus() {
+  int device, cus;
+  TORCH_CHECK(hipGetDevice(&device) == hipSuccess &&
+              hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                                    device) == hipSuccess && cus > 0);
+  return cus;
+}
+
+bool ring_allow(const void* kernel) {
+  TORCH_CHECK(hipFuncSetAttribute(
+                  kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                  RING_LDS) == hipSuccess, "LDS size refused");
+  return true;
+}
+
+template <int MI, int NI, RingForm FORM>
+void ring_run(Ring m, int stretches) {
+  const void* kernel = (const void*)gemm_ring_kernel<MI, NI, FORM>;
+  static const bool once = ring_allow(kernel);
+  (void)once;
+  m.m_tiles = cdiv(m.M, 32 * MI);
+  m.n_tiles = cdiv(m.N, (FORM == GATED ? 16 : 32) * NI);
+  const int64_t total = (int64_t)m.m_tiles * m.n_tiles * stretches;
+  TORCH_CHECK(total < 1 << 30, "a product of too many tiles");
+  m.tiles = m.m_tiles * m.n_tiles;
+  m.total = (int)total;
+  m.by_tiles = Divide(m.tiles);
+  m.by_group = Divide(RING_GROUP * m.n_tiles);
+  void* args[] = {&m};
+  const hipError_t err = hipLaunchKernel(
+      kernel, dim3(std::min(ring_cus(), m.total)), dim3(256), args, RING_LDS,
+      at::hip::getCurrentHIPStream());
+  TORCH_CHECK(err == hipSuccess, hipGetErrorString(err));
+}
+
+}  // namespace
+}  // namespace helix

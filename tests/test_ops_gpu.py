@@ -955,6 +955,65 @@ def test_gemm_bf16_pair():
     torch.testing.assert_close(got.double(), x.double() @ w.double().t(),
                                rtol=2 ** -8, atol=2e-5)
 
+_RING_TILES = [22, 34, 42, 48, 52, 54, 56, 58, 64, 66, 78, 88]
+
+
+@pytest.mark.parametrize("tile", _RING_TILES)
+@pytest.mark.parametrize("m,n,k,act", [
+    (1, 8, 64, 0), (257, 264, 64, 1), (130, 520, 192, 0),
+    (32 * 9 + 31, 32 * 13 + 8, 448, 1), (2051, 3080, 128, 0),
+    (5000, 4104, 64, 1), (900, 264, 1088, 0)])
+def test_gemm_ring_tiles(tile, m, n, k, act):
+    """Every tile: one item and several rounds of them, fewer steps than are
+    ordered ahead, groups of rows that are not full, remainders of rows and
+    columns."""
+    torch.manual_seed(m + tile)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    room = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_bf16(room[:m], x, w, b, act, tile)
+    want = x.double() @ w.double().t() + b.double()
+    if act:
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    # fp32 sums of k products and GELU's exponential, the rounding to bf16
+    torch.testing.assert_close(room[:m].double(), want, rtol=2 ** -8,
+                               atol=2e-5)
+    assert (room[m] == 7).all()
+
+
+def test_gemm_bf16_where_the_ring_ends():
+    """Operands and results off 16-byte boundaries, columns that are no
+    multiple of 8: the same values by the kernels that take them."""
+    torch.manual_seed(50)
+    m, n, k = 300, 520, 192
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n + 1, dtype=torch.bfloat16, device=DEV)
+    off = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)  # noqa: E731
+    native = ops._native().gemm_bf16
+    want = x.double() @ w.double().t() + b[1:].double()
+    for form in ("bias", "x", "w", "out"):
+        out = torch.empty(m * n + 1, dtype=torch.bfloat16, device=DEV)
+        out = out[form == "out":][:m * n].view(m, n)
+        native(out, off(x) if form == "x" else x, off(w) if form == "w" else w,
+               b[1:], 0)
+        # fp32 sums of k products, then the rounding to bf16
+        torch.testing.assert_close(out.double(), want, rtol=2 ** -8, atol=2e-5)
+    with pytest.raises(RuntimeError, match="no tile of"):
+        native(out.new_empty(m, n), x, w, None, 0, 11)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4, 64), (300, 1028, 4160),
+                                   (700, 4096, 2048), (130, 260, 8256)])
+def test_gemm_bf16_sums_by_plan(m, n, k):
+    torch.manual_seed(51)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    sums = ops._native().gemm_bf16_sums(x, w, 0)
+    torch.testing.assert_close(sums.double().sum(0), x.double() @ w.double().t(),
+                               rtol=1e-5, atol=2e-5)  # fp32 sums of k products
+
 
 @pytest.mark.parametrize("n,act", [(3002, 0), (3002, 1), (3004, 1)])
 def test_gemm_bf16_pair_epilogue(n, act):
