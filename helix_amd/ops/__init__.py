@@ -388,18 +388,16 @@ def gemm_fp8(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,
 
 def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
               act: int = 0) -> torch.Tensor:
-    """act(x @ w^T + bias), act 1: GELU (tanh). Up to 64 rows stream their
-    weights instead of going by tiles (us with weights from memory, tiles and
-    streamed: 8 rows of 6144 x 1024 14.1 and 7.6, 33 of 768 x 3072 25.1 and
-    7.3, 64 of 3072 x 768 9.0 and 8.2); up to 128 where the inner dimension is
-    long (2048 x 8192 23.8 and 20.5, 1024 x 8192 23.0 and 17.5), else tiles or
-    their stretches are as fast (1024 x 2048 11.9 and 12.9, 2304 x 768 9.6 and
-    12.3)."""
+    """act(x @ w^T + bias), act 1: GELU (tanh). Up to 64 rows of a small deep
+    matrix stream their weights instead of going by tiles (us with weights from
+    memory, streamed and by tiles: 8 rows of 768 x 3072 7.9 and 8.9, of 1024 x
+    4096 7.9 and 9.1; of 6144 x 1024 7.7 and 7.2, of 2048 x 8192 11.4 and 10.9,
+    64 of 3072 x 768 7.9 and 6.4)."""
     if x.is_cuda:
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
-        if (_rows_fit(x, w, 128 if w.shape[1] >= max(2 * w.shape[0], 4096)
-                      else 64, grads=False)
+        if (w.dim() == 2 and w.shape[1] >= 2 * w.shape[0]
+                and w.numel() <= 8 << 20 and _rows_fit(x, w, 64, grads=False)
                 and x.dtype == torch.bfloat16 and _bias_fits(bias, w)):
             _native().gemm_rows(out, x, w, bias, None, None, act == 1)
         else:
@@ -451,6 +449,7 @@ def gemm_skinny_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
 
 
 ROWS_MAX_M = 128                  # of gemm_rows.hip
+ROWS_ANY = 1 << 30                # of gemm_ring.h
 ROWS_MAX_M_GLU = 64               # of its gated form
 ROWS_CHUNK = 512                  # bytes
 
@@ -498,27 +497,31 @@ def _bias_fits(bias, w: torch.Tensor) -> bool:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
-    """Projection dispatch: a few rows on the owned kernel, everything else
-    (prefill-sized M, CPU, odd dims) via torch/hipBLASLt.
+    """Projection dispatch: owned kernels in inference, everything else (CPU,
+    gradients, other types and strides, odd dims) via torch/hipBLASLt.
 
-    The line is where both were measured equal: up to 16 rows the owned kernel
-    is faster (28672 x 4096: 45 against 65 us) but for vocabularies (128256 x
-    4096: 191 against 189); from 17 to 64 rows it stays so where the inner
-    dimension is the longer one (4096 x 14336: 30 against 34 and 35 against
-    42), elsewhere adding up the stretches costs what it gains. From 65 rows on
-    see _rows_many."""
+    The lines are where both were measured equal, with weights from memory. Up
+    to 16 rows stream their weights (28672 x 4096: 45 against 65 us), but for
+    vocabularies (128256 x 4096: 191 against 189). From 17 rows on tiles
+    (gemm_ring.h) take less than the library's product in most sizes and up to
+    a tenth more in some: 64 rows of 4096 x 14336 29 us and 39, 300 of 6144 x
+    4096 28 and 27, 1540 of 4096 x 4096 48 and 52, 4100 of 4096 x 14336 384 and
+    733, 8192 of 6144 x 4096 269 and 263. Up to 128 rows of a wide matrix, bound
+    by its weights, are the library's (128 of 28672 x 4096: 63 and 55)."""
     if (_SKINNY_ENABLED and x.is_cuda and x.dtype == torch.bfloat16
             and x.dim() == 2
             and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= _SKINNY_MAX_M
             and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0
             and x.is_contiguous() and w.is_contiguous()):
         return gemm_skinny_bf16(x, w, bias)
-    if _rows_fit(x, w) and _bias_fits(bias, w):
-        (M, K), N = x.shape, w.shape[0]
-        if (M <= 16 and N <= 65536 or K >= 2 * N if M <= 64 else
-                _rows_many(N, K) and (N <= 6144 or K > N)):
+    if _rows_fit(x, w, ROWS_ANY) and _bias_fits(bias, w):
+        M, N = x.shape[0], w.shape[0]
+        if N <= 65536 if M <= 16 else N <= 8192 or M > ROWS_MAX_M:
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-            _native().gemm_rows(out, x, w, bias, None, None)
+            if M <= 16:
+                _native().gemm_rows(out, x, w, bias, None, None)
+            else:
+                _native().gemm_bf16(out, x, w, bias, 0)
             return out
     return torch.nn.functional.linear(x, w, bias)
 
@@ -537,15 +540,18 @@ def _rows_many(N: int, K: int) -> bool:
 def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T for a reader that adds up stretches of the inner dimension
     (fused_add_rms_norm, rope_qkv_cache): [stretches, M, N] fp32 for a few
-    rows, else [M, N] in x's type. Wide matrices fill the chip without
-    stretches, and 64 rows of 16384 sums are more bytes than they save. At 64
-    rows of 6144 x 4096 it is 17.6 us against the library's 18.0, at 128 rows
-    20 against 25. From 65 rows on see _rows_many, from 129 on _sums_tile."""
+    rows, else [M, N] in x's type. Up to 16 rows stream their weights, from 17
+    rows on tiles are faster (us, streamed and by tiles: 17 rows of 6144 x 4096
+    12 and 12, 61 rows 16.4 and 13.1; 61 of 4096 x 14336 29.4 and 24.0, 128 34.5
+    and 28.2). Wide matrices fill the chip without stretches, whose sums are
+    more bytes than they save. From 129 rows on see _sums_tile."""
     if _rows_fit(x, w) and w.shape[0] <= 8192:
+        if x.shape[0] > 16:
+            return _native().gemm_bf16_sums(x, w, 0)
         return _native().gemm_rows_sums(x, w, None, None)
-    tile = _sums_tile(*x.shape, w.shape[0]) if x.dim() == 2 else 0
-    if tile and _rows_fit(x, w, SUMS_MAX_M):
-        return _native().gemm_bf16_sums(x, w, tile)
+    if x.dim() == 2 and _sums_tile(*x.shape, w.shape[0]) and \
+            _rows_fit(x, w, SUMS_MAX_M):
+        return _native().gemm_bf16_sums(x, w, 0)
     return linear(x, w)
 
 
@@ -564,21 +570,16 @@ SUMS_MAX_M = 2048
 
 @functools.lru_cache(maxsize=4096)
 def _sums_tile(M: int, K: int, N: int) -> int:
-    """Tile of gemm_bf16_sums for M > 128 rows, 0 where the library takes no
-    longer. Stretches pay where a product has too few tiles to fill the chip:
-    at least two to a tile, and work for four fifths of it (256 workgroups of
-    256 x 256, 512 of 128 x 128).
-
-    Both sides are estimated in us, with the norm that reads the result, from
-    176 sizes measured with weights from memory (130 to 2048 rows of 1024 to
-    8192 columns, 4096 to 28672 deep). Ours, off by 3%: launches, steps of 64,
-    sums written and read. The library's, off by 5%: a launch, steps, 1.3
-    PFLOP/s, weights at 6 TB/s; a size in fifteen takes 1.4 to 2 times that
-    (1540 rows of 4096 x 14336 336 us, 194 in stretches; 1800 203 and 213), so
-    it has to be a tenth faster. Over the sizes 0.90 of the library's times, at
-    worst 1.08; some, the library's and ours: 200 rows of 4096 x 14336 63 and
-    49 (128), 512 98 and 79 (256), 1024 138 and 123; 640 rows of 8192 x 28672
-    273 and 347, left to the library."""
+    """Side of the tiles by which M > 128 rows gain from stretches, 0 where rows
+    are as fast; the tile itself is then chosen by time (gemm_bf16.hip).
+    Stretches pay where a product has too few tiles to fill the chip: at least
+    two to a tile, and work for four fifths of it (256 workgroups of 256 x 256,
+    512 of 128 x 128), and where the estimate in us, with the norm that reads
+    the result (launches, steps of 64, sums written and read), is a tenth below
+    that of a product that fills it (a launch, steps, 1.3 PFLOP/s, weights at 6
+    TB/s). With the reading of the result, as rows and in stretches: 200 rows of
+    4096 x 14336 49 and 32, 512 80 and 65, 1540 160 and 150; 512 of 6144 x 4096,
+    left as rows, 33 and 39."""
     if not 128 < M <= SUMS_MAX_M or N > 8192:
         return 0
     steps = K // 64
@@ -617,8 +618,8 @@ def _glu_fits(M: int, N: int, K: int) -> bool:
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T), w = [gate; up]. A few rows: one launch,
-    whose halves stay in registers (55 us at 64 rows of 2 x 14336 x 4096,
-    product and activation apart 57; 45 against 68 at one)."""
+    whose halves stay in registers (45 us at one row of 2 x 14336 x 4096,
+    product and activation apart 68)."""
     if _rows_fit(x, w, ROWS_MAX_M_GLU):
         out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                           device=x.device)
@@ -629,7 +630,18 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear_silu_mul where one launch is the faster form, product and
-    activation apart elsewhere."""
+    activation apart elsewhere. From 33 rows on one launch goes by tiles: us
+    streamed, apart and by tiles 33 rows of 28672 x 4096 54, 55 and 52, 64 rows
+    57, 56 and 52; apart and by tiles 128 rows 57 and 54, 512 104 and 96, 8192
+    1407 and 1285, 288 rows 75 + 4 and 79."""
+    if x.dim() == 2 and w.dim() == 2 and w.shape[0] % 16 == 0 and (
+            x.shape[0] > ROWS_MAX_M_GLU or
+            x.shape[0] > 32 and _glu_fits(x.shape[0], *w.shape)) and \
+            _rows_fit(x, w, ROWS_ANY):
+        out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                          device=x.device)
+        _native().gemm_bf16_glu(out, x, w)
+        return out
     if x.dim() == 2 and w.dim() == 2 and not _glu_fits(x.shape[0], *w.shape):
         return silu_and_mul(linear(x, w))
     return linear_silu_mul(x, w)

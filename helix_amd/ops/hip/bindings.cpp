@@ -55,7 +55,10 @@ void sample_tokens_ext(torch::Tensor out, torch::Tensor logits,
                        c10::optional<torch::Tensor> row_map);
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, int64_t act, int64_t tile);
-torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile);
+torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
+                             int64_t stretches);
+void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                   int64_t tile);
 void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                       c10::optional<torch::Tensor> bias,
                       c10::optional<torch::Tensor> scratch, int64_t split_k,
@@ -110,7 +113,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("out"), py::arg("x"), py::arg("w"), py::arg("bias"),
         py::arg("act"), py::arg("tile") = 0);
   m.def("gemm_bf16_sums", &gemm_bf16_sums,
-        "x @ w^T, stretches of the inner dimension apart");
+        "x @ w^T, stretches of the inner dimension apart", py::arg("x"),
+        py::arg("w"), py::arg("tile"), py::arg("stretches") = 0);
+  m.def("gemm_bf16_glu", &gemm_bf16_glu,
+        "silu(x @ w[:N]^T) * (x @ w[N:]^T) of more than a few rows",
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("tile") = 0);
   m.def("gemm_skinny_bf16", &gemm_skinny_bf16,
         "Skinny-M decode GEMM: split-K + XCD-chunked tile swizzle");
   m.def("gemm_rows", &gemm_rows, "x @ w^T (+bias, GELU) of at most 128 rows",

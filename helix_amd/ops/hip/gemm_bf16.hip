@@ -170,14 +170,14 @@ void run_tiles(Gemm m, uint16_t* out, const uint16_t* x, const uint16_t* w) {
   TILE(2, 2) TILE(3, 4) TILE(4, 2) TILE(4, 8) TILE(5, 2) TILE(5, 4)          \
   TILE(5, 6) TILE(5, 8) TILE(6, 4) TILE(6, 6) TILE(7, 8) TILE(8, 8)
 #define HELIX_RING_SUMS(TILE)                                                \
-  TILE(2, 2) TILE(4, 2) TILE(4, 4) TILE(4, 8) TILE(5, 4) TILE(5, 8)          \
-  TILE(8, 8)
+  TILE(2, 2) TILE(2, 4) TILE(3, 4) TILE(4, 2) TILE(4, 4) TILE(4, 8)          \
+  TILE(5, 4) TILE(5, 8) TILE(8, 8)
 #define HELIX_TILE(MI, NI) {MI, NI},
-constexpr RingTile ROWS_TILES[] = {HELIX_RING_ROWS(HELIX_TILE)};
-constexpr RingTile SUMS_TILES[] = {HELIX_RING_SUMS(HELIX_TILE)};
+constexpr int ROWS_TILES[][2] = {HELIX_RING_ROWS(HELIX_TILE)};
+constexpr int SUMS_TILES[][2] = {HELIX_RING_SUMS(HELIX_TILE)};
 #undef HELIX_TILE
 
-void run_ring(const Ring& m, RingTile t) {
+void run_ring(const Ring& m, const RingTile& t) {
 #define HELIX_RUN(MI, NI)                                                    \
   if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, ROWS>(m, 1);
   HELIX_RING_ROWS(HELIX_RUN)
@@ -185,7 +185,7 @@ void run_ring(const Ring& m, RingTile t) {
   TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni);
 }
 
-void run_ring_sums(const Ring& m, RingTile t, int stretches) {
+void run_ring_sums(const Ring& m, const RingTile& t, int stretches) {
 #define HELIX_RUN(MI, NI)                                                    \
   if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, SUMS>(m, stretches);
   HELIX_RING_SUMS(HELIX_RUN)
@@ -196,14 +196,15 @@ void run_ring_sums(const Ring& m, RingTile t, int stretches) {
 // Tile and stretches, and their time in us with what it takes to read the
 // stretches: their bytes at 4.5 TB/s.
 struct Plan {
-  RingTile tile{0, 0};
+  RingTile tile{};
   int stretches = 1;
   double us = 1e30;
 };
 Plan plan_rows(const Ring& m) {
   Plan best;
   const int cus = ring_cus();
-  for (const RingTile t : ROWS_TILES) {
+  for (const RingTile& t : RING_TILES) {
+    if (!ring_has(ROWS_TILES, t)) continue;
     const double us = ring_us(m, ROWS, t, 1, cus);
     if (us < best.us) best = Plan{t, 1, us};
   }
@@ -212,8 +213,9 @@ Plan plan_rows(const Ring& m) {
 Plan plan_sums(const Ring& m, int from) {
   Plan best;
   const int steps = m.K / 64, cus = ring_cus();
-  for (const RingTile t : SUMS_TILES)
-    for (int n = from; n <= std::min(8, steps); ++n) {
+  for (const RingTile& t : RING_TILES)
+    for (int n = from; n <= std::min(8, steps) && ring_has(SUMS_TILES, t);
+         ++n) {
       const double us = ring_us(m, SUMS, t, n, cus) +
                         4. * n * m.M * m.N / 4.5e6;
       if (us < best.us) best = Plan{t, n, us};
@@ -227,7 +229,7 @@ int cut(Ring& m, int stretches) {
   return cdiv(m.K, m.stretch);
 }
 
-torch::Tensor sums_of(const torch::Tensor& x, Ring& m, RingTile t,
+torch::Tensor sums_of(const torch::Tensor& x, Ring& m, const RingTile& t,
                       int stretches) {
   stretches = cut(m, stretches);
   torch::Tensor sums = torch::empty({stretches, m.M, m.N},
@@ -282,6 +284,7 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     return;
   }
   TORCH_CHECK(x.is_cuda(), "operands on the GPU");
+  const c10::DeviceGuard on(x.device());
   // tiles are loaded 16 bytes at a time
   if ((uintptr_t)x.data_ptr() % 16 != 0) x = x.clone();
   if ((uintptr_t)w.data_ptr() % 16 != 0) w = w.clone();
@@ -296,7 +299,7 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     r.gelu = m.gelu;
     if (tile != 0) {
       r.bias = m.bias;
-      return run_ring(r, RingTile{(int)tile / 10, (int)tile % 10});
+      return run_ring(r, RingTile{(int)tile / 10, (int)tile % 10, 0});
     }
     // A launch that joins stretches takes 3 us more than what it reads (with
     // it, and whole: 300 x 1024 x 4096 13 and 18, 288 x 768 x 3072 9.6 and 12.1;
@@ -321,10 +324,12 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   else run_tiles<32, 64, 2, 2>(m, o, xp, wp);
 }
 
-// Sums [stretches, M, N] for a reader that adds them up: as many stretches of
-// 128 x 128 (256 x 256) tiles as there are workgroups for, up to 512 (256) and
-// 8. tile 0: those that take least time with their reader.
-torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile) {
+// Sums [stretches, M, N] for a reader that adds them up, those that take least
+// time with it. tile 128 (256): as many stretches of squares of that side as
+// there are workgroups for, up to 512 (256) and 8. stretches: that many, by the
+// tile of 32 * (tile / 10) rows and 32 * (tile % 10) columns.
+torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
+                             int64_t stretches) {
   const c10::DeviceGuard on(x.device());
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.is_cuda() &&
@@ -334,13 +339,16 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile) {
   Ring m = ring_of(x, w);
   TORCH_CHECK(w.size(1) == m.K && m.K > 0 && m.K % 64 == 0 && m.M >= 1 &&
               m.N >= 4 && m.N % 4 == 0 &&
-              (tile == 0 || tile == 256 || tile == 128));
+              (stretches > 0 || tile == 0 || tile == 256 || tile == 128));
   TORCH_CHECK(ring_fits(m, SUMS), "a product of more than the offsets reach");
+  if (stretches > 0)
+    return sums_of(x, m, RingTile{(int)tile / 10, (int)tile % 10, 0},
+                   (int)std::min<int64_t>(stretches, m.K / 64));
   if (tile == 0) {
     const Plan p = plan_sums(m, 1);
     return sums_of(x, m, p.tile, p.stretches);
   }
   const int side = (int)tile, tiles = cdiv(m.M, side) * cdiv(m.N, side);
   const int most = std::min({(side == 256 ? 256 : 512) / tiles, m.K / 64, 8});
-  return sums_of(x, m, RingTile{side / 32, side / 32}, std::max(1, most));
+  return sums_of(x, m, RingTile{side / 32, side / 32, 0}, std::max(1, most));
 }

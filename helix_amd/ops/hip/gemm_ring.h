@@ -40,13 +40,14 @@
 #include "hybrid/tile.h"
 #include <ATen/hip/HIPContext.h>
 #include <torch/extension.h>
+#include <cmath>
 
 namespace helix {
 namespace {
 
 enum RingForm { ROWS, GATED, SUMS };          // of the result
 
-constexpr int RING_GROUP = 4;                 // tiles of rows that share columns
+constexpr int RING_STRIP = 8;                 // tiles of columns, see item_of
 constexpr int RING_LDS = 160 * 1024;
 
 // Quotients of a fixed number below 2^31: d <= 2^shift, mul the rounded up rest
@@ -70,6 +71,7 @@ struct Ring {
   uint16_t* out;
   float* sums;                                // [stretch][M][N]
   int M, N, K, m_tiles, n_tiles, tiles, total, stretch, gelu;
+  int group, strip_shift;      // tiles of rows; of group * RING_STRIP tiles
   Divide by_tiles, by_group;
 };
 
@@ -153,21 +155,32 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
   const int lo = lane & 15, hi = lane >> 4, wr = wid / 2, wc = wid % 2;
 
   // Workgroups of an XCD have neighbouring items of a round, also of the last
-  // one, which may not have one for each.
+  // one, which may not have one for each: 4 x 8 tiles, whose rows and columns
+  // its L2 keeps. Four such blocks, or eight, stand above each other in a strip
+  // and the others' blocks beside them, so that a round reads little of either
+  // matrix (8192 x 28672 x 4096: 1317 us with blocks in one row, 1286 with
+  // four of them above each other, 1270 with eight; 8192 x 4096 x 14336: 617,
+  // 615 and 629).
   auto item_of = [&](int round, RingItem& p)
       __attribute__((always_inline)) -> bool {
     const int all = gridDim.x, n = min(all, m.total - round * all);
     if ((int)blockIdx.x >= n) return false;
     const int at = round * all + xcd_chunk(blockIdx.x, n);
     p.split = m.by_tiles(at);
-    const int tile = at - p.split * m.tiles, group = m.by_group(tile);
-    const int in = tile - group * RING_GROUP * m.n_tiles;
-    const int first = group * RING_GROUP;
-    const int rows = min(RING_GROUP, m.m_tiles - first);
-    const int col = rows == 4 ? in >> 2 : rows == 2 ? in >> 1
-                    : rows == 3 ? (int)__umulhi(in, 0x55555556u) : in;
-    p.m0 = (first + in - col * rows) * BM;
-    p.n0 = col * OUT_N;
+    int in = at - p.split * m.tiles;
+    const int group = m.by_group(in);
+    in -= group * m.group * m.n_tiles;
+    const int high = min(m.group, m.m_tiles - group * m.group);
+    const int strip = high == m.group ? in >> m.strip_shift
+                                      : in / (high * RING_STRIP);
+    in -= strip * high * RING_STRIP;
+    const int wide = min(RING_STRIP, m.n_tiles - strip * RING_STRIP);
+    const int block = wide == RING_STRIP ? in >> 5 : in / (4 * wide);
+    in -= block * 4 * wide;
+    const int rows = min(4, high - block * 4);
+    const int col = rows == 4 ? in >> 2 : in / rows;
+    p.m0 = (group * m.group + block * 4 + in - col * rows) * BM;
+    p.n0 = (strip * RING_STRIP + col) * OUT_N;
     p.k0 = p.split * m.stretch;
     p.k1 = min(m.K, p.k0 + m.stretch);
     return true;
@@ -227,8 +240,10 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
     constexpr int Q = MI * NI, R = MI + NI, L = W ? NI : MI;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      ring_mma<decltype(first)::value>(acc[q / MI][q % MI], wa[q / MI],
-                                       xa[q % MI]);
+      // to and fro: one operand is that of the product before (1% of large
+      // products, by the power it saves)
+      const int j = q / MI, i = j & 1 ? MI - 1 - q % MI : q % MI;
+      ring_mma<decltype(first)::value>(acc[j][i], wa[j], xa[i]);
 #pragma unroll
       for (int r = 0; r < R; ++r)             // in three quarters of the half
         if (r * 3 * Q / (4 * R) == q) {
@@ -352,26 +367,48 @@ bool ring_fits(const Ring& m, RingForm form) {
          (form != GATED || (int64_t)4 * m.N * m.K < INT32_MAX);
 }
 
-// Tiles of 32 mi x 32 ni by workgroups as there are CUs, in us, from 150 sizes
-// (130 to 16600 rows, 768 to 28672 columns, 768 to 14336 deep, weights from
-// memory) with 23 tiles each: what it picks takes 1.6% longer than the best of
-// them, at worst 40% (130 rows of 28672 x 4096, bound by its weights).
-// Workgroups that are alone run faster.
+// Tiles of 32 mi x 32 ni, and us of a step of one with every CU at work.
 struct RingTile {
   int mi, ni;
+  double step;
 };
-double ring_us(const Ring& m, RingForm form, RingTile t, int stretches,
+constexpr RingTile RING_TILES[] = {
+    {1, 4, 0.315}, {2, 2, 0.231}, {2, 4, 0.334}, {3, 4, 0.401}, {4, 2, 0.320},
+    {4, 4, 0.500}, {4, 8, 0.808}, {5, 2, 0.353}, {5, 4, 0.539}, {5, 6, 0.740},
+    {5, 8, 1.010}, {6, 4, 0.616}, {6, 6, 0.891}, {7, 8, 1.216}, {8, 8, 1.300}};
+
+// us of a product by as many workgroups as there are CUs: rounds of items, and
+// what w and sums take to read and write, part of it at the same time. Fitted to
+// 11000 times of 318 sizes (17 to 16000 rows, 768 to 28672 columns, 768 to 14336
+// deep, 1 to 8 stretches, weights from memory). Against the best tile of each
+// size what it picks takes 0.4% longer as rows (at worst 15%), 0.2% gated (4%)
+// and, with the reader of the stretches, 1.6% as sums (at worst 35%, 48 x 768 x
+// 768). An item takes less while other CUs are idle; few workgroups do not reach
+// the rate of the memory.
+double ring_us(const Ring& m, RingForm form, const RingTile& t, int stretches,
                int cus) {
   const int64_t items = (int64_t)cdiv(m.M, 32 * t.mi) *
                         cdiv(m.N, (form == GATED ? 16 : 32) * t.ni) * stretches;
-  const int steps = cdiv(m.K / 64, stretches), q = t.mi * t.ni;
-  const double item = steps * (0.077 + 0.0147 * q + 0.0209 * (t.mi + t.ni)) +
-                      q * (form == ROWS ? m.gelu ? 0.13 : 0.057
-                           : form == GATED ? 0.08 : 0.1);
+  const double end = form == SUMS ? 0.073 : form == GATED ? 0.064
+                     : m.gelu ? 0.11 : 0.038;
+  const double item = cdiv(m.K / 64, stretches) * t.step +
+                      end * t.mi * t.ni + 0.27;
   const double rest = (double)(items % cus) / cus;
-  const double us = (double)(items / cus) + (rest > 0 ? 0.685 + 0.315 * rest : 0);
-  return std::max(3.5 + us * item,
-                  (form == GATED ? 2 : 1) * (double)m.N * m.K / 2e6);
+  const double busy = item * ((double)(items / cus) +
+                              (rest > 0 ? 0.72 + 0.28 * rest : 0));
+  const double fed =
+      (form == GATED ? 4. : 2.) * m.N * m.K / 9e6 /
+          std::sqrt(std::min(1., (double)items / cus)) +
+      (form == SUMS ? 4. * stretches * m.M * m.N / 4.1e6 : 0.);
+  return 3.3 + std::pow(std::pow(busy, 1.8) + std::pow(fed, 1.8), 1 / 1.8);
+}
+
+// Whether a kernel of that tile is in a list of pairs.
+template <int N>
+bool ring_has(const int (&pairs)[N][2], const RingTile& t) {
+  for (const auto& p : pairs)
+    if (p[0] == t.mi && p[1] == t.ni) return true;
+  return false;
 }
 
 int ring_cus() {
@@ -401,7 +438,11 @@ void ring_run(Ring m, int stretches) {
   m.tiles = m.m_tiles * m.n_tiles;
   m.total = (int)total;
   m.by_tiles = Divide(m.tiles);
-  m.by_group = Divide(RING_GROUP * m.n_tiles);
+  // eight blocks of 4 tiles of rows where w is too large for the memory-side
+  // cache beside the rest
+  m.group = (int64_t)m.N * (FORM == GATED ? 2 : 1) * m.K >= 64 << 20 ? 32 : 16;
+  m.strip_shift = m.group == 32 ? 8 : 7;
+  m.by_group = Divide(m.group * m.n_tiles);
   void* args[] = {&m};
   const hipError_t err = hipLaunchKernel(
       kernel, dim3(std::min(ring_cus(), m.total)), dim3(256), args, RING_LDS,

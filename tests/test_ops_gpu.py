@@ -1014,6 +1014,78 @@ def test_gemm_bf16_sums_by_plan(m, n, k):
     torch.testing.assert_close(sums.double().sum(0), x.double() @ w.double().t(),
                                rtol=1e-5, atol=2e-5)  # fp32 sums of k products
 
+@pytest.mark.parametrize("tile", [0, 14, 24, 34, 48, 54, 58, 64, 78, 88])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (65, 264, 192), (515, 1048, 128),
+                                   (2300, 2056, 64), (300, 136, 1088)])
+def test_gemm_gated_tiles(tile, m, n, k):
+    """Every tile of gate and other factor: one item and several rounds,
+    remainders of rows and of columns."""
+    torch.manual_seed(m + tile)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(2 * n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    room = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_bf16_glu(room[:m], x, w, tile)
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    # fp32 sums of k products and the exponential, the rounding to bf16
+    torch.testing.assert_close(
+        room[:m].double(), torch.nn.functional.silu(g) * u, rtol=2 ** -8,
+        atol=5e-5)
+    assert (room[m] == 7).all()
+
+
+def test_gemm_gated_refuses():
+    x, w, out = (torch.zeros(s, dtype=torch.bfloat16, device=DEV)
+                 for s in ((70, 128), (48, 128), (70, 24)))
+    glu = ops._native().gemm_bf16_glu
+    for args, says in (((out, x[:, :96], w), "packed bf16"),
+                       ((out, x, w.float()), "packed bf16"),
+                       ((out[:, :16].contiguous(), x, w), "out is"),
+                       ((out, x, w[:47]), "out is"),
+                       ((out[:, :20].contiguous(), x, w[:40]), "a multiple"),
+                       ((out, x, w, 11), "no tile of")):
+        with pytest.raises(RuntimeError, match=says):
+            glu(*args)
+
+
+@pytest.mark.parametrize("m", [16, 17, 32, 33, 64, 65, 128, 129])
+def test_projections_by_rows(m):
+    """Every form of a projection on either side of the lines between streamed
+    weights, tiles and the library."""
+    torch.manual_seed(52)
+    for n, k in ((1024, 4096), (512, 256), (26624, 2048)):
+        x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+        w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+        b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+        want = x.double() @ w.double().t()
+        g, u = want.chunk(2, -1)
+        with torch.inference_mode():
+            rows, sums = ops.linear(x, w, b), ops.linear_sums(x, w)
+            gated = ops.gated_linear(x, w)
+        if sums.dim() == 3:
+            sums = sums.double().sum(0)
+        # fp32 sums of k products, then the rounding to bf16
+        tol = dict(rtol=2 ** -8, atol=2e-5)
+        torch.testing.assert_close(rows.double(), want + b.double(), **tol)
+        torch.testing.assert_close(sums.double(), want, **tol)
+        # apart, both halves are rounded as well: 2^-9 each of up to 6 x 6
+        torch.testing.assert_close(
+            gated.double(), torch.nn.functional.silu(g) * u, rtol=2 ** -7,
+            atol=36 * 2 ** -8)
+
+
+@pytest.mark.parametrize("tile", [22, 24, 34, 42, 44, 48, 54, 58, 88])
+@pytest.mark.parametrize("m,n,k,stretches", [
+    (1, 4, 64, 1), (130, 516, 704, 3), (700, 1028, 1088, 8),
+    (2200, 2052, 192, 2)])
+def test_gemm_sums_tiles(tile, m, n, k, stretches):
+    """Every tile in stretches, the last of them shorter."""
+    torch.manual_seed(m + tile)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    sums = ops._native().gemm_bf16_sums(x, w, tile, stretches)
+    torch.testing.assert_close(sums.double().sum(0), x.double() @ w.double().t(),
+                               rtol=1e-5, atol=2e-5)  # fp32 sums of k products
+
 
 @pytest.mark.parametrize("n,act", [(3002, 0), (3002, 1), (3004, 1)])
 def test_gemm_bf16_pair_epilogue(n, act):
