@@ -1,12 +1,11 @@
 // Flash-attention prefill (varlen, causal/bidirectional, GQA) for CDNA4.
 //
 // Replaces the prefill attention the reference delegates to vLLM. Bound by
-// instruction issue and power: of a wave's 2200 cycles per tile the matrix
-// cores have 1020, and a SIMD issues one vector instruction in about 5 (170 a
-// tile, half of them for exponentials, and 64 more where a maximum grew); the
-// clock is at 1.85 GHz (on zeros 1 x 8192 takes 451 us instead of 606). LDS is
-// busy for a third. A third wave on a SIMD (tiles of 32 keys), the next scores
-// computed beside the exponentials and two halves of waves a phase apart
+// instruction issue and, at long contexts, by power: a wave takes 1876 cycles a
+// tile, its products 1020 and its 200 vector instructions 1050 (one in 5), and
+// the clock is at 1.75 GHz (on zeros 1 x 8192 takes 451 us instead of 568). LDS
+// is busy for a quarter. A third wave on a SIMD (tiles of 32 keys), the next
+// scores computed beside the exponentials and two halves of waves a phase apart
 // change nothing or cost.
 //
 //  - A workgroup has 128 queries of one head, each of its 4 waves 32 of them,
@@ -25,10 +24,12 @@
 //
 // 32 heads on 8 of 128, us of the first kernel (64 queries, values transposed
 // element by element) -> products of 16x16 with addresses computed per tile
-// (340 vector instructions) -> now (TFLOP/s now): 1 x 8192 2551 -> 645 -> 606
-// (907), 8 x 2048 1918 -> 413 -> 395 (695), 31 of 400..620 440 -> 188 -> 183
-// (393), 1500 behind 5001 with a window of 4096 466 -> 173 -> 159 (632). 12
-// heads of 64, 64 texts of 20..500: 178 -> 68 -> 62. Workgroups of 64 queries
+// (340 vector instructions) -> with the next tile's loads waited for by reads of
+// LDS -> now (TFLOP/s now; the last two on one card): 1 x 8192 2551 -> 645 ->
+// 579 -> 568 (968), 8 x 2048 1918 -> 413 -> 364 -> 341 (806), 31 of 400..620
+// 440 -> 188 -> 168 -> 154 (467), 1500 behind 5001 with a window of 4096 466 ->
+// 173 -> 136 -> 130 (773). 12 heads of 64, 64 texts of 20..500: 178 -> 68 -> 52
+// -> 49.6; 16 heads, 8 x 288: 12.5 -> 10.6. Workgroups of 64 queries
 // (2 waves) took 1.1 to 1.8 times as long from 100 queries on, and no less time
 // below. The distance from 64 bits is what it was.
 //
@@ -91,6 +92,20 @@ __device__ __forceinline__ u16x4 ld_tr4(const uint16_t* p) {
       (__attribute__((address_space(3))) i16x4*)p));
 }
 
+// 64 lanes' 16 bytes at base + offset to 1024 bytes of LDS. As a builtin the
+// compiler lets every transposing read wait for all such loads, the next tile's
+// among them; here the barrier of a tile alone does, after its own wait.
+__device__ __forceinline__ void direct_load(const char* base, unsigned offset,
+                                            uint16_t* lds) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const unsigned to = (unsigned)(uintptr_t)(
+      __attribute__((address_space(3))) uint16_t*)lds;
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, %1"
+               ::"v"(offset), "s"(base), "s"(to) : "memory", "m0");
+#endif
+}
+
 // Piece p of row r lies at p ^ cross(r): 16 rows of a score operand, and 4
 // rows of 4 pieces of a value operand, meet every bank equally.
 template <int D>
@@ -106,8 +121,9 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
     Prefill m) {
   constexpr int NK = D / 16, NV = D / 32, PR = D / 8;
   constexpr int LOADS = KT * PR / NT;
-  __shared__ __attribute__((aligned(16))) uint16_t kl[2][KT * D];
-  __shared__ __attribute__((aligned(16))) uint16_t vl[2][KT * D];
+  extern __shared__ __attribute__((aligned(16))) uint16_t tiles[];
+  uint16_t* const kl[2] = {tiles, tiles + KT * D};
+  uint16_t* const vl[2] = {tiles + 2 * KT * D, tiles + 3 * KT * D};
   const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
   const int total = m.seqs * m.Hq, chunk = cdiv(total, 8);
   const int sh = xcd * chunk + at / m.q_tiles;
@@ -153,11 +169,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
     const char* from = (const char*)(base + t * stride);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) uint32_t*)(from + o[i]),
-          (__attribute__((address_space(3))) uint32_t*)(
-              lds + (i * NW + wid) * WAVE * 8),
-          16, 0, 0);
+      direct_load(from, o[i], lds + (i * NW + wid) * WAVE * 8);
   };
   places(KT, m.k_stride, ko);
   places(KT, m.v_stride, vo);
@@ -220,6 +232,9 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
     }
     __builtin_amdgcn_sched_group_barrier(MFMA, 4, 0);
 
+    // heads of 64 have as much to do here as in products: the other wave's
+    // products go first (8 x 288 11.6 -> 10.5 us; heads of 128 lose 1 to 2%)
+    if (D == 64) __builtin_amdgcn_s_setprio(0);
     const bool edge = (CAUSAL && t + KT - 1 > qa) || t + KT > klen ||
                       (windowed && t <= qz - m.window);
     if (edge) {
@@ -264,6 +279,7 @@ __global__ __launch_bounds__(NT, 2) void attn_prefill_kernel(
       }
       pf[k] = pack8(p);
     }
+    if (D == 64) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int k = 0; k < KT / 16; ++k)
 #pragma unroll
@@ -363,8 +379,8 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
   const dim3 grid(8 * cdiv(B * Hq, 8) * m.q_tiles);
   auto stream = at::hip::getCurrentHIPStream();
 #define LAUNCH(DH, C)                                                        \
-  hipLaunchKernelGGL((attn_prefill_kernel<DH, C>), grid, dim3(NT), 0,        \
-                     stream, (uint16_t*)out.data_ptr(),                      \
+  hipLaunchKernelGGL((attn_prefill_kernel<DH, C>), grid, dim3(NT),           \
+                     4 * KT * DH * 2, stream, (uint16_t*)out.data_ptr(),                      \
                      (const uint16_t*)q.data_ptr(),                          \
                      (const uint16_t*)k.data_ptr(),                          \
                      (const uint16_t*)v.data_ptr(), m)
