@@ -516,7 +516,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
         return gemm_skinny_bf16(x, w, bias)
     if _rows_fit(x, w, ROWS_ANY) and _bias_fits(bias, w):
         M, N = x.shape[0], w.shape[0]
-        if N <= 65536 if M <= 16 else N <= 8192 or M > ROWS_MAX_M:
+        if N <= 65536 if M <= 16 else \
+                _ring_fits(*w.shape) and (N <= 8192 or M > ROWS_MAX_M):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             if M <= 16:
                 _native().gemm_rows(out, x, w, bias, None, None)
@@ -537,6 +538,13 @@ def _rows_many(N: int, K: int) -> bool:
     return N <= 8192 and N * K >= 13 << 20
 
 
+def _ring_fits(N: int, K: int, gated: bool = False) -> bool:
+    """Whether the offsets of gemm_ring.h reach a matrix [N, K]."""
+    if gated:                     # both halves lie behind one descriptor
+        return K <= 1 << 21 and N <= 1 << 21 and 2 * N * K < (1 << 31) - 1
+    return K <= 1 << 21 and N <= 1 << 20
+
+
 def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T for a reader that adds up stretches of the inner dimension
     (fused_add_rms_norm, rope_qkv_cache): [stretches, M, N] fp32 for a few
@@ -546,11 +554,11 @@ def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     and 28.2). Wide matrices fill the chip without stretches, whose sums are
     more bytes than they save. From 129 rows on see _sums_tile."""
     if _rows_fit(x, w) and w.shape[0] <= 8192:
-        if x.shape[0] > 16:
+        if x.shape[0] > 16 and _ring_fits(*w.shape):
             return _native().gemm_bf16_sums(x, w, 0)
         return _native().gemm_rows_sums(x, w, None, None)
     if x.dim() == 2 and _sums_tile(*x.shape, w.shape[0]) and \
-            _rows_fit(x, w, SUMS_MAX_M):
+            _rows_fit(x, w, SUMS_MAX_M) and _ring_fits(*w.shape):
         return _native().gemm_bf16_sums(x, w, 0)
     return linear(x, w)
 
@@ -637,7 +645,7 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if x.dim() == 2 and w.dim() == 2 and w.shape[0] % 16 == 0 and (
             x.shape[0] > ROWS_MAX_M_GLU or
             x.shape[0] > 32 and _glu_fits(x.shape[0], *w.shape)) and \
-            _rows_fit(x, w, ROWS_ANY):
+            _ring_fits(*w.shape, gated=True) and _rows_fit(x, w, ROWS_ANY):
         out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                           device=x.device)
         _native().gemm_bf16_glu(out, x, w)

@@ -1073,6 +1073,32 @@ def test_projections_by_rows(m):
             atol=36 * 2 ** -8)
 
 
+@pytest.mark.parametrize("m,n,k", [(20, 16, (1 << 21) + 256),
+                                   (130, 16, (1 << 21) + 256),
+                                   (70, 4096, 1 << 18)])
+def test_projections_beyond_the_tiles(m, n, k):
+    """Matrices that the offsets of the persistent tiles do not reach, as rows
+    of more than 2^21 or as two halves of 2^31 bytes, go the other ways."""
+    torch.manual_seed(53)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    with torch.inference_mode():
+        sums, gated = ops.linear_sums(x, w), ops.gated_linear(x, w)
+        rows = ops.linear(x, w)
+    want = x.double() @ w.double().t()
+    g, u = want.chunk(2, -1)
+    if sums.dim() == 3:
+        sums = sums.double().sum(0)
+    # fp32 sums of k products (2^-24 of a partial sum each, sums of 1 in all),
+    # then the rounding to bf16; gated as two rounded halves of up to 6 x 6
+    tol = dict(rtol=2 ** -8, atol=2e-4)
+    torch.testing.assert_close(sums.double(), want, **tol)
+    torch.testing.assert_close(rows.double(), want, **tol)
+    torch.testing.assert_close(
+        gated.double(), torch.nn.functional.silu(g) * u, rtol=2 ** -7,
+        atol=36 * 2 ** -8)
+
+
 @pytest.mark.parametrize("tile", [22, 24, 34, 42, 44, 48, 54, 58, 88])
 @pytest.mark.parametrize("m,n,k,stretches", [
     (1, 4, 64, 1), (130, 516, 704, 3), (700, 1028, 1088, 8),
