@@ -1181,6 +1181,28 @@ def test_quantize_rows_bytes(T, K):
     assert torch.equal(got.nan_to_num(), want.float().nan_to_num())
 
 
+@pytest.mark.parametrize("n,t,h", [(1, 1, 8), (3, 5, 64), (9, 2, 1028 * 2),
+                                   (8, 1, 4088), (4, 33, 4096), (2, 3, 4104),
+                                   (17, 2, 4096)])
+def test_norm_over_stretches_by_width(n, t, h):
+    """Rows that stay in registers, up to 4096 columns, and longer ones."""
+    torch.manual_seed(n)
+    x = torch.randn(n, t, h, device=DEV)
+    res = torch.randn(t, h, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(h, dtype=torch.bfloat16, device=DEV)
+    total = x.double().sum(0) + res.double()
+    room = torch.full((t + 1, h), 7.0, dtype=torch.bfloat16, device=DEV)
+    room[:t] = res
+    got, new = ops.fused_add_rms_norm(x, room[:t], w, 1e-5)
+    # n sums in fp32, the rounding to bf16
+    torch.testing.assert_close(new.double(), total, rtol=2 ** -8, atol=1e-5)
+    want = total * (total.square().mean(-1, keepdim=True) + 1e-5).rsqrt() \
+        * w.double()
+    # the row is rounded before its norm and after it
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -7, atol=1e-5)
+    assert (room[t] == 7).all()
+
+
 def test_three_dimensions_of_bf16():
     """Batches of rows and rows of heads are not a product's stretches."""
     torch.manual_seed(34)
