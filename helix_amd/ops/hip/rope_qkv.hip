@@ -10,6 +10,12 @@
 // thread has 8 pairs of a head or 8 values, and a token's threads are spread
 // over workgroups of 128: with one workgroup of 256 a token, a pair a thread
 // at a time, a row took 7.8 us and 16k rows 115.
+//
+// A few rows are bound by a launch and the latency of memory: both halves of a
+// head and its angles are under way together, and a page is found by a shift.
+// us before -> now: 1 row of 4 stretches of 6144 2.85 -> 2.6, 8 of 5 3.1 -> 2.75,
+// 61 of 2 3.1 -> 2.7; rows in bf16 512 4.15 -> 3.8, 1540 7.7 -> 7.35, 16000 74.5
+// -> 74.1.
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -28,35 +34,42 @@ struct Epilogue {
   uint16_t *q, *k, *v;         // compact; k and v may be null
   void *kc, *vc;
   const float* cs;
-  int Hq, Hkv, D, bs, stretches;
+  int Hq, Hkv, D, bs, shift, stretches;      // bs is 1 << shift, or shift -1
 };
 
-// N values of a row at column c.
-template <int N, bool SUMS>
+// P times N values of a row from column c on, apart columns from each other.
+template <int N, int P, bool SUMS>
 __device__ __forceinline__ void read(const Epilogue& m, int64_t t, int c,
-                                     float* o) {
+                                     int apart, float (*o)[N]) {
   if constexpr (SUMS) {
     const float* p = (const float*)m.qkv + t * m.stride + c;
 #pragma unroll
-    for (int i = 0; i < N; ++i) o[i] = 0.f;
-#pragma unroll 4
-    for (int s = 0; s < m.stretches; ++s, p += m.all) {
-      if constexpr (N == 8) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(p);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(p + 4);
+    for (int k = 0; k < P; ++k)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          o[i] += a[i];
-          o[4 + i] += b[i];
+      for (int i = 0; i < N; ++i) o[k][i] = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < m.stretches; ++s, p += m.all)
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        const float* from = p + k * apart;
+        if constexpr (N == 8) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(from);
+          const f32x4 b = *reinterpret_cast<const f32x4*>(from + 4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            o[k][i] += a[i];
+            o[k][4 + i] += b[i];
+          }
+        } else {
+          o[k][0] += *from;
         }
-      } else {
-        o[0] += p[0];
       }
-    }
   } else {
     const uint16_t* p = (const uint16_t*)m.qkv + t * m.stride + c;
-    if constexpr (N == 8) load_bf16x8(p, o);
-    else o[0] = bf16_to_f32(*p);
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+      if constexpr (N == 8) load_bf16x8(p + k * apart, o[k]);
+      else o[k][0] = bf16_to_f32(p[k * apart]);
   }
 }
 template <int N>
@@ -86,28 +99,34 @@ __global__ __launch_bounds__(NT) void rope_qkv_cache_kernel(Epilogue m) {
   const int turned = (m.Hq + m.Hkv) * per;    // then the values
   int i = blockIdx.y * NT + threadIdx.x;
   if (i >= turned + m.Hkv * m.D / N) return;
+  const int64_t position = m.positions[t];
   const int64_t slot = m.slots != nullptr ? m.slots[t] : -1;
-  const int64_t page = slot >= 0 ? slot / m.bs : 0;
-  const int off = slot >= 0 ? (int)(slot % m.bs) : 0;
   auto place = [&](int h) {
-    return ((page * m.Hkv + h) * m.bs + off) * m.D;
+    const int64_t page = m.shift >= 0 ? slot >> m.shift : slot / m.bs;
+    return ((page * m.Hkv + h) * m.bs + (slot - page * m.bs)) * m.D;
   };
   if (i >= turned) {
     i = (i - turned) * N;
-    float v[N];
-    read<N, SUMS>(m, t, (m.Hq + m.Hkv) * m.D + i, v);
-    if (m.v != nullptr) write<N>(m.v + t * m.Hkv * m.D + i, v);
-    if (slot >= 0) write_cache<N, F8>(m.vc, place(i / m.D) + i % m.D, v);
+    float v[1][N];
+    read<N, 1, SUMS>(m, t, (m.Hq + m.Hkv) * m.D + i, 0, v);
+    if (m.v != nullptr) write<N>(m.v + t * m.Hkv * m.D + i, v[0]);
+    if (slot >= 0) write_cache<N, F8>(m.vc, place(i / m.D) + i % m.D, v[0]);
     return;
   }
   const int h = i / per, d = i % per * N;
-  const float* cs = m.cs + m.positions[t] * m.D + d;
-  float x[N], y[N];
-  read<N, SUMS>(m, t, h * m.D + d, x);
-  read<N, SUMS>(m, t, h * m.D + half + d, y);
+  const float* cs = m.cs + position * m.D + d;
+  // before the row, so that they are under way with it
+  float cosine[N], sine[N], xy[2][N];
 #pragma unroll
   for (int j = 0; j < N; ++j) {
-    const float a = x[j], b = y[j], c = cs[j], s = cs[half + j];
+    cosine[j] = cs[j];
+    sine[j] = cs[half + j];
+  }
+  read<N, 2, SUMS>(m, t, h * m.D + d, half, xy);
+  float *x = xy[0], *y = xy[1];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float a = x[j], b = y[j], c = cosine[j], s = sine[j];
     x[j] = a * c - b * s;
     y[j] = b * c + a * s;
   }
@@ -163,12 +182,14 @@ void rope_qkv_cache(torch::Tensor positions, torch::Tensor qkv,
   m.Hkv = num_kv_heads;
   m.D = head_dim;
   m.bs = 1;
+  m.shift = 0;
   bool f8 = false;
   if (k_cache.has_value()) {
     f8 = k_cache->scalar_type() == torch::kUInt8;
     TORCH_CHECK(v_cache.has_value() && slot_mapping.has_value());
     TORCH_CHECK(slot_mapping->scalar_type() == torch::kInt64);
     m.bs = k_cache->size(2);
+    m.shift = (m.bs & (m.bs - 1)) == 0 ? __builtin_ctz(m.bs) : -1;
     m.kc = k_cache->data_ptr();
     m.vc = v_cache->data_ptr();
     m.slots = slot_mapping->data_ptr<int64_t>();
