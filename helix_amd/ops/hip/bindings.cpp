@@ -57,6 +57,7 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, int64_t act, int64_t tile);
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
                              int64_t stretches);
+std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps);
 void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    int64_t tile);
 void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -115,6 +116,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_bf16_sums", &gemm_bf16_sums,
         "x @ w^T, stretches of the inner dimension apart", py::arg("x"),
         py::arg("w"), py::arg("tile"), py::arg("stretches") = 0);
+  m.def("gemm_ring_places", &gemm_ring_places,
+        "Where a workgroup of gemm_bf16 loads along the inner dimension");
   m.def("gemm_bf16_glu", &gemm_bf16_glu,
         "silu(x @ w[:N]^T) * (x @ w[N:]^T) of more than a few rows",
         py::arg("out"), py::arg("x"), py::arg("w"), py::arg("tile") = 0);

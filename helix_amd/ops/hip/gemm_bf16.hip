@@ -352,3 +352,22 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
   const int most = std::min({(side == 256 ? 256 : 512) / tiles, m.K / 64, 8});
   return sums_of(x, m, RingTile{side / 32, side / 32, 0}, std::max(1, most));
 }
+
+// Places along the inner dimension that a workgroup orders in so many steps, of
+// items from k[2 i] to k[2 i + 1] and after the last of them.
+std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps) {
+  RingAt at;
+  size_t item = 0;
+  auto next = [&] {
+    at.close();
+    if (item + 1 < k.size()) at.open((int)k[item], (int)k[item + 1]);
+    item += 2;
+  };
+  next();
+  std::vector<int64_t> places;
+  for (int64_t i = 0; i < steps; ++i) {
+    places.push_back(at.k);
+    if (at.step()) next();
+  }
+  return places;
+}

@@ -49,6 +49,7 @@ enum RingForm { ROWS, GATED, SUMS };          // of the result
 
 constexpr int RING_STRIP = 8;                 // tiles of columns, see item_of
 constexpr int RING_LDS = 160 * 1024;
+constexpr int RING_STEP = 64;                 // of the inner dimension
 
 // Quotients of a fixed number below 2^31: d <= 2^shift, mul the rounded up rest
 // of 2^(32 + shift) / d above 2^32.
@@ -77,6 +78,24 @@ struct Ring {
 
 struct RingItem {
   int m0, n0, split, k0, k1;
+};
+
+// Where loads are along the inner dimension. After the last item they stay at
+// its start: descriptors are empty by then, and what lies past the end of one is
+// checked by a load's own offset, not by this scalar one on top of it.
+struct RingAt {
+  int k, end, ahead;
+  __host__ __device__ __forceinline__ void open(int k0, int k1) {
+    k = k0;
+    end = k1;
+    ahead = RING_STEP;
+  }
+  __host__ __device__ __forceinline__ void close() {
+    k = ahead = 0;
+    end = 0x7fffffff;
+  }
+  // Whether all of the item is ordered.
+  __host__ __device__ __forceinline__ bool step() { return (k += ahead) >= end; }
 };
 
 // A thread's 16-byte pieces of ROWS_ rows of 64, as offsets in bytes.
@@ -139,7 +158,8 @@ __device__ __forceinline__ void ring_wait() {
 template <int MI, int NI, RingForm FORM>
 __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
 #ifdef __HIP_DEVICE_COMPILE__
-  constexpr int BM = 32 * MI, BN = 32 * NI, BK = 64, AU = BM * BK, BU = BN * BK;
+  constexpr int BM = 32 * MI, BN = 32 * NI, BK = RING_STEP;
+  constexpr int AU = BM * BK, BU = BN * BK;
   // steps of w in LDS, and one more of x: x is ordered in the first half of a
   // step, into what the step before has read, w in the second half, into what
   // this step has read by then; both for NB steps later
@@ -200,26 +220,25 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
 
   // where loads are, NB steps ahead; empty descriptors after the last item
   const uint16_t *x_at = m.x, *w_at = m.w;
-  int x_bytes = 0, w_bytes = 0, k = 0, k_end = 0x7fffffff, load_round = 0;
+  int x_bytes = 0, w_bytes = 0, load_round = 0;
+  RingAt order;
   auto order_from = [&](const RingItem& p, bool on)
       __attribute__((always_inline)) {
-    x_bytes = w_bytes = k = 0;
-    k_end = 0x7fffffff;
+    x_bytes = w_bytes = 0;
+    order.close();
     if (!on) return;
     x_at = m.x + (int64_t)p.m0 * m.K;
     w_at = m.w + (int64_t)p.n0 * m.K;
     x_bytes = min(BM, m.M - p.m0) * m.K * 2;
     w_bytes = FORM == GATED ? (2 * m.N - p.n0) * m.K * 2
                             : min(BN, m.N - p.n0) * m.K * 2;
-    k = p.k0;
-    k_end = p.k1;
+    order.open(p.k0, p.k1);
   };
   RingItem cur, next;
   if (!item_of(0, cur)) return;
   order_from(cur, true);
   auto advance = [&]() __attribute__((always_inline)) {
-    k += BK;
-    if (k < k_end) return;
+    if (!order.step()) return;
     const bool more = item_of(++load_round, next);
     order_from(next, more);
   };
@@ -253,8 +272,10 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
 #pragma unroll
       for (int l = 0; l < L; ++l)
         if (l * Q / L + Q / L / 4 == q) {
-          if (W) ring_load(w_at, w_bytes, wu.off[W ? l : 0], k, to + l * 2048);
-          else ring_load(x_at, x_bytes, xu.off[W ? 0 : l], k, to + l * 2048);
+          if (W) ring_load(w_at, w_bytes, wu.off[W ? l : 0], order.k,
+                           to + l * 2048);
+          else ring_load(x_at, x_bytes, xu.off[W ? 0 : l], order.k,
+                           to + l * 2048);
         }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -263,10 +284,12 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
   for (int s = 0; s < NB; ++s) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
-      ring_load(x_at, x_bytes, xu.off[i], k, xs + s * AU + mine + i * 2048);
+      ring_load(x_at, x_bytes, xu.off[i], order.k,
+                xs + s * AU + mine + i * 2048);
 #pragma unroll
     for (int i = 0; i < NI; ++i)
-      ring_load(w_at, w_bytes, wu.off[i], k, ws + s * BU + mine + i * 2048);
+      ring_load(w_at, w_bytes, wu.off[i], order.k,
+                ws + s * BU + mine + i * 2048);
     advance();
   }
   ring_wait<(NB - 1) * (MI + NI)>();

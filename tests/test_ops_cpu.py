@@ -169,6 +169,15 @@ def test_gemm_bf16_refuses(case, says):
         ops._native().gemm_bf16(out, x, w, b, 0)
 
 
+def test_gemm_ring_loads_stay_at_the_start():
+    """Descriptors are empty after the last item; a scalar offset is not part
+    of their check, so it stays at 0 however many steps follow."""
+    places = ops._native().gemm_ring_places
+    assert places([0, 128, 64, 192], 9) == [0, 64, 64, 128, 0, 0, 0, 0, 0]
+    assert places([0, 64], 40) == [0] * 40
+    assert places([], 3) == [0, 0, 0]
+
+
 @pytest.mark.parametrize("case,says", [
     ("out shape", "out is packed"), ("out rows", "out is packed"),
     ("q", "q is packed"), ("cache", "caches are"), ("pages", "caches are"),
