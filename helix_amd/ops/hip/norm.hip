@@ -259,6 +259,7 @@ void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
   const int T = x.size(1);
   const int H = x.size(2);
   TORCH_CHECK(H % 8 == 0, "H must be a multiple of 8");
+  if (T == 0 || H == 0) return;               // no row, or no column of one
   auto stream = at::hip::getCurrentHIPStream();
   if (H <= WIDE * 4) {
     hipLaunchKernelGGL(add_sums_rms_norm_wide_kernel, dim3(T), dim3(WIDE), 0,

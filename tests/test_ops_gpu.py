@@ -1203,6 +1203,16 @@ def test_norm_over_stretches_by_width(n, t, h):
     assert (room[t] == 7).all()
 
 
+@pytest.mark.parametrize("t,h", [(3, 0), (0, 64)])
+def test_norm_over_stretches_of_nothing(t, h):
+    x = torch.randn(2, t, h, device=DEV)
+    res, w = (torch.randn(s, dtype=torch.bfloat16, device=DEV)
+              for s in ((t, h), (h,)))
+    got, new = ops.fused_add_rms_norm(x, res, w, 1e-5)
+    torch.cuda.synchronize()
+    assert got.shape == (t, h) and new is res
+
+
 def test_three_dimensions_of_bf16():
     """Batches of rows and rows of heads are not a product's stretches."""
     torch.manual_seed(34)
