@@ -10,6 +10,7 @@ bool add_norm(c10::optional<torch::Tensor> sum, torch::Tensor out,
               torch::Tensor b, int64_t L, double eps);
 bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L);
+bool norm_in_registers(int64_t rows, int64_t columns);
 void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
                        torch::Tensor residual, torch::Tensor w, double eps);
 void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -91,6 +92,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("add_norm", &add_norm,
         "(Gated) add + LayerNorm with weights or an image's modulation");
   m.def("gated_add", &gated_add, "x + gate * y, a gate per image");
+  m.def("norm_in_registers", &norm_in_registers,
+        "Whether add_sums_rms_norm keeps a row in registers");
   m.def("add_sums_rms_norm", &add_sums_rms_norm,
         "Sum of a product's stretches + residual-add + RMSNorm");
   m.def("layer_norm", &layer_norm, "LayerNorm (bf16)");

@@ -15,6 +15,20 @@ namespace {
 
 constexpr int WIDE = 1024;     // threads to a row that stays in registers
 
+// Whether a row stays in registers. A CU has room for two such rows, and for
+// four of the loop's, whose loads then cover each other: up to one row for each
+// of the 256 CUs registers are never slower, up to two where at least three
+// quarters of the threads have columns. us by the loop and in registers, 4
+// stretches: 256 rows of 256 columns 3.6 and 3.5, 1024 3.8 and 3.6, 4096 6.1
+// and 6.0; 257 of 256 3.6 and 3.9, 300 of 2048 5.2 and 5.3, of 3072 6.1 and
+// 6.0; 512 of 1024 4.8 and 5.0, of 3072 7.7 and 7.6, of 4096 9.2 and 9.1; 513
+// of 4096 9.5 and 10.9, 1024 of 512 4.8 and 7.4. (8 stretches of 257 to 300 rows
+// lose up to 0.9 us by it and gain up to 0.9 from 400 rows on.)
+bool stays_in_registers(int64_t rows, int64_t columns) {
+  return columns <= WIDE * 4 &&
+         (rows <= 256 || (rows <= 512 && columns >= WIDE * 3));
+}
+
 // out[t, :] = x[t, :] / rms(x[t, :]) * w
 // H must be a multiple of 8. One block per token.
 template <int BLOCK>
@@ -140,9 +154,9 @@ __global__ __launch_bounds__(BLOCK) void add_sums_rms_norm_kernel(
 // and all it takes is loaded at once. Bound by the latency of memory, met once
 // instead of three times (sums, the row again, weights): after the product that
 // writes the stretches, us before -> now 1 row of 8 stretches of 4096 4.9 -> 3.4,
-// 16 rows 5.3 -> 3.8; alone, 61 rows of 4 stretches 4.5 -> 4.2, 512 9.8 -> 9.6,
-// 1540 of 2 17.5 -> 17.6. With 8 columns a thread 300 rows of 8192 took 9.3 us
-// instead of 7.7, so longer rows keep the loop.
+// 16 rows 5.3 -> 3.8. With 8 columns a thread 300 rows of 8192 took 9.3 us
+// instead of 7.7, so longer rows keep the loop. stays_in_registers says which
+// others do.
 __global__ __launch_bounds__(WIDE) void add_sums_rms_norm_wide_kernel(
     uint16_t* __restrict__ h, const float* __restrict__ x,
     uint16_t* __restrict__ residual, const uint16_t* __restrict__ w,
@@ -261,7 +275,7 @@ void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
   TORCH_CHECK(H % 8 == 0, "H must be a multiple of 8");
   if (T == 0 || H == 0) return;               // no row, or no column of one
   auto stream = at::hip::getCurrentHIPStream();
-  if (H <= WIDE * 4) {
+  if (stays_in_registers(T, H)) {
     hipLaunchKernelGGL(add_sums_rms_norm_wide_kernel, dim3(T), dim3(WIDE), 0,
                        stream, (uint16_t*)h.data_ptr(), x.data_ptr<float>(),
                        (uint16_t*)residual.data_ptr(),
@@ -274,6 +288,10 @@ void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
                      (uint16_t*)residual.data_ptr(),
                      (const uint16_t*)w.data_ptr(), (float)eps, H,
                      (int)x.size(0));
+}
+
+bool norm_in_registers(int64_t rows, int64_t columns) {
+  return stays_in_registers(rows, columns);
 }
 
 void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,

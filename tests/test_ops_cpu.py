@@ -169,6 +169,15 @@ def test_gemm_bf16_refuses(case, says):
         ops._native().gemm_bf16(out, x, w, b, 0)
 
 
+@pytest.mark.parametrize("rows,columns,stays", [
+    (1, 8, True), (256, 4096, True), (1, 4104, False), (257, 1024, False),
+    (257, 3072, True), (512, 4096, True), (513, 4096, False),
+    (1024, 512, False)])
+def test_norm_in_registers(rows, columns, stays):
+    """Where the loop over a row was measured faster it is taken."""
+    assert ops._native().norm_in_registers(rows, columns) == stays
+
+
 def test_gemm_ring_loads_stay_at_the_start():
     """Descriptors are empty after the last item; a scalar offset is not part
     of their check, so it stays at 0 however many steps follow."""

@@ -1183,9 +1183,10 @@ def test_quantize_rows_bytes(T, K):
 
 @pytest.mark.parametrize("n,t,h", [(1, 1, 8), (3, 5, 64), (9, 2, 1028 * 2),
                                    (8, 1, 4088), (4, 33, 4096), (2, 3, 4104),
-                                   (17, 2, 4096)])
+                                   (17, 2, 4096), (2, 256, 264), (2, 257, 264),
+                                   (3, 512, 3072), (3, 513, 3072)])
 def test_norm_over_stretches_by_width(n, t, h):
-    """Rows that stay in registers, up to 4096 columns, and longer ones."""
+    """Rows that stay in registers, and longer or more of them."""
     torch.manual_seed(n)
     x = torch.randn(n, t, h, device=DEV)
     res = torch.randn(t, h, dtype=torch.bfloat16, device=DEV)
