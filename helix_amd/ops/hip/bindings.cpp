@@ -58,6 +58,8 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, int64_t act, int64_t tile);
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
                              int64_t stretches);
+std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
+    int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus);
 std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps);
 void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    int64_t tile);
@@ -119,6 +121,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_bf16_sums", &gemm_bf16_sums,
         "x @ w^T, stretches of the inner dimension apart", py::arg("x"),
         py::arg("w"), py::arg("tile"), py::arg("stretches") = 0);
+  m.def("gemm_bf16_plan", &gemm_bf16_plan,
+        "Tile, stretches and us of gemm_bf16, or of its sums, as estimated",
+        py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"),
+        py::arg("sums"), py::arg("cus") = 256);
   m.def("gemm_ring_places", &gemm_ring_places,
         "Where a workgroup of gemm_bf16 loads along the inner dimension");
   m.def("gemm_bf16_glu", &gemm_bf16_glu,

@@ -177,50 +177,29 @@ constexpr int ROWS_TILES[][2] = {HELIX_RING_ROWS(HELIX_TILE)};
 constexpr int SUMS_TILES[][2] = {HELIX_RING_SUMS(HELIX_TILE)};
 #undef HELIX_TILE
 
-void run_ring(const Ring& m, const RingTile& t) {
+void run_ring(const Ring& m, const RingTile& t, int cus) {
 #define HELIX_RUN(MI, NI)                                                    \
-  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, ROWS>(m, 1);
+  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, ROWS>(m, 1, cus);
   HELIX_RING_ROWS(HELIX_RUN)
 #undef HELIX_RUN
   TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni);
 }
 
-void run_ring_sums(const Ring& m, const RingTile& t, int stretches) {
+void run_ring_sums(const Ring& m, const RingTile& t, int stretches, int cus) {
 #define HELIX_RUN(MI, NI)                                                    \
-  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, SUMS>(m, stretches);
+  if (t.mi == MI && t.ni == NI)                                              \
+    return ring_run<MI, NI, SUMS>(m, stretches, cus);
   HELIX_RING_SUMS(HELIX_RUN)
 #undef HELIX_RUN
   TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni, " for sums");
 }
 
-// Tile and stretches, and their time in us with what it takes to read the
-// stretches: their bytes at 4.5 TB/s.
-struct Plan {
-  RingTile tile{};
-  int stretches = 1;
-  double us = 1e30;
-};
-Plan plan_rows(const Ring& m) {
-  Plan best;
-  const int cus = ring_cus();
-  for (const RingTile& t : RING_TILES) {
-    if (!ring_has(ROWS_TILES, t)) continue;
-    const double us = ring_us(m, ROWS, t, 1, cus);
-    if (us < best.us) best = Plan{t, 1, us};
-  }
-  return best;
+RingPlan plan_rows(const Ring& m, int cus) {
+  return ring_plan(m, ROWS, ROWS_TILES, 1, 1, cus);
 }
-Plan plan_sums(const Ring& m, int from) {
-  Plan best;
-  const int steps = m.K / 64, cus = ring_cus();
-  for (const RingTile& t : RING_TILES)
-    for (int n = from; n <= std::min(8, steps) && ring_has(SUMS_TILES, t);
-         ++n) {
-      const double us = ring_us(m, SUMS, t, n, cus) +
-                        4. * n * m.M * m.N / 4.5e6;
-      if (us < best.us) best = Plan{t, n, us};
-    }
-  return best;
+RingPlan plan_sums(const Ring& m, int from, int cus, double below = 1e30) {
+  return ring_plan(m, SUMS, SUMS_TILES, from, std::min(8, m.K / RING_STEP), cus,
+                   below);
 }
 
 // The last stretch may be shorter; there are as many as have something to do.
@@ -230,12 +209,12 @@ int cut(Ring& m, int stretches) {
 }
 
 torch::Tensor sums_of(const torch::Tensor& x, Ring& m, const RingTile& t,
-                      int stretches) {
+                      int stretches, int cus) {
   stretches = cut(m, stretches);
   torch::Tensor sums = torch::empty({stretches, m.M, m.N},
                                     x.options().dtype(torch::kFloat32));
   m.sums = sums.data_ptr<float>();
-  run_ring_sums(m, t, stretches);
+  run_ring_sums(m, t, stretches, cus);
   return sums;
 }
 
@@ -297,19 +276,21 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     }
     r.out = o;
     r.gelu = m.gelu;
+    const int cus = ring_cus();
     if (tile != 0) {
       r.bias = m.bias;
-      return run_ring(r, RingTile{(int)tile / 10, (int)tile % 10, 0});
+      return run_ring(r, RingTile{(int)tile / 10, (int)tile % 10, 0}, cus);
     }
     // A launch that joins stretches takes 3 us more than what it reads (with
     // it, and whole: 300 x 1024 x 4096 13 and 18, 288 x 768 x 3072 9.6 and 12.1;
     // 2304 x 768 x 3072 20 and 18).
-    const Plan rows = plan_rows(r), sums = plan_sums(r, 2);
-    if (rows.us <= sums.us + 4) {
+    const RingPlan rows = plan_rows(r, cus);
+    const RingPlan sums = plan_sums(r, 2, cus, rows.us - 4);
+    if (sums.tile.mi == 0) {
       r.bias = m.bias;
-      return run_ring(r, rows.tile);
+      return run_ring(r, rows.tile, cus);
     }
-    const torch::Tensor t = sums_of(x, r, sums.tile, sums.stretches);
+    const torch::Tensor t = sums_of(x, r, sums.tile, sums.stretches, cus);
     const int64_t MN = (int64_t)m.M * m.N;
     hipLaunchKernelGGL(gemm_join_kernel, dim3((MN + 1023) / 1024), dim3(256),
                        0, at::hip::getCurrentHIPStream(), o,
@@ -341,16 +322,38 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
               m.N >= 4 && m.N % 4 == 0 &&
               (stretches > 0 || tile == 0 || tile == 256 || tile == 128));
   TORCH_CHECK(ring_fits(m, SUMS), "a product of more than the offsets reach");
+  const int cus = ring_cus();
   if (stretches > 0)
     return sums_of(x, m, RingTile{(int)tile / 10, (int)tile % 10, 0},
-                   (int)std::min<int64_t>(stretches, m.K / 64));
+                   (int)std::min<int64_t>(stretches, m.K / 64), cus);
   if (tile == 0) {
-    const Plan p = plan_sums(m, 1);
-    return sums_of(x, m, p.tile, p.stretches);
+    const RingPlan p = plan_sums(m, 1, cus);
+    return sums_of(x, m, p.tile, p.stretches, cus);
   }
   const int side = (int)tile, tiles = cdiv(m.M, side) * cdiv(m.N, side);
   const int most = std::min({(side == 256 ? 256 : 512) / tiles, m.K / 64, 8});
-  return sums_of(x, m, RingTile{side / 32, side / 32, 0}, std::max(1, most));
+  return sums_of(x, m, RingTile{side / 32, side / 32, 0}, std::max(1, most),
+                 cus);
+}
+
+// What gemm_bf16 (sums false) and gemm_bf16_sums do with a product on so many
+// CUs: tile, stretches, us with the reader of those, and how many times were
+// worked out to find them.
+std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
+    int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus) {
+  Ring m{};
+  m.M = M;
+  m.N = N;
+  m.K = K;
+  m.gelu = gelu;
+  TORCH_CHECK(M > 0 && N > 0 && K > 0 && cus > 0 && M <= INT32_MAX &&
+              ring_fits(m, sums ? SUMS : ROWS), "a product of tiles");
+  RingPlan best, p;
+  if (!sums) best = plan_rows(m, cus);
+  p = sums ? plan_sums(m, 1, cus) : plan_sums(m, 2, cus, best.us - 4);
+  p.weighed += best.weighed;
+  if (p.tile.mi == 0) best.weighed = p.weighed, p = best;
+  return {10 * p.tile.mi + p.tile.ni, p.stretches, p.us, p.weighed};
 }
 
 // Places along the inner dimension that a workgroup orders in so many steps, of

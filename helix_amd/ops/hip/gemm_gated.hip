@@ -43,18 +43,13 @@ void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               m.K > 0 && out.size(0) == m.M && out.size(1) == m.N,
               "out is [M, N], w [2 N, K]");
   TORCH_CHECK(ring_fits(m, GATED), "columns are a multiple of 8, and K of 64");
-  RingTile best{(int)tile / 10, (int)tile % 10, 0};
-  if (tile == 0) {
-    const int cus = ring_cus();
-    double least = 1e30;
-    for (const RingTile& t : RING_TILES) {
-      if (!ring_has(GATED_TILES, t)) continue;
-      const double us = ring_us(m, GATED, t, 1, cus);
-      if (us < least) least = us, best = t;
-    }
-  }
+  const int cus = ring_cus();
+  const RingTile best =
+      tile == 0 ? ring_plan(m, GATED, GATED_TILES, 1, 1, cus).tile
+                : RingTile{(int)tile / 10, (int)tile % 10, 0};
 #define HELIX_RUN(MI, NI)                                                    \
-  if (best.mi == MI && best.ni == NI) return ring_run<MI, NI, GATED>(m, 1);
+  if (best.mi == MI && best.ni == NI)                                        \
+    return ring_run<MI, NI, GATED>(m, 1, cus);
   HELIX_RING_GATED(HELIX_RUN)
 #undef HELIX_RUN
   TORCH_CHECK(false, "no tile of ", 32 * best.mi, " x ", 16 * best.ni);

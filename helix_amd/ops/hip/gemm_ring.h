@@ -400,6 +400,14 @@ constexpr RingTile RING_TILES[] = {
     {4, 4, 0.500}, {4, 8, 0.808}, {5, 2, 0.353}, {5, 4, 0.539}, {5, 6, 0.740},
     {5, 8, 1.010}, {6, 4, 0.616}, {6, 6, 0.891}, {7, 8, 1.216}, {8, 8, 1.300}};
 
+// Whether a kernel of that tile is in a list of pairs.
+template <int N>
+bool ring_has(const int (&pairs)[N][2], const RingTile& t) {
+  for (const auto& p : pairs)
+    if (p[0] == t.mi && p[1] == t.ni) return true;
+  return false;
+}
+
 // us of a product by as many workgroups as there are CUs: rounds of items, and
 // what w and sums take to read and write, part of it at the same time. Fitted to
 // 11000 times of 318 sizes (17 to 16000 rows, 768 to 28672 columns, 768 to 14336
@@ -408,30 +416,61 @@ constexpr RingTile RING_TILES[] = {
 // and, with the reader of the stretches, 1.6% as sums (at worst 35%, 48 x 768 x
 // 768). An item takes less while other CUs are idle; few workgroups do not reach
 // the rate of the memory.
-double ring_us(const Ring& m, RingForm form, const RingTile& t, int stretches,
-               int cus) {
+struct RingCost {
+  double busy, fed;
+  double least() const { return 3.3 + std::max(busy, fed); }
+  double us() const {
+    return 3.3 + std::pow(std::pow(busy, 1.8) + std::pow(fed, 1.8), 1 / 1.8);
+  }
+};
+RingCost ring_cost(const Ring& m, RingForm form, const RingTile& t,
+                   int stretches, int cus) {
   const int64_t items = (int64_t)cdiv(m.M, 32 * t.mi) *
                         cdiv(m.N, (form == GATED ? 16 : 32) * t.ni) * stretches;
   const double end = form == SUMS ? 0.073 : form == GATED ? 0.064
                      : m.gelu ? 0.11 : 0.038;
-  const double item = cdiv(m.K / 64, stretches) * t.step +
+  const double item = cdiv(m.K / RING_STEP, stretches) * t.step +
                       end * t.mi * t.ni + 0.27;
   const double rest = (double)(items % cus) / cus;
-  const double busy = item * ((double)(items / cus) +
-                              (rest > 0 ? 0.72 + 0.28 * rest : 0));
-  const double fed =
-      (form == GATED ? 4. : 2.) * m.N * m.K / 9e6 /
-          std::sqrt(std::min(1., (double)items / cus)) +
-      (form == SUMS ? 4. * stretches * m.M * m.N / 4.1e6 : 0.);
-  return 3.3 + std::pow(std::pow(busy, 1.8) + std::pow(fed, 1.8), 1 / 1.8);
+  RingCost c;
+  c.busy = item * ((double)(items / cus) +
+                   (rest > 0 ? 0.72 + 0.28 * rest : 0));
+  c.fed = (form == GATED ? 4. : 2.) * m.N * m.K / 9e6 /
+              std::sqrt(std::min(1., (double)items / cus)) +
+          (form == SUMS ? 4. * stretches * m.M * m.N / 4.1e6 : 0.);
+  return c;
 }
 
-// Whether a kernel of that tile is in a list of pairs.
+// Tile and stretches, and their time with what it takes to read the stretches:
+// their bytes at 4.5 TB/s.
+struct RingPlan {
+  RingTile tile{};
+  int stretches = 1;
+  double us = 1e30;
+  int weighed = 0;                            // times that were worked out
+};
+
+// The tile of a list, and the number of stretches, that take least time, if that
+// is below `below`. A host that is behind pays for every call, so a time is only
+// worked out where its larger part leaves a chance: 4 of 12 times and 1 of 72 at
+// 2304 x 3072 x 1024. All of them took 7 us a product.
 template <int N>
-bool ring_has(const int (&pairs)[N][2], const RingTile& t) {
-  for (const auto& p : pairs)
-    if (p[0] == t.mi && p[1] == t.ni) return true;
-  return false;
+RingPlan ring_plan(const Ring& m, RingForm form, const int (&tiles)[N][2],
+                   int from, int to, int cus, double below = 1e30) {
+  RingPlan best;
+  best.us = below;
+  for (const RingTile& t : RING_TILES) {
+    if (!ring_has(tiles, t)) continue;
+    for (int n = from; n <= to; ++n) {
+      const double reader = form == SUMS ? 4. * n * m.M * m.N / 4.5e6 : 0.;
+      const RingCost c = ring_cost(m, form, t, n, cus);
+      if (c.least() + reader >= best.us) continue;
+      ++best.weighed;
+      const double us = c.us() + reader;
+      if (us < best.us) best.tile = t, best.stretches = n, best.us = us;
+    }
+  }
+  return best;
 }
 
 int ring_cus() {
@@ -450,7 +489,7 @@ bool ring_allow(const void* kernel) {
 }
 
 template <int MI, int NI, RingForm FORM>
-void ring_run(Ring m, int stretches) {
+void ring_run(Ring m, int stretches, int cus) {
   const void* kernel = (const void*)gemm_ring_kernel<MI, NI, FORM>;
   static const bool once = ring_allow(kernel);
   (void)once;
@@ -468,7 +507,7 @@ void ring_run(Ring m, int stretches) {
   m.by_group = Divide(m.group * m.n_tiles);
   void* args[] = {&m};
   const hipError_t err = hipLaunchKernel(
-      kernel, dim3(std::min(ring_cus(), m.total)), dim3(256), args, RING_LDS,
+      kernel, dim3(std::min(cus, m.total)), dim3(256), args, RING_LDS,
       at::hip::getCurrentHIPStream());
   TORCH_CHECK(err == hipSuccess, hipGetErrorString(err));
 }

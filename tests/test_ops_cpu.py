@@ -178,6 +178,18 @@ def test_norm_in_registers(rows, columns, stays):
     assert ops._native().norm_in_registers(rows, columns) == stays
 
 
+@pytest.mark.parametrize("m,n,k,gelu,tile,stretches", [
+    (2304, 3072, 1024, True, 56, 1), (2304, 1024, 1024, False, 52, 1),
+    (300, 768, 3072, False, 22, 4), (8, 6144, 1024, False, 22, 1),
+    (16600, 768, 3072, False, 78, 1)])
+def test_gemm_bf16_plan(m, n, k, gelu, tile, stretches):
+    """The tile and stretches of least estimated time, found without working
+    out the times of all 75 or more: a host pays for them at every call."""
+    plan = ops._native().gemm_bf16_plan(m, n, k, gelu, False)
+    assert plan[:2] == (tile, stretches) and plan[3] <= 8
+    assert ops._native().gemm_bf16_plan(m, n, k, gelu, True)[3] <= 32
+
+
 def test_gemm_ring_loads_stay_at_the_start():
     """Descriptors are empty after the last item; a scalar offset is not part
     of their check, so it stays at 0 however many steps follow."""
