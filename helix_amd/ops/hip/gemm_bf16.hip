@@ -6,8 +6,8 @@
 // [stretch][M][N]).
 //
 // gemm_ring.h has the kernel, its times and what bounds it. Here are its tiles
-// and the rule that chooses one, and the kernel for what it does not take:
-// columns that are no multiple of 8, results off 16-byte boundaries.
+// and the rule that chooses one, and the kernel for what it does not take
+// (matrices beyond its offsets) or not as fast (small_tiles).
 #include "gemm_join.h"
 #include "gemm_ring.h"
 #include <c10/core/DeviceGuard.h>
@@ -172,8 +172,15 @@ void run_tiles(Gemm m, uint16_t* out, const uint16_t* x, const uint16_t* w) {
 #define HELIX_RING_SUMS(TILE)                                                \
   TILE(2, 2) TILE(2, 4) TILE(3, 4) TILE(4, 2) TILE(4, 4) TILE(4, 8)          \
   TILE(5, 4) TILE(5, 8) TILE(8, 8)
+// Any columns, us by the tiles of a workgroup each that had these before -> now:
+// 8192 x 4092 x 4096 391 -> 198, 16600 x 3002 x 1024 198 -> 141, 2304 x 766 x
+// 3072 30 -> 21, 100 x 1020 x 4096 32 -> 10 (8 stretches), 777 x 4095 x 4096 58
+// -> 40.
+#define HELIX_RING_ANY(TILE)                                                 \
+  TILE(2, 2) TILE(4, 2) TILE(4, 4) TILE(5, 4) TILE(4, 8) TILE(8, 8)
 #define HELIX_TILE(MI, NI) {MI, NI},
 constexpr int ROWS_TILES[][2] = {HELIX_RING_ROWS(HELIX_TILE)};
+constexpr int ANY_TILES[][2] = {HELIX_RING_ANY(HELIX_TILE)};
 constexpr int SUMS_TILES[][2] = {HELIX_RING_SUMS(HELIX_TILE)};
 #undef HELIX_TILE
 
@@ -181,6 +188,14 @@ void run_ring(const Ring& m, const RingTile& t, int cus) {
 #define HELIX_RUN(MI, NI)                                                    \
   if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, ROWS>(m, 1, cus);
   HELIX_RING_ROWS(HELIX_RUN)
+#undef HELIX_RUN
+  TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni);
+}
+
+void run_ring_any(const Ring& m, const RingTile& t, int cus) {
+#define HELIX_RUN(MI, NI)                                                    \
+  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, ANY>(m, 1, cus);
+  HELIX_RING_ANY(HELIX_RUN)
 #undef HELIX_RUN
   TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 32 * t.ni);
 }
@@ -196,6 +211,9 @@ void run_ring_sums(const Ring& m, const RingTile& t, int stretches, int cus) {
 
 RingPlan plan_rows(const Ring& m, int cus) {
   return ring_plan(m, ROWS, ROWS_TILES, 1, 1, cus);
+}
+RingPlan plan_any(const Ring& m, int cus) {
+  return ring_plan(m, ANY, ANY_TILES, 1, 1, cus);
 }
 RingPlan plan_sums(const Ring& m, int from, int cus, double below = 1e30) {
   return ring_plan(m, SUMS, SUMS_TILES, from, std::min(8, m.K / RING_STEP), cus,
@@ -216,6 +234,20 @@ torch::Tensor sums_of(const torch::Tensor& x, Ring& m, const RingTile& t,
   m.sums = sums.data_ptr<float>();
   run_ring_sums(m, t, stretches, cus);
   return sums;
+}
+
+// Whether a product whose rows are stored in parts goes by workgroups of a tile
+// each. Their stores overlap with other workgroups' work, which pays where
+// columns go one by one and the inner dimension is short, and there is less of
+// them to start. us by persistent tiles and by these: 16600 x 3001 x 1024 195
+// and 172, 8192 x 765 x 3072 51 and 57, 2304 x 2303 x 768 27 and 27; 64 x 1021 x
+// 1024 8.2 and 6.9, 100 of it 8.3 and 8.4; 20 x 100 x 768 6.4 and 5.7, 100 of it
+// 6.6 and 6.7, 20 x 3002 x 1024 7.6 and 10.3, 200 x 258 x 256 5.4 and 5.1.
+bool small_tiles(const Ring& m) {
+  const int64_t work = (int64_t)m.N * m.K;
+  if (m.unit == 1)
+    return (m.K < 2048 && m.M > 512) || work <= (m.M <= 64 ? 5 << 18 : 5 << 17);
+  return m.unit < 8 && work <= (m.M <= 64 ? 1 << 20 : 1 << 17);
 }
 
 Ring ring_of(const torch::Tensor& x, const torch::Tensor& w) {
@@ -264,13 +296,26 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   }
   TORCH_CHECK(x.is_cuda(), "operands on the GPU");
   const c10::DeviceGuard on(x.device());
+  // Columns that would be stored one by one, for many rows of a long inner
+  // dimension: a copy costs less (4600 x 2304 x 2048 70 us, with it 60).
+  if (tile == 0 && (uintptr_t)out.data_ptr() % 4 != 0 && m.N % 4 == 0 &&
+      m.K >= 2048 && m.M > 512) {
+    torch::Tensor t = torch::empty_like(out);
+    gemm_bf16(t, x, w, bias, act, 0);
+    out.copy_(t);
+    return;
+  }
   // tiles are loaded 16 bytes at a time
   if ((uintptr_t)x.data_ptr() % 16 != 0) x = x.clone();
   if ((uintptr_t)w.data_ptr() % 16 != 0) w = w.clone();
   uint16_t* o = (uint16_t*)out.data_ptr();
   Ring r = ring_of(x, w);
-  if (ring_fits(r, ROWS) && (uintptr_t)o % 16 == 0) {
-    if (m.bias != nullptr && (uintptr_t)m.bias % 16 != 0) {
+  const bool whole = m.N % 8 == 0 && (uintptr_t)o % 16 == 0;
+  r.unit = whole ? 8 : 4;
+  while (r.unit > 1 && (m.N % r.unit != 0 || (uintptr_t)o % (2 * r.unit) != 0))
+    r.unit /= 2;
+  if (ring_fits(r, whole ? ROWS : ANY) && (tile != 0 || !small_tiles(r))) {
+    if (whole && m.bias != nullptr && (uintptr_t)m.bias % 16 != 0) {
       bias = bias->clone();
       m.bias = (const uint16_t*)bias->data_ptr();
     }
@@ -279,16 +324,19 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     const int cus = ring_cus();
     if (tile != 0) {
       r.bias = m.bias;
-      return run_ring(r, RingTile{(int)tile / 10, (int)tile % 10, 0}, cus);
+      const RingTile t{(int)tile / 10, (int)tile % 10, 0};
+      return whole ? run_ring(r, t, cus) : run_ring_any(r, t, cus);
     }
     // A launch that joins stretches takes 3 us more than what it reads (with
     // it, and whole: 300 x 1024 x 4096 13 and 18, 288 x 768 x 3072 9.6 and 12.1;
     // 2304 x 768 x 3072 20 and 18).
-    const RingPlan rows = plan_rows(r, cus);
-    const RingPlan sums = plan_sums(r, 2, cus, rows.us - 4);
+    const RingPlan rows = whole ? plan_rows(r, cus) : plan_any(r, cus);
+    RingPlan sums;
+    if (m.N % 4 == 0) sums = plan_sums(r, 2, cus, rows.us - 4);
     if (sums.tile.mi == 0) {
       r.bias = m.bias;
-      return run_ring(r, rows.tile, cus);
+      return whole ? run_ring(r, rows.tile, cus)
+                   : run_ring_any(r, rows.tile, cus);
     }
     const torch::Tensor t = sums_of(x, r, sums.tile, sums.stretches, cus);
     const int64_t MN = (int64_t)m.M * m.N;
@@ -301,7 +349,9 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(tile == 0, "not a product of tiles");
   const uint16_t* xp = (const uint16_t*)x.data_ptr();
   const uint16_t* wp = (const uint16_t*)w.data_ptr();
-  if (m.M > 64) run_tiles<64, 64, 2, 2>(m, o, xp, wp);
+  if ((int64_t)cdiv(m.M, 128) * cdiv(m.N, 128) >= 256)
+    run_tiles<128, 128, 2, 4>(m, o, xp, wp);
+  else if (m.M > 64) run_tiles<64, 64, 2, 2>(m, o, xp, wp);
   else run_tiles<32, 64, 2, 2>(m, o, xp, wp);
 }
 
@@ -347,10 +397,11 @@ std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
   m.K = K;
   m.gelu = gelu;
   TORCH_CHECK(M > 0 && N > 0 && K > 0 && cus > 0 && M <= INT32_MAX &&
-              ring_fits(m, sums ? SUMS : ROWS), "a product of tiles");
+              ring_fits(m, sums ? SUMS : ANY), "a product of tiles");
   RingPlan best, p;
-  if (!sums) best = plan_rows(m, cus);
-  p = sums ? plan_sums(m, 1, cus) : plan_sums(m, 2, cus, best.us - 4);
+  if (!sums) best = N % 8 == 0 ? plan_rows(m, cus) : plan_any(m, cus);
+  if (N % 4 == 0)
+    p = sums ? plan_sums(m, 1, cus) : plan_sums(m, 2, cus, best.us - 4);
   p.weighed += best.weighed;
   if (p.tile.mi == 0) best.weighed = p.weighed, p = best;
   return {10 * p.tile.mi + p.tile.ni, p.stretches, p.us, p.weighed};

@@ -26,7 +26,12 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(
   if (gelu)
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_f32(v[j]);
-  st_bf16x4(out + i, v);
+  if ((uintptr_t)out % 8 == 0) {
+    st_bf16x4(out + i, v);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[i + j] = f32_to_bf16(v[j]);
+  }
 }
 
 }  // namespace

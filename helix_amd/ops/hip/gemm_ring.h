@@ -45,7 +45,8 @@
 namespace helix {
 namespace {
 
-enum RingForm { ROWS, GATED, SUMS };          // of the result
+// Of the result. ANY: rows of any number of columns, on any boundary.
+enum RingForm { ROWS, GATED, SUMS, ANY };
 
 constexpr int RING_STRIP = 8;                 // tiles of columns, see item_of
 constexpr int RING_LDS = 160 * 1024;
@@ -66,6 +67,7 @@ struct Divide {
 };
 
 // x, w, bias on 16-byte boundaries; out as well and N % 8 == 0, sums N % 4 == 0.
+// ANY: neither bias nor out has to be, and N is whatever it is.
 // GATED: w has N rows of the gate and N of the other factor.
 struct Ring {
   const uint16_t *x, *w, *bias;               // bias may be null
@@ -73,6 +75,7 @@ struct Ring {
   float* sums;                                // [stretch][M][N]
   int M, N, K, m_tiles, n_tiles, tiles, total, stretch, gelu;
   int group, strip_shift;      // tiles of rows; of group * RING_STRIP tiles
+  int unit;                    // ANY: columns that are stored at a time
   Divide by_tiles, by_group;
 };
 
@@ -128,6 +131,32 @@ __device__ __forceinline__ void ring_store(void* base, int bytes, int off,
   __builtin_amdgcn_raw_buffer_store_b128(
       v, __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000), off, 0,
       0);
+}
+
+// The same for the first `left` of 8 columns, `unit` at a time: 4 or 2 of them
+// have to lie on boundaries of their own size.
+__device__ __forceinline__ void ring_store_some(void* base, int bytes, int off,
+                                                u32x4 v, int left, int unit) {
+  constexpr int NONE = 0x7fffff00;
+  const auto to = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
+  if (unit == 4) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      __builtin_amdgcn_raw_buffer_store_b64(
+          u32x2{v[2 * q], v[2 * q + 1]}, to, 4 * q < left ? off + 8 * q : NONE,
+          0, 0);
+  } else if (unit == 2) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      __builtin_amdgcn_raw_buffer_store_b32(
+          v[q], to, 2 * q < left ? off + 4 * q : NONE, 0, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      __builtin_amdgcn_raw_buffer_store_b16(
+          (uint16_t)(v[q / 2] >> (q & 1) * 16), to,
+          q < left ? off + 2 * q : NONE, 0, 0);
+  }
 }
 
 // c (+)= a b in place. As a builtin the sums wander from register to register,
@@ -317,6 +346,16 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
     so = sx;
     sx = sx + 1 == NA ? 0 : sx + 1;
     sw = sw + 1 == NB ? 0 : sw + 1;
+    if constexpr (decltype(first)::value && FORM == ANY) {
+#pragma unroll
+      for (int j = 0; j < NI / 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          bias[j][q] = m.bias == nullptr
+                           ? 0
+                           : m.bias[min(cur.n0 + wc * 16 * NI + j * 32 +
+                                        hi * 8 + q, m.N - 1)];
+    }
     if constexpr (decltype(first)::value && FORM == ROWS) {
       // more operations in flight than the waits count: they wait for more
 #pragma unroll
@@ -367,11 +406,15 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
             else
               v[q] += bf16_to_f32(bias[j][q]);
           }
-          if (FORM == ROWS && m.gelu)
+          if (FORM != GATED && m.gelu)
 #pragma unroll
             for (int q = 0; q < 8; ++q) v[q] = gelu_tanh_f32(v[q]);
-          ring_store(m.out + at, bytes, c < m.N ? o + i * down : NONE,
-                     __builtin_bit_cast(u32x4, pack8(v)));
+          const u32x4 packed = __builtin_bit_cast(u32x4, pack8(v));
+          if constexpr (FORM == ANY)
+            ring_store_some(m.out + at, bytes, o + i * down, packed, m.N - c,
+                            m.unit);
+          else
+            ring_store(m.out + at, bytes, c < m.N ? o + i * down : NONE, packed);
         }
       }
     }
@@ -386,7 +429,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
 // What the kernel's offsets of 32 bits reach.
 bool ring_fits(const Ring& m, RingForm form) {
   return m.K % 64 == 0 && m.K <= 1 << 21 && m.N <= 1 << 20 &&
-         m.N % (form == SUMS ? 4 : 8) == 0 &&
+         (form == ANY || m.N % (form == SUMS ? 4 : 8) == 0) &&
          (form != GATED || (int64_t)4 * m.N * m.K < INT32_MAX);
 }
 

@@ -190,6 +190,14 @@ def test_gemm_bf16_plan(m, n, k, gelu, tile, stretches):
     assert ops._native().gemm_bf16_plan(m, n, k, gelu, True)[3] <= 32
 
 
+def test_gemm_bf16_plan_of_any_columns():
+    """Columns that are no multiple of 8 have large tiles and stretches too."""
+    plan = ops._native().gemm_bf16_plan
+    assert plan(8192, 4092, 4096, False, False)[:2] == (88, 1)
+    assert plan(8192, 3001, 2048, False, False)[0] == 48
+    assert plan(100, 1020, 4096, False, False)[1] > 1
+
+
 def test_gemm_ring_loads_stay_at_the_start():
     """Descriptors are empty after the last item; a scalar offset is not part
     of their check, so it stays at 0 however many steps follow."""

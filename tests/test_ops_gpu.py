@@ -947,7 +947,7 @@ def test_gemm_bf16_sums(m, n, k, tile):
 
 
 def test_gemm_bf16_pair():
-    """256 x 256 tiles by two halves: 192 of them and a long inner dimension."""
+    """Columns in pairs, tiles of 256 x 256 and a long inner dimension."""
     torch.manual_seed(30)
     x = torch.randn(4000, 2112, dtype=torch.bfloat16, device=DEV)
     w = torch.randn(3002, 2112, dtype=torch.bfloat16, device=DEV) / 46
@@ -980,6 +980,32 @@ def test_gemm_ring_tiles(tile, m, n, k, act):
     torch.testing.assert_close(room[:m].double(), want, rtol=2 ** -8,
                                atol=2e-5)
     assert (room[m] == 7).all()
+
+
+@pytest.mark.parametrize("tile", [0, 22, 42, 44, 54, 48, 88])
+@pytest.mark.parametrize("m,n,k,act,off", [
+    (1, 1, 64, 0, 0), (257, 263, 64, 1, 0), (130, 522, 192, 0, 0),
+    (331, 428, 448, 1, 0), (2051, 3083, 128, 0, 0), (900, 266, 1088, 1, 0),
+    (300, 264, 192, 0, 1), (300, 264, 192, 1, 2), (300, 260, 192, 0, 4),
+    (64, 1022, 1024, 0, 0), (65, 1022, 1024, 0, 0), (513, 333, 1984, 0, 0),
+    (520, 264, 2048, 1, 1), (100, 1020, 4096, 1, 1)])
+def test_gemm_bf16_any_columns(tile, m, n, k, act, off):
+    """Columns stored one, two and four at a time, by number and by where the
+    result begins; every tile, either kernel, stretches, the copy of a
+    result."""
+    torch.manual_seed(m + tile)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n + 1, dtype=torch.bfloat16, device=DEV)[1:]
+    room = torch.full((off + m * n + 9,), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = room[off:off + m * n].view(m, n)
+    ops._native().gemm_bf16(out, x, w, b, act, tile)
+    want = x.double() @ w.double().t() + b.double()
+    if act:
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    # fp32 sums of k products and GELU's exponential, the rounding to bf16
+    torch.testing.assert_close(out.double(), want, rtol=2 ** -8, atol=2e-5)
+    assert (room[:off] == 7).all() and (room[off + m * n:] == 7).all()
 
 
 def test_gemm_bf16_where_the_ring_ends():
@@ -1115,7 +1141,7 @@ def test_gemm_sums_tiles(tile, m, n, k, stretches):
 
 @pytest.mark.parametrize("n,act", [(3002, 0), (3002, 1), (3004, 1)])
 def test_gemm_bf16_pair_epilogue(n, act):
-    """Bias and GELU of 256 x 256 tiles, columns stored one and four at a
+    """Bias and GELU of 256 x 256 tiles, columns stored two and four at a
     time."""
     torch.manual_seed(41)
     x = torch.randn(4000, 2112, dtype=torch.bfloat16, device=DEV)
