@@ -503,11 +503,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     The lines are where both were measured equal, with weights from memory. Up
     to 16 rows stream their weights (28672 x 4096: 45 against 65 us), but for
     vocabularies (128256 x 4096: 191 against 189). From 17 rows on tiles
-    (gemm_ring.h) take less than the library's product in most sizes and up to
-    a tenth more in some: 64 rows of 4096 x 14336 29 us and 39, 300 of 6144 x
-    4096 28 and 27, 1540 of 4096 x 4096 48 and 52, 4100 of 4096 x 14336 384 and
-    733, 8192 of 6144 x 4096 269 and 263. Up to 128 rows of a wide matrix, bound
-    by its weights, are the library's (128 of 28672 x 4096: 63 and 55)."""
+    (gemm_ring.h) take less than the library's product in most sizes: 64 rows of
+    4096 x 14336 29 us and 39, 1540 of 4096 x 4096 48 and 52, 4100 of 4096 x
+    14336 384 and 733. Where they do not, _tiles_pay sends the product back to
+    what took less before. Up to 128 rows of a wide matrix, bound by its
+    weights, are the library's (128 of 28672 x 4096: 63 and 55). The library's
+    time jumps from size to size: beyond 192 rows tiles take up to a tenth more
+    in some (300 of 6144 x 4096 31 and 29, 777 of 20480 x 5120 181 and 167) and
+    a tenth to half less in the others."""
     if (_SKINNY_ENABLED and x.is_cuda and x.dtype == torch.bfloat16
             and x.dim() == 2
             and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= _SKINNY_MAX_M
@@ -515,16 +518,49 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
             and x.is_contiguous() and w.is_contiguous()):
         return gemm_skinny_bf16(x, w, bias)
     if _rows_fit(x, w, ROWS_ANY) and _bias_fits(bias, w):
-        M, N = x.shape[0], w.shape[0]
-        if N <= 65536 if M <= 16 else \
-                _ring_fits(*w.shape) and (N <= 8192 or M > ROWS_MAX_M):
+        M, (N, K) = x.shape[0], w.shape
+        tiles = M > 16 and _ring_fits(N, K) and _tiles_pay(M, N, K)
+        if tiles or (N <= 65536 if M <= 16 else
+                     M <= 64 and K >= 2 * N and N <= 8192):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-            if M <= 16:
-                _native().gemm_rows(out, x, w, bias, None, None)
-            else:
+            if tiles:
                 _native().gemm_bf16(out, x, w, bias, 0)
+            else:
+                _native().gemm_rows(out, x, w, bias, None, None)
             return out
     return torch.nn.functional.linear(x, w, bias)
+
+
+def _tiles_pay(M: int, N: int, K: int) -> bool:
+    """Whether more than 16 rows go by tiles of 64 x 64 and more rather than by
+    the library's smaller ones or, up to 64 rows of a deep matrix, as streamed
+    weights. us by tiles and by the other:
+    - wide matrices are bound by their weights (128 of 28672 x 4096 63 and 55);
+    - few columns, so that few CUs read the weights: 33 of 768 x 16384 14.6 and
+      13.2 (streamed), of 1024 x 16384 15.3 and 14.4;
+    - up to 128 tiles of a few dozen steps, which end before they have hidden
+      their first loads: 64 of 2048 x 2048 10.1 and 9.4, 192 of 1024 x 2048 10.0
+      and 8.9, 512 of 1024 x 1280 8.3 and 8.0 (577 of it 8.3 and 10.5; 128 of
+      2560 x 2048 10.2 and 12.3, 24 of 1536 x 2048 7.6 and 8.7, 65 of 512 x 3072
+      7.9 and 10.0);
+    - the like of a dozen steps, 100 of 768 x 768 6.1 and 5.3, 32 of 1024 x 1024
+      6.7 and 5.7 (193 of 768 x 768 6.1 and 7.2, 33 of 1280 x 1024 6.8 and 8.6);
+    - rows 16 KB apart, which lie on the same channels: 32 of 8192 x 8192 38 and
+      31, 100 of it 42 and 39, 24 of 7168 x 8192 35 and 28 (48 of it 34 and 33)."""
+    if N > 8192:
+        return M > ROWS_MAX_M
+    if N <= 1024 and K >= 2048 and K >= 2 * N and M <= (
+            64 if K >= 12288 else 48):
+        return False
+    tiles = -(-M // 64) * -(-N // 64)
+    if 1024 < K <= 3072 and N * K <= 8 << 20 and tiles <= 128:
+        return (K >= 2048 and tiles <= (16 if K > 2048 else 12)
+                or N > 2048 and M % 128 == 0 or N <= 2048 <= K and M <= 24)
+    if 512 < K <= 1024:
+        return not (M <= 192 and N * K <= 11 << 16 and (N > 256 or K > 768)
+                    or M <= 32 and N <= 1280)
+    return not (K % 8192 == 0 and K < 2 * N and
+                (M <= 32 and N >= 6144 or M < 128 and N == 8192))
 
 
 def _rows_many(N: int, K: int) -> bool:

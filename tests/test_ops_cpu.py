@@ -283,6 +283,23 @@ def test_few_rows_where_they_pay():
                 glu(32, 28672, 5120) or glu(64, 57344, 8192))
 
 
+@pytest.mark.parametrize("M,N,K,pay", [
+    (128, 28672, 4096, False), (129, 28672, 4096, True),
+    (48, 768, 4096, False), (64, 768, 4096, True), (64, 768, 16384, False),
+    (256, 2048, 2048, False), (257, 2048, 2048, True),
+    (128, 2560, 2048, True), (127, 2560, 2048, False), (24, 1536, 2048, True),
+    (512, 1024, 1280, False), (577, 1024, 1280, True), (128, 512, 3072, True),
+    (129, 512, 3072, False), (192, 768, 768, False), (193, 768, 768, True),
+    (100, 256, 768, True), (100, 256, 1024, False), (32, 1024, 1024, False),
+    (33, 1280, 1024, True), (100, 512, 512, True), (300, 6144, 4096, True),
+    (127, 8192, 8192, False), (128, 8192, 8192, True), (32, 7168, 8192, False),
+    (48, 7168, 8192, True), (32, 8192, 28672, True)])
+def test_tiles_pay(M, N, K, pay):
+    """Where tiles were measured slower than what products took before them,
+    that is taken."""
+    assert ops._tiles_pay(M, N, K) == pay
+
+
 @pytest.mark.parametrize("case,says", [
     ("type", "rows are bf16"), ("out", "rows are bf16"),
     ("keys", "a boundary more"), ("host", "on one GPU")])

@@ -1078,7 +1078,8 @@ def test_projections_by_rows(m):
     """Every form of a projection on either side of the lines between streamed
     weights, tiles and the library."""
     torch.manual_seed(52)
-    for n, k in ((1024, 4096), (512, 256), (26624, 2048)):
+    for n, k in ((1024, 4096), (512, 256), (26624, 2048), (1024, 2048),
+                 (768, 768)):
         x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
         w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
         b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
