@@ -59,7 +59,10 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
                              int64_t stretches);
 std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
-    int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus);
+    int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus,
+    double below);
+std::tuple<int64_t, int64_t> gemm_bf16_glu_plan(int64_t M, int64_t N, int64_t K,
+                                                int64_t cus);
 std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps);
 void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    int64_t tile);
@@ -124,7 +127,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_bf16_plan", &gemm_bf16_plan,
         "Tile, stretches and us of gemm_bf16, or of its sums, as estimated",
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"),
-        py::arg("sums"), py::arg("cus") = 256);
+        py::arg("sums"), py::arg("cus") = 256, py::arg("below") = 1e30);
+  m.def("gemm_bf16_glu_plan", &gemm_bf16_glu_plan,
+        "What gemm_bf16_glu does with a product of w [2 N, K], as estimated: "
+        "its tile, or tile and stretches of sums", py::arg("M"), py::arg("N"),
+        py::arg("K"), py::arg("cus") = 256);
   m.def("gemm_ring_places", &gemm_ring_places,
         "Where a workgroup of gemm_bf16 loads along the inner dimension");
   m.def("gemm_bf16_glu", &gemm_bf16_glu,

@@ -388,9 +388,10 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
 
 // What gemm_bf16 (sums false) and gemm_bf16_sums do with a product on so many
 // CUs: tile, stretches, us with the reader of those, and how many times were
-// worked out to find them.
+// worked out to find them. Tile 0: no sums take less than `below`.
 std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
-    int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus) {
+    int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus,
+    double below) {
   Ring m{};
   m.M = M;
   m.N = N;
@@ -401,9 +402,9 @@ std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
   RingPlan best, p;
   if (!sums) best = N % 8 == 0 ? plan_rows(m, cus) : plan_any(m, cus);
   if (N % 4 == 0)
-    p = sums ? plan_sums(m, 1, cus) : plan_sums(m, 2, cus, best.us - 4);
+    p = sums ? plan_sums(m, 1, cus, below) : plan_sums(m, 2, cus, best.us - 4);
   p.weighed += best.weighed;
-  if (p.tile.mi == 0) best.weighed = p.weighed, p = best;
+  if (!sums && p.tile.mi == 0) best.weighed = p.weighed, p = best;
   return {10 * p.tile.mi + p.tile.ni, p.stretches, p.us, p.weighed};
 }
 

@@ -190,6 +190,15 @@ def test_gemm_bf16_plan(m, n, k, gelu, tile, stretches):
     assert ops._native().gemm_bf16_plan(m, n, k, gelu, True)[3] <= 32
 
 
+@pytest.mark.parametrize("m,n,k,stretches", [
+    (80, 1024, 8192, 8), (512, 512, 16384, 8), (33, 2048, 7168, 8),
+    (100, 2048, 14336, 4), (1540, 14336, 4096, 0), (128, 14336, 4096, 0)])
+def test_gemm_gated_plan(m, n, k, stretches):
+    """Gate and other factor in stretches where one launch, which has none,
+    leaves CUs idle."""
+    assert ops._native().gemm_bf16_glu_plan(m, n, k)[1] == stretches
+
+
 def test_gemm_bf16_plan_of_any_columns():
     """Columns that are no multiple of 8 have large tiles and stretches too."""
     plan = ops._native().gemm_bf16_plan

@@ -1059,6 +1059,25 @@ def test_gemm_gated_tiles(tile, m, n, k):
     assert (room[m] == 7).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 8, 4096), (80, 1024, 8192),
+                                   (129, 520, 4160), (65, 2056, 14336)])
+def test_gemm_gated_stretches(m, n, k):
+    """Both halves in stretches that a second launch adds up: rows and columns
+    that do not fill its workgroups."""
+    torch.manual_seed(54)
+    assert ops._native().gemm_bf16_glu_plan(m, n, k)[1] > 1
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(2 * n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    room = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_bf16_glu(room[:m], x, w)
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    # fp32 sums of k products and the exponential, the rounding to bf16
+    torch.testing.assert_close(
+        room[:m].double(), torch.nn.functional.silu(g) * u, rtol=2 ** -8,
+        atol=5e-5)
+    assert (room[m] == 7).all()
+
+
 def test_gemm_gated_refuses():
     x, w, out = (torch.zeros(s, dtype=torch.bfloat16, device=DEV)
                  for s in ((70, 128), (48, 128), (70, 24)))
