@@ -563,17 +563,6 @@ def _tiles_pay(M: int, N: int, K: int) -> bool:
                 (M <= 32 and N >= 6144 or M < 128 and N == 8192))
 
 
-def _rows_many(N: int, K: int) -> bool:
-    """Whether 65 to 128 rows stream their weights: matrices of some 2^24
-    values, neither wide, for which x is read too often, nor small, which the
-    library's tiles fill the chip with at a launch's cost. us at 128 rows,
-    streamed and joined, and the library's: 4096 x 8192 28 and 44, 2048 x 8192
-    20.5 and 21.8, 1024 x 14336 21 and 26, 4096 x 4096 20 and 25; 6144 x 2048 22
-    and 18, 1024 x 8192 17.5 and 15.4, 2048 x 2048 17 and 9, 14336 x 4096 65
-    and 51."""
-    return N <= 8192 and N * K >= 13 << 20
-
-
 def _ring_fits(N: int, K: int, gated: bool = False) -> bool:
     """Whether the offsets of gemm_ring.h reach a matrix [N, K]."""
     if gated:                     # both halves lie behind one descriptor
@@ -583,28 +572,25 @@ def _ring_fits(N: int, K: int, gated: bool = False) -> bool:
 
 def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T for a reader that adds up stretches of the inner dimension
-    (fused_add_rms_norm, rope_qkv_cache): [stretches, M, N] fp32 for a few
-    rows, else [M, N] in x's type. Up to 16 rows stream their weights, from 17
-    rows on tiles are faster (us, streamed and by tiles: 17 rows of 6144 x 4096
-    12 and 12, 61 rows 16.4 and 13.1; 61 of 4096 x 14336 29.4 and 24.0, 128 34.5
-    and 28.2). Wide matrices fill the chip without stretches, whose sums are
-    more bytes than they save. From 129 rows on see _sums_tile."""
-    if _rows_fit(x, w) and w.shape[0] <= 8192:
-        if x.shape[0] > 16 and _ring_fits(*w.shape):
+    (fused_add_rms_norm, rope_qkv_cache): [stretches, M, N] fp32 for up to 128
+    rows and up to 8192 columns, and for more rows where _sums_pay; else [M, N]
+    in x's type. Wide matrices fill the chip without stretches, whose sums are
+    more bytes than they save."""
+    M = x.shape[0]
+    if _rows_fit(x, w, SUMS_MAX_M) and w.shape[0] <= 8192:
+        tiles = x.dtype == torch.bfloat16 and _ring_fits(*w.shape)
+        if M <= ROWS_MAX_M and (not tiles or _sums_streamed(M, *w.shape)):
+            return _native().gemm_rows_sums(x, w, None, None)
+        if tiles and (M <= ROWS_MAX_M or _sums_pay(M, *w.shape)):
             return _native().gemm_bf16_sums(x, w, 0)
-        return _native().gemm_rows_sums(x, w, None, None)
-    if x.dim() == 2 and _sums_tile(*x.shape, w.shape[0]) and \
-            _rows_fit(x, w, SUMS_MAX_M) and _ring_fits(*w.shape):
-        return _native().gemm_bf16_sums(x, w, 0)
     return linear(x, w)
 
 
 def linear_sums_or_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear_sums where stretches are the faster form for its reader, rows
-    [M, N] elsewhere: 65 to 128 rows of a small or wide matrix (with the norm,
-    us at 128 rows of 2048 x 2048: 20.9 and 11.8)."""
-    if x.dim() == 2 and 64 < x.shape[0] <= ROWS_MAX_M \
-            and not _rows_many(*w.shape):
+    [M, N] elsewhere."""
+    if x.dim() == 2 and x.shape[0] > 64 and _rows_fit(x, w, ROWS_MAX_M) \
+            and not _sums_pay(x.shape[0], *w.shape):
         return linear(x, w)
     return linear_sums(x, w)
 
@@ -612,35 +598,46 @@ def linear_sums_or_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 SUMS_MAX_M = 2048
 
 
+def _sums_streamed(M: int, N: int, K: int) -> bool:
+    """Whether stretches of a few rows come from streamed weights rather than
+    from tiles (us with the norm that reads them, streamed and by tiles): up to
+    16 rows; small products, which tiles start later (33 of 1024 x 768 7.4 and
+    8.2, 48 of 2048 x 2048 10.1 and 10.5; 17 of 3072 x 1536 10.2 and 9.8, 64 of
+    1024 x 1024 8.9 and 8.5); deep ones of few columns (48 of 1024 x 16384 16.4
+    and 17.7, of 1024 x 8192 12.3 and 11.4) and rows 16 KB apart (33 of 8192 x
+    8192 38.4 and 42.6)."""
+    if M <= 16:
+        return True
+    if N * K <= 4 << 20 and K <= 2560:
+        return M <= (64 if K < 1024 else 48)
+    if N <= 1024 and K >= 12288:
+        return M <= 64
+    return K % 8192 == 0 and K < 2 * N and (
+        M <= 24 and N >= 7168 or M <= 64 and N == 8192)
+
+
 @functools.lru_cache(maxsize=4096)
-def _sums_tile(M: int, K: int, N: int) -> int:
-    """Side of the tiles by which M > 128 rows gain from stretches, 0 where rows
-    are as fast; the tile itself is then chosen by time (gemm_bf16.hip).
-    Stretches pay where a product has too few tiles to fill the chip: at least
-    two to a tile, and work for four fifths of it (256 workgroups of 256 x 256,
-    512 of 128 x 128), and where the estimate in us, with the norm that reads
-    the result (launches, steps of 64, sums written and read), is a tenth below
-    that of a product that fills it (a launch, steps, 1.3 PFLOP/s, weights at 6
-    TB/s). With the reading of the result, as rows and in stretches: 200 rows of
-    4096 x 14336 49 and 32, 512 80 and 65, 1540 160 and 150; 512 of 6144 x 4096,
-    left as rows, 33 and 39."""
-    if not 128 < M <= SUMS_MAX_M or N > 8192:
-        return 0
-    steps = K // 64
-    library = 4 + 0.116 * steps + M * N * K / 650e6 + N * K / 3e6
-    best, tile = 1.1 * library, 0
-    for side, room, fixed, written in ((128, 512, 15.5, 59e6),
-                                       (256, 256, 12.4, 6.5e6)):
-        tiles = -(-M // side) * -(-N // side)
-        per = -(-steps // max(1, min(room // tiles, steps, 8)))
-        n = -(-steps // per)
-        if n < 2 or tiles * n < 0.8 * room:
-            continue
-        step = 1.55 if side == 256 else max(0.28, 0.6 * tiles * n / 256)
-        ours = fixed + per * step + n * M * N * 8 / written
-        if ours < best:
-            best, tile = ours, side
-    return tile
+def _sums_pay(M: int, N: int, K: int) -> bool:
+    """Whether more than 64 rows gain from stretches: by the estimates that
+    choose their tiles (gemm_ring.h), with what a reader reads of either form. Half
+    a microsecond is left to rows, and a fifth of them where they do not go by
+    tiles. us with the norm that reads them, as rows and in stretches: 65 of 2048
+    x 2048 11.8 and 10.4, 129 of 4096 x 4096 21.5 and 21.0, 200 of it 22.0 and
+    20.7, 400 of it 28.2 and 30.3; 129 of 6144 x 4096 26.4 and 23.9; 200 of 4096
+    x 14336 47 and 44, 1540 182 and 167. Over 3700 sizes of 65 to 8192 rows what
+    it takes is 1.5% slower than the best form of each (100 of 512 x 1280, in
+    stretches, 9.1 for the library's 7.6)."""
+    if not _ring_fits(N, K):
+        return M <= ROWS_MAX_M
+    if M > SUMS_MAX_M or N > 8192:
+        return False
+    plan = _native().gemm_bf16_plan
+    tile, stretches, rows, _ = plan(M, N, K, False, False)
+    if stretches > 1:
+        rows += 4                       # the launch that joins them
+    if not _tiles_pay(M, N, K):
+        rows *= 0.8
+    return plan(M, N, K, False, True)[2] + 0.5 <= rows + 2 * M * N / 4.5e6
 
 
 def _glu_fits(M: int, N: int, K: int) -> bool:

@@ -269,22 +269,35 @@ def test_linear_with_a_vector():
                            torch.nn.functional.linear(z, w))
 
 
-@pytest.mark.parametrize("M,N,K,tile", [
-    (128, 4096, 14336, 0), (130, 4096, 14336, 128), (512, 4096, 14336, 256),
-    (1540, 4096, 14336, 256), (2049, 4096, 14336, 0), (640, 8192, 28672, 0),
-    (2048, 8192, 28672, 0), (200, 1024, 4096, 0), (2048, 1024, 4096, 0),
-    (1024, 4096, 4096, 0), (200, 8200, 32768, 0), (130, 8, 64, 0)])
-def test_sums_tile(M, N, K, tile):
-    """Where the library's product is the faster one it stays: at the ends of
-    the range, where tiles alone fill the chip, where there is little to do."""
-    assert ops._sums_tile(M, K, N) == tile
+@pytest.mark.parametrize("M,N,K,pay", [
+    (128, 4096, 14336, True), (130, 4096, 14336, True),
+    (512, 4096, 14336, True), (1540, 4096, 14336, True),
+    (2049, 4096, 14336, False), (640, 8192, 28672, True),
+    (2048, 8192, 28672, False), (200, 1024, 4096, True),
+    (2048, 1024, 4096, False), (1024, 4096, 4096, False),
+    (200, 8200, 32768, False), (130, 8, 64, False), (65, 2048, 2048, True),
+    (129, 4096, 4096, True), (200, 4096, 4096, True), (400, 4096, 4096, False),
+    (128, 512, 1280, False), (128, 16, (1 << 21) + 256, True),
+    (129, 16, (1 << 21) + 256, False)])
+def test_sums_pay(M, N, K, pay):
+    """Stretches where they are the faster form with their reader: at the ends
+    of the range, where tiles alone fill the chip, where there is little to
+    do, beyond the offsets of tiles."""
+    assert ops._sums_pay(M, N, K) == pay
+
+
+@pytest.mark.parametrize("M,N,K,streamed", [
+    (16, 8192, 28672, True), (17, 8192, 28672, False),
+    (48, 2048, 2048, True), (49, 2048, 2048, False), (64, 4096, 768, True),
+    (65, 4096, 768, False), (17, 3072, 1536, False), (64, 1024, 16384, True),
+    (64, 1024, 8192, False), (24, 7168, 8192, True), (33, 7168, 8192, False),
+    (64, 8192, 8192, True)])
+def test_sums_streamed(M, N, K, streamed):
+    assert ops._sums_streamed(M, N, K) == streamed
 
 
 def test_few_rows_where_they_pay():
-    """The lines between the products of few rows and the library's."""
-    many = ops._rows_many
-    assert many(4096, 4096) and many(1024, 14336) and many(8192, 2048)
-    assert not (many(6144, 2048) or many(1024, 8192) or many(14336, 4096))
+    """The lines between the gated products of few rows and the library's."""
     glu = ops._glu_fits
     assert glu(1, 28672, 4096) and glu(16, 12288, 4096) and glu(64, 64, 1024)
     assert glu(17, 28672, 4096) and glu(64, 26624, 2048)

@@ -916,15 +916,15 @@ def test_gemm_rows_forms(m, n, k):
                                atol=25 * 2 ** -8)
 
 
-@pytest.mark.parametrize("m", [64, 65, 128, 129])
+@pytest.mark.parametrize("m", [48, 49, 64, 65, 128, 129])
 def test_linear_sums_or_rows(m):
     torch.manual_seed(43)
-    for n, k, many in ((2048, 2048, False), (4096, 4096, True)):
+    for n, k in ((2048, 2048), (4096, 4096), (512, 1280)):
         x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
         w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
         with torch.inference_mode():
             got = ops.linear_sums_or_rows(x, w)
-        assert m > 128 or (got.dim() == 3) == (many or m <= 64)
+        assert (got.dim() == 3) == (m <= 64 or ops._sums_pay(m, n, k))
         if got.dim() == 3:
             got = got.sum(0)
         torch.testing.assert_close(got.double(), x.double() @ w.double().t(),
