@@ -277,7 +277,7 @@ def test_linear_with_a_vector():
     (2048, 1024, 4096, False), (1024, 4096, 4096, False),
     (200, 8200, 32768, False), (130, 8, 64, False), (65, 2048, 2048, True),
     (129, 4096, 4096, True), (200, 4096, 4096, True), (400, 4096, 4096, False),
-    (128, 512, 1280, False), (128, 16, (1 << 21) + 256, True),
+    (300, 512, 1280, False), (128, 16, (1 << 21) + 256, True),
     (129, 16, (1 << 21) + 256, False)])
 def test_sums_pay(M, N, K, pay):
     """Stretches where they are the faster form with their reader: at the ends
