@@ -2,7 +2,8 @@
 
 Replaces the model execution the reference delegates to vLLM containers
 (SURVEY.md §2.8): hand-written HIP kernels for RMSNorm/RoPE/attention/
-activation; plain projection GEMMs via hipBLASLt (torch.linear); paged KV.
+activation and projections (ops.linear; the library's GEMM where it is the
+faster one, vocabularies of few rows among them); paged KV.
 
 Tensor-parallel sharding (RCCL over xGMI) is applied by
 helix_amd.parallel when tp_size > 1: column-parallel QKV/gate_up,
@@ -135,8 +136,9 @@ PRESETS = {
 
 
 class HLinear(nn.Linear):
-    """nn.Linear routed through ops.linear: a few rows run the owned MFMA
-    kernel, prefill-shaped ones stay on hipBLASLt.
+    """nn.Linear routed through ops.linear: owned MFMA kernels, for a few rows
+    by streamed weights, else by tiles; sizes and calls they do not take, or not
+    as fast, stay with torch's.
 
     A plain call returns rows [T, N]. The modules here ask each other for
     other forms (_own says when): "sums" -> what ops.linear_sums_or_rows

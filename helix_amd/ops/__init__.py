@@ -641,15 +641,16 @@ def _sums_pay(M: int, N: int, K: int) -> bool:
 
 
 def _glu_fits(M: int, N: int, K: int) -> bool:
-    """Whether the gated product of a few rows takes no longer than product and
-    activation apart. It is not cut along the inner dimension, so it needs
-    columns enough to fill the chip, or few chunks. us apart and at once, with
-    weights from memory: one row of 28672 x 4096 66 and 50, 10240 x 4096 28 and
-    29, 4096 x 4096 18 and 27, 16384 x 1024 12.3 and 10.2. From 17 rows on x is read by
-    every workgroup, and the library's product is the faster one but for inner
-    dimensions of a power of two: 64 rows of 28672 x 4096 60 and 60, 17 of them
-    62 and 51, 64 of 28672 x 5120 64 and 75, of 57344 x 8192 192 and 218. Widths
-    that the activation alone does not take go here."""
+    """Whether the gated product of up to 64 rows takes no longer in one launch
+    than product and activation apart: up to 32 rows by streamed weights, which
+    are not cut along the inner dimension and so need columns enough to fill the
+    chip, or few chunks; from 33 rows on, of more than 8192 columns, by tiles. us
+    apart and at once, with weights from memory: one row of 28672 x 4096 66 and
+    50, 10240 x 4096 28 and 29, 4096 x 4096 18 and 27, 16384 x 1024 12.3 and 10.2.
+    From 17 rows on x is read by every workgroup, and the library's product is the
+    faster one but for inner dimensions of a power of two: 17 of 28672 x 4096 62
+    and 51, 33 60 and 57, 64 61 and 58; 48 of 37888 x 3584 64 and 69, of 10240 x
+    8192 44 and 53. Widths that the activation alone does not take go here."""
     if K <= 1024 or N % 16 != 0:
         return True
     if M <= 16:

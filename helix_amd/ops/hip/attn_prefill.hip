@@ -3,7 +3,7 @@
 // Replaces the prefill attention the reference delegates to vLLM. Bound by
 // instruction issue and, at long contexts, by power: a wave takes 1876 cycles a
 // tile, its products 1020 and its 200 vector instructions 1050 (one in 5), and
-// the clock is at 1.75 GHz (on zeros 1 x 8192 takes 451 us instead of 568). LDS
+// the clock is at 1.75 GHz (on zeros 1 x 8192 takes 403 us instead of 562). LDS
 // is busy for a quarter. A third wave on a SIMD (tiles of 32 keys), the next
 // scores computed beside the exponentials and two halves of waves a phase apart
 // change nothing or cost.
@@ -380,7 +380,7 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
   auto stream = at::hip::getCurrentHIPStream();
 #define LAUNCH(DH, C)                                                        \
   hipLaunchKernelGGL((attn_prefill_kernel<DH, C>), grid, dim3(NT),           \
-                     4 * KT * DH * 2, stream, (uint16_t*)out.data_ptr(),                      \
+                     4 * KT * DH * 2, stream, (uint16_t*)out.data_ptr(),      \
                      (const uint16_t*)q.data_ptr(),                          \
                      (const uint16_t*)k.data_ptr(),                          \
                      (const uint16_t*)v.data_ptr(), m)

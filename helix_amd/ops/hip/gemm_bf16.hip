@@ -356,9 +356,8 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 }
 
 // Sums [stretches, M, N] for a reader that adds them up, those that take least
-// time with it. tile 128 (256): as many stretches of squares of that side as
-// there are workgroups for, up to 512 (256) and 8. stretches: that many, by the
-// tile of 32 * (tile / 10) rows and 32 * (tile % 10) columns.
+// time with it. stretches: that many, by the tile of 32 * (tile / 10) rows and
+// 32 * (tile % 10) columns.
 torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
                              int64_t stretches) {
   const c10::DeviceGuard on(x.device());
@@ -369,21 +368,14 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
                 (uintptr_t)t.data_ptr() % 16 == 0);
   Ring m = ring_of(x, w);
   TORCH_CHECK(w.size(1) == m.K && m.K > 0 && m.K % 64 == 0 && m.M >= 1 &&
-              m.N >= 4 && m.N % 4 == 0 &&
-              (stretches > 0 || tile == 0 || tile == 256 || tile == 128));
+              m.N >= 4 && m.N % 4 == 0 && (stretches > 0 || tile == 0));
   TORCH_CHECK(ring_fits(m, SUMS), "a product of more than the offsets reach");
   const int cus = ring_cus();
   if (stretches > 0)
     return sums_of(x, m, RingTile{(int)tile / 10, (int)tile % 10, 0},
                    (int)std::min<int64_t>(stretches, m.K / 64), cus);
-  if (tile == 0) {
-    const RingPlan p = plan_sums(m, 1, cus);
-    return sums_of(x, m, p.tile, p.stretches, cus);
-  }
-  const int side = (int)tile, tiles = cdiv(m.M, side) * cdiv(m.N, side);
-  const int most = std::min({(side == 256 ? 256 : 512) / tiles, m.K / 64, 8});
-  return sums_of(x, m, RingTile{side / 32, side / 32, 0}, std::max(1, most),
-                 cus);
+  const RingPlan p = plan_sums(m, 1, cus);
+  return sums_of(x, m, p.tile, p.stretches, cus);
 }
 
 // What gemm_bf16 (sums false) and gemm_bf16_sums do with a product on so many

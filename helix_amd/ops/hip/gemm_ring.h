@@ -26,13 +26,16 @@
 // us by the kernels that were here before -> now, weights in the caches; the
 // former had 256 x 256 by two halves of waves a phase apart, and 128 x 128 with
 // one barrier and all loads drained each step (tile now; TFLOP/s):
-//   16600 x 2304 x 768    84 -> 59  (160 x 192;  998)
-//   16600 x 768 x 768     32 -> 21  (224 x 256;  919)
-//   16600 x 768 x 3072    74 -> 58  (224 x 256; 1350)
-//   2304 x 3072 x 1024    22 -> 17  (256 x 128;  853)
-//   2304 x 1024 x 1024  12.1 -> 8.9 (160 x 64;   544)
-//   2304 x 1024 x 4096    33 -> 24  (160 x 64;   793)
-//   8192 x 4096 x 4096   221 -> 182 (256 x 256; 1511)
+//   16600 x 2304 x 768    90 -> 60   (224 x 256;  983)
+//   16600 x 768 x 768     34 -> 23   (224 x 256;  840)
+//   16600 x 3072 x 768   113 -> 74   (224 x 256; 1056)
+//   16600 x 768 x 3072    80 -> 62   (224 x 256; 1254)
+//   2304 x 3072 x 1024    23 -> 19   (160 x 192;  756)
+//   2304 x 4096 x 1024    32 -> 21   (160 x 256;  901)
+//   2304 x 1024 x 1024  12.5 -> 10.1 (160 x 64;   477)
+//   2304 x 1024 x 4096    34 -> 26   (160 x 64;   749)
+//   8192 x 4096 x 4096   225 -> 189  (256 x 256; 1456)
+//   8192 x 8192 x 8192   879 -> 696  (256 x 256; 1581)
 // Steps of 32 and 3 to 5 buffers of them, reads of LDS early in a half, loads
 // closer together gave nothing or cost.
 #pragma once
@@ -52,8 +55,9 @@ constexpr int RING_STRIP = 8;                 // tiles of columns, see item_of
 constexpr int RING_LDS = 160 * 1024;
 constexpr int RING_STEP = 64;                 // of the inner dimension
 
-// Quotients of a fixed number below 2^31: d <= 2^shift, mul the rounded up rest
-// of 2^(32 + shift) / d above 2^32.
+// Quotients of a fixed number below 2^31, by the method of Granlund and
+// Montgomery (Division by invariant integers using multiplication): d <=
+// 2^shift, mul the rounded up rest of 2^(32 + shift) / d above 2^32.
 struct Divide {
   uint32_t mul, shift;
   Divide() = default;

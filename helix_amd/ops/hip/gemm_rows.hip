@@ -7,9 +7,10 @@
 // lies at p ^ r % 16, so operands leave LDS without bank conflicts.
 //
 // Narrow matrices leave CUs idle, so the inner dimension is cut into stretches
-// until there are about as many workgroups as Shape wants (cut). Their sums (fp32, [stretch][M][N])
-// are added by whatever reads the result (norm, rotation), in order, or by a
-// launch of their own; nothing is added with atomics.
+// until there are about as many workgroups as Shape wants (cut). Their sums
+// (fp32, [stretch][M][N]) are added by whatever reads the result (norm,
+// rotation), in order, or by a launch of their own; nothing is added with
+// atomics.
 //
 // Gated feed-forward: a wave has 16 columns of the gate and the same 16 of the
 // other half and writes silu(gate) * up; neither half goes to memory.
@@ -20,17 +21,17 @@
 //   M 16   12.4 (15.7)   8.9 (15.6)   45.4 (65.1)   25.2 (27.3)
 //   M 32   15.2 (16.3)  10.4 (13.9)   51.8 (54.2)   27.8 (33.8)
 //   M 64   17.6 (18.0)  12.2 (15.2)   55.4 (52.3)   31.9 (41.9)
-// From 65 rows on a wave has 32 columns, so that x is read from LDS half as
-// often, chunks are half as long and 256 workgroups are enough; matrices as
-// wide as 28672 are the library's there (52, here 66 us):
+// Tiles (gemm_ring.h) have taken over bf16 from 17 rows on, but for the stretches
+// of small products and of deep ones with few columns. From 65 rows on a wave has
+// 32 columns, so that x is read from LDS half as often, chunks are half as long
+// and 256 workgroups are enough:
 //   M 128  20.0 (24.6)  15.5 (24.7)                   34.6 (73.9)
-// Adding them up in a launch, with bias and GELU, takes 2.5 to 3 us more; so do
-// the encoder's and the image model's products, with which by tiles in brackets
-// 8 rows of 6144 x 1024 take 7.6 (14.1) and 33 of 768 x 3072 7.3 (25.1). The gated product
-// replaces a launch of 4.5 us as well. Reading 28672 x 4096 at 44.5 us is 5.3
-// TB/s. Eight waves a workgroup, chunks half or twice as long, and for up to
-// 64 rows 32 columns a wave and 256 or 768 workgroups were each slower on most
-// of these.
+// Adding them up in a launch, with bias and GELU, takes 2.5 to 3 us more; up to
+// 64 rows of small deep matrices of the encoder and the image model do so (8 of
+// 768 x 3072 7.9, by tiles 8.9). The gated product replaces a launch of 4.5 us as
+// well. Reading 28672 x 4096 at 44.5 us is 5.3 TB/s. Eight waves a workgroup,
+// chunks half or twice as long, and for up to 64 rows 32 columns a wave and 256
+// or 768 workgroups were each slower on most of these.
 //
 // e4m3 (weights with a scale per column, x with one per row) runs the scaled
 // 16x16x128 instruction with unity scales; the scales meet the fp32 sums of

@@ -314,10 +314,12 @@ def test_gemm_bf16(m, n, k):
 
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("m,n,k", [
-    (1, 8, 64), (33, 70, 128), (64, 62, 64),          # tiles of 32 x 64
-    (65, 64, 192), (130, 1030, 64),                   # of 64
-    (2049, 2050, 64),                                 # of 128
-    (3585, 3500, 64),                                 # of 128 as well
+    (1, 8, 64), (65, 64, 192),                        # persistent
+    (33, 70, 128), (64, 62, 64),                      # of 32 x 64 each
+    (130, 1030, 64),                                  # of 64 x 64
+    (2049, 2050, 64),                                 # persistent, in pairs
+    (3585, 3500, 64),                                 # in fours
+    (2049, 2051, 64),                                 # of 128 x 128
 ])
 def test_gemm_bf16_tiles(m, n, k, act):
     """Remainders of rows and columns for every tile, one step and several,
@@ -868,10 +870,11 @@ def test_gemm_rows(m, n, k):
         got = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
         ops._native().gemm_rows(got, dx, dw, db, None, None)
         torch.testing.assert_close(got.float().cpu(), want + b.float(), **tol)
-        sums = ops.linear_sums(dx, dw)
-        assert sums.dim() == 3
-        torch.testing.assert_close(sums.sum(0).cpu(), want, rtol=1e-5,
-                                   atol=2e-5)
+        for sums in (ops.linear_sums(dx, dw),
+                     ops._native().gemm_rows_sums(dx, dw, None, None)):
+            assert sums.dim() == 3
+            torch.testing.assert_close(sums.sum(0).cpu(), want, rtol=1e-5,
+                                       atol=2e-5)
         res = torch.randn(m, n, dtype=torch.bfloat16)
         nw = torch.randn(n, dtype=torch.bfloat16)
         dres = res.to(DEV)
@@ -931,22 +934,23 @@ def test_linear_sums_or_rows(m):
                                    rtol=2 ** -8, atol=2e-5)
 
 
-@pytest.mark.parametrize("tile", [128, 256])
-@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (257, 260, 192),
-                                   (130, 516, 4160), (700, 1024, 1088)])
-def test_gemm_bf16_sums(m, n, k, tile):
+@pytest.mark.parametrize("tile", [44, 88])
+@pytest.mark.parametrize("m,n,k,stretches", [
+    (1, 8, 64, 1), (257, 260, 192, 3), (130, 516, 4160, 8),
+    (700, 1024, 1088, 8)])
+def test_gemm_bf16_sums(m, n, k, stretches, tile):
     """One step, fewer steps than buffers, stretches of unequal length,
     remainders of rows and columns."""
     torch.manual_seed(29)
     x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
     w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
-    sums = ops._native().gemm_bf16_sums(x, w, tile)
+    sums = ops._native().gemm_bf16_sums(x, w, tile, stretches)
     want = x.double() @ w.double().t()
     torch.testing.assert_close(sums.double().sum(0), want, rtol=1e-5,
                                atol=2e-5)       # fp32 sums of k products
 
 
-def test_gemm_bf16_pair():
+def test_gemm_bf16_columns_in_pairs():
     """Columns in pairs, tiles of 256 x 256 and a long inner dimension."""
     torch.manual_seed(30)
     x = torch.randn(4000, 2112, dtype=torch.bfloat16, device=DEV)
@@ -1160,7 +1164,7 @@ def test_gemm_sums_tiles(tile, m, n, k, stretches):
 
 
 @pytest.mark.parametrize("n,act", [(3002, 0), (3002, 1), (3004, 1)])
-def test_gemm_bf16_pair_epilogue(n, act):
+def test_gemm_bf16_epilogue_of_any_columns(n, act):
     """Bias and GELU of 256 x 256 tiles, columns stored two and four at a
     time."""
     torch.manual_seed(41)
