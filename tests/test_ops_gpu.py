@@ -1082,6 +1082,32 @@ def test_gemm_gated_stretches(m, n, k):
     assert (room[m] == 7).all()
 
 
+def test_projections_replayed():
+    """Workspaces of products in stretches belong to the graph that captured
+    them: replays give what eager calls give, with other work between them."""
+    torch.manual_seed(55)
+    x = torch.randn(80, 4096, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(1024, 4096, dtype=torch.bfloat16, device=DEV) / 64
+
+    def run():
+        return (ops.gated_linear(x, w), ops.linear(x, w), ops.linear_sums(x, w),
+                ops.gemm_bf16(x, w[:1020], None, 1))
+
+    with torch.inference_mode():
+        run()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = run()
+        for _ in range(3):
+            x.copy_(torch.randn_like(x))
+            want = run()
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
+
+
 def test_gemm_gated_refuses():
     x, w, out = (torch.zeros(s, dtype=torch.bfloat16, device=DEV)
                  for s in ((70, 128), (48, 128), (70, 24)))
