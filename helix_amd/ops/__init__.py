@@ -501,12 +501,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     gradients, other types and strides, odd dims) via torch/hipBLASLt.
 
     The lines are where both were measured equal, with weights from memory. Up
-    to 16 rows stream their weights (28672 x 4096: 45 against 65 us), but for
-    vocabularies (128256 x 4096: 191 against 189). From 17 rows on tiles
+    to 16 rows stream their weights (28672 x 4096: 42 against 60 us), vocabularies
+    and up to 48 rows of wide matrices where _streams_pay. From 17 rows on tiles
     (gemm_ring.h) take less than the library's product in most sizes: 64 rows of
     4096 x 14336 29 us and 39, 1540 of 4096 x 4096 48 and 52, 4100 of 4096 x
     14336 384 and 733. Where they do not, _tiles_pay sends the product back to
-    what took less before. Up to 128 rows of a wide matrix, bound by its
+    what took less before. Up to 128 rows of other wide matrices, bound by their
     weights, are the library's (128 of 28672 x 4096: 63 and 55). The library's
     time jumps from size to size: beyond 192 rows tiles take up to a tenth more
     in some (300 of 6144 x 4096 31 and 29, 777 of 20480 x 5120 181 and 167) and
@@ -520,8 +520,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     if _rows_fit(x, w, ROWS_ANY) and _bias_fits(bias, w):
         M, (N, K) = x.shape[0], w.shape
         tiles = M > 16 and _ring_fits(N, K) and _tiles_pay(M, N, K)
-        if tiles or (N <= 65536 if M <= 16 else
-                     M <= 64 and K >= 2 * N and N <= 8192):
+        if tiles or _streams_pay(M, N, K):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             if tiles:
                 _native().gemm_bf16(out, x, w, bias, 0)
@@ -529,6 +528,21 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
                 _native().gemm_rows(out, x, w, bias, None, None)
             return out
     return torch.nn.functional.linear(x, w, bias)
+
+
+def _streams_pay(M: int, N: int, K: int) -> bool:
+    """Whether up to 64 rows that do not go by tiles stream their weights rather
+    than take the library's product: up to 16 rows of up to 65536 columns, and
+    deep narrow ones. Beyond, of rows 4 or 8 KB apart: workgroups that begin apart
+    (gemm_rows.hip) read these from all channels at once, which the library's do
+    not. us streamed and by the library: 16 rows of 128256 x 4096 175 and 186,
+    of 65536 x 2048 48 and 66, 32 of 32000 x 4096 46 and 63, 48 of it 52 and 64, 32
+    of 28672 x 4096 45 and 54 (64 of it 53 and 53, of 16384 x 4096 35 and 32; 16
+    of 128256 x 8192 373 and 364, 32 of 64000 x 5120 129 and 112, of 62024 x 3584
+    88 and 79)."""
+    if K in (2048, 4096) and (N > 65536 or M > 16 and N >= 24576):
+        return M <= 48
+    return N <= 65536 if M <= 16 else M <= 64 and K >= 2 * N and N <= 8192
 
 
 def _tiles_pay(M: int, N: int, K: int) -> bool:
@@ -660,8 +674,8 @@ def _glu_fits(M: int, N: int, K: int) -> bool:
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T), w = [gate; up]. A few rows: one launch,
-    whose halves stay in registers (45 us at one row of 2 x 14336 x 4096,
-    product and activation apart 68)."""
+    whose halves stay in registers (42 us at one row of 2 x 14336 x 4096,
+    product and activation apart 59)."""
     if _rows_fit(x, w, ROWS_MAX_M_GLU):
         out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                           device=x.device)

@@ -3,8 +3,16 @@
 //
 // Bound by reading w once. A wave streams its columns of w straight into MFMA
 // operands, a chunk of 512 bytes of the inner dimension ahead; x goes to LDS
-// by direct loads, once for the columns of all waves. 16-byte piece p of row r
-// lies at p ^ r % 16, so operands leave LDS without bank conflicts.
+// by direct loads, once for the columns of all waves, and only the rows there
+// are. 16-byte piece p of row r lies at p ^ r % 16, so operands leave LDS without
+// bank conflicts.
+//
+// Where the inner dimension is not cut, groups of columns begin at different
+// chunks and go round: rows of w that are a power of two apart lie on the same
+// channels, and workgroups that started together would all read those (us at 1
+// row of 28672 x 4096 gated 44.9 -> 42.2, of 32000 x 4096 52.1 -> 46.0, of 128256 x
+// 4096 180 -> 172; e4m3 gated 26.1 -> 22.6). Stretches have few chunks, and where
+// to begin takes longer than it saves (6144 x 4096 11.4 -> 11.7).
 //
 // Narrow matrices leave CUs idle, so the inner dimension is cut into stretches
 // until there are about as many workgroups as Shape wants (cut). Their sums
@@ -17,10 +25,10 @@
 //
 // us for N x K = 6144x4096, 4096x4096, 28672x4096, 4096x14336 (the sums left
 // to the reader), library kernel in brackets:
-//   M  1   11.7 (14.4)   8.6 (15.5)   44.5 (63.4)   23.2 (26.6)
-//   M 16   12.4 (15.7)   8.9 (15.6)   45.4 (65.1)   25.2 (27.3)
-//   M 32   15.2 (16.3)  10.4 (13.9)   51.8 (54.2)   27.8 (33.8)
-//   M 64   17.6 (18.0)  12.2 (15.2)   55.4 (52.3)   31.9 (41.9)
+//   M  1   11.2 (14.4)   8.0 (15.5)   42.2 (63.4)   22.1 (26.6)
+//   M 16   12.7 (15.7)   8.6 (15.6)   42.7 (65.1)   23.6 (27.3)
+//   M 32   14.4 (16.3)   9.3 (13.9)   46.8 (54.2)   24.9 (33.8)
+//   M 64   17.6 (18.0)  12.2 (15.2)   54.0 (52.3)   31.9 (41.9)
 // Tiles (gemm_ring.h) have taken over bf16 from 17 rows on, but for the stretches
 // of small products and of deep ones with few columns. From 65 rows on a wave has
 // 32 columns, so that x is read from LDS half as often, chunks are half as long
@@ -29,7 +37,7 @@
 // Adding them up in a launch, with bias and GELU, takes 2.5 to 3 us more; up to
 // 64 rows of small deep matrices of the encoder and the image model do so (8 of
 // 768 x 3072 7.9, by tiles 8.9). The gated product replaces a launch of 4.5 us as
-// well. Reading 28672 x 4096 at 44.5 us is 5.3 TB/s. Eight waves a workgroup,
+// well. Reading 28672 x 4096 at 42.2 us is 5.6 TB/s. Eight waves a workgroup,
 // chunks half or twice as long, and for up to 64 rows 32 columns a wave and 256
 // or 768 workgroups were each slower on most of these.
 //
@@ -70,8 +78,9 @@ __device__ __forceinline__ v8i join(u32x4 a, u32x4 b) {
 }
 
 // 16 MI rows, NW waves of 16 NI columns each, chunks of CB bytes. GLU (NI 2):
-// columns n and N + n are a pair of a wave.
-template <int MI, int NI, int NW, int CB, bool GLU, bool F8>
+// columns n and N + n are a pair of a wave. TURN: one stretch, whose groups of
+// columns begin apart.
+template <int MI, int NI, int NW, int CB, bool GLU, bool F8, bool TURN>
 __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
     uint16_t* __restrict__ out, float* __restrict__ sums,
     const char* __restrict__ x, const char* __restrict__ w, Product m) {
@@ -101,17 +110,26 @@ __global__ __launch_bounds__(NW* WAVE, 2) void gemm_rows_kernel(
     const int e = i * TH + tid, r = e / PR, p = e % PR ^ (r & 15);
     xp[i] = x + min(r, m.M - 1) * m.row + p * 16;
   }
-  auto load_x = [&](int c, int b) {
+  const int from = TURN ? (int)(blockIdx.x % m.chunks) : 0;
+  auto place = [&](int c) {
+    if (TURN) c = c + from < m.chunks ? c + from : c + from - m.chunks;
+    return c;
+  };
+  // rows past the last one stay as LDS was: no row's sums see another's
+  auto load_x = [&](int at, int b) {
+    const int c = place(at);
 #pragma unroll
     for (int i = 0; i < XL; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) uint32_t*)(xp[i] + c * CB),
-          (__attribute__((address_space(3))) uint32_t*)(
-              xl[b] + (i * TH + wid * WAVE) * 16),
-          16, 0, 0);
+      if ((i * TH + tid) / PR < m.M)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) uint32_t*)(xp[i] + c * CB),
+            (__attribute__((address_space(3))) uint32_t*)(
+                xl[b] + (i * TH + wid * WAVE) * 16),
+            16, 0, 0);
   };
   u32x4 wr[2][U][NI];
-  auto load_w = [&](int c, int b) {
+  auto load_w = [&](int at, int b) {
+    const int c = place(at);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -248,11 +266,11 @@ int cut(Product& m, bool join) {
   return cdiv(m.chunks, m.per);
 }
 
-template <bool GLU, bool F8>
+template <bool GLU, bool F8, bool TURN>
 void run_as(uint16_t* out, float* sums, const torch::Tensor& x,
             const torch::Tensor& w, const Product& m, int stretches) {
 #define HELIX_GR(MI, NI, NW, CB)                                             \
-  hipLaunchKernelGGL((gemm_rows_kernel<MI, NI, NW, CB, GLU, F8>),            \
+  hipLaunchKernelGGL((gemm_rows_kernel<MI, NI, NW, CB, GLU, F8, TURN>),      \
                      dim3(m.n_tiles * stretches), dim3(NW * WAVE), 0,        \
                      at::hip::getCurrentHIPStream(), out, sums,              \
                      (const char*)x.data_ptr(), (const char*)w.data_ptr(), m)
@@ -271,8 +289,16 @@ void run_as(uint16_t* out, float* sums, const torch::Tensor& x,
 template <bool GLU>
 void run(uint16_t* out, float* sums, const torch::Tensor& x,
          const torch::Tensor& w, const Product& m, int stretches) {
-  if (m.xs != nullptr) run_as<GLU, true>(out, sums, x, w, m, stretches);
-  else run_as<GLU, false>(out, sums, x, w, m, stretches);
+#define HELIX_AS(F8)                                                         \
+  if (GLU || stretches == 1)                                                 \
+    return run_as<GLU, F8, true>(out, sums, x, w, m, stretches);             \
+  if constexpr (!GLU) run_as<GLU, F8, false>(out, sums, x, w, m, stretches)
+  if (m.xs != nullptr) {
+    HELIX_AS(true);
+  } else {
+    HELIX_AS(false);
+  }
+#undef HELIX_AS
 }
 
 torch::Tensor sums_for(const torch::Tensor& x, const Product& m,

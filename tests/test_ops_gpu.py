@@ -919,6 +919,27 @@ def test_gemm_rows_forms(m, n, k):
                                atol=25 * 2 ** -8)
 
 
+@pytest.mark.parametrize("m", [1, 5, 16, 31, 48, 49, 128])
+@pytest.mark.parametrize("n,k", [(16456, 256), (32776, 768), (24576, 2048),
+                                 (24568, 2048), (65544, 2048)])
+def test_gemm_rows_uncut(m, n, k):
+    """Columns enough for an inner dimension that is not cut, whose groups begin
+    at different chunks, of one chunk and more; rows that are not there; either
+    side of the line to the library."""
+    torch.manual_seed(54)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    want = x.double() @ w.double().t() + b.double()
+    got = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_rows(got, x, w, b, None, None)
+    # fp32 sums of k products, then the rounding to bf16
+    tol = dict(rtol=2 ** -8, atol=2e-5)
+    torch.testing.assert_close(got.double(), want, **tol)
+    with torch.inference_mode():
+        torch.testing.assert_close(ops.linear(x, w, b).double(), want, **tol)
+
+
 @pytest.mark.parametrize("m", [48, 49, 64, 65, 128, 129])
 def test_linear_sums_or_rows(m):
     torch.manual_seed(43)
