@@ -13,8 +13,9 @@ MI355X-first rectified-flow DiT ("flux-lite" architecture class):
   — the same `ops.attn_prefill` the bge/ViT encoders run;
 - DiT blocks with adaLN modulation from (timestep, pooled prompt);
   every projection runs on the hand-written MFMA bf16 GEMM
-  (`ops.gemm_bf16`), norms with their modulation and the gated sum
-  before them on `ops.modulated_norm`;
+  (`ops.gemm_bf16`; the modulations of all blocks in one launch,
+  `ops.gemm_bf16_many`), norms with their modulation and the gated sum
+  before them, of this block or the last, on `ops.modulated_norm`;
 - Euler integration of the rectified-flow ODE (velocity prediction,
   sigma-shifted schedule), deterministic per seed: noise is drawn on a
   CPU generator so CPU and GPU runs of the same seed share a prior.
@@ -34,6 +35,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from helix_amd import ops
+from helix_amd.models.llama import _own
 
 
 @dataclass
@@ -145,11 +147,20 @@ class DiTBlock(nn.Module):
 
     def forward(self, x: torch.Tensor, cond: torch.Tensor,
                 cu: torch.Tensor, L: int) -> torch.Tensor:
+        mod = ops.gemm_bf16(cond, self.mod_w, self.mod_b)
+        return ops.gated_add(*self.open_sum(x, None, None, mod, cu, L), L)
+
+    def open_sum(self, x: torch.Tensor, y: Optional[torch.Tensor],
+                 gate: Optional[torch.Tensor], mod: torch.Tensor,
+                 cu: torch.Tensor, L: int):
+        """The block's result as (x, y, gate) that x + gate y is still to be
+        taken of, for input of that form (y None: x); mod: the modulation of
+        both halves. The sum is left to the norm that reads it (8 images:
+        a launch of 5 us and a pass over the rows)."""
         h = self.cfg.hidden
         T = x.shape[0]
-        sa, ca, ga, sm, cm, gm = ops.gemm_bf16(
-            cond, self.mod_w, self.mod_b).chunk(6, dim=-1)
-        _, n = ops.modulated_norm(x, ca, sa, L, self.cfg.eps)
+        sa, ca, ga, sm, cm, gm = mod.chunk(6, dim=-1)
+        x, n = ops.modulated_norm(x, ca, sa, L, self.cfg.eps, y, gate)
         qkv = ops.gemm_bf16(n, self.qkv_w, self.qkv_b)
         nh = self.cfg.heads
         q, k, v = (t.view(T, nh, self.hd)
@@ -159,7 +170,7 @@ class DiTBlock(nn.Module):
         x, n = ops.modulated_norm(x, cm, sm, L, self.cfg.eps, a, ga)
         m = ops.gemm_bf16(n, self.up_w, self.up_b, act=1)     # fused GELU
         m = ops.gemm_bf16(m, self.down_w, self.down_b)
-        return ops.gated_add(x, m, gm, L)
+        return x, m, gm
 
 
 class DiTModel(nn.Module):
@@ -225,11 +236,19 @@ class DiTModel(nn.Module):
         cond = (cond.float() + tx.float().mean(dim=1)).to(dtype)
         cu = torch.arange(0, (B + 1) * L, L, dtype=torch.int32,
                           device=lat.device)
-        for blk in self.blocks:
-            x = blk(x, cond, cu, L)
-        fm = ops.gemm_bf16(cond, self.fin_mod_w, self.fin_mod_b)
+        y = gate = None
+        if all(_own(blk, DiTBlock) for blk in self.blocks):
+            *mods, fm = ops.gemm_bf16_many(
+                cond, [b.mod_w for b in self.blocks] + [self.fin_mod_w],
+                [b.mod_b for b in self.blocks] + [self.fin_mod_b])
+            for blk, mod in zip(self.blocks, mods):
+                x, y, gate = blk.open_sum(x, y, gate, mod, cu, L)
+        else:
+            for blk in self.blocks:
+                x = blk(x, cond, cu, L)
+            fm = ops.gemm_bf16(cond, self.fin_mod_w, self.fin_mod_b)
         shift, scale = fm.chunk(2, dim=-1)
-        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps)
+        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps, y, gate)
         out = ops.gemm_bf16(n, self.fin_w, self.fin_b)
         patch_rows = out.view(B, L, -1)[:, Tt:, :].reshape(
             B * P, cfg.patch_dim)

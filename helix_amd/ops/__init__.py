@@ -406,6 +406,17 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias=None,
     return ref.gemm_bf16(x, w, bias, act)
 
 
+def gemm_bf16_many(x: torch.Tensor, ws: list, biases: list) -> list:
+    """[x @ w^T + bias] for several matrices: up to 64 rows in one launch, which
+    is bound by reading the matrices and not by starting (8 rows of 12 x 6144 x
+    1024 and 2048 x 1024 91 us as 13 launches, 31 as one)."""
+    if x.is_cuda and x.shape[0] <= 64:
+        out = _native().gemm_rows_many(x, ws, biases)
+        if out:
+            return out
+    return [gemm_bf16(x, w, b) for w, b in zip(ws, biases)]
+
+
 # The earlier kernel for few rows: called directly, or by linear with
 # HELIX_SKINNY_GEMM=1. Llama's projections ask linear_sums and linear_silu_mul
 # first, so that switch compares little of a decode step.

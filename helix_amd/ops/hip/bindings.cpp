@@ -75,6 +75,9 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
                OptT x_scale, OptT w_scale, bool gelu);
 torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
                              OptT w_scale);
+std::vector<torch::Tensor> gemm_rows_many(torch::Tensor x,
+                                          std::vector<torch::Tensor> ws,
+                                          std::vector<torch::Tensor> biases);
 void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    OptT x_scale, OptT w_scale);
 void quantize_rows(torch::Tensor out, torch::Tensor scales, torch::Tensor x);
@@ -144,6 +147,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x_scale"), py::arg("w_scale"), py::arg("gelu") = false);
   m.def("gemm_rows_sums", &gemm_rows_sums,
         "x @ w^T of at most 128 rows, stretches of the inner dimension apart");
+  m.def("gemm_rows_many", &gemm_rows_many,
+        "x @ w^T + bias of at most 64 rows for several w, in one launch");
   m.def("gemm_rows_glu", &gemm_rows_glu,
         "silu(x @ gate^T) * (x @ up^T) of at most 64 rows");
   m.def("quantize_rows", &quantize_rows,

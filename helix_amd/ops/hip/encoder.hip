@@ -24,7 +24,7 @@ constexpr int NT = 256;
 struct Rows {
   const uint16_t *x, *y, *gate, *a, *b;       // y, gate may be null
   uint16_t *sum, *out;                        // sum may be null
-  int64_t mod_stride;          // of an image's row in gate, a and b
+  int64_t gate_stride, mod_stride;      // of an image's row in gate; in a and b
   int T, H, L;                 // rows of an image; 0: a and b are weights
   float eps;
 };
@@ -35,7 +35,7 @@ __global__ __launch_bounds__(NT) void add_norm_kernel(Rows m) {
   const int64_t t = (int64_t)blockIdx.x * (NT / WAVE) + threadIdx.x / WAVE;
   if (t >= m.T) return;
   const int lane = threadIdx.x & (WAVE - 1), nvec = m.H / 8;
-  const int64_t img = m.L > 0 ? t / m.L * m.mod_stride : 0;
+  const int64_t of = m.L > 0 ? t / m.L : 0, img = of * m.mod_stride;
   float v[NV][8], total = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(NT) void add_norm_kernel(Rows m) {
         load_bf16x8(m.y + t * m.H + c, y);
         if (m.gate != nullptr) {
           float g[8];
-          load_bf16x8(m.gate + img + c, g);
+          load_bf16x8(m.gate + of * m.gate_stride + c, g);
 #pragma unroll
           for (int j = 0; j < 8; ++j) y[j] *= g[j];
         }
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(NT) void gated_add_kernel(Rows m, int64_t total) {
   float x[8], y[8], g[8];
   load_bf16x8(m.x + i, x);
   load_bf16x8(m.y + i, y);
-  load_bf16x8(m.gate + t / m.L * m.mod_stride + i % m.H, g);
+  load_bf16x8(m.gate + t / m.L * m.gate_stride + i % m.H, g);
 #pragma unroll
   for (int j = 0; j < 8; ++j) x[j] += g[j] * y[j];
   store_bf16x8(m.out + i, x);
@@ -111,14 +111,14 @@ bool reads(const torch::Tensor& t, const torch::Tensor& x) {
 bool like(const torch::Tensor& t, const torch::Tensor& x) {
   return reads(t, x) && t.is_contiguous() && t.sizes() == x.sizes();
 }
-// A row for every L of x, each as far from the next as m's others.
-bool of_image(const torch::Tensor& t, const torch::Tensor& x, Rows& m,
-              const uint16_t** at) {
+// A row for every L of x, each `stride` from the next (-1: not known yet).
+bool of_image(const torch::Tensor& t, const torch::Tensor& x, const Rows& m,
+              int64_t& stride, const uint16_t** at) {
   if (!reads(t, x) || t.dim() != 2 || t.size(1) != m.H || t.stride(1) != 1 ||
       t.stride(0) % 8 != 0 || m.L <= 0 || t.size(0) * m.L < m.T ||
-      (m.mod_stride != 0 && m.mod_stride != t.stride(0)))
+      (stride >= 0 && stride != t.stride(0)))
     return false;
-  m.mod_stride = t.stride(0);
+  stride = t.stride(0);
   *at = (const uint16_t*)t.data_ptr();
   return true;
 }
@@ -131,6 +131,7 @@ bool rows_of(const torch::Tensor& x, const torch::Tensor& out, int64_t L,
   m.T = x.size(0);
   m.H = x.size(1);
   m.L = L;
+  m.gate_stride = m.mod_stride = -1;
   m.x = (const uint16_t*)x.data_ptr();
   m.out = (uint16_t*)out.data_ptr();
   return true;
@@ -155,8 +156,10 @@ bool add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
     m.sum = (uint16_t*)sum->data_ptr();
   }
   if (L > 0) {
-    if (!of_image(a, x, m, &m.a) || !of_image(b, x, m, &m.b) ||
-        (gate.has_value() && !of_image(*gate, x, m, &m.gate)))
+    if (!of_image(a, x, m, m.mod_stride, &m.a) ||
+        !of_image(b, x, m, m.mod_stride, &m.b) ||
+        (gate.has_value() &&
+         !of_image(*gate, x, m, m.gate_stride, &m.gate)))
       return false;
   } else {
     for (const auto& t : {a, b})
@@ -183,7 +186,8 @@ bool add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
 bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L) {
   Rows m{};
-  if (!rows_of(x, out, L, m) || !like(y, x) || !of_image(gate, x, m, &m.gate))
+  if (!rows_of(x, out, L, m) || !like(y, x) ||
+      !of_image(gate, x, m, m.gate_stride, &m.gate))
     return false;
   m.y = (const uint16_t*)y.data_ptr();
   const int64_t total = (int64_t)m.T * m.H;

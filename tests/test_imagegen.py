@@ -162,3 +162,32 @@ def test_dit_generate_gpu():
     assert a.shape == (2, 3, 32, 32) and a.dtype == torch.uint8
     assert torch.equal(a, b)
     assert int(a.max()) - int(a.min()) > 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("images", [1, 3])
+def test_dit_blocks_apart_gpu(images):
+    """A hook on one block sees its result; the velocity is that of sums taken
+    by the next norm, but for the roundings of those to bf16 (2^-9 of each, over
+    12 blocks)."""
+    from dataclasses import replace
+    from helix_amd.models.dit import DiTModel
+    cfg = replace(DIT_PRESETS["flux-lite"], depth=3, vocab_size=512)
+    torch.manual_seed(5)
+    m = DiTModel(cfg).to(torch.bfloat16).to("cuda")
+    for p in m.parameters():
+        p.data.normal_(0.0, 0.02)
+    args = (torch.randn(images, 4, 32, 32, device="cuda").bfloat16(),
+            torch.full((images,), 0.75, device="cuda"),
+            torch.randint(0, 512, (images, cfg.text_len), device="cuda"))
+    seen = []
+    with torch.inference_mode():
+        whole = m(*args)
+        h = m.blocks[1].register_forward_hook(
+            lambda mod, a, out: seen.append(out))
+        apart = m(*args)
+        h.remove()
+    assert len(seen) == 1 and seen[0].shape == (images * cfg.seq_len,
+                                                cfg.hidden)
+    err = (whole - apart).double().norm() / apart.double().norm()
+    assert err < 12 * 2 ** -9

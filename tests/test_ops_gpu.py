@@ -135,6 +135,72 @@ def test_add_norm_forms(form):
                                **tol)
 
 
+def test_add_norm_strides():
+    """A gate from another matrix than scale and shift, and modulations that
+    are one row for all images."""
+    torch.manual_seed(55)
+    T, H, L = 12, 64, 3
+    x, y = torch.randn(2, T, H, dtype=torch.bfloat16, device=DEV)
+    gate = torch.randn(4, 6 * H, dtype=torch.bfloat16, device=DEV)[:, H:2 * H]
+    scale, shift = torch.randn(4, 2 * H, dtype=torch.bfloat16,
+                               device=DEV).chunk(2, -1)
+    one = torch.randn(1, H, dtype=torch.bfloat16, device=DEV).expand(4, H)
+    norm = lambda t: torch.nn.functional.layer_norm(t, (H,), eps=1e-6)  # noqa: E731
+    for gate, scale, shift in ((gate, scale, shift), (gate, one, shift),
+                               (one, one, one)):
+        g, c, s = (t.repeat_interleave(L, 0)[:T].double()
+                   for t in (gate, scale, shift))
+        total = x.double() + g * y.double()
+        if shift.stride(0) == scale.stride(0):
+            tol = dict(rtol=2 ** -8, atol=2e-5)
+        else:                     # as separate steps, see test_add_norm_forms
+            tol = dict(rtol=2 ** -7, atol=20 * 2 ** -8)
+        new, got = ops.modulated_norm(x, scale, shift, L, 1e-6, y, gate)
+        torch.testing.assert_close(new.double(), total, **tol)
+        torch.testing.assert_close(got.double(), norm(total) * (1 + c) + s,
+                                   **tol)
+
+
+@pytest.mark.parametrize("m", [1, 17, 64])
+@pytest.mark.parametrize("k,ns", [(256, [64]), (1024, [384, 128, 384]),
+                                  (512, [192, 64 * 50]), (768, [3072] * 49)])
+def test_gemm_bf16_many(m, k, ns):
+    """One matrix, some of several widths, more parts than a launch takes."""
+    torch.manual_seed(56)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    ws = [torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+          for n in ns]
+    bs = [torch.randn(n, dtype=torch.bfloat16, device=DEV) for n in ns]
+    got = ops._native().gemm_rows_many(x, ws, bs)
+    assert len(got) == len(ns)
+    for o, w, b in zip(got, ws, bs):
+        # fp32 sums of k products, then the rounding to bf16
+        torch.testing.assert_close(
+            o.double(), x.double() @ w.double().t() + b.double(),
+            rtol=2 ** -8, atol=2e-5)
+
+
+def test_gemm_bf16_many_forms():
+    """What the one launch does not read goes as a product each."""
+    torch.manual_seed(57)
+    x = torch.randn(65, 256, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(128, 256, dtype=torch.bfloat16, device=DEV) / 16
+    b = torch.randn(128, dtype=torch.bfloat16, device=DEV)
+    off = (torch.randn(128 * 256 + 1, dtype=torch.bfloat16, device=DEV)
+           / 16)[1:].view(128, 256)
+    few = x[:3]
+    many = ops._native().gemm_rows_many
+    for a, ws, bs in ((x, [w], [b]), (few[:, :128].contiguous(),
+                                      [w[:, :128].contiguous()], [b]),
+                      (few, [w, w[:40]], [b, b[:40]]), (few, [off], [b]),
+                      (few, [], []), (few[:0], [w], [b])):
+        assert many(a, ws, bs) == []
+        for o, v, c in zip(ops.gemm_bf16_many(a, ws, bs), ws, bs):
+            torch.testing.assert_close(
+                o.double(), a.double() @ v.double().t() + c.double(),
+                rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("hq,hk,d", [(32, 8, 128), (12, 12, 64)])
 def test_rope(hq, hk, d):
     torch.manual_seed(3)
