@@ -517,8 +517,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     (gemm_ring.h) take less than the library's product in most sizes: 64 rows of
     4096 x 14336 29 us and 39, 1540 of 4096 x 4096 48 and 52, 4100 of 4096 x
     14336 384 and 733. Where they do not, _tiles_pay sends the product back to
-    what took less before. Up to 128 rows of other wide matrices, bound by their
-    weights, are the library's (128 of 28672 x 4096: 63 and 55). The library's
+    what took less before. Up to 128 rows of most wide matrices, bound by their
+    weights, are the library's (128 of 12288 x 4096: 33 and 32). The library's
     time jumps from size to size: beyond 192 rows tiles take up to a tenth more
     in some (300 of 6144 x 4096 31 and 29, 777 of 20480 x 5120 181 and 167) and
     a tenth to half less in the others."""
@@ -530,7 +530,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
         return gemm_skinny_bf16(x, w, bias)
     if _rows_fit(x, w, ROWS_ANY) and _bias_fits(bias, w):
         M, (N, K) = x.shape[0], w.shape
-        tiles = M > 16 and _ring_fits(N, K) and _tiles_pay(M, N, K)
+        tiles = M > 16 and _ring_fits(N, K) and (
+            _tiles_pay(M, N, K) or _tiles_apart_pay(M, N, K))
         if tiles or _streams_pay(M, N, K):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             if tiles:
@@ -550,17 +551,31 @@ def _streams_pay(M: int, N: int, K: int) -> bool:
     of 65536 x 2048 48 and 66, 32 of 32000 x 4096 46 and 63, 48 of it 52 and 64, 32
     of 28672 x 4096 45 and 54 (64 of it 53 and 53, of 16384 x 4096 35 and 32; 16
     of 128256 x 8192 373 and 364, 32 of 64000 x 5120 129 and 112, of 62024 x 3584
-    88 and 79)."""
+    88 and 79). From 33 rows on tiles of 4096 are faster still."""
     if K in (2048, 4096) and (N > 65536 or M > 16 and N >= 24576):
         return M <= 48
     return N <= 65536 if M <= 16 else M <= 64 and K >= 2 * N and N <= 8192
+
+
+def _tiles_apart_pay(M: int, N: int, K: int) -> bool:
+    """Whether 17 to 128 rows of a wide matrix go by tiles all the same: of rows a
+    multiple of 8 KB apart, whose tiles begin apart (ring_turn in gemm_ring.h), and
+    columns that fill the chip. us by tiles and by the library: 33 of 28672 x 4096
+    41 and 53, 128 51 and 56, 61 of 128256 x 4096 183 and 209, 128 191 and 234, of
+    57344 x 8192 164 and 184 (80 of 37888 x 4096 80 and 72, 33 of 28672 x 8192 110
+    and 100; 64 of 20480 x 4096 47 and 41, of 12288 x 4096 26 and 25). Up to 32 rows
+    while there is a tile of 128 columns a CU, else streamed (24 of 28672 x 4096 40
+    and streamed 47, of 100352 x 4096 197 and 153)."""
+    return (K % 4096 == 0 and N >= 24576 and 16 < M <= ROWS_MAX_M
+            and (M > 32 or K == 4096 and N <= 32768))
 
 
 def _tiles_pay(M: int, N: int, K: int) -> bool:
     """Whether more than 16 rows go by tiles of 64 x 64 and more rather than by
     the library's smaller ones or, up to 64 rows of a deep matrix, as streamed
     weights. us by tiles and by the other:
-    - wide matrices are bound by their weights (128 of 28672 x 4096 63 and 55);
+    - wide matrices are bound by their weights (128 of 12288 x 4096 33 and 32),
+      see _tiles_apart_pay;
     - few columns, so that few CUs read the weights: 33 of 768 x 16384 14.6 and
       13.2 (streamed), of 1024 x 16384 15.3 and 14.4;
     - up to 128 tiles of a few dozen steps, which end before they have hidden

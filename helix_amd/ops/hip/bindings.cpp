@@ -63,7 +63,8 @@ std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
     double below);
 std::tuple<int64_t, int64_t> gemm_bf16_glu_plan(int64_t M, int64_t N, int64_t K,
                                                 int64_t cus);
-std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps);
+std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps,
+                                      int64_t turn);
 void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    int64_t tile);
 void gemm_skinny_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -136,7 +137,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "its tile, or tile and stretches of sums", py::arg("M"), py::arg("N"),
         py::arg("K"), py::arg("cus") = 256);
   m.def("gemm_ring_places", &gemm_ring_places,
-        "Where a workgroup of gemm_bf16 loads along the inner dimension");
+        "Where a workgroup of gemm_bf16 loads along the inner dimension",
+        py::arg("k"), py::arg("steps"), py::arg("turn") = 0);
   m.def("gemm_bf16_glu", &gemm_bf16_glu,
         "silu(x @ w[:N]^T) * (x @ w[N:]^T) of more than a few rows",
         py::arg("out"), py::arg("x"), py::arg("w"), py::arg("tile") = 0);

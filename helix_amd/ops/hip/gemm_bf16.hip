@@ -401,13 +401,15 @@ std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
 }
 
 // Places along the inner dimension that a workgroup orders in so many steps, of
-// items from k[2 i] to k[2 i + 1] and after the last of them.
-std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps) {
+// items from k[2 i] to k[2 i + 1], `turn` after their start, and after the last
+// of them.
+std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps,
+                                      int64_t turn) {
   RingAt at;
   size_t item = 0;
   auto next = [&] {
     at.close();
-    if (item + 1 < k.size()) at.open((int)k[item], (int)k[item + 1]);
+    if (item + 1 < k.size()) at.open((int)k[item], (int)k[item + 1], (int)turn);
     item += 2;
   };
   next();

@@ -22,6 +22,8 @@
 //    waits for the stores (before, 5.5 us of 1 x 768 steps of 256 x 256 were
 //    first loads, 7.5 the stores). Rows of w are put into LDS in such an order
 //    that a lane has 8 neighbouring columns: 16-byte stores.
+//  - With one tile of rows nobody else reads a tile's w, and tiles of columns
+//    may begin at different places of the inner dimension (ring_turn).
 //
 // us by the kernels that were here before -> now, weights in the caches; the
 // former had 256 x 256 by two halves of waves a phase apart, and 128 x 128 with
@@ -80,6 +82,7 @@ struct Ring {
   int M, N, K, m_tiles, n_tiles, tiles, total, stretch, gelu;
   int group, strip_shift;      // tiles of rows; of group * RING_STRIP tiles
   int unit;                    // ANY: columns that are stored at a time
+  int turn;                    // see ring_turn
   Divide by_tiles, by_group;
 };
 
@@ -87,22 +90,29 @@ struct RingItem {
   int m0, n0, split, k0, k1;
 };
 
-// Where loads are along the inner dimension. After the last item they stay at
-// its start: descriptors are empty by then, and what lies past the end of one is
-// checked by a load's own offset, not by this scalar one on top of it.
+// Where loads are along the inner dimension: from k0 + turn to k1, then from k0.
+// After the last item they stay at its start: descriptors are empty by then, and
+// what lies past the end of one is checked by a load's own offset, not by this
+// scalar one on top of it.
 struct RingAt {
-  int k, end, ahead;
-  __host__ __device__ __forceinline__ void open(int k0, int k1) {
-    k = k0;
+  int k, from, end, left, ahead;
+  __host__ __device__ __forceinline__ void open(int k0, int k1, int turn) {
+    k = k0 + turn;
+    from = k0;
     end = k1;
+    left = k1 - k0;
     ahead = RING_STEP;
   }
   __host__ __device__ __forceinline__ void close() {
-    k = ahead = 0;
-    end = 0x7fffffff;
+    k = from = ahead = 0;
+    end = left = 0x7fffffff;
   }
   // Whether all of the item is ordered.
-  __host__ __device__ __forceinline__ bool step() { return (k += ahead) >= end; }
+  __host__ __device__ __forceinline__ bool step() {
+    k += ahead;
+    if (k >= end) k = from;
+    return (left -= ahead) <= 0;
+  }
 };
 
 // A thread's 16-byte pieces of ROWS_ rows of 64, as offsets in bytes.
@@ -265,7 +275,8 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
     x_bytes = min(BM, m.M - p.m0) * m.K * 2;
     w_bytes = FORM == GATED ? (2 * m.N - p.n0) * m.K * 2
                             : min(BN, m.N - p.n0) * m.K * 2;
-    order.open(p.k0, p.k1);
+    order.open(p.k0, p.k1,
+               (p.n0 / OUT_N & m.turn) * RING_STEP);
   };
   RingItem cur, next;
   if (!item_of(0, cur)) return;
@@ -520,6 +531,21 @@ RingPlan ring_plan(const Ring& m, RingForm form, const int (&tiles)[N][2],
   return best;
 }
 
+// Mask of a tile of columns' number: at which step of an inner dimension that is
+// not cut it begins. Rows of w a multiple of 8 KB apart lie on the same channels, and
+// workgroups that start together would all read those; but where several tiles of
+// rows share a tile of w, or x does not stay in an XCD's L2, going through it in
+// step is worth more. us in step and apart, weights from memory: 24 rows of 2 x
+// 14336 x 4096 51.7 and 44.4, 61 51.3 and 45.7, 96 of 28672 x 4096 54 and 44, 128 of
+// 128256 x 4096 247 and 189, 61 of 2 x 28672 x 8192 167 and 161; 512 of 2 x 14336 x
+// 4096 97 and 111; 37 of 2 x 8192 x 2048 19.1 and 19.8, 64 of 2 x 10240 x 5120 52
+// and 54. In stretches 61 of 4096 x 14336 24.9 and 25.7.
+int ring_turn(const Ring& m) {
+  constexpr int UNIT = 4096;
+  return m.m_tiles == 1 && m.K % UNIT == 0 && m.stretch >= m.K
+             ? UNIT / RING_STEP - 1 : 0;
+}
+
 int ring_cus() {
   int device, cus;
   TORCH_CHECK(hipGetDevice(&device) == hipSuccess &&
@@ -547,6 +573,7 @@ void ring_run(Ring m, int stretches, int cus) {
   m.tiles = m.m_tiles * m.n_tiles;
   m.total = (int)total;
   m.by_tiles = Divide(m.tiles);
+  m.turn = ring_turn(m);
   // eight blocks of 4 tiles of rows where w is too large for the memory-side
   // cache beside the rest
   m.group = (int64_t)m.N * (FORM == GATED ? 2 : 1) * m.K >= 64 << 20 ? 32 : 16;

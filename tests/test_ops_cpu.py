@@ -214,6 +214,9 @@ def test_gemm_ring_loads_stay_at_the_start():
     assert places([0, 128, 64, 192], 9) == [0, 64, 64, 128, 0, 0, 0, 0, 0]
     assert places([0, 64], 40) == [0] * 40
     assert places([], 3) == [0, 0, 0]
+    # begun elsewhere, an item goes round to its start
+    assert places([0, 256], 6, 128) == [128, 192, 0, 64, 0, 0]
+    assert places([0, 128, 0, 128], 6, 64) == [64, 0, 64, 0, 0, 0]
 
 
 @pytest.mark.parametrize("case,says", [
@@ -320,6 +323,23 @@ def test_tiles_pay(M, N, K, pay):
     """Where tiles were measured slower than what products took before them,
     that is taken."""
     assert ops._tiles_pay(M, N, K) == pay
+
+
+@pytest.mark.parametrize("M,N,K,way", [
+    (16, 128256, 4096, "stream"), (16, 65537, 3584, "library"),
+    (16, 65536, 3584, "stream"), (24, 28672, 4096, "tiles"),
+    (24, 32776, 4096, "stream"), (32, 128256, 2048, "stream"),
+    (33, 128256, 4096, "tiles"), (48, 24576, 2048, "stream"),
+    (49, 24576, 2048, "library"), (48, 24568, 2048, "library"),
+    (128, 24576, 8192, "tiles"), (32, 28672, 8192, "library"),
+    (128, 24568, 4096, "library"), (129, 24568, 4096, "tiles"),
+    (61, 37888, 3584, "library")])
+def test_wide_products(M, N, K, way):
+    """Streamed, by tiles or by the library, on either side of the lines."""
+    tiles = M > 16 and (ops._tiles_pay(M, N, K)
+                        or ops._tiles_apart_pay(M, N, K))
+    assert way == ("tiles" if tiles else
+                   "stream" if ops._streams_pay(M, N, K) else "library")
 
 
 @pytest.mark.parametrize("case,says", [

@@ -987,7 +987,8 @@ def test_gemm_rows_forms(m, n, k):
 
 @pytest.mark.parametrize("m", [1, 5, 16, 31, 48, 49, 128])
 @pytest.mark.parametrize("n,k", [(16456, 256), (32776, 768), (24576, 2048),
-                                 (24568, 2048), (65544, 2048)])
+                                 (24568, 2048), (65544, 2048),
+                                 (32776, 4096)])
 def test_gemm_rows_uncut(m, n, k):
     """Columns enough for an inner dimension that is not cut, whose groups begin
     at different chunks, of one chunk and more; rows that are not there; either
@@ -1004,6 +1005,35 @@ def test_gemm_rows_uncut(m, n, k):
     torch.testing.assert_close(got.double(), want, **tol)
     with torch.inference_mode():
         torch.testing.assert_close(ops.linear(x, w, b).double(), want, **tol)
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    (1, 8, 4096, 22), (40, 1030, 4096, 22), (64, 4168, 8192, 22),
+    (65, 8328, 4096, 34), (128, 8328, 4096, 48), (129, 2056, 4096, 58),
+    (33, 24576, 4096, 0), (17, 32776, 4096, 0), (128, 24584, 8192, 0)])
+def test_gemm_bf16_begins_apart(m, n, k, tile):
+    """One tile of rows and an inner dimension of whole 4096: fewer tiles of
+    columns than steps and more, several rounds of them."""
+    torch.manual_seed(58)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    want = x.double() @ w.double().t()
+    got = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_bf16(got, x, w, b, 0, tile)
+    # fp32 sums of k products, then the rounding to bf16
+    tol = dict(rtol=2 ** -8, atol=2e-5)
+    torch.testing.assert_close(got.double(), want + b.double(), **tol)
+    with torch.inference_mode():
+        torch.testing.assert_close(ops.linear(x, w, b).double(),
+                                   want + b.double(), **tol)
+    if n % 16 == 0:
+        gated = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+        ops._native().gemm_bf16_glu(gated, x, w, 88 if m > 128 else 48)
+        g, u = want.chunk(2, -1)
+        torch.testing.assert_close(
+            gated.double(), torch.nn.functional.silu(g) * u, rtol=2 ** -8,
+            atol=5e-5)
 
 
 @pytest.mark.parametrize("m", [48, 49, 64, 65, 128, 129])
