@@ -31,10 +31,6 @@ namespace {
 constexpr int GATED_TILES[][2] = {HELIX_RING_GATED(HELIX_TILE)};
 #undef HELIX_TILE
 
-__device__ __forceinline__ float gated(float g, float u) {
-  return g / (1.f + __expf(-g)) * u;
-}
-
 // out[M,N] of sums [stretches][M][2 N], 4 columns a thread. Bound by their
 // bytes and a launch.
 __global__ __launch_bounds__(256) void glu_join_kernel(
@@ -53,7 +49,7 @@ __global__ __launch_bounds__(256) void glu_join_kernel(
   }
   float v[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = gated(g[j], u[j]);
+  for (int j = 0; j < 4; ++j) v[j] = silu_f32(g[j]) * u[j];
   st_bf16x4(out + (int64_t)row * N + c, v);
 }
 
