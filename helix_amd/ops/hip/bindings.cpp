@@ -61,6 +61,10 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
 std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
     int64_t M, int64_t N, int64_t K, bool gelu, bool sums, int64_t cus,
     double below);
+std::tuple<bool, int64_t, int64_t, int64_t, double> gemm_bf16_cut(
+    int64_t M, int64_t N, int64_t K, bool gelu, int64_t cus);
+std::tuple<bool, int64_t, int64_t, int64_t, double> gemm_bf16_glu_cut(
+    int64_t M, int64_t N, int64_t K, int64_t cus);
 std::tuple<int64_t, int64_t> gemm_bf16_glu_plan(int64_t M, int64_t N, int64_t K,
                                                 int64_t cus);
 std::vector<int64_t> gemm_ring_places(std::vector<int64_t> k, int64_t steps,
@@ -132,6 +136,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "Tile, stretches and us of gemm_bf16, or of its sums, as estimated",
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"),
         py::arg("sums"), py::arg("cus") = 256, py::arg("below") = 1e30);
+  m.def("gemm_bf16_cut", &gemm_bf16_cut,
+        "Whether gemm_bf16 cuts a product by rows, behind how many rows or "
+        "columns (0: not at all), tiles of both parts, us", py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("gelu"), py::arg("cus") = 256);
+  m.def("gemm_bf16_glu_cut", &gemm_bf16_glu_cut,
+        "gemm_bf16_cut of gemm_bf16_glu", py::arg("M"), py::arg("N"),
+        py::arg("K"), py::arg("cus") = 256);
   m.def("gemm_bf16_glu_plan", &gemm_bf16_glu_plan,
         "What gemm_bf16_glu does with a product of w [2 N, K], as estimated: "
         "its tile, or tile and stretches of sums", py::arg("M"), py::arg("N"),

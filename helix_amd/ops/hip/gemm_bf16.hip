@@ -220,6 +220,10 @@ RingPlan plan_sums(const Ring& m, int from, int cus, double below = 1e30) {
                    below);
 }
 
+RingCut cut_rows(const Ring& m, int cus, double us) {
+  return ring_cut(m, ROWS, ROWS_TILES, cus, ring_cut_below(us, 0.03));
+}
+
 // The last stretch may be shorter; there are as many as have something to do.
 int cut(Ring& m, int stretches) {
   m.stretch = cdiv(m.K / 64, stretches) * 64;
@@ -335,6 +339,14 @@ void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     if (m.N % 4 == 0) sums = plan_sums(r, 2, cus, rows.us - 4);
     if (sums.tile.mi == 0) {
       r.bias = m.bias;
+      const RingCut cut = whole ? cut_rows(r, cus, rows.us) : RingCut{};
+      if (cut.at > 0) {
+        Ring a, b;
+        r.ld = r.N;
+        ring_parts(r, cut, a, b);
+        run_ring(a, cut.first, cus);
+        return run_ring(b, cut.rest, cus);
+      }
       return whole ? run_ring(r, rows.tile, cus)
                    : run_ring_any(r, rows.tile, cus);
     }
@@ -398,6 +410,22 @@ std::tuple<int64_t, int64_t, double, int64_t> gemm_bf16_plan(
   p.weighed += best.weighed;
   if (!sums && p.tile.mi == 0) best.weighed = p.weighed, p = best;
   return {10 * p.tile.mi + p.tile.ni, p.stretches, p.us, p.weighed};
+}
+
+// How gemm_bf16 cuts a product that is not in stretches: whether by rows, behind
+// how many (0: not at all), the tiles of both parts and us.
+std::tuple<bool, int64_t, int64_t, int64_t, double> gemm_bf16_cut(
+    int64_t M, int64_t N, int64_t K, bool gelu, int64_t cus) {
+  Ring m{};
+  m.M = M;
+  m.N = N;
+  m.K = K;
+  m.gelu = gelu;
+  TORCH_CHECK(M > 0 && N > 0 && K > 0 && cus > 0 && M <= INT32_MAX &&
+              ring_fits(m, ROWS), "a product of tiles");
+  const RingCut c = cut_rows(m, cus, plan_rows(m, cus).us);
+  return {c.rows, c.at, 10 * c.first.mi + c.first.ni, 10 * c.rest.mi + c.rest.ni,
+          c.us};
 }
 
 // Places along the inner dimension that a workgroup orders in so many steps, of

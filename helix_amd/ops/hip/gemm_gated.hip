@@ -57,20 +57,49 @@ __global__ __launch_bounds__(256) void glu_join_kernel(
 // launch takes 4 us beside what it reads.
 struct GluPlan {
   int tile, stretches;
+  double us;
 };
 GluPlan plan_glu(const Ring& m, int cus) {
   const RingPlan one = ring_plan(m, GATED, GATED_TILES, 1, 1, cus);
-  GluPlan p{10 * one.tile.mi + one.tile.ni, 0};
+  GluPlan p{10 * one.tile.mi + one.tile.ni, 0, one.us};
   if (m.N <= 1 << 19 && (int64_t)m.M * (m.N / 4) < 1 << 30) {
     const auto two = gemm_bf16_plan(m.M, 2 * m.N, m.K, false, true, cus,
                                     one.us - 4);
     if (std::get<0>(two) != 0)
-      p = GluPlan{(int)std::get<0>(two), (int)std::get<1>(two)};
+      p = GluPlan{(int)std::get<0>(two), (int)std::get<1>(two),
+                  std::get<2>(two)};
   }
   return p;
 }
 
+RingCut cut_glu(const Ring& m, int cus, double us) {
+  return ring_cut(m, GATED, GATED_TILES, cus, ring_cut_below(us, 0.02));
+}
+
+void run_glu(const Ring& m, const RingTile& t, int cus) {
+#define HELIX_RUN(MI, NI)                                                    \
+  if (t.mi == MI && t.ni == NI) return ring_run<MI, NI, GATED>(m, 1, cus);
+  HELIX_RING_GATED(HELIX_RUN)
+#undef HELIX_RUN
+  TORCH_CHECK(false, "no tile of ", 32 * t.mi, " x ", 16 * t.ni);
+}
+
 }  // namespace
+
+// As gemm_bf16_cut, of one launch.
+std::tuple<bool, int64_t, int64_t, int64_t, double> gemm_bf16_glu_cut(
+    int64_t M, int64_t N, int64_t K, int64_t cus) {
+  Ring m{};
+  m.M = M;
+  m.N = N;
+  m.K = K;
+  TORCH_CHECK(M > 0 && N > 0 && K > 0 && cus > 0 && M <= INT32_MAX &&
+              ring_fits(m, GATED), "a product of tiles");
+  const GluPlan p = plan_glu(m, cus);
+  const RingCut c = p.stretches > 0 ? RingCut{} : cut_glu(m, cus, p.us);
+  return {c.rows, c.at, 10 * c.first.mi + c.first.ni, 10 * c.rest.mi + c.rest.ni,
+          c.us};
+}
 
 std::tuple<int64_t, int64_t> gemm_bf16_glu_plan(int64_t M, int64_t N,
                                                          int64_t K,
@@ -108,7 +137,7 @@ void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               "out is [M, N], w [2 N, K]");
   TORCH_CHECK(ring_fits(m, GATED), "columns are a multiple of 8, and K of 64");
   const int cus = ring_cus();
-  GluPlan plan{(int)tile, 0};
+  GluPlan plan{(int)tile, 0, 0};
   if (tile == 0) plan = plan_glu(m, cus);
   if (plan.stretches > 0) {
     const torch::Tensor sums = gemm_bf16_sums(x, w, plan.tile, plan.stretches);
@@ -119,11 +148,13 @@ void gemm_bf16_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                        Divide(m.N / 4));
     return;
   }
-  const RingTile best{plan.tile / 10, plan.tile % 10, 0};
-#define HELIX_RUN(MI, NI)                                                    \
-  if (best.mi == MI && best.ni == NI)                                        \
-    return ring_run<MI, NI, GATED>(m, 1, cus);
-  HELIX_RING_GATED(HELIX_RUN)
-#undef HELIX_RUN
-  TORCH_CHECK(false, "no tile of ", 32 * best.mi, " x ", 16 * best.ni);
+  const RingCut cut = tile == 0 ? cut_glu(m, cus, plan.us) : RingCut{};
+  if (cut.at > 0) {
+    Ring a, b;
+    m.ld = m.up = m.N;
+    ring_parts(m, cut, a, b);
+    run_glu(a, cut.first, cus);
+    return run_glu(b, cut.rest, cus);
+  }
+  run_glu(m, RingTile{plan.tile / 10, plan.tile % 10, 0}, cus);
 }

@@ -80,6 +80,8 @@ struct Ring {
   uint16_t* out;
   float* sums;                                // [stretch][M][N]
   int M, N, K, m_tiles, n_tiles, tiles, total, stretch, gelu;
+  int ld, up;                  // columns of a row of out; GATED: rows of w from
+                               // a gate to its other factor (0: N)
   int group, strip_shift;      // tiles of rows; of group * RING_STRIP tiles
   int unit;                    // ANY: columns that are stored at a time
   int turn;                    // see ring_turn
@@ -95,23 +97,26 @@ struct RingItem {
 // what lies past the end of one is checked by a load's own offset, not by this
 // scalar one on top of it.
 struct RingAt {
-  int k, from, end, left, ahead;
+  int k, end, ahead, from, wrap;              // from and wrap: what is behind end
   __host__ __device__ __forceinline__ void open(int k0, int k1, int turn) {
     k = k0 + turn;
-    from = k0;
     end = k1;
-    left = k1 - k0;
     ahead = RING_STEP;
+    from = k0;
+    wrap = turn;
   }
   __host__ __device__ __forceinline__ void close() {
-    k = from = ahead = 0;
-    end = left = 0x7fffffff;
+    k = ahead = 0;
+    end = 0x7fffffff;
   }
   // Whether all of the item is ordered.
   __host__ __device__ __forceinline__ bool step() {
-    k += ahead;
-    if (k >= end) k = from;
-    return (left -= ahead) <= 0;
+    if ((k += ahead) < end) return false;
+    if (wrap == 0) return true;
+    k = from;
+    end = from + wrap;
+    wrap = 0;
+    return false;
   }
 };
 
@@ -256,7 +261,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
     const int n = (r & ~31) | (r & 12) << 1 | (r & 16) >> 2 | (r & 3);
     if constexpr (FORM == GATED) {            // half of a wave's from either
       const int wave = n / (16 * NI), c = n % (16 * NI);
-      return wave * 8 * NI + (c < 8 * NI ? c : (int64_t)m.N + c - 8 * NI);
+      return wave * 8 * NI + (c < 8 * NI ? c : (int64_t)m.up + c - 8 * NI);
     }
     return n;
   });
@@ -273,7 +278,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
     x_at = m.x + (int64_t)p.m0 * m.K;
     w_at = m.w + (int64_t)p.n0 * m.K;
     x_bytes = min(BM, m.M - p.m0) * m.K * 2;
-    w_bytes = FORM == GATED ? (2 * m.N - p.n0) * m.K * 2
+    w_bytes = FORM == GATED ? (m.up + m.N - p.n0) * m.K * 2
                             : min(BN, m.N - p.n0) * m.K * 2;
     order.open(p.k0, p.k1,
                (p.n0 / OUT_N & m.turn) * RING_STEP);
@@ -396,13 +401,13 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_kernel(Ring m) {
     // also those that are dropped: stores_open counts on them.
     constexpr int NONE = 0x7fffff00;          // past the end of any tile
     constexpr int SIZE = FORM == SUMS ? 4 : 2;
-    const int row = wr * 16 * MI + lo, down = 16 * m.N * SIZE;
-    const int bytes = min(BM, m.M - cur.m0) * m.N * SIZE;
-    const int64_t at = ((int64_t)cur.split * m.M + cur.m0) * m.N;
+    const int row = wr * 16 * MI + lo, down = 16 * m.ld * SIZE;
+    const int bytes = ((min(BM, m.M - cur.m0) - 1) * m.ld + m.N) * SIZE;
+    const int64_t at = ((int64_t)cur.split * m.M + cur.m0) * m.ld;
 #pragma unroll
     for (int j = 0; j < NI / (FORM == GATED ? 4 : 2); ++j) {
       const int c = cur.n0 + wc * (OUT_N / 2) + j * 32 + hi * 8;
-      const int o = (row * m.N + c) * SIZE;
+      const int o = (row * m.ld + c) * SIZE;
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         if constexpr (FORM == SUMS) {
@@ -531,6 +536,70 @@ RingPlan ring_plan(const Ring& m, RingForm form, const int (&tiles)[N][2],
   return best;
 }
 
+// A product in two launches: the first has rounds of large tiles that leave no CU
+// idle, the second what is left, in tiles of its own choice; cut behind that many
+// rows or columns. Where one launch ends with a round of few tiles that takes
+// three quarters of a full one, the second takes less and its start, 3 us. Other
+// tiles than the two largest and fewer rounds than all full ones gain nothing more
+// by the estimates. us in one launch and cut: 660 of 2 x 14336 x 4096 gated 157 and
+// 129, 1537 295 and 268, 5188 848 and 829; 8540 of 4096 x 14336 759 and 700, 5537 of
+// 4096 x 4096 154 and 136, 3330 of 6144 x 4096 140 and 128, 12476 of 4096 x 1024 99
+// and 95. Over 90 sizes that it takes at a gain of 2% or more, 4.5% in the mean;
+// what ring_cut_below asks for leaves out those that lost (8065 of 2304 x 768 31 and
+// 34, 4788 of 4096 x 1024 41 and 44).
+constexpr double ring_cut_below(double us, double part) {
+  return us * (1 - part) - 2.5;
+}
+struct RingCut {
+  bool rows = false;
+  int at = 0;
+  RingTile first{}, rest{};
+  double us = 1e30;
+};
+
+template <int N>
+RingCut ring_cut(const Ring& m, RingForm form, const int (&tiles)[N][2], int cus,
+                 double below) {
+  RingCut best;
+  best.us = below;
+  for (const RingTile& t : RING_TILES) {
+    if (t.mi < 7 || t.ni < 8 || !ring_has(tiles, t)) continue;
+    const int rows = 32 * t.mi, columns = (form == GATED ? 16 : 32) * t.ni;
+    const int64_t down = cdiv(m.M, rows), right = cdiv(m.N, columns);
+    const int64_t full = down * right / cus * cus;
+    for (const bool by_rows : {true, false}) {
+      const int64_t at = by_rows ? full / right * rows : full / down * columns;
+      if (at <= 0 || at >= (by_rows ? m.M : m.N)) continue;
+      Ring a = m, b = m;
+      (by_rows ? a.M : a.N) = (int)at;
+      (by_rows ? b.M : b.N) -= (int)at;
+      const double us = ring_cost(a, form, t, 1, cus).us();
+      if (us >= best.us) continue;
+      const RingPlan rest = ring_plan(b, form, tiles, 1, 1, cus, best.us - us);
+      if (rest.tile.mi != 0)
+        best = RingCut{by_rows, (int)at, t, rest.tile, us + rest.us};
+    }
+  }
+  return best;
+}
+
+// The two parts of a product.
+void ring_parts(const Ring& m, const RingCut& cut, Ring& a, Ring& b) {
+  a = b = m;
+  if (cut.rows) {
+    a.M = cut.at;
+    b.M -= cut.at;
+    b.x += (int64_t)cut.at * m.K;
+    b.out += (int64_t)cut.at * m.ld;
+  } else {
+    a.N = cut.at;
+    b.N -= cut.at;
+    b.w += (int64_t)cut.at * m.K;
+    b.out += cut.at;
+    if (m.bias != nullptr) b.bias += cut.at;
+  }
+}
+
 // Mask of a tile of columns' number: at which step of an inner dimension that is
 // not cut it begins. Rows of w a multiple of 8 KB apart lie on the same channels, and
 // workgroups that start together would all read those; but where several tiles of
@@ -566,6 +635,8 @@ void ring_run(Ring m, int stretches, int cus) {
   const void* kernel = (const void*)gemm_ring_kernel<MI, NI, FORM>;
   static const bool once = ring_allow(kernel);
   (void)once;
+  if (m.ld == 0) m.ld = m.N;
+  if (m.up == 0) m.up = m.N;
   m.m_tiles = cdiv(m.M, 32 * MI);
   m.n_tiles = cdiv(m.N, (FORM == GATED ? 16 : 32) * NI);
   const int64_t total = (int64_t)m.m_tiles * m.n_tiles * stretches;

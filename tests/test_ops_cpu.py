@@ -207,6 +207,27 @@ def test_gemm_bf16_plan_of_any_columns():
     assert plan(100, 1020, 4096, False, False)[1] > 1
 
 
+def test_gemm_bf16_cuts():
+    """Behind the full rounds of large tiles, by rows or columns, where that
+    takes less than one launch by more than the estimates are off."""
+    cut, glu = ops._native().gemm_bf16_cut, ops._native().gemm_bf16_glu_cut
+    assert cut(5537, 4096, 4096, False)[:3] == (True, 4096, 88)
+    assert cut(3195, 6144, 4096, False)[:3] == (False, 4864, 88)
+    assert glu(1540, 14336, 4096)[:2] == (False, 13952)
+    assert glu(4101, 14336, 4096)[:2] == (True, 4096)
+    for M, N, K in ((8192, 4096, 4096), (300, 4096, 4096), (8065, 2304, 768)):
+        assert cut(M, N, K, False)[1] == 0
+    for M, N, K in ((8192, 14336, 4096), (33, 14336, 4096), (1, 8, 64)):
+        assert glu(M, N, K)[1] == 0
+    for M in range(257, 9000, 613):
+        rows, at, first, rest, us = cut(M, 4104, 2048, False)
+        if at:
+            assert 0 < at < (M if rows else 4104)
+            assert at % (32 * (first // 10 if rows else first % 10)) == 0
+            assert us < ops._native().gemm_bf16_plan(M, 4104, 2048, False,
+                                                     False)[2]
+
+
 def test_gemm_ring_loads_stay_at_the_start():
     """Descriptors are empty after the last item; a scalar offset is not part
     of their check, so it stays at 0 however many steps follow."""

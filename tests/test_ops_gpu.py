@@ -1007,6 +1007,49 @@ def test_gemm_rows_uncut(m, n, k):
         torch.testing.assert_close(ops.linear(x, w, b).double(), want, **tol)
 
 
+@pytest.mark.parametrize("m,n,k,act", [
+    (5537, 4096, 2048, 0), (5537, 4104, 2048, 1), (8206, 2312, 2048, 1),
+    (5400, 6144, 1024, 0)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_bf16_in_two_launches(m, n, k, act, bias):
+    """Cut by rows and by columns, remainders of either in both parts."""
+    native = ops._native()
+    assert native.gemm_bf16_cut(m, n, k, act == 1)[1] > 0
+    assert native.gemm_bf16_plan(m, n, k, act == 1, False)[1] == 1
+    torch.manual_seed(59)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV) if bias else None
+    want = x.double() @ w.double().t()
+    if bias:
+        want += b.double()
+    if act:
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    out = torch.full((m + 1, n), 7., dtype=torch.bfloat16, device=DEV)
+    native.gemm_bf16(out[:m], x, w, b, act)
+    # fp32 sums of k products and GELU's exponential, the rounding to bf16
+    torch.testing.assert_close(out[:m].double(), want, rtol=2 ** -8, atol=2e-5)
+    assert (out[m] == 7).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(660, 14336, 1024), (661, 14344, 1024),
+                                   (4101, 4104, 2048)])
+def test_gemm_bf16_glu_in_two_launches(m, n, k):
+    native = ops._native()
+    assert native.gemm_bf16_glu_cut(m, n, k)[1] > 0
+    torch.manual_seed(60)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(2 * n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    out = torch.full((m + 1, n), 7., dtype=torch.bfloat16, device=DEV)
+    native.gemm_bf16_glu(out[:m], x, w)
+    # fp32 sums of k products, the rounding to bf16
+    torch.testing.assert_close(out[:m].double(),
+                               torch.nn.functional.silu(g) * u, rtol=2 ** -8,
+                               atol=5e-5)
+    assert (out[m] == 7).all()
+
+
 @pytest.mark.parametrize("m,n,k,tile", [
     (1, 8, 4096, 22), (40, 1030, 4096, 22), (64, 4168, 8192, 22),
     (65, 8328, 4096, 34), (128, 8328, 4096, 48), (129, 2056, 4096, 58),
