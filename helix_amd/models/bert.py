@@ -14,6 +14,7 @@ import torch
 import torch.nn as nn
 
 from helix_amd import ops
+from helix_amd.models.llama import _own
 
 
 @dataclass
@@ -38,6 +39,11 @@ BERT_PRESETS = {
                             intermediate_size=256, num_layers=2, num_heads=2,
                             max_position=128),
 }
+
+
+def _plain(emb: nn.Module) -> bool:
+    """Whether an embedding does no more than look up rows of its weight."""
+    return _own(emb, nn.Embedding) and emb.max_norm is None
 
 
 class BertLayer(nn.Module):
@@ -100,19 +106,28 @@ class BertEmbeddingModel(nn.Module):
             raise ValueError(f"boundaries {cu} do not cut {T} tokens")
         if self.cfg.pooling != "mean" and cu[-2] == T:
             raise IndexError("a last text without tokens")
-        start = cu_seqlens[:-1].long()
-        positions = torch.arange(T, device=input_ids.device) - \
-            torch.repeat_interleave(start, cu_seqlens.diff(), output_size=T)
-        x = self.word_emb(input_ids) + self.pos_emb(positions)
-        x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
-                           self.cfg.layer_norm_eps)
+        x = None
+        if _plain(self.word_emb) and _plain(self.pos_emb):
+            x = ops.text_embed(input_ids, cu_seqlens, self.word_emb.weight,
+                               self.pos_emb.weight, self.emb_ln_w,
+                               self.emb_ln_b, self.cfg.layer_norm_eps)
+        if x is None:
+            positions = torch.arange(T, device=input_ids.device) - \
+                torch.repeat_interleave(cu_seqlens[:-1].long(),
+                                        cu_seqlens.diff(), output_size=T)
+            x = self.word_emb(input_ids) + self.pos_emb(positions)
+            x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
+                               self.cfg.layer_norm_eps)
         for layer in self.layers:
             x = layer(x, cu_seqlens, max_len)
         if self.cfg.pooling == "mean":
             emb = torch.stack([x[s:e].float().mean(0)
                                for s, e in zip(cu, cu[1:])])
         else:
-            emb = x[start].float()
+            emb = ops.text_pool(x, cu_seqlens)
+            if emb is not None:
+                return emb
+            emb = x[cu_seqlens[:-1].long()].float()
         return torch.nn.functional.normalize(emb, dim=-1)
 
     @torch.inference_mode()

@@ -35,6 +35,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from helix_amd import ops
+from helix_amd.models.bert import _plain
 from helix_amd.models.llama import _own
 
 
@@ -219,8 +220,63 @@ class DiTModel(nn.Module):
         """lat [B,C,s,s], t [B] in [0,1], text_ids [B,text_len] ->
         velocity [B,C,s,s] float32."""
         cfg = self.cfg
+        B, Tt, L = lat.shape[0], cfg.text_len, cfg.seq_len
+        x, cond, cu = self._open(lat, t, text_ids) or \
+            self._open_in_steps(lat, t, text_ids)
+        y = gate = None
+        if all(_own(blk, DiTBlock) for blk in self.blocks):
+            *mods, fm = ops.gemm_bf16_many(
+                cond, [b.mod_w for b in self.blocks] + [self.fin_mod_w],
+                [b.mod_b for b in self.blocks] + [self.fin_mod_b])
+            for blk, mod in zip(self.blocks, mods):
+                x, y, gate = blk.open_sum(x, y, gate, mod, cu, L)
+        else:
+            for blk in self.blocks:
+                x = blk(x, cond, cu, L)
+            fm = ops.gemm_bf16(cond, self.fin_mod_w, self.fin_mod_b)
+        shift, scale = fm.chunk(2, dim=-1)
+        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps, y, gate)
+        out = ops.gemm_bf16(n, self.fin_w, self.fin_b)
+        if type(self) is DiTModel:
+            v = ops.image_velocity(out, (B, cfg.latent_ch, cfg.latent_size,
+                                         cfg.latent_size), cfg.patch, Tt)
+            if v is not None:
+                return v
+        patch_rows = out.view(B, L, -1)[:, Tt:, :].reshape(
+            B * cfg.num_patches, cfg.patch_dim)
+        return self._unpatchify(patch_rows.float(), B)
+
+    def _open(self, lat: torch.Tensor, t: torch.Tensor,
+              text_ids: torch.Tensor):
+        """What the blocks begin with (_open_in_steps), by a launch for each of
+        its parts; None where these do not read what is given."""
+        cfg = self.cfg
+        if type(self) is not DiTModel or not lat.is_cuda or \
+                self.in_w.dtype != torch.bfloat16 or lat.shape[1:] != (
+                cfg.latent_ch, cfg.latent_size, cfg.latent_size) or \
+                text_ids.shape != (lat.shape[0], cfg.text_len) or \
+                t.shape != lat.shape[:1] or \
+                not (_plain(self.txt_emb) and _plain(self.pos_emb)):
+            return None
+        rows = ops.image_rows(lat, cfg.patch, self.in_k)
+        temb = ops.time_embed(t, cfg.time_dim)
+        if rows is None or temb is None:
+            return None
+        image = ops.gemm_bf16(rows, self.in_w, self.in_b)
+        cond = ops.gemm_bf16(temb, self.t_w1, self.t_b1, act=1)
+        cond = ops.gemm_bf16(cond, self.t_w2, self.t_b2)
+        both = ops.image_tokens(text_ids, self.txt_emb.weight,
+                                self.pos_emb.weight, image, cond)
+        return both and (both[0], cond, both[1])
+
+    def _open_in_steps(self, lat: torch.Tensor, t: torch.Tensor,
+                       text_ids: torch.Tensor):
+        """(x [B * L, h], cond [B, h], cu): the text's and the image's tokens with
+        their places, the conditioning of the modulations, boundaries of the
+        images."""
+        cfg = self.cfg
         B = lat.shape[0]
-        P, Tt, L = cfg.num_patches, cfg.text_len, cfg.seq_len
+        P, L = cfg.num_patches, cfg.seq_len
         dtype = self.in_w.dtype
         rows = self._patchify(lat).to(dtype)
         if self.in_k != cfg.patch_dim:
@@ -236,23 +292,7 @@ class DiTModel(nn.Module):
         cond = (cond.float() + tx.float().mean(dim=1)).to(dtype)
         cu = torch.arange(0, (B + 1) * L, L, dtype=torch.int32,
                           device=lat.device)
-        y = gate = None
-        if all(_own(blk, DiTBlock) for blk in self.blocks):
-            *mods, fm = ops.gemm_bf16_many(
-                cond, [b.mod_w for b in self.blocks] + [self.fin_mod_w],
-                [b.mod_b for b in self.blocks] + [self.fin_mod_b])
-            for blk, mod in zip(self.blocks, mods):
-                x, y, gate = blk.open_sum(x, y, gate, mod, cu, L)
-        else:
-            for blk in self.blocks:
-                x = blk(x, cond, cu, L)
-            fm = ops.gemm_bf16(cond, self.fin_mod_w, self.fin_mod_b)
-        shift, scale = fm.chunk(2, dim=-1)
-        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps, y, gate)
-        out = ops.gemm_bf16(n, self.fin_w, self.fin_b)
-        patch_rows = out.view(B, L, -1)[:, Tt:, :].reshape(
-            B * P, cfg.patch_dim)
-        return self._unpatchify(patch_rows.float(), B)
+        return x, cond, cu
 
 
 def rf_schedule(steps: int, shift: float = 3.0) -> torch.Tensor:

@@ -126,6 +126,74 @@ def gated_add(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor,
     return (x.float() + g.float() * y.float()).to(x.dtype)
 
 
+def text_embed(ids: torch.Tensor, cu: torch.Tensor, word: torch.Tensor,
+               pos: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float):
+    """Layer norm of word[ids] + pos[place within the text], or None for other
+    forms than the kernel reads (the CPU's among them)."""
+    if ids.is_cuda and word.dim() == 2:
+        out = torch.empty(ids.shape[0], word.shape[1], dtype=torch.bfloat16,
+                          device=ids.device)
+        if _native().text_embed(out, ids, cu, word, pos, w, b, eps):
+            return out
+    return None
+
+
+def text_pool(x: torch.Tensor, cu: torch.Tensor):
+    """Rows cu[:-1] of x (fp32), each divided by its length, or None as above."""
+    if x.is_cuda:
+        out = torch.empty(cu.shape[0] - 1, x.shape[1], device=x.device,
+                          dtype=torch.float32)
+        if _native().text_pool(out, x, cu):
+            return out
+    return None
+
+
+def image_rows(lat: torch.Tensor, patch: int, columns: int):
+    """Patches of the latents [B, C, S, S] as rows of so many columns (bf16, zeros
+    behind a patch), or None as above."""
+    if lat.is_cuda and lat.dim() == 4:
+        n = (lat.shape[2] // patch) * (lat.shape[3] // patch)
+        out = torch.empty(lat.shape[0] * n, columns, dtype=torch.bfloat16,
+                          device=lat.device)
+        if _native().image_rows(out, lat, patch):
+            return out
+    return None
+
+
+def image_velocity(rows: torch.Tensor, shape, patch: int, text: int):
+    """Rows of the image tokens, behind so many of text in each image, as latents
+    of that shape (fp32), or None as above."""
+    if rows.is_cuda:
+        out = torch.empty(shape, dtype=torch.float32, device=rows.device)
+        if _native().image_velocity(out, rows, patch, text):
+            return out
+    return None
+
+
+def image_tokens(ids: torch.Tensor, word: torch.Tensor, pos: torch.Tensor,
+                 image: torch.Tensor, cond: torch.Tensor):
+    """(x, cu): word[ids] and the image's rows, each with its place, image after
+    image, and their boundaries; the mean of word[ids] is added to cond. None as
+    above."""
+    if ids.is_cuda and pos.dim() == 2:
+        B, (L, h) = ids.shape[0], pos.shape
+        x = torch.empty(B * L, h, dtype=torch.bfloat16, device=ids.device)
+        cu = torch.empty(B + 1, dtype=torch.int32, device=ids.device)
+        if _native().image_tokens(x, cond, cu, ids, word, pos, image):
+            return x, cu
+    return None
+
+
+def time_embed(t: torch.Tensor, dim: int):
+    """Sinusoidal embedding of times (bf16), or None as above."""
+    if t.is_cuda and t.dim() == 1:
+        out = torch.empty(t.shape[0], dim, dtype=torch.bfloat16,
+                          device=t.device)
+        if _native().time_embed(out, t):
+            return out
+    return None
+
+
 def rotary_embedding(positions: torch.Tensor, q: torch.Tensor,
                      k: torch.Tensor, cos_sin: torch.Tensor, head_dim: int):
     """In-place on GPU. Returns (q, k)."""

@@ -8,6 +8,17 @@ bool add_norm(c10::optional<torch::Tensor> sum, torch::Tensor out,
               torch::Tensor x, c10::optional<torch::Tensor> y,
               c10::optional<torch::Tensor> gate, torch::Tensor a,
               torch::Tensor b, int64_t L, double eps);
+bool text_embed(torch::Tensor out, torch::Tensor ids, torch::Tensor cu,
+                torch::Tensor word, torch::Tensor pos, torch::Tensor w,
+                torch::Tensor b, double eps);
+bool text_pool(torch::Tensor out, torch::Tensor x, torch::Tensor cu);
+bool image_rows(torch::Tensor out, torch::Tensor lat, int64_t patch);
+bool image_velocity(torch::Tensor out, torch::Tensor rows, int64_t patch,
+                    int64_t text);
+bool image_tokens(torch::Tensor x, torch::Tensor cond, torch::Tensor cu,
+                  torch::Tensor ids, torch::Tensor word, torch::Tensor pos,
+                  torch::Tensor image);
+bool time_embed(torch::Tensor out, torch::Tensor t);
 bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L);
 bool norm_in_registers(int64_t rows, int64_t columns);
@@ -105,6 +116,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("add_norm", &add_norm,
         "(Gated) add + LayerNorm with weights or an image's modulation");
   m.def("gated_add", &gated_add, "x + gate * y, a gate per image");
+  m.def("text_embed", &text_embed,
+        "LayerNorm of a text's word and position embeddings");
+  m.def("text_pool", &text_pool, "First rows of texts, divided by their length");
+  m.def("image_rows", &image_rows, "Patches of latents as rows");
+  m.def("image_velocity", &image_velocity, "Rows of image tokens as latents");
+  m.def("image_tokens", &image_tokens,
+        "Text and image rows with their places, mean of the text");
+  m.def("time_embed", &time_embed, "Sinusoidal embedding of times");
   m.def("norm_in_registers", &norm_in_registers,
         "Whether add_sums_rms_norm keeps a row in registers");
   m.def("add_sums_rms_norm", &add_sums_rms_norm,

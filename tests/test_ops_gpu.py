@@ -161,6 +161,101 @@ def test_add_norm_strides():
                                    **tol)
 
 
+@pytest.mark.parametrize("lens", [[1], [5, 0, 3, 1], [3] * 130, [200, 7]])
+@pytest.mark.parametrize("h", [8, 520, 768, 4096])
+def test_text_embed_and_pool(lens, h):
+    """Texts without tokens among others, more texts than a wave has lanes,
+    places and words past the end of their tables."""
+    torch.manual_seed(61)
+    T = sum(lens)
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    ids = torch.randint(0, 50, (T,), device=DEV)
+    ids[-1] = 77
+    word, pos = (torch.randn(n, h, dtype=torch.bfloat16, device=DEV)
+                 for n in (50, 150))
+    w, b = torch.randn(2, h, dtype=torch.bfloat16, device=DEV)
+    place = torch.cat([torch.arange(n, device=DEV) for n in lens])
+    x = word[ids.clamp(max=49)] + pos[place.clamp(max=149)]
+    want = torch.nn.functional.layer_norm(
+        x.double(), (h,), w.double(), b.double(), 1e-12)
+    got = ops.text_embed(ids, cu, word, pos, w, b, 1e-12)
+    # 32-bit sums of h values, then the rounding to bf16 (2^-9, doubled)
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2e-5)
+    if lens[-1] == 0:
+        return
+    first = got[cu[:-1].long()].double()
+    torch.testing.assert_close(
+        ops.text_pool(got, cu).double(),
+        torch.nn.functional.normalize(first, dim=-1), rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("B,C,S,p,text,h", [(1, 4, 32, 2, 32, 1024),
+                                            (3, 3, 6, 3, 1, 8),
+                                            (70, 1, 4, 1, 5, 264)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_image_ends(B, C, S, p, text, h, dtype):
+    """Patches, tokens and latents are those of torch's own steps, bit for bit;
+    the text's mean and the time as far as sums and functions go."""
+    from helix_amd.models.dit import timestep_embedding
+    torch.manual_seed(62)
+    g, d = S // p, C * p * p
+    P, L, K = g * g, g * g + text, -(-d // 64) * 64
+    lat = torch.randn(B, C, S, S, dtype=dtype, device=DEV)
+    rows = lat.unfold(2, p, p).unfold(3, p, p).permute(
+        0, 2, 3, 1, 4, 5).reshape(B * P, d).to(torch.bfloat16)
+    got = ops.image_rows(lat, p, K)
+    assert torch.equal(got[:, :d], rows) and not got[:, d:].any()
+    out = torch.randn(B * L, d, dtype=torch.bfloat16, device=DEV)
+    want = out.view(B, L, d)[:, text:].reshape(B, g, g, C, p, p).permute(
+        0, 3, 1, 4, 2, 5).reshape(B, C, S, S).float()
+    assert torch.equal(ops.image_velocity(out, (B, C, S, S), p, text), want)
+    ids = torch.randint(-2, 12, (B, text), device=DEV)
+    word, pos, image, cond = (
+        torch.randn(n, h, dtype=torch.bfloat16, device=DEV)
+        for n in (9, L, B * P, B))
+    tx = word[ids.clamp(0, 8)]
+    x = (torch.cat([tx, image.view(B, P, h)], 1) + pos).view(B * L, h)
+    mean = cond.double() + tx.double().mean(1)
+    new, cu = ops.image_tokens(ids, word, pos, image, cond)
+    assert torch.equal(new, x)
+    assert cu.tolist() == list(range(0, (B + 1) * L, L))
+    # a sum of text values in 32 bits, the rounding to bf16
+    torch.testing.assert_close(cond.double(), mean, rtol=2 ** -8, atol=1e-5)
+    t = torch.rand(B, device=DEV)
+    # arguments of up to 1000 in 32 bits (2^-14 each), the rounding to bf16
+    torch.testing.assert_close(
+        ops.time_embed(t, 64).double(), timestep_embedding(t.double(), 64)
+        .double(), rtol=2 ** -8, atol=2 ** -12)
+
+
+def test_ends_of_other_forms():
+    """What these kernels do not read is left to the steps."""
+    x = torch.zeros(4, 64, dtype=torch.bfloat16, device=DEV)
+    cu = torch.tensor([0, 4], dtype=torch.int32, device=DEV)
+    ids = torch.zeros(4, dtype=torch.int64, device=DEV)
+    assert ops.text_embed(ids, cu, x, x, x[0], x[0], 1e-5) is not None
+    assert ops.text_embed(ids.int(), cu, x, x, x[0], x[0], 1e-5) is None
+    assert ops.text_embed(ids, cu.long(), x, x, x[0], x[0], 1e-5) is None
+    assert ops.text_embed(ids, cu, x.float(), x, x[0], x[0], 1e-5) is None
+    assert ops.text_embed(ids, cu, x, x, x[0, 1:], x[0], 1e-5) is None
+    assert ops.text_pool(x.float(), cu) is None
+    assert ops.text_pool(x.t(), cu) is None
+    lat = torch.zeros(2, 4, 8, 8, dtype=torch.bfloat16, device=DEV)
+    assert ops.image_rows(lat, 2, 64) is not None
+    assert ops.image_rows(lat, 3, 64) is None
+    assert ops.image_rows(lat, 2, 8) is None
+    assert ops.image_rows(lat.half(), 2, 64) is None
+    assert ops.image_rows(lat.transpose(2, 3), 2, 64) is None
+    assert ops.image_rows(lat[:0], 2, 64) is None
+    assert ops.image_velocity(x, (1, 4, 8, 8), 4, 0) is not None
+    assert ops.image_velocity(x, (1, 4, 8, 8), 4, 1) is None
+    assert ops.image_tokens(ids.view(1, 4), x, x, x, x[:1]) is None
+    assert ops.image_tokens(ids[:1].view(1, 1), x, x, x[:3], x[:1]) is not None
+    assert ops.image_tokens(ids[:1].view(1, 1), x, x, x, x[:1]) is None
+    assert ops.time_embed(torch.zeros(2, device=DEV), 63) is None
+    assert ops.time_embed(torch.zeros(2, device=DEV).double(), 64) is None
+
+
 @pytest.mark.parametrize("m", [1, 17, 64])
 @pytest.mark.parametrize("k,ns", [(256, [64]), (1024, [384, 128, 384]),
                                   (512, [192, 64 * 50]), (768, [3072] * 49)])
