@@ -47,6 +47,10 @@ def _plain(emb: nn.Module) -> bool:
 
 
 class BertLayer(nn.Module):
+    PARAMS = ("qkv_w", "qkv_b", "attn_out_w", "attn_out_b", "attn_ln_w",
+              "attn_ln_b", "up_w", "up_b", "down_w", "down_b", "out_ln_w",
+              "out_ln_b")
+
     def __init__(self, cfg: BertConfig):
         super().__init__()
         h = cfg.hidden_size
@@ -67,6 +71,12 @@ class BertLayer(nn.Module):
         self.scale = self.hd ** -0.5
 
     def forward(self, x, cu, max_len):
+        if tuple(self._parameters) == self.PARAMS:
+            out = ops.text_block(x, cu, max_len, self.cfg.num_heads, self.scale,
+                                 self.cfg.layer_norm_eps,
+                                 list(self._parameters.values()))
+            if out is not None:
+                return out
         T = x.shape[0]
         h = self.cfg.hidden_size
         qkv = ops.gemm_bf16(x, self.qkv_w, self.qkv_b)

@@ -128,6 +128,8 @@ class TinyVAE(nn.Module):
 class DiTBlock(nn.Module):
     """Pre-norm transformer block with adaLN modulation (shift/scale/
     gate x attn/mlp from the conditioning vector)."""
+    PARAMS = ("qkv_w", "qkv_b", "out_w", "out_b", "up_w", "up_b", "down_w",
+              "down_b", "mod_w", "mod_b")
 
     def __init__(self, cfg: DiTConfig):
         super().__init__()
@@ -158,6 +160,12 @@ class DiTBlock(nn.Module):
         taken of, for input of that form (y None: x); mod: the modulation of
         both halves. The sum is left to the norm that reads it (8 images:
         a launch of 5 us and a pass over the rows)."""
+        if tuple(self._parameters) == self.PARAMS:
+            out = ops.image_block(x, y, gate, mod, cu, L, self.cfg.heads,
+                                  self.scale, self.cfg.eps,
+                                  list(self._parameters.values()))
+            if out is not None:
+                return out
         h = self.cfg.hidden
         T = x.shape[0]
         sa, ca, ga, sm, cm, gm = mod.chunk(6, dim=-1)

@@ -148,6 +148,32 @@ def text_pool(x: torch.Tensor, cu: torch.Tensor):
     return None
 
 
+def text_block(x: torch.Tensor, cu: torch.Tensor, max_len: int, heads: int,
+               scale: float, eps: float, params: list):
+    """A block of the text encoder by one call (blocks.hip): attention and
+    feed-forward, each with the norm of its sum, or None as above."""
+    if x.is_cuda and not _seen_by_torch():
+        return _native().text_block(x, cu, max_len, heads, scale, eps, params)
+    return None
+
+
+def image_block(x: torch.Tensor, y, gate, mod: torch.Tensor,
+                cu: torch.Tensor, L: int, heads: int, scale: float, eps: float,
+                params: list):
+    """A block of the image model by one call (blocks.hip), (x, y, gate) of a sum
+    that is still to be taken, or None as above."""
+    if x.is_cuda and not _seen_by_torch():
+        return _native().image_block(x, y, gate, mod, cu, L, heads, scale, eps,
+                                     params) or None
+    return None
+
+
+def _seen_by_torch() -> bool:
+    """Whether something wants to see the steps one by one."""
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling()
+            or torch.is_autocast_enabled("cuda"))
+
+
 def image_rows(lat: torch.Tensor, patch: int, columns: int):
     """Patches of the latents [B, C, S, S] as rows of so many columns (bf16, zeros
     behind a patch), or None as above."""

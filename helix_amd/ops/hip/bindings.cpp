@@ -19,6 +19,14 @@ bool image_tokens(torch::Tensor x, torch::Tensor cond, torch::Tensor cu,
                   torch::Tensor ids, torch::Tensor word, torch::Tensor pos,
                   torch::Tensor image);
 bool time_embed(torch::Tensor out, torch::Tensor t);
+c10::optional<torch::Tensor> text_block(
+    torch::Tensor x, torch::Tensor cu, int64_t max_len, int64_t heads,
+    double scale, double eps, std::vector<torch::Tensor> p);
+std::vector<torch::Tensor> image_block(
+    torch::Tensor x, c10::optional<torch::Tensor> y,
+    c10::optional<torch::Tensor> gate, torch::Tensor mod, torch::Tensor cu,
+    int64_t L, int64_t heads, double scale, double eps,
+    std::vector<torch::Tensor> p);
 bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L);
 bool norm_in_registers(int64_t rows, int64_t columns);
@@ -124,6 +132,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("image_tokens", &image_tokens,
         "Text and image rows with their places, mean of the text");
   m.def("time_embed", &time_embed, "Sinusoidal embedding of times");
+  m.def("text_block", &text_block, "A block of the text encoder");
+  m.def("image_block", &image_block, "A block of the image model");
   m.def("norm_in_registers", &norm_in_registers,
         "Whether add_sums_rms_norm keeps a row in registers");
   m.def("add_sums_rms_norm", &add_sums_rms_norm,

@@ -228,6 +228,72 @@ def test_image_ends(B, C, S, p, text, h, dtype):
         .double(), rtol=2 ** -8, atol=2 ** -12)
 
 
+@pytest.mark.parametrize("lens,h,inner,heads", [
+    ([1], 128, 256, 2), ([20, 0, 44], 768, 3072, 12), ([70, 3], 768, 3072, 12),
+    ([64], 256, 512, 2), ([300], 1024, 4096, 16)])
+def test_text_block(lens, h, inner, heads, monkeypatch):
+    """The steps of a block in one call give the same bits, streamed products of
+    few rows among them."""
+    from helix_amd.models.bert import BertConfig, BertLayer
+    torch.manual_seed(63)
+    layer = BertLayer(BertConfig(hidden_size=h, intermediate_size=inner,
+                                 num_heads=heads)).to(torch.bfloat16).to(DEV)
+    for p in layer.parameters():
+        p.data.normal_(0.0, 0.05)
+    x = torch.randn(sum(lens), h, dtype=torch.bfloat16, device=DEV)
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    kept = x.clone()
+    args = (x, cu, max(lens))
+    with torch.inference_mode():
+        params = list(layer._parameters.values())
+        got = ops.text_block(*args, heads, layer.scale, 1e-12, params)
+        assert torch.equal(layer(*args), got)
+        for form in (params[:11], [params[0].float()] + params[1:],
+                     [params[1]] + params[1:]):
+            assert ops.text_block(*args, heads, layer.scale, 1e-12,
+                                  form) is None
+        assert ops.text_block(x, cu.long(), max(lens), heads, layer.scale,
+                              1e-12, params) is None
+        with torch.autocast("cuda"):
+            assert ops.text_block(*args, heads, layer.scale, 1e-12,
+                                  params) is None
+        monkeypatch.setattr(ops, "text_block", lambda *a: None)
+        assert torch.equal(layer(*args), got)
+    assert torch.equal(x, kept)
+
+
+@pytest.mark.parametrize("images,L,h,heads", [(1, 9, 128, 2), (3, 288, 1024, 16),
+                                              (2, 33, 256, 2)])
+@pytest.mark.parametrize("sum_open", [False, True])
+def test_image_block(images, L, h, heads, sum_open, monkeypatch):
+    from helix_amd.models.dit import DiTBlock, DiTConfig
+    torch.manual_seed(64)
+    block = DiTBlock(DiTConfig(hidden=h, heads=heads)).to(torch.bfloat16).to(DEV)
+    for p in block.parameters():
+        p.data.normal_(0.0, 0.05)
+    x, y = torch.randn(2, images * L, h, dtype=torch.bfloat16, device=DEV)
+    mod = torch.randn(images, 6 * h, dtype=torch.bfloat16, device=DEV)
+    gate = torch.randn(images, 2 * h, dtype=torch.bfloat16, device=DEV)[:, h:]
+    cu = torch.arange(0, (images + 1) * L, L, dtype=torch.int32, device=DEV)
+    if not sum_open:
+        y = gate = None
+    kept = x.clone()
+    with torch.inference_mode():
+        params = list(block._parameters.values())
+        tail = (cu, L, heads, block.scale, 1e-6)
+        got = ops.image_block(x, y, gate, mod, *tail, params)
+        for a, b in zip(block.open_sum(x, y, gate, mod, cu, L), got):
+            assert torch.equal(a, b)
+        assert ops.image_block(x, y, gate, mod[:, 1:], *tail, params) is None
+        assert ops.image_block(x, x, None, mod, *tail, params) is None
+        assert ops.image_block(x, y, gate, mod.float(), *tail, params) is None
+        assert ops.image_block(x[1:], y, gate, mod, *tail, params) is None
+        monkeypatch.setattr(ops, "image_block", lambda *a: None)
+        for a, b in zip(block.open_sum(x, y, gate, mod, cu, L), got):
+            assert torch.equal(a, b)
+    assert torch.equal(x, kept)
+
+
 def test_ends_of_other_forms():
     """What these kernels do not read is left to the steps."""
     x = torch.zeros(4, 64, dtype=torch.bfloat16, device=DEV)
