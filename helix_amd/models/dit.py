@@ -151,25 +151,28 @@ class DiTBlock(nn.Module):
     def forward(self, x: torch.Tensor, cond: torch.Tensor,
                 cu: torch.Tensor, L: int) -> torch.Tensor:
         mod = ops.gemm_bf16(cond, self.mod_w, self.mod_b)
-        return ops.gated_add(*self.open_sum(x, None, None, mod, cu, L), L)
+        x, y, gate, _ = self.open_sum(x, None, None, None, mod, cu, L)
+        return ops.gated_add(x, y, gate, L)
 
     def open_sum(self, x: torch.Tensor, y: Optional[torch.Tensor],
-                 gate: Optional[torch.Tensor], mod: torch.Tensor,
-                 cu: torch.Tensor, L: int):
-        """The block's result as (x, y, gate) that x + gate y is still to be
-        taken of, for input of that form (y None: x); mod: the modulation of
-        both halves. The sum is left to the norm that reads it (8 images:
-        a launch of 5 us and a pass over the rows)."""
+                 gate: Optional[torch.Tensor], y_bias: Optional[torch.Tensor],
+                 mod: torch.Tensor, cu: torch.Tensor, L: int,
+                 stretches: bool = False):
+        """The block's result as (x, y, gate, y_bias) that x + gate y is still to
+        be taken of, for input of that form (y None: x); mod: the modulation of
+        both halves. The sum is left to the norm that reads it (8 images: a
+        launch of 5 us and a pass over the rows). y_bias: y is in stretches, see
+        ops.modulated_norm; only where these are asked for."""
         if tuple(self._parameters) == self.PARAMS:
-            out = ops.image_block(x, y, gate, mod, cu, L, self.cfg.heads,
-                                  self.scale, self.cfg.eps,
-                                  list(self._parameters.values()))
+            out = ops.image_block(x, y, gate, y_bias, mod, cu, L,
+                                  self.cfg.heads, self.scale, self.cfg.eps,
+                                  list(self._parameters.values()), stretches)
             if out is not None:
                 return out
         h = self.cfg.hidden
         T = x.shape[0]
         sa, ca, ga, sm, cm, gm = mod.chunk(6, dim=-1)
-        x, n = ops.modulated_norm(x, ca, sa, L, self.cfg.eps, y, gate)
+        x, n = ops.modulated_norm(x, ca, sa, L, self.cfg.eps, y, gate, y_bias)
         qkv = ops.gemm_bf16(n, self.qkv_w, self.qkv_b)
         nh = self.cfg.heads
         q, k, v = (t.view(T, nh, self.hd)
@@ -179,7 +182,7 @@ class DiTBlock(nn.Module):
         x, n = ops.modulated_norm(x, cm, sm, L, self.cfg.eps, a, ga)
         m = ops.gemm_bf16(n, self.up_w, self.up_b, act=1)     # fused GELU
         m = ops.gemm_bf16(m, self.down_w, self.down_b)
-        return x, m, gm
+        return x, m, gm, None
 
 
 class DiTModel(nn.Module):
@@ -231,19 +234,20 @@ class DiTModel(nn.Module):
         B, Tt, L = lat.shape[0], cfg.text_len, cfg.seq_len
         x, cond, cu = self._open(lat, t, text_ids) or \
             self._open_in_steps(lat, t, text_ids)
-        y = gate = None
+        y = gate = y_bias = None
         if all(_own(blk, DiTBlock) for blk in self.blocks):
             *mods, fm = ops.gemm_bf16_many(
                 cond, [b.mod_w for b in self.blocks] + [self.fin_mod_w],
                 [b.mod_b for b in self.blocks] + [self.fin_mod_b])
             for blk, mod in zip(self.blocks, mods):
-                x, y, gate = blk.open_sum(x, y, gate, mod, cu, L)
+                x, y, gate, y_bias = blk.open_sum(x, y, gate, y_bias, mod, cu,
+                                                  L, stretches=True)
         else:
             for blk in self.blocks:
                 x = blk(x, cond, cu, L)
             fm = ops.gemm_bf16(cond, self.fin_mod_w, self.fin_mod_b)
         shift, scale = fm.chunk(2, dim=-1)
-        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps, y, gate)
+        _, n = ops.modulated_norm(x, scale, shift, L, cfg.eps, y, gate, y_bias)
         out = ops.gemm_bf16(n, self.fin_w, self.fin_b)
         if type(self) is DiTModel:
             v = ops.image_velocity(out, (B, cfg.latent_ch, cfg.latent_size,

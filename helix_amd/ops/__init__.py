@@ -96,16 +96,20 @@ def add_layer_norm(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor,
 
 def modulated_norm(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor,
                    L: int, eps: float, y: torch.Tensor | None = None,
-                   gate: torch.Tensor | None = None):
+                   gate: torch.Tensor | None = None,
+                   y_bias: torch.Tensor | None = None):
     """(s, norm(s) (1 + scale) + shift), s = x + gate y (x without y). norm
     is a layer norm without weights; gate, scale and shift have a row for
-    every L rows of x."""
+    every L rows of x. y_bias: y is in stretches [n, T, H] (fp32) of a product
+    that this bias belongs to."""
     if x.is_cuda:
         out = torch.empty_like(x)
         s = x if y is None else torch.empty_like(x)
         if _native().add_norm(None if y is None else s, out, x, y, gate,
-                              scale, shift, L, eps):
+                              scale, shift, L, eps, y_bias):
             return s, out
+    if y_bias is not None:
+        y = (y.sum(0) + y_bias.float()).to(x.dtype)
     if y is not None:
         x = gated_add(x, y, gate, L)
     h = x.shape[-1]
@@ -157,14 +161,17 @@ def text_block(x: torch.Tensor, cu: torch.Tensor, max_len: int, heads: int,
     return None
 
 
-def image_block(x: torch.Tensor, y, gate, mod: torch.Tensor,
+def image_block(x: torch.Tensor, y, gate, y_bias, mod: torch.Tensor,
                 cu: torch.Tensor, L: int, heads: int, scale: float, eps: float,
-                params: list):
-    """A block of the image model by one call (blocks.hip), (x, y, gate) of a sum
-    that is still to be taken, or None as above."""
+                params: list, stretches: bool = False):
+    """A block of the image model by one call (blocks.hip), (x, y, gate, y_bias)
+    of a sum that is still to be taken, or None as above. stretches: y may be such
+    as modulated_norm adds up, with a bias; else y_bias is None."""
     if x.is_cuda and not _seen_by_torch():
-        return _native().image_block(x, y, gate, mod, cu, L, heads, scale, eps,
-                                     params) or None
+        out = _native().image_block(x, y, gate, y_bias, mod, cu, L, heads,
+                                    scale, eps, params, stretches)
+        if out:
+            return (*out, None)[:4]
     return None
 
 

@@ -7,7 +7,10 @@ void fused_add_rms_norm(torch::Tensor x, torch::Tensor residual,
 bool add_norm(c10::optional<torch::Tensor> sum, torch::Tensor out,
               torch::Tensor x, c10::optional<torch::Tensor> y,
               c10::optional<torch::Tensor> gate, torch::Tensor a,
-              torch::Tensor b, int64_t L, double eps);
+              torch::Tensor b, int64_t L, double eps,
+              c10::optional<torch::Tensor> y_bias);
+torch::Tensor gemm_bf16_summand(torch::Tensor x, torch::Tensor w,
+                                torch::Tensor bias);
 bool text_embed(torch::Tensor out, torch::Tensor ids, torch::Tensor cu,
                 torch::Tensor word, torch::Tensor pos, torch::Tensor w,
                 torch::Tensor b, double eps);
@@ -24,9 +27,9 @@ c10::optional<torch::Tensor> text_block(
     double scale, double eps, std::vector<torch::Tensor> p);
 std::vector<torch::Tensor> image_block(
     torch::Tensor x, c10::optional<torch::Tensor> y,
-    c10::optional<torch::Tensor> gate, torch::Tensor mod, torch::Tensor cu,
-    int64_t L, int64_t heads, double scale, double eps,
-    std::vector<torch::Tensor> p);
+    c10::optional<torch::Tensor> gate, c10::optional<torch::Tensor> y_bias,
+    torch::Tensor mod, torch::Tensor cu, int64_t L, int64_t heads,
+    double scale, double eps, std::vector<torch::Tensor> p, bool stretches);
 bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L);
 bool norm_in_registers(int64_t rows, int64_t columns);
@@ -122,7 +125,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "Fused residual-add + RMSNorm (in-place)");
   m.def("add_norm", &add_norm,
-        "(Gated) add + LayerNorm with weights or an image's modulation");
+        "(Gated) add + LayerNorm with weights or an image's modulation",
+        py::arg("sum"), py::arg("out"), py::arg("x"), py::arg("y"),
+        py::arg("gate"), py::arg("a"), py::arg("b"), py::arg("L"),
+        py::arg("eps"), py::arg("y_bias") = py::none());
+  m.def("gemm_bf16_summand", &gemm_bf16_summand,
+        "x @ w^T + bias as rows, or its stretches for a norm that adds them up");
   m.def("gated_add", &gated_add, "x + gate * y, a gate per image");
   m.def("text_embed", &text_embed,
         "LayerNorm of a text's word and position embeddings");

@@ -4,8 +4,8 @@
 // A small batch is bound by the host: views, allocations and the arguments of seven
 // calls a block. us of the host, step by step -> by one call: one image through 12
 // blocks 890 -> 563, eight 848 -> 561; a text of 60 tokens through 12 blocks, which
-// the GPU now takes as long for, 748 -> 526. The kernels, their order and their
-// operands are the same, and so is every bit of the results.
+// the GPU now takes as long for, 748 -> 526. The kernels are those of the steps, but
+// that sums behind deep products take these in stretches (gemm_bf16_summand).
 #include "common.h"
 #include <torch/extension.h>
 #include <c10/core/DeviceGuard.h>
@@ -23,7 +23,10 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
                   torch::Tensor cu_seqlens_k, int64_t max_seqlen, double scale,
                   bool causal, int64_t window);
 bool add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
-              torch::Tensor a, torch::Tensor b, int64_t L, double eps);
+              torch::Tensor a, torch::Tensor b, int64_t L, double eps,
+              OptT y_bias);
+torch::Tensor gemm_bf16_summand(torch::Tensor x, torch::Tensor w,
+                                torch::Tensor bias);
 
 namespace {
 
@@ -49,6 +52,20 @@ torch::Tensor product(const torch::Tensor& x, const torch::Tensor& w,
   else
     gemm_bf16(out, x, w, b, act, 0);
   return out;
+}
+
+// The same for a norm that adds it to something: rows, or stretches of them that
+// the norm adds up (add_norm's y_bias).
+struct Summand {
+  torch::Tensor y;
+  OptT bias;                   // still to be added
+};
+Summand summand(const torch::Tensor& x, const torch::Tensor& w,
+                const torch::Tensor& b) {
+  Summand s;
+  s.y = x.size(0) <= 64 ? product(x, w, b, 0) : gemm_bf16_summand(x, w, b);
+  if (s.y.dim() == 3) s.bias = b;
+  return s;
 }
 
 torch::Tensor attend(const torch::Tensor& x, const torch::Tensor& w,
@@ -91,54 +108,70 @@ OptT text_block(torch::Tensor x, torch::Tensor cu, int64_t max_len,
   for (int i : {4, 5, 10, 11})
     if (!packed(p[i], x, {H})) return {};
   const c10::DeviceGuard on(x.device());
-  auto norm = [&](const torch::Tensor& a, const torch::Tensor& b, int i) {
+  auto norm = [&](const torch::Tensor& a, const Summand& b, int i) {
     torch::Tensor out = at::empty_like(a);
-    TORCH_CHECK(add_norm({}, out, a, b, {}, p[i], p[i + 1], 0, eps),
+    TORCH_CHECK(add_norm({}, out, a, b.y, {}, p[i], p[i + 1], 0, eps, b.bias),
                 "a norm of other operands");
     return out;
   };
   const torch::Tensor o = attend(x, p[0], p[1], cu, max_len, heads, scale);
-  x = norm(x, product(o, p[2], p[3], 0), 4);
+  x = norm(x, summand(o, p[2], p[3]), 4);
   const torch::Tensor up = product(x, p[6], p[7], 1);
-  return norm(x, product(up, p[8], p[9], 0), 10);
+  return norm(x, summand(up, p[8], p[9]), 10);
 }
 
 // x (+ gate y) through a block: the result as x, y and gate of a sum that is still
-// to be taken. mod: shift, scale and gate of either half, a row for every L of x.
-// p: weight and bias of q k v, attention's end, the way up, the way down.
-Tensors image_block(torch::Tensor x, OptT y, OptT gate, torch::Tensor mod,
-                    torch::Tensor cu, int64_t L, int64_t heads, double scale,
-                    double eps, Tensors p) {
+// to be taken, and where y is in stretches the bias that is still to be added to
+// it. mod: shift, scale and gate of either half, a row for every L of x. p: weight
+// and bias of q k v, attention's end, the way up, the way down. stretches: whether y
+// may be in such.
+Tensors image_block(torch::Tensor x, OptT y, OptT gate, OptT y_bias,
+                    torch::Tensor mod, torch::Tensor cu, int64_t L,
+                    int64_t heads, double scale, double eps, Tensors p,
+                    bool stretches) {
   if (p.size() < 8 || !rows_of(x, cu, heads) || p[4].dim() != 2) return {};
   const int64_t T = x.size(0), H = x.size(1), I = p[4].size(0);
   if (I < 1 || I % 64 != 0 || L < 1 || T % L != 0 ||
       !packed(mod, x, {T / L, 6 * H}) || !layer(p, 0, x, 3 * H, H) ||
       !layer(p, 2, x, H, H) || !layer(p, 4, x, I, H) ||
-      !layer(p, 6, x, H, I) || y.has_value() != gate.has_value())
+      !layer(p, 6, x, H, I) || y.has_value() != gate.has_value() ||
+      (y_bias.has_value() && !y.has_value()))
     return {};
-  if (y.has_value() &&
-      (!packed(*y, x, x.sizes()) || gate->dim() != 2 || !gate->is_cuda() ||
-       gate->device() != x.device() ||
-       gate->scalar_type() != torch::kBFloat16 || gate->size(0) != T / L ||
-       gate->size(1) != H || gate->stride(1) != 1 ||
-       gate->stride(0) % 8 != 0 || (uintptr_t)gate->data_ptr() % 16 != 0))
-    return {};
+  if (y.has_value()) {
+    const bool rows = !y_bias.has_value();
+    if (rows ? !packed(*y, x, x.sizes())
+             : !packed(*y_bias, x, {H}) || y->dim() != 3 || y->size(0) < 1 ||
+                   y->size(1) != T || y->size(2) != H ||
+                   y->scalar_type() != torch::kFloat32 ||
+                   y->device() != x.device() || !y->is_contiguous() ||
+                   (uintptr_t)y->data_ptr() % 16 != 0)
+      return {};
+    if (gate->dim() != 2 || gate->device() != x.device() ||
+        gate->scalar_type() != torch::kBFloat16 || gate->size(0) != T / L ||
+        gate->size(1) != H || gate->stride(1) != 1 ||
+        gate->stride(0) % 8 != 0 || (uintptr_t)gate->data_ptr() % 16 != 0)
+      return {};
+  }
   const c10::DeviceGuard on(x.device());
   auto of = [&](int64_t i) {
     return mod.as_strided({T / L, H}, {6 * H, 1}, mod.storage_offset() + i * H);
   };
-  auto norm = [&](const OptT& b, const OptT& g, int shift) {
+  auto norm = [&](const OptT& b, const OptT& bias, const OptT& g, int shift) {
     torch::Tensor out = at::empty_like(x);
     OptT sum;
     if (b.has_value()) sum = at::empty_like(x);
-    TORCH_CHECK(add_norm(sum, out, x, b, g, of(shift + 1), of(shift), L, eps),
+    TORCH_CHECK(add_norm(sum, out, x, b, g, of(shift + 1), of(shift), L, eps,
+                         bias),
                 "a norm of other operands");
     if (sum.has_value()) x = *sum;
     return out;
   };
   const torch::Tensor o =
-      attend(norm(y, gate, 0), p[0], p[1], cu, L, heads, scale);
-  const torch::Tensor a = product(o, p[2], p[3], 0);
-  const torch::Tensor up = product(norm(a, of(2), 3), p[4], p[5], 1);
-  return {x, product(up, p[6], p[7], 0), of(5)};
+      attend(norm(y, y_bias, gate, 0), p[0], p[1], cu, L, heads, scale);
+  const Summand a = summand(o, p[2], p[3]);
+  const torch::Tensor up = product(norm(a.y, a.bias, of(2), 3), p[4], p[5], 1);
+  if (!stretches) return {x, product(up, p[6], p[7], 0), of(5)};
+  const Summand m = summand(up, p[6], p[7]);
+  if (!m.bias.has_value()) return {x, m.y, of(5)};
+  return {x, m.y, of(5), *m.bias};
 }

@@ -3,6 +3,9 @@
 //   norm:  s = x (+ y, or + gate * y);  out = norm(s) * a + b
 //   add:   x + gate * y
 //
+// y may be the stretches of a product (fp32), which are added up here, with its
+// bias, instead of in a launch of their own that rounds them.
+//
 // norm is a layer norm; a and b are its weights, or belong to the image a row
 // is part of (a = 1 + scale). Everything inside is fp32, s is rounded only
 // where it is kept. Bound by memory: a wave has a row and keeps it in
@@ -23,14 +26,17 @@ constexpr int NT = 256;
 
 struct Rows {
   const uint16_t *x, *y, *gate, *a, *b;       // y, gate may be null
+  const float* sums;           // in the place of y: [stretches][T][H]
+  const uint16_t* bias;        // of sums
+  int stretches;
   uint16_t *sum, *out;                        // sum may be null
   int64_t gate_stride, mod_stride;      // of an image's row in gate; in a and b
   int T, H, L;                 // rows of an image; 0: a and b are weights
   float eps;
 };
 
-// NV: vectors of 8 that a lane has
-template <int NV>
+// NV: vectors of 8 that a lane has. SUMS: y is m.sums.
+template <int NV, bool SUMS>
 __global__ __launch_bounds__(NT) void add_norm_kernel(Rows m) {
   const int64_t t = (int64_t)blockIdx.x * (NT / WAVE) + threadIdx.x / WAVE;
   if (t >= m.T) return;
@@ -42,9 +48,29 @@ __global__ __launch_bounds__(NT) void add_norm_kernel(Rows m) {
     const int c = (i * WAVE + lane) * 8;
     if (i * WAVE + lane < nvec) {
       load_bf16x8(m.x + t * m.H + c, v[i]);
-      if (m.y != nullptr) {
+      if (SUMS || m.y != nullptr) {
         float y[8];
-        load_bf16x8(m.y + t * m.H + c, y);
+        if constexpr (SUMS) {
+          const float* p = m.sums + t * m.H + c;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) y[j] = 0.f;
+#pragma unroll 4
+          for (int s = 0; s < m.stretches; ++s, p += (int64_t)m.T * m.H) {
+            const f32x4 u = *reinterpret_cast<const f32x4*>(p);
+            const f32x4 w = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              y[j] += u[j];
+              y[4 + j] += w[j];
+            }
+          }
+          float bias[8];
+          load_bf16x8(m.bias + c, bias);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) y[j] += bias[j];
+        } else {
+          load_bf16x8(m.y + t * m.H + c, y);
+        }
         if (m.gate != nullptr) {
           float g[8];
           load_bf16x8(m.gate + of * m.gate_stride + c, g);
@@ -141,13 +167,25 @@ bool rows_of(const torch::Tensor& x, const torch::Tensor& out, int64_t L,
 
 // L = 0: out = norm(x + y) a + b with weights a, b; else rows of images of L
 // tokens each: sum = x + gate y, out = norm(sum) (1 + a) + b. False, and nothing
-// done, for other forms of operands than the kernel reads.
+// done, for other forms of operands than the kernel reads. y may be the stretches
+// [n, T, H] (fp32) of a product whose bias is y_bias.
 bool add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
-              torch::Tensor a, torch::Tensor b, int64_t L, double eps) {
+              torch::Tensor a, torch::Tensor b, int64_t L, double eps,
+              OptT y_bias) {
   Rows m{};
   if (!rows_of(x, out, L, m)) return false;
   m.eps = (float)eps;
-  if (y.has_value()) {
+  if (y_bias.has_value()) {
+    if (!y.has_value() || y->dim() != 3 || y->size(0) < 1 ||
+        y->size(1) != m.T || y->size(2) != m.H || !y->is_contiguous() ||
+        y->scalar_type() != torch::kFloat32 || y->device() != x.device() ||
+        (uintptr_t)y->data_ptr() % 16 != 0 || !reads(*y_bias, x) ||
+        !y_bias->is_contiguous() || y_bias->numel() != m.H)
+      return false;
+    m.sums = y->data_ptr<float>();
+    m.bias = (const uint16_t*)y_bias->data_ptr();
+    m.stretches = y->size(0);
+  } else if (y.has_value()) {
     if (!like(*y, x)) return false;
     m.y = (const uint16_t*)y->data_ptr();
   }
@@ -173,7 +211,14 @@ bool add_norm(OptT sum, torch::Tensor out, torch::Tensor x, OptT y, OptT gate,
   const dim3 grid(cdiv(m.T, NT / WAVE));
   auto stream = at::hip::getCurrentHIPStream();
 #define HELIX_AN(NV)                                                         \
-  hipLaunchKernelGGL(add_norm_kernel<NV>, grid, dim3(NT), 0, stream, m)
+  do {                                                                       \
+    if (m.sums != nullptr)                                                   \
+      hipLaunchKernelGGL((add_norm_kernel<NV, true>), grid, dim3(NT), 0,     \
+                         stream, m);                                         \
+    else                                                                     \
+      hipLaunchKernelGGL((add_norm_kernel<NV, false>), grid, dim3(NT), 0,    \
+                         stream, m);                                         \
+  } while (0)
   if (m.H <= 512) HELIX_AN(1);
   else if (m.H <= 1024) HELIX_AN(2);
   else if (m.H <= 2048) HELIX_AN(4);

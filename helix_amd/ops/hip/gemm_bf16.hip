@@ -390,6 +390,39 @@ torch::Tensor gemm_bf16_sums(torch::Tensor x, torch::Tensor w, int64_t tile,
   return sums_of(x, m, p.tile, p.stretches, cus);
 }
 
+// x @ w^T for a layer norm that adds it to something: rows with the bias [M, N], or
+// two to four stretches [n, M, N] (fp32) without it where those take less with
+// their reader, which would have read rows; half a microsecond is left to rows. The
+// norm has a wave to a row, so more stretches cost it 0.5 us each. us with the
+// norm, rows and stretches: 100 x 1024 x 4096 13.9 and 13.4, 288 16.6 and 14.8, 576
+// 19.8 and 17.5, 1152 24.2 and 21.2, 2000 26.3 and 27.9; 400 x 768 x 3072 15.9 and
+// 14.2. Up to 64 rows, and where the inner dimension is not deep, it is 0.5 us at
+// most (60 x 1024 x 4096 13.8 and 13.1, 200 x 768 x 768 10.2 and 9.9).
+torch::Tensor gemm_bf16_summand(torch::Tensor x, torch::Tensor w,
+                                torch::Tensor bias) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.is_cuda() &&
+              x.scalar_type() == torch::kBFloat16, "bf16 matrices on the GPU");
+  const c10::DeviceGuard on(x.device());
+  Ring m = ring_of(x, w);
+  if (m.M > 64 && m.N > 0 && m.K >= 2 * m.N && w.size(1) == m.K &&
+      m.N % 8 == 0 && (int64_t)m.M * m.N <= 4 << 20 && ring_fits(m, SUMS) &&
+      ring_fits(m, ROWS) && x.is_contiguous() && w.is_contiguous() &&
+      w.scalar_type() == torch::kBFloat16 && w.device() == x.device() &&
+      (uintptr_t)m.x % 16 == 0 && (uintptr_t)m.w % 16 == 0) {
+    const int cus = ring_cus();
+    const RingPlan rows = plan_rows(m, cus);
+    const RingPlan sums = ring_plan(m, SUMS, SUMS_TILES, 2,
+                                    std::min(4, m.K / RING_STEP), cus);
+    // rows in stretches that a launch of 4 us joins
+    if (sums.us + 0.5 <=
+        std::min(rows.us, sums.us + 4) + 2. * m.M * m.N / 4.5e6)
+      return sums_of(x, m, sums.tile, sums.stretches, cus);
+  }
+  torch::Tensor out = torch::empty({x.size(0), w.size(0)}, x.options());
+  gemm_bf16(out, x, w, bias, 0, 0);
+  return out;
+}
+
 // What gemm_bf16 (sums false) and gemm_bf16_sums do with a product on so many
 // CUs: tile, stretches, us with the reader of those, and how many times were
 // worked out to find them. Tile 0: no sums take less than `below`.

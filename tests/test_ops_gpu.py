@@ -232,8 +232,8 @@ def test_image_ends(B, C, S, p, text, h, dtype):
     ([1], 128, 256, 2), ([20, 0, 44], 768, 3072, 12), ([70, 3], 768, 3072, 12),
     ([64], 256, 512, 2), ([300], 1024, 4096, 16)])
 def test_text_block(lens, h, inner, heads, monkeypatch):
-    """The steps of a block in one call give the same bits, streamed products of
-    few rows among them."""
+    """A block in one call and step by step: the same, but for what the norms add
+    up unrounded."""
     from helix_amd.models.bert import BertConfig, BertLayer
     torch.manual_seed(63)
     layer = BertLayer(BertConfig(hidden_size=h, intermediate_size=inner,
@@ -258,7 +258,9 @@ def test_text_block(lens, h, inner, heads, monkeypatch):
             assert ops.text_block(*args, heads, layer.scale, 1e-12,
                                   params) is None
         monkeypatch.setattr(ops, "text_block", lambda *a: None)
-        assert torch.equal(layer(*args), got)
+        # norms of two sums, whose parts were rounded to bf16 before
+        torch.testing.assert_close(layer(*args).double(), got.double(),
+                                   rtol=2 ** -7, atol=2 ** -5)
     assert torch.equal(x, kept)
 
 
@@ -281,17 +283,88 @@ def test_image_block(images, L, h, heads, sum_open, monkeypatch):
     with torch.inference_mode():
         params = list(block._parameters.values())
         tail = (cu, L, heads, block.scale, 1e-6)
-        got = ops.image_block(x, y, gate, mod, *tail, params)
-        for a, b in zip(block.open_sum(x, y, gate, mod, cu, L), got):
-            assert torch.equal(a, b)
-        assert ops.image_block(x, y, gate, mod[:, 1:], *tail, params) is None
-        assert ops.image_block(x, x, None, mod, *tail, params) is None
-        assert ops.image_block(x, y, gate, mod.float(), *tail, params) is None
-        assert ops.image_block(x[1:], y, gate, mod, *tail, params) is None
-        monkeypatch.setattr(ops, "image_block", lambda *a: None)
-        for a, b in zip(block.open_sum(x, y, gate, mod, cu, L), got):
-            assert torch.equal(a, b)
+        got = ops.image_block(x, y, gate, None, mod, *tail, params)
+        assert got[3] is None
+        for a, b in zip(block.open_sum(x, y, gate, None, mod, cu, L), got):
+            assert a is b is None or torch.equal(a, b)
+        assert ops.image_block(x, y, gate, None, mod[:, 1:], *tail,
+                               params) is None
+        assert ops.image_block(x, x, None, None, mod, *tail, params) is None
+        assert ops.image_block(x, None, None, params[1], mod, *tail,
+                               params) is None
+        assert ops.image_block(x, x, gate, params[3], mod, *tail,
+                               params) is None
+        assert ops.image_block(x, y, gate, None, mod.float(), *tail,
+                               params) is None
+        assert ops.image_block(x[1:], y, gate, None, mod, *tail, params) is None
+        # stretches are the rows but for their rounding, here and in the next
+        open_ = block.open_sum(x, y, gate, None, mod, cu, L, stretches=True)
+        rows = open_[1] if open_[3] is None else \
+            open_[1].sum(0) + open_[3].float()
+        assert torch.equal(open_[0], got[0])
+        torch.testing.assert_close(rows.double(), got[1].double(),
+                                   rtol=2 ** -8, atol=2e-5)
+        after = [block.open_sum(*t, mod, cu, L) for t in (open_, got)]
+        monkeypatch.setattr(ops, "image_block", lambda *a, **k: None)
+        after.append(block.open_sum(*open_, mod, cu, L))
+        steps = block.open_sum(x, y, gate, None, mod, cu, L)
+    # sums of parts of up to 2^4 that were rounded to bf16 before, their norms
+    # times modulations of up to 2^2 and products of 2^4 of those
+    close = dict(rtol=2 ** -6, atol=2 ** -3)
+    for a, b in zip(steps[:2], got):
+        torch.testing.assert_close(a.double(), b.double(), **close)
+    for t in after[1:]:
+        for a, b in zip(t[:2], after[0]):
+            err = (a.double() - b.double()).norm() / b.double().norm()
+            assert err < 2 ** -6
     assert torch.equal(x, kept)
+
+
+@pytest.mark.parametrize("T,H,n", [(1, 8, 1), (5, 520, 3), (66, 768, 8),
+                                   (4, 4096, 16)])
+def test_add_norm_of_stretches(T, H, n):
+    torch.manual_seed(65)
+    L = 3
+    x = torch.randn(T, H, dtype=torch.bfloat16, device=DEV)
+    sums = torch.randn(n, T, H, device=DEV)
+    w, b, bias = torch.randn(3, H, dtype=torch.bfloat16, device=DEV)
+    gate, scale, shift = torch.randn(-(-T // L), 3 * H, dtype=torch.bfloat16,
+                                     device=DEV).chunk(3, -1)
+    g, c, s = (t.repeat_interleave(L, 0)[:T].double()
+               for t in (gate, scale, shift))
+    norm = lambda t: torch.nn.functional.layer_norm(t, (H,), eps=1e-6)  # noqa: E731
+    y = sums.double().sum(0) + bias.double()
+    # 32-bit sums of H values, then the rounding to bf16 (2^-9, doubled)
+    tol = dict(rtol=2 ** -8, atol=1e-4)
+    total = x.double() + g * y
+    new, got = ops.modulated_norm(x, scale, shift, L, 1e-6, sums, gate, bias)
+    torch.testing.assert_close(new.double(), total, **tol)
+    torch.testing.assert_close(got.double(), norm(total) * (1 + c) + s, **tol)
+    out = torch.empty_like(x)
+    assert ops._native().add_norm(None, out, x, sums, None, w, b, 0, 1e-6, bias)
+    torch.testing.assert_close(
+        out.double(), norm(x.double() + y) * w.double() + b.double(), **tol)
+    for other in (sums.half(), sums[:, :, 1:], sums[0]):
+        assert not ops._native().add_norm(None, out, x, other, None, w, b, 0,
+                                          1e-6, bias)
+
+
+@pytest.mark.parametrize("m,n,k,form", [
+    (1, 8, 64, 2), (64, 1024, 4096, 2), (288, 1024, 4096, 3), (65, 8, 1024, 3),
+    (2304, 1024, 4096, 2), (2304, 1024, 1024, 2), (700, 768, 3072, 3)])
+def test_gemm_bf16_summand(m, n, k, form):
+    """Rows with the bias or stretches without."""
+    torch.manual_seed(66)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    b = torch.randn(n, dtype=torch.bfloat16, device=DEV)
+    got = ops._native().gemm_bf16_summand(x, w, b)
+    assert got.dim() == form
+    if form == 3:
+        got = got.double().sum(0) + b.double()
+    torch.testing.assert_close(got.double(),
+                               x.double() @ w.double().t() + b.double(),
+                               rtol=2 ** -8, atol=2e-5)
 
 
 def test_ends_of_other_forms():
