@@ -814,14 +814,19 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear_silu_mul where that is the faster form, product and activation
     apart elsewhere. From 33 rows on by tiles, whose halves meet before they are
-    rounded: in one launch (us apart and now: 64 rows of 28672 x 4096 56 and 52,
-    512 107 and 95, 8192 1407 and 1285), and where that leaves CUs idle, narrow
-    or deep, in stretches that a second one adds up (apart, in one launch and
-    now: 80 of 2048 x 8192 20, 43 and 15, 100 of 4096 x 14336 43, 79 and 37, 512
-    of 1024 x 16384 50, 90 and 30). Up to 64 rows of more than 8192 columns, where
+    rounded: in one launch (us apart and now: 64 rows of 28672 x 4096 56 and 46,
+    512 107 and 93, 8192 1407 and 1246), from 17 on where tiles of wide matrices
+    begin apart (ring_turn in gemm_ring.h; us streamed and by tiles: 17 of 28672 x
+    4096 43.8 and 43.6, 24 45.2 and 43.5, 32 46.9 and 43.8, of 26624 x 4096 46.4
+    and 39.7, of 32768 x 4096 49.0 and 48.6, but 24 47.9 and 48.4), and where
+    that leaves CUs idle, narrow or deep, in stretches that a second one adds up
+    (apart, in one launch and now: 80 of 2048 x 8192 20, 43 and 15, 100 of 4096 x
+    14336 43, 79 and 37, 512 of 1024 x 16384 50, 90 and 30). Up to 64 rows of more than 8192 columns, where
     _glu_fits does not take them, are bound by their weights and stay apart (48 of
     10240 x 8192 53 in one launch, 44 apart; 64 of 14336 x 4096 36 and 31)."""
-    if x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and \
+    apart = 16 if w.dim() == 2 and w.shape[1] % 4096 == 0 and \
+        w.shape[0] > 8192 else 32
+    if x.dim() == 2 and w.dim() == 2 and x.shape[0] > apart and \
             w.shape[0] % 16 == 0 and x.dtype == torch.bfloat16 and (
                 x.shape[0] > ROWS_MAX_M_GLU or w.shape[0] <= 8192 or
                 _glu_fits(x.shape[0], *w.shape)) and \

@@ -1219,6 +1219,28 @@ def test_gemm_rows_forms(m, n, k):
                                atol=25 * 2 ** -8)
 
 
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (16, 26624, 4096, False), (17, 26624, 4096, True), (32, 26640, 4096, True),
+    (32, 26624, 2048, False)])
+def test_gated_few_rows(m, n, k, tiles):
+    """Either side of the line between streamed weights and tiles."""
+    torch.manual_seed(59)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV) / k ** 0.5
+    with torch.inference_mode():
+        got = ops.gated_linear(x, w)
+    same = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    if tiles:
+        ops._native().gemm_bf16_glu(same, x, w)
+    else:
+        ops._native().gemm_rows_glu(same, x, w, None, None)
+    assert torch.equal(got, same)
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    # fp32 sums of k products, then the rounding to bf16
+    torch.testing.assert_close(got.double(), torch.nn.functional.silu(g) * u,
+                               rtol=2 ** -8, atol=5e-5)
+
+
 @pytest.mark.parametrize("m", [1, 5, 16, 31, 48, 49, 128])
 @pytest.mark.parametrize("n,k", [(16456, 256), (32776, 768), (24576, 2048),
                                  (24568, 2048), (65544, 2048),
