@@ -258,6 +258,13 @@ class MLP(nn.Module):
         return _project(self.down_proj, h, form)
 
 
+def _norm_for(m: nn.Module, kind: type, proj: str):
+    """The norm before m: where m as written here hands the rows to an 8-bit
+    projection, and to nothing else, it writes their bytes."""
+    bytes_ = _own(m, kind) and _own(getattr(m, proj), FP8Linear)
+    return ops.fused_add_rms_norm_fp8 if bytes_ else ops.fused_add_rms_norm
+
+
 class DecoderLayer(nn.Module):
     def __init__(self, cfg: LlamaConfig, tp_size: int = 1, tp_rank: int = 0):
         super().__init__()
@@ -274,12 +281,12 @@ class DecoderLayer(nn.Module):
             residual = x.clone()
             h = ops.rms_norm(x, self.input_norm_w, self.eps)
         else:
-            h, residual = ops.fused_add_rms_norm(x, residual,
-                                                 self.input_norm_w, self.eps)
+            h, residual = _norm_for(self.attn, Attention, "qkv_proj")(
+                x, residual, self.input_norm_w, self.eps)
         h = self.attn(h, cos_sin, kv_cache, meta,
                       *(["sums"] if _own(self.attn, Attention) else []))
-        h, residual = ops.fused_add_rms_norm(h, residual, self.post_norm_w,
-                                             self.eps)
+        h, residual = _norm_for(self.mlp, MLP, "gate_up_proj")(
+            h, residual, self.post_norm_w, self.eps)
         h = self.mlp(h, *([form] if _own(self.mlp, MLP) else []))
         return h, residual
 

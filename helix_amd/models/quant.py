@@ -36,13 +36,16 @@ class FP8Linear(nn.Module):
         w8, ws = ops.quantize_fp8(lin.weight.data)
         return cls(w8.contiguous(), ws.contiguous())
 
-    def forward(self, x: torch.Tensor, form: str = "rows") -> torch.Tensor:
+    def forward(self, x: torch.Tensor | ops.Quantized,
+                form: str = "rows") -> torch.Tensor:
         """form: as of the projection it stands for ("rows", "sums" for a
         reader that adds up stretches, "glu")."""
         shape = x.shape[:-1]
-        x2 = x.reshape(-1, self.in_features)
-        x8, xs = ops.quantize_fp8(x2)
-        if form == "sums" and x.dim() == 2:
+        if isinstance(x, ops.Quantized):
+            x8, xs = x
+        else:
+            x8, xs = ops.quantize_fp8(x.reshape(-1, self.in_features))
+        if form == "sums" and len(shape) == 1:
             return ops.gemm_fp8_sums(x8, self.weight8, xs, self.w_scale)
         if form == "glu":
             out = ops.gemm_fp8_silu_mul(x8, self.weight8, xs, self.w_scale)

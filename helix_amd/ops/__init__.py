@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import functools
 import os
+from typing import NamedTuple
 from dataclasses import dataclass
 
 import torch
@@ -73,6 +74,30 @@ def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor,
     x.copy_(out)
     residual.copy_(new_res)
     return x, residual
+
+
+class Quantized(NamedTuple):
+    """Rows as e4m3 bytes and a float32 scale of each (quantize_fp8)."""
+    bytes: torch.Tensor
+    scales: torch.Tensor
+
+    @property
+    def shape(self):
+        return self.bytes.shape
+
+
+def fused_add_rms_norm_fp8(x: torch.Tensor, residual: torch.Tensor,
+                           w: torch.Tensor, eps: float):
+    """fused_add_rms_norm for 8-bit projections alone: stretches on GPU give
+    Quantized rows, what quantize_fp8 makes of the norm, in the same launch.
+    Other forms of x as there."""
+    if x.is_cuda and x.dim() == 3 and x.dtype == torch.float32:
+        h = Quantized(torch.empty_like(residual, dtype=torch.uint8),
+                      torch.empty(residual.shape[0], dtype=torch.float32,
+                                  device=x.device))
+        _native().add_sums_rms_norm_fp8(*h, x, residual, w, eps)
+        return h, residual
+    return fused_add_rms_norm(x, residual, w, eps)
 
 
 def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor,

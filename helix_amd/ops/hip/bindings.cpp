@@ -35,6 +35,9 @@ bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
 bool norm_in_registers(int64_t rows, int64_t columns);
 void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
                        torch::Tensor residual, torch::Tensor w, double eps);
+void add_sums_rms_norm_fp8(torch::Tensor h, torch::Tensor scales,
+                           torch::Tensor x, torch::Tensor residual,
+                           torch::Tensor w, double eps);
 void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                 torch::Tensor b, double eps);
 void rotary_embedding(torch::Tensor positions, torch::Tensor q,
@@ -146,6 +149,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "Whether add_sums_rms_norm keeps a row in registers");
   m.def("add_sums_rms_norm", &add_sums_rms_norm,
         "Sum of a product's stretches + residual-add + RMSNorm");
+  m.def("add_sums_rms_norm_fp8", &add_sums_rms_norm_fp8,
+        "The same, rows as e4m3 bytes and scales (bf16 residual, fp32 in)");
   m.def("layer_norm", &layer_norm, "LayerNorm (bf16)");
   m.def("rotary_embedding", &rotary_embedding,
         "Apply rotary embedding to q,k in-place");

@@ -5,7 +5,7 @@
 //
 // Replaces the RMSNorm and the residual addition that the reference delegates
 // to vLLM's containers.
-#include "common.h"
+#include "quant.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -102,18 +102,20 @@ __global__ void fused_add_rms_norm_kernel(uint16_t* __restrict__ x,
 // residual' = sum of x's stretches + residual ; h = rmsnorm(residual') * w
 // x is a product whose inner dimension was cut (fp32 [stretches, T, H]); its
 // sum is taken here, in order, instead of in a launch of its own (2.5 to 3 us)
-// and is not rounded before it meets the residual.
-template <int BLOCK>
+// and is not rounded before it meets the residual. FP8: the row leaves as e4m3 and a
+// scale, bit by bit what quantize_rows makes of h, for 8-bit projections. That
+// launch is bound by its start and its latency: us of both and of one, 4
+// stretches: 32 rows of 4096 6.4 and 4.9, of 8192 (the loop) 9.7 and 8.6.
+template <int BLOCK, bool FP8>
 __global__ __launch_bounds__(BLOCK) void add_sums_rms_norm_kernel(
-    uint16_t* __restrict__ h, const float* __restrict__ x,
-    uint16_t* __restrict__ residual, const uint16_t* __restrict__ w,
-    float eps, int H, int stretches) {
+    void* __restrict__ h, float* __restrict__ scales,
+    const float* __restrict__ x, uint16_t* __restrict__ residual,
+    const uint16_t* __restrict__ w, float eps, int H, int stretches) {
   __shared__ float red[BLOCK / WAVE];
   const int t = blockIdx.x;
   const int64_t all = (int64_t)gridDim.x * H;
   const float* xrow = x + (int64_t)t * H;
   uint16_t* rrow = residual + (int64_t)t * H;
-  uint16_t* hrow = h + (int64_t)t * H;
 
   float ss = 0.f;
   const int nvec = H / 8;
@@ -140,13 +142,39 @@ __global__ __launch_bounds__(BLOCK) void add_sums_rms_norm_kernel(
   ss = block_reduce_sum(ss, red);
   const float inv = rsqrtf(ss / H + eps);
 
-  for (int v = threadIdx.x; v < nvec; v += BLOCK) {
-    float e[8], ww[8];
+  auto normed = [&](int v, float (&e)[8]) {
+    float ww[8];
     load_bf16x8(rrow + v * 8, e);
     load_bf16x8(w + v * 8, ww);
 #pragma unroll
     for (int i = 0; i < 8; ++i) e[i] = e[i] * inv * ww[i];
-    store_bf16x8(hrow + v * 8, e);
+  };
+  if constexpr (FP8) {
+    __shared__ uint32_t tops[BLOCK / WAVE];
+    auto half = [](const float* e) {
+      return u16x4{f32_to_bf16(e[0]), f32_to_bf16(e[1]), f32_to_bf16(e[2]),
+                   f32_to_bf16(e[3])};
+    };
+    uint32_t top = 0;
+    for (int v = threadIdx.x; v < nvec; v += BLOCK) {
+      float e[8];
+      normed(v, e);
+      top = max(top, max(top_of(half(e)), top_of(half(e + 4))));
+    }
+    const float scale = fp8_scale(block_reduce_top<BLOCK>(top, tops));
+    if (threadIdx.x == 0) scales[t] = scale;
+    for (int v = threadIdx.x; v < nvec; v += BLOCK) {
+      float e[8];
+      normed(v, e);
+      reinterpret_cast<u32x2*>((uint8_t*)h + (int64_t)t * H)[v] =
+          u32x2{fp8x4(half(e), scale), fp8x4(half(e + 4), scale)};
+    }
+  } else {
+    for (int v = threadIdx.x; v < nvec; v += BLOCK) {
+      float e[8];
+      normed(v, e);
+      store_bf16x8((uint16_t*)h + (int64_t)t * H + v * 8, e);
+    }
   }
 }
 
@@ -157,10 +185,11 @@ __global__ __launch_bounds__(BLOCK) void add_sums_rms_norm_kernel(
 // 16 rows 5.3 -> 3.8. With 8 columns a thread 300 rows of 8192 took 9.3 us
 // instead of 7.7, so longer rows keep the loop. stays_in_registers says which
 // others do.
+template <bool FP8>
 __global__ __launch_bounds__(WIDE) void add_sums_rms_norm_wide_kernel(
-    uint16_t* __restrict__ h, const float* __restrict__ x,
-    uint16_t* __restrict__ residual, const uint16_t* __restrict__ w,
-    float eps, int H, int stretches) {
+    void* __restrict__ h, float* __restrict__ scales,
+    const float* __restrict__ x, uint16_t* __restrict__ residual,
+    const uint16_t* __restrict__ w, float eps, int H, int stretches) {
   __shared__ float red[WIDE / WAVE];
   const int64_t row = (int64_t)blockIdx.x * H, all = (int64_t)gridDim.x * H;
   const bool mine = (int)threadIdx.x * 4 < H;
@@ -185,7 +214,16 @@ __global__ __launch_bounds__(WIDE) void add_sums_rms_norm_wide_kernel(
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     o[i] = f32_to_bf16(bf16_to_f32(b[i]) * inv * bf16_to_f32(wc[i]));
-  if (mine) *reinterpret_cast<u16x4*>(h + row + c) = o;
+  if constexpr (FP8) {
+    __shared__ uint32_t tops[WIDE / WAVE];
+    const float scale =
+        fp8_scale(block_reduce_top<WIDE>(mine ? top_of(o) : 0, tops));
+    if (threadIdx.x == 0) scales[blockIdx.x] = scale;
+    if (mine)
+      *reinterpret_cast<uint32_t*>((uint8_t*)h + row + c) = fp8x4(o, scale);
+  } else if (mine) {
+    *reinterpret_cast<u16x4*>((uint16_t*)h + row + c) = o;
+  }
 }
 
 // LayerNorm (for encoder / bge-class models): out = (x - mu)/sigma * w + b
@@ -258,16 +296,22 @@ void fused_add_rms_norm(torch::Tensor x, torch::Tensor residual,
                      (const uint16_t*)w.data_ptr(), (float)eps, H);
 }
 
-void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
-                       torch::Tensor residual, torch::Tensor w, double eps) {
+namespace {
+
+// h: rows of bf16, or with scales of e4m3 bytes
+template <bool FP8>
+void add_sums(const torch::Tensor& h, float* scales, const torch::Tensor& x,
+              const torch::Tensor& residual, const torch::Tensor& w,
+              double eps) {
   TORCH_CHECK(x.dim() == 3 && x.is_contiguous() &&
               x.scalar_type() == torch::kFloat32 && h.is_contiguous() &&
               residual.is_contiguous() && residual.dim() == 2 &&
               residual.size(0) == x.size(1) && residual.size(1) == x.size(2) &&
               h.sizes() == residual.sizes());
   for (const auto& t : {h, residual, w})
-    TORCH_CHECK(t.scalar_type() == torch::kBFloat16 &&
-                t.device() == x.device() && t.is_contiguous(),
+    TORCH_CHECK(t.device() == x.device() && t.is_contiguous() &&
+                t.scalar_type() == (FP8 && t.is_same(h) ? torch::kUInt8
+                                                        : torch::kBFloat16),
                 "packed bf16 beside the stretches");
   TORCH_CHECK(w.numel() == x.size(2) && x.is_cuda(), "weights of a row");
   const int T = x.size(1);
@@ -276,18 +320,34 @@ void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
   if (T == 0 || H == 0) return;               // no row, or no column of one
   auto stream = at::hip::getCurrentHIPStream();
   if (stays_in_registers(T, H)) {
-    hipLaunchKernelGGL(add_sums_rms_norm_wide_kernel, dim3(T), dim3(WIDE), 0,
-                       stream, (uint16_t*)h.data_ptr(), x.data_ptr<float>(),
+    hipLaunchKernelGGL(add_sums_rms_norm_wide_kernel<FP8>, dim3(T), dim3(WIDE),
+                       0, stream, h.data_ptr(), scales, x.data_ptr<float>(),
                        (uint16_t*)residual.data_ptr(),
                        (const uint16_t*)w.data_ptr(), (float)eps, H,
                        (int)x.size(0));
     return;
   }
-  hipLaunchKernelGGL((add_sums_rms_norm_kernel<512>), dim3(T), dim3(512), 0,
-                     stream, (uint16_t*)h.data_ptr(), x.data_ptr<float>(),
+  hipLaunchKernelGGL((add_sums_rms_norm_kernel<512, FP8>), dim3(T), dim3(512),
+                     0, stream, h.data_ptr(), scales, x.data_ptr<float>(),
                      (uint16_t*)residual.data_ptr(),
                      (const uint16_t*)w.data_ptr(), (float)eps, H,
                      (int)x.size(0));
+}
+
+}  // namespace
+
+void add_sums_rms_norm(torch::Tensor h, torch::Tensor x,
+                       torch::Tensor residual, torch::Tensor w, double eps) {
+  add_sums<false>(h, nullptr, x, residual, w, eps);
+}
+
+void add_sums_rms_norm_fp8(torch::Tensor h, torch::Tensor scales,
+                           torch::Tensor x, torch::Tensor residual,
+                           torch::Tensor w, double eps) {
+  TORCH_CHECK(scales.is_contiguous() && scales.device() == x.device() &&
+              scales.scalar_type() == torch::kFloat32 && x.dim() == 3 &&
+              scales.numel() == x.size(1));
+  add_sums<true>(h, scales.data_ptr<float>(), x, residual, w, eps);
 }
 
 bool norm_in_registers(int64_t rows, int64_t columns) {

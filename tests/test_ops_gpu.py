@@ -1653,6 +1653,52 @@ def test_gemm_rows_e4m3(m, n, k):
         atol=2 * lost * float(want.abs().max() + 1))
 
 
+@pytest.mark.parametrize("T,K", [
+    (1, 2048), (3, 2056), (512, 4096), (513, 4096), (2, 4104), (2, 16384),
+    (3, 16392), (2, 32768), (2, 32776)])
+def test_quantize_rows_in_registers(T, K):
+    """Rows in registers, edges of their widths, and rows of the loop: bits of
+    the steps one by one, and nothing past the rows."""
+    from helix_amd.ops import _native
+    torch.manual_seed(K)
+    x = torch.randn(T, K, dtype=torch.bfloat16, device=DEV) * 7
+    x[0, -1], x[-1, 0] = 300.0, -301.0
+    got = torch.full((T + 1, K), 99, dtype=torch.uint8, device=DEV)
+    scale = torch.full((T + 1,), 99.0, device=DEV)
+    _native().quantize_rows(got[:T], scale[:T], x)
+    f = x.float()
+    s = f.abs().amax(-1, keepdim=True).clamp(min=1e-8) * (
+        torch.tensor(1.0) / 448).to(DEV)
+    assert torch.equal(scale[:T], s[:, 0]) and scale[T] == 99
+    want = (f / s).to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(got[:T], want) and (got[T] == 99).all()
+
+
+@pytest.mark.parametrize("n,t,h", [(1, 1, 8), (3, 5, 264), (4, 33, 4096),
+                                   (2, 3, 4104), (2, 257, 264), (5, 32, 8192),
+                                   (3, 128, 3072)])
+def test_norm_to_bytes(n, t, h):
+    """The norm of stretches to e4m3: bytes, scales and residual are those of the
+    norm and quantize_rows, also of rows of zeros, infinities and NaN."""
+    torch.manual_seed(h)
+    x = torch.randn(n, t, h, device=DEV)
+    res = torch.randn(t, h, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(h, dtype=torch.bfloat16, device=DEV)
+    if t > 3:
+        x[0, 1, 2], x[0, 2, 5] = float("nan"), float("inf")
+        x[:, 3], res[3] = 0, 0
+    kept = res.clone()
+    h16, kept = ops.fused_add_rms_norm(x, kept, w, 1e-5)
+    want, scales = ops.quantize_fp8(h16)
+    got, res = ops.fused_add_rms_norm_fp8(x, res, w, 1e-5)
+    assert got.shape == h16.shape
+    assert torch.equal(got.bytes, want)
+    assert torch.equal(got.scales.view(torch.int32), scales.view(torch.int32))
+    assert torch.equal(res.view(torch.int16), kept.view(torch.int16))
+    y = torch.randn(t, h, dtype=torch.bfloat16, device=DEV)   # rows stay rows
+    assert ops.fused_add_rms_norm_fp8(y, res, w, 1e-5)[0] is y
+
+
 @pytest.mark.parametrize("T,K", [(1, 8), (3, 264), (33, 4096), (5, 14336)])
 def test_quantize_rows_bytes(T, K):
     """Bytes and scales are those of the same steps as library calls."""

@@ -85,3 +85,22 @@ def test_eval_quant_harness_runs(tmp_path):
     assert set(rep["variants"]) == {"bf16", "fp8_weights", "fp8_kv",
                                     "fp8_both"}
     assert rep["variants"]["fp8_weights"]["mean_kl"] < 0.05
+
+
+def test_bytes_only_where_the_projection_reads_them():
+    """Which norm precedes a block: a hook, a module put in another's place or
+    bf16 weights are given rows."""
+    from helix_amd.models import llama
+    mlp = llama.MLP(llama.PRESETS["tiny"])
+    norm = lambda: llama._norm_for(mlp, llama.MLP, "gate_up_proj")
+    rows, to_bytes = ops.fused_add_rms_norm, ops.fused_add_rms_norm_fp8
+    assert norm() is rows
+    quantize_model_fp8(mlp)
+    assert norm() is to_bytes
+    for m in (mlp, mlp.gate_up_proj):
+        hook = m.register_forward_pre_hook(lambda *a: None)
+        assert norm() is rows
+        hook.remove()
+    assert norm() is to_bytes
+    mlp.gate_up_proj = torch.nn.Linear(256, 1024)
+    assert norm() is rows
