@@ -671,14 +671,21 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
 def _streams_pay(M: int, N: int, K: int) -> bool:
     """Whether up to 64 rows that do not go by tiles stream their weights rather
     than take the library's product: up to 16 rows of up to 65536 columns, and
-    deep narrow ones. Beyond, of rows 4 or 8 KB apart: workgroups that begin apart
+    deep narrow ones. Of rows 4 or 8 KB apart: workgroups that begin apart
     (gemm_rows.hip) read these from all channels at once, which the library's do
     not. us streamed and by the library: 16 rows of 128256 x 4096 175 and 186,
     of 65536 x 2048 48 and 66, 32 of 32000 x 4096 46 and 63, 48 of it 52 and 64, 32
     of 28672 x 4096 45 and 54 (64 of it 53 and 53, of 16384 x 4096 35 and 32; 16
-    of 128256 x 8192 373 and 364, 32 of 64000 x 5120 129 and 112, of 62024 x 3584
-    88 and 79). From 33 rows on tiles of 4096 are faster still."""
-    if K in (2048, 4096) and (N > 65536 or M > 16 and N >= 24576):
+    of 128256 x 8192 373 and 364, 32 of 62024 x 3584 88 and 79). From 33 rows on
+    tiles of 4096 are faster still. Vocabularies, whose time by the library jumps
+    from size to size: 1 row of 128256 x 768 38 and 45, of 151936 x 3584 194 and
+    227, of 131072 x 3584 163 and 162 (16 of it 166 and 160, 1 of 131072 x 5120 232
+    and 227); 24 of 100352 x 1024 44 and 136, 32 of 66048 x 3584 104 and 110; 64 of
+    128256 x 2048 114 and 119."""
+    if N > 65536 and 768 <= K <= 4096:
+        return (M <= 8 or 16 < M <= 32
+                or K in (2048, 4096) and M <= (64 if K == 2048 else 48))
+    if K in (2048, 4096) and M > 16 and N >= 24576:
         return M <= 48
     return N <= 65536 if M <= 16 else M <= 64 and K >= 2 * N and N <= 8192
 
@@ -690,10 +697,21 @@ def _tiles_apart_pay(M: int, N: int, K: int) -> bool:
     41 and 53, 128 51 and 56, 61 of 128256 x 4096 183 and 209, 128 191 and 234, of
     57344 x 8192 164 and 184 (80 of 37888 x 4096 80 and 72, 33 of 28672 x 8192 110
     and 100; 64 of 20480 x 4096 47 and 41, of 12288 x 4096 26 and 25). Up to 32 rows
-    while there is a tile of 128 columns a CU, else streamed (24 of 28672 x 4096 40
-    and streamed 47, of 100352 x 4096 197 and 153)."""
-    return (K % 4096 == 0 and N >= 24576 and 16 < M <= ROWS_MAX_M
-            and (M > 32 or K == 4096 and N <= 32768))
+    where tiles of 128 columns leave at most 96 of 256 CUs idle in their last round,
+    else streamed (24 of 28672 x 4096 40 and streamed 47, of 57344 x 4096 83 and
+    94, of 128256 x 4096 182 and 186, but of 81920 x 4096 147 and 122, of 114688 x
+    4096 206 and 166). Vocabularies of other rows likewise (32 of 128256 x 3584 156,
+    streamed 174, library 180; 24 of 100352 x 3584 148, 142 and 172) but for those
+    4 KB apart (128256 x 2048 115 and streamed 97), and from 33 rows on while the
+    inner dimension is short (64 of 151936 x 1536 101, library 111; 48 of 131072 x
+    2560 130 and 127, of 100352 x 3072 129 and 119)."""
+    if not 16 < M <= ROWS_MAX_M:
+        return False
+    full = (N // -128) % 256 <= 96
+    if N > 65536 and 768 <= K < 4096:
+        return K != 2048 and full if M <= 32 else K <= 1536
+    return (K % 4096 == 0 and N >= 24576
+            and (M > 32 or K == 4096 and full))
 
 
 def _tiles_pay(M: int, N: int, K: int) -> bool:

@@ -354,7 +354,15 @@ def test_tiles_pay(M, N, K, pay):
     (49, 24576, 2048, "library"), (48, 24568, 2048, "library"),
     (128, 24576, 8192, "tiles"), (32, 28672, 8192, "library"),
     (128, 24568, 4096, "library"), (129, 24568, 4096, "tiles"),
-    (61, 37888, 3584, "library")])
+    (61, 37888, 3584, "library"),
+    # vocabularies
+    (8, 65537, 768, "stream"), (9, 65537, 768, "library"),
+    (8, 65537, 5120, "library"), (8, 65537, 512, "library"),
+    (17, 128256, 3584, "tiles"), (32, 86016, 768, "tiles"),
+    (32, 85888, 768, "stream"), (32, 81920, 4096, "stream"),
+    (32, 128256, 4096, "tiles"), (33, 128256, 2560, "library"),
+    (128, 100352, 1536, "tiles"), (64, 128256, 2048, "stream"),
+    (65, 128256, 2048, "library"), (17, 128256, 5120, "library")])
 def test_wide_products(M, N, K, way):
     """Streamed, by tiles or by the library, on either side of the lines."""
     tiles = M > 16 and (ops._tiles_pay(M, N, K)
