@@ -9,9 +9,18 @@
 //    stands between loads. Keys go straight from their pages into MFMA
 //    operands (scores key x query); they are permuted so that lane group hi
 //    ends up with the scores of the 8 keys whose values it loads itself. The
-//    query columns repeat every four lanes, so a weight of another head is a
-//    quad broadcast away and the value product runs in fp32 on whole 16-byte
-//    rows, without a transpose and without rounding the weights.
+//    query columns repeat every four lanes.
+//  - From four heads on the value product runs on matrix instructions without
+//    rounding the weights: a lane of each four has a head's weight in one of three
+//    bf16 parts that add up to its 24 bits, so the 16 rows of an operand are four
+//    heads in all parts, and a sum's are added at the end. Values meet them as
+//    columns of 8 keys, which takes an instruction for every two. Up to two heads
+//    the product runs in fp32, a weight of another head a quad broadcast away.
+//    In fp32 it was most of a tile's instructions and kept e4m3 and eight heads
+//    from the rate of the memory; us before and now: 64 heads on 8, 16 of 100..6000 53 and 49, e4m3 45 and 39, heads of 64
+//    33 and 28, e4m3 28 and 23; 32 on 8 of 128, 61 of 1000..4096 118.8 and 117.0,
+//    e4m3 75.7 and 72.0, 512 of 513..640 e4m3 115.6 and 112.4. Distance from 64 bits
+//    the same (1.66e-3, the rounding of results, of which 1 in 4000 differs).
 //  - The next tile's keys are under way during softmax and value product, its
 //    values during the next scores; page numbers are read a tile earlier.
 //  - Work is cut by the lengths themselves, on the device, because a captured
@@ -24,10 +33,10 @@
 // heads. Measured with 32 heads on 8, 16-token pages in random order, merge
 // included (us before -> now, TB/s now):
 //   1 row of 777            22.5 -> 10.0      (launches and latency)
-//   8 of 300..6000, window  89 -> 31          3.3
-//   61 of 1000..4096        345 -> 127        5.0
-//   512 of 513..640         279 -> 209        5.8
-//   24 of 4000..16000, fp8  487 -> 113        4.5
+//   8 of 300..6000, window  89 -> 25          3.5
+//   61 of 1000..4096        345 -> 117        5.3
+//   512 of 513..640         279 -> 193        6.2
+//   24 of 4000..16000, fp8  487 -> 99         5.0
 // Values by ordinary loads: 133 us for the 61, 226 for the 512; keys by
 // streaming loads as well: 128 and 218.
 // A large read-only sum reaches 6.1 TB/s. TARGET of 512 to 2048 is within 5%
@@ -167,6 +176,13 @@ template <int BYTES> struct Raw;
 template <> struct Raw<4> { typedef uint32_t T; };
 template <> struct Raw<8> { typedef u32x2 T; };
 template <> struct Raw<16> { typedef u32x4 T; };
+template <typename R>
+__device__ __forceinline__ uint32_t word_of(const R& row, int i) {
+  if constexpr (sizeof(R) == 4)
+    return row;
+  else
+    return row[i];
+}
 
 template <bool F8, int DPL>
 __device__ __forceinline__ void widen(const void* raw, float* v) {
@@ -220,6 +236,37 @@ __device__ __forceinline__ void rescale(float (*acc)[DPL], const float* c) {
   }
 }
 
+// Weights as three bf16 that add up to all their 24 bits: a lane's part is what the
+// parts before it leave.
+__device__ __forceinline__ float part_of(float w, bool second, bool third) {
+  auto lower = [](float v) {
+    return v - __uint_as_float(__float_as_uint(v) & 0xffff0000u);
+  };
+  const float a = lower(w);
+  w = second ? a : w;
+  const float b = lower(a);
+  return third ? b : w;
+}
+// The upper (lower) halves of two words.
+__device__ __forceinline__ uint32_t uppers(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302);
+}
+__device__ __forceinline__ uint32_t lowers(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x05040100);
+}
+// Values 2 c and 2 c + 1 of a row.
+template <bool F8, typename R>
+__device__ __forceinline__ uint32_t two_values(const R& row, int c) {
+  if constexpr (F8) {
+    const uint32_t w = word_of(row, c >> 1);
+    return __builtin_bit_cast(
+        uint32_t, (c & 1) ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)
+                          : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false));
+  } else {
+    return word_of(row, c);
+  }
+}
+
 // What fits the registers without spilling.
 constexpr int waves_per_simd(int D, int G) {
   return D == 128 ? (G > 4 ? 2 : 3) : (G > 4 ? 3 : 4);
@@ -241,10 +288,20 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
   __shared__ float sh[NW][G][D];
   __shared__ float st[2][NW][G];
 
-  const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lo = lane & 15, hi = lane >> 4;
   int seq, part, parts;
   if (!find(m, seq, part, parts)) return;
+  // The same in all lanes: scalar registers, so that a wave more fits a SIMD. Not
+  // for up to four heads of bf16, which have waves enough and lose by more (32
+  // heads of 64 on 8, 16 of 100..6000 24 us and 26; 16 on 16 of 128, 1 of 900
+  // 13.4 and 15.7; e4m3 of the first 20.5 and 19.4).
+  if constexpr (F8 || G > 4) {
+    seq = __builtin_amdgcn_readfirstlane(seq);
+    part = __builtin_amdgcn_readfirstlane(part);
+    parts = __builtin_amdgcn_readfirstlane(parts);
+  }
   const int g = blockIdx.y, Hq = m.Hkv * G;
   const int len = len_of(m, seq), first = first_key(m, len);
   const int tile0 = first / KT, tiles = max(0, cdiv(len, KT) - tile0);
@@ -319,11 +376,20 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
           row[i % VG] + (i / VG) * D * EB));
   };
 
-  float acc[G][DPL], m_run[QS], l[QS];
+  // from four heads on by matrix instructions: rows are 4 heads in each of the
+  // weights' parts, columns the dimensions lo DPL + d
+  constexpr bool MMA = G >= 4;
+  float acc[MMA ? 1 : G][DPL], m_run[QS], l[QS];
+  floatx4 sum[QS][MMA ? DPL : 1];
 #pragma unroll
-  for (int j = 0; j < G; ++j)
+  for (int d = 0; d < DPL; ++d) {
 #pragma unroll
-    for (int d = 0; d < DPL; ++d) acc[j][d] = 0.f;
+    for (int j = 0; j < (MMA ? 1 : G); ++j) acc[j][d] = 0.f;
+    if constexpr (MMA)
+#pragma unroll
+      for (int s = 0; s < QS; ++s) sum[s][d] = floatx4{0, 0, 0, 0};
+  }
+  const bool second = lo >= 4, third = lo >= 8;
 #pragma unroll
   for (int s = 0; s < QS; ++s) {
     m_run[s] = LOWEST;
@@ -389,14 +455,58 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
       for (int i = 0; i < 8; ++i)
         vr[i] = key0 + i < first || key0 + i >= len ? VRaw(0) : vr[i];
     }
-    if (!__all(keep)) rescale<G, 0, DPL>(acc, corr);
+    if constexpr (MMA) {
+      if (!__all(keep)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float v[DPL];
-      widen<F8, DPL>(&vr[i], v);
-      add_values<G, 0, DPL>(acc, p[i], v);
-      // else all values are widened at once and registers run out
-      __builtin_amdgcn_sched_barrier(0);
+        for (int s = 0; s < QS; ++s) {
+          const floatx4 c = {quad<0>(corr[s]), quad<1>(corr[s]),
+                             quad<2>(corr[s]), quad<3>(corr[s])};
+#pragma unroll
+          for (int d = 0; d < DPL; ++d)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[s][d][r] *= c[r];
+        }
+      }
+      u32x4 w[QS];
+#pragma unroll
+      for (int s = 0; s < QS; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          w[s][i] = uppers(
+              __float_as_uint(part_of(p[2 * i][s], second, third)),
+              __float_as_uint(part_of(p[2 * i + 1][s], second, third)));
+#pragma unroll
+      for (int c = 0; c < DPL / 2; ++c) {
+        uint32_t two[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) two[i] = two_values<F8>(vr[i], c);
+        u32x4 even, odd;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          even[i] = lowers(two[2 * i], two[2 * i + 1]);
+          odd[i] = uppers(two[2 * i], two[2 * i + 1]);
+        }
+#pragma unroll
+        for (int s = 0; s < QS; ++s) {
+          const bf16x8 ws = __builtin_bit_cast(bf16x8, w[s]);
+          sum[s][2 * c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              ws, __builtin_bit_cast(bf16x8, even), sum[s][2 * c], 0, 0, 0);
+          sum[s][2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              ws, __builtin_bit_cast(bf16x8, odd), sum[s][2 * c + 1], 0, 0, 0);
+        }
+        // else all values are widened at once and registers run out
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      if (!__all(keep)) rescale<G, 0, DPL>(acc, corr);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float v[DPL];
+        widen<F8, DPL>(&vr[i], v);
+        add_values<G, 0, DPL>(acc, p[i], v);
+        // else all values are widened at once and registers run out
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     load_v(more ? t + NW : t);
     pages(min(t + 2 * NW, t_end - 1));
@@ -415,8 +525,16 @@ __global__ __launch_bounds__(NT, waves_per_simd(D, G)) void paged_rows_kernel(
   for (int j = 0; j < G; ++j)
 #pragma unroll
     for (int d = 0; d < DPL; ++d) {
-      const float v = sum_over_groups(acc[j][d]);
-      if (hi == (j & 3)) sh[wid][j][lo * DPL + d] = v;
+      if constexpr (MMA) {
+        // the parts; infinite values count by the first, as a later one may be 0
+        const float first = sum[j >> 2][d][j & 3];
+        const float all = sum_over_groups(hi < 3 ? first : 0.f);
+        if (hi == 0)
+          sh[wid][j][lo * DPL + d] = fabsf(first) <= FLT_MAX ? all : first;
+      } else {
+        const float v = sum_over_groups(acc[j][d]);
+        if (hi == (j & 3)) sh[wid][j][lo * DPL + d] = v;
+      }
     }
   __syncthreads();
   for (int i = threadIdx.x; i < G * D; i += NT) {

@@ -864,6 +864,38 @@ def test_paged_attn_decode_pages_given_back(window, n, bs):
                                atol=5e-5)
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (8, 1, 64), (4, 2, 64)])
+@pytest.mark.parametrize("n", [31, 400])
+def test_paged_attn_decode_infinite_values(hq, hkv, d, n):
+    """Infinite values come out as such, of either sign, and both as no number,
+    whatever parts a weight is taken in; the other dimensions are untouched."""
+    torch.manual_seed(60)
+    nb = -(-n // 16)
+    k = torch.zeros(nb, hkv, 16, d, dtype=torch.bfloat16, device=DEV)
+    v = torch.randn(nb, hkv, 16, d, dtype=torch.bfloat16, device=DEV)
+    inf = float("inf")
+    v[0, :, 3, 1], v[1, :, 5, 6], v[1, :, 2, 1] = inf, -inf, inf
+    v[0, :, 4, d - 1], v[1, :, 4, d - 1] = inf, -inf
+    # scores of 0 and a little: weights of one bit, and of all their bits
+    k[0, :, 4:, 0] = 0.37
+    q = torch.zeros(2, hq, d, dtype=torch.bfloat16, device=DEV)
+    q[1, :, 0] = -1.3
+    bt = torch.arange(nb, device=DEV, dtype=torch.int32).expand(2, nb)
+    out = ops.paged_attn_decode(
+        q, k, v, bt.contiguous(),
+        torch.full((2,), n, dtype=torch.int32, device=DEV), d ** -0.5,
+        ops.decode_workspace(2, hq, d, 512, DEV), 512)
+    assert (out[..., 1] == inf).all() and (out[..., 6] == -inf).all()
+    assert out[..., d - 1].isnan().all()
+    rest = [c for c in range(d) if c not in (1, 6, d - 1)]
+    keys, values = [t.transpose(1, 2).reshape(nb * 16, hkv, d)[:n].double()
+                    .repeat_interleave(hq // hkv, 1) for t in (k, v)]
+    w = ((q.double()[:, None] * keys).sum(-1) * d ** -0.5).softmax(1)
+    want = (w[..., None] * values[..., rest]).sum(1)
+    torch.testing.assert_close(out[..., rest].double(), want, rtol=2 ** -8,
+                               atol=1e-5)
+
+
 @pytest.mark.parametrize("max_len", [300, 4096])
 def test_paged_attn_decode_large_scores(max_len):
     """Scores of some -2^126, of -inf for some keys or for all, and no keys."""
