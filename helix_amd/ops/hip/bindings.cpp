@@ -24,12 +24,13 @@ bool image_tokens(torch::Tensor x, torch::Tensor cond, torch::Tensor cu,
 bool time_embed(torch::Tensor out, torch::Tensor t);
 c10::optional<torch::Tensor> text_block(
     torch::Tensor x, torch::Tensor cu, int64_t max_len, int64_t heads,
-    double scale, double eps, std::vector<torch::Tensor> p);
+    double scale, double eps, std::vector<c10::optional<torch::Tensor>> p);
 std::vector<torch::Tensor> image_block(
     torch::Tensor x, c10::optional<torch::Tensor> y,
     c10::optional<torch::Tensor> gate, c10::optional<torch::Tensor> y_bias,
     torch::Tensor mod, torch::Tensor cu, int64_t L, int64_t heads,
-    double scale, double eps, std::vector<torch::Tensor> p, bool stretches);
+    double scale, double eps, std::vector<c10::optional<torch::Tensor>> p,
+    bool stretches);
 bool gated_add(torch::Tensor out, torch::Tensor x, torch::Tensor y,
                torch::Tensor gate, int64_t L);
 bool norm_in_registers(int64_t rows, int64_t columns);
@@ -107,7 +108,7 @@ torch::Tensor gemm_rows_sums(torch::Tensor x, torch::Tensor w, OptT x_scale,
                              OptT w_scale);
 std::vector<torch::Tensor> gemm_rows_many(torch::Tensor x,
                                           std::vector<torch::Tensor> ws,
-                                          std::vector<torch::Tensor> biases);
+                                          std::vector<OptT> biases);
 void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    OptT x_scale, OptT w_scale);
 void quantize_rows(torch::Tensor out, torch::Tensor scales, torch::Tensor x);

@@ -12,6 +12,7 @@
 
 using OptT = c10::optional<torch::Tensor>;
 using Tensors = std::vector<torch::Tensor>;
+using OptTs = std::vector<OptT>;
 
 // of gemm_bf16.hip, gemm_rows.hip, attn_prefill.hip and encoder.hip
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
@@ -36,6 +37,16 @@ bool packed(const torch::Tensor& t, const torch::Tensor& x,
   return t.scalar_type() == torch::kBFloat16 && t.device() == x.device() &&
          t.sizes() == sizes && t.is_contiguous() &&
          (uintptr_t)t.data_ptr() % 16 == 0;
+}
+// The first n of p: none where one of them is missing (a bias that is None).
+Tensors present(const OptTs& p, size_t n) {
+  if (p.size() < n) return {};
+  Tensors all;
+  for (size_t i = 0; i < n; ++i) {
+    if (!p[i].has_value()) return {};
+    all.push_back(*p[i]);
+  }
+  return all;
 }
 bool layer(const Tensors& p, size_t i, const torch::Tensor& x, int64_t out,
            int64_t in) {
@@ -99,8 +110,11 @@ bool rows_of(const torch::Tensor& x, const torch::Tensor& cu, int64_t heads) {
 // p: weight and bias of q k v, attention's end, its norm, the way up, the way down,
 // the last norm.
 OptT text_block(torch::Tensor x, torch::Tensor cu, int64_t max_len,
-                int64_t heads, double scale, double eps, Tensors p) {
-  if (p.size() != 12 || !rows_of(x, cu, heads) || p[6].dim() != 2) return {};
+                int64_t heads, double scale, double eps, OptTs params) {
+  const Tensors p = present(params, 12);
+  if (p.empty() || params.size() != 12 || !rows_of(x, cu, heads) ||
+      p[6].dim() != 2)
+    return {};
   const int64_t H = x.size(1), I = p[6].size(0);
   if (I < 1 || I % 64 != 0 || !layer(p, 0, x, 3 * H, H) ||
       !layer(p, 2, x, H, H) || !layer(p, 6, x, I, H) || !layer(p, 8, x, H, I))
@@ -127,9 +141,10 @@ OptT text_block(torch::Tensor x, torch::Tensor cu, int64_t max_len,
 // may be in such.
 Tensors image_block(torch::Tensor x, OptT y, OptT gate, OptT y_bias,
                     torch::Tensor mod, torch::Tensor cu, int64_t L,
-                    int64_t heads, double scale, double eps, Tensors p,
+                    int64_t heads, double scale, double eps, OptTs params,
                     bool stretches) {
-  if (p.size() < 8 || !rows_of(x, cu, heads) || p[4].dim() != 2) return {};
+  const Tensors p = present(params, 8);
+  if (p.empty() || !rows_of(x, cu, heads) || p[4].dim() != 2) return {};
   const int64_t T = x.size(0), H = x.size(1), I = p[4].size(0);
   if (I < 1 || I % 64 != 0 || L < 1 || T % L != 0 ||
       !packed(mod, x, {T / L, 6 * H}) || !layer(p, 0, x, 3 * H, H) ||

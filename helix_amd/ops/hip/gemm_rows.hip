@@ -402,7 +402,7 @@ void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 // 91 us -> 31.
 std::vector<torch::Tensor> gemm_rows_many(torch::Tensor x,
                                           std::vector<torch::Tensor> ws,
-                                          std::vector<torch::Tensor> biases) {
+                                          std::vector<OptT> biases) {
   std::vector<torch::Tensor> outs;
   auto reads = [&](const torch::Tensor& t, int64_t to) {
     return t.scalar_type() == torch::kBFloat16 && t.device() == x.device() &&
@@ -415,8 +415,9 @@ std::vector<torch::Tensor> gemm_rows_many(torch::Tensor x,
   int64_t width = 0;
   for (size_t i = 0; i < ws.size(); ++i) {
     if (ws[i].dim() != 2 || ws[i].size(1) != x.size(1) || !reads(ws[i], 16) ||
-        biases[i].dim() != 1 || biases[i].size(0) != ws[i].size(0) ||
-        !reads(biases[i], 2))
+        (biases[i].has_value() &&
+         (biases[i]->dim() != 1 || biases[i]->size(0) != ws[i].size(0) ||
+          !reads(*biases[i], 2))))
       return outs;
     width = std::gcd(width, ws[i].size(0));
   }
@@ -441,7 +442,8 @@ std::vector<torch::Tensor> gemm_rows_many(torch::Tensor x,
     for (int64_t c = 0; c < N; c += width) {
       auto& one = many.at[n++];
       one.w = (const uint16_t*)ws[i].data_ptr() + c * x.size(1);
-      one.bias = (const uint16_t*)biases[i].data_ptr() + c;
+      one.bias = biases[i].has_value()
+                     ? (const uint16_t*)biases[i]->data_ptr() + c : nullptr;
       one.out = (uint16_t*)outs[i].data_ptr() + c;
       one.ld = N;
       if (n == Many::MOST) launch();

@@ -389,3 +389,16 @@ def test_attn_prefill_refuses(case, says):
         cu_k = cu[:2]
     with pytest.raises(RuntimeError, match=says):
         ops._native().attn_prefill(out, q, k, v, cu, cu_k, 5, 0.125, True, 0)
+
+
+@pytest.mark.parametrize("gone", range(12))
+def test_blocks_without_a_bias_go_step_by_step(gone):
+    """A parameter that is None is a form that the calls decline, not an
+    argument that they refuse."""
+    x, cu = torch.zeros(4, 64, dtype=torch.bfloat16), torch.tensor([0, 4]).int()
+    params = [None if i == gone else x for i in range(12)]
+    native = ops._native()
+    assert native.text_block(x, cu, 4, 1, 1.0, 1e-6, params) is None
+    assert native.image_block(x, None, None, None, x, cu, 4, 1, 1.0, 1e-6,
+                              params[:10], True) == []
+    assert native.gemm_rows_many(x, [x, x], [x, None]) == []

@@ -414,6 +414,70 @@ def test_gemm_bf16_many(m, k, ns):
             rtol=2 ** -8, atol=2e-5)
 
 
+@pytest.mark.parametrize("m", [3, 65])
+def test_gemm_bf16_many_without_biases(m):
+    torch.manual_seed(58)
+    x = torch.randn(m, 256, dtype=torch.bfloat16, device=DEV)
+    ws = [torch.randn(n, 256, dtype=torch.bfloat16, device=DEV) / 16
+          for n in (192, 64, 128)]
+    bs = [None, torch.randn(64, dtype=torch.bfloat16, device=DEV), None]
+    got = ops.gemm_bf16_many(x, ws, bs)
+    if m <= 64:
+        for o, p in zip(got, ops._native().gemm_rows_many(x, ws, bs)):
+            assert torch.equal(o, p)
+    for o, w, b in zip(got, ws, bs):
+        want = x.double() @ w.double().t()
+        torch.testing.assert_close(o.double(),
+                                   want if b is None else want + b.double(),
+                                   rtol=2 ** -8, atol=2e-5)
+
+
+@pytest.mark.parametrize("name", ["qkv_b", "attn_out_b", "up_b", "down_b"])
+def test_text_layer_without_a_bias(name):
+    """The same as with zeros there."""
+    from helix_amd.models.bert import BertConfig, BertLayer
+    torch.manual_seed(59)
+    layer = BertLayer(BertConfig(hidden_size=128, intermediate_size=256,
+                                 num_heads=2)).to(torch.bfloat16).to(DEV)
+    for p in layer.parameters():
+        p.data.normal_(0.0, 0.1)
+    x = torch.randn(37, 128, dtype=torch.bfloat16, device=DEV)
+    cu = torch.tensor([0, 37], device=DEV).int()
+    with torch.inference_mode():
+        getattr(layer, name).data.zero_()
+        want = layer(x, cu, 37).double()
+        setattr(layer, name, None)
+        got = layer(x, cu, 37).double()
+    # sums that may be rounded to bf16 before their norm (2^-9)
+    assert (got - want).norm() < 2 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("name", ["qkv_b", "out_b", "up_b", "down_b", "mod_b",
+                                  "fin_mod_b"])
+def test_image_model_without_a_bias(name):
+    """The same as with zeros there."""
+    from dataclasses import replace
+    from helix_amd.models.dit import DIT_PRESETS, DiTModel
+    torch.manual_seed(60)
+    cfg = replace(DIT_PRESETS["flux-lite"], depth=2, vocab_size=64, hidden=256,
+                  heads=4)
+    model = DiTModel(cfg).to(torch.bfloat16).to(DEV)
+    for p in model.parameters():
+        p.data.normal_(0.0, 0.1)
+    of = model if hasattr(model, name) else model.blocks[1]
+    args = (torch.randn(2, cfg.latent_ch, cfg.latent_size, cfg.latent_size,
+                        device=DEV), torch.tensor([0.25, 0.75], device=DEV),
+            torch.randint(0, 64, (2, cfg.text_len), device=DEV))
+    with torch.inference_mode():
+        getattr(of, name).data.zero_()
+        want = model(*args).double()
+        setattr(of, name, None)
+        got = model(*args).double()
+    # of a block that goes step by step, three sums are rounded to bf16 before
+    # their norms
+    assert (got - want).norm() < 3 * 2 ** -8 * want.norm()
+
+
 def test_gemm_bf16_many_forms():
     """What the one launch does not read goes as a product each."""
     torch.manual_seed(57)
