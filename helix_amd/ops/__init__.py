@@ -858,7 +858,7 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear_silu_mul where that is the faster form, product and activation
     apart elsewhere. From 33 rows on by tiles, whose halves meet before they are
     rounded: in one launch (us apart and now: 64 rows of 28672 x 4096 56 and 46,
-    512 107 and 93, 8192 1407 and 1246), from 17 on where tiles of wide matrices
+    512 107 and 95, 8192 1407 and 1249), from 17 on where tiles of wide matrices
     begin apart (ring_turn in gemm_ring.h; us streamed and by tiles: 17 of 28672 x
     4096 43.8 and 43.6, 24 45.2 and 43.5, 32 46.9 and 43.8, of 26624 x 4096 46.4
     and 39.7, of 32768 x 4096 49.0 and 48.6, but 24 47.9 and 48.4), and where

@@ -2,6 +2,8 @@
 
 All marked `gpu`; run on an MI355X via gpurun. Tolerances are bf16-scale.
 """
+import math
+
 import pytest
 import torch
 
@@ -1335,6 +1337,29 @@ def test_gated_few_rows(m, n, k, tiles):
     # fp32 sums of k products, then the rounding to bf16
     torch.testing.assert_close(got.double(), torch.nn.functional.silu(g) * u,
                                rtol=2 ** -8, atol=5e-5)
+
+
+@pytest.mark.parametrize("k", [256, 16384])
+def test_gated_over_the_range_of_silu(k):
+    """By tiles and, deep, by stretches: gates down to where e^-v leaves 32 bits,
+    subnormal reciprocals among them, and those that are not finite."""
+    gates = torch.cat([torch.arange(-88.5, -87, 0.5), torch.arange(-87., 128.),
+                       torch.tensor([-0.5, 1e-3, -1e30, 1e18, math.inf,
+                                     -math.inf, math.nan])]).bfloat16()
+    n, m = 256, 100
+    x = torch.zeros(m, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(2 * n, k, dtype=torch.bfloat16, device=DEV)
+    x[:, 5] = 1
+    w[:len(gates), 5], w[n:, 5] = gates.to(DEV), 2. ** 64
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    assert (ops._native().gemm_bf16_glu_plan(m, n, k)[1] > 1) == (k > 256)
+    ops._native().gemm_bf16_glu(out, x, w)
+    g, u = w[:n, 5].double(), 2. ** 64
+    # the exponent of up to 2^7 in 32 bits (2^-17), the rounding to bf16
+    torch.testing.assert_close(out[0].double(), g / (1 + torch.exp(-g)) * u,
+                               rtol=2 ** -8, atol=0, equal_nan=True)
+    assert all(torch.equal(a[~a.isnan()], b[~b.isnan()])
+               for a, b in zip(out, out[:1].expand(m, n)))
 
 
 @pytest.mark.parametrize("m", [1, 5, 16, 31, 48, 49, 128])
