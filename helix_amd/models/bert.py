@@ -107,7 +107,9 @@ class BertEmbeddingModel(nn.Module):
     @torch.inference_mode()
     def forward(self, input_ids: torch.Tensor, cu_seqlens: torch.Tensor,
                 max_len: int) -> torch.Tensor:
-        """input_ids: [T] varlen concat; returns [B, H] L2-normalized."""
+        """input_ids: [T] varlen concat; returns [B, H] L2-normalized. A text
+        longer than the table of places is refused; on GPU an id outside the
+        vocabulary, which the host doesn't see, makes its text's result NaN."""
         T = input_ids.shape[0]
         # one read by the host, for the checks and the mean's bounds
         cu = cu_seqlens.tolist()
@@ -116,6 +118,10 @@ class BertEmbeddingModel(nn.Module):
             raise ValueError(f"boundaries {cu} do not cut {T} tokens")
         if self.cfg.pooling != "mean" and cu[-2] == T:
             raise IndexError("a last text without tokens")
+        if _plain(self.pos_emb):
+            places = self.pos_emb.weight.shape[0]
+            if any(b - a > places for a, b in zip(cu, cu[1:])):
+                raise IndexError(f"a text of more than {places} tokens")
         x = None
         if _plain(self.word_emb) and _plain(self.pos_emb):
             x = ops.text_embed(input_ids, cu_seqlens, self.word_emb.weight,

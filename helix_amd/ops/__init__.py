@@ -157,8 +157,9 @@ def gated_add(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor,
 
 def text_embed(ids: torch.Tensor, cu: torch.Tensor, word: torch.Tensor,
                pos: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float):
-    """Layer norm of word[ids] + pos[place within the text], or None for other
-    forms than the kernel reads (the CPU's among them)."""
+    """Layer norm of word[ids] + pos[place within the text], NaN where either is
+    outside its table, or None for other forms than the kernel reads (the CPU's
+    among them)."""
     if ids.is_cuda and word.dim() == 2:
         out = torch.empty(ids.shape[0], word.shape[1], dtype=torch.bfloat16,
                           device=ids.device)

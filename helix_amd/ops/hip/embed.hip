@@ -44,8 +44,8 @@ struct Text {
   float eps;
 };
 
-// Norm of word + position, a wave to a token; NV: vectors of 8 that a lane has.
-// Rows of tables beyond their end are those at it.
+// Norm of word + position, a wave to a token; NV: vectors of 8 that a lane has. A
+// word or place outside its table reads a row that is there and gives no number.
 template <int NV>
 __global__ __launch_bounds__(NT) void text_embed_kernel(Text m) {
   const int t = blockIdx.x * (NT / WAVE) + threadIdx.x / WAVE;
@@ -58,9 +58,11 @@ __global__ __launch_bounds__(NT) void text_embed_kernel(Text m) {
     if (n < WAVE) break;
   }
   const int at = t - m.cu[min(seq, m.B - 1)];
-  const uint16_t* word = m.word + (int64_t)clamp_to(m.ids[t], m.V) * m.H;
+  const int64_t id = m.ids[t];
+  const bool known = id >= 0 && id < m.V && at >= 0 && at < m.P;
+  const uint16_t* word = m.word + (int64_t)clamp_to(id, m.V) * m.H;
   const uint16_t* pos = m.pos + (int64_t)clamp_to(at, m.P) * m.H;
-  float v[NV][8], total = 0.f;
+  float v[NV][8], total = known ? 0.f : __builtin_nanf("");
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (i * WAVE + lane) * 8;

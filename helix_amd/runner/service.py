@@ -276,6 +276,9 @@ class EmbeddingInstance:
         for ids in ids_list:
             flat.extend(ids)
             cu.append(cu[-1] + len(ids))
+        if flat and not 0 <= min(flat) <= max(flat) < cfg.vocab_size:
+            raise IndexError(f"a token outside a vocabulary of "
+                             f"{cfg.vocab_size}")
         with self.lock:
             ids_t = torch.tensor(flat, dtype=torch.int64, device=self.device)
             cu_t = torch.tensor(cu, dtype=torch.int32, device=self.device)

@@ -167,28 +167,55 @@ def test_add_norm_strides():
 @pytest.mark.parametrize("h", [8, 520, 768, 4096])
 def test_text_embed_and_pool(lens, h):
     """Texts without tokens among others, more texts than a wave has lanes,
-    places and words past the end of their tables."""
+    places and words outside their tables, which are no number."""
     torch.manual_seed(61)
     T = sum(lens)
     cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
     ids = torch.randint(0, 50, (T,), device=DEV)
-    ids[-1] = 77
+    ids[-1], ids[T // 2] = 50, -1
     word, pos = (torch.randn(n, h, dtype=torch.bfloat16, device=DEV)
                  for n in (50, 150))
     w, b = torch.randn(2, h, dtype=torch.bfloat16, device=DEV)
     place = torch.cat([torch.arange(n, device=DEV) for n in lens])
-    x = word[ids.clamp(max=49)] + pos[place.clamp(max=149)]
+    x = word[ids.clamp(0, 49)] + pos[place.clamp(max=149)]
     want = torch.nn.functional.layer_norm(
         x.double(), (h,), w.double(), b.double(), 1e-12)
+    want[(ids < 0) | (ids >= 50) | (place >= 150)] = math.nan
     got = ops.text_embed(ids, cu, word, pos, w, b, 1e-12)
     # 32-bit sums of h values, then the rounding to bf16 (2^-9, doubled)
-    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2e-5)
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2e-5,
+                               equal_nan=True)
     if lens[-1] == 0:
         return
     first = got[cu[:-1].long()].double()
     torch.testing.assert_close(
         ops.text_pool(got, cu).double(),
-        torch.nn.functional.normalize(first, dim=-1), rtol=1e-5, atol=1e-7)
+        torch.nn.functional.normalize(first, dim=-1), rtol=1e-5, atol=1e-7,
+        equal_nan=True)
+
+
+@pytest.mark.parametrize("bad", [-1, 512, 1 << 40])
+def test_text_outside_its_tables(bad):
+    """No number for the text with such a word, and for no other; a text too
+    long is refused."""
+    from helix_amd.models.bert import BERT_PRESETS, BertEmbeddingModel
+    cfg = BERT_PRESETS["tiny-bert"]
+    model = BertEmbeddingModel(cfg).to(torch.bfloat16).to(DEV).init_random(1)
+    assert cfg.vocab_size == 512
+    lens = [5, 40, 7]
+    ids = torch.randint(0, 512, (sum(lens),), device=DEV)
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    want = model(ids, cu, 40)
+    ids[20] = bad
+    got = model(ids, cu, 40)
+    assert got[1].isnan().all()
+    assert torch.equal(got[::2], want[::2]) and not want.isnan().any()
+    long = torch.zeros(cfg.max_position + 1, dtype=torch.int64, device=DEV)
+    with pytest.raises(IndexError, match="more than"):
+        model(long, torch.tensor([0, len(long)], device=DEV).int(), len(long))
+    assert not model(long[1:], torch.tensor([0, len(long) - 1],
+                                            device=DEV).int(),
+                     len(long) - 1).isnan().any()
 
 
 @pytest.mark.parametrize("B,C,S,p,text,h", [(1, 4, 32, 2, 32, 1024),

@@ -281,6 +281,23 @@ def test_runner_metrics_endpoint():
         svc.shutdown()
 
 
+@pytest.mark.parametrize("bad", [-1, 512])
+def test_embedding_of_a_token_outside_the_vocabulary(bad):
+    """Refused on the host, on every device."""
+    from helix_amd.runner.service import EmbeddingInstance
+    inst = EmbeddingInstance(ModelSpec("tiny-bert", "embedding", "tiny-bert"),
+                             "cpu")
+    assert inst.model.cfg.vocab_size == 512 and len(inst.embed(["a", "b"])) == 2
+
+    class Tokens:
+        def encode(self, text):
+            return [1, bad, 2]
+
+    inst.tokenizer = Tokens()
+    with pytest.raises(IndexError, match="vocabulary"):
+        inst.embed(["a"])
+
+
 def test_vision_embeddings_instance():
     """SigLIP2-role image embedder (reference kodit vision path):
     base64/data-URL images embed to stable normalized vectors through
