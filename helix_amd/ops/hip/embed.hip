@@ -120,7 +120,8 @@ __global__ __launch_bounds__(NT) void text_pool_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j) square += v[j] * v[j];
   }
-  const float length = fmaxf(sqrtf(wave_reduce_sum(square)), 1e-12f);
+  const float root = sqrtf(wave_reduce_sum(square));
+  const float length = root < 1e-12f ? 1e-12f : root;     // NaN stays NaN
   for (int c = lane * 8; c < H; c += WAVE * 8) {
     float v[8];
     load_bf16x8(row + c, v);

@@ -194,6 +194,21 @@ def test_text_embed_and_pool(lens, h):
         equal_nan=True)
 
 
+def test_text_pool_of_odd_rows():
+    """Rows with a NaN, with infinities, of zeros and next to it, as torch's
+    normalize has them."""
+    x = torch.randn(5, 768, device=DEV).bfloat16()
+    x[0, 700] = math.nan
+    x[1, 3], x[1, 9] = math.inf, -math.inf
+    x[2] = 0
+    x[3] = 1e-15
+    cu = torch.arange(6, dtype=torch.int32, device=DEV)
+    torch.testing.assert_close(
+        ops.text_pool(x, cu),
+        torch.nn.functional.normalize(x.float(), dim=-1), rtol=1e-5,
+        atol=1e-7, equal_nan=True)
+
+
 @pytest.mark.parametrize("bad", [-1, 512, 1 << 40])
 def test_text_outside_its_tables(bad):
     """No number for the text with such a word, and for no other; a text too
