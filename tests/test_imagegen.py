@@ -168,15 +168,15 @@ def test_dit_generate_gpu():
 @pytest.mark.parametrize("images", [1, 3])
 def test_dit_blocks_apart_gpu(images):
     """A hook on one block sees its result; the velocity is that of sums taken
-    by the next norm, but for the roundings of those to bf16 (2^-9 of each, over
-    12 blocks)."""
+    by the next norm, but for the roundings of those to bf16: 2^-9 of each of two
+    in 3 blocks. A bias of the blocks that is lost changes it by 8% and more."""
     from dataclasses import replace
     from helix_amd.models.dit import DiTModel
     cfg = replace(DIT_PRESETS["flux-lite"], depth=3, vocab_size=512)
     torch.manual_seed(5)
     m = DiTModel(cfg).to(torch.bfloat16).to("cuda")
     for p in m.parameters():
-        p.data.normal_(0.0, 0.02)
+        p.data.normal_(0.0, p.shape[1] ** -0.5 if p.dim() == 2 else 1.0)
     args = (torch.randn(images, 4, 32, 32, device="cuda").bfloat16(),
             torch.full((images,), 0.75, device="cuda"),
             torch.randint(0, 512, (images, cfg.text_len), device="cuda"))
@@ -195,4 +195,4 @@ def test_dit_blocks_apart_gpu(images):
     assert len(seen) == 1 and seen[0].shape == (images * cfg.seq_len,
                                                 cfg.hidden)
     err = (whole - apart).double().norm() / apart.double().norm()
-    assert err < 12 * 2 ** -9
+    assert err < 6 * 2 ** -9
