@@ -827,15 +827,16 @@ def _sums_pay(M: int, N: int, K: int) -> bool:
 
 def _glu_fits(M: int, N: int, K: int) -> bool:
     """Whether the gated product of up to 64 rows takes no longer in one launch
-    than product and activation apart: up to 32 rows by streamed weights, which
+    than product and activation apart: up to 16 rows by streamed weights, which
     are not cut along the inner dimension and so need columns enough to fill the
-    chip, or few chunks; from 33 rows on, of more than 8192 columns, by tiles. us
-    apart and at once, with weights from memory: one row of 28672 x 4096 66 and
-    50, 10240 x 4096 28 and 29, 4096 x 4096 18 and 27, 16384 x 1024 12.3 and 10.2.
-    From 17 rows on x is read by every workgroup, and the library's product is the
-    faster one but for inner dimensions of a power of two: 17 of 28672 x 4096 62
-    and 51, 33 60 and 57, 64 61 and 58; 48 of 37888 x 3584 64 and 69, of 10240 x
-    8192 44 and 53. Widths that the activation alone does not take go here."""
+    chip, or few chunks; then by the same or by tiles (gated_linear). us apart and
+    at once, with weights from memory: one row of 28672 x 4096 59 and 42, 10240 x
+    4096 28 and 29, 4096 x 4096 18 and 27, 16384 x 1024 12.3 and 10.2. From 17 rows
+    on x is read by every workgroup, and the product apart is the faster one but
+    for rows of 4 or 8 KB, which the library's workgroups all read from the same
+    channels at once: 64 of 28672 x 4096 56 and 46; 48 of 37888 x 3584 64 and 69,
+    of 10240 x 8192 44 and 53. Widths that the activation alone does not take go
+    here."""
     if K <= 1024 or N % 16 != 0:
         return True
     if M <= 16:
@@ -865,9 +866,10 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     and 39.7, of 32768 x 4096 49.0 and 48.6, but 24 47.9 and 48.4), and where
     that leaves CUs idle, narrow or deep, in stretches that a second one adds up
     (apart, in one launch and now: 80 of 2048 x 8192 20, 43 and 15, 100 of 4096 x
-    14336 43, 79 and 37, 512 of 1024 x 16384 50, 90 and 30). Up to 64 rows of more than 8192 columns, where
-    _glu_fits does not take them, are bound by their weights and stay apart (48 of
-    10240 x 8192 53 in one launch, 44 apart; 64 of 14336 x 4096 36 and 31)."""
+    14336 43, 79 and 37, 512 of 1024 x 16384 50, 90 and 30). Up to 64 rows of more
+    than 8192 columns, where _glu_fits does not take them, are bound by their
+    weights and stay apart (48 of 10240 x 8192 53 in one launch, 44 apart; 64 of
+    14336 x 4096 36 and 31)."""
     apart = 16 if w.dim() == 2 and w.shape[1] % 4096 == 0 and \
         w.shape[0] > 8192 else 32
     if x.dim() == 2 and w.dim() == 2 and x.shape[0] > apart and \

@@ -479,8 +479,9 @@ bool ring_has(const int (&pairs)[N][2], const RingTile& t) {
 // and, with the reader of the stretches, 1.6% as sums (at worst 35%, 48 x 768 x
 // 768). The end of a gated tile with its SiLU as corrected (gelu.h) is 0.055, with
 // an exact division 0.064: 47 of 2900 sizes go by other tiles than with 0.035, which
-// is what the uncorrected one took, 1.7% faster in the mean (0.90 to 1.15). An item takes less while other CUs are idle; few workgroups do not reach
-// the rate of the memory.
+// is what the uncorrected one took, 1.7% faster in the mean (0.90 to 1.15). An item
+// takes less while other CUs are idle; few workgroups do not reach the rate of the
+// memory.
 struct RingCost {
   double busy, fed;
   double least() const { return 3.3 + std::max(busy, fed); }

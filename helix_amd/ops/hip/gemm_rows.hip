@@ -30,9 +30,10 @@
 //   M 32   14.4 (16.3)   9.3 (13.9)   46.8 (54.2)   24.9 (33.8)
 //   M 64   17.6 (18.0)  12.2 (15.2)   54.0 (52.3)   31.9 (41.9)
 // Tiles (gemm_ring.h) have taken over bf16 from 17 rows on, but for the stretches
-// of small products and of deep ones with few columns. From 65 rows on a wave has
-// 32 columns, so that x is read from LDS half as often, chunks are half as long
-// and 256 workgroups are enough:
+// of small products and of deep ones with few columns, up to 48 rows of wide
+// matrices and up to 64 of vocabularies whose rows are 4 or 8 KB (_streams_pay in
+// ops/__init__.py). From 65 rows on a wave has 32 columns, so that x is read from
+// LDS half as often, chunks are half as long and 256 workgroups are enough:
 //   M 128  20.0 (24.6)  15.5 (24.7)                   34.6 (73.9)
 // Adding them up in a launch, with bias and GELU, takes 2.5 to 3 us more; up to
 // 64 rows of small deep matrices of the encoder and the image model do so (8 of

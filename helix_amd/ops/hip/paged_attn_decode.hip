@@ -17,10 +17,11 @@
 //    columns of 8 keys, which takes an instruction for every two. Up to two heads
 //    the product runs in fp32, a weight of another head a quad broadcast away.
 //    In fp32 it was most of a tile's instructions and kept e4m3 and eight heads
-//    from the rate of the memory; us before and now: 64 heads on 8, 16 of 100..6000 53 and 49, e4m3 45 and 39, heads of 64
-//    33 and 28, e4m3 28 and 23; 32 on 8 of 128, 61 of 1000..4096 118.8 and 117.0,
-//    e4m3 75.7 and 72.0, 512 of 513..640 e4m3 115.6 and 112.4. Distance from 64 bits
-//    the same (1.66e-3, the rounding of results, of which 1 in 4000 differs).
+//    from the rate of the memory; us before and now: 64 heads on 8, 16 of
+//    100..6000 53 and 49, e4m3 45 and 39, heads of 64 33 and 28, e4m3 28 and 23;
+//    32 on 8 of 128, 61 of 1000..4096 118.8 and 117.0, e4m3 75.7 and 72.0, 512 of
+//    513..640 e4m3 115.6 and 112.4. Distance from 64 bits the same (1.66e-3, the
+//    rounding of results, of which 1 in 4000 differs).
 //  - The next tile's keys are under way during softmax and value product, its
 //    values during the next scores; page numbers are read a tile earlier.
 //  - Work is cut by the lengths themselves, on the device, because a captured
@@ -35,13 +36,14 @@
 //   1 row of 777            22.5 -> 10.0      (launches and latency)
 //   8 of 300..6000, window  89 -> 25          3.5
 //   61 of 1000..4096        345 -> 117        5.3
-//   512 of 513..640         279 -> 193        6.2
+//   512 of 513..640         279 -> 193        6.3
 //   24 of 4000..16000, fp8  487 -> 99         5.0
 // Values by ordinary loads: 133 us for the 61, 226 for the 512; keys by
 // streaming loads as well: 128 and 218.
-// A large read-only sum reaches 6.1 TB/s. TARGET of 512 to 2048 is within 5%
-// of each other; the results' distance from 64 bits is what it was (their
-// rounding to bf16).
+// The 512 take the same where every pass reads another of six caches of 1.2 GB, so
+// theirs is the rate of the memory. TARGET of 512 to 2048 is within 5% of each
+// other; the results' distance from 64 bits is what it was (their rounding to
+// bf16).
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
