@@ -188,9 +188,9 @@ class Attention(nn.Module):
         self.o_proj = HLinear(q, h, bias=False)
 
     def forward(self, x: torch.Tensor, cos_sin: torch.Tensor, kv_cache,
-                meta, form: str = "rows") -> torch.Tensor:
+                meta, form: str = "rows", join=None) -> torch.Tensor:
+        """join (residual, norm_w, eps): few rows, see DecoderLayer."""
         T = x.shape[0]
-        qkv = _project(self.qkv_proj, x, "sums")
         # fused strided split + rope + paged-cache write (one kernel, no
         # .contiguous() copies); compact K/V emitted only when the
         # fresh-prefill attention path consumes them directly
@@ -198,10 +198,14 @@ class Attention(nn.Module):
         prefill = meta.prefill if mixed else meta
         want_kv = meta.is_prefill and \
             getattr(prefill, "cu_seqlens_k", None) is None
-        q, k, v = ops.rope_qkv_cache(
-            meta.positions, qkv, cos_sin, self.nh, self.nkv, self.hd,
-            kv_cache=kv_cache, slot_mapping=meta.slot_mapping,
-            want_kv=want_kv)
+        heads = (cos_sin, self.nh, self.nkv, self.hd, kv_cache,
+                 meta.slot_mapping, want_kv)
+        if join is not None:
+            q, k, v = ops.rows_qkv(meta.positions, x, self.qkv_proj.weight,
+                                   self.qkv_proj.bias, *heads)
+        else:
+            q, k, v = ops.rope_qkv_cache(
+                meta.positions, _project(self.qkv_proj, x, "sums"), *heads)
         if mixed:
             n = meta.num_decode
             o = torch.empty_like(q)
@@ -214,6 +218,8 @@ class Attention(nn.Module):
         else:
             o = self._attend_decode(q, kv_cache, meta)
         o = o.view(T, -1)
+        if join is not None:
+            return ops.rows_join(o, self.o_proj.weight, *join)
         if self.tp_size > 1:
             from helix_amd import parallel
             return parallel.tp_all_reduce(self.o_proj(o))
@@ -250,8 +256,15 @@ class MLP(nn.Module):
         self.gate_up_proj = HLinear(cfg.hidden_size, 2 * i, bias=False)
         self.down_proj = HLinear(i, cfg.hidden_size, bias=False)
 
-    def forward(self, x: torch.Tensor, form: str = "rows") -> torch.Tensor:
-        h = _project(self.gate_up_proj, x, "glu")
+    def forward(self, x: torch.Tensor, form: str = "rows",
+                join=None) -> torch.Tensor:
+        """x Unscaled: few rows, see DecoderLayer; join as of Attention."""
+        if isinstance(x, ops.Unscaled):
+            h = ops.rows_glu(x, self.gate_up_proj.weight)
+        else:
+            h = _project(self.gate_up_proj, x, "glu")
+        if join is not None:
+            return ops.rows_join(h, self.down_proj.weight, *join)
         if self.tp_size > 1:
             from helix_amd import parallel
             return parallel.tp_all_reduce(self.down_proj(h))
@@ -274,15 +287,38 @@ class DecoderLayer(nn.Module):
         self.mlp = MLP(cfg, tp_size)
         self.eps = cfg.rms_norm_eps
 
+    def few(self, x) -> bool:
+        """Whether these rows go through the layer in launches that take norm,
+        rotation and residual along (layer_rows.hip): all of it is as written
+        here, and whole on this GPU."""
+        a, m = self.attn, self.mlp
+        if not (_own(a, Attention) and _own(m, MLP)
+                and a.tp_size == m.tp_size == 1):
+            return False
+        ps = (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj)
+        return (all(_own(p, HLinear) for p in ps)
+                and all(p.bias is None for p in ps[1:])
+                and ops._bias_fits(ps[0].bias, ps[0].weight)
+                and ops.layer_rows_fit(x, *(p.weight for p in ps), a.hd))
+
     def forward(self, x, residual, cos_sin, kv_cache, meta,
-                form: str = "rows"):
-        """form "sums": the result's stretches, for the next norm."""
+                form: str = "rows", few: bool = False, after=None):
+        """form "sums": the result's stretches, for the next norm. few: as few()
+        says; after (few): the weight of that norm, which the result then is but
+        for its division (ops.Unscaled)."""
         if residual is None:
             residual = x.clone()
             h = ops.rms_norm(x, self.input_norm_w, self.eps)
+        elif isinstance(x, ops.Unscaled):
+            h = x
         else:
             h, residual = _norm_for(self.attn, Attention, "qkv_proj")(
                 x, residual, self.input_norm_w, self.eps)
+        if few:
+            h = self.attn(h, cos_sin, kv_cache, meta,
+                          join=(residual, self.post_norm_w, self.eps))
+            join = None if after is None else (residual, after, self.eps)
+            return self.mlp(h, form, join), residual
         h = self.attn(h, cos_sin, kv_cache, meta,
                       *(["sums"] if _own(self.attn, Attention) else []))
         h, residual = _norm_for(self.mlp, MLP, "gate_up_proj")(
@@ -325,11 +361,16 @@ class LlamaForCausalLM(nn.Module):
     def forward(self, input_ids: torch.Tensor, kv_caches, meta) -> torch.Tensor:
         x = self.embed_tokens(input_ids)
         residual, own = None, True
+        few = [x.shape[0] <= ops.LAYER_ROWS and _own(layer, DecoderLayer)
+               and layer.few(x) for layer in self.layers] + [False]
         for i, layer in enumerate(self.layers):
             cache = kv_caches[i] if kv_caches is not None else None
             own = _own(layer, DecoderLayer)
-            x, residual = layer(x, residual, self.cos_sin, cache, meta,
-                                *(["sums"] if own else []))
+            extra = ["sums"] if own else []
+            if few[i]:
+                extra += [True, self.layers[i + 1].input_norm_w
+                          if few[i + 1] else None]
+            x, residual = layer(x, residual, self.cos_sin, cache, meta, *extra)
         if not own:                # what a hook has kept stays as it was
             x, residual = x.clone(), residual.clone()
         return ops.fused_add_rms_norm(x, residual, self.final_norm_w,

@@ -886,6 +886,82 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return linear_silu_mul(x, w)
 
 
+class Unscaled(NamedTuple):
+    """Rows times a norm's weight that are still to be divided by the root of
+    their mean square, which is eps and the mean of squares' sum over a row: what
+    multiplies them may do so last (layer_rows.hip)."""
+    rows: torch.Tensor                  # [M, H] bf16
+    squares: torch.Tensor               # [M, parts] fp32
+    eps: float
+
+    @property
+    def shape(self):
+        return self.rows.shape
+
+
+LAYER_ROWS = 16                   # of layer_rows.hip
+
+
+def layer_rows_fit(x, qkv: torch.Tensor, o: torch.Tensor,
+                   gate_up: torch.Tensor, down: torch.Tensor,
+                   head_dim: int) -> bool:
+    """Whether a layer's four projections of these rows go by layer_rows.hip:
+    sizes it takes, up to 4 rows of up to 8192 columns and up to 16 of up to
+    4096. Beyond, its workgroups of 16 columns read x more often than the launches
+    that they save are worth. us of the four with norms and rotation, apart and so: 1
+    row of 4096 (llama3-8b) 94.8 and 84.4, 16 101 and 96; of 3584 (qwen2-7b) 115.6
+    and 100.9, 118 and 115; of 2048 with 2 x 8192 48.6 and 35.0, 49.6 and 45.9; of
+    8192 (llama3-70b) 332 and 317, 8 334 and 336, 16 337 and 357; of 5120 with 2 x
+    13824 137 and 132, 8 142 and 144."""
+    x = x.rows if isinstance(x, Unscaled) else x
+    if not x.is_cuda or x.dim() != 2 or x.shape[0] > LAYER_ROWS:
+        return False
+    H = x.shape[1]
+    return (H % 64 == 0 and H <= (4096 if x.shape[0] > 4 else 8192)
+            and head_dim % 32 == 0
+            and x.dtype == torch.bfloat16
+            and o.dim() == 2 and down.dim() == 2
+            and o.shape[0] == H and down.shape[0] == H
+            and _rows_fit(x, qkv, LAYER_ROWS)
+            and _rows_fit(x, gate_up, LAYER_ROWS)
+            and gate_up.shape[0] % 64 == 0
+            and gate_up.shape[0] == 2 * down.shape[1]
+            and all(w.dtype == torch.bfloat16 and w.is_contiguous()
+                    and w.shape[1] * 2 % ROWS_CHUNK == 0
+                    and w.device == x.device and _aligned(w)
+                    for w in (o, down)))
+
+
+def rows_join(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+              norm_w: torch.Tensor, eps: float) -> Unscaled:
+    """residual += x @ w^T; its norm times norm_w, but for the division."""
+    return Unscaled(*_native().layer_rows_join(x, w, residual, norm_w), eps)
+
+
+def rows_glu(x: Unscaled, w: torch.Tensor) -> torch.Tensor:
+    """silu(first half) * second half of x's norm @ w^T."""
+    return _native().layer_rows_glu(x.rows, w, x.squares, x.eps)
+
+
+def rows_qkv(positions: torch.Tensor, x, w: torch.Tensor, bias,
+             cos_sin: torch.Tensor, num_q: int, num_kv: int, head_dim: int,
+             kv_cache=None, slot_mapping=None, want_kv: bool = False):
+    """rope_qkv_cache of x @ w^T + bias in one launch; x are rows or Unscaled."""
+    squares, eps = None, 0.0
+    if isinstance(x, Unscaled):
+        x, squares, eps = x
+    T = x.shape[0]
+    q = torch.empty(T, num_q, head_dim, dtype=x.dtype, device=x.device)
+    k = v = None
+    if want_kv:
+        k = torch.empty(T, num_kv, head_dim, dtype=x.dtype, device=x.device)
+        v = torch.empty_like(k)
+    kc, vc = kv_cache if kv_cache is not None else (None, None)
+    _native().layer_rows_qkv(x, w, bias, squares, eps, positions, cos_sin, q, k,
+                             v, kc, vc, slot_mapping, num_q, num_kv, head_dim)
+    return q, k, v
+
+
 def gemm_fp8_sums(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,
                   w_scale: torch.Tensor) -> torch.Tensor:
     """gemm_fp8 for a reader that adds up stretches (linear_sums)."""

@@ -111,6 +111,16 @@ std::vector<torch::Tensor> gemm_rows_many(torch::Tensor x,
                                           std::vector<OptT> biases);
 void gemm_rows_glu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                    OptT x_scale, OptT w_scale);
+std::vector<torch::Tensor> layer_rows_join(torch::Tensor x, torch::Tensor w,
+                                           torch::Tensor residual,
+                                           torch::Tensor norm);
+torch::Tensor layer_rows_glu(torch::Tensor x, torch::Tensor w, OptT squares,
+                             double eps);
+void layer_rows_qkv(torch::Tensor x, torch::Tensor w, OptT bias, OptT squares,
+                    double eps, torch::Tensor positions, torch::Tensor cos_sin,
+                    torch::Tensor q, OptT k, OptT v, OptT k_cache,
+                    OptT v_cache, OptT slots, int64_t num_q, int64_t num_kv,
+                    int64_t head_dim);
 void quantize_rows(torch::Tensor out, torch::Tensor scales, torch::Tensor x);
 void gemm_fp8(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               torch::Tensor x_scale, torch::Tensor w_scale,
@@ -207,6 +217,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "x @ w^T + bias of at most 64 rows for several w, in one launch");
   m.def("gemm_rows_glu", &gemm_rows_glu,
         "silu(x @ gate^T) * (x @ up^T) of at most 64 rows");
+  m.def("layer_rows_join", &layer_rows_join,
+        "residual += x @ w^T of at most 16 rows, (rows times norm, squares)");
+  m.def("layer_rows_glu", &layer_rows_glu,
+        "silu(x @ gate^T f) * (x @ up^T f) of at most 16 rows, f by squares");
+  m.def("layer_rows_qkv", &layer_rows_qkv,
+        "Heads of x @ w^T f + bias of at most 16 rows, turned and cached");
   m.def("quantize_rows", &quantize_rows,
         "bf16 rows to e4m3 bytes with a scale each");
   m.def("gemm_fp8", &gemm_fp8,
