@@ -1,6 +1,6 @@
 """A layer's projections of a few rows, with norm, rotation and residual in their
 launches (layer_rows.hip), against the same in 64 bits. Sums are fp32 over K, so
-what a result differs by is its rounding to bf16 (2^-9 of its size)."""
+what a result differs by is its rounding to bf16 (2^-8 of its size)."""
 import pytest
 import torch
 
