@@ -209,10 +209,13 @@ class Attention(nn.Module):
         if mixed:
             n = meta.num_decode
             o = torch.empty_like(q)
-            self._attend_decode(q[:n], kv_cache, meta.decode, o[:n])
-            self._attend_prefill(q[n:], k[n:] if want_kv else None,
-                                 v[n:] if want_kv else None, kv_cache,
-                                 prefill, o[n:])
+            if want_kv:
+                k, v = k[n:], v[n:]
+            else:
+                k, v = self._gather(q, kv_cache, prefill)
+            if not self._attend_both(q, k, v, kv_cache, meta, o):
+                self._attend_decode(q[:n], kv_cache, meta.decode, o[:n])
+                self._attend_prefill(q[n:], k, v, kv_cache, prefill, o[n:])
         elif meta.is_prefill:
             o = self._attend_prefill(q, k, v, kv_cache, meta)
         else:
@@ -225,16 +228,30 @@ class Attention(nn.Module):
             return parallel.tp_all_reduce(self.o_proj(o))
         return _project(self.o_proj, o, form)
 
+    @staticmethod
+    def _gather(q, kv_cache, meta):
+        """Full-context K/V of a cached-prefix prefill, gathered from the paged
+        cache (new tokens were just written)."""
+        return ops.gather_kv(*kv_cache, meta.gather_blk, meta.gather_off,
+                             q.dtype)
+
+    def _attend_both(self, q, k, v, kv_cache, meta, out) -> bool:
+        """Replies and portions in one launch, or False and nothing done."""
+        n, d, p = meta.num_decode, meta.decode, meta.prefill
+        if not (d.workspace and d.max_len):
+            return False
+        tmp_out, tmp_ml = d.workspace
+        cu_k = p.cu_seqlens if p.cu_seqlens_k is None else p.cu_seqlens_k
+        return ops.mixed_attention(
+            (out[n:], q[n:], k, v, p.cu_seqlens, cu_k, p.max_seqlen),
+            (out[:n], q[:n], *kv_cache, d.block_tables, d.seq_lens,
+             tmp_out[:n], tmp_ml[:n], d.max_len), self.scale, self.window)
+
     def _attend_prefill(self, q, k, v, kv_cache, meta, out=None):
-        if meta.cu_seqlens_k is None:
-            return ops.attn_prefill(q, k, v, meta.cu_seqlens,
-                                    meta.max_seqlen, self.scale,
-                                    window=self.window, out=out)
-        # cached-prefix prefill: full-context K/V gathered from the paged
-        # cache (new tokens were just written)
-        k_all, v_all = ops.gather_kv(*kv_cache, meta.gather_blk,
-                                     meta.gather_off, q.dtype)
-        return ops.attn_prefill(q, k_all, v_all, meta.cu_seqlens,
+        """k and v of all tokens; None: to be gathered."""
+        if k is None:
+            k, v = self._gather(q, kv_cache, meta)
+        return ops.attn_prefill(q, k, v, meta.cu_seqlens,
                                 meta.max_seqlen, self.scale,
                                 window=self.window,
                                 cu_seqlens_k=meta.cu_seqlens_k, out=out)

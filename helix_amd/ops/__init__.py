@@ -444,6 +444,17 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor,
     return o if out is None else out.copy_(o)
 
 
+def mixed_attention(portions: tuple, replies: tuple, scale: float,
+                    window: int) -> bool:
+    """attn_prefill of portions (out, q, k, v, cu_seqlens, cu_seqlens_k,
+    max_seqlen) and paged_attn_decode of replies (out, q, k_cache, v_cache,
+    block_tables, seq_lens, tmp_out, tmp_ml, max_len) in one launch, or False
+    and nothing done for what only those two take."""
+    if not portions[1].is_cuda:
+        return False
+    return _native().attn_mixed(*portions, *replies, scale, window)
+
+
 def sample_tokens(logits: torch.Tensor, temperatures: torch.Tensor,
                   seeds: torch.Tensor) -> torch.Tensor:
     if logits.is_cuda:

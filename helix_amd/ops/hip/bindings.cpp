@@ -70,6 +70,14 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
                   torch::Tensor v, torch::Tensor cu_seqlens,
                   torch::Tensor cu_seqlens_k, int64_t max_seqlen,
                   double scale, bool causal, int64_t window);
+bool attn_mixed(torch::Tensor out_p, torch::Tensor q_p, torch::Tensor k,
+                torch::Tensor v, torch::Tensor cu_seqlens,
+                torch::Tensor cu_seqlens_k, int64_t max_seqlen,
+                torch::Tensor out_d, torch::Tensor q_d, torch::Tensor k_cache,
+                torch::Tensor v_cache, torch::Tensor block_tables,
+                torch::Tensor seq_lens, torch::Tensor tmp_out,
+                torch::Tensor tmp_ml, int64_t max_len, double scale,
+                int64_t window);
 void sample_tokens(torch::Tensor out, torch::Tensor logits,
                    torch::Tensor temperatures, torch::Tensor seeds);
 void sample_tokens_ext(torch::Tensor out, torch::Tensor logits,
@@ -176,6 +184,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "Paged decode attention (GQA, flash-decoding partitions)");
   m.def("attn_prefill", &attn_prefill,
         "Varlen causal flash prefill attention (MFMA)");
+  m.def("attn_mixed", &attn_mixed,
+        "Prompt portions' and replies' attention in one launch");
   m.def("sample_tokens", &sample_tokens, "Greedy/Gumbel token sampling");
   m.def("sample_tokens_ext", &sample_tokens_ext,
         "Fused top-k/top-p/penalty Gumbel sampling (histogram threshold)");
