@@ -478,11 +478,16 @@ class LLMEngine:
                 positions=torch.cat([dmeta.positions, meta.positions]))
         ids = torch.tensor([t for i in order for t in spans[i].ids],
                            dtype=torch.int64, device=dev)
-        hidden = self.model(ids, self.kv.caches, meta)
         if not rows:
+            self.model(ids, self.kv.caches, meta)
             return None
-        return self.model.compute_logits(
-            hidden[torch.tensor(rows, dtype=torch.int64, device=dev)])
+        at = torch.tensor(rows, dtype=torch.int64, device=dev)
+        some = getattr(self.model, "forward_rows", None)
+        if some is not None:
+            hidden = some(ids, self.kv.caches, meta, at)
+        else:
+            hidden = self.model(ids, self.kv.caches, meta)[at]
+        return self.model.compute_logits(hidden)
 
     def _run_prefill(self, batch: List[Sequence],
                      decode: List[Sequence] = ()):

@@ -46,6 +46,15 @@ def _plain(emb: nn.Module) -> bool:
     return _own(emb, nn.Embedding) and emb.max_norm is None
 
 
+def _first_pays(cu: list) -> bool:
+    """Whether the last block is computed for first rows only: three launches more,
+    of fewer rows. us of the model (bge-base) with all rows and so: 1 text of 511
+    689 and 691, 3 of 400 763 and 761, 64 of 20 718 and 718, 64 of 40 905 and 888,
+    64 of 250 3283 and 3100."""
+    return cu[-1] >= max(1024, 8 * (len(cu) - 1)) and all(
+        b > a for a, b in zip(cu, cu[1:]))
+
+
 class BertLayer(nn.Module):
     PARAMS = ("qkv_w", "qkv_b", "attn_out_w", "attn_out_b", "attn_ln_w",
               "attn_ln_b", "up_w", "up_b", "down_w", "down_b", "out_ln_w",
@@ -69,6 +78,15 @@ class BertLayer(nn.Module):
         self.cfg = cfg
         self.hd = cfg.hidden_size // cfg.num_heads
         self.scale = self.hd ** -0.5
+
+    def first_rows(self, x, cu, max_len):
+        """The first row of each text, all of which have tokens, and the
+        boundaries of texts of a row each; None where forward is to be asked."""
+        if not _own(self, BertLayer) or tuple(self._parameters) != self.PARAMS:
+            return None
+        return ops.text_block_first(x, cu, max_len, self.cfg.num_heads,
+                                    self.scale, self.cfg.layer_norm_eps,
+                                    list(self._parameters.values()))
 
     def forward(self, x, cu, max_len):
         if tuple(self._parameters) == self.PARAMS:
@@ -134,8 +152,15 @@ class BertEmbeddingModel(nn.Module):
             x = self.word_emb(input_ids) + self.pos_emb(positions)
             x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
                                self.cfg.layer_norm_eps)
-        for layer in self.layers:
+        for layer in self.layers[:-1]:
             x = layer(x, cu_seqlens, max_len)
+        if self.cfg.pooling != "mean" and _first_pays(cu):
+            first = self.layers[-1].first_rows(x, cu_seqlens, max_len)
+            if first is not None:
+                emb = ops.text_pool(*first)
+                if emb is not None:
+                    return emb
+        x = self.layers[-1](x, cu_seqlens, max_len)
         if self.cfg.pooling == "mean":
             emb = torch.stack([x[s:e].float().mean(0)
                                for s, e in zip(cu, cu[1:])])

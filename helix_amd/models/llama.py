@@ -188,8 +188,10 @@ class Attention(nn.Module):
         self.o_proj = HLinear(q, h, bias=False)
 
     def forward(self, x: torch.Tensor, cos_sin: torch.Tensor, kv_cache,
-                meta, form: str = "rows", join=None) -> torch.Tensor:
-        """join (residual, norm_w, eps): few rows, see DecoderLayer."""
+                meta, form: str = "rows", join=None,
+                rows=None) -> torch.Tensor:
+        """join (residual, norm_w, eps): few rows, see DecoderLayer. rows: those
+        of the result that are asked for (None: all)."""
         T = x.shape[0]
         # fused strided split + rope + paged-cache write (one kernel, no
         # .contiguous() copies); compact K/V emitted only when the
@@ -221,6 +223,8 @@ class Attention(nn.Module):
         else:
             o = self._attend_decode(q, kv_cache, meta)
         o = o.view(T, -1)
+        if rows is not None:
+            o = o[rows]
         if join is not None:
             return ops.rows_join(o, self.o_proj.weight, *join)
         if self.tp_size > 1:
@@ -304,6 +308,15 @@ class DecoderLayer(nn.Module):
         self.mlp = MLP(cfg, tp_size)
         self.eps = cfg.rms_norm_eps
 
+    def unseen(self) -> bool:
+        """Whether all of it is as written here: nobody sees its rows but those who
+        ask for the result."""
+        a, m = self.attn, self.mlp
+        return (_own(self, DecoderLayer) and _own(a, Attention)
+                and _own(m, MLP) and all(
+                    _own(p, HLinear, FP8Linear) for p in
+                    (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj)))
+
     def few(self, x) -> bool:
         """Whether these rows go through the layer in launches that take norm,
         rotation and residual along (layer_rows.hip): all of it is as written
@@ -319,10 +332,11 @@ class DecoderLayer(nn.Module):
                 and ops.layer_rows_fit(x, *(p.weight for p in ps), a.hd))
 
     def forward(self, x, residual, cos_sin, kv_cache, meta,
-                form: str = "rows", few: bool = False, after=None):
+                form: str = "rows", few: bool = False, after=None, rows=None):
         """form "sums": the result's stretches, for the next norm. few: as few()
         says; after (few): the weight of that norm, which the result then is but
-        for its division (ops.Unscaled)."""
+        for its division (ops.Unscaled). rows: those that are asked for, where attn
+        is as written here; the others leave behind attention."""
         if residual is None:
             residual = x.clone()
             h = ops.rms_norm(x, self.input_norm_w, self.eps)
@@ -337,7 +351,10 @@ class DecoderLayer(nn.Module):
             join = None if after is None else (residual, after, self.eps)
             return self.mlp(h, form, join), residual
         h = self.attn(h, cos_sin, kv_cache, meta,
-                      *(["sums"] if _own(self.attn, Attention) else []))
+                      *(["sums", None, rows] if _own(self.attn, Attention)
+                        else []))
+        if rows is not None:
+            residual = residual[rows]
         h, residual = _norm_for(self.mlp, MLP, "gate_up_proj")(
             h, residual, self.post_norm_w, self.eps)
         h = self.mlp(h, *([form] if _own(self.mlp, MLP) else []))
@@ -376,6 +393,22 @@ class LlamaForCausalLM(nn.Module):
 
     @torch.inference_mode()
     def forward(self, input_ids: torch.Tensor, kv_caches, meta) -> torch.Tensor:
+        return self._hidden(input_ids, kv_caches, meta)
+
+    @torch.inference_mode()
+    def forward_rows(self, input_ids: torch.Tensor, kv_caches, meta,
+                     rows: torch.Tensor) -> torch.Tensor:
+        """Rows of what forward returns. Of a prompt, scores of the last token are
+        asked for: the others end with the last layer's attention, whose
+        feed-forward is 2 to 3% of all products. To take rows apart costs two
+        launches, so this is for prompts of which at least half leave."""
+        if input_ids.shape[0] >= 256 and \
+                0 < 2 * rows.numel() <= input_ids.shape[0] and \
+                _own(self, LlamaForCausalLM) and self.layers[-1].unseen():
+            return self._hidden(input_ids, kv_caches, meta, rows)
+        return self(input_ids, kv_caches, meta)[rows]
+
+    def _hidden(self, input_ids, kv_caches, meta, rows=None) -> torch.Tensor:
         x = self.embed_tokens(input_ids)
         residual, own = None, True
         few = [x.shape[0] <= ops.LAYER_ROWS and _own(layer, DecoderLayer)
@@ -387,6 +420,8 @@ class LlamaForCausalLM(nn.Module):
             if few[i]:
                 extra += [True, self.layers[i + 1].input_norm_w
                           if few[i + 1] else None]
+            elif rows is not None and i + 1 == len(self.layers):
+                extra += [False, None, rows]
             x, residual = layer(x, residual, self.cos_sin, cache, meta, *extra)
         if not own:                # what a hook has kept stays as it was
             x, residual = x.clone(), residual.clone()

@@ -187,6 +187,18 @@ def text_block(x: torch.Tensor, cu: torch.Tensor, max_len: int, heads: int,
     return None
 
 
+def text_block_first(x: torch.Tensor, cu: torch.Tensor, max_len: int,
+                     heads: int, scale: float, eps: float, params: list):
+    """text_block of texts that all have tokens, for one who only asks for the
+    first row of each: (those rows, cu of texts of a row each), or None as
+    above."""
+    if x.is_cuda and not _seen_by_torch():
+        out = _native().text_block_first(x, cu, max_len, heads, scale, eps,
+                                         params)
+        return tuple(out) or None
+    return None
+
+
 def image_block(x: torch.Tensor, y, gate, y_bias, mod: torch.Tensor,
                 cu: torch.Tensor, L: int, heads: int, scale: float, eps: float,
                 params: list, stretches: bool = False):

@@ -25,6 +25,9 @@ bool time_embed(torch::Tensor out, torch::Tensor t);
 c10::optional<torch::Tensor> text_block(
     torch::Tensor x, torch::Tensor cu, int64_t max_len, int64_t heads,
     double scale, double eps, std::vector<c10::optional<torch::Tensor>> p);
+std::vector<torch::Tensor> text_block_first(
+    torch::Tensor x, torch::Tensor cu, int64_t max_len, int64_t heads,
+    double scale, double eps, std::vector<c10::optional<torch::Tensor>> p);
 std::vector<torch::Tensor> image_block(
     torch::Tensor x, c10::optional<torch::Tensor> y,
     c10::optional<torch::Tensor> gate, c10::optional<torch::Tensor> y_bias,
@@ -163,6 +166,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "Text and image rows with their places, mean of the text");
   m.def("time_embed", &time_embed, "Sinusoidal embedding of times");
   m.def("text_block", &text_block, "A block of the text encoder");
+  m.def("text_block_first", &text_block_first,
+        "A block of the text encoder, for the first row of each text");
   m.def("image_block", &image_block, "A block of the image model");
   m.def("norm_in_registers", &norm_in_registers,
         "Whether add_sums_rms_norm keeps a row in registers");

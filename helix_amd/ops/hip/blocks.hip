@@ -14,7 +14,9 @@ using OptT = c10::optional<torch::Tensor>;
 using Tensors = std::vector<torch::Tensor>;
 using OptTs = std::vector<OptT>;
 
-// of gemm_bf16.hip, gemm_rows.hip, attn_prefill.hip and encoder.hip
+// of gemm_bf16.hip, gemm_rows.hip, attn_prefill.hip, embed.hip and encoder.hip
+void text_first(torch::Tensor out, torch::Tensor starts, torch::Tensor x,
+                torch::Tensor cu);
 void gemm_bf16(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
                int64_t act, int64_t tile);
 void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w, OptT bias,
@@ -102,15 +104,15 @@ bool rows_of(const torch::Tensor& x, const torch::Tensor& cu, int64_t heads) {
          cu.dim() == 1 && cu.numel() >= 2 && cu.is_contiguous();
 }
 
-}  // namespace
-
-// Both: nothing, and nothing done, for other forms of operands than all of the
-// steps' kernels read.
 
 // p: weight and bias of q k v, attention's end, its norm, the way up, the way down,
-// the last norm.
-OptT text_block(torch::Tensor x, torch::Tensor cu, int64_t max_len,
-                int64_t heads, double scale, double eps, OptTs params) {
+// the last norm. first: only the first row of each text, which has one, and the
+// boundaries of texts of a row each. Keys and values are of all rows then, and the
+// rest is of as many rows as there are texts: 16000 tokens of 64 texts, 768 columns,
+// 273 us -> 90.
+Tensors through_text(torch::Tensor x, const torch::Tensor& cu, int64_t max_len,
+                     int64_t heads, double scale, double eps,
+                     const OptTs& params, bool first) {
   const Tensors p = present(params, 12);
   if (p.empty() || params.size() != 12 || !rows_of(x, cu, heads) ||
       p[6].dim() != 2)
@@ -128,10 +130,53 @@ OptT text_block(torch::Tensor x, torch::Tensor cu, int64_t max_len,
                 "a norm of other operands");
     return out;
   };
-  const torch::Tensor o = attend(x, p[0], p[1], cu, max_len, heads, scale);
+  torch::Tensor o, starts;
+  if (first) {
+    const int64_t T = x.size(0), B = cu.numel() - 1, D = H / heads;
+    const torch::Tensor rows = at::empty({B, H}, x.options());
+    starts = at::empty({B + 1}, cu.options());
+    text_first(rows, starts, x, cu);
+    const torch::Tensor kv = product(x, p[0].narrow(0, H, 2 * H),
+                                     p[1].narrow(0, H, 2 * H), 0);
+    const torch::Tensor q = product(rows, p[0].narrow(0, 0, H),
+                                    p[1].narrow(0, 0, H), 0);
+    auto part = [&](int64_t i) {
+      return kv.as_strided({T, heads, D}, {2 * H, D, 1},
+                           kv.storage_offset() + i * H);
+    };
+    o = at::empty({B, heads, D}, x.options());
+    attn_prefill(o, q.view({B, heads, D}), part(0), part(1), starts, cu, 1,
+                 scale, false, 0);
+    o = o.view({B, H});
+    x = rows;
+  } else {
+    o = attend(x, p[0], p[1], cu, max_len, heads, scale);
+  }
   x = norm(x, summand(o, p[2], p[3]), 4);
   const torch::Tensor up = product(x, p[6], p[7], 1);
-  return norm(x, summand(up, p[8], p[9]), 10);
+  x = norm(x, summand(up, p[8], p[9]), 10);
+  if (first) return {x, starts};
+  return {x};
+}
+
+}  // namespace
+
+// All: nothing, and nothing done, for other forms of operands than all of the
+// steps' kernels read.
+
+OptT text_block(torch::Tensor x, torch::Tensor cu, int64_t max_len,
+                int64_t heads, double scale, double eps, OptTs params) {
+  const Tensors out = through_text(x, cu, max_len, heads, scale, eps, params,
+                                   false);
+  return out.empty() ? OptT{} : out[0];
+}
+
+// Its result for the first row of each text, which has one, and the boundaries of
+// texts of a row each.
+Tensors text_block_first(torch::Tensor x, torch::Tensor cu, int64_t max_len,
+                         int64_t heads, double scale, double eps,
+                         OptTs params) {
+  return through_text(x, cu, max_len, heads, scale, eps, params, true);
 }
 
 // x (+ gate y) through a block: the result as x, y and gate of a sum that is still

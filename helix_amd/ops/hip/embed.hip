@@ -131,6 +131,20 @@ __global__ __launch_bounds__(NT) void text_pool_kernel(
   }
 }
 
+// Rows cu[:-1] of x side by side, and their boundaries 0, 1, ..: a workgroup each,
+// and one more for the last of those.
+__global__ __launch_bounds__(NT) void text_first_kernel(
+    uint16_t* __restrict__ out, int* __restrict__ starts,
+    const uint16_t* __restrict__ x, const int* __restrict__ cu, int B, int H) {
+  const int s = blockIdx.x;
+  if (threadIdx.x == 0) starts[s] = s;
+  if (s == B) return;
+  const int64_t from = (int64_t)cu[s] * H, to = (int64_t)s * H;
+  for (int c = threadIdx.x * 8; c < H; c += NT * 8)
+    *reinterpret_cast<u16x8*>(out + to + c) =
+        *reinterpret_cast<const u16x8*>(x + from + c);
+}
+
 struct Image {
   int B, C, S, p;              // latents [B, C, S, S] in patches of p x p
   int L, text;                 // tokens of an image, of them text
@@ -321,6 +335,23 @@ bool text_pool(torch::Tensor out, torch::Tensor x, torch::Tensor cu) {
                      (const uint16_t*)x.data_ptr(), cu.data_ptr<int>(), B,
                      (int)x.size(1));
   return true;
+}
+
+// out[B, H], starts[B + 1]: rows cu[:-1] of x and the boundaries of texts of a token
+// each. The texts have tokens; x and out are packed rows on 16-byte boundaries.
+void text_first(torch::Tensor out, torch::Tensor starts, torch::Tensor x,
+                torch::Tensor cu) {
+  const int64_t B = cu.numel() - 1;
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 &&
+              table(x, x, x.size(0), x.size(1)) && x.size(1) % 8 == 0 &&
+              numbers(cu, torch::kInt32, x) && cu.dim() == 1 && B >= 1 &&
+              table(out, x, B, x.size(1)) &&
+              numbers(starts, torch::kInt32, x) && starts.numel() == B + 1,
+              "rows of texts");
+  hipLaunchKernelGGL(text_first_kernel, dim3(B + 1), dim3(NT), 0,
+                     at::hip::getCurrentHIPStream(), (uint16_t*)out.data_ptr(),
+                     starts.data_ptr<int>(), (const uint16_t*)x.data_ptr(),
+                     cu.data_ptr<int>(), (int)B, (int)x.size(1));
 }
 
 // out[B patches, K]: patches of the latents (bf16 or fp32) as rows.

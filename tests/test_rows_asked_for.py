@@ -1,0 +1,81 @@
+"""Rows of a prompt that nobody asks for leave before the last layer's feed-forward:
+those asked for are what a pass over all rows gives, and hooks see all of them."""
+import pytest
+import torch
+
+from helix_amd.models.llama import PRESETS, LlamaForCausalLM
+from helix_amd.models.meta import PrefillMeta
+
+
+def _step(lens):
+    T = sum(lens)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(),
+                      dtype=torch.int32)
+    pos = torch.cat([torch.arange(n) for n in lens])
+    return torch.arange(T) % 500, PrefillMeta(
+        cu_seqlens=cu, max_seqlen=max(lens),
+        slot_mapping=torch.arange(T), positions=pos)
+
+
+def _caches(cfg, T):
+    n = -(-T // 16)
+    return [(torch.zeros(n, cfg.num_kv_heads, 16, cfg.head_dim),
+             torch.zeros(n, cfg.num_kv_heads, 16, cfg.head_dim))
+            for _ in range(cfg.num_layers)]
+
+
+# too few tokens, one row, several, more than half
+@pytest.mark.parametrize("lens,rows", [
+    ([200], [199]), ([256], [255]), ([300, 40], [299, 339, 7]),
+    ([256], list(range(129))), ([256], list(range(0, 256, 2)))])
+def test_same_rows(lens, rows):
+    cfg = PRESETS["tiny"]
+    model = LlamaForCausalLM(cfg).init_random(3)
+    ids, meta = _step(lens)
+    a, b = _caches(cfg, sum(lens)), _caches(cfg, sum(lens))
+    want = model(ids, a, meta)[torch.tensor(rows)]
+    got = model.forward_rows(ids, b, meta, torch.tensor(rows))
+    # sums of the products in another order: fp32
+    torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
+    for (k, v), (x, y) in zip(a, b):
+        assert torch.equal(k, x) and torch.equal(v, y)
+
+
+@pytest.mark.parametrize("where", [
+    "layers.1", "layers.1.attn.o_proj", "layers.1.mlp.down_proj", ""])
+def test_hooks_see_all(where):
+    model = LlamaForCausalLM(PRESETS["tiny"]).init_random(3)
+    seen = []
+    model.get_submodule(where).register_forward_hook(
+        lambda m, i, o: seen.append((o[0] if isinstance(o, tuple)
+                                     else o).shape[0]))
+    ids, meta = _step([300])
+    out = model.forward_rows(ids, _caches(model.cfg, 300), meta,
+                             torch.tensor([299]))
+    assert seen == [300] and out.shape[0] == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,h,inner,heads", [
+    ([1], 128, 256, 2), ([20, 1, 44, 500], 768, 3072, 12),
+    ([64] * 70, 256, 512, 2), ([300, 129], 1024, 4096, 8)])
+def test_first_rows_of_texts(lens, h, inner, heads):
+    """Two ways through a block round what five products and sums of unit spread
+    give to bf16, 2^-9 of it in the mean each."""
+    from helix_amd import ops
+    torch.manual_seed(len(lens))
+    r = lambda *s, std=1.0: (torch.randn(*s, device="cuda") * std).bfloat16()  # noqa: E731
+    p = [r(3 * h, h, std=h ** -0.5), r(3 * h, std=0.3), r(h, h, std=h ** -0.5),
+         r(h, std=0.3), 1 + r(h, std=0.1), r(h, std=0.1),
+         r(inner, h, std=h ** -0.5), r(inner, std=0.3),
+         r(h, inner, std=inner ** -0.5), r(h, std=0.3), 1 + r(h, std=0.1),
+         r(h, std=0.1)]
+    x = r(sum(lens), h)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(),
+                      dtype=torch.int32, device="cuda")
+    with torch.inference_mode():
+        args = (x, cu, max(lens), heads, (h // heads) ** -0.5, 1e-12, p)
+        want = ops.text_block(*args)[cu[:-1].long()].float()
+        got, starts = ops.text_block_first(*args)
+    assert starts.tolist() == list(range(len(lens) + 1))
+    assert ((got.float() - want).norm() / want.norm()).item() < 5 * 2 ** -9
