@@ -206,8 +206,7 @@ class Attention(nn.Module):
             q, k, v = ops.rows_qkv(meta.positions, x, self.qkv_proj.weight,
                                    self.qkv_proj.bias, *heads)
         else:
-            q, k, v = ops.rope_qkv_cache(
-                meta.positions, _project(self.qkv_proj, x, "sums"), *heads)
+            q, k, v = self._heads(x, meta.positions, heads)
         if mixed:
             n = meta.num_decode
             o = torch.empty_like(q)
@@ -231,6 +230,19 @@ class Attention(nn.Module):
             from helix_amd import parallel
             return parallel.tp_all_reduce(self.o_proj(o))
         return _project(self.o_proj, o, form)
+
+    def _heads(self, x, positions, heads):
+        """Turned and cached heads of x: of a few rows in the projection's launch."""
+        p = self.qkv_proj
+        if x.shape[0] <= ops.ROWS_QKV:
+            if _own(p, HLinear) and \
+                    ops.rows_qkv_fit(x, p.weight, p.bias, self.hd):
+                return ops.rows_qkv(positions, x, p.weight, p.bias, *heads)
+            if _own(p, FP8Linear) and isinstance(x, ops.Quantized) and \
+                    ops.rows_qkv_fit(x, p.weight8, None, self.hd):
+                return ops.rows_qkv(positions, x, p.weight8, None, *heads,
+                                    w_scale=p.w_scale)
+        return ops.rope_qkv_cache(positions, _project(p, x, "sums"), *heads)
 
     @staticmethod
     def _gather(q, kv_cache, meta):

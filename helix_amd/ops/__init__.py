@@ -968,21 +968,51 @@ def rows_glu(x: Unscaled, w: torch.Tensor) -> torch.Tensor:
 
 def rows_qkv(positions: torch.Tensor, x, w: torch.Tensor, bias,
              cos_sin: torch.Tensor, num_q: int, num_kv: int, head_dim: int,
-             kv_cache=None, slot_mapping=None, want_kv: bool = False):
-    """rope_qkv_cache of x @ w^T + bias in one launch; x are rows or Unscaled."""
-    squares, eps = None, 0.0
+             kv_cache=None, slot_mapping=None, want_kv: bool = False,
+             w_scale: torch.Tensor | None = None):
+    """rope_qkv_cache of x @ w^T + bias in one launch; x are rows or Unscaled, or
+    Quantized where w are e4m3 bytes with a scale of each row."""
+    squares, eps, x_scale = None, 0.0, None
     if isinstance(x, Unscaled):
         x, squares, eps = x
+    elif isinstance(x, Quantized):
+        x, x_scale = x
     T = x.shape[0]
-    q = torch.empty(T, num_q, head_dim, dtype=x.dtype, device=x.device)
+    q = torch.empty(T, num_q, head_dim, dtype=torch.bfloat16, device=x.device)
     k = v = None
     if want_kv:
-        k = torch.empty(T, num_kv, head_dim, dtype=x.dtype, device=x.device)
+        k = torch.empty(T, num_kv, head_dim, dtype=q.dtype, device=x.device)
         v = torch.empty_like(k)
     kc, vc = kv_cache if kv_cache is not None else (None, None)
     _native().layer_rows_qkv(x, w, bias, squares, eps, positions, cos_sin, q, k,
-                             v, kc, vc, slot_mapping, num_q, num_kv, head_dim)
+                             v, kc, vc, slot_mapping, num_q, num_kv, head_dim,
+                             x_scale, w_scale)
     return q, k, v
+
+
+ROWS_QKV = 32                     # of layer_rows.hip, without squares
+
+
+def rows_qkv_fit(x, w: torch.Tensor, bias, head_dim: int) -> bool:
+    """Whether rows_qkv takes rows or Quantized ones, and takes no longer than the
+    product in stretches with rope_qkv_cache: its workgroups read x more often, the
+    more the more rows and the deeper they are, and tiles take over wide matrices
+    from 17 rows on. us apart and at once: 1 row of 6144 x 4096 14.5 and 12.0, 32
+    16.4 and 15.6; 16 of 15360 x 5120 37.8 and 36.2, 32 33.7 and 42; 4 of 10240 x
+    8192 39.9 and 39.0, 8 39 and 47; 32 of 12288 x 4096 25 and 29. e4m3: 32 of 6144 x
+    4096 13.4 and 10.3, of 15360 x 5120 25.8 and 23.9, 8 of 10240 x 8192 24.3 and
+    23.9, 16 24.0 and 25.2."""
+    bytes_ = isinstance(x, Quantized)
+    x = x.bytes if bytes_ else x
+    if not (_rows_fit(x, w, ROWS_QKV) and _bias_fits(bias, w)
+            and head_dim % 32 == 0):
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    if bytes_:
+        return K <= (8192 if M <= 8 else 5120)
+    if M > 16:
+        return K <= 4096 and N <= 8192
+    return K <= (8192 if M <= 4 else 5120)
 
 
 def gemm_fp8_sums(x8: torch.Tensor, w8: torch.Tensor, x_scale: torch.Tensor,

@@ -131,7 +131,7 @@ void layer_rows_qkv(torch::Tensor x, torch::Tensor w, OptT bias, OptT squares,
                     double eps, torch::Tensor positions, torch::Tensor cos_sin,
                     torch::Tensor q, OptT k, OptT v, OptT k_cache,
                     OptT v_cache, OptT slots, int64_t num_q, int64_t num_kv,
-                    int64_t head_dim);
+                    int64_t head_dim, OptT x_scale, OptT w_scale);
 void quantize_rows(torch::Tensor out, torch::Tensor scales, torch::Tensor x);
 void gemm_fp8(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               torch::Tensor x_scale, torch::Tensor w_scale,
@@ -237,7 +237,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("layer_rows_glu", &layer_rows_glu,
         "silu(x @ gate^T f) * (x @ up^T f) of at most 16 rows, f by squares");
   m.def("layer_rows_qkv", &layer_rows_qkv,
-        "Heads of x @ w^T f + bias of at most 16 rows, turned and cached");
+        "Heads of x @ w^T f + bias of at most 32 rows, turned and cached");
   m.def("quantize_rows", &quantize_rows,
         "bf16 rows to e4m3 bytes with a scale each");
   m.def("gemm_fp8", &gemm_fp8,

@@ -1,4 +1,4 @@
-// Projections of up to 16 rows of a language model's layer, bf16 with fp32 sums,
+// Projections of a few rows of a language model's layer, bf16 with fp32 sums, up to 16,
 // with what comes before and behind them: x[M,K] @ w[N,K]^T and
 //   JOIN  the residual is added, and rows leave times the next norm's weight, with
 //         sums of squares beside them; whoever multiplies them divides by their
@@ -27,6 +27,10 @@
 //   M  4  15.1  13.4     13.6   9.7     27.9  23.9     43.3  43.3
 //   M  8  15.6  13.4     13.8   9.7     28.3  25.0     43.5  44.7
 //   M 16  15.9  14.9     14.2  10.6     29.2  28.5     44.7  45.8
+// QKV goes on to 32 rows, without squares, and takes e4m3 (scaled 16x16x128 with
+// unity scales; those of rows meet the sums): 32 rows of 6144 x 4096 16.4 us apart
+// and 15.6, e4m3 13.4 and 10.3. The other forms would not gain there: 24 rows of
+// 4096 x 14336 29 and 31, the gated product of e4m3 26 and 29.
 #include "hybrid/tile.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -39,12 +43,15 @@ namespace {
 
 constexpr int NW = 4, NT = NW * WAVE;
 constexpr int MOST_ROWS = 16, MOST_PARTS = 512;
+constexpr int MOST_ROWS_QKV = 32;
+constexpr int UNITY = 0x7F7F7F7F;             // e8m0 2^0 in all four bytes
 
 enum Form { JOIN, QKV, GLU };
 
 struct LayerRows {
-  const uint16_t *x, *w;       // [M, K]; [N, K], GLU [2 N, K]
+  const char *x, *w;           // [M, K]; [N, K], GLU [2 N, K]
   const float* squares;        // [M, parts] of x's rows, or null
+  const float *xs, *ws;        // e4m3: scales of rows of x and of w
   uint16_t* out;               // JOIN and GLU [M, N]
   int M, N, K, parts;
   float eps;
@@ -74,21 +81,30 @@ __device__ __forceinline__ void write_cache4(void* c, int64_t at,
   }
 }
 
-// MR: rows that there is room for, at least M. NI: tiles of 16 rows of w of a
-// workgroup, which go to half as many columns of GLU. CHUNK: of the inner
-// dimension. F8: e4m3 pages (QKV).
-template <int MR, int NI, int CHUNK, Form FORM, bool F8>
+typedef int v8i __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ v8i both(u32x4 a, u32x4 b) {
+  return v8i{(int)a[0], (int)a[1], (int)a[2], (int)a[3],
+             (int)b[0], (int)b[1], (int)b[2], (int)b[3]};
+}
+
+// MR: rows that there is room for, at least M; more than 16 only without squares.
+// NI: tiles of 16 rows of w of a workgroup, which go to half as many columns of GLU.
+// CHUNK: bytes of the inner dimension. F8: e4m3 pages (QKV). F8X: x and w are e4m3.
+template <int MR, int NI, int CHUNK, Form FORM, bool F8, bool F8X>
 __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
-  constexpr int U = CHUNK / 32, PIECES = CHUNK / 8, XL = MR * PIECES / WAVE;
+  constexpr int U = CHUNK / 64, PIECES = CHUNK / 16, XL = MR * PIECES / WAVE;
+  constexpr int MI = MR > 16 ? MR / 16 : 1;   // tiles of 16 rows of x
+  constexpr bool SQUARES = FORM != JOIN && MI == 1 && !F8X;
   constexpr int PART = MOST_PARTS / (4 * WAVE);
-  __shared__ f32x4 red[NW][NI][WAVE];
+  __shared__ f32x4 red[NW][MI * NI][WAVE];
   __shared__ u32x4 xs[NW][MR * PIECES];
   __shared__ float inv[MOST_ROWS];
   const int tid = threadIdx.x, lane = tid & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lo = lane & 15, hi = lane >> 4;
   const int tile = blockIdx.x, half = m.D / 2;
-  const int row = min(lo, m.M - 1);
+  // of the tile of x that this wave ends
+  const int r_end = (MI > 1 ? wid * 16 : 0) + lo, row = min(r_end, m.M - 1);
   // QKV: a workgroup has pairs that are turned together, x and then y
   constexpr int PAIRS = 8 * NI;
   const int per = FORM == QKV ? half / PAIRS : 1;
@@ -103,8 +119,8 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
   };
 
   // Loads come back in order, so what else is read goes before the weights.
-  f32x4 part[MR / NW][PART];
-  if (FORM != JOIN && m.squares != nullptr) {
+  f32x4 part[SQUARES ? MR / NW : 1][PART];
+  if (SQUARES && m.squares != nullptr) {
 #pragma unroll
     for (int r = 0; r < MR / NW; ++r)
       if (r * NW + wid < m.M)
@@ -128,19 +144,25 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
     if (m.slots != nullptr) slot = m.slots[row];
   }
 
-  const uint16_t* wp[NI];
+  // A lane's 16 bytes u of a chunk's row: bf16 has four lane groups to 64 bytes,
+  // e4m3 two pieces side by side to 128.
+  auto piece = [&](int u) {
+    return F8X ? (u >> 1) * 8 + hi * 2 + (u & 1) : u * 4 + hi;
+  };
+  const int64_t bytes = (int64_t)m.K * (F8X ? 1 : 2);
+  const char* wp[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j)
-    wp[j] = m.w + (int64_t)row_of(j) * m.K + hi * 8;
-  // 16-byte piece p of row r lies at p ^ r: operands leave LDS without bank
+    wp[j] = m.w + row_of(j) * bytes;
+  // 16-byte piece p of row r lies at p ^ r % 16: operands leave LDS without bank
   // conflicts
-  const uint16_t* xp[XL];
+  const char* xp[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int e = i * WAVE + lane, r = e / PIECES;
-    xp[i] = m.x + (int64_t)min(r, m.M - 1) * m.K + (e % PIECES ^ r) * 8;
+    xp[i] = m.x + min(r, m.M - 1) * bytes + (e % PIECES ^ (r & 15)) * 16;
   }
-  const int chunks = m.K / CHUNK, share = cdiv(chunks, NW);
+  const int chunks = (int)(bytes / CHUNK), share = cdiv(chunks, NW);
   const int start = min(chunks, wid * share), end = min(chunks, start + share);
   const int turn = FORM == GLU && end > start ? tile % (end - start) : 0;
   u32x4 wr[2][U][NI], xr[2][XL];
@@ -155,29 +177,41 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int j = 0; j < NI; ++j)
-        wr[b][u][j] =
-            *reinterpret_cast<const u32x4*>(wp[j] + c * CHUNK + u * 32);
+        wr[b][u][j] = *reinterpret_cast<const u32x4*>(wp[j] + c * CHUNK +
+                                                      piece(u) * 16);
     __builtin_amdgcn_sched_barrier(0);
   };
-  floatx4 acc[NI];
+  floatx4 acc[MI][NI];
 #pragma unroll
-  for (int j = 0; j < NI; ++j) acc[j] = floatx4{0, 0, 0, 0};
+  for (int t = 0; t < MI; ++t)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[t][j] = floatx4{0, 0, 0, 0};
   u32x4* const mine = xs[wid];
   auto multiply = [&](auto buf) {
     constexpr int b = decltype(buf)::value;
 #pragma unroll
     for (int i = 0; i < XL; ++i) mine[i * WAVE + lane] = xr[b][i];
-    // columns past the last row repeat others, and nobody looks at them
-    const int r = lo & (MR - 1);
-    u16x8 xf[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      xf[u] = __builtin_bit_cast(u16x8, mine[r * PIECES + ((u * 4 + hi) ^ r)]);
+    for (int t = 0; t < MI; ++t) {
+      // columns past the last row repeat others, and nobody looks at them
+      const int r = MI > 1 ? t * 16 + lo : lo & (MR - 1);
+      u32x4 xf[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u)
+        xf[u] = mine[r * PIECES + (piece(u) ^ (r & 15))];
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
-        acc[j] = mfma16(__builtin_bit_cast(u16x8, wr[b][u][j]), xf[u], acc[j]);
+      for (int u = 0; u < U; u += F8X ? 2 : 1)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          if constexpr (F8X)
+            acc[t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                both(wr[b][u][j], wr[b][u + 1][j]), both(xf[u], xf[u + 1]),
+                acc[t][j], 0, 0, 0, UNITY, 0, UNITY);
+          else
+            acc[t][j] = mfma16(__builtin_bit_cast(u16x8, wr[b][u][j]),
+                               __builtin_bit_cast(u16x8, xf[u]), acc[t][j]);
+        }
+    }
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr std::integral_constant<int, 0> A;
@@ -193,7 +227,7 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
       sine[q] = cs[half + q];
     }
   }
-  if (FORM != JOIN && m.squares != nullptr) {
+  if (SQUARES && m.squares != nullptr) {
 #pragma unroll
     for (int r = 0; r < MR / NW; ++r)
       if (r * NW + wid < m.M) {
@@ -222,19 +256,21 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
     }
   }
 #pragma unroll
-  for (int j = 0; j < NI; ++j)
-    red[wid][j][lane] = __builtin_bit_cast(f32x4, acc[j]);
+  for (int t = 0; t < MI; ++t)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+      red[wid][t * NI + j][lane] = __builtin_bit_cast(f32x4, acc[t][j]);
   __syncthreads();
-  if (wid != 0) return;
-  // lane: columns 4 hi + i of row lo
+  if (wid >= MI) return;
+  // lane: columns 4 hi + i of row lo of a tile
   f32x4 s[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) {
-    s[j] = red[0][j][lane];
+    s[j] = red[0][wid * NI + j][lane];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) s[j] += red[w][j][lane];
+    for (int w = 1; w < NW; ++w) s[j] += red[w][wid * NI + j][lane];
   }
-  const bool there = lo < m.M;
+  const bool there = r_end < m.M;
   float v[4];
   if constexpr (FORM == JOIN) {
     const int64_t at = (int64_t)row * m.N + tile * 16 + hi * 4;
@@ -254,7 +290,8 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
     if (hi == 0) m.squares_out[row * gridDim.x + tile] = ss;
     return;
   }
-  const float f = m.squares != nullptr ? inv[row] : 1.f;
+  const float f = F8X ? m.xs[row]
+                  : SQUARES && m.squares != nullptr ? inv[row] : 1.f;
   if constexpr (FORM == GLU) {
     if (!there) return;
 #pragma unroll
@@ -275,10 +312,10 @@ __global__ __launch_bounds__(NT) void layer_rows_kernel(LayerRows m) {
     for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        const int n = head * m.D + (second || j == 1 ? half : 0) + d + i;
         o[j][i] = s[j][i] * f;
-        if (m.bias != nullptr)
-          o[j][i] += bf16_to_f32(
-              m.bias[head * m.D + (second || j == 1 ? half : 0) + d + i]);
+        if constexpr (F8X) o[j][i] *= m.ws[n];
+        if (m.bias != nullptr) o[j][i] += bf16_to_f32(m.bias[n]);
       }
     if (!value) {
 #pragma unroll
@@ -320,20 +357,23 @@ void check(const torch::Tensor& t, const torch::Tensor& x,
 }
 
 LayerRows rows_of(const torch::Tensor& x, const torch::Tensor& w,
-                  const OptT& squares, double eps) {
-  check(x, x, torch::kBFloat16, 16);
-  check(w, x, torch::kBFloat16, 16);
+                  const OptT& squares, double eps,
+                  torch::ScalarType type = torch::kBFloat16,
+                  int most = MOST_ROWS) {
+  check(x, x, type, 16);
+  check(w, x, type, 16);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1));
   LayerRows m{};
-  m.x = (const uint16_t*)x.data_ptr();
-  m.w = (const uint16_t*)w.data_ptr();
+  m.x = (const char*)x.data_ptr();
+  m.w = (const char*)w.data_ptr();
   m.M = x.size(0);
   m.N = w.size(0);
   m.K = x.size(1);
   m.eps = (float)eps;
-  TORCH_CHECK(m.M >= 1 && m.M <= MOST_ROWS && m.K > 0 && m.K % 256 == 0 &&
+  TORCH_CHECK(m.M >= 1 && x.size(0) <= most && m.K > 0 &&
+              x.size(1) * x.element_size() % 512 == 0 &&
               x.size(1) <= 1 << 24 && m.N > 0 && w.size(0) <= 1 << 24,
-              "up to 16 rows of whole chunks");
+              "a few rows of whole chunks");
   if (squares.has_value()) {
     check(*squares, x, torch::kFloat32, 16);
     TORCH_CHECK(squares->dim() == 2 && squares->size(0) == m.M &&
@@ -348,19 +388,20 @@ LayerRows rows_of(const torch::Tensor& x, const torch::Tensor& w,
 // on; few columns would leave CUs idle by them (us of 1, 8 and 16 rows by 16 and
 // by 32: 6144 x 4096 11.8 and 12.1, 13.5 and 12.2, 15.7 and 13.2; 4096 x 14336 23
 // and 37). Of the gated product a wave has 32 columns of either factor, in chunks of
-// 128 that begin apart: 41.2, 42.8 and 45.7 us of 2 x 14336 x 4096, with 16 in
-// chunks of 256 41.3, 43.8 and 46.4.
-template <Form FORM, bool F8 = false>
+// 256 bytes that begin apart: 41.2, 42.8 and 45.7 us of 2 x 14336 x 4096, with 16 in
+// chunks of 512 41.3, 43.8 and 46.4.
+template <Form FORM, bool F8 = false, bool F8X = false>
 void run(const LayerRows& m) {
 #define HELIX_LR(MR, NI, CHUNK)                                              \
-  hipLaunchKernelGGL((layer_rows_kernel<MR, NI, CHUNK, FORM, F8>),           \
+  hipLaunchKernelGGL((layer_rows_kernel<MR, NI, CHUNK, FORM, F8, F8X>),      \
                      dim3(m.N / (FORM == GLU ? 8 * NI : 16 * NI)), dim3(NT), \
                      0, at::hip::getCurrentHIPStream(), m)
   constexpr int NI = FORM == GLU ? 4 : 1, MORE = FORM == QKV ? 2 : NI;
-  constexpr int CHUNK = FORM == GLU ? 128 : 256;
+  constexpr int CHUNK = FORM == GLU ? 256 : 512;
   if (m.M <= 4) HELIX_LR(4, NI, CHUNK);
   else if (m.M <= 8) HELIX_LR(8, MORE, CHUNK);
-  else HELIX_LR(16, MORE, CHUNK);
+  else if (m.M <= 16) HELIX_LR(16, MORE, CHUNK);
+  else if constexpr (FORM == QKV) HELIX_LR(32, 2, 256);
 #undef HELIX_LR
 }
 
@@ -402,14 +443,26 @@ torch::Tensor layer_rows_glu(torch::Tensor x, torch::Tensor w, OptT squares,
   return out;
 }
 
-// Heads of x w^T f + bias, turned, to q (and k, v) and the pages of slots.
+// Heads of x w^T f + bias, turned, to q (and k, v) and the pages of slots. x and w
+// are bf16, or e4m3 with scales of their rows; squares of up to 16 rows of bf16.
 void layer_rows_qkv(torch::Tensor x, torch::Tensor w, OptT bias, OptT squares,
                     double eps, torch::Tensor positions, torch::Tensor cos_sin,
                     torch::Tensor q, OptT k, OptT v, OptT k_cache,
                     OptT v_cache, OptT slots, int64_t num_q, int64_t num_kv,
-                    int64_t head_dim) {
+                    int64_t head_dim, OptT x_scale, OptT w_scale) {
   const c10::DeviceGuard on(x.device());
-  LayerRows m = rows_of(x, w, squares, eps);
+  const bool f8x = x_scale.has_value();
+  LayerRows m = rows_of(x, w, squares, eps,
+                        f8x ? torch::kUInt8 : torch::kBFloat16, MOST_ROWS_QKV);
+  TORCH_CHECK(w_scale.has_value() == f8x &&
+              (m.squares == nullptr || (!f8x && m.M <= MOST_ROWS)));
+  if (f8x) {
+    check(*x_scale, x, torch::kFloat32, 4);
+    check(*w_scale, x, torch::kFloat32, 4);
+    TORCH_CHECK(x_scale->numel() == m.M && w_scale->numel() == m.N);
+    m.xs = x_scale->data_ptr<float>();
+    m.ws = w_scale->data_ptr<float>();
+  }
   TORCH_CHECK(num_q > 0 && num_kv > 0 && head_dim > 0 && head_dim % 32 == 0 &&
               (num_q + 2 * num_kv) * head_dim == m.N);
   m.Hq = num_q;
@@ -457,6 +510,12 @@ void layer_rows_qkv(torch::Tensor x, torch::Tensor w, OptT bias, OptT squares,
     m.slots = slots->data_ptr<int64_t>();
   }
   m.shift = (m.bs & (m.bs - 1)) == 0 ? __builtin_ctz(m.bs) : -1;
-  if (f8) run<QKV, true>(m);
-  else run<QKV>(m);
+  if (f8x) {
+    if (f8) run<QKV, true, true>(m);
+    else run<QKV, false, true>(m);
+  } else if (f8) {
+    run<QKV, true>(m);
+  } else {
+    run<QKV>(m);
+  }
 }

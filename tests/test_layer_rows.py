@@ -61,14 +61,16 @@ def test_glu(m, n, k, parts):
     (4, 256, 4, 4, 2, 64, 16, True, True, True),
     (5, 512, 0, 6, 2, 96, 24, False, True, True),
     (8, 3584, 224, 28, 4, 128, 16, True, True, False),
-    (16, 1024, 64, 8, 8, 32, 8, False, False, True)])
+    (16, 1024, 64, 8, 8, 32, 8, False, False, True),
+    (17, 512, 0, 4, 2, 64, 16, False, True, True),
+    (32, 4096, 0, 32, 8, 128, 16, True, False, False)])
 def test_qkv(m, k, parts, hq, hkv, d, bs, fp8, bias, want_kv):
     r, x, sq, inv = _rows(m, k, parts)
     n = (hq + 2 * hkv) * d
     w = (r(n, k) * 0.02).bfloat16()
     b = r(n).bfloat16() if bias else None
-    cs = ops.make_cos_sin_cache(d, 512, 10000.0).to(DEV)
-    pos = torch.arange(m, device=DEV) * 29 + 3
+    cs = ops.make_cos_sin_cache(d, 1024, 10000.0).to(DEV)
+    pos = torch.arange(m, device=DEV) * 29 + 3          # up to 902
     slots = torch.randperm(4 * m * bs, device=DEV)[:m]
     slots[m // 2] = -1 if m > 1 else slots[m // 2]      # padding: not written
     kc, vc = (torch.zeros(4 * m, hkv, bs, d, device=DEV, dtype=torch.uint8 if
@@ -100,6 +102,41 @@ def test_qkv(m, k, parts, hq, hkv, d, bs, fp8, bias, want_kv):
             _near(got_rows, want[there])
         got[at // bs, :, at % bs] = 0
         assert not got.any()
+
+
+@pytest.mark.parametrize("m,k,hq,hkv,d,fp8", [
+    (1, 512, 4, 2, 64, False), (4, 4096, 32, 8, 128, False),
+    (8, 1536, 4, 4, 32, True), (13, 512, 6, 2, 96, False),
+    (17, 1024, 4, 2, 64, True), (32, 4096, 32, 8, 128, False)])
+def test_qkv_bytes(m, k, hq, hkv, d, fp8):
+    r, x, _, _ = _rows(m, k)
+    n = (hq + 2 * hkv) * d
+    w8, ws = ops.quantize_fp8((r(n, k) * 0.02).bfloat16())
+    x8 = ops.Quantized(*ops.quantize_fp8(x))
+    cs = ops.make_cos_sin_cache(d, 512, 10000.0).to(DEV)
+    pos = torch.arange(m, device=DEV) * 15
+    kc, vc = (torch.zeros(m, hkv, 16, d, device=DEV, dtype=torch.uint8 if fp8
+                          else torch.bfloat16) for _ in range(2))
+    slots = torch.randperm(m * 16, device=DEV)[:m]
+    q, ko, vo = ops.rows_qkv(pos, x8, w8, None, cs, hq, hkv, d, (kc, vc),
+                             slots, True, ws)
+    back = lambda b, s: (b.view(torch.float8_e4m3fn).double()  # noqa: E731
+                         * s.double()[:, None])
+    y = (back(*x8) @ back(w8, ws).t()).view(m, -1, d)
+    c, s = cs[pos].double()[:, None].chunk(2, -1)
+    u, v = y.chunk(2, -1)
+    t = torch.cat([u * c - v * s, v * c + u * s], -1)
+    _near(q, t[:, :hq])
+    _near(ko, t[:, hq:hq + hkv])
+    _near(vo, y[:, hq + hkv:])
+    for cache, want in ((kc, ko), (vc, vo)):
+        got = cache[slots // 16, :, slots % 16]
+        assert torch.equal(got, ops.kv_fp8_quant(want) if fp8 else want) \
+            or fp8       # of sums before they were rounded to bf16
+        if fp8:
+            got = got.view(torch.float8_e4m3fn).double()
+            assert ((got - want.double()).abs()
+                    <= 2 ** -3.9 * want.double().abs() + 2 ** -9).all()
 
 
 def test_refuses():
