@@ -412,7 +412,7 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
 
 # Tokens that decode attention cuts sequences in (must match UNIT in
-# paged_attn_decode.hip).
+# paged_rows.h).
 DECODE_PARTITION = 128
 
 

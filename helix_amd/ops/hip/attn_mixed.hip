@@ -29,8 +29,7 @@ __global__ __launch_bounds__(prefill::NT, 2) void attn_mixed_kernel(
   if (at < 0) {
     prefill::queries<D, true>(out, qp, k, v, pm, blockIdx.x, lds);
   } else {
-    const int g = at / pieces;
-    paged::rows<D, G, F8, true>(qd, kc, vc, dm, at - g * pieces, g,
+    paged::rows<D, G, F8, true>(qd, kc, vc, dm, at, pieces,
                                 *reinterpret_cast<paged::Shared<D, G>*>(lds));
   }
 }
@@ -62,13 +61,13 @@ bool attn_mixed(torch::Tensor out_p, torch::Tensor q_p, torch::Tensor k,
   auto stream = at::hip::getCurrentHIPStream();
 #define HELIX_AM(G, F8)                                                      \
   hipLaunchKernelGGL((attn_mixed_kernel<G, F8>),                             \
-                     dim3(p.grid + d.grid.x * d.grid.y), dim3(prefill::NT),  \
+                     dim3(p.grid + d.pieces * d.m.Hkv), dim3(prefill::NT),   \
                      prefill::lds_of(D), stream, (uint16_t*)out_p.data_ptr(),\
                      (const uint16_t*)q_p.data_ptr(),                        \
                      (const uint16_t*)k.data_ptr(),                          \
                      (const uint16_t*)v.data_ptr(), p.m, p.grid,             \
                      (const uint16_t*)q_d.data_ptr(), k_cache.data_ptr(),    \
-                     v_cache.data_ptr(), d.m, (int)d.grid.x)
+                     v_cache.data_ptr(), d.m, d.pieces)
   if (G == 4) {
     if (d.f8) HELIX_AM(4, true); else HELIX_AM(4, false);
   } else {

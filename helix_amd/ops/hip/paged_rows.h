@@ -27,7 +27,8 @@
 //  - Work is cut by the lengths themselves, on the device, because a captured
 //    graph only knows its bucket: all (sequence, head) pairs share TARGET
 //    workgroups in proportion to their tokens, in units of 128. Sequences in
-//    one piece are written at once, others are merged by a second launch.
+//    one piece are written at once, others are merged by a second launch. Short
+//    or many rows are not cut at all (see `whole`).
 //
 // Before, a partition was a share of the bucket, its two waves met at three
 // barriers per 128 tokens and the value product waited for the softmax of all
@@ -284,12 +285,12 @@ struct Shared {
   float st[2][NW][G];
 };
 
-// Work of workgroup `block` of KV head g.
+// Work of workgroup `at`; each KV head has `pieces` of them.
 template <int D, int G, bool F8, bool PAGE8>
 __device__ __forceinline__ void rows(const uint16_t* __restrict__ q,
                                      const void* __restrict__ kc,
                                      const void* __restrict__ vc,
-                                     const Rows& m, int block, int g,
+                                     const Rows& m, int at, int pieces,
                                      Shared<D, G>& lds) {
   constexpr int NC = D / 32;                  // inner steps of the scores
   constexpr int DPL = D / 16;                 // value dimensions of a lane
@@ -304,8 +305,14 @@ __device__ __forceinline__ void rows(const uint16_t* __restrict__ q,
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lo = lane & 15, hi = lane >> 4;
+  // The heads of an uncut row follow each other, so that a long row's lie on different
+  // XCDs (32 heads on 8, one of 1000 beside 63 of 100 27.8 us before and 18.9, 256
+  // of 20..1000 104.4 and 99.6).
+  const int per_g = m.split ? pieces : m.Hkv;
+  const int high = at / per_g, low = at - high * per_g;
+  const int g = m.split ? high : low;
   int seq, part, parts;
-  if (!find(m, block, seq, part, parts)) return;
+  if (!find(m, m.split ? low : high, seq, part, parts)) return;
   // The same in all lanes: scalar registers, so that a wave more fits a SIMD. Not
   // for up to four heads of bf16, which have waves enough and lose by more (32
   // heads of 64 on 8, 16 of 100..6000 24 us and 26; 16 on 16 of 128, 1 of 900
@@ -623,8 +630,7 @@ __global__ __launch_bounds__(NT) void paged_merge_kernel(Rows m, int Hq) {
 // copied where it does not begin on 16 bytes.
 struct Plan {
   Rows m{};
-  dim3 grid;
-  int Hq, D, G;
+  int pieces, Hq, D, G;                       // pieces: workgroups of a KV head
   bool f8;
 };
 
@@ -681,13 +687,26 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor k_cache,
   m.limit = (int)std::min<int64_t>(
       cdiv((int)max_len_hint, UNIT) * UNIT, (int64_t)m.max_blocks * m.bs);
   m.mul = (float)scale * LOG2E;
-  // Nothing to cut where a row is at most a unit long, nor where the rows
-  // alone fill the chip twice and none can be long: cuts cost 512 rows of
-  // 513..640 5 us, most of it the merge launch.
+  // A row in one workgroup needs no search for its piece and no second launch, but
+  // takes as long as its length, and the chip waits for the longest. Cut only where
+  // that is the longer of the two; the graph knows rows and bound, not lengths. us
+  // cut and uncut, 32 heads on 8 of 128, lengths up to the bound evenly spread:
+  //   512 and below: 1 row of 512 10.1 and 10.1, of 300 10.0 and 8.4; 16 rows 13.3
+  //     and 10.4, 64 28.0 and 17.3. With 8 heads of 128 a row's own time is longer:
+  //     1 row of 512 13.0 and 14.4, 8 13.6 and 14.6, but 16 16.7 and 14.7.
+  //   1024: 8 rows 13.3 and 16.1, 16 17.0 and 16.4, 32 22.8 and 18.2, 128 61.3 and
+  //     53.5 (e4m3 40.1 and 28.5). The least good are single long rows: one of 1000
+  //     beside 47 of 100 16.9 and 18.9.
+  //   2048: 16 heads on 8, 128 rows 103 and 108, 256 198 and 187; one of 2036 beside
+  //     255 of 100 46 and 37.
   const int most = cdiv((int)(window > 0 ? std::min(max_len_hint, window + KT)
                                          : max_len_hint), UNIT);
-  m.split = m.max_parts > 1 && most > 1 &&
-            !(B * Hkv >= 2 * TARGET && most <= 8);
+  const int64_t rows = (int64_t)B * Hkv;
+  const bool whole = most <= 1 ||
+                     (most <= 4 && (rows >= 128 || G * D < 1024)) ||
+                     (most <= 8 && rows >= 128) ||
+                     (most <= 16 && rows >= 2 * TARGET);
+  m.split = m.max_parts > 1 && !whole;
   const int64_t pieces = (int64_t)B * Hq * m.max_parts;
   TORCH_CHECK(!m.split || (tmp_out.is_contiguous() && tmp_ml.is_contiguous() &&
                            tmp_out.numel() >= pieces * D &&
@@ -698,7 +717,7 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor k_cache,
     TORCH_CHECK(t.is_cuda() && t.device() == q.device(),
                 "everything on one GPU");
   // a workgroup without a piece costs its search, so no more than can be
-  p.grid = dim3(m.split ? std::min(B * most, B + TARGET / Hkv + 1) : B, Hkv);
+  p.pieces = m.split ? std::min(B * most, B + TARGET / Hkv + 1) : B;
   return p;
 }
 
