@@ -49,8 +49,8 @@ def _plain(emb: nn.Module) -> bool:
 def _first_pays(cu: list) -> bool:
     """Whether the last block is computed for first rows only: three launches more,
     of fewer rows. us of the model (bge-base) with all rows and so: 1 text of 511
-    689 and 691, 3 of 400 763 and 761, 64 of 20 718 and 718, 64 of 40 905 and 888,
-    64 of 250 3283 and 3100."""
+    658 and 653, 3 of 400 755 and 746, 64 of 20 719 and 717, 64 of 40 933 and 915,
+    64 of 250 3512 and 3322."""
     return cu[-1] >= max(1024, 8 * (len(cu) - 1)) and all(
         b > a for a, b in zip(cu, cu[1:]))
 
@@ -152,15 +152,15 @@ class BertEmbeddingModel(nn.Module):
             x = self.word_emb(input_ids) + self.pos_emb(positions)
             x = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b,
                                self.cfg.layer_norm_eps)
-        for layer in self.layers[:-1]:
+        last = len(self.layers) - 1
+        for i, layer in enumerate(self.layers):
+            if i == last and self.cfg.pooling != "mean" and _first_pays(cu):
+                first = layer.first_rows(x, cu_seqlens, max_len)
+                if first is not None:
+                    emb = ops.text_pool(*first)
+                    if emb is not None:
+                        return emb
             x = layer(x, cu_seqlens, max_len)
-        if self.cfg.pooling != "mean" and _first_pays(cu):
-            first = self.layers[-1].first_rows(x, cu_seqlens, max_len)
-            if first is not None:
-                emb = ops.text_pool(*first)
-                if emb is not None:
-                    return emb
-        x = self.layers[-1](x, cu_seqlens, max_len)
         if self.cfg.pooling == "mean":
             emb = torch.stack([x[s:e].float().mean(0)
                                for s, e in zip(cu, cu[1:])])
