@@ -28,7 +28,8 @@
 // 32 heads on 8 of 128, us of the first kernel (64 queries, values transposed
 // element by element) -> products of 16x16 with addresses computed per tile
 // (340 vector instructions) -> with the next tile's loads waited for by reads of
-// LDS -> now (TFLOP/s now; the last two on one card): 1 x 8192 2551 -> 645 ->
+// LDS -> as now but for the heads' order (TFLOP/s; the last two on one card): 1 x
+// 8192 2551 -> 645 ->
 // 579 -> 568 (968), 8 x 2048 1918 -> 413 -> 364 -> 341 (806), 31 of 400..620
 // 440 -> 188 -> 168 -> 154 (467), 1500 behind 5001 with a window of 4096 466 ->
 // 173 -> 136 -> 130 (773). 12 heads of 64, 64 texts of 20..500: 178 -> 68 -> 52
@@ -68,7 +69,7 @@ struct Prefill {
   const int* cu_q;             // [B + 1] query rows
   const int* cu_k;             // [B + 1] key rows (>= query rows)
   int64_t q_stride, k_stride, v_stride;       // of a row, in elements
-  int Hq, G, q_tiles, seqs, window;
+  int Hq, G, groups, q_tiles, seqs, window;   // groups: of G heads
   bool flip;                   // negative scale: of negated queries
   bool spread;                 // groups of heads go round the XCDs
   float mul, far_mul;          // |scale| * log2(e); a power of two above it
@@ -135,15 +136,17 @@ __device__ __forceinline__ void queries(uint16_t* __restrict__ out,
   uint16_t* const kl[2] = {tiles, tiles + KT * D};
   uint16_t* const vl[2] = {tiles + 2 * KT * D, tiles + 3 * KT * D};
   const int xcd = block & 7, at = block >> 3;
-  int b, h, tile;
+  int b, g, h, tile;
   if (m.spread) {
     // a group's heads, latest queries first, behind the XCD's groups before
-    const int all = m.G * m.q_tiles, in = at % all, groups = m.Hq / m.G;
-    const int group = at / all * 8 + xcd;
-    if (group >= m.seqs * groups) return;
-    b = group / groups;
-    tile = in / m.G;
-    h = (group - b * groups) * m.G + in - tile * m.G;
+    // (divisions are 0.2 us of a launch: as few as there can be, 8 x 288 10.74 -> 10.56)
+    const int all = m.G * m.q_tiles, before = at / all, in = at - before * all;
+    const int group = before * 8 + xcd;
+    if (group >= m.seqs * m.groups) return;
+    b = group / m.groups;
+    tile = m.G == 1 ? in : in / m.G;
+    g = group - b * m.groups;
+    h = g * m.G + in - tile * m.G;
   } else {
     const int total = m.seqs * m.Hq, chunk = cdiv(total, 8);
     const int sh = xcd * chunk + at / m.q_tiles;
@@ -151,8 +154,9 @@ __device__ __forceinline__ void queries(uint16_t* __restrict__ out,
     b = sh / m.Hq;
     h = sh - b * m.Hq;
     tile = at % m.q_tiles;
+    g = h / m.G;
   }
-  const int g = h / m.G, q0 = (m.q_tiles - 1 - tile) * QT;
+  const int q0 = (m.q_tiles - 1 - tile) * QT;
   const int row0 = m.cu_q[b], qlen = m.cu_q[b + 1] - row0;
   if (q0 >= qlen) return;
   const int key0 = m.cu_k[b], klen = m.cu_k[b + 1] - key0;
@@ -412,6 +416,7 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor& k,
   // Groups of heads that share keys go round the XCDs, and each sees some of every
   // sequence, whatever their lengths; a few that leave XCDs without one are cut
   // into heads.
+  m.groups = Hkv;
   const int groups = B * Hkv;
   m.spread = groups % 8 == 0 || groups >= 32;
   p.grid = m.spread ? 8 * cdiv(groups, 8) * m.G * m.q_tiles
