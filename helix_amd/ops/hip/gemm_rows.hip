@@ -29,7 +29,8 @@
 //   M 16   12.7 (15.7)   8.6 (15.6)   42.7 (65.1)   23.6 (27.3)
 //   M 32   14.4 (16.3)   9.3 (13.9)   46.8 (54.2)   24.9 (33.8)
 //   M 64   17.6 (18.0)  12.2 (15.2)   54.0 (52.3)   31.9 (41.9)
-// Tiles (gemm_ring.h) have taken over bf16 from 17 rows on, but for the stretches
+// A language model's layers of up to 16 rows have kernels of their own
+// (layer_rows.hip). Tiles (gemm_ring.h) have taken over bf16 from 17 rows on, but for the stretches
 // of small products and of deep ones with few columns, up to 48 rows of wide
 // matrices and up to 64 of vocabularies whose rows are 4 or 8 KB (_streams_pay in
 // ops/__init__.py). From 65 rows on a wave has 32 columns, so that x is read from

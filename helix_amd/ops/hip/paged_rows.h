@@ -702,15 +702,17 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor k_cache,
   const int most = cdiv((int)(window > 0 ? std::min(max_len_hint, window + KT)
                                          : max_len_hint), UNIT);
   const int64_t rows = (int64_t)B * Hkv;
-  const bool whole = most <= 1 ||
-                     (most <= 4 && (rows >= 128 || G * D < 1024)) ||
+  const bool cuts = m.max_parts > 1 && most > 1 &&
+                    !(rows >= 2 * TARGET && most <= 8);
+  const bool whole = (most <= 4 && (rows >= 128 || G * D < 1024)) ||
                      (most <= 8 && rows >= 128) ||
                      (most <= 16 && rows >= 2 * TARGET);
-  m.split = m.max_parts > 1 && !whole;
+  m.split = cuts && !whole;
+  // a workspace is looked at whether or not these rows would be cut
   const int64_t pieces = (int64_t)B * Hq * m.max_parts;
-  TORCH_CHECK(!m.split || (tmp_out.is_contiguous() && tmp_ml.is_contiguous() &&
-                           tmp_out.numel() >= pieces * D &&
-                           tmp_ml.numel() >= pieces * 2),
+  TORCH_CHECK(!cuts || (tmp_out.is_contiguous() && tmp_ml.is_contiguous() &&
+                        tmp_out.numel() >= pieces * D &&
+                        tmp_ml.numel() >= pieces * 2),
               "a workspace of [B, Hq, parts, D] and [B, Hq, parts, 2]");
   for (const auto& t : {q, out, k_cache, v_cache, block_tables, seq_lens,
                         tmp_out, tmp_ml})
