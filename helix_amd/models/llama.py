@@ -321,13 +321,13 @@ class DecoderLayer(nn.Module):
         self.eps = cfg.rms_norm_eps
 
     def unseen(self) -> bool:
-        """Whether all of it is as written here: nobody sees its rows but those who
-        ask for the result."""
+        """Whether all within it is as written here: nobody sees its rows but those
+        who ask for the result. Asked of a layer that is _own itself: a module
+        around one may hand on the question, but not its answer."""
         a, m = self.attn, self.mlp
-        return (_own(self, DecoderLayer) and _own(a, Attention)
-                and _own(m, MLP) and all(
-                    _own(p, HLinear, FP8Linear) for p in
-                    (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj)))
+        return (_own(a, Attention) and _own(m, MLP) and all(
+            _own(p, HLinear, FP8Linear) for p in
+            (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj)))
 
     def few(self, x) -> bool:
         """Whether these rows go through the layer in launches that take norm,
@@ -416,7 +416,9 @@ class LlamaForCausalLM(nn.Module):
         launches, so this is for prompts of which at least half leave."""
         if input_ids.shape[0] >= 256 and \
                 0 < 2 * rows.numel() <= input_ids.shape[0] and \
-                _own(self, LlamaForCausalLM) and self.layers[-1].unseen():
+                _own(self, LlamaForCausalLM) and \
+                _own(self.layers[-1], DecoderLayer) and \
+                self.layers[-1].unseen():
             return self._hidden(input_ids, kv_caches, meta, rows)
         return self(input_ids, kv_caches, meta)[rows]
 
@@ -428,13 +430,13 @@ class LlamaForCausalLM(nn.Module):
         for i, layer in enumerate(self.layers):
             cache = kv_caches[i] if kv_caches is not None else None
             own = _own(layer, DecoderLayer)
-            extra = ["sums"] if own else []
+            extra = {"form": "sums"} if own else {}
             if few[i]:
-                extra += [True, self.layers[i + 1].input_norm_w
-                          if few[i + 1] else None]
+                extra.update(few=True, after=self.layers[i + 1].input_norm_w
+                             if few[i + 1] else None)
             elif rows is not None and i + 1 == len(self.layers):
-                extra += [False, None, rows]
-            x, residual = layer(x, residual, self.cos_sin, cache, meta, *extra)
+                extra["rows"] = rows
+            x, residual = layer(x, residual, self.cos_sin, cache, meta, **extra)
         if not own:                # what a hook has kept stays as it was
             x, residual = x.clone(), residual.clone()
         return ops.fused_add_rms_norm(x, residual, self.final_norm_w,

@@ -79,3 +79,65 @@ def test_first_rows_of_texts(lens, h, inner, heads):
         got, starts = ops.text_block_first(*args)
     assert starts.tolist() == list(range(len(lens) + 1))
     assert ((got.float() - want).norm() / want.norm()).item() < 5 * 2 ** -9
+
+
+class Delegating(torch.nn.Module):
+    """A wrapper in the manner of adapters: a forward of its own, every other
+    attribute the inner module's."""
+
+    def __init__(self, inner, add=0.0):
+        super().__init__()
+        self.inner, self.add, self.calls = inner, add, 0
+
+    def __getattr__(self, name):
+        try:
+            return super().__getattr__(name)
+        except AttributeError:
+            return getattr(super().__getattr__("inner"), name)
+
+    def forward(self, *args):
+        self.calls += 1
+        out = self.inner(*args)
+        return (out[0] + self.add, *out[1:]) if isinstance(out, tuple) \
+            else out + self.add
+
+
+class Plain(torch.nn.Module):
+    """A layer in place of the model's with nothing but a forward."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, *args):
+        return self.inner(*args)
+
+
+def _engine(model):
+    from helix_amd.engine.engine import EngineConfig, LLMEngine
+    return LLMEngine(EngineConfig(model="tiny", max_num_seqs=4,
+                                  max_model_len=512, kv_cache_blocks=64,
+                                  eos_token_id=-1), "cpu", model=model)
+
+
+def _last_scores(eng, n):
+    """Scores behind the last of n tokens, through the engine's step."""
+    return eng.extend([("a", [t % 500 for t in range(n)], [n - 1])])
+
+
+WRAPPERS = {"plain": Plain, "delegating": Delegating,
+            "compiled": lambda m: torch.compile(m, backend="eager")}
+
+
+@pytest.mark.parametrize("wrap", list(WRAPPERS))
+@pytest.mark.parametrize("n", [200, 300])
+def test_other_last_layer(wrap, n):
+    """It gets and gives all rows, and the scores are those asked for."""
+    model = LlamaForCausalLM(PRESETS["tiny"]).init_random(3)
+    ids, meta = _step([n])
+    want = model.compute_logits(model(ids, _caches(model.cfg, n),
+                                      meta)[n - 1:])
+    model.layers[-1] = WRAPPERS[wrap](model.layers[-1])
+    got = _last_scores(_engine(model), n)
+    assert got.shape == want.shape
+    torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
