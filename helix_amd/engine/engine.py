@@ -482,9 +482,10 @@ class LLMEngine:
             self.model(ids, self.kv.caches, meta)
             return None
         at = torch.tensor(rows, dtype=torch.int64, device=dev)
-        some = getattr(self.model, "forward_rows", None)
-        if some is not None:
-            hidden = some(ids, self.kv.caches, meta, at)
+        # of the model itself: one around it that hands on attributes would not
+        # be called
+        if hasattr(type(self.model), "forward_rows"):
+            hidden = self.model.forward_rows(ids, self.kv.caches, meta, at)
         else:
             hidden = self.model(ids, self.kv.caches, meta)[at]
         return self.model.compute_logits(hidden)

@@ -141,3 +141,25 @@ def test_other_last_layer(wrap, n):
     got = _last_scores(_engine(model), n)
     assert got.shape == want.shape
     torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("wrap", ["delegating", "compiled"])
+@pytest.mark.parametrize("n", [200, 300])
+def test_other_model(wrap, n):
+    """A wrapper around the whole model is what the engine calls."""
+    model = LlamaForCausalLM(PRESETS["tiny"]).init_random(3)
+    ids, meta = _step([n])
+    hidden = model(ids, _caches(model.cfg, n), meta)[n - 1:]
+    eng = _engine(model)
+    if wrap == "compiled":
+        graphs = []
+        eng.model = torch.compile(
+            model, backend=lambda g, _: graphs.append(g) or g.forward)
+        add = 0.0
+    else:
+        eng.model = Delegating(model, add=0.25)
+        add = 0.25
+    got = _last_scores(eng, n)
+    assert graphs if wrap == "compiled" else eng.model.calls == 1
+    torch.testing.assert_close(got, model.compute_logits(hidden + add),
+                               atol=1e-5, rtol=1e-5)
