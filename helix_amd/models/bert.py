@@ -81,8 +81,9 @@ class BertLayer(nn.Module):
 
     def first_rows(self, x, cu, max_len):
         """The first row of each text, all of which have tokens, and the
-        boundaries of texts of a row each; None where forward is to be asked."""
-        if not _own(self, BertLayer) or tuple(self._parameters) != self.PARAMS:
+        boundaries of texts of a row each; None where forward is to be asked.
+        For a layer that is _own: a hook or a module around it would not see it."""
+        if tuple(self._parameters) != self.PARAMS:
             return None
         return ops.text_block_first(x, cu, max_len, self.cfg.num_heads,
                                     self.scale, self.cfg.layer_norm_eps,
@@ -154,7 +155,8 @@ class BertEmbeddingModel(nn.Module):
                                self.cfg.layer_norm_eps)
         last = len(self.layers) - 1
         for i, layer in enumerate(self.layers):
-            if i == last and self.cfg.pooling != "mean" and _first_pays(cu):
+            if i == last and self.cfg.pooling != "mean" and \
+                    _own(layer, BertLayer) and _first_pays(cu):
                 first = layer.first_rows(x, cu_seqlens, max_len)
                 if first is not None:
                     emb = ops.text_pool(*first)

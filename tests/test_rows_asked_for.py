@@ -163,3 +163,27 @@ def test_other_model(wrap, n):
     assert graphs if wrap == "compiled" else eng.model.calls == 1
     torch.testing.assert_close(got, model.compute_logits(hidden + add),
                                atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("wrap", list(WRAPPERS))
+@pytest.mark.parametrize("pooling", ["cls", "mean"])
+def test_other_last_layer_of_texts(monkeypatch, wrap, pooling):
+    """The text encoder's: its forward is called, with all rows. First rows alone
+    are computed on the GPU; a stand-in counts who asks for them."""
+    from dataclasses import replace
+    from helix_amd import ops
+    from helix_amd.models.bert import BERT_PRESETS, BertEmbeddingModel
+    asked = []
+    monkeypatch.setattr(ops, "text_block_first",
+                        lambda x, *a: asked.append(x.shape[0]))
+    model = BertEmbeddingModel(replace(BERT_PRESETS["tiny-bert"],
+                                       pooling=pooling)).init_random(5)
+    cu = torch.arange(0, 1281, 128, dtype=torch.int32)
+    ids = torch.arange(1280) % 500
+    want = model(ids, cu, 128)
+    assert asked == ([1280] if pooling == "cls" else [])
+    model.layers[-1] = WRAPPERS[wrap](model.layers[-1])
+    torch.testing.assert_close(model(ids, cu, 128), want, atol=1e-5, rtol=1e-5)
+    assert asked == ([1280] if pooling == "cls" else [])
+    if wrap == "delegating":
+        assert model.layers[-1].calls == 1
