@@ -189,9 +189,9 @@ def text_block(x: torch.Tensor, cu: torch.Tensor, max_len: int, heads: int,
 
 def text_block_first(x: torch.Tensor, cu: torch.Tensor, max_len: int,
                      heads: int, scale: float, eps: float, params: list):
-    """text_block of texts that all have tokens, for one who only asks for the
-    first row of each: (those rows, cu of texts of a row each), or None as
-    above."""
+    """text_block for one who only asks for the first row of each text: (those
+    rows, cu of texts of a row each), or None as above. A text without tokens is
+    NaN."""
     if x.is_cuda and not _seen_by_torch():
         out = _native().text_block_first(x, cu, max_len, heads, scale, eps,
                                          params)

@@ -132,17 +132,24 @@ __global__ __launch_bounds__(NT) void text_pool_kernel(
 }
 
 // Rows cu[:-1] of x side by side, and their boundaries 0, 1, ..: a workgroup each,
-// and one more for the last of those.
+// and one more for the last of those. A text without tokens, or with its first
+// outside of x, is no number: the host has not seen the boundaries.
 __global__ __launch_bounds__(NT) void text_first_kernel(
     uint16_t* __restrict__ out, int* __restrict__ starts,
-    const uint16_t* __restrict__ x, const int* __restrict__ cu, int B, int H) {
+    const uint16_t* __restrict__ x, const int* __restrict__ cu, int B, int T,
+    int H) {
   const int s = blockIdx.x;
   if (threadIdx.x == 0) starts[s] = s;
   if (s == B) return;
-  const int64_t from = (int64_t)cu[s] * H, to = (int64_t)s * H;
-  for (int c = threadIdx.x * 8; c < H; c += NT * 8)
-    *reinterpret_cast<u16x8*>(out + to + c) =
-        *reinterpret_cast<const u16x8*>(x + from + c);
+  const int first = cu[s];
+  const bool there = first >= 0 && first < T && cu[s + 1] > first;
+  const int64_t from = (int64_t)(there ? first : 0) * H, to = (int64_t)s * H;
+  for (int c = threadIdx.x * 8; c < H; c += NT * 8) {
+    u16x8 v = *reinterpret_cast<const u16x8*>(x + from + c);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = there ? v[i] : (uint16_t)0x7FC0;
+    *reinterpret_cast<u16x8*>(out + to + c) = v;
+  }
 }
 
 struct Image {
@@ -338,12 +345,13 @@ bool text_pool(torch::Tensor out, torch::Tensor x, torch::Tensor cu) {
 }
 
 // out[B, H], starts[B + 1]: rows cu[:-1] of x and the boundaries of texts of a token
-// each. The texts have tokens; x and out are packed rows on 16-byte boundaries.
+// each. A text without tokens is NaN; x and out are packed rows on 16-byte boundaries.
 void text_first(torch::Tensor out, torch::Tensor starts, torch::Tensor x,
                 torch::Tensor cu) {
   const int64_t B = cu.numel() - 1;
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 &&
               table(x, x, x.size(0), x.size(1)) && x.size(1) % 8 == 0 &&
+              x.size(0) >= 1 && x.size(0) <= INT32_MAX &&
               numbers(cu, torch::kInt32, x) && cu.dim() == 1 && B >= 1 &&
               table(out, x, B, x.size(1)) &&
               numbers(starts, torch::kInt32, x) && starts.numel() == B + 1,
@@ -351,7 +359,8 @@ void text_first(torch::Tensor out, torch::Tensor starts, torch::Tensor x,
   hipLaunchKernelGGL(text_first_kernel, dim3(B + 1), dim3(NT), 0,
                      at::hip::getCurrentHIPStream(), (uint16_t*)out.data_ptr(),
                      starts.data_ptr<int>(), (const uint16_t*)x.data_ptr(),
-                     cu.data_ptr<int>(), (int)B, (int)x.size(1));
+                     cu.data_ptr<int>(), (int)B, (int)x.size(0),
+                     (int)x.size(1));
 }
 
 // out[B patches, K]: patches of the latents (bf16 or fp32) as rows.

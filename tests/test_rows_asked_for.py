@@ -187,3 +187,23 @@ def test_other_last_layer_of_texts(monkeypatch, wrap, pooling):
     assert asked == ([1280] if pooling == "cls" else [])
     if wrap == "delegating":
         assert model.layers[-1].calls == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[0, 40, 0, 0, 7, 0], [0, 0], [1]])
+def test_first_rows_of_texts_without_tokens(lens):
+    """Of a text without tokens, the last one too, there is no row: NaN, and
+    nothing behind the rows is read. The others as above."""
+    from helix_amd.models.bert import BERT_PRESETS, BertEmbeddingModel
+    layer = BertEmbeddingModel(BERT_PRESETS["tiny-bert"]).init_random(
+        5).bfloat16().cuda().layers[0]
+    x = torch.randn(max(sum(lens), 1), 128).bfloat16().cuda()
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(),
+                      dtype=torch.int32, device="cuda")
+    full = [i for i, n in enumerate(lens) if n]
+    with torch.inference_mode():
+        want = layer(x, cu, max(lens))[cu[full].long()].float()
+        got, starts = layer.first_rows(x, cu, max(lens))
+    assert starts.tolist() == list(range(len(lens) + 1))
+    assert got[[i for i, n in enumerate(lens) if not n]].isnan().all()
+    assert (got[full].float() - want).norm() <= 5 * 2 ** -9 * want.norm()
