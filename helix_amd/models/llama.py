@@ -210,11 +210,12 @@ class Attention(nn.Module):
         if mixed:
             n = meta.num_decode
             o = torch.empty_like(q)
+            both = self._attends_as_here()
             if want_kv:
                 k, v = k[n:], v[n:]
-            else:
+            elif both:
                 k, v = self._gather(q, kv_cache, prefill)
-            if not self._attend_both(q, k, v, kv_cache, meta, o):
+            if not (both and self._attend_both(q, k, v, kv_cache, meta, o)):
                 self._attend_decode(q[:n], kv_cache, meta.decode, o[:n])
                 self._attend_prefill(q[n:], k, v, kv_cache, prefill, o[n:])
         elif meta.is_prefill:
@@ -250,6 +251,12 @@ class Attention(nn.Module):
         cache (new tokens were just written)."""
         return ops.gather_kv(*kv_cache, meta.gather_blk, meta.gather_off,
                              q.dtype)
+
+    def _attends_as_here(self) -> bool:
+        """Whether nobody has put a way to attend of their own in place of these."""
+        return all(name not in self.__dict__ and
+                   getattr(type(self), name) is getattr(Attention, name)
+                   for name in ("_attend_prefill", "_attend_decode"))
 
     def _attend_both(self, q, k, v, kv_cache, meta, out) -> bool:
         """Replies and portions in one launch, or False and nothing done."""

@@ -207,3 +207,45 @@ def test_first_rows_of_texts_without_tokens(lens):
     assert starts.tolist() == list(range(len(lens) + 1))
     assert got[[i for i, n in enumerate(lens) if not n]].isnan().all()
     assert (got[full].float() - want).norm() <= 5 * 2 ** -9 * want.norm()
+
+
+def _mixed(model, monkeypatch):
+    """Scores of a step with a reply and a portion, and how often both were to be
+    attended in one launch (the CPU declines)."""
+    from helix_amd import ops
+    eng, asked = _engine(model), []
+    monkeypatch.setattr(ops, "mixed_attention",
+                        lambda *a: asked.append(a) is not None)
+    w = eng.decode_ws = eng.decode_ws or (torch.zeros(4, 4, 4, 64),
+                                          torch.zeros(4, 4, 4, 2))
+    assert len(w) == 2
+    eng.extend([("a", list(range(20)), [19])])
+    return eng.extend([("a", [7], [0]), ("b", list(range(30)), [29])]), \
+        len(asked)
+
+
+@pytest.mark.parametrize("which", ["_attend_decode", "_attend_prefill"])
+@pytest.mark.parametrize("where", ["class", "instance"])
+def test_attention_of_its_own_in_mixed_steps(monkeypatch, which, where):
+    """An Attention with another way to attend is asked for it in mixed steps."""
+    from helix_amd.models.llama import Attention
+    make = lambda: LlamaForCausalLM(PRESETS["tiny"]).init_random(3)  # noqa: E731
+    want, asked = _mixed(make(), monkeypatch)
+    assert asked == 2                           # layers
+    model, calls = make(), []
+    attn = model.layers[0].attn
+    base = getattr(Attention, which)
+
+    def other(self, *args):
+        calls.append(args)
+        return base(self, *args)
+
+    if where == "class":
+        attn.__class__ = type("Other", (Attention,), {which: other})
+    else:
+        setattr(attn, which, other.__get__(attn))
+    got, asked = _mixed(model, monkeypatch)
+    assert asked == 1 and len(calls) == (1 if which == "_attend_decode" else 2)
+    if which == "_attend_prefill":
+        assert calls[1][1] is not None          # a fresh portion's keys
+    torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
