@@ -353,7 +353,7 @@ class DecoderLayer(nn.Module):
     def forward(self, x, residual, cos_sin, kv_cache, meta,
                 form: str = "rows", few: bool = False, after=None, rows=None):
         """form "sums": the result's stretches, for the next norm. few: as few()
-        says; after (few): the weight of that norm, which the result then is but
+        says; after (few): weight and eps of that norm, which the result then is but
         for its division (ops.Unscaled). rows: those that are asked for, where attn
         is as written here; the others leave behind attention."""
         if residual is None:
@@ -367,7 +367,7 @@ class DecoderLayer(nn.Module):
         if few:
             h = self.attn(h, cos_sin, kv_cache, meta,
                           join=(residual, self.post_norm_w, self.eps))
-            join = None if after is None else (residual, after, self.eps)
+            join = None if after is None else (residual, *after)
             return self.mlp(h, form, join), residual
         h = self.attn(h, cos_sin, kv_cache, meta,
                       *(["sums", None, rows] if _own(self.attn, Attention)
@@ -439,8 +439,9 @@ class LlamaForCausalLM(nn.Module):
             own = _own(layer, DecoderLayer)
             extra = {"form": "sums"} if own else {}
             if few[i]:
-                extra.update(few=True, after=self.layers[i + 1].input_norm_w
-                             if few[i + 1] else None)
+                then = self.layers[i + 1] if few[i + 1] else None
+                extra.update(few=True, after=then and (then.input_norm_w,
+                                                       then.eps))
             elif rows is not None and i + 1 == len(self.layers):
                 extra["rows"] = rows
             x, residual = layer(x, residual, self.cos_sin, cache, meta, **extra)
