@@ -461,7 +461,7 @@ def mixed_attention(portions: tuple, replies: tuple, scale: float,
     """attn_prefill of portions (out, q, k, v, cu_seqlens, cu_seqlens_k,
     max_seqlen) and paged_attn_decode of replies (out, q, k_cache, v_cache,
     block_tables, seq_lens, tmp_out, tmp_ml, max_len) in one launch, or False
-    and nothing done for what only those two take."""
+    and nothing done for what only those two take, or take faster."""
     if not portions[1].is_cuda:
         return False
     return _native().attn_mixed(*portions, *replies, scale, window)

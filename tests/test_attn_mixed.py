@@ -61,3 +61,30 @@ def test_left_alone(hq, hkv, d, bs):
     assert not ops.mixed_attention((op, qp, k, v, cu, cuk, most),
                                    (od, qd, kc, vc, bt, sl, *ws, 50), 0.1, 0)
     assert (op == 7).all() and (od == 7).all()
+
+
+# many short replies leave the joint launch to portions that hide more than they lose
+@pytest.mark.parametrize("rows,bound,fp8,new,cached,joint", [
+    (230, 300, True, [17], [0], True), (256, 300, True, [17], [0], False),
+    (256, 300, True, [17], [100], True), (512, 300, True, [300], [0], False),
+    (512, 300, True, [17], [700], True), (256, 1025, True, [17], [0], True),
+    (512, 300, False, [17], [0], False), (512, 385, False, [17], [0], True),
+    (512, 300, False, [17], [100], True), (450, 300, False, [17], [0], True)])
+def test_where_one_launch_pays(rows, bound, fp8, new, cached, joint):
+    """Either way the model's step has the same bits: what is declined is done by
+    the two launches."""
+    lens = [bound] + [1 + 37 * i % 40 for i in range(1, rows)]
+    (qp, k, v, cu, cuk, most), (qd, kc, vc, bt, sl) = _inputs(
+        32, 8, 128, 16, fp8, lens, new, cached)
+    ws = ops.decode_workspace(rows, 32, 128, bound, DEV)
+    op, od = torch.full_like(qp, 7.0), torch.full_like(qd, 7.0)
+    assert joint == ops.mixed_attention(
+        (op, qp, k, v, cu, cuk, most), (od, qd, kc, vc, bt, sl, *ws, bound),
+        0.1, 0)
+    if joint:
+        assert torch.equal(od, ops.paged_attn_decode(qd, kc, vc, bt, sl, 0.1,
+                                                     ws, bound))
+        assert torch.equal(op, ops.attn_prefill(qp, k, v, cu, most, 0.1, True,
+                                                0, cuk))
+    else:
+        assert (op == 7).all() and (od == 7).all()
