@@ -30,7 +30,10 @@ __global__ __launch_bounds__(prefill::NT, 2) void attn_mixed_kernel(
   if (at < 0) {
     prefill::queries<D, true>(out, qp, k, v, pm, blockIdx.x, lds);
   } else {
-    paged::rows<D, G, F8, true>(qd, kc, vc, dm, at, pieces,
+    const int per = dm.heads_first ? dm.Hkv : pieces;
+    const int high = at / per, low = at - high * per;
+    paged::rows<D, G, F8, true>(qd, kc, vc, dm, dm.heads_first ? high : low,
+                                dm.heads_first ? low : high,
                                 *reinterpret_cast<paged::Shared<D, G>*>(lds));
   }
 }

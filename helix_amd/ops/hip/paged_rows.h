@@ -70,7 +70,7 @@ struct Rows {
   float* part;                 // [B, Hq, max_parts, D]
   float* ml;                   // [B, Hq, max_parts, 2]
   int B, Hkv, bs, shift, max_blocks, max_parts, window, limit;
-  bool split;
+  bool split, heads_first;     // whose neighbours are heads, not rows or pieces
   float mul;                   // scale * log2(e)
 };
 
@@ -276,8 +276,6 @@ constexpr int waves_per_simd(int D, int G) {
   return D == 128 ? (G > 4 ? 2 : 3) : (G > 4 ? 3 : 4);
 }
 
-// PAGE8: pages are a power of two of at least 8 tokens, so the 8 keys of a
-// lane group lie in one page.
 // The waves' results.
 template <int D, int G>
 struct Shared {
@@ -285,12 +283,16 @@ struct Shared {
   float st[2][NW][G];
 };
 
-// Work of workgroup `at`; each KV head has `pieces` of them.
+// Work of a workgroup: `block` of those of KV head g. The heads of an uncut row
+// follow each other, so that a long row's lie on different XCDs (32 heads on 8, one of
+// 1000 beside 63 of 100 27.8 us before and 18.9, 256 of 20..1000 104.4 and 99.6).
+// PAGE8: pages are a power of two of at least 8 tokens, so the 8 keys of a
+// lane group lie in one page.
 template <int D, int G, bool F8, bool PAGE8>
 __device__ __forceinline__ void rows(const uint16_t* __restrict__ q,
                                      const void* __restrict__ kc,
                                      const void* __restrict__ vc,
-                                     const Rows& m, int at, int pieces,
+                                     Rows m, int block, int g,
                                      Shared<D, G>& lds) {
   constexpr int NC = D / 32;                  // inner steps of the scores
   constexpr int DPL = D / 16;                 // value dimensions of a lane
@@ -305,14 +307,8 @@ __device__ __forceinline__ void rows(const uint16_t* __restrict__ q,
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lo = lane & 15, hi = lane >> 4;
-  // The heads of an uncut row follow each other, so that a long row's lie on different
-  // XCDs (32 heads on 8, one of 1000 beside 63 of 100 27.8 us before and 18.9, 256
-  // of 20..1000 104.4 and 99.6).
-  const int per_g = m.split ? pieces : m.Hkv;
-  const int high = at / per_g, low = at - high * per_g;
-  const int g = m.split ? high : low;
   int seq, part, parts;
-  if (!find(m, m.split ? low : high, seq, part, parts)) return;
+  if (!find(m, block, seq, part, parts)) return;
   // The same in all lanes: scalar registers, so that a wave more fits a SIMD. Not
   // for up to four heads of bf16, which have waves enough and lose by more (32
   // heads of 64 on 8, 16 of 100..6000 24 us and 26; 16 on 16 of 128, 1 of 900
@@ -708,6 +704,7 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor k_cache,
                      (most <= 8 && rows >= 128) ||
                      (most <= 16 && rows >= 2 * TARGET);
   m.split = cuts && !whole;
+  m.heads_first = !m.split && B < 1 << 16;    // a grid has no more along y
   // a workspace is looked at whether or not these rows would be cut
   const int64_t pieces = (int64_t)B * Hq * m.max_parts;
   TORCH_CHECK(!cuts || (tmp_out.is_contiguous() && tmp_ml.is_contiguous() &&

@@ -25,6 +25,18 @@ def test_many(rows, bound):
     check(8, 8, 64, rows, bound, False)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [65535, 65536])
+def test_more_rows_than_a_grid_has_along_y(rows):
+    """Of one key, a row's result is its value."""
+    kc, vc = (torch.randn(3, 2, 8, 64).bfloat16().to(DEV) for _ in range(2))
+    bt = (torch.arange(rows) % 3).int()[:, None].to(DEV)
+    got = ops.paged_attn_decode(
+        torch.randn(rows, 2, 64).bfloat16().to(DEV), kc, vc, bt,
+        torch.ones(rows, dtype=torch.int32, device=DEV), 0.125, max_len=1)
+    assert torch.equal(got, vc[bt[:, 0].long(), :, 0])
+
+
 def check(hq, hkv, d, rows, bound, fp8):
     """Lengths from nothing to the bound, heads of a row on every XCD; caches end
     with the last page, and what lies behind a row's end is not a number."""
