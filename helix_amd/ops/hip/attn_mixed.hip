@@ -28,7 +28,8 @@ __global__ __launch_bounds__(prefill::NT, 2) void attn_mixed_kernel(
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int at = (int)blockIdx.x - portions;
   if (at < 0) {
-    prefill::queries<D, true>(out, qp, k, v, pm, blockIdx.x, lds);
+    prefill::queries<D, true>(out, qp, k, v, pm,
+                              prefill::place_of(pm, blockIdx.x), lds);
   } else {
     const int per = dm.heads_first ? dm.Hkv : pieces;
     const int high = at / per, low = at - high * per;
@@ -87,7 +88,8 @@ bool attn_mixed(torch::Tensor out_p, torch::Tensor q_p, torch::Tensor k,
   const paged::Plan d = paged::plan(out_d, q_d, k_cache, v_cache, block_tables,
                                     seq_lens, scale, tmp_out, tmp_ml, max_len,
                                     window);
-  if (p.grid == 0 || d.m.B == 0) return false;
+  const int portions = p.blocks();
+  if (portions == 0 || d.m.B == 0) return false;
   const auto seen = [&](int64_t n, int64_t more) {
     return window > 0 ? std::min(n, window + more) : n;
   };
@@ -96,11 +98,11 @@ bool attn_mixed(torch::Tensor out_p, torch::Tensor q_p, torch::Tensor k,
   auto stream = at::hip::getCurrentHIPStream();
 #define HELIX_AM(G, F8)                                                      \
   hipLaunchKernelGGL((attn_mixed_kernel<G, F8>),                             \
-                     dim3(p.grid + d.pieces * d.m.Hkv), dim3(prefill::NT),   \
+                     dim3(portions + d.pieces * d.m.Hkv), dim3(prefill::NT), \
                      prefill::lds_of(D), stream, (uint16_t*)out_p.data_ptr(),\
                      (const uint16_t*)q_p.data_ptr(),                        \
                      (const uint16_t*)k.data_ptr(),                          \
-                     (const uint16_t*)v.data_ptr(), p.m, p.grid,             \
+                     (const uint16_t*)v.data_ptr(), p.m, portions,           \
                      (const uint16_t*)q_d.data_ptr(), k_cache.data_ptr(),    \
                      v_cache.data_ptr(), d.m, d.pieces)
   if (G == 4) {

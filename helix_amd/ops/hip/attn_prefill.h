@@ -72,6 +72,7 @@ struct Prefill {
   int Hq, G, groups, q_tiles, seqs, window;   // groups: of G heads
   bool flip;                   // negative scale: of negated queries
   bool spread;                 // groups of heads go round the XCDs
+  int whole;                   // spread: rounds in which each XCD has a group
   float mul, far_mul;          // |scale| * log2(e); a power of two above it
 };
 
@@ -123,40 +124,49 @@ __device__ __forceinline__ int cross(int r) {
 // Bytes of LDS that a workgroup takes.
 constexpr int lds_of(int D) { return 4 * KT * D * 2; }
 
-// Work of workgroup `block`; tiles: lds_of(D) bytes.
+// A workgroup's XCD, tile of queries (latest first), head within its group and the
+// group's number among those of this XCD. Not spread: heads are groups of their own.
+struct Place {
+  int xcd, head, tile, round;
+};
+// By a number, which goes up in this order. A launch of prompts alone has a grid of
+// three dimensions instead of the divisions (28 heads on 4, 8 x 128 9.7 us and 9.5).
+__device__ __forceinline__ Place place_of(const Prefill& m, int block) {
+  const int heads = m.spread ? m.G : 1, all = heads * m.q_tiles;
+  const int at = block >> 3, round = at / all, in = at - round * all;
+  const int tile = in / heads;
+  return {block & 7, in - tile * heads, tile, round};
+}
+
+// tiles: lds_of(D) bytes
 template <int D, bool CAUSAL>
 __device__ __forceinline__ void queries(uint16_t* __restrict__ out,
                                         const uint16_t* __restrict__ q,
                                         const uint16_t* __restrict__ k,
                                         const uint16_t* __restrict__ v,
-                                        const Prefill& m, int block,
-                                        uint16_t* tiles) {
+                                        Prefill m, Place at, uint16_t* tiles) {
   constexpr int NK = D / 16, NV = D / 32, PR = D / 8;
   constexpr int LOADS = KT * PR / NT;
   uint16_t* const kl[2] = {tiles, tiles + KT * D};
   uint16_t* const vl[2] = {tiles + 2 * KT * D, tiles + 3 * KT * D};
-  const int xcd = block & 7, at = block >> 3;
-  int b, g, h, tile;
-  if (m.spread) {
-    // a group's heads, latest queries first, behind the XCD's groups before
-    // (divisions are 0.2 us of a launch: as few as there can be, 8 x 288 10.74 -> 10.56)
-    const int all = m.G * m.q_tiles, before = at / all, in = at - before * all;
-    const int group = before * 8 + xcd;
-    if (group >= m.seqs * m.groups) return;
+  int b, g, h;
+  if (m.spread && at.round < m.whole) {
+    const int group = at.round * 8 + at.xcd;
     b = group / m.groups;
-    tile = m.G == 1 ? in : in / m.G;
     g = group - b * m.groups;
-    h = g * m.G + in - tile * m.G;
+    h = g * m.G + at.head;
   } else {
-    const int total = m.seqs * m.Hq, chunk = cdiv(total, 8);
-    const int sh = xcd * chunk + at / m.q_tiles;
-    if (at / m.q_tiles >= chunk || sh >= total) return;
+    // heads one by one: of all groups, or of those that are too few for a round
+    const int from = m.spread ? m.whole * 8 * m.G : 0;
+    const int left = m.seqs * m.Hq - from, chunk = cdiv(left, 8);
+    const int in = m.spread ? at.head : at.round, item = at.xcd * chunk + in;
+    if (in >= chunk || item >= left) return;
+    const int sh = from + item;
     b = sh / m.Hq;
     h = sh - b * m.Hq;
-    tile = at % m.q_tiles;
     g = h / m.G;
   }
-  const int q0 = (m.q_tiles - 1 - tile) * QT;
+  const int q0 = (m.q_tiles - 1 - at.tile) * QT;
   const int row0 = m.cu_q[b], qlen = m.cu_q[b + 1] - row0;
   if (q0 >= qlen) return;
   const int key0 = m.cu_k[b], klen = m.cu_k[b + 1] - key0;
@@ -167,7 +177,7 @@ __device__ __forceinline__ void queries(uint16_t* __restrict__ out,
   const int lo = lane & 31, hi = lane >> 5;
   // a wave without queries only loads; which of the four that is goes round, or
   // one SIMD would have all of them
-  const int qw = q0 + (wid + at & 3) * 32;
+  const int qw = q0 + (wid + at.head + at.round & 3) * 32;
   const bool idle = qw >= qlen;
   u16x8 qf[NK];
   const int qi = qw + lo;                     // of this lane
@@ -362,11 +372,12 @@ inline torch::Tensor rows(const torch::Tensor& t) {
   return (uintptr_t)r.data_ptr() % 16 == 0 ? r : r.clone();
 }
 
-// Work of a call and its workgroups, checked (none: grid is 0). q, k and v are copied
+// Work of a call and its workgroups, checked (none: blocks is 0). q, k and v are copied
 // where the kernel would not read them as they lie.
 struct Plan {
   Prefill m{};
-  int grid = 0;
+  dim3 grid{0, 0, 0};          // Place: XCDs and heads, tiles, rounds
+  int blocks() const { return (int)(grid.x * grid.y * grid.z); }
 };
 
 inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor& k,
@@ -415,12 +426,15 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor& k,
   m.flip = scale < 0;
   // Groups of heads that share keys go round the XCDs, and each sees some of every
   // sequence, whatever their lengths; a few that leave XCDs without one are cut
-  // into heads.
+  // into heads, and so are those left over by whole rounds: the XCDs that had one
+  // of them more took that much longer (28 heads on 4, 9 x 128 12.4 us, 10.0
+  // now; 8 on 1, 41 x 600 65.6 and 62.8; 24 on 3, 17 x 600 77.8 and 75.5).
   m.groups = Hkv;
   const int groups = B * Hkv;
   m.spread = groups % 8 == 0 || groups >= 32;
-  p.grid = m.spread ? 8 * cdiv(groups, 8) * m.G * m.q_tiles
-                    : 8 * cdiv(B * Hq, 8) * m.q_tiles;
+  m.whole = groups / 8;
+  p.grid = m.spread ? dim3(8 * m.G, m.q_tiles, cdiv(groups, 8))
+                    : dim3(8, m.q_tiles, cdiv(B * Hq, 8));
   return p;
 }
 

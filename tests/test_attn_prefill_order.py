@@ -61,3 +61,26 @@ def test_rising_scores(rise, d, causal):
     k[..., 0] = (at * rise * 0.6931 * d ** 0.5)[:, None]
     _check([n], h, h, d, causal, q.bfloat16(), k.bfloat16(), v.bfloat16(),
            d ** -0.5)
+
+
+# whole rounds of groups and some left over, which are cut into heads: fewer heads
+# than XCDs, more, and seven groups
+@pytest.mark.parametrize("lens,hq,hkv,d,causal", [
+    ([128] * 9, 28, 4, 128, True), ([130, 1, 40] * 11, 8, 1, 128, True),
+    ([33, 200, 129] * 7, 6, 3, 64, False), ([70] * 35, 4, 1, 64, True),
+    ([140, 20, 7, 129, 260] * 2 + [64], 14, 7, 64, False),
+    ([150] * 41, 2, 1, 64, True)])
+def test_groups_left_over(lens, hq, hkv, d, causal):
+    g = torch.Generator(device=DEV).manual_seed(len(lens))
+    q, k, v = (torch.randn(sum(lens), n, d, device=DEV, generator=g).bfloat16()
+               for n in (hq, hkv, hkv))
+    _check(lens, hq, hkv, d, causal, q, k, v, d ** -0.5)
+
+
+@pytest.mark.parametrize("texts", [32767, 32768])
+def test_more_groups_than_a_grid_has_along_z(texts):
+    """Of one key, a result is its value."""
+    q, k, v = (torch.randn(texts, 16, 64, device=DEV).bfloat16()
+               for _ in range(3))
+    cu = torch.arange(texts + 1, dtype=torch.int32, device=DEV)
+    assert torch.equal(ops.attn_prefill(q, k, v, cu, 1, 0.125, False), v)
