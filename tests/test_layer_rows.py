@@ -118,6 +118,8 @@ def test_qkv_bytes(m, k, hq, hkv, d, fp8):
     kc, vc = (torch.zeros(m, hkv, 16, d, device=DEV, dtype=torch.uint8 if fp8
                           else torch.bfloat16) for _ in range(2))
     slots = torch.randperm(m * 16, device=DEV)[:m]
+    if m > 1:
+        slots[m // 2] = -1                              # padding: not written
     q, ko, vo = ops.rows_qkv(pos, x8, w8, None, cs, hq, hkv, d, (kc, vc),
                              slots, True, ws)
     back = lambda b, s: (b.view(torch.float8_e4m3fn).double()  # noqa: E731
@@ -129,14 +131,19 @@ def test_qkv_bytes(m, k, hq, hkv, d, fp8):
     _near(q, t[:, :hq])
     _near(ko, t[:, hq:hq + hkv])
     _near(vo, y[:, hq + hkv:])
-    for cache, want in ((kc, ko), (vc, vo)):
-        got = cache[slots // 16, :, slots % 16]
-        assert torch.equal(got, ops.kv_fp8_quant(want) if fp8 else want) \
-            or fp8       # of sums before they were rounded to bf16
-        if fp8:
-            got = got.view(torch.float8_e4m3fn).double()
-            assert ((got - want.double()).abs()
-                    <= 2 ** -3.9 * want.double().abs() + 2 ** -9).all()
+    there = slots >= 0
+    at = slots[there]
+    for cache, rows, want in ((kc, ko, t[:, hq:hq + hkv]),
+                              (vc, vo, y[:, hq + hkv:])):
+        got = cache[at // 16, :, at % 16]
+        if fp8:               # of sums before they were rounded to bf16: 3 bits
+            want = want[there]
+            assert ((got.view(torch.float8_e4m3fn).double() - want).abs()
+                    <= 2 ** -4 * want.abs() + 2 ** -9).all()
+        else:
+            assert torch.equal(got, rows[there])
+        cache[at // 16, :, at % 16] = 0
+        assert not cache.any()
 
 
 def test_refuses():
