@@ -73,6 +73,7 @@ struct Prefill {
   bool flip;                   // negative scale: of negated queries
   bool spread;                 // groups of heads go round the XCDs
   int whole;                   // spread: rounds in which each XCD has a group
+  int in_round;                // workgroups of a round
   float mul, far_mul;          // |scale| * log2(e); a power of two above it
 };
 
@@ -129,13 +130,18 @@ constexpr int lds_of(int D) { return 4 * KT * D * 2; }
 struct Place {
   int xcd, head, tile, round;
 };
-// By a number, which goes up in this order. A launch of prompts alone has a grid of
-// three dimensions instead of the divisions (28 heads on 4, 8 x 128 9.7 us and 9.5).
+// By a number within a round and the round's, or by one number, which is a division
+// more.
+__device__ __forceinline__ Place place_of(const Prefill& m, int block,
+                                          int round) {
+  const int in = block >> 3;
+  if (!m.spread || m.G == 1) return {block & 7, 0, in, round};
+  const int tile = in / m.G;
+  return {block & 7, in - tile * m.G, tile, round};
+}
 __device__ __forceinline__ Place place_of(const Prefill& m, int block) {
-  const int heads = m.spread ? m.G : 1, all = heads * m.q_tiles;
-  const int at = block >> 3, round = at / all, in = at - round * all;
-  const int tile = in / heads;
-  return {block & 7, in - tile * heads, tile, round};
+  const int round = block / m.in_round;
+  return place_of(m, block - round * m.in_round, round);
 }
 
 // tiles: lds_of(D) bytes
@@ -376,8 +382,8 @@ inline torch::Tensor rows(const torch::Tensor& t) {
 // where the kernel would not read them as they lie.
 struct Plan {
   Prefill m{};
-  dim3 grid{0, 0, 0};          // Place: XCDs and heads, tiles, rounds
-  int blocks() const { return (int)(grid.x * grid.y * grid.z); }
+  int rounds = 0;
+  int blocks() const { return m.in_round * rounds; }
 };
 
 inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor& k,
@@ -433,8 +439,8 @@ inline Plan plan(torch::Tensor out, torch::Tensor& q, torch::Tensor& k,
   const int groups = B * Hkv;
   m.spread = groups % 8 == 0 || groups >= 32;
   m.whole = groups / 8;
-  p.grid = m.spread ? dim3(8 * m.G, m.q_tiles, cdiv(groups, 8))
-                    : dim3(8, m.q_tiles, cdiv(B * Hq, 8));
+  m.in_round = 8 * m.q_tiles * (m.spread ? m.G : 1);
+  p.rounds = cdiv(m.spread ? groups : B * Hq, 8);
   return p;
 }
 

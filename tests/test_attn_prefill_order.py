@@ -78,7 +78,7 @@ def test_groups_left_over(lens, hq, hkv, d, causal):
 
 
 @pytest.mark.parametrize("texts", [32767, 32768])
-def test_more_groups_than_a_grid_has_along_z(texts):
+def test_more_rounds_than_a_grid_has_along_y(texts):
     """Of one key, a result is its value."""
     q, k, v = (torch.randn(texts, 16, 64, device=DEV).bfloat16()
                for _ in range(3))
