@@ -930,12 +930,12 @@ def layer_rows_fit(x, qkv: torch.Tensor, o: torch.Tensor,
                    head_dim: int) -> bool:
     """Whether a layer's four projections of these rows go by layer_rows.hip:
     sizes it takes, up to 4 rows of up to 8192 columns and up to 16 of up to
-    4096. Beyond, its workgroups of 16 columns read x more often than the launches
-    that they save are worth. us of the four with norms and rotation, apart and so: 1
-    row of 4096 (llama3-8b) 94.8 and 84.4, 16 101 and 96; of 3584 (qwen2-7b) 115.6
-    and 100.9, 118 and 115; of 2048 with 2 x 8192 48.6 and 35.0, 49.6 and 45.9; of
-    8192 (llama3-70b) 332 and 317, 8 334 and 336, 16 337 and 357; of 5120 with 2 x
-    13824 137 and 132, 8 142 and 144."""
+    4096. Beyond, its workgroups of 16 and 32 columns read x more often than the
+    launches that they save are worth. us of the four with norms and rotation, apart
+    and so: 1 row of 4096 (llama3-8b) 94.8 and 84.4, 16 101 and 96; of 3584
+    (qwen2-7b) 115.6 and 100.9, 118 and 115; of 2048 with 2 x 8192 48.6 and 35.0,
+    49.6 and 45.9; of 8192 (llama3-70b) 332 and 317, 8 334 and 336, 16 337 and 357;
+    of 5120 with 2 x 13824 137 and 132, 8 142 and 144."""
     x = x.rows if isinstance(x, Unscaled) else x
     if not x.is_cuda or x.dim() != 2 or x.shape[0] > LAYER_ROWS:
         return False

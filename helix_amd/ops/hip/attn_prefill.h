@@ -22,8 +22,10 @@
 //  - The heads that share keys run on one XCD, the latest queries, which see the
 //    most keys, first. Such groups go round the XCDs: with each XCD's sequences in
 //    a row, the one with the longest took 1.2 to 1.3 times the mean of them. Waves
-//    past the last query only load. us before -> now: 64 texts 56.2 -> 48.4, 31
-//    of 400..620 168 -> 147, 2000 and 5000 467 -> 262, 1 x 8192 574 -> 548.
+//    past the last query only load. us alone, before -> now: 64 texts 52 -> 49, 31
+//    of 400..620 154 -> 146, 2000 and 5000 467 -> 262, 1 x 8192 560 -> 528; in steps
+//    between products, where the clock is lower, the second takes 164, the last 561.
+//    Some sizes lose by the order: 3 x 600 22.7 -> 23.8.
 //
 // 32 heads on 8 of 128, us of the first kernel (64 queries, values transposed
 // element by element) -> products of 16x16 with addresses computed per tile

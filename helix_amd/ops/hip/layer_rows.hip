@@ -10,14 +10,16 @@
 // 4.4 us each, three of nine launches of a layer.
 //
 // A workgroup has all of the inner dimension, so that it sees whole sums: its four
-// waves have a quarter each, for the same 16 columns (GLU: of either factor), and
-// pass their sums through LDS. All waves begin at the start of their quarter: with
-// groups of columns beginning at different chunks, chunks dealt to the waves one by
-// one, or eight waves, 1 row of 4096 x 4096 took 7.6 to 11.5 us instead of 7.5.
-// Weights go straight to MFMA operands, a chunk of 256 of the inner dimension
-// ahead. Rows of x come by whole lines and become operands through a wave's own LDS:
-// by loads in operand order, which take half lines, 16 rows of it took 11.0 us
-// instead of 9.5, 8 rows of 4096 x 14336 27.5 instead of 25.2.
+// waves have a quarter each, for the same columns, and pass their sums through LDS.
+// Columns are 16 (JOIN, QKV of up to 4 rows) or 32 (QKV of more; GLU, of either
+// factor). Waves begin at the start of their quarter: with groups of columns beginning
+// at different chunks, chunks dealt to the waves one by one, or eight waves, 1 row of
+// 4096 x 4096 took 7.6 to 11.5 us instead of 7.5. GLU's groups do begin apart (`turn`).
+// Weights go straight to MFMA operands, a chunk of the inner dimension ahead, which is
+// 512 bytes, and 256 of GLU and of more than 16 rows (see `run`). Rows of x come by
+// whole lines and become operands through a wave's own LDS: by loads in operand order,
+// which take half lines, 16 rows of it took 11.0 us instead of 9.5, 8 rows of 4096 x
+// 14336 27.5 instead of 25.2.
 //
 // us of a product and the launch before or behind it (gemm_rows.hip with norm.hip
 // or rope_qkv.hip), and of all here, weights from memory:
@@ -27,6 +29,8 @@
 //   M  4  15.1  13.4     13.6   9.7     27.9  23.9     43.3  43.3
 //   M  8  15.6  13.4     13.8   9.7     28.3  25.0     43.5  44.7
 //   M 16  15.9  14.9     14.2  10.6     29.2  28.5     44.7  45.8
+// GLU gains nothing by itself: it is here to take rows whose division is still to come,
+// which is what spares JOIN a norm behind it.
 // QKV goes on to 32 rows, without squares, and takes e4m3 (scaled 16x16x128 with
 // unity scales; those of rows meet the sums): 32 rows of 6144 x 4096 16.4 us apart
 // and 15.6, e4m3 13.4 and 10.3. The other forms would not gain there: 24 rows of
