@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 
 from helix_amd import ops
-from helix_amd.models.llama import _own
+from helix_amd.models.llama import _own, _written
 
 
 @dataclass
@@ -55,6 +55,7 @@ def _first_pays(cu: list) -> bool:
         b > a for a, b in zip(cu, cu[1:]))
 
 
+@_written
 class BertLayer(nn.Module):
     PARAMS = ("qkv_w", "qkv_b", "attn_out_w", "attn_out_b", "attn_ln_w",
               "attn_ln_b", "up_w", "up_b", "down_w", "down_b", "out_ln_w",

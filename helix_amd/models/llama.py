@@ -135,6 +135,18 @@ PRESETS = {
 }
 
 
+_WRITTEN = {}                     # class -> its forward as written
+
+
+def _written(kind: type) -> type:
+    _WRITTEN[kind] = kind.forward
+    return kind
+
+
+_written(FP8Linear)
+
+
+@_written
 class HLinear(nn.Linear):
     """nn.Linear routed through ops.linear: owned MFMA kernels, for a few rows
     by streamed weights, else by tiles; sizes and calls they do not take, or not
@@ -155,9 +167,11 @@ class HLinear(nn.Linear):
 
 def _own(m: nn.Module, *kinds: type) -> bool:
     """Whether m is one of these modules as written here: a subclass, a module
-    put in its place or a hook gets and returns what torch's linear would,
-    [T, N], and never a form."""
-    if type(m) not in kinds:
+    put in its place, a forward put in place of its class's or a hook gets and
+    returns what torch's linear would, [T, N], and never a form."""
+    kind = type(m)
+    if kind not in kinds or \
+            kind.forward is not _WRITTEN.get(kind, kind.forward):
         return False
     d = m.__dict__
     return not (d["_forward_hooks"] or d["_forward_pre_hooks"]
@@ -172,6 +186,7 @@ def _project(proj: nn.Module, x: torch.Tensor, form: str) -> torch.Tensor:
     return ops.silu_and_mul(out) if form == "glu" else out
 
 
+@_written
 class Attention(nn.Module):
     def __init__(self, cfg: LlamaConfig, tp_size: int = 1, tp_rank: int = 0):
         super().__init__()
@@ -287,6 +302,7 @@ class Attention(nn.Module):
                                      window=self.window, out=out)
 
 
+@_written
 class MLP(nn.Module):
     def __init__(self, cfg: LlamaConfig, tp_size: int = 1):
         super().__init__()
@@ -318,6 +334,7 @@ def _norm_for(m: nn.Module, kind: type, proj: str):
     return ops.fused_add_rms_norm_fp8 if bytes_ else ops.fused_add_rms_norm
 
 
+@_written
 class DecoderLayer(nn.Module):
     def __init__(self, cfg: LlamaConfig, tp_size: int = 1, tp_rank: int = 0):
         super().__init__()
@@ -369,9 +386,10 @@ class DecoderLayer(nn.Module):
                           join=(residual, self.post_norm_w, self.eps))
             join = None if after is None else (residual, *after)
             return self.mlp(h, form, join), residual
-        h = self.attn(h, cos_sin, kv_cache, meta,
-                      *(["sums", None, rows] if _own(self.attn, Attention)
-                        else []))
+        extra = {"form": "sums"} if _own(self.attn, Attention) else {}
+        if rows is not None:
+            extra["rows"] = rows
+        h = self.attn(h, cos_sin, kv_cache, meta, **extra)
         if rows is not None:
             residual = residual[rows]
         h, residual = _norm_for(self.mlp, MLP, "gate_up_proj")(
@@ -380,6 +398,7 @@ class DecoderLayer(nn.Module):
         return h, residual
 
 
+@_written
 class LlamaForCausalLM(nn.Module):
     paged_prefill = False        # cached prefixes are gathered
     extension = "_C"             # native library of its kernels

@@ -249,3 +249,24 @@ def test_attention_of_its_own_in_mixed_steps(monkeypatch, which, where):
     if which == "_attend_prefill":
         assert calls[1][1] is not None          # a fresh portion's keys
     torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["LlamaForCausalLM", "DecoderLayer",
+                                  "Attention", "MLP", "HLinear"])
+def test_forward_of_a_class_put_in_place(monkeypatch, kind):
+    """It is called for prompts of any length, as often and with as many rows."""
+    from helix_amd.models import llama
+    cls = getattr(llama, kind)
+    base, seen = cls.forward, []
+
+    def forward(self, x, *args):
+        seen.append(x.shape[0])
+        return base(self, x, *args)
+
+    model = LlamaForCausalLM(PRESETS["tiny"]).init_random(3)
+    want = _last_scores(_engine(model), 300)
+    monkeypatch.setattr(cls, "forward", forward)
+    got = _last_scores(_engine(model), 300)
+    rows = {"LlamaForCausalLM": [300], "HLinear": [300] * 8 + [1]}
+    assert seen == rows.get(kind, [300] * 2)
+    torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
