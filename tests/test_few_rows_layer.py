@@ -64,3 +64,26 @@ def test_layers_of_a_few_rows(monkeypatch, preset, other):
     for a, b in zip(kept, caches):
         for x, y in zip(a, b):
             torch.testing.assert_close(x, y, atol=1e-5, rtol=1e-5)
+
+
+def test_a_layer_is_asked_shortly_before_its_turn(monkeypatch):
+    """What a layer's launches may be is asked while those of the layer before are
+    under way, not of all layers before the first."""
+    from helix_amd.models.llama import DecoderLayer
+    model = LlamaForCausalLM(PRESETS["tiny-gqa"]).init_random(3)
+    for name, f in (("layer_rows_fit", lambda *a: True), ("rows_join", _join),
+                    ("rows_glu", _glu), ("rows_qkv", _qkv)):
+        monkeypatch.setattr(ops, name, f)
+    order, few = [], DecoderLayer.few
+
+    def asked(self, x):
+        order.append(("few", list(model.layers).index(self)))
+        return few(self, x)
+
+    monkeypatch.setattr(DecoderLayer, "few", asked)
+    glu = ops.rows_glu
+    monkeypatch.setattr(ops, "rows_glu", lambda *a: order.append(
+        ("run", sum(k == "run" for k, _ in order))) or glu(*a))
+    _pass(model)
+    assert order == [("few", 0), ("few", 1), ("run", 0), ("few", 2),
+                     ("run", 1), ("few", 3), ("run", 2), ("run", 3)]
