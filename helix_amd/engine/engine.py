@@ -476,12 +476,13 @@ class LLMEngine:
                 slot_mapping=torch.cat([dmeta.slot_mapping,
                                         meta.slot_mapping]),
                 positions=torch.cat([dmeta.positions, meta.positions]))
-        ids = torch.tensor([t for i in order for t in spans[i].ids],
-                           dtype=torch.int64, device=dev)
+        tokens = [t for i in order for t in spans[i].ids]
+        # in one copy: the pass begins once they are there
+        ids, at = torch.tensor(tokens + rows, dtype=torch.int64,
+                               device=dev).split([len(tokens), len(rows)])
         if not rows:
             self.model(ids, self.kv.caches, meta)
             return None
-        at = torch.tensor(rows, dtype=torch.int64, device=dev)
         # of the model itself: one around it that hands on attributes would not
         # be called
         if hasattr(type(self.model), "forward_rows"):
